@@ -4,6 +4,8 @@
 
 Every .hip file in this directory is one translation unit; they are compiled in parallel and linked
 into flash_dropout/_lib/libsparsedrop.so next to the Python package, which loads it with ctypes.
+torch_bridge.cpp (host code only: autograd nodes around the library's C ABI) becomes the extension module
+flash_dropout/_lib/sparsedrop_torch.so next to it.
 hipcc cross-compiles for gfx950 without a GPU present.
 """
 from __future__ import annotations
@@ -21,6 +23,8 @@ ROOT = CSRC.parent.parent
 OUT_DIR = CSRC.parent / "flash_dropout" / "_lib"
 OBJ_DIR = CSRC / "build"
 LIB = OUT_DIR / "libsparsedrop.so"
+BRIDGE = OUT_DIR / "sparsedrop_torch.so"
+BRIDGE_SRC = CSRC / "torch_bridge.cpp"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -46,7 +50,7 @@ def source_hash() -> str:
     """Hash of everything the library is compiled from; the library reports the one it was built with
     (sd_source_hash) and the loader refuses a library whose sources have changed since."""
     h = hashlib.sha256()
-    for f in [*sources(), *sorted(CSRC.glob("*.h")), *sorted((ROOT / "include").glob("*.h"))]:
+    for f in [*sources(), *sorted(CSRC.glob("*.cpp")), *sorted(CSRC.glob("*.h")), *sorted((ROOT / "include").glob("*.h"))]:
         h.update(f.name.encode())
         h.update(f.read_bytes())
     return h.hexdigest()[:16]
@@ -77,16 +81,33 @@ def write_source_hash() -> Path:
     return inc
 
 
+def bridge_command() -> list[str]:
+    """g++ on the autograd bridge: host code, against torch's headers and libraries and libsparsedrop.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [f"-I{p}" for p in (ROOT / "include", OBJ_DIR)]
+    inc += [f"-isystem{p}" for p in (*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"])]
+    libs = Path(torch.__file__).resolve().parent / "lib"
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=sparsedrop_torch",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, str(BRIDGE_SRC), "-o", str(BRIDGE),
+            f"-L{libs}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python",
+            f"-L{OUT_DIR}", "-lsparsedrop", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libs}"]
+
+
 def build(force: bool = False, verbose: bool = False) -> Path:
     OUT_DIR.mkdir(parents=True, exist_ok=True)
     headers = sorted(CSRC.glob("*.h")) + sorted((ROOT / "include").glob("*.h"))
-    headers.append(write_source_hash())
+    hash_inc = write_source_hash()  # included by api.hip (and the bridge) only
     jobs = []
     objs = []
     for src in sources():
         obj = OBJ_DIR / (src.stem + ".o")
         objs.append(obj)
-        if force or _stale(obj, [src, *headers]):
+        if force or _stale(obj, [src, *headers, *([hash_inc] if src.stem == "api" else [])]):
             jobs.append([HIPCC, *FLAGS, "-c", str(src), "-o", str(obj)])
     if verbose:
         for j in jobs:
@@ -94,7 +115,11 @@ def build(force: bool = False, verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         list(ex.map(_run, jobs))
     if force or jobs or _stale(LIB, objs):
-        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs)])
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname,libsparsedrop.so", "-o", str(LIB),
+              *map(str, objs)])
+    # (the bridge carries the hash of all sources too, so it follows every change of the library)
+    if force or _stale(BRIDGE, [BRIDGE_SRC, LIB, hash_inc]):
+        _run(bridge_command())
     return LIB
 
 

@@ -1,0 +1,741 @@
+// The autograd side of the package in native code: one Python call per layer (or stack) and direction instead of a
+// Python autograd function around ctypes calls.
+//
+// What bounds a step of a small layer is the host: at 128 x 256 -> 256 the two launches of a step run for 19 us and
+// the Python path around them (argument checks, tensor views, 45-argument ctypes calls, the backward's hop into the
+// interpreter on autograd's thread) took 64-146 us, depending on the host.  Here the checks, the allocations, the
+// library calls and the backward node are compiled, and the backward runs without the interpreter lock.
+//
+// Every computation is a call into libsparsedrop.so through its C ABI; torch owns memory, streams and the graph.
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <torch/extension.h>
+
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <array>
+#include <atomic>
+#include <string>
+#include <vector>
+
+#include "sparsedrop.h"
+
+#if __has_include("source_hash.inc")
+#include "source_hash.inc"
+#else
+#define SD_SOURCE_HASH "unknown"
+#endif
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+PyObject* library_error = nullptr;  // SparseDropError, once the loader has handed it over
+
+// Raised on whatever thread a call failed on (a backward runs on autograd's), so with the interpreter lock taken.
+[[noreturn]] void raise_library_error(const std::string& msg) {
+  pybind11::gil_scoped_acquire gil;
+  PyErr_SetString(library_error ? library_error : PyExc_RuntimeError, msg.c_str());
+  python_error err;
+  err.persist();
+  throw std::move(err);
+}
+
+void check(int rc, const char* fn) {
+  if (rc == SD_OK) return;
+  const std::string msg = std::string(fn) + ": " + sd_last_error();
+  TORCH_CHECK_VALUE(rc != SD_ERR_INVALID, msg);
+  TORCH_CHECK_NOT_IMPLEMENTED(rc != SD_ERR_UNSUPPORTED, msg);
+  raise_library_error(msg);
+}
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+int dtype_of(const Tensor& t) { return t.scalar_type() == at::kBFloat16 ? SD_BF16 : SD_F16; }
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// ---- operands -----------------------------------------------------------------------------------------------------
+// `x` itself when it is a row- or column-major matrix in memory, else a contiguous copy (expanded or doubly strided).
+Tensor as_matrix(const Tensor& x) {
+  const int64_t rows = x.size(0), cols = x.size(1), sr = x.stride(0), sc = x.stride(1);
+  if (sc == 1 && (rows <= 1 || sr >= cols)) return x;
+  if (sr == 1 && (cols <= 1 || sc >= rows)) return x;
+  return x.contiguous();
+}
+
+// pointer and element strides; the stride of an extent-1 dimension is arbitrary in torch and normalised here
+struct Mat {
+  void* ptr = nullptr;
+  int64_t sr = 0, sc = 0;
+  Mat() = default;
+  explicit Mat(const Tensor& t) : ptr(t.data_ptr()), sr(t.stride(0)), sc(t.stride(1)) {
+    const int64_t rows = t.size(0), cols = t.size(1);
+    if (rows <= 1 && sc == 1) sr = std::max<int64_t>(cols, 1);
+    if (cols <= 1 && sr == 1) sc = std::max<int64_t>(rows, 1);
+    sr = std::max<int64_t>(sr, 1);
+    sc = std::max<int64_t>(sc, 1);
+  }
+};
+#define MAT(m) (m).ptr, (m).sr, (m).sc
+
+void check_operand(const char* name, const Tensor& x) {
+  TORCH_CHECK_VALUE(x.is_cuda(), name, " must be on the GPU (got ", x.device(), ")");
+  TORCH_CHECK_VALUE(x.dim() == 2, name, " must be 2D (got ", x.dim(), "D)");
+  TORCH_CHECK_TYPE(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, name,
+                   " must be float16 or bfloat16 (got ", x.dtype(), ")");
+  TORCH_CHECK_VALUE(x.numel() == 0 || x.stride(0) == 1 || x.stride(1) == 1, name,
+                    " must be row or column major (strides ", x.strides(), ")");
+}
+
+void check_pair(const Tensor& a, const Tensor& b) {
+  check_operand("A", a);
+  check_operand("B", b);
+  TORCH_CHECK_TYPE(a.scalar_type() == b.scalar_type(), "A and B must have the same dtype (", a.dtype(), " vs ",
+                   b.dtype(), ")");
+  TORCH_CHECK_VALUE(a.device() == b.device(), "A and B must be on the same device");
+  TORCH_CHECK_VALUE(a.size(1) == b.size(1), "reduction dims differ: A ", a.sizes(), ", B ", b.sizes());
+}
+
+Tensor check_mask(const Tensor& mask, int64_t mb, int64_t kb, const Tensor& like) {
+  TORCH_CHECK_TYPE(mask.scalar_type() == at::kBool, "Mask must be bool (got ", mask.dtype(), ")");
+  TORCH_CHECK_VALUE(mask.device() == like.device(), "mask must be on the same device as the operands");
+  TORCH_CHECK_VALUE(mask.dim() == 2 && mask.size(0) == mb && mask.size(1) == kb, "mask shape ", mask.sizes(),
+                    " does not match blocks [", mb, ", ", kb, "]");
+  if (mask.numel() && mask.stride(0) != 1 && mask.stride(1) != 1) return mask.contiguous();
+  return mask;
+}
+
+struct MaskArg {
+  const uint8_t* ptr = nullptr;
+  int64_t sr = 0, sc = 0;
+  MaskArg() = default;
+  explicit MaskArg(const Tensor& m) : ptr(static_cast<const uint8_t*>(m.data_ptr())), sr(m.stride(0)), sc(m.stride(1)) {
+    if (sr != 1 && sc != 1) {  // only possible for degenerate shapes
+      sr = m.size(1);
+      sc = 1;
+    }
+    sr = std::max<int64_t>(sr, 1);
+    sc = std::max<int64_t>(sc, 1);
+  }
+};
+
+Tensor new_matrix(const Tensor& like, int64_t rows, int64_t cols) { return at::empty({rows, cols}, like.options()); }
+
+// fp32 scratch for a split reduction, when the library wants one for this shape
+struct Scratch {
+  Tensor t;
+  void* ptr = nullptr;
+  int64_t bytes = 0;
+  Scratch(const Tensor& like, int64_t nbytes) {
+    if (nbytes <= 0) return;
+    t = at::empty({nbytes / 4}, like.options().dtype(at::kFloat));
+    ptr = t.data_ptr();
+    bytes = nbytes;
+  }
+};
+
+// ---- mask and kept-block lists of one layer ---------------------------------------------------------------------------
+// One int32 buffer: row_ptr | col_ptr | col_idx | row_idx | bytes of a drawn mask.  `given` keeps a caller's mask alive.
+struct Lists {
+  Tensor buf, given;
+  int64_t bs = 0;         // block size of the mask
+  int64_t kernel_bs = 0;  // what the list-taking calls are told: 64, or 32 when the lists carry quadrant bits
+  int64_t mb = 0, kb = 0;          // mask grid
+  int64_t out_mb = 0, out_kb = 0;  // listed grid
+
+  void shape(int64_t rows, int64_t cols, int64_t bs_) {
+    bs = bs_;
+    const int64_t g = bs % 32 == 0 ? 64 : bs;
+    kernel_bs = bs % 64 == 32 ? 32 : g;
+    mb = ceil_div(rows, bs);
+    kb = ceil_div(cols, bs);
+    out_mb = ceil_div(rows, g);
+    out_kb = ceil_div(cols, g);
+    TORCH_CHECK_VALUE(mb > 0 && kb > 0, "mask must be non-empty");
+  }
+  void allocate(const Tensor& like, const OptTensor& mask) {
+    if (mask) given = check_mask(*mask, mb, kb, like);
+    const int64_t ints = out_mb + out_kb + 2 + 2 * out_mb * out_kb + (mask ? 0 : (mb * kb + 3) / 4);
+    buf = at::empty({ints}, like.options().dtype(at::kInt));
+  }
+  int32_t* row_ptr() const { return static_cast<int32_t*>(buf.data_ptr()); }
+  int32_t* col_ptr() const { return row_ptr() + out_mb + 1; }
+  int32_t* col_idx() const { return col_ptr() + out_kb + 1; }
+  int32_t* row_idx() const { return col_idx() + out_mb * out_kb; }
+  uint8_t* drawn() const { return given.defined() ? nullptr : reinterpret_cast<uint8_t*>(row_idx() + out_mb * out_kb); }
+  MaskArg mask() const {
+    if (given.defined()) return MaskArg(given);
+    MaskArg m;
+    m.ptr = drawn();
+    m.sr = kb;
+    m.sc = 1;
+    return m;
+  }
+};
+
+// Where a layer's mask comes from: given, pinned by a seed, or from the device-resident generator state.
+struct Draw {
+  OptTensor mask;
+  std::optional<uint64_t> seed;
+  OptTensor state;
+  uint64_t* state_ptr() const {
+    return (mask || seed || !state) ? nullptr : static_cast<uint64_t*>(state->data_ptr());
+  }
+};
+
+void check_p(double p) { TORCH_CHECK_VALUE(p >= 0.0 && p < 1.0, "p must be in [0, 1), got ", p); }
+
+// ---- the products of one layer ----------------------------------------------------------------------------------------
+// Y = act(s (keep . X) W^T) with mask and lists, one library call; pre: receives the pre-activation when wanted.
+Tensor layer_forward(const Tensor& x, const Tensor& w, int64_t bs, double p, const Draw& draw, int act, bool want_pre,
+                     Lists& lists, Tensor* pre) {
+  check_pair(x, w);
+  check_p(p);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  lists.shape(M, K, bs);
+  lists.allocate(x, draw.mask);
+  Tensor y = new_matrix(x, M, N);
+  if (want_pre && act != SD_ACT_NONE) *pre = new_matrix(x, M, N);
+  const int64_t g = bs % 32 == 0 ? 64 : bs;
+  Scratch ws(x, sd_splitk_workspace_bytes(M, N, K, g, 1));
+  const MaskArg given = draw.mask ? lists.mask() : MaskArg();
+  Mat pm;
+  if (pre && pre->defined()) pm = Mat(*pre);
+  const Mat xm(x), wm(w), ym(y);
+  c10::DeviceGuard guard(x.device());
+  check(sd_dropout_matmul_forward_act(MAT(xm), MAT(wm), MAT(ym), given.ptr, given.sr, given.sc, draw.state_ptr(),
+                                      draw.seed.value_or(0), 0, p, lists.drawn(), lists.row_ptr(), lists.col_idx(),
+                                      lists.col_ptr(), lists.row_idx(), M, N, K, bs, dtype_of(x), act, MAT(pm), ws.ptr,
+                                      ws.bytes, stream_of(x)),
+        "sd_dropout_matmul_forward_act");
+  return y;
+}
+
+// dX and / or dW of one layer in one library call; act_at: what dX's fused activation derivative is evaluated at.
+std::pair<Tensor, Tensor> layer_backward(const Tensor& dy, const Tensor& w, const Tensor& x, const Lists& lists,
+                                         double p, bool need_dx, bool need_dw, int act, const Tensor& act_at) {
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK_VALUE(dy.size(0) == M && dy.size(1) == N && dy.device() == x.device(), "dy must be a [", M, ", ", N,
+                    "] tensor on ", x.device());
+  if (N % 8 && N > 0 && M > 0 && K > 0 && (need_dx || need_dw)) {
+    // An output width that is not a multiple of 8 (a 10-class head) would put 16-byte loads across row ends in both
+    // products.  Zero-padded copies of dY and W (the reference pads its head to 128 outputs up front,
+    // eval/mlp/model.py:22-24,40) keep them on the specialised kernels: the extra columns of dY are zeros, so dX is
+    // unchanged, and the extra rows of dW are dropped.
+    const int64_t n8 = ceil_div(N, 8) * 8;
+    Tensor dyp = at::zeros({M, n8}, dy.options()), wp = at::zeros({n8, K}, w.options());
+    dyp.narrow(1, 0, N).copy_(dy);
+    if (need_dx) wp.narrow(0, 0, N).copy_(w);
+    auto [dx, dw] = layer_backward(dyp, wp, x, lists, p, need_dx, need_dw, act, act_at);
+    return {dx, dw.defined() ? dw.narrow(0, 0, N) : dw};
+  }
+  Tensor dx = need_dx ? new_matrix(x, M, K) : Tensor(), dw = need_dw ? new_matrix(x, N, K) : Tensor();
+  if (!(need_dx || need_dw) || M == 0 || K == 0) return {dx, dw};
+  if (N == 0) return {need_dx ? dx.zero_() : dx, dw};
+  const int64_t g = lists.kernel_bs == 32 ? 64 : lists.kernel_bs;
+  Scratch ws(x, need_dw ? sd_splitk_workspace_bytes(K, N, M, g, 1) : 0);
+  if (!need_dx) act = SD_ACT_NONE;
+  Mat am, dxm, dwm;
+  if (act != SD_ACT_NONE) am = Mat(act_at);
+  if (need_dx) dxm = Mat(dx);
+  if (need_dw) dwm = Mat(dw);
+  const Mat gm(dy), wm(w), xm(x);
+  c10::DeviceGuard guard(x.device());
+  check(sd_dropout_matmul_backward_act(MAT(gm), MAT(wm), MAT(xm), MAT(dxm), MAT(dwm), lists.row_ptr(), lists.col_idx(),
+                                       lists.col_ptr(), lists.row_idx(), M, N, K, lists.kernel_bs, p, dtype_of(x), act,
+                                       MAT(am), ws.ptr, ws.bytes, stream_of(x)),
+        "sd_dropout_matmul_backward_act");
+  return {dx, dw};
+}
+
+// A . B^T without dropout, with the activation in the store.
+Tensor dense(const Tensor& a, const Tensor& b, int act, bool want_pre, Tensor* pre) {
+  check_pair(a, b);
+  const int64_t M = a.size(0), N = b.size(0), K = a.size(1);
+  Tensor c = new_matrix(a, M, N);
+  if (want_pre && act != SD_ACT_NONE) *pre = new_matrix(a, M, N);
+  if (M == 0 || N == 0) return c;
+  Mat pm;
+  if (pre && pre->defined()) {
+    pm = Mat(*pre);
+    if (K == 0) pre->zero_();
+  }
+  if (K == 0) return c.zero_();
+  Scratch ws(a, sd_splitk_workspace_bytes(M, N, K, 0, 0));
+  const Mat am(a), bm(b), cm(c);
+  c10::DeviceGuard guard(a.device());
+  check(sd_gemm_act(MAT(am), MAT(bm), MAT(cm), M, N, K, dtype_of(a), act, MAT(pm), ws.ptr, ws.bytes, stream_of(a)),
+        "sd_gemm_act");
+  return c;
+}
+
+Tensor grad_matrix(const Tensor& g, const Tensor& like) {
+  return as_matrix(g.scalar_type() == like.scalar_type() ? g : g.to(like.scalar_type()));
+}
+
+template <typename N>
+bool records(const N& inputs) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor& t : inputs)
+    if (t.requires_grad()) return true;
+  return false;
+}
+
+// A product computed without recording; the node is attached to its result afterwards.
+struct NoRecord {
+  at::AutoDispatchBelowADInplaceOrView below;
+};
+
+// Autocast contract of the reference (custom_fwd(cast_inputs=torch.float16), blockwise_dropout_matmul_cuda.py:9): under
+// autocast the operands are cast to the autocast dtype; outside it they must already be float16 / bfloat16.
+Tensor autocast(const Tensor& t) {
+  return at::autocast::is_autocast_enabled(at::kCUDA) ? t.to(at::autocast::get_autocast_dtype(at::kCUDA)) : t;
+}
+
+// ---- one layer ----------------------------------------------------------------------------------------------------------
+struct LinearBackward : Node {
+  SavedVariable x, w;
+  Lists lists;
+  double p = 0;
+  variable_list apply(variable_list&& grads) override {
+    at::NoGradGuard no_grad;
+    variable_list out(2);
+    if (!grads[0].defined()) return out;
+    const Tensor xs = x.unpack(), ws = w.unpack();
+    const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
+    std::tie(out[0], out[1]) = layer_backward(grad_matrix(grads[0], xs), ws, xs, lists, p, need_dx, need_dw,
+                                              SD_ACT_NONE, Tensor());
+    return out;
+  }
+  void release_variables() override {
+    x.reset_data();
+    w.reset_data();
+    lists = Lists();
+  }
+  std::string name() const override { return "BlockwiseDropoutMatmulHIPBackward"; }
+};
+
+template <typename B>
+std::shared_ptr<B> make_node(const variable_list& inputs) {
+  std::shared_ptr<B> node(new B(), torch::autograd::deleteNode);
+  node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+  return node;
+}
+
+Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, int64_t bs, double p,
+              std::optional<uint64_t> seed, const OptTensor& state) {
+  TORCH_CHECK_VALUE(input.dim() == 2 && weight.dim() == 2, "input must be [M, K] and weight [N, K]");
+  const Tensor x = as_matrix(autocast(input)), w = as_matrix(autocast(weight));
+  Lists lists;
+  Tensor y;
+  {
+    NoRecord guard;
+    y = layer_forward(x, w, bs, p, Draw{mask, seed, state}, SD_ACT_NONE, false, lists, nullptr);
+  }
+  if (records(std::array<Tensor, 2>{x, w})) {
+    auto node = make_node<LinearBackward>({x, w});
+    node->x = SavedVariable(x, false);
+    node->w = SavedVariable(w, false);
+    node->lists = std::move(lists);
+    node->p = p;
+    torch::autograd::set_history(y, node);
+  }
+  return y;
+}
+
+// ---- a stack of layers with an activation between consecutive ones -------------------------------------------------------
+// (see functional/blockwise_dropout_mlp_hip.py for what is computed)
+struct MlpBackward : Node {
+  SavedVariable x;
+  std::vector<SavedVariable> ws;
+  std::vector<Tensor> hidden, pre;  // activated outputs of all layers but the last; GELU: their pre-activations
+  std::vector<Lists> lists;         // undefined buffer: the layer ran dense
+  std::vector<double> ps;
+  int act = SD_ACT_NONE;
+  variable_list apply(variable_list&& grads) override {
+    at::NoGradGuard no_grad;
+    const int n = (int)ws.size();
+    variable_list out(1 + n);
+    if (!grads[0].defined()) return out;
+    const Tensor x0 = x.unpack();
+    Tensor g = grad_matrix(grads[0], x0);
+    for (int i = n - 1; i >= 0; --i) {
+      const Tensor w = ws[i].unpack();
+      const Tensor& h = i ? hidden[i - 1] : x0;
+      const bool need_w = task_should_compute_output(1 + i), need_in = i > 0 || task_should_compute_output(0);
+      if (!lists[i].buf.defined()) {  // the dense first layer: only its weight gradient is wanted, dW = g^T . h
+        if (need_w) {
+          const int64_t N = w.size(0), n8 = ceil_div(N, 8) * 8;
+          Tensor gp = g;
+          if (N % 8) {  // the kernels take gradients whose width is a multiple of 8: zero columns up to the next one
+            gp = at::zeros({g.size(0), n8}, g.options());
+            gp.narrow(1, 0, N).copy_(g);
+          }
+          const Tensor dw = dense(gp.t(), h.t(), SD_ACT_NONE, false, nullptr);
+          out[1 + i] = N % 8 ? dw.narrow(0, 0, N) : dw;
+        }
+        break;
+      }
+      Tensor at;
+      if (i > 0 && need_in && act != SD_ACT_NONE) at = act == SD_ACT_GELU ? pre[i - 1] : h;
+      // both gradients of the layer in one library call, the activation's derivative riding on the dX store
+      auto [dx, dw] = layer_backward(g, w, h, lists[i], ps[i], need_in, need_w, at.defined() ? act : SD_ACT_NONE, at);
+      out[1 + i] = dw;
+      if (!need_in) break;
+      g = dx;
+      if (i == 0) out[0] = dx;
+    }
+    return out;
+  }
+  void release_variables() override {
+    x.reset_data();
+    for (auto& w : ws) w.reset_data();
+    hidden.clear();
+    pre.clear();
+    for (auto& l : lists) l.buf.reset(), l.given.reset();
+  }
+  std::string name() const override { return "BlockwiseDropoutMLPHIPBackward"; }
+};
+
+Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, const std::vector<double>& ps, int act,
+           const std::optional<std::vector<Tensor>>& masks, std::optional<uint64_t> seed, const OptTensor& state) {
+  const int n = (int)weights.size();
+  bool two_d = input.dim() == 2;
+  for (const Tensor& w : weights) two_d = two_d && w.dim() == 2;
+  TORCH_CHECK_VALUE(two_d, "input must be [M, K] and every weight [out, in]");
+  const Tensor x = as_matrix(autocast(input));
+  std::vector<Tensor> ws;
+  ws.reserve(n);
+  for (const Tensor& w : weights) ws.push_back(as_matrix(autocast(w)));
+  variable_list inputs{x};
+  inputs.insert(inputs.end(), ws.begin(), ws.end());
+  const bool rec = records(inputs);
+  const bool x_grad = rec && x.requires_grad();
+  std::vector<Lists> lists(n);
+  std::vector<Tensor> hidden, pres;
+  Tensor h = x;
+  {
+    NoRecord guard;
+    for (int i = 0; i < n; ++i) {
+      const bool last = i + 1 == n;
+      const int a = last ? SD_ACT_NONE : act;
+      const bool want_pre = a == SD_ACT_GELU && rec;
+      Tensor pre, out;
+      if (i == 0 && ps[0] == 0.0 && !masks && !x_grad) {
+        // a first layer without dropout whose input needs no gradient (the reference's models start with one,
+        // eval/mlp/model.py:31-33): the dense product with the same fused store, no mask and no lists
+        out = dense(h, ws[0], a, want_pre, &pre);
+      } else {
+        Draw draw{masks ? OptTensor((*masks)[i]) : OptTensor(),
+                  seed ? std::optional<uint64_t>(*seed + (uint64_t)i) : std::nullopt, state};
+        out = layer_forward(h, ws[i], bs, ps[i], draw, a, want_pre, lists[i], &pre);
+      }
+      if (!last) {
+        hidden.push_back(out);
+        pres.push_back(pre);
+      }
+      h = out;
+    }
+  }
+  if (rec) {
+    auto node = make_node<MlpBackward>(inputs);
+    node->x = SavedVariable(x, false);
+    for (const Tensor& w : ws) node->ws.emplace_back(w, false);
+    node->hidden = std::move(hidden);
+    node->pre = std::move(pres);
+    node->lists = std::move(lists);
+    node->ps = ps;
+    node->act = act;
+    torch::autograd::set_history(h, node);
+  }
+  return h;
+}
+
+// ---- convolution --------------------------------------------------------------------------------------------------------
+// (see functional/im2col_conv2d.py for what is computed)
+// Which route each product of the process's last convolution took; 0 = not computed.
+enum Route { kNone = 0, kImplicit = 1, kFused = 2, kExplicit = 3 };
+std::atomic<int> last_routes[3];  // forward, dx, dw
+
+struct ConvGeom {
+  int64_t n, c, h, w, k, r, s, pad[2], stride[2], dil[2], po, qo;
+  int64_t rows() const { return n * po * qo; }
+  int64_t cols() const { return c * r * s; }
+};
+#define GEOM_X(g) (g).n, (g).c, (g).h, (g).w
+#define GEOM_W(g) (g).pad[0], (g).pad[1], (g).stride[0], (g).stride[1], (g).dil[0], (g).dil[1]
+#define STRIDES4(t) (t).stride(0), (t).stride(1), (t).stride(2), (t).stride(3)
+
+void conv_lists(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
+  check_p(p);
+  l.shape(g.rows(), g.cols(), bs);
+  if (draw.mask)
+    TORCH_CHECK_VALUE(draw.mask->dim() == 2 && draw.mask->size(0) == l.mb && draw.mask->size(1) == l.kb, "mask shape ",
+                      draw.mask->sizes(), " != [", l.mb, ", ", l.kb, "] for a [", g.rows(), ", ", g.cols(),
+                      "] matrix in blocks of ", bs);
+  l.allocate(x, draw.mask);
+  const int64_t split = bs / 64;
+  c10::DeviceGuard guard(x.device());
+  if (draw.mask) {
+    const MaskArg m = l.mask();
+    check(sd_build_lists_split(m.ptr, l.mb, l.kb, m.sr, m.sc, split, l.out_mb, l.out_kb, l.row_ptr(), l.col_idx(),
+                               l.col_ptr(), l.row_idx(), stream_of(x)),
+          "sd_build_lists_split");
+  } else if (uint64_t* st = draw.state_ptr()) {
+    check(sd_random_lists_state(st, (float)p, l.mb, l.kb, l.drawn(), split, l.out_mb, l.out_kb, l.row_ptr(),
+                                l.col_idx(), l.col_ptr(), l.row_idx(), stream_of(x)),
+          "sd_random_lists_state");
+  } else {
+    check(sd_random_lists(draw.seed.value_or(0), 0, (float)p, l.mb, l.kb, l.drawn(), split, l.out_mb, l.out_kb,
+                          l.row_ptr(), l.col_idx(), l.col_ptr(), l.row_idx(), stream_of(x)),
+          "sd_random_lists");
+  }
+}
+
+Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
+  Tensor cols = new_matrix(x, g.rows(), g.cols());
+  c10::DeviceGuard guard(x.device());
+  check(sd_im2col(x.data_ptr(), STRIDES4(x), cols.data_ptr(), cols.stride(0), GEOM_X(g), g.r, g.s, GEOM_W(g),
+                  l ? l->row_ptr() : nullptr, l ? l->col_idx() : nullptr, l ? l->kernel_bs : 0, dtype_of(x),
+                  stream_of(x)),
+        "sd_im2col");
+  return cols;
+}
+
+Tensor conv_dw(const Tensor& x, const Tensor& dy2, const ConvGeom& g, const Lists* l, float scale) {
+  Tensor dw = new_matrix(x, g.k, g.cols());
+  Scratch ws(x, sd_conv2d_dw_workspace_bytes(g.n, g.c, g.k, g.r, g.s, g.po, g.qo));
+  c10::DeviceGuard guard(x.device());
+  const int rc = sd_conv2d_dw_lists(x.data_ptr(), STRIDES4(x), dy2.data_ptr(), dy2.stride(0), dw.data_ptr(),
+                                    dw.stride(0), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), l ? l->col_ptr() : nullptr,
+                                    l ? l->row_idx() : nullptr, l ? l->kernel_bs : 0, scale, dtype_of(x), ws.ptr,
+                                    ws.bytes, stream_of(x));
+  if (rc == SD_ERR_UNSUPPORTED) return Tensor();  // geometry not taken: nothing was launched
+  check(rc, "sd_conv2d_dw_lists");
+  return dw;
+}
+
+Tensor new_image(const Tensor& like, const ConvGeom& g, bool channels_last) {
+  return at::empty({g.n, g.c, g.h, g.w}, like.options().memory_format(channels_last ? at::MemoryFormat::ChannelsLast
+                                                                                     : at::MemoryFormat::Contiguous));
+}
+
+// The mask on the 64 grid the fused input gradient works on: every entry of a larger block size repeated.
+Tensor mask_on_64_grid(const Tensor& like, const Lists& l) {
+  Tensor m = l.given.defined() ? l.given
+                               : at::from_blob(l.drawn(), {l.mb, l.kb}, like.options().dtype(at::kBool));
+  const int64_t f = l.bs / 64;
+  if (f == 1) return m;
+  m = m.repeat_interleave(f, 0).repeat_interleave(f, 1);
+  return m.narrow(0, 0, l.out_mb).narrow(1, 0, l.out_kb).contiguous();
+}
+
+Tensor conv_dx(const Tensor& dy2, const Tensor& w2, const ConvGeom& g, const Lists* l, float scale, bool channels_last) {
+  Tensor m64;
+  MaskArg m;
+  if (l) {
+    m64 = mask_on_64_grid(dy2, *l);
+    m = MaskArg(m64);
+  }
+  Tensor dx = new_image(dy2, g, channels_last);
+  c10::DeviceGuard guard(dy2.device());
+  const int rc = sd_conv2d_dx(dy2.data_ptr(), dy2.stride(0), w2.data_ptr(), w2.stride(0), dx.data_ptr(), STRIDES4(dx),
+                              m.ptr, m.sr, m.sc, GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), 64, scale, dtype_of(dy2),
+                              stream_of(dy2));
+  if (rc == SD_ERR_UNSUPPORTED) return Tensor();
+  check(rc, "sd_conv2d_dx");
+  return dx;
+}
+
+// (N, K, P, Q) gradient -> [N*P*Q, K] row-major (free when it is channels-last in memory)
+Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) {
+  Tensor d = grad.scalar_type() == like.scalar_type() ? grad : grad.to(like.scalar_type());
+  d = d.permute({0, 2, 3, 1}).reshape({g.rows(), g.k});
+  if (d.stride(1) != 1 || d.stride(0) < g.k) d = d.contiguous();  // e.g. the expanded (stride 0) gradient of a sum()
+  return d;
+}
+
+struct ConvBackward : Node {
+  SavedVariable x, w2;  // w2: the kernel as [K, C*R*S]
+  Tensor cols;          // the patch matrix, when the forward made one
+  Lists lists;          // undefined buffer: no dropout
+  ConvGeom g{};
+  double p = 0;
+  bool fused_dx = true, channels_last = false;
+  variable_list apply(variable_list&& grads) override {
+    at::NoGradGuard no_grad;
+    variable_list out(2);
+    if (!grads[0].defined()) return out;
+    const Tensor w = w2.unpack(), image = x.unpack();
+    Tensor patches = cols;
+    const Tensor dy2 = rows_gradient(grads[0], g, w);
+    const Lists* l = lists.buf.defined() ? &lists : nullptr;
+    const float scale = (float)(1.0 / (1.0 - p));
+    if (task_should_compute_output(0)) {
+      Tensor dx;
+      if (fused_dx) dx = conv_dx(dy2, w, g, l, scale, channels_last);
+      last_routes[1] = dx.defined() ? kFused : kExplicit;
+      if (!dx.defined()) {
+        Tensor dcols = new_matrix(dy2, g.rows(), g.cols());
+        dx = new_image(dy2, g, channels_last);
+        const Mat gm(dy2), dm(dcols);
+        const Mat wt(w.t());
+        c10::DeviceGuard guard(dy2.device());
+        MaskArg m;
+        if (l) {
+          // col2im skips the dropped blocks, so the product need not zero them
+          check(sd_gemm_sdd_lists_ex(MAT(gm), MAT(wt), MAT(dm), l->row_ptr(), l->col_idx(), g.rows(), g.cols(), g.k,
+                                     l->kernel_bs, scale, dtype_of(dy2), 1, 1.f / scale, stream_of(dy2)),
+                "sd_gemm_sdd_lists_ex");
+          m = l->mask();
+        } else {
+          Scratch ws(dy2, sd_splitk_workspace_bytes(g.rows(), g.cols(), g.k, 0, 0));
+          check(sd_gemm(MAT(gm), MAT(wt), MAT(dm), g.rows(), g.cols(), g.k, dtype_of(dy2), ws.ptr, ws.bytes,
+                        stream_of(dy2)),
+                "sd_gemm");
+        }
+        check(sd_col2im(dcols.data_ptr(), dcols.stride(0), dx.data_ptr(), STRIDES4(dx), GEOM_X(g), g.r, g.s, GEOM_W(g),
+                        m.ptr, m.sr, m.sc, l ? l->bs : 0, dtype_of(dy2), stream_of(dy2)),
+              "sd_col2im");
+      }
+      out[0] = dx;
+    }
+    if (task_should_compute_output(1)) {
+      Tensor dk;
+      if (!patches.defined()) {  // the forward kept the input, not the patch matrix
+        dk = conv_dw(image, dy2, g, l, scale);
+        if (!dk.defined()) patches = im2col(image, g, l);
+      }
+      last_routes[2] = dk.defined() ? kImplicit : kExplicit;
+      if (!dk.defined()) {
+        dk = new_matrix(dy2, g.k, g.cols());
+        const Mat am(patches.t()), bm(dy2.t()), cm(dk.t());
+        c10::DeviceGuard guard(dy2.device());
+        if (l) {
+          Scratch ws(dy2, sd_splitk_workspace_bytes(g.cols(), g.k, g.rows(), l->kernel_bs, 1));
+          check(sd_gemm_dsd_lists(MAT(am), MAT(bm), MAT(cm), l->col_ptr(), l->row_idx(), g.cols(), g.k, g.rows(),
+                                  l->kernel_bs, scale, dtype_of(dy2), ws.ptr, ws.bytes, stream_of(dy2)),
+                "sd_gemm_dsd_lists");
+        } else {
+          Scratch ws(dy2, sd_splitk_workspace_bytes(g.cols(), g.k, g.rows(), 0, 0));
+          check(sd_gemm(MAT(am), MAT(bm), MAT(cm), g.cols(), g.k, g.rows(), dtype_of(dy2), ws.ptr, ws.bytes,
+                        stream_of(dy2)),
+                "sd_gemm");
+        }
+      }
+      out[1] = dk.view({g.k, g.c, g.r, g.s});
+    }
+    return out;
+  }
+  void release_variables() override {
+    x.reset_data();
+    w2.reset_data();
+    cols.reset();
+    lists = Lists();
+  }
+  std::string name() const override { return "Im2colConv2dBackward"; }
+};
+
+using Pair = std::array<int64_t, 2>;
+
+// block size 0: no dropout
+Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mask, int64_t bs, double p,
+              const Pair& padding, const Pair& stride, const Pair& dilation, std::optional<uint64_t> seed,
+              const OptTensor& state, bool implicit_forward, bool fused_dx) {
+  TORCH_CHECK_VALUE(input.dim() == 4 && kernel_in.dim() == 4, "input must be (N, C, H, W) and kernel (K, C, R, S)");
+  TORCH_CHECK_VALUE(input.size(1) == kernel_in.size(1), "channel mismatch: input ", input.size(1), ", kernel ",
+                    kernel_in.size(1));
+  const Tensor x = autocast(input), kernel = autocast(kernel_in).contiguous();
+  TORCH_CHECK_VALUE(x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16),
+                    "x must be a 4D float16/bfloat16 tensor on the GPU");
+  TORCH_CHECK_VALUE(kernel.scalar_type() == x.scalar_type() && kernel.device() == x.device(), "kernel must be a ",
+                    x.dtype(), " tensor on ", x.device());
+  ConvGeom g{x.size(0), x.size(1), x.size(2), x.size(3), kernel.size(0), kernel.size(2), kernel.size(3)};
+  for (int i = 0; i < 2; ++i) {
+    g.pad[i] = padding[i];
+    g.stride[i] = stride[i];
+    g.dil[i] = dilation[i];
+  }
+  auto out_size = [](int64_t in, int64_t pad, int64_t dil, int64_t taps, int64_t step) {
+    const int64_t room = in + 2 * pad - dil * (taps - 1) - 1;
+    return room < 0 ? 0 : room / step + 1;
+  };
+  g.po = out_size(g.h, g.pad[0], g.dil[0], g.r, g.stride[0]);
+  g.qo = out_size(g.w, g.pad[1], g.dil[1], g.s, g.stride[1]);
+  TORCH_CHECK_VALUE(g.po > 0 && g.qo > 0, "kernel does not fit the padded image");
+  Lists lists;
+  Tensor y, y2, cols;
+  const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;
+  {
+    NoRecord guard;
+    if (bs) conv_lists(x, g, bs, p, Draw{mask, seed, state}, lists);
+    const Lists* l = bs ? &lists : nullptr;
+    y2 = new_matrix(x, g.rows(), g.k);
+    bool done = false;
+    c10::DeviceGuard device(x.device());
+    if (implicit_forward) {  // no patch matrix in memory where the library takes the geometry
+      const int rc = sd_conv2d_dsd_lists(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(), y2.data_ptr(),
+                                         y2.stride(0), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), l ? l->row_ptr() : nullptr,
+                                         l ? l->col_idx() : nullptr, l ? l->kernel_bs : 0, scale, dtype_of(x),
+                                         stream_of(x));
+      if (rc != SD_ERR_UNSUPPORTED) check(rc, "sd_conv2d_dsd_lists");
+      done = rc == SD_OK;
+    }
+    last_routes[0] = done ? kImplicit : kExplicit;
+    last_routes[1] = last_routes[2] = kNone;
+    if (!done) {
+      cols = im2col(x, g, l);
+      Mat am(cols), bm, cm(y2);
+      bm.ptr = kernel.data_ptr();
+      bm.sr = std::max<int64_t>(g.cols(), 1);
+      bm.sc = 1;
+      Scratch ws(x, sd_splitk_workspace_bytes(g.rows(), g.k, g.cols(), l ? l->kernel_bs : 0, l ? 1 : 0));
+      if (l)
+        check(sd_gemm_dsd_lists(MAT(am), MAT(bm), MAT(cm), l->row_ptr(), l->col_idx(), g.rows(), g.k, g.cols(),
+                                l->kernel_bs, scale, dtype_of(x), ws.ptr, ws.bytes, stream_of(x)),
+              "sd_gemm_dsd_lists");
+      else
+        check(sd_gemm(MAT(am), MAT(bm), MAT(cm), g.rows(), g.k, g.cols(), dtype_of(x), ws.ptr, ws.bytes, stream_of(x)),
+              "sd_gemm");
+    }
+    // the result is an (N, K, P, Q) view of an (N, P*Q, K) buffer, as the reference's is (im2col_conv2d.py:26-27)
+    y = y2.view({g.n, g.po, g.qo, g.k}).permute({0, 3, 1, 2});
+  }
+  if (records(std::array<Tensor, 2>{x, kernel})) {
+    auto node = make_node<ConvBackward>({x, kernel});
+    node->x = SavedVariable(x, false);
+    node->w2 = SavedVariable(kernel.detach().view({g.k, g.cols()}), false);
+    node->cols = cols;
+    node->lists = std::move(lists);
+    node->g = g;
+    node->p = bs ? p : 0.0;
+    node->fused_dx = fused_dx;
+    node->channels_last = x.is_contiguous(at::MemoryFormat::ChannelsLast) && !x.is_contiguous();
+    torch::autograd::set_history(y, node);
+  }
+  return y;
+}
+
+std::array<int, 3> conv_routes() { return {last_routes[0].load(), last_routes[1].load(), last_routes[2].load()}; }
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  namespace py = pybind11;
+  m.def("source_hash", [] { return SD_SOURCE_HASH; });
+  m.def("set_library_error", [](py::object cls) { library_error = cls.release().ptr(); });
+  m.def("linear", torch::wrap_pybind_function(linear));
+  m.def("mlp", torch::wrap_pybind_function(mlp));
+  m.def("conv2d", torch::wrap_pybind_function(conv2d));
+  m.def("conv_routes", &conv_routes);
+}

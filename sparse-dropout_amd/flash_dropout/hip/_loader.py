@@ -13,6 +13,7 @@ from functools import lru_cache
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent.parent / "_lib" / "libsparsedrop.so"
+BRIDGE_PATH = LIB_PATH.with_name("sparsedrop_torch.so")
 
 _mat = [c_void_p, c_int64, c_int64]  # ptr, stride_r, stride_c
 
@@ -100,7 +101,7 @@ def source_hash() -> str | None:
     hips = sorted(csrc.glob("*.hip"))
     if not hips:
         return None
-    files = [*hips, *sorted(csrc.glob("*.h")), *sorted(include.glob("*.h"))]
+    files = [*hips, *sorted(csrc.glob("*.cpp")), *sorted(csrc.glob("*.h")), *sorted(include.glob("*.h"))]
     h = hashlib.sha256()
     for f in files:
         h.update(f.name.encode())
@@ -127,3 +128,27 @@ def load() -> ctypes.CDLL:
             "`python sparse-dropout_amd/csrc/build.py`"
         )
     return lib
+
+
+@lru_cache(maxsize=None)
+def bridge():
+    """The extension module sparsedrop_torch.so (csrc/torch_bridge.cpp): the autograd functions in native code, on the
+    same libsparsedrop.so that :func:`load` returns."""
+    load()
+    if not BRIDGE_PATH.exists():
+        raise RuntimeError(f"{BRIDGE_PATH} not found: build it with `python sparse-dropout_amd/csrc/build.py`")
+    import importlib.util
+
+    import torch  # noqa: F401  (the module's libtorch symbols)
+
+    spec = importlib.util.spec_from_file_location("sparsedrop_torch", BRIDGE_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    built, now = mod.source_hash(), source_hash()
+    if now is not None and built != now:
+        raise RuntimeError(f"{BRIDGE_PATH} was built from other sources ({built}, tree {now}): rebuild it with "
+                           "`python sparse-dropout_amd/csrc/build.py`")
+    from .binding_gemm import SparseDropError
+
+    mod.set_library_error(SparseDropError)
+    return mod
