@@ -160,15 +160,15 @@ __device__ inline uint32_t entry_quads(int32_t e) {
 // ---- fused epilogues --------------------------------------------------------------------------
 // GELU is the exact (erf) form, torch.nn.GELU's default: gelu(x) = x * Phi(x), gelu'(x) = Phi(x) + x * phi(x).
 // Phi comes from the rational approximation of erf in Abramowitz & Stegun 7.1.26 (absolute error below 1.5e-7, far
-// under the resolution of the fp16 / bf16 results): one exponential, one reciprocal and a degree-5 polynomial, a
-// third of the instructions of erff, which matters because the epilogue of a GEMM has nothing to hide them behind.
+// under the resolution of the fp16 / bf16 results): one exponential, one reciprocal and a degree-5 polynomial, with the
+// factors 1/sqrt(2), log2(e)/2 and 1/2 folded into the constants.  In a store that applies it to 25 M elements the
+// vector instructions are what costs (a wave64 instruction takes 4 clocks, a transcendental one 16).
 // *pdf receives exp(-x^2 / 2), which the derivative needs as well.
 __device__ inline float normal_cdf(float x, float* pdf) {
-  const float z = fabsf(x) * 0.70710678118654752f;
-  const float e = __expf(-z * z);
-  const float t = __builtin_amdgcn_rcpf(1.f + 0.3275911f * z);
-  const float poly = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-  const float tail = 0.5f * poly * e;  // Phi(-|x|)
+  const float e = __builtin_amdgcn_exp2f((x * -0.72134752044448170f) * x);
+  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.23164189f, fabsf(x), 1.f));
+  const float poly = t * (0.127414796f + t * (-0.142248368f + t * (0.7107068705f + t * (-0.7265760135f + t * 0.5307027145f))));
+  const float tail = poly * e;  // Phi(-|x|)
   *pdf = e;
   return x >= 0.f ? 1.f - tail : tail;
 }
@@ -204,73 +204,106 @@ __device__ inline void store_result(const GemmArgs& g, int64_t m, int64_t n, flo
   g.c[m * g.c_sr + n * g.c_sc] = T::from_float(v);
 }
 
+// 16 bytes at any 2-byte boundary (one instruction on global memory whatever the alignment)
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+
+// What storing along C's contiguous index needs to know, worked out once.  along_n: that index is n (row-major C).
+struct StoreLayout {
+  bool along_n, unit, has_aux, aux_unit;
+  int64_t s_ext, c_ext, ld, ald;
+  __device__ inline StoreLayout(const GemmArgs& g, bool along_n_) : along_n(along_n_) {
+    s_ext = along_n ? g.M : g.N;
+    c_ext = along_n ? g.N : g.M;
+    ld = along_n ? g.c_sr : g.c_sc;
+    unit = (along_n ? g.c_sc : g.c_sr) == 1;
+    has_aux = g.act != SD_ACT_NONE && g.aux != nullptr;
+    ald = along_n ? g.aux_sr : g.aux_sc;
+    aux_unit = (along_n ? g.aux_sc : g.aux_sr) == 1;
+  }
+};
+
+// Eight consecutive elements of C's contiguous index, unscaled fp32 accumulators: scaled, put through the fused
+// epilogue, rounded once and stored in one 16-byte piece (element by element at the matrix's edge).  si / ci: position
+// along C's strided / contiguous index (ci a multiple of 8).  part: fp32 partial sums of a split reduction go to `part`
+// (C's element order, unscaled) instead.
+template <typename T, bool SDD>
+__device__ inline void store_eight(const GemmArgs& g, const StoreLayout& s, int64_t si, int64_t ci, float (&r)[8], float* part) {
+  if (si >= s.s_ext || ci >= s.c_ext) return;
+  const int valid = s.c_ext - ci < 8 ? (int)(s.c_ext - ci) : 8;
+  if (part) {
+    float* dst = part + si * s.c_ext + ci;
+    if (valid == 8 && s.c_ext % 4 == 0) {
+      *reinterpret_cast<f32x4*>(dst) = f32x4{r[0], r[1], r[2], r[3]};
+      *reinterpret_cast<f32x4*>(dst + 4) = f32x4{r[4], r[5], r[6], r[7]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < valid) dst[i] = r[i];
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] *= g.scale;
+  if (!(s.unit && valid == 8 && (!s.has_aux || s.aux_unit))) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < valid) store_result<T, SDD>(g, s.along_n ? si : ci + i, s.along_n ? ci + i : si, r[i]);
+    return;
+  }
+  auto pack = [&](const float (&v)[8]) {
+    return u32x4{(uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16),
+                 (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16),
+                 (uint32_t)T::from_float(v[4]) | ((uint32_t)T::from_float(v[5]) << 16),
+                 (uint32_t)T::from_float(v[6]) | ((uint32_t)T::from_float(v[7]) << 16)};
+  };
+  if (g.act != SD_ACT_NONE) {
+    if (SDD) {
+      const u32x4 a = *reinterpret_cast<const u32x4_any*>(g.aux + si * s.ald + ci);
+      const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint16_t h = (uint16_t)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu);
+        if (r[i] != 0.f) r[i] *= act_derivative(g.act, T::to_float(h));  // dropped tiles stay exact zeros
+      }
+    } else {
+      if (s.has_aux) *reinterpret_cast<u32x4_any*>(g.aux + si * s.ald + ci) = pack(r);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r[i] = act_apply(g.act, r[i]);
+    }
+  }
+  *reinterpret_cast<u32x4_any*>(g.c + si * s.ld + ci) = pack(r);
+}
+
 // One wave's [ROWS][COLS] tile of unscaled fp32 accumulators, staged in the wave's own LDS region (pitch COLS + 4
-// floats) with COLS running along C's contiguous index, goes out in full 16-byte pieces: a lane takes 8 consecutive
-// elements of one row, scales them, applies the fused epilogue, rounds once and stores them (128-byte lines are
-// written whole by 8 neighbouring lanes).  s0 / c0: where the tile starts along C's strided / contiguous index
-// (c0 a multiple of 8); along_n: the contiguous index is n (row-major C).  part: fp32 partial sums of a split
-// reduction go to `part` (C's element order, unscaled) instead.
+// floats) with COLS running along C's contiguous index: a lane takes 8 consecutive elements of one row (128-byte lines
+// are written whole by 8 neighbouring lanes).  s0 / c0: where the tile starts along C's strided / contiguous index.
 template <typename T, bool SDD, int ROWS, int COLS>
 __device__ inline void store_staged_tile(const GemmArgs& g, const float* stg, int lane, bool along_n, int64_t s0,
                                          int64_t c0, float* part) {
   constexpr int PITCH = COLS + 4, LPR = COLS / 8, RPP = 64 / LPR;  // lanes per row, rows per pass
-  const int64_t s_ext = along_n ? g.M : g.N, c_ext = along_n ? g.N : g.M;
-  const int64_t ld = along_n ? g.c_sr : g.c_sc, unit = along_n ? g.c_sc : g.c_sr;
-  bool vec = unit == 1 && ld % 8 == 0 && reinterpret_cast<uintptr_t>(g.c) % 16 == 0;
-  const bool has_aux = g.act != SD_ACT_NONE && g.aux != nullptr;
-  const int64_t ald = along_n ? g.aux_sr : g.aux_sc, aunit = along_n ? g.aux_sc : g.aux_sr;
-  if (has_aux) vec = vec && aunit == 1 && ald % 8 == 0 && reinterpret_cast<uintptr_t>(g.aux) % 16 == 0;
+  const StoreLayout s(g, along_n);
 #pragma unroll
   for (int pass = 0; pass < ROWS / RPP; ++pass) {
     const int row = pass * RPP + lane / LPR, ch = lane % LPR;
-    const int64_t si = s0 + row, ci = c0 + ch * 8;
-    if (si >= s_ext || ci >= c_ext) continue;
     const f32x4 lo = *reinterpret_cast<const f32x4*>(stg + row * PITCH + ch * 8);
     const f32x4 hi = *reinterpret_cast<const f32x4*>(stg + row * PITCH + ch * 8 + 4);
     float r[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    const int valid = c_ext - ci < 8 ? (int)(c_ext - ci) : 8;
-    if (part) {
-      float* dst = part + si * c_ext + ci;
-      if (valid == 8 && c_ext % 4 == 0) {
-        *reinterpret_cast<f32x4*>(dst) = lo;
-        *reinterpret_cast<f32x4*>(dst + 4) = hi;
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (i < valid) dst[i] = r[i];
-      }
-      continue;
+    store_eight<T, SDD>(g, s, s0 + row, c0 + ch * 8, r, part);
+  }
+}
+
+// Zeros over the 64 x 64 tile of a row-major C at (m0, n0), by a whole workgroup.
+template <int THREADS>
+__device__ inline void zero_tile(const GemmArgs& g, int64_t m0, int64_t n0) {
+  for (int i = threadIdx.x; i < 512; i += THREADS) {
+    const int64_t m = m0 + i / 8, n = n0 + i % 8 * 8;
+    if (m >= g.M || n >= g.N) continue;
+    uint16_t* p = g.c + m * g.c_sr + n;
+    if (g.N - n >= 8) {
+      *reinterpret_cast<u32x4_any*>(p) = u32x4{0u, 0u, 0u, 0u};
+    } else {
+      for (int64_t k = 0; k < g.N - n; ++k) p[k] = 0;
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] *= g.scale;
-    if (!(vec && valid == 8)) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < valid) store_result<T, SDD>(g, along_n ? si : ci + i, along_n ? ci + i : si, r[i]);
-      continue;
-    }
-    auto pack = [&](const float (&v)[8]) {
-      return u32x4{(uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16),
-                   (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16),
-                   (uint32_t)T::from_float(v[4]) | ((uint32_t)T::from_float(v[5]) << 16),
-                   (uint32_t)T::from_float(v[6]) | ((uint32_t)T::from_float(v[7]) << 16)};
-    };
-    if (g.act != SD_ACT_NONE) {
-      if (SDD) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(g.aux + si * ald + ci);
-        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint16_t h = (uint16_t)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu);
-          if (r[i] != 0.f) r[i] *= act_derivative(g.act, T::to_float(h));  // dropped tiles stay exact zeros
-        }
-      } else {
-        if (has_aux) *reinterpret_cast<u32x4*>(g.aux + si * ald + ci) = pack(r);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = act_apply(g.act, r[i]);
-      }
-    }
-    *reinterpret_cast<u32x4*>(g.c + si * ld + ci) = pack(r);
   }
 }
 

@@ -18,7 +18,7 @@
 //    barrier per phase; see "the step loop of the 256 x 256 shape" in dsd_body.  A wave that stands at a load or a
 //    fragment read (the texture path takes a 1 KB load every 25 clocks or so) issues no MFMA behind it, so with both
 //    waves of a SIMD in the same phase the parts of a step add up instead of overlapping.
-//  * ragged operands, masks of block size 32 and the 128 x 128 shape: one barrier per step, in front of the MFMAs of
+//  * ragged operands: one barrier per step, in front of the MFMAs of
 //    the step's last (row block, half of the K block) unit, when every fragment of the current stage is in
 //    registers; the loads of the step after next and the fragment reads of the next step's first unit are issued
 //    behind it and run under those MFMAs.
@@ -50,6 +50,8 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_device.h"
+#include "gemm_tile_api.h"
 #include "mask_source.h"
 #include "tile_map.h"
 
@@ -57,29 +59,19 @@ namespace sd {
 namespace {
 
 constexpr int R = 4;          // row blocks per workgroup
-constexpr int BS = 64;        // mask block = tile edge along M and K
 constexpr int BN = 256;       // output columns per workgroup
 constexpr int THREADS = 512;  // 8 waves
-constexpr int TILE = BS * BS * 2;              // bytes of one 64 x 64 tile (rows of 128 B)
 constexpr int MAX_STEPS = 1024;
-// step table: one uint32 per step of the union walk, reduction block | keep bits << 16 (four bits per row block
-// of the workgroup: which 32 x 32 quadrants of its tile are kept; all four unless the mask has block size 32),
-// followed by STEP_PAD zero entries so that look-ahead reads past the end are harmless
-constexpr int STEP_PAD = 4;
 // Shape of a DSD workgroup: RH groups of RW row blocks x NS column slices of NT * 32 columns; wave
 // (rh, ns) multiplies its slice of the W tile with the kept X tiles of its RW row blocks.  Waves (rh, ns)
 // with equal ns share a SIMD, so a SIMD's MFMA work per step depends on how many row blocks keep the K
 // block, not on which.
-//   DsdBig  256 rows x 256 columns, 8 waves of 2 row blocks x 64 columns: the least operand traffic per
-//           MFMA; what large products run on
-//   DsdMid  128 rows x 128 columns, 8 waves of 1 row block x 32 columns: four times as many workgroups, for
-//           products whose 256 x 256 tiles would leave most of the 256 CUs without one; two workgroups fit
-//           a CU (72 KB of LDS, under 128 VGPRs).  More LDS fragment traffic per MFMA (1.5 KB against
-//           0.75 KB), which is why the big shape wins as soon as it can fill the chip
-template <int RH_, int NS_, int NT_, int RW_ = 2, int NST_ = 2>
+//   DsdBig   256 rows x 256 columns, 8 waves of 2 row blocks x 64 columns: the least operand traffic per MFMA; what large
+//            products run on (smaller ones: gemm_tile.h)
+template <int RH_, int NS_, int NT_>
 struct DsdShape {
-  static constexpr int RH = RH_, NS = NS_, NT = NT_, RW = RW_;  // RW: row blocks a wave owns (2 or 1)
-  static constexpr int NST = NST_;           // stages of LDS (steps whose tiles are resident or on their way)
+  static constexpr int RH = RH_, NS = NS_, NT = NT_, RW = 2;  // RW: row blocks a wave owns
+  static constexpr int NST = 2;              // stages of LDS (steps whose tiles are resident or on their way)
   static constexpr int R = RW * RH;          // row blocks per workgroup
   static constexpr int NW = RH * NS;         // waves
   static constexpr int THREADS = 64 * NW;
@@ -94,84 +86,12 @@ struct DsdShape {
   static constexpr int SMEM_BYTES = SMEM_SCRATCH + 4 * MAX_STEPS + 16;
   static_assert(BL >= 1 && AL >= 1 && BL * NW * 1024 == B_TILE && AL * NW * 1024 == TILE, "loads must divide evenly");
 };
-using DsdBig = DsdShape<2, 4, 2>;  // (8 waves of 1 row block x 128 columns, DsdShape<4, 2, 4, 1>, measured 2-4 % slower)
-using DsdMid = DsdShape<2, 4, 1, 1>;
-// The same on aligned operands with four stages: a step of this shape is 16 MFMAs per wave, far shorter than a load's
-// way through L2 and memory, so three steps are kept in flight instead of one (one workgroup per CU: 136 KB of LDS)
-using DsdMidDeep = DsdShape<2, 4, 1, 1, 4>;
+using DsdBig = DsdShape<2, 4, 2>;  // (8 waves of 1 row block x 128 columns measured 2-4 % slower)
 // 256 rows x 128 columns, 8 waves: the shape of the implicit-GEMM convolution, whose input patch has to
 // fit in LDS next to the stages
 using DsdConv = DsdShape<2, 4, 1>;
 constexpr int CONV_PATCH_MAX = 163840 - DsdConv::SMEM_BYTES - 16;  // bytes left for patch + column table
 constexpr int CONV_T_PATCH_MAX = 24 * 1024;  // weight gradient: bytes of one step's copy of its input rows
-__device__ inline int step_block(uint32_t e) { return (int)(e & 0xffffu); }
-__device__ inline uint32_t step_flags(uint32_t e) { return e >> 16; }
-__device__ inline uint32_t row_quads(uint32_t flags, int r) { return (flags >> (4 * r)) & 0xfu; }  // of row block r
-__device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); }
-
-typedef __attribute__((address_space(3))) void lds_void;
-
-// One wave-wide 1 KB direct global->LDS load: lane i's 16 bytes land at lds_dst + 16*i (lds_dst is
-// wave-uniform and goes through M0).  Issued as inline assembly on purpose: when the compiler sees a
-// direct-to-LDS load in flight it stops counting LDS reads precisely (every wait becomes
-// lgkmcnt(0), and transpose reads get a vmcnt(0) in front), which serialises the fragment reads with
-// the MFMAs.  Written this way the loads are invisible to its counters; the kernels wait for them
-// themselves with s_waitcnt vmcnt(0) before the barrier that publishes a stage.
-// lds_dst is the destination's LDS byte address (lds_address() of a pointer, plus wave-uniform offsets): kept as
-// an integer in scalar registers, so no pointer conversion is made per load.
-__device__ inline uint32_t lds_address(const void* p) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_void*)p);
-}
-__device__ inline void load16_to_lds(const void* g, uint32_t lds_dst) {
-  const uint32_t a = uniform(lds_dst);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(a) : "memory");
-}
-// The same with the address split into a wave-uniform 64-bit base (SGPRs) and a 32-bit per-lane byte
-// offset: half the VGPR reads per load and no 64-bit VALU add to form the lane addresses.
-__device__ inline void load16_to_lds(const char* base, uint32_t lane_off, uint32_t lds_dst) {
-  const uint64_t b = (uint64_t)(uintptr_t)base;
-  const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
-                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t a = uniform(lds_dst);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(sb), "s"(a)
-               : "memory");
-}
-
-// Waits until at most n of the wave's loads are outstanding (they return in order: everything issued before the last
-// n has landed).  n is wave-uniform and only known at run time, the instruction takes an immediate.
-__device__ inline void wait_loads_all_but(int n) {
-  if (n >= 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-  else if (n == 11) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
-  else if (n == 10) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-  else if (n == 9) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
-  else if (n == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-  else if (n == 7) asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-  else if (n == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-  else if (n == 5) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-  else if (n == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-  else if (n == 3) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-  else if (n == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-  else if (n == 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-// 4 reduction-consecutive halfs of one column, gathered from 4 LDS rows (see the file comment)
-__device__ inline u32x2 lds_read_tr(const char* p) {
-  s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
-  return __builtin_bit_cast(u32x2, v);
-}
-
-// Chunk swizzles of tiles kept in memory order [reduction row][columns] (read with ds_read_b64_tr_b16).  One
-// transposing read takes, per 16-lane group, 4 consecutive reduction rows x 32 bytes, and the groups of a wave
-// are 8 reduction rows apart.  A 64-column tile has rows of 128 B: rows r and r+2 would share banks, so bit 2 of
-// the 16-byte chunk index follows bit 1 of the row; rows 8 apart would too, so bit 1 follows bit 3 of the row.
-// Rows of a 256- or 128-column tile are a multiple of 256 B apart: chunk bits 2-3 follow the row's low two bits.
-__device__ inline int swz_x(int row) { return (((row >> 1) & 1) << 2) ^ (((row >> 3) & 1) << 1); }
-__device__ inline int swz_w(int row) { return ((row & 3) << 2) ^ (((row >> 3) & 1) << 1); }
-
 // TRANS = false: A[row][red], B[col][red] with the reduction index contiguous (forward / dense)
 // TRANS = true : A and B are given as transposed views, the reduction index is the strided one (dW)
 // In both cases "Mb" counts the row blocks of A (of X^T for dW) and "Kb" the reduction blocks.
@@ -724,7 +644,7 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
   // clocks or more, so the loads are kept to one branch per group and six instructions each: the same loads issued
   // from a per-load choice between the groups' code (a few branches and a dozen scalar instructions more per load)
   // cost 20 % of the kernel; the same loads as buffer loads with a scalar offset (three instructions each) gain nothing.
-  constexpr bool PINGPONG = IMPLICIT == 0 && !RAGGED && RW == 2 && S::RH == 2 && S::NS == 4 && NT == 2;
+  constexpr bool PINGPONG = IMPLICIT == 0 && !RAGGED && S::RH == 2 && S::NS == 4 && NT == 2;
   if constexpr (PINGPONG) {
     const int rh_u = __builtin_amdgcn_readfirstlane(rh);
     const bool grp1 = rh_u != 0;
@@ -849,101 +769,6 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
         e2 = uniform(e3);
       }
     }
-  } else if constexpr (IMPLICIT == 0 && !RAGGED && S::NST > 2) {
-    // ---- the step loop of the 128 x 128 shape on aligned operands: three steps in flight ---------------------------
-    // A step here is 12 fragment reads and 16 MFMAs per wave; with one step in flight every step waits out a whole
-    // load latency (measured: 2200 clocks a step, whatever the drop rate).  So the tiles of steps s + 1 .. s + 3 are on
-    // their way while step s computes: four stages, one barrier per step (it publishes step s and frees the stage of
-    // step s - 1, into which the loads of step s + 3 go right behind it).  A wave waits for its own loads of step s
-    // only: loads return in order, so it allows as many outstanding as it issued for the two steps after - a number
-    // that depends on which X tiles those steps keep, hence the choice among waits below.
-    static_assert(RW == 1 && S::NST == 4, "one row block per wave, four stages");
-    constexpr int NST = S::NST;
-    const int rh_u = (int)uniform((uint32_t)rh);
-    const bool w_any = TRANS || wave_u * BL * 8 < nvalid;  // this wave's rows of the W tile are columns inside C
-    // (reduction-strided W tile: lanes whose columns lie past N fetch column 0 of their row instead - readable, and
-    // those columns are never stored)
-    uint32_t b_ld[BL];
-#pragma unroll
-    for (int jj = 0; jj < BL; ++jj) {
-      b_ld[jj] = b_lane[jj];
-      if constexpr (TRANS) {
-        constexpr int CPR = BN / 8;
-        const int row = (wave * BL + jj) * (64 / CPR) + lane / CPR;
-        if (!b_valid[jj]) b_ld[jj] = (uint32_t)(row * g.b.sc) * 2u;
-      }
-    }
-    auto loads_of = [&](uint32_t e) {  // load instructions this wave issues for a step
-      const uint32_t fl = step_flags(e);
-      int n = w_any ? BL : 0;
-#pragma unroll
-      for (int r = 0; r < R; ++r) n += row_quads(fl, r) ? AL : 0;
-      return n;
-    };
-    auto issue = [&](uint32_t e, int stage) {
-      const int kb = step_block(e);
-      const uint32_t fl = step_flags(e);
-      const uint32_t st_a = smem_a + (uint32_t)(stage * STAGE);
-      const char* bp = b_tile0 + kb * b_red_stride;
-      const char* ap = a_tile0 + kb * red_stride;
-      if (w_any) {
-#pragma unroll
-        for (int jj = 0; jj < BL; ++jj) load16_to_lds(bp, b_ld[jj], st_a + (uint32_t)((wave_u * BL + jj) * 1024));
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (row_quads(fl, r)) {
-#pragma unroll
-          for (int i = 0; i < AL; ++i)
-            load16_to_lds(ap + r * a_rstride, a_lane[i], st_a + (uint32_t)(A_OFF + r * TILE + (wave_u * AL + i) * 1024));
-        }
-    };
-    if (nsteps > 0) {
-      uint32_t e0 = uniform(step_e[0]), e1 = uniform(step_e[1]), e2 = uniform(step_e[2]), e3 = uniform(step_e[3]);
-      issue(e0, 0);
-      int c1 = 0, c2 = 0;
-      if (nsteps > 1) {
-        issue(e1, 1);
-        c1 = (int)uniform((uint32_t)loads_of(e1));
-      }
-      if (nsteps > 2) {
-        issue(e2, 2);
-        c2 = (int)uniform((uint32_t)loads_of(e2));
-      }
-      u32x4 bf[NT16][2];
-      u32x4 af[2][4];
-      for (int step = 0; step < nsteps; ++step) {
-        const uint32_t e4 = step_e[step + 4];  // a VGPR until the end of the step
-        wait_loads_all_but(c1 + c2);
-        __syncthreads();
-        int c3 = 0;
-        if (step + 3 < nsteps) {
-          issue(e3, (step + 3) % NST);
-          c3 = (int)uniform((uint32_t)loads_of(e3));
-        }
-        if (row_quads(step_flags(e0), rh_u)) {
-          const char* st = smem + (step % NST) * STAGE;
-          const char* at = st + A_OFF + rh * TILE;
-          read_b(st, 0, bf);
-          read_a(at, 0, af[0]);
-          read_b(st, 1, bf);
-          read_a(at, 1, af[1]);
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-              for (int nt = 0; nt < NT16; ++nt) acc[0][mt][nt] = T::mfma16(af[kk][mt], bf[nt][kk], acc[0][mt][nt]);
-        }
-        e0 = e1;
-        e1 = e2;
-        e2 = e3;
-        e3 = uniform(e4);
-        c1 = c2;
-        c2 = c3;
-      }
-      __syncthreads();  // the epilogue reuses the stages
-    }
   } else if constexpr (IMPLICIT == 0) {
     // The products that read their operands from memory run the units of all steps as one chain: the barrier
     // that publishes the next stage stands in front of the MFMAs of a step's LAST unit, not behind them.  By
@@ -954,7 +779,7 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
     u32x4 bf[NT16][2];
     u32x4 af[2][4];
     auto wave_quads = [&](uint32_t e) { return (step_flags(e) >> (4 * RW * rh)) & ((1u << (4 * RW)) - 1u); };
-    auto wave_mine = [&](uint32_t q) { return ((q & 0xfu) ? 1u : 0u) | ((RW == 2 && (q >> 4)) ? 2u : 0u); };
+    auto wave_mine = [&](uint32_t q) { return ((q & 0xfu) ? 1u : 0u) | ((q >> 4) ? 2u : 0u); };
     // fragments of the first unit of the step with table word e, whose tiles are in `stage`
     auto first_reads = [&](uint32_t e, int stage) {
       const uint32_t m = wave_mine(wave_quads(e));
@@ -1027,15 +852,10 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
       const uint32_t quads = wave_quads(e_cur);
       const uint32_t mine = wave_mine(quads);
       const bool red_tail = RAGGED && step_block(e_cur) == kb_tail;
-      if constexpr (RW == 2) {
-        if (mine == 3u) units(std::integral_constant<int, 3>{}, step, stage, e_next, e_after, red_tail, quads);
-        else if (mine == 1u) units(std::integral_constant<int, 1>{}, step, stage, e_next, e_after, red_tail, quads);
-        else if (mine == 2u) units(std::integral_constant<int, 2>{}, step, stage, e_next, e_after, red_tail, quads);
-        else boundary(step, stage, e_next, e_after);
-      } else {
-        if (mine) units(std::integral_constant<int, 1>{}, step, stage, e_next, e_after, red_tail, quads);
-        else boundary(step, stage, e_next, e_after);
-      }
+      if (mine == 3u) units(std::integral_constant<int, 3>{}, step, stage, e_next, e_after, red_tail, quads);
+      else if (mine == 1u) units(std::integral_constant<int, 1>{}, step, stage, e_next, e_after, red_tail, quads);
+      else if (mine == 2u) units(std::integral_constant<int, 2>{}, step, stage, e_next, e_after, red_tail, quads);
+      else boundary(step, stage, e_next, e_after);
       e_cur = e_next;
       e_next = uniform(e_after);
     }
@@ -1065,18 +885,14 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
     }
     // keep bits of this wave's row blocks (four per block); a block takes part when any of them is set
     const uint32_t quads = (step_flags(e_cur) >> (4 * RW * rh)) & ((1u << (4 * RW)) - 1u);
-    const uint32_t mine = ((quads & 0xfu) ? 1u : 0u) | ((RW == 2 && (quads >> 4)) ? 2u : 0u);
+    const uint32_t mine = ((quads & 0xfu) ? 1u : 0u) | ((quads >> 4) ? 2u : 0u);
     const bool mid = late && more && mine != 0u;
     if (more && !mid) issue_loads(e_next, stage ^ 1);
     const char* st = smem + stage * STAGE;
     const bool red_tail = RAGGED && step_block(e_cur) == kb_tail;
-    if constexpr (RW == 2) {
-      if (mine == 3u) compute(std::integral_constant<int, 3>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
-      else if (mine == 1u) compute(std::integral_constant<int, 1>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
-      else if (mine == 2u) compute(std::integral_constant<int, 2>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
-    } else {
-      if (mine) compute(std::integral_constant<int, 1>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
-    }
+    if (mine == 3u) compute(std::integral_constant<int, 3>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
+    else if (mine == 1u) compute(std::integral_constant<int, 1>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
+    else if (mine == 2u) compute(std::integral_constant<int, 2>{}, st, mid, e_next, stage ^ 1, red_tail, quads);
     if constexpr (STEP_COPIES) {
       if (step + 2 < nsteps) tpatch_store((step & 1) ? patch1 : patch);  // last read for this step's tiles, a step ago
     }
@@ -1171,11 +987,9 @@ __global__ __launch_bounds__(S::THREADS) void forward_lists_kernel(GemmArgs g, i
 // statically indexed by the wave's slot, operand tiles addressed dynamically.
 // SddBig   4 row blocks x groups of at most 6 active column blocks and 16 kept tiles, two tile slots per wave:
 //           two 80 KB stages, all of the LDS
-// SddMid   2 row blocks x at most 4 active column blocks and 8 kept tiles, one slot per wave: twice as many
-//           workgroups with half the loads per step each, for outputs that give the big shape too few
-template <int R_, int GW_, int SLOTS_, int NST_ = 2>
+template <int R_, int GW_, int SLOTS_>
 struct SddShape {
-  static constexpr int NST = NST_;       // stages of LDS (steps whose tiles are resident or on their way)
+  static constexpr int NST = 2;          // stages of LDS (steps whose tiles are resident or on their way)
   static constexpr int R = R_;           // row blocks per workgroup
   static constexpr int GW = GW_;         // column blocks with kept tiles per group
   static constexpr int SLOTS = SLOTS_;   // whole tiles a wave can own
@@ -1192,12 +1006,6 @@ struct SddShape {
   static constexpr int GPW = WINDOW / MINCOLS;  // groups a whole window can have at most
 };
 using SddBig = SddShape<4, 6, 2>;
-using SddMid = SddShape<2, 4, 1>;
-// On aligned operands, outputs too small for the big shape run with more steps in flight (a step of these shapes is
-// far shorter than a load's way through L2 and memory): the shape above with three stages, and for outputs that give
-// even that one too few workgroups, 2 row blocks x 2 column blocks (4 tiles, on waves 0-3; all 8 waves load) with four
-using SddMidDeep = SddShape<2, 4, 1, 3>;
-using SddSmall = SddShape<2, 2, 1, 4>;
 constexpr int G_MAX_CB = 8192;             // per-column flags share the first stage (of either shape) before the loads start
 
 // EDGE = the output width or the reduction length is not a multiple of 64 (both multiples of 8): the
@@ -1480,30 +1288,6 @@ __device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gma
       for (int nt = 0; nt < 4; ++nt) acc[k][mt][nt] = T::mfma16(af[u & 1][mt], bf[u & 1][nt], acc[k][mt][nt]);
   };
 
-  if constexpr (!EDGE && G::NST > 2) {
-    // ---- more than one step in flight: the tiles of steps s + 1 .. s + NST - 2 are on their way while step s
-    // computes; one barrier per step publishes step s and frees the stage of step s - 1, which the loads of step
-    // s + NST - 1 go into right behind it.  Every step costs this wave the same number of loads, so "my loads of
-    // step s have landed" is "at most (steps still in flight) x (loads per step) outstanding".
-    static_assert(SLOTS == 1, "one tile per wave");
-    constexpr int NST = G::NST;
-    const int n_ld = __builtin_popcount(rowmask) + ncols;
-    for (int s0 = 0; s0 < NST - 1 && s0 < nsteps; ++s0) issue_loads(s0, s0);
-    for (int step = 0; step < nsteps; ++step) {
-      const int left = nsteps - 1 - step;
-      wait_loads_all_but((left < NST - 2 ? left : NST - 2) * n_ld);
-      __syncthreads();
-      if (step + NST - 1 < nsteps) issue_loads(step + NST - 1, (step + NST - 1) % NST);
-      if (act[0]) {
-        const int stage = step % NST;
-        read_unit(stage, 0);
-        read_unit(stage, 1);
-        mfma_unit(std::integral_constant<int, 0>{}, 0, false);
-        mfma_unit(std::integral_constant<int, 0>{}, 1, false);
-      }
-    }
-    __syncthreads();  // the epilogue reuses the stages
-  } else {
   issue_loads(0, 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -1541,7 +1325,6 @@ __device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gma
     } else {
       boundary(step, stage, false);
     }
-  }
   }
 
   // ---- epilogue ---------------------------------------------------------------------------------------
@@ -1944,8 +1727,11 @@ int allow_big_lds(const void* kernel, int bytes, std::atomic<bool> (&done)[kMaxD
 
 std::atomic<int> tile_policy{0};
 
-template <typename T, bool TRANS, bool CM, bool RAGGED, typename S>
-int launch_dsd_s(const GemmArgs& g, int splits, hipStream_t stream) {
+bool is_bf16(int dtype) { return dtype == SD_BF16; }
+
+template <typename T, bool TRANS, bool CM, bool RAGGED>
+int launch_big_t(const GemmArgs& g, int splits, hipStream_t stream) {
+  using S = DsdBig;
   static std::atomic<bool> configured[kMaxDevices] = {};
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(&dsd_kernel<T, TRANS, CM, RAGGED, S>), S::SMEM_BYTES,
                              configured))
@@ -1954,41 +1740,33 @@ int launch_dsd_s(const GemmArgs& g, int splits, hipStream_t stream) {
   const int tiles_m = (Mb + S::R - 1) / S::R, tiles_n = (int)((g.N + S::BN - 1) / S::BN);
   hipLaunchKernelGGL((dsd_kernel<T, TRANS, CM, RAGGED, S>), dim3((unsigned)(tiles_m * tiles_n), (unsigned)splits),
                      dim3(S::THREADS), S::SMEM_BYTES, stream, g, tiles_m, tiles_n, Mb, Kb, ImplicitConv{});
-  if (int rc = check_launch("dsd_kernel")) return rc;
-  note_kernel("dsd:%s%s%s splits=%d", S::R * BS == 256 && S::BN == 256 ? "big" : "mid", TRANS ? ":strided" : "",
-              RAGGED ? ":ragged" : "", splits);
-  if (splits > 1) return launch_splitk_reduce(g, splits, CM, T::id, stream);
-  return SD_OK;
+  return check_launch("dsd_kernel");
+}
+template <typename T, bool TRANS, bool CM>
+int launch_big(const GemmArgs& g, bool ragged, int splits, hipStream_t stream) {
+  return ragged ? launch_big_t<T, TRANS, CM, true>(g, splits, stream) : launch_big_t<T, TRANS, CM, false>(g, splits, stream);
+}
+template <typename T>
+int launch_big(const GemmArgs& g, bool kc, bool cm, bool ragged, int splits, hipStream_t stream) {
+  if (kc) return cm ? launch_big<T, false, true>(g, ragged, splits, stream) : launch_big<T, false, false>(g, ragged, splits, stream);
+  return cm ? launch_big<T, true, true>(g, ragged, splits, stream) : launch_big<T, true, false>(g, ragged, splits, stream);
 }
 
 template <typename S>
 int64_t dsd_tiles(int64_t M, int64_t N) {
   return ((M + BS * S::R - 1) / (BS * S::R)) * ((N + S::BN - 1) / S::BN);
 }
-bool mid_tiles_fit_one_round(const GemmArgs& g, int splits) { return dsd_tiles<DsdMid>(g.M, g.N) * splits <= 256; }
+int64_t blocks_of(int64_t n) { return (n + BS - 1) / BS; }
 
-template <typename T, bool TRANS, bool CM>
-int launch_dsd(const GemmArgs& g, bool mid, int splits, hipStream_t stream) {
-  // masks of block size 32 (quadrant keep bits in the lists): the 256 x 256 shape leaves out the MFMAs of dropped
-  // quadrants on aligned operands; elsewhere they run on the ragged-edge instance, which zeroes fragments
-  const bool ragged = g.M % BS != 0 || g.N % BS != 0 || g.K % BS != 0 || (g.quads && mid);
-  if (mid) {
-    if (ragged) return launch_dsd_s<T, TRANS, CM, true, DsdMid>(g, splits, stream);
-    // one round of workgroups or less: a CU has one workgroup whatever its LDS, and the four-stage loop is the faster
-    // one (4096 x 1024 x 4096: 67 -> 52 us; 2048^3: 39 -> 30 us).  With more, two workgroups of the two-stage shape
-    // share a CU and keep its LDS busier than one of the four-stage shape can (8192^3 on this shape: 1.09 against
-    // 1.34 ms).
-    return mid_tiles_fit_one_round(g, splits) ? launch_dsd_s<T, TRANS, CM, false, DsdMidDeep>(g, splits, stream)
-                                              : launch_dsd_s<T, TRANS, CM, false, DsdMid>(g, splits, stream);
-  }
-  return ragged ? launch_dsd_s<T, TRANS, CM, true, DsdBig>(g, splits, stream)
-                : launch_dsd_s<T, TRANS, CM, false, DsdBig>(g, splits, stream);
+// Workgroups of a shape for an M x N output.
+int64_t shape_tiles(int shape, int64_t M, int64_t N) {
+  const int64_t edge = shape == kShapeOne ? 1 : (shape == kShapeBig ? 4 : 2);
+  return ((blocks_of(M) + edge - 1) / edge) * ((blocks_of(N) + edge - 1) / edge);
 }
 
-
-// workgroups a tile shape gives and how many ways the reduction is then split
+// Which shape a DSD (or dense) product runs on and how many ways its reduction is split.
 struct DsdPlan {
-  bool mid;
+  int shape;
   int splits;
 };
 // One round of workgroups (one per CU) when the output alone gives fewer than half of that and the
@@ -2001,21 +1779,72 @@ int splits_for(int64_t tiles, int64_t M, int64_t N, int64_t K) {
   while (want > 1 && want * M * N * 4 > (256LL << 20)) --want;
   return want < 2 ? 1 : (int)want;
 }
-DsdPlan plan_dsd(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0 || K <= 0) return {false, 1};
+// Microseconds a product is expected to take, from measured times per step (a 64-deep slice of the reduction) of a full
+// round of workgroups: 0.32 / 0.42 for 64 x 64 tiles at one / two per CU, 0.55 for 128 x 128 at one, 1.03 at two, 1.62
+// for 256 x 256 (two thirds more where its edges are ragged: that instance runs the older loop), plus what a round costs
+// outside its loop and, for a split reduction, the pass over the fp32 partials.  The drop rate is not known here; a step
+// of the smaller shapes is skipped more often (every row block of the tile must drop it), for which three quarters
+// of the blocks kept are assumed.
+double product_time(int shape, int64_t M, int64_t N, int64_t kb, int splits, bool ragged) {
+  const int64_t wgs = shape_tiles(shape, M, N) * splits;
+  const double steps = (double)((kb + splits - 1) / splits);
+  double t;
+  if (shape == kShapeOne) {
+    const int64_t rounds = (wgs + 511) / 512, last = wgs - (rounds - 1) * 512;
+    t = 0.75 * steps * (0.42 * (double)(rounds - 1) + (last <= 256 ? 0.32 : 0.42)) + 2.0 * (double)rounds;
+  } else if (shape == kShapeQuad) {
+    t = (double)((wgs + 255) / 256) * (0.94 * 0.55 * steps + 3.0);
+  } else if (shape == kShapeWide) {
+    const int64_t rounds = (wgs + 511) / 512, last = wgs - (rounds - 1) * 512;
+    t = 0.94 * steps * (1.03 * (double)(rounds - 1) + (last <= 256 ? 0.70 : 1.03)) + 4.0 * (double)rounds;
+  } else {
+    t = (double)((wgs + 255) / 256) * ((ragged ? 2.7 : 1.62) * steps + 7.0);
+  }
+  if (splits > 1) t += 4.0 + (double)splits * (double)M * (double)N * 8.0 / 4.0e6;
+  return t;
+}
+// kc: reduction-contiguous operands.  Those (the forward) are split by a rule on the extents alone, whatever the shape:
+// where a sum is cut decides its last bit, and a ReLU behind it must see the same signs on every shape.
+DsdPlan plan_dsd(int64_t M, int64_t N, int64_t K, bool kc) {
+  if (M <= 0 || N <= 0 || K <= 0) return {kShapeBig, 1};
   const int policy = tile_policy.load(std::memory_order_relaxed);
-  const int64_t big = dsd_tiles<DsdBig>(M, N), midt = dsd_tiles<DsdMid>(M, N);
-  // the 256 x 256 shape when it gives more than half of the CUs a workgroup (measured: 1024^3 forward 29 us on
-  // 16 big tiles, 13 us on 64 mid tiles; 2048^3 29 + 18 us on 64 big tiles x 4 splits and the reduce pass,
-  // 24 us on 256 mid tiles; 8192 x 1024 x 1024, 128 big tiles, 30 against 22 us; 3072^3, 144 big tiles, 79
-  // against 94 us; 4096^3, 256 big tiles, 127 against 158 us; weight gradients over 16384 to 131072 rows
-  // 15-30 % faster on mid tiles x fewer splits)
-  const bool mid = policy == kTileMid || (policy == kTileAuto && big <= 128);
-  return {mid, splits_for(mid ? midt : big, M, N, K)};
+  const int64_t kb = blocks_of(K), big = shape_tiles(kShapeBig, M, N);
+  if (policy == kTileBig) return {kShapeBig, splits_for(big, M, N, K)};
+  const int64_t fixed = !kc ? 0 : splits_for(policy == kTileMid || big <= 128 ? shape_tiles(kShapeQuad, M, N) : big, M, N, K);
+  const bool ragged = M % BS || N % BS || K % BS;
+  DsdPlan best{kShapeWide, 1};
+  double t_best = 1e30;
+  for (int shape = kShapeOne; shape <= kShapeBig; ++shape) {
+    if (policy == kTileMid && shape != kShapeQuad && shape != kShapeWide) continue;
+    const int64_t tiles = shape_tiles(shape, M, N);
+    if (shape == kShapeQuad && tiles > 256) continue;
+    // no split, a full round of workgroups, or half of one
+    const int64_t round = shape == kShapeOne ? 512 : 256;
+    for (int64_t want = kc ? fixed : 1;;) {
+      const int64_t most = shape == kShapeBig ? 1024 : kTileMaxSteps;
+      int64_t s = want;
+      if (!kc && s > kb / 4) s = kb / 4;
+      while (s > 1 && s * M * N * 4 > (256LL << 20)) --s;
+      if (s < 1) s = 1;
+      if ((kb + s - 1) / s <= most) {
+        const double t = product_time(shape, M, N, kb, (int)s, ragged);
+        if (t < t_best) {
+          t_best = t;
+          best = {shape, (int)s};
+        }
+      }
+      if (kc || shape == kShapeWide || shape == kShapeBig || 2 * tiles > round) break;
+      if (want == 1) want = (round / 2) / tiles > 1 ? (round / 2) / tiles : round / tiles;
+      else if (want == round / tiles) break;
+      else want = round / tiles;
+    }
+  }
+  return best;
 }
 
-template <typename T, bool EDGE, typename G>
-int launch_sdd_shape(const GemmArgs& g, hipStream_t stream) {
+template <typename T, bool EDGE>
+int launch_sdd_big(const GemmArgs& g, hipStream_t stream) {
+  using G = SddBig;
   static std::atomic<bool> configured[kMaxDevices] = {};
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(&sdd_group_kernel<T, EDGE, G>), G::SMEM, configured)) return rc;
   const int Mb = (int)((g.M + BS - 1) / BS), Cb = (int)((g.N + BS - 1) / BS);
@@ -2023,48 +1852,59 @@ int launch_sdd_shape(const GemmArgs& g, hipStream_t stream) {
   const int tiles_m = (Mb + G::R - 1) / G::R, gmax = (Cb + G::MINCOLS - 1) / G::MINCOLS;
   hipLaunchKernelGGL((sdd_group_kernel<T, EDGE, G>), dim3((unsigned)(tiles_m * gmax)), dim3(THREADS), G::SMEM, stream,
                      g, tiles_m, gmax, Mb, Cb);
-  note_kernel("sdd:%s%s", G::R == 4 ? "big" : (G::GW == 2 ? "small" : "mid"), EDGE ? ":ragged" : "");
   return check_launch("sdd_group_kernel");
 }
 
-// the big shape when its grid (a workgroup per 4 x 4 tiles, per 4 x 6 at high drop rates) gives more than half of
-// the CUs a workgroup
-template <typename T>
-int launch_sdd_group(const GemmArgs& g, bool ragged, hipStream_t stream) {
-  const int64_t Mb = (g.M + BS - 1) / BS, Cb = (g.N + BS - 1) / BS;
-  // workgroups the big shape would have: a group spans 4 column blocks with everything kept, 6 once few enough tiles
-  // are kept for the width and not the tile count to end a group (measured: worth counting that way from p = 0.7).
-  // The kept fraction is the caller's hint (the lists live on the device); unknown counts as everything kept.
-  const float keep = (g.row_ptr && g.keep_hint >= 0.f && g.keep_hint <= 1.f) ? g.keep_hint : 1.f;
-  const int64_t cols = keep <= 0.3f ? SddBig::GW : SddBig::MINCOLS;
-  const int64_t big = ((Mb + 3) / 4) * ((Cb + cols - 1) / cols);
+float kept_fraction(const GemmArgs& g) {  // the caller's hint; unknown counts as everything kept
+  return (g.row_ptr && g.keep_hint >= 0.f && g.keep_hint <= 1.f) ? g.keep_hint : 1.f;
+}
+
+// workgroups the big SDD shape would have: a group spans 4 column blocks with everything kept, 6 once few enough tiles
+// are kept for the width and not the tile count to end a group (measured: worth counting that way from p = 0.7)
+int64_t sdd_big_groups(const GemmArgs& g) {
+  const int64_t cols = kept_fraction(g) <= 0.3f ? SddBig::GW : SddBig::MINCOLS;
+  return ((blocks_of(g.M) + 3) / 4) * ((blocks_of(g.N) + cols - 1) / cols);
+}
+
+// what the kernels of either kind ask of an SDD product's operands, and what the big ones ask on top
+bool sdd_operands_ok(const GemmArgs& g) {
+  return g.a.sc == 1 && g.b.sr == 1 && g.b.sc != 1 && g.c_sc == 1 && g.M > 0 && g.N > 0 && g.K > 0 && g.K % 8 == 0 &&
+         aligned16(g.a.ptr) && aligned16(g.b.ptr) && g.a.sr % 8 == 0 && g.b.sc % 8 == 0 && g.a.sr < (1 << 22) &&
+         g.b.sc < (1 << 22);  // per-lane byte offsets are 32-bit
+}
+bool sdd_big_ok(const GemmArgs& g) {
+  return g.N % 8 == 0 && g.c_sr % 8 == 0 && aligned16(g.c) && (!(g.act && g.aux) || (g.aux_sr % 8 == 0 && aligned16(g.aux))) &&
+         blocks_of(g.N) <= G_MAX_CB;
+}
+
+// The big shape when its grid gives more than half of the CUs a workgroup (on aligned operands: its edge instance runs
+// the older loop); else by the number of kept tiles: up to about one 64 x 64 tile per CU one to a workgroup, else
+// strips of four while their grid is at most two rounds, else strips of two, three workgroups to a CU.
+int plan_sdd(const GemmArgs& g) {
   const int policy = tile_policy.load(std::memory_order_relaxed);
-  const bool mid = policy == kTileMid || (policy == kTileAuto && big <= 128);
-  // masks of block size 32 (quadrant keep bits in the lists): the big shape leaves out the MFMAs of dropped quadrants
-  // on aligned operands; the other instances zero them in the epilogue, which lives in the ragged-edge code
-  if (!mid) return (ragged ? launch_sdd_shape<T, true, SddBig> : launch_sdd_shape<T, false, SddBig>)(g, stream);
-  if (ragged || g.quads) return launch_sdd_shape<T, true, SddMid>(g, stream);
-  // aligned: the loops with several steps in flight (the two-stage shape holds a CU alone as well: its epilogue's
-  // staging tiles take 136 KB).  Half a round of workgroups or less on the 2 x 4 shape: the 2 x 2 shape, twice as many
-  // (4096 x 4096 -> 1024 columns: 93 us on 128 workgroups of the two-stage shape).
-  const int64_t mid_wgs = ((Mb + 1) / 2) * ((Cb + 3) / 4);
-  if (policy == kTileAuto && mid_wgs <= 128) return launch_sdd_shape<T, false, SddSmall>(g, stream);
-  return launch_sdd_shape<T, false, SddMidDeep>(g, stream);
+  const int64_t Mb = blocks_of(g.M), Cb = blocks_of(g.N);
+  const bool ragged = g.N % BS || g.K % BS;
+  if (sdd_big_ok(g)) {
+    if (policy == kTileBig) return kShapeBig;
+    if (policy == kTileAuto && !ragged && sdd_big_groups(g) > 128) return kShapeBig;
+  }
+  if (policy == kTileMid) return kShapeWide;
+  if ((double)(Mb * Cb) * kept_fraction(g) <= 320.0) return kShapeOne;
+  return Mb * ((Cb + 3) / 4) <= 512 ? kShapeQuad : kShapeWide;
 }
 
 int try_sdd(const GemmArgs& g, int dtype, hipStream_t stream) {
   if (g.row_ptr && g.bs != BS) return SD_ERR_UNSUPPORTED;
-  const bool layout_ok = g.a.sc == 1 && g.b.sr == 1 && g.b.sc != 1 && g.c_sc == 1;
-  const bool shape_ok = g.M > 0 && g.N > 0 && g.N % 8 == 0 && g.K > 0 && g.K % 8 == 0;  // any M
-  const bool align_ok = aligned16(g.a.ptr) && aligned16(g.b.ptr) && aligned16(g.c) && g.a.sr % 8 == 0 &&
-                        g.b.sc % 8 == 0 && g.c_sr % 8 == 0 && g.a.sr < (1 << 22) &&
-                        g.b.sc < (1 << 22);  // per-lane byte offsets are 32-bit
-  const int64_t Cb = (g.N + BS - 1) / BS;
-  const int64_t tiles = (((g.M + BS - 1) / BS + 1) / 2) * ((Cb + 3) / 4);  // the larger of the two shapes' grids
-  if (!layout_ok || !shape_ok || !align_ok || tiles > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
-  if (Cb > G_MAX_CB) return SD_ERR_UNSUPPORTED;
+  if (!sdd_operands_ok(g) || blocks_of(g.M) * blocks_of(g.N) > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
+  const int shape = plan_sdd(g);
   const bool ragged = g.N % BS != 0 || g.K % BS != 0;
-  return dtype == SD_BF16 ? launch_sdd_group<BF16>(g, ragged, stream) : launch_sdd_group<F16>(g, ragged, stream);
+  if (shape == kShapeBig) {
+    note_kernel("sdd:big%s", ragged ? ":ragged" : "");
+    if (is_bf16(dtype)) return ragged ? launch_sdd_big<BF16, true>(g, stream) : launch_sdd_big<BF16, false>(g, stream);
+    return ragged ? launch_sdd_big<F16, true>(g, stream) : launch_sdd_big<F16, false>(g, stream);
+  }
+  note_kernel("sdd:%s", shape == kShapeWide ? "mid" : "small");  // small: with loading waves
+  return is_bf16(dtype) ? tile_sdd<BF16>(g, shape, stream) : tile_sdd<F16>(g, shape, stream);
 }
 
 template <typename T, bool RAGGED, int FORM>
@@ -2187,23 +2027,42 @@ int launch_conv_implicit(const GemmArgs& g, const ImplicitConv& cg, int64_t P, i
   return ragged ? launch_conv_t<F16, true, 1>(g, cg, smem, stream) : launch_conv_t<F16, false, 1>(g, cg, smem, stream);
 }
 
-// How many ways the DSD kernel splits the reduction of this product: the plan's count cut down to what the caller's
-// scratch holds; 0 = the specialised kernel should not take the product (its step table is per workgroup, and with
-// scratch too small for its own partials the generic kernel's split may still fit).
-int usable_splits(const GemmArgs& g, const DsdPlan& plan, int mode) {
-  const int64_t tiles = plan.mid ? dsd_tiles<DsdMid>(g.M, g.N) : dsd_tiles<DsdBig>(g.M, g.N);
-  int splits = plan.splits;
-  const int64_t part_bytes = g.M * g.N * 4;
-  if (splits > 1 && (g.ws == nullptr || g.ws_bytes < part_bytes * splits))
-    splits = g.ws ? (int)(g.ws_bytes / part_bytes) : 1;
-  if (splits < 1) splits = 1;
-  if (((g.K + BS - 1) / BS + splits - 1) / splits > MAX_STEPS) return 0;
-  if (splits == 1 && tiles < 128 && g.ws != nullptr) {
-    const int gs = generic_splits(g.M, g.N, g.K, g.bs, mode);
-    if (gs > 1 && g.ws_bytes >= (int64_t)gs * part_bytes) return 0;
-  }
-  return splits;
+// What a DSD (or dense) product's operands have to look like for the specialised kernels, and for the big ones on top.
+// kc: reduction-contiguous operands, else reduction-strided.
+struct DsdForm {
+  bool ok, big_ok, kc, cm, ragged;
+};
+DsdForm dsd_form(const GemmArgs& g) {
+  const bool nt = g.a.sc == 1 && g.b.sc == 1;         // reduction-contiguous operands
+  const bool tn = !nt && g.a.sr == 1 && g.b.sr == 1;  // reduction-strided operands
+  const int64_t lda = nt ? g.a.sr : g.a.sc, ldb = nt ? g.b.sr : g.b.sc;
+  DsdForm f;
+  f.kc = nt;
+  f.cm = g.c_sc != 1;  // column-major C
+  f.ragged = g.M % BS != 0 || g.N % BS != 0 || g.K % BS != 0;
+  f.ok = (nt || tn) && g.M > 0 && g.N > 0 && g.K > 0 && (tn || g.K % 8 == 0) && blocks_of(g.K) < 65536 &&
+         aligned16(g.a.ptr) && aligned16(g.b.ptr) && lda % 8 == 0 && ldb % 8 == 0 && lda < (1 << 22) &&
+         ldb < (1 << 22) &&  // per-lane byte offsets are 32-bit
+         shape_tiles(kShapeOne, g.M, g.N) <= 0x7fffffffLL;
+  // the big kernels' edge instance works in multiples of 8 along contiguous indices
+  f.big_ok = f.ok && (nt || (g.M % 8 == 0 && g.N % 8 == 0));
+  return f;
 }
+
+// The plan for this product and these operands, its splits cut down to what the caller's scratch holds; splits == 0: a
+// workgroup could not walk its share of the reduction.
+DsdPlan plan_for(const GemmArgs& g, const DsdForm& f) {
+  DsdPlan plan = plan_dsd(g.M, g.N, g.K, f.kc);
+  if (plan.shape == kShapeBig && !f.big_ok) plan.shape = kShapeWide;
+  const int64_t part_bytes = g.M * g.N * 4;
+  if (plan.splits > 1 && (g.ws == nullptr || g.ws_bytes < part_bytes * plan.splits))
+    plan.splits = g.ws ? (int)(g.ws_bytes / part_bytes) : 1;
+  if (plan.splits < 1) plan.splits = 1;
+  const int64_t most = plan.shape == kShapeBig ? MAX_STEPS : kTileMaxSteps;
+  if ((blocks_of(g.K) + plan.splits - 1) / plan.splits > most) plan.splits = 0;
+  return plan;
+}
+const char* dsd_name(int shape) { return shape == kShapeBig ? "big" : (shape == kShapeOne ? "one" : "mid"); }
 
 // most workgroups either product of a single-launch backward may have (SPARSEDROP_PAIR_LIMIT overrides, for measuring)
 int64_t pair_limit() {
@@ -2220,30 +2079,21 @@ int launch_fast(const GemmArgs& g, int mode, int dtype, hipStream_t stream) {
   // kernel with every tile kept
   if (mode == kDense && g.a.sc == 1 && g.b.sr == 1 && g.b.sc != 1 && g.c_sc == 1) return try_sdd(g, dtype, stream);
   if (mode == kDsd && g.bs != BS) return SD_ERR_UNSUPPORTED;
-  // everything tile-aligned and 16-byte aligned; A and B agree on whether the reduction index is contiguous
-  const bool nt = g.a.sc == 1 && g.b.sc == 1;         // reduction-contiguous operands
-  const bool tn = !nt && g.a.sr == 1 && g.b.sr == 1;  // reduction-strided operands
-  const bool cm = g.c_sc != 1;                        // column-major C
-  // ragged edges: any extent along a strided index, multiples of 8 (the 16 bytes of a load) along a contiguous one
-  const bool shape_ok = g.M > 0 && (nt || g.M % 8 == 0) && g.N > 0 && (nt || g.N % 8 == 0) && g.K > 0 &&
-                        (tn || g.K % 8 == 0) && (g.K + BS - 1) / BS < 65536;
-  const int64_t lda = nt ? g.a.sr : g.a.sc, ldb = nt ? g.b.sr : g.b.sc;
-  const bool align_ok = aligned16(g.a.ptr) && aligned16(g.b.ptr) && lda % 8 == 0 && ldb % 8 == 0 &&
-                        lda < (1 << 22) && ldb < (1 << 22);  // per-lane byte offsets are 32-bit
-  const DsdPlan plan = plan_dsd(g.M, g.N, g.K);
-  const int64_t tiles = plan.mid ? dsd_tiles<DsdMid>(g.M, g.N) : dsd_tiles<DsdBig>(g.M, g.N);
-  if (!(nt || tn) || !shape_ok || !align_ok || tiles > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
-  // few output tiles and a long reduction (the weight gradient of a tall matrix): split the reduction
-  // over workgroups when the caller gave scratch for the fp32 partials
-  const int splits = usable_splits(g, plan, mode);
-  if (splits < 1) return SD_ERR_UNSUPPORTED;
-  const bool mid = plan.mid;
-  if (dtype == SD_BF16) {
-    if (nt) return cm ? launch_dsd<BF16, false, true>(g, mid, splits, stream) : launch_dsd<BF16, false, false>(g, mid, splits, stream);
-    return cm ? launch_dsd<BF16, true, true>(g, mid, splits, stream) : launch_dsd<BF16, true, false>(g, mid, splits, stream);
-  }
-  if (nt) return cm ? launch_dsd<F16, false, true>(g, mid, splits, stream) : launch_dsd<F16, false, false>(g, mid, splits, stream);
-  return cm ? launch_dsd<F16, true, true>(g, mid, splits, stream) : launch_dsd<F16, true, false>(g, mid, splits, stream);
+  const DsdForm f = dsd_form(g);
+  if (!f.ok) return SD_ERR_UNSUPPORTED;
+  const DsdPlan plan = plan_for(g, f);
+  if (plan.splits < 1) return SD_ERR_UNSUPPORTED;
+  int rc;
+  if (plan.shape == kShapeBig)
+    rc = is_bf16(dtype) ? launch_big<BF16>(g, f.kc, f.cm, f.ragged, plan.splits, stream)
+                        : launch_big<F16>(g, f.kc, f.cm, f.ragged, plan.splits, stream);
+  else
+    rc = is_bf16(dtype) ? tile_dsd<BF16>(g, f.kc, f.cm, plan.shape, plan.splits, stream)
+                        : tile_dsd<F16>(g, f.kc, f.cm, plan.shape, plan.splits, stream);
+  if (rc) return rc;
+  note_kernel("dsd:%s%s%s splits=%d", dsd_name(plan.shape), f.kc ? "" : ":strided",
+              f.ragged && plan.shape == kShapeBig ? ":ragged" : "", plan.splits);
+  return plan.splits > 1 ? launch_splitk_reduce(g, plan.splits, f.cm, dtype, stream) : SD_OK;
 }
 
 // ---- the forward product and the kept lists of its mask in one launch -------------------------------------------
@@ -2257,8 +2107,9 @@ int64_t forward_lists_limit() {
   return limit;
 }
 
-template <typename T, bool RAGGED, typename S>
+template <typename T, bool RAGGED>
 int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
+  using S = DsdBig;
   static std::atomic<bool> configured[kMaxDevices] = {};
   auto* kernel = &forward_lists_kernel<T, RAGGED, S>;
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(kernel), S::SMEM_BYTES, configured)) return rc;
@@ -2267,11 +2118,7 @@ int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hip
   const int n_gemm = tiles_m * tiles_n * splits;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::SMEM_BYTES, stream, g, tiles_m,
                      tiles_n, Mb, Kb, splits, n_gemm, f);
-  if (int rc = check_launch("forward_lists_kernel")) return rc;
-  note_kernel("dsd+lists:%s%s splits=%d", S::R * BS == 256 && S::BN == 256 ? "big" : "mid", RAGGED ? ":ragged" : "",
-              splits);
-  if (splits > 1) return launch_splitk_reduce(g, splits, false, T::id, stream);
-  return SD_OK;
+  return check_launch("forward_lists_kernel");
 }
 
 // g: the forward product (reduction-contiguous operands, row-major C) on the 64 grid; src: its mask, listed on an
@@ -2283,44 +2130,37 @@ int launch_forward_with_lists(const GemmArgs& g, const MaskSrc& src, int64_t mb,
                               int64_t mask_rows, int dtype, hipStream_t stream) {
   if (g.bs != BS || mb * kb > kFlatMaxEntries) return SD_ERR_UNSUPPORTED;
   if (mb != (g.M + BS - 1) / BS || kb != (g.K + BS - 1) / BS) return SD_ERR_UNSUPPORTED;
-  // the forward's conditions (launch_fast)
-  const bool nt = g.a.sc == 1 && g.b.sc == 1 && g.c_sc == 1;
-  const bool shape_ok = g.M > 0 && g.N > 0 && g.K > 0 && g.K % 8 == 0 && (g.K + BS - 1) / BS < 65536;
-  const bool align_ok = aligned16(g.a.ptr) && aligned16(g.b.ptr) && g.a.sr % 8 == 0 && g.b.sr % 8 == 0 &&
-                        g.a.sr < (1 << 22) && g.b.sr < (1 << 22);
-  if (!nt || !shape_ok || !align_ok) return SD_ERR_UNSUPPORTED;
-  const DsdPlan plan = plan_dsd(g.M, g.N, g.K);
-  const int64_t tiles = plan.mid ? dsd_tiles<DsdMid>(g.M, g.N) : dsd_tiles<DsdBig>(g.M, g.N);
-  const int splits = usable_splits(g, plan, kDsd);
-  if (splits < 1 || tiles * splits > forward_lists_limit()) return SD_ERR_UNSUPPORTED;
-  const bool ragged = g.M % BS != 0 || g.N % BS != 0 || g.K % BS != 0 || (g.quads && plan.mid);
+  const DsdForm form = dsd_form(g);
+  if (!form.ok || !form.kc || form.cm) return SD_ERR_UNSUPPORTED;
+  const DsdPlan plan = plan_for(g, form);
+  if (plan.splits < 1 || dsd_tiles<DsdBig>(g.M, g.N) > forward_lists_limit()) return SD_ERR_UNSUPPORTED;
   const FlatJobs f = flat_jobs(src, mb, kb, row_ptr, col_idx, col_ptr, row_idx, mask_out, mask_rows,
-                               plan.mid ? DsdMid::THREADS : DsdBig::THREADS);
-  // the four-stage shape holds a CU alone, the list builder's blocks included: only when they all find a CU of their own
-  // in one round (else the blocks that build the lists wait for a product workgroup to finish, and the two-stage shape,
-  // which shares a CU with them, is as fast)
-  const bool deep = plan.mid && !ragged && tiles * splits + f.blocks() <= 256;
-  if (dtype == SD_BF16) {
-    if (deep) return launch_forward_lists_t<BF16, false, DsdMidDeep>(g, splits, f, stream);
-    if (plan.mid) return ragged ? launch_forward_lists_t<BF16, true, DsdMid>(g, splits, f, stream)
-                                : launch_forward_lists_t<BF16, false, DsdMid>(g, splits, f, stream);
-    return ragged ? launch_forward_lists_t<BF16, true, DsdBig>(g, splits, f, stream)
-                  : launch_forward_lists_t<BF16, false, DsdBig>(g, splits, f, stream);
-  }
-  if (deep) return launch_forward_lists_t<F16, false, DsdMidDeep>(g, splits, f, stream);
-  if (plan.mid) return ragged ? launch_forward_lists_t<F16, true, DsdMid>(g, splits, f, stream)
-                              : launch_forward_lists_t<F16, false, DsdMid>(g, splits, f, stream);
-  return ragged ? launch_forward_lists_t<F16, true, DsdBig>(g, splits, f, stream)
-                : launch_forward_lists_t<F16, false, DsdBig>(g, splits, f, stream);
+                               plan.shape == kShapeBig ? DsdBig::THREADS : tile_threads(plan.shape));
+  int rc;
+  if (plan.shape != kShapeBig)
+    rc = is_bf16(dtype) ? tile_forward<BF16>(g, plan.shape, plan.splits, f, stream)
+                        : tile_forward<F16>(g, plan.shape, plan.splits, f, stream);
+  else if (is_bf16(dtype))
+    rc = form.ragged ? launch_forward_lists_t<BF16, true>(g, plan.splits, f, stream)
+                     : launch_forward_lists_t<BF16, false>(g, plan.splits, f, stream);
+  else
+    rc = form.ragged ? launch_forward_lists_t<F16, true>(g, plan.splits, f, stream)
+                     : launch_forward_lists_t<F16, false>(g, plan.splits, f, stream);
+  if (rc) return rc;
+  note_kernel("dsd+lists:%s%s splits=%d", dsd_name(plan.shape), form.ragged && plan.shape == kShapeBig ? ":ragged" : "",
+              plan.splits);
+  return plan.splits > 1 ? launch_splitk_reduce(g, plan.splits, false, dtype, stream) : SD_OK;
 }
 
 // ---- both gradients in one launch ------------------------------------------------------------------------
 // gx: the SDD product dX = s (dY . W) on the kept tiles; gw: the DSD product dW^T = s X^T(kept blocks) . dY with
 // reduction-strided operands and column-major C.  SD_ERR_UNSUPPORTED (nothing launched) unless each would run on its
-// specialised kernel by itself, unsplit, and both on the same size of workgroup shape; the caller then launches them
-// one after the other.
-template <typename T, bool EDGE, typename G, typename S>
+// specialised kernel by itself and both on the same size of workgroup shape; the caller then launches them one after
+// the other.
+template <typename T, bool EDGE>
 int launch_pair_t(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_t stream) {
+  using G = SddBig;
+  using S = DsdBig;
   constexpr int SMEM = G::SMEM > S::SMEM_BYTES ? G::SMEM : S::SMEM_BYTES;
   static std::atomic<bool> configured[kMaxDevices] = {};
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(&backward_pair_kernel<T, EDGE, G, S>), SMEM, configured))
@@ -2331,60 +2171,45 @@ int launch_pair_t(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_
   const int w_Mb = (int)((gw.M + BS - 1) / BS), w_Kb = (int)((gw.K + BS - 1) / BS);
   const int w_tiles_m = (w_Mb + S::R - 1) / S::R, w_tiles_n = (int)((gw.N + S::BN - 1) / S::BN);
   const int64_t total = n_dx + (int64_t)w_tiles_m * w_tiles_n * splits;
-  if (total > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
   hipLaunchKernelGGL((backward_pair_kernel<T, EDGE, G, S>), dim3((unsigned)total), dim3(THREADS), SMEM, stream, gx,
                      x_tiles_m, x_gmax, x_Mb, x_Cb, (int)n_dx, gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, splits);
-  note_kernel("pair:sdd+dsd:%s%s splits=%d", G::R == 4 ? "big" : "mid", EDGE ? ":ragged" : "", splits);
-  if (int rc = check_launch("backward_pair_kernel")) return rc;
-  if (splits > 1) return launch_splitk_reduce(gw, splits, true, T::id, stream);
-  return SD_OK;
+  return check_launch("backward_pair_kernel");
 }
 
 int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipStream_t stream) {
-  // the SDD product's conditions (try_sdd)
-  if (!gx.row_ptr || gx.bs != BS || gx.kept_only) return SD_ERR_UNSUPPORTED;
-  const int64_t x_Cb = (gx.N + BS - 1) / BS, x_Mb = (gx.M + BS - 1) / BS;
-  const bool x_ok = gx.a.sc == 1 && gx.b.sr == 1 && gx.b.sc != 1 && gx.c_sc == 1 && gx.M > 0 && gx.N > 0 &&
-                    gx.N % 8 == 0 && gx.K > 0 && gx.K % 8 == 0 && aligned16(gx.a.ptr) && aligned16(gx.b.ptr) &&
-                    aligned16(gx.c) && gx.a.sr % 8 == 0 && gx.b.sc % 8 == 0 && gx.c_sr % 8 == 0 &&
-                    gx.a.sr < (1 << 22) && gx.b.sc < (1 << 22) && x_Cb <= G_MAX_CB;
-  // the weight gradient's (launch_fast), in the one form the autograd step produces
-  if (!gw.row_ptr || gw.bs != BS || gw.act) return SD_ERR_UNSUPPORTED;
-  const bool w_ok = gw.a.sr == 1 && gw.b.sr == 1 && gw.a.sc != 1 && gw.b.sc != 1 && gw.c_sc != 1 && gw.c_sr == 1 &&
-                    gw.M > 0 && gw.M % 8 == 0 && gw.N > 0 && gw.N % 8 == 0 && gw.K > 0 && (gw.K + BS - 1) / BS < 65536 &&
-                    aligned16(gw.a.ptr) && aligned16(gw.b.ptr) && aligned16(gw.c) && gw.a.sc % 8 == 0 &&
-                    gw.b.sc % 8 == 0 && gw.c_sc % 8 == 0 && gw.a.sc < (1 << 22) && gw.b.sc < (1 << 22);
-  if (!x_ok || !w_ok) return SD_ERR_UNSUPPORTED;
-  const DsdPlan plan = plan_dsd(gw.M, gw.N, gw.K);
-  const int splits = usable_splits(gw, plan, kDsd);
-  if (splits < 1) return SD_ERR_UNSUPPORTED;
-  // the SDD shape as launch_sdd_group picks it; both products must want the same size
-  const float keep = (gx.keep_hint >= 0.f && gx.keep_hint <= 1.f) ? gx.keep_hint : 1.f;
-  const int64_t cols = keep <= 0.3f ? SddBig::GW : SddBig::MINCOLS;
-  const int64_t big = ((x_Mb + 3) / 4) * ((x_Cb + cols - 1) / cols);
-  const int policy = tile_policy.load(std::memory_order_relaxed);
-  const bool x_mid = policy == kTileMid || (policy == kTileAuto && big <= 128);
-  if (x_mid != plan.mid) return SD_ERR_UNSUPPORTED;
+  if (!gx.row_ptr || gx.bs != BS || gx.kept_only || !sdd_operands_ok(gx)) return SD_ERR_UNSUPPORTED;
+  // the weight gradient in the one form the autograd step produces
+  const DsdForm form = dsd_form(gw);
+  if (!gw.row_ptr || gw.bs != BS || gw.act || !form.ok || form.kc || !form.cm || gw.c_sr != 1) return SD_ERR_UNSUPPORTED;
+  const DsdPlan plan = plan_for(gw, form);
+  if (plan.splits < 1) return SD_ERR_UNSUPPORTED;
+  const int x_shape = plan_sdd(gx);
   // Worth it only while neither product fills the chip by itself: side by side, two large products get in each
   // other's way in the L2 (8192^3 at p = 0.5: 1.33 ms in one launch against 1.28 in two; 1024^3: 27 us against 46).
-  const int64_t x_wgs = x_mid ? ((x_Mb + 1) / 2) * ((x_Cb + 3) / 4) : big;
-  const int64_t w_wgs = (plan.mid ? dsd_tiles<DsdMid>(gw.M, gw.N) : dsd_tiles<DsdBig>(gw.M, gw.N)) * splits;
-  if (x_wgs > pair_limit() || w_wgs > pair_limit()) return SD_ERR_UNSUPPORTED;
-  if ((x_Mb + 1) / 2 * ((x_Cb + 3) / 4) + dsd_tiles<DsdMid>(gw.M, gw.N) > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
-  // either product ragged (or, on the smaller shapes, on a block-size-32 mask): the instances that handle edges, for both
-  const bool edge = gx.N % BS != 0 || gx.K % BS != 0 || gw.M % BS != 0 || gw.N % BS != 0 || gw.K % BS != 0 ||
-                    ((gx.quads || gw.quads) && x_mid);
-  if (dtype == SD_BF16) {
-    // (the smaller SDD shape holds a CU alone anyway: the loops with more stages cost nothing)
-    if (x_mid) return edge ? launch_pair_t<BF16, true, SddMid, DsdMid>(gx, gw, splits, stream)
-                           : launch_pair_t<BF16, false, SddMidDeep, DsdMidDeep>(gx, gw, splits, stream);
-    return edge ? launch_pair_t<BF16, true, SddBig, DsdBig>(gx, gw, splits, stream)
-                : launch_pair_t<BF16, false, SddBig, DsdBig>(gx, gw, splits, stream);
+  if (x_shape == kShapeBig || plan.shape == kShapeBig) {
+    if (x_shape != plan.shape || sdd_big_groups(gx) > pair_limit() ||
+        shape_tiles(kShapeBig, gw.M, gw.N) * plan.splits > pair_limit())
+      return SD_ERR_UNSUPPORTED;
+    const bool edge = gx.N % BS != 0 || gx.K % BS != 0 || form.ragged;
+    int rc;
+    if (is_bf16(dtype))
+      rc = edge ? launch_pair_t<BF16, true>(gx, gw, plan.splits, stream) : launch_pair_t<BF16, false>(gx, gw, plan.splits, stream);
+    else
+      rc = edge ? launch_pair_t<F16, true>(gx, gw, plan.splits, stream) : launch_pair_t<F16, false>(gx, gw, plan.splits, stream);
+    if (rc) return rc;
+    note_kernel("pair:sdd+dsd:big%s splits=%d", edge ? ":ragged" : "", plan.splits);
+    return plan.splits > 1 ? launch_splitk_reduce(gw, plan.splits, true, dtype, stream) : SD_OK;
   }
-  if (x_mid) return edge ? launch_pair_t<F16, true, SddMid, DsdMid>(gx, gw, splits, stream)
-                         : launch_pair_t<F16, false, SddMidDeep, DsdMidDeep>(gx, gw, splits, stream);
-  return edge ? launch_pair_t<F16, true, SddBig, DsdBig>(gx, gw, splits, stream)
-              : launch_pair_t<F16, false, SddBig, DsdBig>(gx, gw, splits, stream);
+  // The loading-wave shapes go together: dX takes the weight gradient's workgroup size (its results are the same bits on
+  // either, and a launch saved is more than the shapes differ by).
+  if (x_shape == kShapeWide || plan.shape == kShapeWide) return SD_ERR_UNSUPPORTED;
+  const int64_t x_wgs = blocks_of(gx.M) * (plan.shape == kShapeOne ? blocks_of(gx.N) : (blocks_of(gx.N) + 3) / 4);
+  if (x_wgs > 2 * pair_limit() || shape_tiles(plan.shape, gw.M, gw.N) * plan.splits > pair_limit()) return SD_ERR_UNSUPPORTED;
+  const int rc = is_bf16(dtype) ? tile_pair<BF16>(gx, gw, plan.shape, plan.splits, stream)
+                                : tile_pair<F16>(gx, gw, plan.shape, plan.splits, stream);
+  if (rc) return rc;
+  note_kernel("pair:sdd+dsd:%s splits=%d", dsd_name(plan.shape), plan.splits);
+  return plan.splits > 1 ? launch_splitk_reduce(gw, plan.splits, true, dtype, stream) : SD_OK;
 }
 
 int set_tile_policy(int policy) {
@@ -2392,6 +2217,9 @@ int set_tile_policy(int policy) {
   return tile_policy.exchange(policy, std::memory_order_relaxed);
 }
 
-int fast_splits(int64_t M, int64_t N, int64_t K) { return plan_dsd(M, N, K).splits; }
+int fast_splits(int64_t M, int64_t N, int64_t K) {  // for either operand form
+  const int a = plan_dsd(M, N, K, true).splits, b = plan_dsd(M, N, K, false).splits;
+  return a > b ? a : b;
+}
 
 }  // namespace sd

@@ -1,0 +1,184 @@
+// Launchers of the 64 x 64 ... 128 x 128 tile kernels for one element type; gemm_tile_f16.hip and gemm_tile_bf16.hip
+// compile one each.
+#pragma once
+#include <atomic>
+
+#include "gemm_tile.h"
+#include "gemm_tile_api.h"
+
+namespace sd {
+namespace {
+
+// Shapes.  All of them are bound by what comes through the LDS (about 30 B/clk and CU in, 128 B/clk out); what differs is how
+// much of it a product costs and how many workgroups the output gives.
+//   One   64 x 64 output, 4 + 2 waves, four 16 KB stages, two workgroups per CU: the smallest products, where the number of
+//         workgroups counts (1024^3: 8.7 us forward on 256 of them, 16 us on 64 of the 128 x 128 shape it replaced)
+//   Quad  128 x 128, 8 + 2 waves, four 32 KB stages, a CU each: outputs of up to one round (2048^3 forward 28 -> 22 us,
+//         4096 x 4096 -> 1024: 52 -> 37)
+//   Wide  128 x 128, 8 waves, two stages, two workgroups per CU: more than a round; one workgroup's store runs under
+//         the other's products (16384 x 384 -> 1536 with a GELU in the store: 65 -> 45 us against the 256 x 256 shape)
+// reduction-contiguous operands (forward, dense): one running sum per element
+using FwdOne = TileShape<1, 1, 4, 2, false, 2, 2>;
+using FwdQuad = TileShape<2, 2, 4, 2, false, 4, 2>;
+using FwdWide = TileShape<2, 2, 2, 0, false, 2, 4>;
+// reduction-strided operands (weight gradient): the depth halves apart
+using GradOne = TileShape<1, 1, 4, 2, true, 4, 2>;
+using GradQuad = TileShape<2, 2, 4, 2, true>;
+using GradWide = TileShape<2, 2, 2, 0, true>;
+//   SDD: one row block and 1 / 4 / 2 of its kept column blocks
+using SddOne = TileShape<1, 1, 4, 2, true, 4, 2>;
+using SddStrip = TileShape<1, 4, 3, 2, true>;
+using SddWide = TileShape<1, 2, 2, 0, true>;
+
+template <typename T, bool KC, bool CM, typename S>
+__global__ __launch_bounds__(S::THREADS) void tile_dsd_kernel(GemmArgs g, int tiles_m, int tiles_n, int Mb, int Kb) {
+  tile_dsd_body<T, KC, CM, S>(g, tiles_m, tiles_n, Mb, Kb, (int)blockIdx.x, (int)gridDim.y, (int)blockIdx.y);
+}
+
+template <typename T, typename S>
+__global__ __launch_bounds__(S::THREADS) void tile_sdd_kernel(GemmArgs g, int tiles_n, int Mb, int Cb) {
+  tile_sdd_body<T, S>(g, tiles_n, Mb, Cb, (int)blockIdx.x);
+}
+
+// The forward product and the kept lists of its mask in one launch (see forward_lists_kernel of the large shapes).
+template <typename T, typename S>
+__global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, int tiles_m, int tiles_n, int Mb, int Kb,
+                                                                  int nsplit, int n_gemm, FlatJobs f) {
+  const int bid = (int)blockIdx.x;
+  if (bid < n_gemm) {
+    MaskSrc ms = f.job0.src;
+    ms.resolve();
+    const int tiles = tiles_m * tiles_n;
+    tile_dsd_body<T, true, false, S>(g, tiles_m, tiles_n, Mb, Kb, bid % tiles, nsplit, bid / tiles, &ms);
+  } else {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    flat_lists_block<S::THREADS>(f, bid - n_gemm, reinterpret_cast<int32_t*>(smem));
+  }
+  report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
+}
+
+// Both gradients in one launch: workgroups [0, n_dx) are the input gradient's (a multiple of 8, so that the second
+// product's tile map keeps its XCD assignment), the rest the weight gradient's.
+template <typename T, typename X, typename W>
+__global__ __launch_bounds__(W::THREADS) void tile_pair_kernel(GemmArgs gx, int x_tiles_n, int x_Mb, int x_Cb, int n_dx,
+                                                               GemmArgs gw, int w_tiles_m, int w_tiles_n, int w_Mb,
+                                                               int w_Kb, int w_splits) {
+  static_assert(X::THREADS == W::THREADS, "both products run on the same number of threads");
+  const int bid = (int)blockIdx.x;
+  if (bid < n_dx) {
+    if (bid < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_tiles_n, x_Mb, x_Cb, bid);
+  } else {
+    const int wb = bid - n_dx, tiles = w_tiles_m * w_tiles_n;
+    tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, wb % tiles, w_splits, wb / tiles);
+  }
+}
+
+// Raises a kernel's dynamic LDS limit once per device; `done` is the caller's per-kernel record.
+int allow_lds(const void* kernel, int bytes, std::atomic<bool> (&done)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
+    return fail(SD_ERR_RUNTIME, "hipGetDevice failed or device index out of range");
+  if (!done[dev].load(std::memory_order_acquire)) {
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return fail(SD_ERR_RUNTIME, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    done[dev].store(true, std::memory_order_release);
+  }
+  return SD_OK;
+}
+
+int blocks_of(int64_t n) { return (int)((n + BS - 1) / BS); }
+
+template <typename T, bool KC, bool CM, typename S>
+int dsd_launch(const GemmArgs& g, int splits, hipStream_t stream) {
+  static std::atomic<bool> done[64] = {};
+  auto* kernel = &tile_dsd_kernel<T, KC, CM, S>;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
+  const int Mb = blocks_of(g.M), Kb = blocks_of(g.K), tm = (Mb + S::R - 1) / S::R, tn = (blocks_of(g.N) + S::C - 1) / S::C;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tm * tn), (unsigned)splits), dim3(S::THREADS), S::SMEM, stream, g, tm, tn, Mb, Kb);
+  return check_launch("tile_dsd_kernel");
+}
+
+template <typename T, typename S>
+int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
+  static std::atomic<bool> done[64] = {};
+  auto* kernel = &tile_forward_kernel<T, S>;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
+  const int Mb = blocks_of(g.M), Kb = blocks_of(g.K), tm = (Mb + S::R - 1) / S::R, tn = (blocks_of(g.N) + S::C - 1) / S::C;
+  const int n_gemm = tm * tn * splits;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::SMEM, stream, g, tm, tn, Mb, Kb,
+                     splits, n_gemm, f);
+  return check_launch("tile_forward_kernel");
+}
+
+template <typename T, typename S>
+int sdd_launch(const GemmArgs& g, hipStream_t stream) {
+  static std::atomic<bool> done[64] = {};
+  auto* kernel = &tile_sdd_kernel<T, S>;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
+  const int Mb = blocks_of(g.M), Cb = blocks_of(g.N), tn = (Cb + S::C - 1) / S::C;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(Mb * tn)), dim3(S::THREADS), S::SMEM, stream, g, tn, Mb, Cb);
+  return check_launch("tile_sdd_kernel");
+}
+
+template <typename T, typename X, typename W>
+int pair_launch(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_t stream) {
+  static std::atomic<bool> done[64] = {};
+  constexpr int SMEM = X::SMEM > W::SMEM ? X::SMEM : W::SMEM;
+  auto* kernel = &tile_pair_kernel<T, X, W>;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), SMEM, done)) return rc;
+  const int x_Mb = blocks_of(gx.M), x_Cb = blocks_of(gx.N), x_tn = (x_Cb + X::C - 1) / X::C;
+  const int n_dx = (x_Mb * x_tn + 7) / 8 * 8;
+  const int w_Mb = blocks_of(gw.M), w_Kb = blocks_of(gw.K), w_tm = (w_Mb + W::R - 1) / W::R, w_tn = (blocks_of(gw.N) + W::C - 1) / W::C;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_dx + w_tm * w_tn * splits)), dim3(W::THREADS), SMEM, stream, gx, x_tn, x_Mb,
+                     x_Cb, n_dx, gw, w_tm, w_tn, w_Mb, w_Kb, splits);
+  return check_launch("tile_pair_kernel");
+}
+
+template <typename T, bool KC, bool CM>
+int dsd_shape(const GemmArgs& g, int shape, int splits, hipStream_t stream) {
+  switch (shape) {
+    case kShapeOne: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdOne, GradOne>>(g, splits, stream);
+    case kShapeQuad: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdQuad, GradQuad>>(g, splits, stream);
+    default: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdWide, GradWide>>(g, splits, stream);
+  }
+}
+
+}  // namespace
+
+template <typename T>
+int tile_dsd(const GemmArgs& g, bool kc, bool cm, int shape, int splits, hipStream_t stream) {
+  if (kc) return cm ? dsd_shape<T, true, true>(g, shape, splits, stream) : dsd_shape<T, true, false>(g, shape, splits, stream);
+  return cm ? dsd_shape<T, false, true>(g, shape, splits, stream) : dsd_shape<T, false, false>(g, shape, splits, stream);
+}
+
+template <typename T>
+int tile_forward(const GemmArgs& g, int shape, int splits, const FlatJobs& f, hipStream_t stream) {
+  switch (shape) {
+    case kShapeOne: return forward_launch<T, FwdOne>(g, splits, f, stream);
+    case kShapeQuad: return forward_launch<T, FwdQuad>(g, splits, f, stream);
+    default: return forward_launch<T, FwdWide>(g, splits, f, stream);
+  }
+}
+
+template <typename T>
+int tile_sdd(const GemmArgs& g, int shape, hipStream_t stream) {
+  switch (shape) {
+    case kShapeOne: return sdd_launch<T, SddOne>(g, stream);
+    case kShapeQuad: return sdd_launch<T, SddStrip>(g, stream);
+    default: return sdd_launch<T, SddWide>(g, stream);
+  }
+}
+
+template <typename T>
+int tile_pair(const GemmArgs& gx, const GemmArgs& gw, int shape, int splits, hipStream_t stream) {
+  return shape == kShapeOne ? pair_launch<T, SddOne, GradOne>(gx, gw, splits, stream)
+                            : pair_launch<T, SddStrip, GradQuad>(gx, gw, splits, stream);
+}
+
+#define SD_TILE_INSTANCES(T)                                                                    \
+  template int tile_dsd<T>(const GemmArgs&, bool, bool, int, int, hipStream_t);                 \
+  template int tile_forward<T>(const GemmArgs&, int, int, const FlatJobs&, hipStream_t);        \
+  template int tile_sdd<T>(const GemmArgs&, int, hipStream_t);                                  \
+  template int tile_pair<T>(const GemmArgs&, const GemmArgs&, int, int, hipStream_t);
+
+}  // namespace sd

@@ -1,0 +1,79 @@
+"""The 64 x 64 and 128 x 128 tile kernels at the sizes where they can go wrong: one step, fewer steps than stages, one more
+than a full round of stages, ragged last blocks in every extent, widths that are not multiples of 8, row blocks and
+tiles without a kept block, quadrant masks, split reductions."""
+import numpy as np
+import pytest
+import torch
+
+from _util import REL_FRO_TOL, cpu_mask, make_operand, max_tile_rel_fro, to_np
+from oracle import sparsedrop_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K,bs,p", [
+    (64, 64, 64, 64, 0.0),         # one workgroup, one step
+    (65, 72, 72, 64, 0.4),         # one past a tile everywhere
+    (127, 136, 200, 64, 0.5),      # fewer steps than stages, ragged last step
+    (190, 200, 328, 32, 0.6),      # quadrant keep bits, ragged everywhere
+    (1, 8, 264, 64, 0.3),          # a single row
+    (300, 1096, 1032, 64, 0.95),   # row blocks with nothing kept; the first extent past the 64 x 64 shape's round
+    (1100, 1288, 520, 96, 0.3),    # 128 x 128 tiles, an odd multiple of 32
+    (2200, 2056, 136, 64, 0.2),    # more than a round of 128 x 128 tiles
+    (72, 200, 16456, 64, 0.5),     # long reduction, few tiles: split in the forward and in the weight gradient
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_products_on_the_tile_shapes(M, N, K, bs, p, dtype):
+    """Forward, dX and dW of a layer X[M, K] -> N against the fp32 oracle on the same rounded operands, per 64-tile.
+    The bar is the suite's relative Frobenius one; sums are fp32 and rounded once, so it has orders of magnitude of room."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(M * 7 + N * 3 + K + bs)
+    x = make_operand(M, K, dtype, "cuda", gen=gen)
+    w = make_operand(N, K, dtype, "cuda", scale=K ** -0.5, gen=gen)
+    dy = make_operand(M, N, dtype, "cuda", gen=gen)
+    mask = cpu_mask(O.mask_shape(M, K, bs), p, gen)
+    mk = mask.numpy()
+    y, _, lists, kbs = ext.dropout_matmul_forward(x, w, bs, p, mask=mask.cuda())
+    assert ext.last_kernel() == "specialised"
+    dx, dw = ext.dropout_matmul_backward(dy, w, x, lists, kbs, p)
+    assert ext.last_kernel() == "specialised"
+    xn, wn, dyn = to_np(x), to_np(w), to_np(dy)
+    for got, ref, what in ((y, O.dsd_forward(xn, wn, mk, bs, p, np.float32), "y"),
+                           (dx, O.sdd_dx(dyn, wn, mk, bs, p, np.float32), "dx"),
+                           (dw, O.dsd_dw(dyn, xn, mk, bs, p, np.float32), "dw")):
+        assert max_tile_rel_fro(got, ref) <= REL_FRO_TOL, what
+    keep = O.expand_keep(mk, bs, M, K)
+    assert (dx.float().cpu().numpy()[~keep] == 0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 13, 64), (200, 77, 136), (515, 301, 264)])
+@pytest.mark.parametrize("act", ["relu", "gelu"])
+def test_unaligned_output_rows(M, N, K, act):
+    """Output rows that start at any 2-byte boundary (N odd), with the activation and its pre-activation in the store;
+    kept-only and zeroed SDD tiles into such rows."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(M + N)
+    x = make_operand(M, K, torch.float16, "cuda", gen=gen)
+    w = make_operand(N, K, torch.float16, "cuda", scale=K ** -0.5, gen=gen)
+    mask = cpu_mask(O.mask_shape(M, K, 64), 0.4, gen)
+    lists = ext.build_lists(mask.cuda())
+    got, pre = ext.gemm_dsd_lists_act(x, w, lists, 64, 2.0, act, want_pre=True)
+    assert ext.last_kernel() == "specialised"
+    ref = O.gemm_dsd(to_np(x), to_np(w), mask.numpy(), 64, 2.0, np.float32)
+    assert max_tile_rel_fro(pre, ref) <= REL_FRO_TOL
+    t = torch.from_numpy(np.asarray(ref))
+    assert max_tile_rel_fro(got, (torch.relu(t) if act == "relu" else torch.nn.functional.gelu(t)).numpy()) <= REL_FRO_TOL
+    # SDD into odd rows: B is [N, K] with its reduction index strided, in rows wide enough for 16-byte loads
+    wide = torch.randn(K, -(-N // 8) * 8, generator=gen).half().cuda()
+    b = wide[:, :N].t()
+    mask = cpu_mask(O.mask_shape(M, N, 64), 0.5, gen)
+    lists = ext.build_lists(mask.cuda())
+    out = torch.full((M, N), 7.0, dtype=torch.float16, device="cuda")
+    ext.gemm_sdd_lists(x, b, lists, 64, 0.5, out=out)
+    assert ext.last_kernel() == "specialised"
+    assert max_tile_rel_fro(out, O.gemm_sdd(to_np(x), to_np(b), mask.numpy(), 64, 0.5, np.float32)) <= REL_FRO_TOL
+    assert (out.cpu().numpy()[~O.expand_keep(mask.numpy(), 64, M, N)] == 0).all()
