@@ -165,6 +165,12 @@ int sd_random_lists_state(uint64_t* state, float p, int64_t mb, int64_t kb, uint
                           int64_t out_mb, int64_t out_kb, int32_t* row_ptr, int32_t* col_idx, int32_t* col_ptr,
                           int32_t* row_idx, void* stream);
 
+/* Copies up to four row-major matrices into rows that start on 16-byte boundaries and end in zeros, in one launch:
+ * matrix i is rows[i] x cols[i] with pitch ld[i] (elements, 16-bit, any alignment); dst[i] (16-byte aligned) receives
+ * dst_rows[i] x dst_ld[i] elements, dst_ld[i] a multiple of 8, everything outside the source zero. */
+int sd_pad_rows(int n, const void* const* src, const int64_t* ld, const int64_t* rows, const int64_t* cols,
+                void* const* dst, const int64_t* dst_rows, const int64_t* dst_ld, void* stream);
+
 /* Pointer-increment table of flash_dropout/functional/utils.py:19-69 from a CSR list:
  * table[i] = col_idx[i]*block_k for the first kept block of a row, else (col_idx[i]-col_idx[i-1])*block_k;
  * row_indices[r] = row_ptr[r]; row_widths[r] = row_ptr[r+1]-row_ptr[r].
