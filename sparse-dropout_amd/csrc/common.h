@@ -60,6 +60,7 @@ struct F16 {
     _Float16 h = (_Float16)x;
     return __builtin_bit_cast(uint16_t, h);
   }
+  __device__ static inline uint32_t pack2(float lo, float hi) { return from_float(lo) | ((uint32_t)from_float(hi) << 16); }
   __device__ static inline float to_float(uint16_t v) { return (float)__builtin_bit_cast(_Float16, v); }
   // D(32x32) += A(32x16) * B(16x32); lane l supplies row/col l%32, k = 8*(l/32)..+7 of its operand.
   __device__ static inline f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
@@ -78,6 +79,11 @@ struct BF16 {
   __device__ static inline uint16_t from_float(float x) {
     __bf16 h = (__bf16)x;
     return __builtin_bit_cast(uint16_t, h);
+  }
+  __device__ static inline uint32_t pack2(float lo, float hi) {  // one conversion for the pair
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
   }
   __device__ static inline float to_float(uint16_t v) {
     return __builtin_bit_cast(float, (uint32_t)v << 16);
@@ -251,24 +257,35 @@ __device__ inline void store_eight(const GemmArgs& g, const StoreLayout& s, int6
     return;
   }
   auto pack = [&](const float (&v)[8]) {
-    return u32x4{(uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16),
-                 (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16),
-                 (uint32_t)T::from_float(v[4]) | ((uint32_t)T::from_float(v[5]) << 16),
-                 (uint32_t)T::from_float(v[6]) | ((uint32_t)T::from_float(v[7]) << 16)};
+    return u32x4{T::pack2(v[0], v[1]), T::pack2(v[2], v[3]), T::pack2(v[4], v[5]), T::pack2(v[6], v[7])};
   };
+  // The activation is chosen once for the eight and every element is computed without a branch, so that the exponentials
+  // and reciprocals of the eight overlap: input gradient of 16384 x 1536 from 384 with GELU's derivative 85 -> 71 us (47
+  // without an activation) against a chain per element under its own execution mask, of 16384 x 1024 from 256 40 -> 33.
   if (g.act != SD_ACT_NONE) {
     if (SDD) {
       const u32x4 a = *reinterpret_cast<const u32x4_any*>(g.aux + si * s.ald + ci);
       const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+      float at[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint16_t h = (uint16_t)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu);
-        if (r[i] != 0.f) r[i] *= act_derivative(g.act, T::to_float(h));  // dropped tiles stay exact zeros
-      }
+      for (int i = 0; i < 8; ++i) at[i] = T::to_float((uint16_t)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu));
+      auto times = [&](int act) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float d = r[i] * act_derivative(act, at[i]);
+          r[i] = r[i] != 0.f ? d : r[i];  // dropped tiles stay exact zeros
+        }
+      };
+      if (g.act == SD_ACT_GELU) times(SD_ACT_GELU);
+      else times(SD_ACT_RELU);
     } else {
       if (s.has_aux) *reinterpret_cast<u32x4_any*>(g.aux + si * s.ald + ci) = pack(r);
+      auto apply = [&](int act) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) r[i] = act_apply(g.act, r[i]);
+        for (int i = 0; i < 8; ++i) r[i] = act_apply(act, r[i]);
+      };
+      if (g.act == SD_ACT_GELU) apply(SD_ACT_GELU);
+      else apply(SD_ACT_RELU);
     }
   }
   *reinterpret_cast<u32x4_any*>(g.c + si * s.ld + ci) = pack(r);
