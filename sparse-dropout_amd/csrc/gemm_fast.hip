@@ -1877,16 +1877,34 @@ bool sdd_big_ok(const GemmArgs& g) {
          blocks_of(g.N) <= G_MAX_CB;
 }
 
+// Whether the strips of two beat the big shape on a short reduction, where what counts is how the grid fills its rounds
+// and whose store runs under other products.  Fitted (us) to sizes of 2048 to 16384 rows and 1024 to 8192 columns over
+// reductions of 256 to 2048 at p = 0.1, 0.3, 0.5, without and with GELU's derivative: the big shape takes whole rounds of
+// 256 groups whatever is kept, the strips (three to a CU) as many rounds as there are kept tiles.  With the derivative at
+// p = 0.1 / 0.5, big against strips: 16384 x 1536 from 384 (a round and a half) 71 / 64 us, 65 / 45; 16384 x 1024 from 256
+// (one round) 33 / 32, 36 / 28; 4096 x 4096 from 1024 58 / 51, 67 / 47; from 2048 75 / 70, 102 / 75: deeper ones are the
+// big shape's, and so are masks of 32-blocks, which were not measured.
+bool strips_beat_big(const GemmArgs& g) {
+  const double kb = (double)blocks_of(g.K), kept = (double)(blocks_of(g.M) * blocks_of(g.N)) * kept_fraction(g);
+  if (kb > 32 || g.quads || !g.row_ptr) return false;
+  const bool gelu = g.act == SD_ACT_GELU;
+  const double rounds = (double)((sdd_big_groups(g) + 255) / 256), strip_rounds = kept / 1536.0;
+  const double big = rounds * (15.0 + 1.5 * kb) * (rounds >= 4 ? 0.9 : 1.0) + (gelu ? 11.0 * rounds : 0.0);
+  const double strips = 10.0 + (strip_rounds + 0.5) * (2.0 + 0.95 * kb) * (strip_rounds > 4.0 ? 1.2 : 1.0) + (gelu ? 0.0036 * kept : 0.0);
+  return strips < 0.95 * big;
+}
+
 // The big shape when its grid gives more than half of the CUs a workgroup (on aligned operands: its edge instance runs
-// the older loop); else by the number of kept tiles: up to about one 64 x 64 tile per CU one to a workgroup, else
+// the older loop), unless strips of two are faster and nothing wants the big shape (`with_big`: a weight gradient on it
+// shares the launch); else by the number of kept tiles: up to about one 64 x 64 tile per CU one to a workgroup, else
 // strips of four while their grid is at most two rounds, else strips of two, three workgroups to a CU.
-int plan_sdd(const GemmArgs& g) {
+int plan_sdd(const GemmArgs& g, bool with_big = false) {
   const int policy = tile_policy.load(std::memory_order_relaxed);
   const int64_t Mb = blocks_of(g.M), Cb = blocks_of(g.N);
   const bool ragged = g.N % BS || g.K % BS;
   if (sdd_big_ok(g)) {
     if (policy == kTileBig) return kShapeBig;
-    if (policy == kTileAuto && !ragged && sdd_big_groups(g) > 128) return kShapeBig;
+    if (policy == kTileAuto && !ragged && sdd_big_groups(g) > 128) return !with_big && strips_beat_big(g) ? kShapeWide : kShapeBig;
   }
   if (policy == kTileMid) return kShapeWide;
   if ((double)(Mb * Cb) * kept_fraction(g) <= 320.0) return kShapeOne;
@@ -2183,7 +2201,7 @@ int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipS
   if (!gw.row_ptr || gw.bs != BS || gw.act || !form.ok || form.kc || !form.cm || gw.c_sr != 1) return SD_ERR_UNSUPPORTED;
   const DsdPlan plan = plan_for(gw, form);
   if (plan.splits < 1) return SD_ERR_UNSUPPORTED;
-  const int x_shape = plan_sdd(gx);
+  const int x_shape = plan_sdd(gx, plan.shape == kShapeBig);
   // Worth it only while neither product fills the chip by itself: side by side, two large products get in each
   // other's way in the L2 (8192^3 at p = 0.5: 1.33 ms in one launch against 1.28 in two; 1024^3: 27 us against 46).
   if (x_shape == kShapeBig || plan.shape == kShapeBig) {

@@ -77,3 +77,30 @@ def test_unaligned_output_rows(M, N, K, act):
     assert ext.last_kernel() == "specialised"
     assert max_tile_rel_fro(out, O.gemm_sdd(to_np(x), to_np(b), mask.numpy(), 64, 0.5, np.float32)) <= REL_FRO_TOL
     assert (out.cpu().numpy()[~O.expand_keep(mask.numpy(), 64, M, N)] == 0).all()
+
+
+@pytest.mark.parametrize("act", [None, "gelu"])
+def test_input_gradient_of_a_short_reduction(act):
+    """A grid of one and a half rounds of the big shape, which strips of two take over.  Reference in fp32 on the same
+    rounded operands; one rounding to bf16 (2^-9 relative on average of at most 2^-8)."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    M, C, K = 4096, 6144, 200
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    dy, w, at = (torch.randn(*s, generator=gen, device="cuda").bfloat16() for s in ((M, K), (K, C), (M, C)))
+    mask = torch.rand(M // 64, C // 64, generator=gen, device="cuda") < 0.5
+    lists = ext.build_lists(mask)
+    for k in (192, K):  # aligned reduction; a ragged one, which stays where it was
+        a, b = dy[:, :k].contiguous(), w[:k].contiguous()
+        if act:
+            got = ext.gemm_sdd_lists_actgrad(a, b.t(), lists, 64, 2.0, act, at, keep_hint=0.5)
+        else:
+            got = ext.gemm_sdd_lists(a, b.t(), lists, 64, 2.0, keep_hint=0.5)
+        assert k != 192 or ext.last_kernel_detail() == "sdd:mid"
+        ref = 2.0 * (a.float() @ b.float())
+        if act:
+            t = at.float()
+            ref *= 0.5 * (1 + torch.erf(t * 0.5 ** 0.5)) + t * torch.exp(-0.5 * t * t) * 0.3989422804014327
+        ref *= (~mask).repeat_interleave(64, 0).repeat_interleave(64, 1)
+        assert (got[ref == 0] == 0).all() and (got.float() - ref).norm() <= 2.0 ** -8 * ref.norm()
