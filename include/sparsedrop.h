@@ -171,6 +171,10 @@ int sd_random_lists_state(uint64_t* state, float p, int64_t mb, int64_t kb, uint
 int sd_pad_rows(int n, const void* const* src, const int64_t* ld, const int64_t* rows, const int64_t* cols,
                 void* const* dst, const int64_t* dst_rows, const int64_t* dst_ld, void* stream);
 
+/* Row-major [n * p, c] matrix of an image tensor stored plane by plane: dst[(i * p + j) * c + k] = src[i * sn + k * sc + j]
+ * (16-bit elements, any alignment; dst contiguous). */
+int sd_rows_from_planes(const void* src, int64_t sn, int64_t sc, void* dst, int64_t n, int64_t c, int64_t p, void* stream);
+
 /* Pointer-increment table of flash_dropout/functional/utils.py:19-69 from a CSR list:
  * table[i] = col_idx[i]*block_k for the first kept block of a row, else (col_idx[i]-col_idx[i-1])*block_k;
  * row_indices[r] = row_ptr[r]; row_widths[r] = row_ptr[r+1]-row_ptr[r].

@@ -1,4 +1,5 @@
-// Operands brought into the layout the GEMM kernels load: rows that start on 16-byte boundaries and end in zeros.
+// Operands brought into the layout the GEMM kernels load: rows that start on 16-byte boundaries and end in zeros, and
+// the rows [N*P*Q, K] of an image tensor stored plane by plane.
 #include "common.h"
 
 namespace sd {
@@ -47,6 +48,69 @@ __global__ __launch_bounds__(kPadThreads) void pad_rows_kernel(PadJobs js) {
   reinterpret_cast<u32x4*>(p.dst)[piece] = v;
 }
 
+constexpr int kTurn = 64;               // a workgroup turns a 64 x 64 tile
+constexpr int kTurnLd = kTurn + 2;      // halfs per LDS row: 33 words, so that the reads down a column hit every bank once
+
+// dst[(n * P + i) * C + c] = src[n * sn + c * sc + i], i < P.  Bound by its reads and writes (a 64 MB copy at 128 images
+// of 128 x 32 x 32): both sides move in 128-byte pieces, 16 bytes per lane, and the tile is turned in LDS.  The
+// elementwise copy it replaces reads 2 bytes per lane, a plane apart.
+__global__ __launch_bounds__(256) void rows_from_planes_kernel(const uint16_t* __restrict__ src, int64_t sn, int64_t sc,
+                                                               uint16_t* __restrict__ dst, int C, int P, int tiles_c,
+                                                               int tiles_p) {
+  __shared__ __attribute__((aligned(4))) uint16_t tile[kTurn * kTurnLd];  // [c][i]
+  const int t = threadIdx.x;
+  const uint32_t b = blockIdx.x;
+  const int tc = (int)(b % (uint32_t)tiles_c);
+  const uint32_t rest = b / (uint32_t)tiles_c;
+  const int tp = (int)(rest % (uint32_t)tiles_p);
+  const int64_t n = rest / (uint32_t)tiles_p;
+  const int c0 = tc * kTurn, i0 = tp * kTurn;
+  const int row = t / 8, ch = (t % 8) * 8;
+  u32x4 v[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = c0 + row + 32 * k, left = P - (i0 + ch);
+    v[k] = u32x4{0u, 0u, 0u, 0u};
+    if (c < C && left > 0) {
+      const uint16_t* s = src + n * sn + (int64_t)c * sc + i0 + ch;
+      if (left >= 8) {
+        v[k] = *reinterpret_cast<const u32x4_any*>(s);
+      } else {
+        uint32_t h[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) h[i] = i < left ? s[i] : 0u;
+        v[k] = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    uint32_t* d = reinterpret_cast<uint32_t*>(tile + (row + 32 * k) * kTurnLd + ch);
+    d[0] = v[k].x;
+    d[1] = v[k].y;
+    d[2] = v[k].z;
+    d[3] = v[k].w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int il = row + 32 * k, left = C - (c0 + ch);
+    if (i0 + il >= P || left <= 0) continue;
+    uint16_t h[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) h[j] = tile[(ch + j) * kTurnLd + il];
+    uint16_t* d = dst + (n * P + i0 + il) * (int64_t)C + c0 + ch;
+    if (left >= 8) {
+      *reinterpret_cast<u32x4_any*>(d) = u32x4{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16),
+                                               h[4] | ((uint32_t)h[5] << 16), h[6] | ((uint32_t)h[7] << 16)};
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < left) d[j] = h[j];
+    }
+  }
+}
+
 }  // namespace
 }  // namespace sd
 
@@ -76,4 +140,18 @@ extern "C" int sd_pad_rows(int n, const void* const* src, const int64_t* ld, con
   SD_REQUIRE(blocks < (1ull << 31), "pad_rows: too large");
   hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)blocks), dim3(kPadThreads), 0, (hipStream_t)stream, js);
   return check_launch("pad_rows_kernel");
+}
+
+extern "C" int sd_rows_from_planes(const void* src, int64_t sn, int64_t sc, void* dst, int64_t n, int64_t c, int64_t p,
+                                   void* stream) {
+  SD_REQUIRE(n >= 0 && c >= 0 && p >= 0, "rows_from_planes: negative size");
+  if (n == 0 || c == 0 || p == 0) return SD_OK;
+  SD_REQUIRE(src && dst, "rows_from_planes: null pointer");
+  SD_REQUIRE(c < (1LL << 31) && p < (1LL << 31) - kTurn && n < (1LL << 31), "rows_from_planes: too large");
+  const int64_t tiles_c = ceil_div(c, kTurn), tiles_p = ceil_div(p, kTurn);
+  SD_REQUIRE(tiles_c * tiles_p < (1LL << 31) && tiles_c * tiles_p * n < (1LL << 31), "rows_from_planes: too large");
+  hipLaunchKernelGGL(rows_from_planes_kernel, dim3((unsigned)(tiles_c * tiles_p * n)), dim3(256), 0, (hipStream_t)stream,
+                     static_cast<const uint16_t*>(src), sn, sc, static_cast<uint16_t*>(dst), (int)c, (int)p, (int)tiles_c,
+                     (int)tiles_p);
+  return check_launch("rows_from_planes_kernel");
 }

@@ -629,6 +629,14 @@ Tensor conv_dx(const Tensor& dy2, const Tensor& w2, const ConvGeom& g, const Lis
 // (N, K, P, Q) gradient -> [N*P*Q, K] row-major (free when it is channels-last in memory)
 Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) {
   Tensor d = grad.scalar_type() == like.scalar_type() ? grad : grad.to(like.scalar_type());
+  const bool planes = d.stride(3) == 1 && (d.size(2) == 1 || d.stride(2) == d.size(3)) && d.stride(1) >= g.po * g.qo;
+  if (planes && g.k > 1 && g.po * g.qo > 1) {
+    Tensor rows = new_matrix(d, g.rows(), g.k);
+    c10::DeviceGuard guard(d.device());
+    check(sd_rows_from_planes(d.data_ptr(), d.stride(0), d.stride(1), rows.data_ptr(), g.n, g.k, g.po * g.qo, stream_of(d)),
+          "sd_rows_from_planes");
+    return rows;
+  }
   d = d.permute({0, 2, 3, 1}).reshape({g.rows(), g.k});
   if (d.stride(1) != 1 || d.stride(0) < g.k) d = d.contiguous();  // e.g. the expanded (stride 0) gradient of a sum()
   return d;
