@@ -8,6 +8,8 @@
 // q while reading (consecutive pixels of an image row), the 64x64 tile is turned in LDS, and lanes run
 // along the column index while writing, so both sides are coalesced.  With a kept-block list only
 // kept blocks are produced: dropped blocks are never read by the DSD kernels, so they are not written.
+#include <type_traits>
+
 #include "common.h"
 
 namespace sd {
@@ -115,49 +117,78 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict_
   }
 }
 
-// Patch-staged variant for the common case that the 64 rows of a workgroup lie in one image
-// ((P*Q) % 64 == 0): per 64-column tile the (at most 64/(R*S) + 2) input channels it touches are copied
-// once into LDS as a zero-padded patch [channel][input row][padded input column]; every output element
-// is then an LDS read with no bounds check, and a thread assembles 8 consecutive columns of one row
-// into a single 16-byte store.  Global reads drop to the unique bytes, global writes are full lines.
+// Patch-staged variant: what the 64 rows of a workgroup read is copied into LDS once, zero-padded, and every output
+// element is then an LDS read with no bounds check; a thread assembles 8 consecutive columns of one row into a single
+// 16-byte store.  Global reads drop to the unique bytes, global writes are full lines.
+//  * Row space of the copy: the output rows (n, p) that the group touches belong to one image or to consecutive ones
+//    (28 x 28 images: 784 positions are 12 groups and a quarter); each image's share gets the input rows it reads,
+//    one behind the other, listed in `src_row` once per workgroup.  Nothing ties the image size to the group.
+//  * Column space: `tpg` column tiles' channels are staged at a time (all of them where they fit), with one barrier pair
+//    per group of tiles; the tiles themselves follow without barriers.
+// 256 x 32 x 28 x 28, 3 x 3, p = 0.25: 126 us on im2col_kernel, 46 here; 70 x 64 x 56 x 56, p = 0.5: 102 with the image's
+// channels staged tile by tile, 90.
 constexpr int PATCH_MAX_BYTES = 48 * 1024;
+constexpr int PATCH_ROWS_MAX = 256;
 
 __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __restrict__ x,
                                                            uint16_t* __restrict__ cols, int64_t ld,
                                                            ConvGeom g, const int32_t* row_ptr,
-                                                           const int32_t* col_idx, int bs, int hp,
-                                                           int wp, int max_ch) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t patch[];  // [max_ch][hp][wp]
-  __shared__ int col_off[TILE];  // patch offset of each column of the tile (0 past the last column: never stored)
+                                                           const int32_t* col_idx, int bs, int wp,
+                                                           int tpg) {
+  extern __shared__ __attribute__((aligned(16))) char patch_mem[];
+  int* col_off = reinterpret_cast<int*>(patch_mem);                     // [tpg * 64]: offset of a column in the copy
+  uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp]
+  __shared__ int64_t src_row[PATCH_ROWS_MAX];  // element offset of an input row in x (channel 0), -1: zeros
   const int t = threadIdx.x;
   const int ncols = g.c * g.r * g.s;
   const int rs_n = g.r * g.s;
   const int pq = g.p * g.q;
+  const int64_t rows = (int64_t)g.n * pq;
   const int64_t r0 = (int64_t)blockIdx.x * TILE;
-  const int n_i = (int)(r0 / pq);
-  const int pq0 = (int)(r0 % pq);
-  const int p_lo = pq0 / g.q;
-  const int h_lo = p_lo * g.str_h - g.pad_h;  // input row of patch row 0
-  const uint16_t* xn = x + (int64_t)n_i * g.xs_n;
+  const int64_t r_last = (r0 + TILE < rows ? r0 + TILE : rows) - 1;
+  const int n_lo = (int)(r0 / pq), n_hi = (int)(r_last / pq);
+  const int p_first = (int)(r0 - (int64_t)n_lo * pq) / g.q;  // of image n_lo
+  const int p_last = (int)(r_last - (int64_t)n_hi * pq) / g.q;
+  const int reach = (g.r - 1) * g.dil_h + 1;
+  // input rows of one image's output rows [pa, pb]
+  auto in_rows = [&](int pa, int pb) { return (pb - pa) * g.str_h + reach; };
+  const int hp_first = in_rows(p_first, n_lo == n_hi ? p_last : g.p - 1), hp_whole = in_rows(0, g.p - 1);
+  const int hp = n_lo == n_hi ? hp_first : hp_first + (n_hi - n_lo - 1) * hp_whole + in_rows(0, p_last);
+  // where image n's share starts
+  auto base_of = [&](int n) { return n == n_lo ? 0 : hp_first + (n - n_lo - 1) * hp_whole; };
 
-  // per-thread output rows (two per tile): patch offset of their top-left tap
+  for (int i = t; i < hp; i += 256) {
+    int n = n_lo, k = i;
+    if (k >= hp_first) {
+      k -= hp_first;
+      n += 1 + k / hp_whole;
+      k %= hp_whole;
+    }
+    const int hh = (n == n_lo ? p_first : 0) * g.str_h - g.pad_h + k;
+    src_row[i] = hh >= 0 && hh < g.h ? (int64_t)n * g.xs_n + (int64_t)hh * g.xs_h : -1;
+  }
+  // per-thread output rows (two per tile): offset of their top-left tap in a channel's plane of the copy
   int row_off[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int row_l = t / 8 + 32 * i;
-    const int pql = pq0 + row_l;
-    row_off[i] = ((pql / g.q - p_lo) * g.str_h) * wp + (pql % g.q) * g.str_w;
+    const int64_t row = r0 + t / 8 + 32 * i;
+    row_off[i] = 0;
+    if (row < rows) {
+      const int n = (int)(row / pq), at = (int)(row - (int64_t)n * pq), pp = at / g.q;
+      row_off[i] = (base_of(n) + (pp - (n == n_lo ? p_first : 0)) * g.str_h) * wp + (at - pp * g.q) * g.str_w;
+    }
   }
 
   const int sub_per_block = bs / TILE;
   const int ntiles = (ncols + TILE - 1) / TILE;
+  const int per_ch = hp * wp;
   int32_t pos = 0, end = 0;
   if (row_ptr) {
     const int64_t rb = r0 / bs;
     pos = row_ptr[rb];
     end = row_ptr[rb + 1];
   }
-  int sub = 0, ct = -1;
+  int sub = 0, ct = -1, group = -1;
   for (;;) {
     if (row_ptr) {
       if (pos >= end) break;
@@ -167,41 +198,81 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
     } else {
       if (++ct >= ntiles) break;
     }
-    const int c0 = ct * TILE;
-    const int ch_lo = c0 / rs_n;
-    const int last = (c0 + TILE - 1 < ncols ? c0 + TILE - 1 : ncols - 1);
-    const int nch = last / rs_n - ch_lo + 1;
-    // stage the patch: lanes along the padded input column
-    const int per_ch = hp * wp;
-    for (int e = t; e < nch * per_ch; e += 256) {
-      const int ci = e / per_ch, rem = e - ci * per_ch;
-      const int hh = h_lo + rem / wp, ww = rem % wp - g.pad_w;
-      uint16_t v = 0;
-      if (hh >= 0 && hh < g.h && ww >= 0 && ww < g.w)
-        v = xn[(int64_t)(ch_lo + ci) * g.xs_c + (int64_t)hh * g.xs_h + (int64_t)ww * g.xs_w];
-      patch[e] = v;
-    }
-    if (t < TILE) {
-      const int col = c0 + t;
-      int off = 0;
-      if (col < ncols) {
-        const int ci = col / rs_n, rs = col - ci * rs_n;
-        off = ((ci - ch_lo) * hp + (rs / g.s) * g.dil_h) * wp + (rs % g.s) * g.dil_w;
+    if (ct / tpg != group) {  // the same for every thread
+      group = ct / tpg;
+      const int g0 = group * tpg * TILE, g_end = g0 + tpg * TILE < ncols ? g0 + tpg * TILE : ncols;
+      const int ch_lo = g0 / rs_n, nch = (g_end - 1) / rs_n - ch_lo + 1;
+      __syncthreads();  // src_row is written; nobody reads the previous group's copy any more
+      // A channels-last image is read along the channels, any other along its rows, LW lanes to a line and four lines'
+      // loads ahead of their stores.  Copying costs instructions, not bytes: no division per line along the rows.
+      if (g.xs_c == 1 && g.xs_w != 1) {
+        for (int ci = t % 32; ci < nch; ci += 32)
+          for (int line0 = t / 32; line0 < per_ch; line0 += 32) {
+            uint16_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const int line = line0 + 8 * k;
+              v[k] = 0;
+              if (line < per_ch) {
+                const int hr = line / wp, ww = line - hr * wp - g.pad_w;
+                const int64_t so = src_row[hr];
+                if (so >= 0 && ww >= 0 && ww < g.w) v[k] = x[so + (int64_t)ww * g.xs_w + ch_lo + ci];
+              }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (line0 + 8 * k < per_ch) patch[ci * per_ch + line0 + 8 * k] = v[k];
+          }
+      } else {
+        auto along_rows = [&](auto lanes) {
+          constexpr int LW = decltype(lanes)::value;
+          for (int w0 = t % LW; w0 < wp; w0 += LW) {
+            const int ww = w0 - g.pad_w;
+            const bool w_ok = ww >= 0 && ww < g.w;
+            for (int ci = t / LW; ci < nch; ci += 256 / LW) {
+              const uint16_t* xc = x + (int64_t)(ch_lo + ci) * g.xs_c + (int64_t)ww * g.xs_w;
+              uint16_t* to = patch + ci * per_ch + w0;
+              for (int h0 = 0; h0 < hp; h0 += 4) {
+                uint16_t v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                  v[k] = 0;
+                  if (w_ok && h0 + k < hp) {
+                    const int64_t so = src_row[h0 + k];
+                    if (so >= 0) v[k] = xc[so];
+                  }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                  if (h0 + k < hp) to[(h0 + k) * wp] = v[k];
+              }
+            }
+          }
+        };
+        if (wp <= 16) along_rows(std::integral_constant<int, 16>{});
+        else along_rows(std::integral_constant<int, 32>{});
       }
-      col_off[t] = off;
+      for (int i = t; i < tpg * TILE; i += 256) {
+        const int col = g0 + i;
+        int off = 0;
+        if (col < ncols) {
+          const int ci = col / rs_n, rs = col - ci * rs_n;
+          off = (ci - ch_lo) * per_ch + (rs / g.s) * g.dil_h * wp + (rs % g.s) * g.dil_w;
+        }
+        col_off[i] = off;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    const int ch8 = (t % 8) * 8;
+    const int c0 = ct * TILE, ch8 = (t % 8) * 8;
+    const int* off = col_off + (ct - group * tpg) * TILE + ch8;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int row_l = t / 8 + 32 * i;
+      const int64_t row = r0 + t / 8 + 32 * i;
+      if (row >= rows) continue;
       uint16_t e[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int off = col_off[ch8 + j];
-        e[j] = patch[off + row_off[i]];
-      }
-      uint16_t* dst = cols + (r0 + row_l) * ld + c0 + ch8;
+      for (int j = 0; j < 8; ++j) e[j] = patch[off[j] + row_off[i]];
+      uint16_t* dst = cols + row * ld + c0 + ch8;
       if (c0 + ch8 + 8 <= ncols) {
         u32x4 v;
         v.x = e[0] | ((uint32_t)e[1] << 16);
@@ -215,7 +286,6 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
           if (c0 + ch8 + j < ncols) dst[j] = e[j];
       }
     }
-    __syncthreads();
   }
 }
 
@@ -504,18 +574,29 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
   const int64_t rows = n * g.p * g.q;
   const int64_t blocks = ceil_div(rows, TILE);
   SD_REQUIRE(blocks <= 0x7fffffffLL, "im2col: too many rows");
-  // patch-staged kernel: workgroup rows inside one image, 16-byte aligned stores, patch fits in LDS
+  // patch-staged kernel: 16-byte aligned stores, and a copy of the rows of one column tile's channels fits in LDS.  The
+  // most input rows a 64-row group can read: its output rows spread over as many images as it can touch.
   const int64_t pq = (int64_t)g.p * g.q;
-  const int rows_p = (int)((TILE + g.q - 2) / g.q + 1);  // output rows p a 64-row group can touch
-  const int hp = (rows_p - 1) * g.str_h + (g.r - 1) * g.dil_h + 1;
-  const int wp = (g.q - 1) * g.str_w + (g.s - 1) * g.dil_w + 1;
-  const int max_ch = (int)((TILE + r * s - 2) / (r * s) + 1);
-  const int64_t patch_bytes = (int64_t)max_ch * hp * wp * 2;
-  if (pq % TILE == 0 && ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 &&
-      patch_bytes <= PATCH_MAX_BYTES) {
-    hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks), dim3(256), (size_t)patch_bytes, stream,
+  const int64_t out_rows = (TILE + g.q - 2) / g.q + 1, images = (TILE + pq - 2) / pq + 1;
+  const int64_t reach = (int64_t)(g.r - 1) * g.dil_h + 1;
+  const int64_t spread = out_rows < images ? out_rows : images;
+  const int64_t one = (out_rows - 1) * g.str_h + reach, many = (out_rows - spread) * g.str_h + spread * reach;
+  const int64_t hp = one > many ? one : many;
+  const int64_t wp = (int64_t)(g.q - 1) * g.str_w + (int64_t)(g.s - 1) * g.dil_w + 1;
+  const int64_t ntiles = ceil_div(c * r * s, TILE);
+  auto group_bytes = [&](int64_t tiles) {
+    int64_t ch = (tiles * TILE + r * s - 2) / (r * s) + 1;
+    if (ch > c) ch = c;
+    return tiles * TILE * 4 + (ch * hp * wp * 2 + 15) / 16 * 16;
+  };
+  if (ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 && hp <= PATCH_ROWS_MAX &&
+      group_bytes(1) <= PATCH_MAX_BYTES) {
+    // as many tiles to a group as fit a quarter of the LDS a workgroup may ask for: several workgroups share a CU
+    int64_t tpg = 1;
+    while (tpg < ntiles && group_bytes(tpg + 1) <= PATCH_MAX_BYTES / 2) ++tpg;
+    hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks), dim3(256), (size_t)group_bytes(tpg), stream,
                        (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
-                       row_ptr ? (int)bs : TILE, hp, wp, max_ch);
+                       row_ptr ? (int)bs : TILE, (int)wp, (int)tpg);
     return check_launch("im2col_patch");
   }
   hipLaunchKernelGGL(im2col_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,

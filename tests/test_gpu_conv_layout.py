@@ -1,9 +1,41 @@
 """The convolution's data movement at its edges: 64-row groups that end inside an image or span several, column groups
 that need more than one copy of the input rows, and the gradient's planes turned into rows."""
+import numpy as np
 import pytest
 import torch
 
+from _util import cpu_mask
+from oracle import sparsedrop_oracle as O
+
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,c,hw,r,stride,pad,dil", [
+    (3, 8, 28, 3, 1, 1, 1),     # 784 positions: groups across two images, the last one ragged
+    (9, 16, 7, 3, 1, 1, 1),     # 49 positions: up to three images to a group
+    (70, 8, 3, 3, 2, 1, 1),     # 4 positions an image: 16 or 17 images to a group
+    (2, 8, 30, 5, 2, 2, 1),     # stride 2, 225 positions
+    (2, 8, 33, 3, 1, 2, 2),     # dilation, rows longer than half a wave
+    (2, 200, 14, 3, 1, 1, 1),   # more channels than one copy holds
+    (5, 24, 9, 1, 1, 0, 1),     # 1 x 1
+])
+@pytest.mark.parametrize("bs", [64, 128])
+def test_patch_matrix_any_image_size(n, c, hw, r, stride, pad, dil, bs):
+    """Bit exact (a gather), whole and kept blocks only; nothing outside the kept blocks is written."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    geo = dict(padding=(pad, pad), stride=(stride, stride), dilation=(dil, dil))
+    gen = torch.Generator().manual_seed(n * c + hw)
+    x = torch.randn(n, c, hw, hw, generator=gen).half()
+    ref = O.im2col(x.float().numpy(), r, r, **geo)
+    full = ext.im2col(x.cuda(), (r, r), **geo)
+    assert np.array_equal(full.float().cpu().numpy(), ref)
+    mask = cpu_mask(O.mask_shape(*ref.shape, bs), 0.5, gen)
+    part = torch.full_like(full, 7.0)
+    ext.im2col(x.cuda(), (r, r), lists=ext.build_lists(mask.cuda()), block_size=bs, out=part, **geo)
+    keep = O.expand_keep(mask.numpy(), bs, *ref.shape)
+    assert np.array_equal(part.float().cpu().numpy(), np.where(keep, ref, 7.0))
 
 
 @pytest.mark.parametrize("n,c,p", [(1, 2, 2), (2, 64, 64), (3, 65, 63), (2, 130, 784), (5, 7, 49), (1, 128, 1)])
