@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import cpu_mask
+from _util import REL_FRO_TOL, cpu_mask, max_tile_rel_fro, to_np
 from oracle import sparsedrop_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +50,25 @@ def test_rows_from_planes(n, c, p, gap):
     dst = torch.full((n * p + 1, c), 77, dtype=torch.int16, device="cuda")
     ext._call(ext.lib.sd_rows_from_planes, src.data_ptr(), src.stride(0), src.stride(1), dst.data_ptr(), n, c, p, ext._stream(dst))
     assert torch.equal(dst[:-1].view(n, p, c), src.transpose(1, 2)) and (dst[-1] == 77).all()
+
+
+@pytest.mark.parametrize("n,c,hw,k", [(3, 40, 9, 24), (2, 96, 14, 168), (1, 8, 3, 8)])
+@pytest.mark.parametrize("p", [0.0, 0.5])
+def test_pointwise_convolution_of_pixel_rows(n, c, hw, k, p):
+    """1 x 1 on a channels-last image: its pixels are the patch matrix and the patch gradient, dropped blocks zero."""
+    import flash_dropout.functional as F
+
+    gen = torch.Generator().manual_seed(c)
+    x = torch.randn(n, c, hw, hw, generator=gen).half().cuda().to(memory_format=torch.channels_last).requires_grad_()
+    w = (torch.randn(k, c, 1, 1, generator=gen) * c ** -0.5).half().cuda().requires_grad_()
+    mask = cpu_mask(O.mask_shape(n * hw * hw, c, 64), p, gen)
+    y = F.blockwise_dropout_conv2d_mask(x, mask.cuda(), 64, p, w)
+    dy = torch.randn(*y.shape, generator=gen).half().cuda()
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    assert dx.shape == x.shape and dx.is_contiguous(memory_format=torch.channels_last)
+    rows = lambda t: to_np(t.permute(0, 2, 3, 1).reshape(n * hw * hw, -1))
+    xn, wn, dyn = rows(x), to_np(w).reshape(k, c), rows(dy)
+    for got, ref in ((rows(y), O.dsd_forward(xn, wn, mask.numpy(), 64, p, np.float32)),
+                     (rows(dx), O.sdd_dx(dyn, wn, mask.numpy(), 64, p, np.float32)),
+                     (to_np(dw).reshape(k, c), O.dsd_dw(dyn, xn, mask.numpy(), 64, p, np.float32))):
+        assert max_tile_rel_fro(got, ref) <= REL_FRO_TOL
