@@ -1,6 +1,7 @@
 // Launchers of the 64 x 64 ... 128 x 128 tile kernels for one element type; gemm_tile_f16.hip and gemm_tile_bf16.hip
 // compile one each.
 #pragma once
+#include <algorithm>
 #include <atomic>
 
 #include "gemm_tile.h"
@@ -114,9 +115,14 @@ template <typename T, typename S>
 int sdd_launch(const GemmArgs& g, hipStream_t stream) {
   static std::atomic<bool> done[64] = {};
   auto* kernel = &tile_sdd_kernel<T, S>;
-  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM_STEPS, done)) return rc;
   const int Mb = blocks_of(g.M), Cb = blocks_of(g.N), tn = (Cb + S::C - 1) / S::C;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(Mb * tn)), dim3(S::THREADS), S::SMEM, stream, g, tn, Mb, Cb);
+  // No step table, and no more stages than there are steps, down to what the halves meet in.  With the table's 8 KB behind
+  // its stages a CU held two workgroups of SddWide, not three: 16384 x 1536 from 384 at p = 0.1 45 -> 39 us, at p = 0.5
+  // 33 -> 26; 8192 x 8192 from 1024 at p = 0.5 132 -> 114; 200704 x 288 from 64 (a convolution's, one step) 51 -> 41.
+  const int64_t stages = std::min<int64_t>(blocks_of(g.K), S::NST);
+  const int smem = std::max((int)stages * S::STAGE, S::NW * 2 * S::NT16 * 1024);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(Mb * tn)), dim3(S::THREADS), smem, stream, g, tn, Mb, Cb);
   return check_launch("tile_sdd_kernel");
 }
 
