@@ -1877,21 +1877,23 @@ bool sdd_big_ok(const GemmArgs& g) {
          blocks_of(g.N) <= G_MAX_CB;
 }
 
-// Whether the strips of two beat the big shape on a short reduction, where what counts is how the grid fills its rounds
-// and whose store runs under other products.  Fitted (us) to sizes of 2048 to 16384 rows and 1024 to 8192 columns over
-// reductions of 256 to 2048 at p = 0.1, 0.3, 0.5, without and with GELU's derivative: the big shape takes whole rounds of
-// 256 groups whatever is kept, the strips (three to a CU) as many rounds as there are kept tiles.  With the derivative at
-// p = 0.1 / 0.5, big against strips: 16384 x 1536 from 384 (a round and a half) 71 / 64 us, 65 / 45; 16384 x 1024 from 256
-// (one round) 33 / 32, 36 / 28; 4096 x 4096 from 1024 58 / 51, 67 / 47; from 2048 75 / 70, 102 / 75: deeper ones are the
-// big shape's, and so are masks of 32-blocks, which were not measured.
+// Whether the strips of two beat the big shape: on short reductions, where what counts is how the grid fills its rounds and
+// whose store runs under other products, and on few kept tiles.  Fitted (us) to sizes of 4096 to 16384 rows and 1024 to
+// 8192 columns over reductions of 256 to 4096 at p = 0.1, 0.3, 0.5, 0.75, without and with GELU's derivative: the big shape
+// takes whole rounds of 256 groups whatever is kept, the strips (three to a CU) as many rounds as there are kept tiles.
+// With the derivative, at p = 0.1 / 0.5, big against strips: 16384 x 1536 from 384 (a round and a half) 72 / 65 us, 53 / 37;
+// 16384 x 1024 from 256 (one round) 34 / 33, 33 / 24; 4096 x 4096 from 1024 58 / 52, 58 / 39; from 2048 76 / 74, 89 / 60; from
+// 4096 118 / 112, 156 / 107, and at p = 0.75 104 against 62.  Not on outputs wider than twice their height, where a
+// strip's share of W is not in the L2 any more (2048 x 8192 from 2048 at p = 0.5: 61 against 83), nor on masks of
+// 32-blocks, which were not measured.
 bool strips_beat_big(const GemmArgs& g) {
   const double kb = (double)blocks_of(g.K), kept = (double)(blocks_of(g.M) * blocks_of(g.N)) * kept_fraction(g);
-  if (kb > 32 || g.quads || !g.row_ptr) return false;
+  if (kb > 64 || g.quads || !g.row_ptr || blocks_of(g.N) > 2 * blocks_of(g.M)) return false;
   const bool gelu = g.act == SD_ACT_GELU;
   const double rounds = (double)((sdd_big_groups(g) + 255) / 256), strip_rounds = kept / 1536.0;
-  const double big = rounds * (15.0 + 1.5 * kb) * (rounds >= 4 ? 0.9 : 1.0) + (gelu ? 11.0 * rounds : 0.0);
-  const double strips = 10.0 + (strip_rounds + 0.5) * (2.0 + 0.95 * kb) * (strip_rounds > 4.0 ? 1.2 : 1.0) + (gelu ? 0.0036 * kept : 0.0);
-  return strips < 0.95 * big;
+  const double big = rounds * (17.0 + 1.4 * kb) * (rounds >= 4 ? 0.9 : 1.0) + (gelu ? 11.0 * rounds : 0.0);
+  const double strips = 9.0 + (strip_rounds + 0.5) * (2.0 + 0.75 * kb) * (strip_rounds > 4.0 ? 1.2 : 1.0) + (gelu ? 0.0026 * kept : 0.0);
+  return strips < 0.92 * big;
 }
 
 // The big shape when its grid gives more than half of the CUs a workgroup (on aligned operands: its edge instance runs
