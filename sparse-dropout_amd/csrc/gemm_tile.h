@@ -45,7 +45,9 @@ struct TileShape {
   static constexpr int STAGE = (R + C) * TILE;
   static constexpr int MAX_STEPS = 2048;  // kTileMaxSteps
   static constexpr int SMEM_STEPS = NST * STAGE;
-  static constexpr int SMEM = SMEM_STEPS + 4 * (MAX_STEPS + TILE_PAD) + 16;
+  // the number of steps and the step table behind the stages, for a reduction of kb blocks
+  static constexpr int smem_for(int64_t kb) { return SMEM_STEPS + 16 + 4 * (int)((kb < MAX_STEPS ? kb : MAX_STEPS) + TILE_PAD); }
+  static constexpr int SMEM = SMEM_STEPS + 16 + 4 * (MAX_STEPS + TILE_PAD);
   static_assert(LPW * LOADERS == 8 && 4 * MAX_STEPS <= SMEM_STEPS, "loads divide evenly; the merge scratch lies in the stages");
   static_assert(!HALVES || (MT == 4 && NW * 2 * NT16 * 1024 <= SMEM_STEPS), "the halves meet in the stages");
 };
@@ -218,8 +220,8 @@ __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, in
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t smem_a = lds_address(smem);
   uint32_t* scratch = reinterpret_cast<uint32_t*>(smem);  // uint32 per K block while merging; the stages come later
-  uint32_t* step_e = reinterpret_cast<uint32_t*>(smem + S::SMEM_STEPS);
-  int* nsteps_p = reinterpret_cast<int*>(smem + S::SMEM_STEPS + 4 * (S::MAX_STEPS + TILE_PAD));
+  int* nsteps_p = reinterpret_cast<int*>(smem + S::SMEM_STEPS);
+  uint32_t* step_e = reinterpret_cast<uint32_t*>(smem + S::SMEM_STEPS + 16);
 
   int tm, tn;
   tile_of_block<DSD_GROUP_M>(bid, tiles_m, tiles_n, tm, tn);

@@ -20,6 +20,10 @@ namespace {
 //         the other's products (16384 x 384 -> 1536 with a GELU in the store: 65 -> 45 us against the 256 x 256 shape)
 // reduction-contiguous operands (forward, dense): one running sum per element
 using FwdOne = TileShape<1, 1, 4, 2, false, 2, 2>;
+// the same with three stages, three workgroups to a CU: more than the 512 that are resident with four (a result up to 64
+// columns wide), where a workgroup's way to its first tile counts:
+// 200704 x 288 -> 64 at p = 0.25 35 -> 30 us, 219520 x 576 -> 64 at p = 0.5 38 -> 33
+using FwdOneMany = TileShape<1, 1, 3, 2, false, 2, 2>;
 using FwdQuad = TileShape<2, 2, 4, 2, false, 4, 2>;
 using FwdWide = TileShape<2, 2, 2, 0, false, 2, 4>;
 // reduction-strided operands (weight gradient): the depth halves apart
@@ -89,13 +93,17 @@ int allow_lds(const void* kernel, int bytes, std::atomic<bool> (&done)[64]) {
 
 int blocks_of(int64_t n) { return (int)((n + BS - 1) / BS); }
 
+bool more_than_resident(const GemmArgs& g, int splits) {  // of the 64 x 64 shape with four stages
+  return (int64_t)blocks_of(g.M) * blocks_of(g.N) * splits > 512;
+}
+
 template <typename T, bool KC, bool CM, typename S>
 int dsd_launch(const GemmArgs& g, int splits, hipStream_t stream) {
   static std::atomic<bool> done[64] = {};
   auto* kernel = &tile_dsd_kernel<T, KC, CM, S>;
   if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
   const int Mb = blocks_of(g.M), Kb = blocks_of(g.K), tm = (Mb + S::R - 1) / S::R, tn = (blocks_of(g.N) + S::C - 1) / S::C;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(tm * tn), (unsigned)splits), dim3(S::THREADS), S::SMEM, stream, g, tm, tn, Mb, Kb);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tm * tn), (unsigned)splits), dim3(S::THREADS), S::smem_for(Kb), stream, g, tm, tn, Mb, Kb);
   return check_launch("tile_dsd_kernel");
 }
 
@@ -106,7 +114,7 @@ int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t
   if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
   const int Mb = blocks_of(g.M), Kb = blocks_of(g.K), tm = (Mb + S::R - 1) / S::R, tn = (blocks_of(g.N) + S::C - 1) / S::C;
   const int n_gemm = tm * tn * splits;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::SMEM, stream, g, tm, tn, Mb, Kb,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::smem_for(Kb), stream, g, tm, tn, Mb, Kb,
                      splits, n_gemm, f);
   return check_launch("tile_forward_kernel");
 }
@@ -143,7 +151,9 @@ int pair_launch(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_t 
 template <typename T, bool KC, bool CM>
 int dsd_shape(const GemmArgs& g, int shape, int splits, hipStream_t stream) {
   switch (shape) {
-    case kShapeOne: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdOne, GradOne>>(g, splits, stream);
+    case kShapeOne:
+      if (KC && more_than_resident(g, splits)) return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdOneMany, GradOne>>(g, splits, stream);
+      return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdOne, GradOne>>(g, splits, stream);
     case kShapeQuad: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdQuad, GradQuad>>(g, splits, stream);
     default: return dsd_launch<T, KC, CM, std::conditional_t<KC, FwdWide, GradWide>>(g, splits, stream);
   }
@@ -160,7 +170,9 @@ int tile_dsd(const GemmArgs& g, bool kc, bool cm, int shape, int splits, hipStre
 template <typename T>
 int tile_forward(const GemmArgs& g, int shape, int splits, const FlatJobs& f, hipStream_t stream) {
   switch (shape) {
-    case kShapeOne: return forward_launch<T, FwdOne>(g, splits, f, stream);
+    case kShapeOne:
+      if (more_than_resident(g, splits)) return forward_launch<T, FwdOneMany>(g, splits, f, stream);
+      return forward_launch<T, FwdOne>(g, splits, f, stream);
     case kShapeQuad: return forward_launch<T, FwdQuad>(g, splits, f, stream);
     default: return forward_launch<T, FwdWide>(g, splits, f, stream);
   }

@@ -104,3 +104,26 @@ def test_input_gradient_of_a_short_reduction(act):
             ref *= 0.5 * (1 + torch.erf(t * 0.5 ** 0.5)) + t * torch.exp(-0.5 * t * t) * 0.3989422804014327
         ref *= (~mask).repeat_interleave(64, 0).repeat_interleave(64, 1)
         assert (got[ref == 0] == 0).all() and (got.float() - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("M,N,K,bs", [
+    (32832, 50, 200, 64),   # one tile past the 512 that are resident, a ragged last step
+    (33001, 64, 64, 32),    # fewer steps than stages, quadrant keep bits
+    (34000, 61, 520, 64),   # more steps than stages, an odd width
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_more_small_tiles_than_are_resident(M, N, K, bs, dtype):
+    """The forward on the three-stage 64 x 64 shape, with the lists in the same launch and from lists, and dense."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(K)
+    x = make_operand(M, K, dtype, "cuda", gen=gen)
+    w = make_operand(N, K, dtype, "cuda", scale=K ** -0.5, gen=gen)
+    mask = cpu_mask(O.mask_shape(M, K, bs), 0.4, gen)
+    y, _, lists, kbs = ext.dropout_matmul_forward(x, w, bs, 0.4, mask=mask.cuda())
+    again = ext.gemm_dsd_lists(x, w, lists, kbs, 1 / 0.6)
+    assert ext.last_kernel_detail().startswith("dsd:one")
+    ref = O.dsd_forward(to_np(x), to_np(w), mask.numpy(), bs, 0.4, np.float32)
+    assert max_tile_rel_fro(y, ref) <= REL_FRO_TOL and torch.equal(y, again)
+    assert max_tile_rel_fro(ext.gemm(x, w), to_np(x) @ to_np(w).T) <= REL_FRO_TOL
