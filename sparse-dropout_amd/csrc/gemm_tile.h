@@ -215,7 +215,7 @@ __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0
 // large shapes' dsd_body.
 template <typename T, bool KC, bool CM, typename S>
 __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, int tiles_n, int Mb, int Kb_all, int bid,
-                                              int nsplit, int split, const MaskSrc* ms = nullptr) {
+                                              int nsplit, const MaskSrc* ms = nullptr) {
   constexpr int R = S::R, C = S::C, NST = S::NST, LPW = S::LPW, MT = S::MT, NT16 = S::NT16, KG = S::HALVES ? 2 : 1;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t smem_a = lds_address(smem);
@@ -223,8 +223,8 @@ __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, in
   int* nsteps_p = reinterpret_cast<int*>(smem + S::SMEM_STEPS);
   uint32_t* step_e = reinterpret_cast<uint32_t*>(smem + S::SMEM_STEPS + 16);
 
-  int tm, tn;
-  tile_of_block<DSD_GROUP_M>(bid, tiles_m, tiles_n, tm, tn);
+  int tm, tn, split;
+  tile_of_split_block<DSD_GROUP_M>(bid, tiles_m, tiles_n, nsplit, tm, tn, split);
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = (int)uniform((uint32_t)(tid / 64));
   const int lwave = S::LW ? wave - S::NW : wave;  // index among the waves that load

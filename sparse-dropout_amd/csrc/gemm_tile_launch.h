@@ -37,7 +37,7 @@ using SddWide = TileShape<1, 2, 2, 0, true>;
 
 template <typename T, bool KC, bool CM, typename S>
 __global__ __launch_bounds__(S::THREADS) void tile_dsd_kernel(GemmArgs g, int tiles_m, int tiles_n, int Mb, int Kb) {
-  tile_dsd_body<T, KC, CM, S>(g, tiles_m, tiles_n, Mb, Kb, (int)blockIdx.x, (int)gridDim.y, (int)blockIdx.y);
+  tile_dsd_body<T, KC, CM, S>(g, tiles_m, tiles_n, Mb, Kb, (int)(blockIdx.y * gridDim.x + blockIdx.x), (int)gridDim.y);
 }
 
 template <typename T, typename S>
@@ -53,8 +53,7 @@ __global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, in
   if (bid < n_gemm) {
     MaskSrc ms = f.job0.src;
     ms.resolve();
-    const int tiles = tiles_m * tiles_n;
-    tile_dsd_body<T, true, false, S>(g, tiles_m, tiles_n, Mb, Kb, bid % tiles, nsplit, bid / tiles, &ms);
+    tile_dsd_body<T, true, false, S>(g, tiles_m, tiles_n, Mb, Kb, bid, nsplit, &ms);
   } else {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     flat_lists_block<S::THREADS>(f, bid - n_gemm, reinterpret_cast<int32_t*>(smem));
@@ -73,8 +72,7 @@ __global__ __launch_bounds__(W::THREADS) void tile_pair_kernel(GemmArgs gx, int 
   if (bid < n_dx) {
     if (bid < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_tiles_n, x_Mb, x_Cb, bid);
   } else {
-    const int wb = bid - n_dx, tiles = w_tiles_m * w_tiles_n;
-    tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, wb % tiles, w_splits, wb / tiles);
+    tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, bid - n_dx, w_splits);
   }
 }
 
