@@ -1883,12 +1883,12 @@ bool sdd_big_ok(const GemmArgs& g) {
 // takes whole rounds of 256 groups whatever is kept, the strips (three to a CU) as many rounds as there are kept tiles.
 // With the derivative, at p = 0.1 / 0.5, big against strips: 16384 x 1536 from 384 (a round and a half) 72 / 65 us, 53 / 37;
 // 16384 x 1024 from 256 (one round) 34 / 33, 33 / 24; 4096 x 4096 from 1024 58 / 52, 58 / 39; from 2048 76 / 74, 89 / 60; from
-// 4096 118 / 112, 156 / 107, and at p = 0.75 104 against 62.  Not on outputs wider than 1.5 times their height, where a
+// 4096 118 / 112, 156 / 107, and at p = 0.75 104 against 62.  Not on outputs wider than twice their height, where a
 // strip's share of W is not in the L2 any more (2048 x 8192 from 2048 at p = 0.5: 61 against 83), nor on masks of
 // 32-blocks or reductions outside that range, which were not measured.
 bool strips_beat_big(const GemmArgs& g) {
   const double kb = (double)blocks_of(g.K), kept = (double)(blocks_of(g.M) * blocks_of(g.N)) * kept_fraction(g);
-  if (kb < 4 || kb > 64 || g.quads || !g.row_ptr || 2 * blocks_of(g.N) > 3 * blocks_of(g.M)) return false;
+  if (kb < 4 || kb > 64 || g.quads || !g.row_ptr || blocks_of(g.N) > 2 * blocks_of(g.M)) return false;
   const bool gelu = g.act == SD_ACT_GELU;
   const double rounds = (double)((sdd_big_groups(g) + 255) / 256), strip_rounds = kept / 1536.0;
   const double big = rounds * (17.0 + 1.4 * kb) * (rounds >= 4 ? 0.9 : 1.0) + (gelu ? 11.0 * rounds : 0.0);
