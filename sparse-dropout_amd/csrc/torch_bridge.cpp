@@ -372,7 +372,7 @@ Tensor autocast(const Tensor& t) {
 
 // ---- one layer ----------------------------------------------------------------------------------------------------------
 struct LinearBackward : Node {
-  SavedVariable x, w;
+  SavedVariable x, w, mask;  // mask: a given one, which must not change before the backward
   Lists lists;
   double p = 0;
   variable_list apply(variable_list&& grads) override {
@@ -380,6 +380,7 @@ struct LinearBackward : Node {
     variable_list out(2);
     if (!grads[0].defined()) return out;
     const Tensor xs = x.unpack(), ws = w.unpack();
+    mask.unpack();
     const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
     std::tie(out[0], out[1]) = layer_backward(grad_matrix(grads[0], xs), ws, xs, lists, p, need_dx, need_dw,
                                               SD_ACT_NONE, Tensor());
@@ -388,6 +389,7 @@ struct LinearBackward : Node {
   void release_variables() override {
     x.reset_data();
     w.reset_data();
+    mask.reset_data();
     lists = Lists();
   }
   std::string name() const override { return "BlockwiseDropoutMatmulHIPBackward"; }
@@ -414,6 +416,7 @@ Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, 
     auto node = make_node<LinearBackward>({x, w});
     node->x = SavedVariable(x, false);
     node->w = SavedVariable(w, false);
+    node->mask = SavedVariable(lists.given, false);
     node->lists = std::move(lists);
     node->p = p;
     torch::autograd::set_history(y, node);
@@ -425,7 +428,7 @@ Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, 
 // (see functional/blockwise_dropout_mlp_hip.py for what is computed)
 struct MlpBackward : Node {
   SavedVariable x;
-  std::vector<SavedVariable> ws;
+  std::vector<SavedVariable> ws, masks;  // masks: the given ones
   std::vector<Tensor> hidden, pre;  // activated outputs of all layers but the last; GELU: their pre-activations
   std::vector<Lists> lists;         // undefined buffer: the layer ran dense
   std::vector<double> ps;
@@ -436,6 +439,7 @@ struct MlpBackward : Node {
     variable_list out(1 + n);
     if (!grads[0].defined()) return out;
     const Tensor x0 = x.unpack();
+    for (const auto& m : masks) m.unpack();
     Tensor g = grad_matrix(grads[0], x0);
     for (int i = n - 1; i >= 0; --i) {
       const Tensor w = ws[i].unpack();
@@ -469,6 +473,7 @@ struct MlpBackward : Node {
   void release_variables() override {
     x.reset_data();
     for (auto& w : ws) w.reset_data();
+    for (auto& m : masks) m.reset_data();
     hidden.clear();
     pre.clear();
     for (auto& l : lists) l.buf.reset(), l.given.reset();
@@ -520,6 +525,7 @@ Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, 
     auto node = make_node<MlpBackward>(inputs);
     node->x = SavedVariable(x, false);
     for (const Tensor& w : ws) node->ws.emplace_back(w, false);
+    for (const Lists& l : lists) node->masks.emplace_back(l.given, false);
     node->hidden = std::move(hidden);
     node->pre = std::move(pres);
     node->lists = std::move(lists);
@@ -658,7 +664,7 @@ Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) 
 }
 
 struct ConvBackward : Node {
-  SavedVariable x, w2;  // w2: the kernel as [K, C*R*S]
+  SavedVariable x, w2, mask;  // w2: the kernel as [K, C*R*S]; mask: a given one, read again for the input gradient
   Tensor cols;          // the patch matrix, when the forward made one
   Lists lists;          // undefined buffer: no dropout
   ConvGeom g{};
@@ -669,6 +675,7 @@ struct ConvBackward : Node {
     variable_list out(2);
     if (!grads[0].defined()) return out;
     const Tensor w = w2.unpack(), image = x.unpack();
+    mask.unpack();
     Tensor patches = cols;
     const Tensor dy2 = rows_gradient(grads[0], g, w);
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
@@ -736,6 +743,7 @@ struct ConvBackward : Node {
   void release_variables() override {
     x.reset_data();
     w2.reset_data();
+    mask.reset_data();
     cols.reset();
     lists = Lists();
   }
@@ -811,6 +819,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     auto node = make_node<ConvBackward>({x, kernel});
     node->x = SavedVariable(x, false);
     node->w2 = SavedVariable(kernel.detach().view({g.k, g.cols()}), false);
+    if (mask && bs) node->mask = SavedVariable(*mask, false);
     node->cols = cols;
     node->lists = std::move(lists);
     node->g = g;

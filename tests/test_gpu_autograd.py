@@ -1,0 +1,95 @@
+"""The public functions as autograd sees them: what they keep for the backward and how, what they refuse, what a changed
+mask or input does.  Results are compared with calls of the same functions that nothing interferes with."""
+import gc
+
+import pytest
+import torch
+
+from _util import cpu_mask
+from oracle import sparsedrop_oracle as O
+
+pytestmark = pytest.mark.gpu
+BS, P = 64, 0.4
+
+
+def _t(*shape, seed, scale=1.0, dtype=torch.float16):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=gen) * scale).to(dtype).cuda()
+
+
+def _mask(rows, cols, seed=0):
+    return cpu_mask(O.mask_shape(rows, cols, BS), P, torch.Generator().manual_seed(seed)).cuda()
+
+
+def _linear():
+    """(call, its tensors): call(mask) runs the function on them."""
+    import flash_dropout.functional as F
+
+    x, w = _t(192, 136, seed=1).requires_grad_(), _t(72, 136, seed=2, scale=0.1).requires_grad_()
+
+    def call(mask="drawn"):
+        if mask == "drawn":
+            return F.hip_blockwise_dropout_matmul(x, w, BS, P, seed=5)
+        return F.hip_blockwise_dropout_matmul_mask(x, mask, BS, P, w)
+
+    return call, (x, w), _mask(192, 136)
+
+
+def _mlp(act="gelu", rows=192):
+    import flash_dropout.functional as F
+
+    x = _t(rows, 136, seed=1).requires_grad_()
+    ws = [_t(o, i, seed=3 + i, scale=i ** -0.5).requires_grad_() for i, o in ((136, 256), (256, 200), (200, 10))]
+
+    def call(mask="drawn"):
+        if mask == "drawn":
+            return F.hip_blockwise_dropout_mlp(x, ws, BS, P, act, seed=5)
+        return F.hip_blockwise_dropout_mlp(x, ws, BS, P, act, masks=[mask, _mask(rows, 256, 1), _mask(rows, 200, 2)])
+
+    return call, (x, *ws), _mask(rows, 136)
+
+
+# rows of 8 and 18 output positions: the routes without and with a patch matrix; a pointwise kernel on pixels in rows, whose
+# patch matrix is the image itself
+CONVS = {"implicit": (8, 3, 1, False), "explicit": (18, 3, 1, False), "pointwise": (12, 1, 0, True)}
+
+
+def _conv(form):
+    import flash_dropout.functional as F
+
+    hw, r, pad, channels_last = CONVS[form]
+    x, k = _t(4, 16, hw, hw, seed=1), _t(40, 16, r, r, seed=2, scale=0.1).requires_grad_()
+    if channels_last:
+        x = x.to(memory_format=torch.channels_last)
+    x.requires_grad_()
+    rows, cols = F.conv_patch_matrix_shape(x.shape, k.shape, (pad, pad))
+
+    def call(mask="drawn"):
+        if mask == "drawn":
+            return F.blockwise_dropout_conv2d(x, k, BS, P, padding=pad, seed=5)
+        return F.blockwise_dropout_conv2d_mask(x, mask, BS, P, k, padding=pad)
+
+    return call, (x, k), _mask(rows, cols)
+
+
+FUNCTIONS = {"linear": _linear, "mlp": _mlp, **{f"conv {f}": (lambda f=f: _conv(f)) for f in CONVS}}
+every_function = pytest.mark.parametrize("name", FUNCTIONS)
+
+
+def _grads(y, wrt, **kw):
+    return torch.autograd.grad(y, wrt, _t(*y.shape, seed=9), **kw)
+
+
+def _same(a, b):
+    return all(torch.equal(s, t) for s, t in zip(a, b))
+
+
+@every_function
+def test_a_given_mask_changed_before_the_backward_is_refused(name):
+    call, wrt, mask = FUNCTIONS[name]()
+    want = _grads(call(mask.clone()), wrt)
+    y = call(mask)
+    assert _same(_grads(y, wrt, retain_graph=True), want)
+    mask.logical_not_()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        _grads(y, wrt)
