@@ -359,6 +359,15 @@ bool records(const N& inputs) {
   return false;
 }
 
+// There is no forward-mode formula, and the launches read the primal values only: an input that carries a forward gradient
+// would silently lose it.
+template <typename N>
+void refuse_forward_mode(const N& inputs) {
+  for (const Tensor& t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!torch::autograd::isFwGradDefined(t), "block dropout products have no jvp: forward mode AD is "
+                                "not supported");
+}
+
 // A product computed without recording; the node is attached to its result afterwards.
 struct NoRecord {
   at::AutoDispatchBelowADInplaceOrView below;
@@ -406,6 +415,7 @@ Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, 
               std::optional<uint64_t> seed, const OptTensor& state) {
   TORCH_CHECK_VALUE(input.dim() == 2 && weight.dim() == 2, "input must be [M, K] and weight [N, K]");
   const Tensor x = as_matrix(autocast(input)), w = as_matrix(autocast(weight));
+  refuse_forward_mode(std::array<Tensor, 2>{x, w});
   Lists lists;
   Tensor y;
   {
@@ -493,6 +503,7 @@ Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, 
   for (const Tensor& w : weights) ws.push_back(as_matrix(autocast(w)));
   variable_list inputs{x};
   inputs.insert(inputs.end(), ws.begin(), ws.end());
+  refuse_forward_mode(inputs);
   const bool rec = records(inputs);
   const bool x_grad = rec && x.requires_grad();
   std::vector<Lists> lists(n);
@@ -760,6 +771,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   TORCH_CHECK_VALUE(input.size(1) == kernel_in.size(1), "channel mismatch: input ", input.size(1), ", kernel ",
                     kernel_in.size(1));
   const Tensor x = autocast(input), kernel = autocast(kernel_in).contiguous();
+  refuse_forward_mode(std::array<Tensor, 2>{x, kernel});
   TORCH_CHECK_VALUE(x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16),
                     "x must be a 4D float16/bfloat16 tensor on the GPU");
   TORCH_CHECK_VALUE(kernel.scalar_type() == x.scalar_type() && kernel.device() == x.device(), "kernel must be a ",

@@ -93,3 +93,45 @@ def test_a_given_mask_changed_before_the_backward_is_refused(name):
     mask.logical_not_()
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         _grads(y, wrt)
+
+
+@every_function
+def test_inputs_that_carry_a_forward_gradient_are_refused(name):
+    import torch.autograd.forward_ad as fwd
+
+    call, wrt, mask = FUNCTIONS[name]()
+    import flash_dropout.functional as F
+
+    with fwd.dual_level():
+        for i in range(2):  # the input, a weight
+            dual = [t.detach() for t in wrt]
+            dual[i] = fwd.make_dual(dual[i], torch.ones_like(dual[i]))
+            with pytest.raises(NotImplementedError, match="jvp"):
+                if name == "linear":
+                    F.hip_blockwise_dropout_matmul(*dual, BS, P, seed=5)
+                elif name == "mlp":
+                    F.hip_blockwise_dropout_mlp(dual[0], dual[1:], BS, P, "gelu", seed=5)
+                else:
+                    F.blockwise_dropout_conv2d(*dual, BS, P, seed=5)
+
+
+@every_function
+def test_function_transforms_are_refused(name):
+    """The launches read raw pointers, which a transform's wrapped tensors do not have."""
+    import flash_dropout.functional as F
+
+    _, wrt, _ = FUNCTIONS[name]()
+    plain = [t.detach() for t in wrt]
+
+    def f(x):
+        if name == "linear":
+            return F.hip_blockwise_dropout_matmul(x, plain[1], BS, P, seed=5)
+        if name == "mlp":
+            return F.hip_blockwise_dropout_mlp(x, plain[1:], BS, P, "gelu", seed=5)
+        return F.blockwise_dropout_conv2d(x, plain[1], BS, P, seed=5)
+
+    for transformed in (lambda: torch.func.vmap(f)(torch.stack([plain[0]] * 2)),
+                        lambda: torch.func.grad(lambda x: f(x).float().sum())(plain[0]),
+                        lambda: torch.func.jvp(f, (plain[0],), (plain[0],))):
+        with pytest.raises((RuntimeError, NotImplementedError, ValueError)):
+            transformed()
