@@ -20,6 +20,7 @@
 
 #include <array>
 #include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -233,6 +234,61 @@ struct Lists {
   }
 };
 
+// ---- what a node keeps for its backward ----------------------------------------------------------------------------------
+// A tensor that goes through torch's saved-tensor hooks (offloading and checkpoints take its memory in between) and is
+// checked for writes since it was saved.  A hook may hand back any tensor, and the launches trust pointers and extents:
+// what comes back has to have the type, device and extents of what was saved; its strides may be others.
+struct Saved {
+  SavedVariable tensor;
+  at::DimVector sizes;
+  at::ScalarType dtype = at::kHalf;
+  c10::Device device = c10::Device(at::kCPU);
+  void keep(const Tensor& t) {
+    if (!t.defined()) return;
+    tensor = SavedVariable(t, false);
+    sizes = t.sizes();
+    dtype = t.scalar_type();
+    device = t.device();
+  }
+  Tensor get() const {  // undefined when nothing was kept
+    Tensor t = tensor.unpack();
+    TORCH_CHECK_VALUE(!t.defined() || (t.sizes() == at::IntArrayRef(sizes) && t.scalar_type() == dtype && t.device() == device),
+                      "a saved-tensor hook returned a ", t.sizes(), " ", t.dtype(), " tensor on ", t.device(), " for a ",
+                      at::IntArrayRef(sizes), " ", dtype, " tensor on ", device);
+    return t;
+  }
+  Tensor matrix() const {
+    const Tensor t = get();
+    return t.defined() ? as_matrix(t) : t;
+  }
+  void drop() { tensor.reset_data(); }
+};
+
+struct SavedLists {
+  Saved buf, given;
+  Lists shape;  // without its tensors
+  // mask: the tensor whose changes count, when that is not the one in the lists
+  void keep(Lists&& lists, const Tensor& mask = Tensor()) {
+    buf.keep(lists.buf);
+    given.keep(mask.defined() ? mask : lists.given);
+    shape = std::move(lists);
+    shape.buf.reset();
+    shape.given.reset();
+  }
+  Lists get() const {  // undefined buffer: no lists were made
+    Lists l = shape;
+    l.buf = buf.get();
+    if (l.buf.defined()) l.buf = l.buf.contiguous();
+    const Tensor mask = given.get();
+    if (mask.defined()) l.given = check_mask(mask, l.mb, l.kb, mask);
+    return l;
+  }
+  void drop() {
+    buf.drop();
+    given.drop();
+  }
+};
+
 // Where a layer's mask comes from: given, pinned by a seed, or from the device-resident generator state.
 struct Draw {
   OptTensor mask;
@@ -381,25 +437,25 @@ Tensor autocast(const Tensor& t) {
 
 // ---- one layer ----------------------------------------------------------------------------------------------------------
 struct LinearBackward : Node {
-  SavedVariable x, w, mask;  // mask: a given one, which must not change before the backward
-  Lists lists;
+  Saved x, w;
+  SavedLists lists;
   double p = 0;
   variable_list apply(variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     variable_list out(2);
     if (!grads[0].defined()) return out;
-    const Tensor xs = x.unpack(), ws = w.unpack();
-    mask.unpack();
+    const Tensor xs = x.matrix(), ws = w.matrix();
     const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
-    std::tie(out[0], out[1]) = layer_backward(grad_matrix(grads[0], xs), ws, xs, lists, p, need_dx, need_dw,
+    std::tie(out[0], out[1]) = layer_backward(grad_matrix(grads[0], xs), ws, xs, lists.get(), p, need_dx, need_dw,
                                               SD_ACT_NONE, Tensor());
     return out;
   }
   void release_variables() override {
-    x.reset_data();
-    w.reset_data();
-    mask.reset_data();
-    lists = Lists();
+    std::lock_guard<std::mutex> lock(mutex_);
+    x.drop();
+    w.drop();
+    lists.drop();
   }
   std::string name() const override { return "BlockwiseDropoutMatmulHIPBackward"; }
 };
@@ -424,10 +480,9 @@ Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, 
   }
   if (records(std::array<Tensor, 2>{x, w})) {
     auto node = make_node<LinearBackward>({x, w});
-    node->x = SavedVariable(x, false);
-    node->w = SavedVariable(w, false);
-    node->mask = SavedVariable(lists.given, false);
-    node->lists = std::move(lists);
+    node->x.keep(x);
+    node->w.keep(w);
+    node->lists.keep(std::move(lists));
     node->p = p;
     torch::autograd::set_history(y, node);
   }
@@ -437,25 +492,25 @@ Tensor linear(const Tensor& input, const Tensor& weight, const OptTensor& mask, 
 // ---- a stack of layers with an activation between consecutive ones -------------------------------------------------------
 // (see functional/blockwise_dropout_mlp_hip.py for what is computed)
 struct MlpBackward : Node {
-  SavedVariable x;
-  std::vector<SavedVariable> ws, masks;  // masks: the given ones
-  std::vector<Tensor> hidden, pre;  // activated outputs of all layers but the last; GELU: their pre-activations
-  std::vector<Lists> lists;         // undefined buffer: the layer ran dense
+  Saved x;
+  std::vector<Saved> ws;
+  std::vector<Saved> hidden, pre;  // activated outputs of all layers but the last; GELU: their pre-activations
+  std::vector<SavedLists> lists;   // nothing kept: the layer ran dense
   std::vector<double> ps;
   int act = SD_ACT_NONE;
   variable_list apply(variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     const int n = (int)ws.size();
     variable_list out(1 + n);
     if (!grads[0].defined()) return out;
-    const Tensor x0 = x.unpack();
-    for (const auto& m : masks) m.unpack();
+    const Tensor x0 = x.matrix();
     Tensor g = grad_matrix(grads[0], x0);
     for (int i = n - 1; i >= 0; --i) {
-      const Tensor w = ws[i].unpack();
-      const Tensor& h = i ? hidden[i - 1] : x0;
+      const Tensor w = ws[i].matrix(), h = i ? hidden[i - 1].matrix() : x0;
+      const Lists l = lists[i].get();
       const bool need_w = task_should_compute_output(1 + i), need_in = i > 0 || task_should_compute_output(0);
-      if (!lists[i].buf.defined()) {  // the dense first layer: only its weight gradient is wanted, dW = g^T . h
+      if (!l.buf.defined()) {  // the dense first layer: only its weight gradient is wanted, dW = g^T . h
         if (need_w) {
           const int64_t N = w.size(0);
           Tensor gp = g, hp = h;
@@ -470,9 +525,9 @@ struct MlpBackward : Node {
         break;
       }
       Tensor at;
-      if (i > 0 && need_in && act != SD_ACT_NONE) at = act == SD_ACT_GELU ? pre[i - 1] : h;
+      if (i > 0 && need_in && act != SD_ACT_NONE) at = act == SD_ACT_GELU ? pre[i - 1].matrix() : h;
       // both gradients of the layer in one library call, the activation's derivative riding on the dX store
-      auto [dx, dw] = layer_backward(g, w, h, lists[i], ps[i], need_in, need_w, at.defined() ? act : SD_ACT_NONE, at);
+      auto [dx, dw] = layer_backward(g, w, h, l, ps[i], need_in, need_w, at.defined() ? act : SD_ACT_NONE, at);
       out[1 + i] = dw;
       if (!need_in) break;
       g = dx;
@@ -481,12 +536,11 @@ struct MlpBackward : Node {
     return out;
   }
   void release_variables() override {
-    x.reset_data();
-    for (auto& w : ws) w.reset_data();
-    for (auto& m : masks) m.reset_data();
-    hidden.clear();
-    pre.clear();
-    for (auto& l : lists) l.buf.reset(), l.given.reset();
+    std::lock_guard<std::mutex> lock(mutex_);
+    x.drop();
+    for (auto* saved : {&ws, &hidden, &pre})
+      for (Saved& s : *saved) s.drop();
+    for (SavedLists& l : lists) l.drop();
   }
   std::string name() const override { return "BlockwiseDropoutMLPHIPBackward"; }
 };
@@ -534,12 +588,18 @@ Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, 
   }
   if (rec) {
     auto node = make_node<MlpBackward>(inputs);
-    node->x = SavedVariable(x, false);
-    for (const Tensor& w : ws) node->ws.emplace_back(w, false);
-    for (const Lists& l : lists) node->masks.emplace_back(l.given, false);
-    node->hidden = std::move(hidden);
-    node->pre = std::move(pres);
-    node->lists = std::move(lists);
+    node->x.keep(x);
+    node->ws.resize(n);
+    node->hidden.resize(n - 1);
+    node->pre.resize(n - 1);
+    node->lists.resize(n);
+    for (int i = 0; i < n; ++i) {
+      node->ws[i].keep(ws[i]);
+      node->lists[i].keep(std::move(lists[i]));
+      if (i + 1 == n) break;
+      node->hidden[i].keep(hidden[i]);
+      node->pre[i].keep(pres[i]);
+    }
     node->ps = ps;
     node->act = act;
     torch::autograd::set_history(h, node);
@@ -675,19 +735,20 @@ Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) 
 }
 
 struct ConvBackward : Node {
-  SavedVariable x, w2, mask;  // w2: the kernel as [K, C*R*S]; mask: a given one, read again for the input gradient
-  Tensor cols;          // the patch matrix, when the forward made one
-  Lists lists;          // undefined buffer: no dropout
+  Saved x, w2;       // w2: the kernel as [K, C*R*S]
+  Saved cols;        // the patch matrix, when the forward made one
+  SavedLists saved;  // nothing kept: no dropout
   ConvGeom g{};
   double p = 0;
   bool fused_dx = true, channels_last = false;
   variable_list apply(variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     variable_list out(2);
     if (!grads[0].defined()) return out;
-    const Tensor w = w2.unpack(), image = x.unpack();
-    mask.unpack();
-    Tensor patches = cols;
+    const Tensor w = w2.get().contiguous(), image = x.get();
+    Tensor patches = cols.matrix();
+    const Lists lists = saved.get();
     const Tensor dy2 = rows_gradient(grads[0], g, w);
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
@@ -752,11 +813,9 @@ struct ConvBackward : Node {
     return out;
   }
   void release_variables() override {
-    x.reset_data();
-    w2.reset_data();
-    mask.reset_data();
-    cols.reset();
-    lists = Lists();
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (Saved* s : {&x, &w2, &cols}) s->drop();
+    saved.drop();
   }
   std::string name() const override { return "Im2colConv2dBackward"; }
 };
@@ -829,11 +888,10 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   }
   if (records(std::array<Tensor, 2>{x, kernel})) {
     auto node = make_node<ConvBackward>({x, kernel});
-    node->x = SavedVariable(x, false);
-    node->w2 = SavedVariable(kernel.detach().view({g.k, g.cols()}), false);
-    if (mask && bs) node->mask = SavedVariable(*mask, false);
-    node->cols = cols;
-    node->lists = std::move(lists);
+    node->x.keep(x);
+    node->w2.keep(kernel.detach().view({g.k, g.cols()}));
+    node->cols.keep(cols);
+    if (bs) node->saved.keep(std::move(lists), mask.value_or(Tensor()));
     node->g = g;
     node->p = bs ? p : 0.0;
     node->fused_dx = fused_dx;

@@ -5,7 +5,7 @@ import gc
 import pytest
 import torch
 
-from _util import cpu_mask
+from _util import cpu_mask, rel_fro
 from oracle import sparsedrop_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -135,3 +135,69 @@ def test_function_transforms_are_refused(name):
                         lambda: torch.func.jvp(f, (plain[0],), (plain[0],))):
         with pytest.raises((RuntimeError, NotImplementedError, ValueError)):
             transformed()
+
+
+@every_function
+@pytest.mark.parametrize("given", [False, True])
+def test_everything_kept_for_the_backward_goes_through_saved_tensor_hooks(name, given):
+    """With hooks that take what is saved to host memory, the device holds the output and no more, and the gradients that
+    come out of the copies are the same bits."""
+    call, wrt, mask = FUNCTIONS[name]()
+    args = (mask,) if given else ()
+    want = _grads(call(*args), wrt)
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
+        y = call(*args)
+    gc.collect()
+    # (the result of the convolution and of a layer is one buffer; the allocator hands out multiples of 512 bytes)
+    assert torch.cuda.memory_allocated() - before <= -(-y.numel() * 2 // 512) * 512
+    assert _same(_grads(y, wrt), want)
+
+
+@every_function
+def test_what_a_hook_hands_back_is_checked_and_may_have_other_strides(name):
+    """The launches trust extents, types and devices; a hook may return any tensor."""
+    call, wrt, mask = FUNCTIONS[name]()
+    for unpack in (lambda t: t.cpu(), lambda t: t.double(), lambda t: t[:-1]):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            y = call(mask)
+        with pytest.raises(ValueError, match="saved-tensor hook"):
+            _grads(y, wrt)
+
+    def strided(t):
+        """The same values with a gap behind every element."""
+        wide = torch.zeros(*t.shape, 2, dtype=t.dtype, device=t.device)
+        wide[..., 0] = t
+        return wide[..., 0]
+
+    want = _grads(call(mask), wrt)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, strided):
+        y = call(mask)
+    # an image with gaps goes through a patch matrix: the same fp32 sums in another order, so an element may round to the
+    # neighbouring fp16 value, 2^-10 of it at most
+    assert all(rel_fro(g, r) <= 2 ** -10 for g, r in zip(_grads(y, wrt), want))
+
+
+@every_function
+def test_a_checkpoint_frees_what_the_function_keeps(name):
+    from torch.utils.checkpoint import checkpoint
+
+    call, wrt, _ = FUNCTIONS[name]()
+    want = _grads(call(), wrt)
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    y = checkpoint(call, use_reentrant=False)
+    gc.collect()
+    assert torch.cuda.memory_allocated() - before <= -(-y.numel() * 2 // 512) * 512
+    assert _same(_grads(y, wrt), want)
+
+
+@every_function
+def test_a_second_backward(name):
+    call, wrt, _ = FUNCTIONS[name]()
+    y = call()
+    want = _grads(y, wrt, retain_graph=True)
+    assert _same(_grads(y, wrt), want)
+    with pytest.raises(RuntimeError, match="second time"):
+        _grads(y, wrt)
