@@ -735,20 +735,21 @@ Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) 
 }
 
 struct ConvBackward : Node {
-  Saved x, w2;       // w2: the kernel as [K, C*R*S]
-  Saved cols;        // the patch matrix, when the forward made one
+  // the kernel as [K, C*R*S], and what the kernel's gradient reads: the patch matrix when the forward made one in memory, else
+  // the image (an implicit forward, or a pointwise kernel whose patch matrix is the image's own pixels)
+  Saved w2, x, cols;
   SavedLists saved;  // nothing kept: no dropout
   ConvGeom g{};
   double p = 0;
-  bool fused_dx = true, channels_last = false;
+  bool fused_dx = true, channels_last = false, pixels = false;
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     variable_list out(2);
     if (!grads[0].defined()) return out;
     const Tensor w = w2.get().contiguous(), image = x.get();
-    Tensor patches = cols.matrix();
     const Lists lists = saved.get();
+    Tensor patches = cols.matrix();
     const Tensor dy2 = rows_gradient(grads[0], g, w);
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
@@ -787,7 +788,8 @@ struct ConvBackward : Node {
     }
     if (task_should_compute_output(1)) {
       Tensor dk;
-      if (!patches.defined()) {  // the forward kept the input, not the patch matrix
+      if (pixels) patches = im2col(image, g, l);
+      if (!patches.defined()) {  // the forward was implicit
         dk = conv_dw(image, dy2, g, l, scale);
         if (!dk.defined()) patches = im2col(image, g, l);
       }
@@ -888,9 +890,10 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   }
   if (records(std::array<Tensor, 2>{x, kernel})) {
     auto node = make_node<ConvBackward>({x, kernel});
-    node->x.keep(x);
+    node->pixels = cols.defined() && cols.is_alias_of(x);
+    if (cols.defined() && !node->pixels) node->cols.keep(cols);
+    else node->x.keep(x);
     node->w2.keep(kernel.detach().view({g.k, g.cols()}));
-    node->cols.keep(cols);
     if (bs) node->saved.keep(std::move(lists), mask.value_or(Tensor()));
     node->g = g;
     node->p = bs ? p : 0.0;

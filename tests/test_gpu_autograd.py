@@ -201,3 +201,34 @@ def test_a_second_backward(name):
     assert _same(_grads(y, wrt), want)
     with pytest.raises(RuntimeError, match="second time"):
         _grads(y, wrt)
+
+
+@every_function
+@pytest.mark.parametrize("which", [0, 1])
+def test_an_operand_changed_before_the_backward_is_refused_where_it_is_read(name, which):
+    """(the image behind a patch matrix is not: the matrix is what was kept)"""
+    call, wrt, _ = FUNCTIONS[name]()
+    want = _grads(call(), wrt)
+    y = call()
+    with torch.no_grad():
+        wrt[which].mul_(2)
+    if name == "conv explicit" and which == 0:
+        assert _same(_grads(y, wrt), want)
+    else:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            _grads(y, wrt)
+
+
+def test_the_convolution_keeps_the_image_or_its_patch_matrix():
+    call, wrt, _ = _conv("explicit")
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+        call()
+    assert (4 * 18 * 18, 16 * 9) in kept and tuple(wrt[0].shape) not in kept
+    for form in ("implicit", "pointwise"):
+        call, wrt, _ = _conv(form)
+        kept.clear()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+            call()
+        big = [s for s in kept if len(s) == 4 or s[0] >= 256]
+        assert big == [tuple(wrt[0].shape)], form
