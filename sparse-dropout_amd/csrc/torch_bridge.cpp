@@ -546,7 +546,7 @@ struct MlpBackward : Node {
 };
 
 Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, const std::vector<double>& ps, int act,
-           const std::optional<std::vector<Tensor>>& masks, std::optional<uint64_t> seed, const OptTensor& state) {
+           const std::optional<std::vector<OptTensor>>& masks, std::optional<uint64_t> seed, const OptTensor& state) {
   const int n = (int)weights.size();
   bool two_d = input.dim() == 2;
   for (const Tensor& w : weights) two_d = two_d && w.dim() == 2;
@@ -575,7 +575,7 @@ Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, 
         // eval/mlp/model.py:31-33): the dense product with the same fused store, no mask and no lists
         out = dense(h, ws[0], a, want_pre, &pre);
       } else {
-        Draw draw{masks ? OptTensor((*masks)[i]) : OptTensor(),
+        Draw draw{masks ? (*masks)[i] : OptTensor(),
                   seed ? std::optional<uint64_t>(*seed + (uint64_t)i) : std::nullopt, state};
         out = layer_forward(h, ws[i], bs, ps[i], draw, a, want_pre, lists[i], &pre);
       }

@@ -30,8 +30,8 @@ def blockwise_dropout_mlp(input: torch.Tensor, weights, block_size, p, activatio
     """``W_n drop(act(... W_2 drop(act(W_1 drop(x))) ...))``: every layer drops blocks of its INPUT with
     probability p (a number, or one per layer; 0 keeps everything) and scales by 1/(1-p), ``activation``
     ("relu", "gelu" or None) sits between consecutive layers, none after the last.  ``masks`` (one bool mask per
-    layer, True = dropped) pins the masks, ``seed`` pins the draws (layer i uses seed + i); otherwise they come
-    from the device-resident generator.  ``input`` is [M, K], ``weights[i]`` is [out_i, in_i].
+    layer, True = dropped, or None where the layer draws one) pins the masks, ``seed`` pins the draws (layer i uses
+    seed + i); otherwise they come from the device-resident generator.  ``input`` is [M, K], ``weights[i]`` is [out_i, in_i].
 
     With the device-resident generator a first layer with p = 0 whose input needs no gradient draws nothing (it runs as
     a dense product): the following layers then use the generator's draws 0, 1, ...; when the input does require a

@@ -232,3 +232,15 @@ def test_the_convolution_keeps_the_image_or_its_patch_matrix():
             call()
         big = [s for s in kept if len(s) == 4 or s[0] >= 256]
         assert big == [tuple(wrt[0].shape)], form
+
+
+def test_masks_may_be_given_for_some_layers_only():
+    import flash_dropout.functional as F
+    from flash_dropout.hip import GEMM
+
+    _, (x, *ws), m0 = _mlp()
+    drawn = GEMM().random_lists(O.mask_shape(192, 256, BS), P, seed=7 + 1)[0]  # layer i draws from seed + i
+    m2 = _mask(192, 200, 2)
+    y = F.hip_blockwise_dropout_mlp(x, ws, BS, P, "relu", masks=[m0, None, m2], seed=7)
+    ref = F.hip_blockwise_dropout_mlp(x, ws, BS, P, "relu", masks=[m0, drawn, m2])
+    assert torch.equal(y, ref) and _same(_grads(y, (x, *ws)), _grads(ref, (x, *ws)))
