@@ -107,13 +107,14 @@ void check_pair(const Tensor& a, const Tensor& b) {
   TORCH_CHECK_VALUE(a.size(1) == b.size(1), "reduction dims differ: A ", a.sizes(), ", B ", b.sizes());
 }
 
+// The mask itself when it is row- or column-major in memory, else (expanded: stride 0, or doubly strided) a copy.
 Tensor check_mask(const Tensor& mask, int64_t mb, int64_t kb, const Tensor& like) {
   TORCH_CHECK_TYPE(mask.scalar_type() == at::kBool, "Mask must be bool (got ", mask.dtype(), ")");
   TORCH_CHECK_VALUE(mask.device() == like.device(), "mask must be on the same device as the operands");
   TORCH_CHECK_VALUE(mask.dim() == 2 && mask.size(0) == mb && mask.size(1) == kb, "mask shape ", mask.sizes(),
                     " does not match blocks [", mb, ", ", kb, "]");
-  if (mask.numel() && mask.stride(0) != 1 && mask.stride(1) != 1) return mask.contiguous();
-  return mask;
+  const bool expanded = (mb > 1 && mask.stride(0) == 0) || (kb > 1 && mask.stride(1) == 0);
+  return expanded || (mask.stride(0) != 1 && mask.stride(1) != 1) ? mask.contiguous() : mask;
 }
 
 struct MaskArg {
@@ -125,7 +126,7 @@ struct MaskArg {
       sr = m.size(1);
       sc = 1;
     }
-    sr = std::max<int64_t>(sr, 1);
+    sr = std::max<int64_t>(sr, 1);  // (of an extent of 1: no stride over more is 0 here)
     sc = std::max<int64_t>(sc, 1);
   }
 };

@@ -146,9 +146,14 @@ def _check_mask(mask: torch.Tensor, shape: tuple[int, int], like: torch.Tensor) 
         raise ValueError("mask must be on the same device as the operands")
     if tuple(mask.shape) != shape:
         raise ValueError(f"mask shape {tuple(mask.shape)} does not match blocks {shape}")
-    if mask.numel() and mask.stride(0) != 1 and mask.stride(1) != 1:
-        mask = mask.contiguous()
-    return mask
+    return _mask_matrix(mask)
+
+
+def _mask_matrix(mask: torch.Tensor) -> torch.Tensor:
+    """The mask itself when it is row- or column-major in memory, else (expanded: stride 0, or doubly strided) a copy."""
+    (mb, kb), (sr, sc) = mask.shape, mask.stride()
+    expanded = (mb > 1 and sr == 0) or (kb > 1 and sc == 0)
+    return mask.contiguous() if expanded or (mask.numel() and sr != 1 and sc != 1) else mask
 
 
 def _mask_strides(mask: torch.Tensor):
@@ -327,8 +332,7 @@ class GEMM:
         if mb == 0 or kb == 0:
             raise ValueError("mask must be non-empty")
         split, out_mb, out_kb = self._list_grid(mb, kb, split, grid)
-        if mask.stride(0) != 1 and mask.stride(1) != 1:
-            mask = mask.contiguous()
+        mask = _mask_matrix(mask)
         row_ptr, col_ptr, col_idx, row_idx = self._list_buffers(out_mb, out_kb, mask.device)
         with _guard(mask.device):
             self._call(self.lib.sd_build_lists_split, mask.data_ptr(), mb, kb, *_mask_strides(mask),

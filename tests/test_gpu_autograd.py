@@ -234,6 +234,15 @@ def test_the_convolution_keeps_the_image_or_its_patch_matrix():
         assert big == [tuple(wrt[0].shape)], form
 
 
+@every_function
+@pytest.mark.parametrize("along", [0, 1])
+def test_an_expanded_mask_is_the_mask_it_shows(name, along):
+    call, wrt, mask = FUNCTIONS[name]()
+    expanded = mask.narrow(along, 0, 1).expand(mask.shape)
+    y, want = call(expanded), call(expanded.contiguous())
+    assert torch.equal(y, want) and _same(_grads(y, wrt), _grads(want, wrt))
+
+
 def test_masks_may_be_given_for_some_layers_only():
     import flash_dropout.functional as F
     from flash_dropout.hip import GEMM

@@ -249,6 +249,25 @@ def test_as_matrix_lays_out_expanded_and_strided_views():
     assert _mat(torch.zeros(1, 8))[1:] == (8, 1)
 
 
+def test_masks_are_laid_out_before_their_strides_are_read():
+    """Element (r, c) has to lie at r * strides[0] + c * strides[1] of what is launched on, expanded masks included."""
+    from flash_dropout.hip.binding_gemm import _check_mask, _mask_strides
+
+    one_row, one_col = torch.rand(1, 7) < 0.5, torch.rand(5, 1) < 0.5
+    full = torch.rand(10, 14) < 0.5
+    masks = [one_row.expand(5, 7), one_col.expand(5, 7), one_row[:, :1].expand(5, 7), full[:5, :7], full[:5, :7].t(),
+             full[::2, ::2], one_row, one_col, one_row[:, ::2], one_row[:, :1].expand(5, 1), one_row[:, :1].expand(1, 7)]
+    for mask in masks:
+        m = _check_mask(mask, tuple(mask.shape), mask)
+        sr, sc = _mask_strides(m)
+        assert torch.equal(m, mask)
+        base = m.storage_offset()
+        last = base + (m.shape[0] - 1) * sr + (m.shape[1] - 1) * sc
+        assert last < m.untyped_storage().nbytes()
+        got = [[bool(m.untyped_storage()[base + r * sr + c * sc]) for c in range(m.shape[1])] for r in range(m.shape[0])]
+        assert got == mask.tolist(), (mask.shape, mask.stride())
+
+
 @pytest.mark.parametrize("name", ["mfma_ceiling.hip", "lds_load_ceiling.hip"])
 def test_ceiling_probes_compile_for_gfx950(name, tmp_path):
     """The stand-alone measurement programs under benchmark/ are only ever run on a GPU box by hand: keep them
