@@ -24,6 +24,7 @@ import torch
 
 from ..hip import _loader
 from ..hip.binding_gemm import GEMM, _block_size
+from .tracing import traceable
 
 
 def draw_source(like: torch.Tensor, seed: int | None):
@@ -33,6 +34,7 @@ def draw_source(like: torch.Tensor, seed: int | None):
     return None, (GEMM().rng_state(like.device) if like.is_cuda else None)
 
 
+@traceable
 def blockwise_dropout_matmul_mask(input: torch.Tensor, mask: torch.Tensor, block_size, p: float,
                                   weight: torch.Tensor) -> torch.Tensor:
     """Same as :func:`blockwise_dropout_matmul` with the mask given (True = dropped); argument order
@@ -42,6 +44,7 @@ def blockwise_dropout_matmul_mask(input: torch.Tensor, mask: torch.Tensor, block
     return _loader.bridge().linear(input, weight, mask, _block_size(block_size), p, None, None)
 
 
+@traceable
 def blockwise_dropout_matmul(input: torch.Tensor, weight: torch.Tensor, block_size, p: float,
                              seed: int | None = None) -> torch.Tensor:
     """``(keep ⊙ input)/(1-p) @ weight.T`` with a fresh block mask (reference: …_cuda.py:56-59).

@@ -23,8 +23,10 @@ import torch
 from ..hip import _loader
 from ..hip.binding_gemm import _activation, _block_size
 from .blockwise_dropout_matmul_hip import draw_source
+from .tracing import traceable
 
 
+@traceable
 def blockwise_dropout_mlp(input: torch.Tensor, weights, block_size, p, activation: str | None = "relu",
                           masks=None, seed: int | None = None) -> torch.Tensor:
     """``W_n drop(act(... W_2 drop(act(W_1 drop(x))) ...))``: every layer drops blocks of its INPUT with

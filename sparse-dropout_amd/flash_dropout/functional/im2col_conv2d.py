@@ -20,6 +20,7 @@ import torch.nn.functional as F
 from ..hip import _loader
 from ..hip.binding_gemm import GEMM, _block_size
 from .blockwise_dropout_matmul_hip import draw_source
+from .tracing import traceable
 
 
 # Use the implicit-GEMM forward (sd_conv2d_dsd_lists) where the library takes the geometry.  Module-level
@@ -51,6 +52,7 @@ def _conv2d(input, kernel, mask, block_size, p, padding, stride, dilation, draw=
                                    *draw, IMPLICIT_FORWARD, FUSED_INPUT_GRADIENT)
 
 
+@traceable
 def im2col_conv2d(input: torch.Tensor, kernel: torch.Tensor, padding=(0, 0), stride=(1, 1),
                   dilation=(1, 1)) -> torch.Tensor:
     """Dense convolution through the patch matrix (reference: im2col_conv2d.py:5-27)."""
@@ -65,6 +67,7 @@ def conv_patch_matrix_shape(input_shape, kernel_shape, padding=(0, 0), stride=(1
     return n * po * qo, c * r * s
 
 
+@traceable
 def blockwise_dropout_conv2d_mask(input, mask, block_size, p: float, kernel, padding=(0, 0),
                                   stride=(1, 1), dilation=(1, 1)) -> torch.Tensor:
     """Block-dropout convolution with the mask given: ``mask`` is bool
@@ -77,6 +80,7 @@ def blockwise_dropout_conv2d_mask(input, mask, block_size, p: float, kernel, pad
     return _conv2d(input, kernel, mask, bs, p, padding, stride, dilation)
 
 
+@traceable
 def blockwise_dropout_conv2d(input, kernel, block_size, p: float, padding=(0, 0), stride=(1, 1),
                              dilation=(1, 1), seed: int | None = None) -> torch.Tensor:
     """Block-dropout convolution with a fresh mask over the patch matrix, drawn on the device inside the

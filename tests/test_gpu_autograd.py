@@ -253,3 +253,38 @@ def test_masks_may_be_given_for_some_layers_only():
     y = F.hip_blockwise_dropout_mlp(x, ws, BS, P, "relu", masks=[m0, None, m2], seed=7)
     ref = F.hip_blockwise_dropout_mlp(x, ws, BS, P, "relu", masks=[m0, drawn, m2])
     assert torch.equal(y, ref) and _same(_grads(y, (x, *ws)), _grads(ref, (x, *ws)))
+
+
+@every_function
+def test_a_trace_records_the_function(name):
+    """The traced program computes on what it is given, gradients included."""
+    import flash_dropout.functional as F
+
+    _, wrt, _ = FUNCTIONS[name]()
+
+    def f(x, *ws):
+        if name == "linear":
+            y = F.hip_blockwise_dropout_matmul(x, ws[0], BS, P, seed=5)
+        elif name == "mlp":
+            y = F.hip_blockwise_dropout_mlp(x, list(ws), BS, P, "gelu", seed=5)
+        else:
+            y = F.blockwise_dropout_conv2d(x, ws[0], BS, P, seed=5)
+        return y * 2
+
+    traced = torch.jit.trace(f, wrt, check_trace=False)
+    other = [(t.detach() * 0.5).requires_grad_() for t in wrt]
+    y, want = traced(*other), f(*other)
+    assert torch.equal(y, want)
+    assert _same(_grads(y, other), _grads(want, other))
+    with torch.no_grad():
+        assert torch.equal(torch.jit.trace(f, wrt, check_trace=False)(*other), want)
+
+
+def test_a_trace_under_autocast_keeps_its_casts():
+    import flash_dropout.functional as F
+
+    x, w = _t(192, 136, seed=1, dtype=torch.float32), _t(72, 136, seed=2, dtype=torch.float32)
+    f = lambda a, b: F.hip_blockwise_dropout_matmul(a, b, BS, P, seed=5)  # noqa: E731
+    with torch.autocast("cuda", torch.bfloat16):
+        traced, want = torch.jit.trace(f, (x, w), check_trace=False), f(x, w)
+    assert torch.equal(traced(x, w), want) and want.dtype == torch.bfloat16

@@ -283,3 +283,40 @@ def test_ceiling_probes_compile_for_gfx950(name, tmp_path):
     assert proc.returncode == 0, proc.stderr[-2000:]
 
 
+
+
+def test_a_traced_call_is_one_operation_on_its_tensors():
+    """The recording itself, around a stand-in for the native call (its result is filled behind torch's back)."""
+    from flash_dropout.functional.tracing import traceable
+
+    class Native(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, *ws):
+            ctx.save_for_backward(x, *ws)
+            y = torch.empty(x.shape[0], ws[0].shape[0])
+            y.numpy()[:] = sum(x.detach().numpy() @ w.detach().numpy().T for w in ws)
+            return y
+
+        @staticmethod
+        def backward(ctx, g):
+            x, *ws = ctx.saved_tensors
+            return (sum(g @ w for w in ws), *(g.t() @ x for _ in ws))
+
+    @traceable
+    def product(x, ws, flag, mask=None):
+        assert flag == "flag" and (mask is None or mask.dtype == torch.bool)
+        return Native.apply(x if mask is None else x * mask, *ws)
+
+    def f(x, a, b, mask):
+        return product(x, (w for w in (a, b)), "flag", mask=mask) * 2
+
+    make = lambda seed: [torch.randn(*s, generator=torch.Generator().manual_seed(seed)).requires_grad_()  # noqa: E731
+                         for s in ((5, 4), (3, 4), (3, 4))] + [torch.arange(4) % 2 == seed % 2]
+    traced = torch.jit.trace(f, tuple(make(0)), check_trace=False)
+    args = make(1)
+    got, want = traced(*args), f(*args)
+    assert torch.equal(got, want)
+    dy = torch.randn(5, 3)
+    assert all(torch.equal(s, t) for s, t in zip(torch.autograd.grad(got, args[:3], dy), torch.autograd.grad(want, args[:3], dy)))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(got, args[:3], dy)
