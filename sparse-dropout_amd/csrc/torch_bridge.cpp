@@ -436,6 +436,9 @@ Tensor autocast(const Tensor& t) {
   return at::autocast::is_autocast_enabled(at::kCUDA) ? t.to(at::autocast::get_autocast_dtype(at::kCUDA)) : t;
 }
 
+// A gradient that is not there (a function behind the output returned none) counts as zeros in the nodes below, as it does
+// in Python autograd functions: the parameters get a gradient of zeros, not none.
+
 // ---- one layer ----------------------------------------------------------------------------------------------------------
 struct LinearBackward : Node {
   Saved x, w;
@@ -445,11 +448,10 @@ struct LinearBackward : Node {
     std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     variable_list out(2);
-    if (!grads[0].defined()) return out;
     const Tensor xs = x.matrix(), ws = w.matrix();
+    const Tensor dy = grads[0].defined() ? grad_matrix(grads[0], xs) : at::zeros({xs.size(0), ws.size(0)}, xs.options());
     const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
-    std::tie(out[0], out[1]) = layer_backward(grad_matrix(grads[0], xs), ws, xs, lists.get(), p, need_dx, need_dw,
-                                              SD_ACT_NONE, Tensor());
+    std::tie(out[0], out[1]) = layer_backward(dy, ws, xs, lists.get(), p, need_dx, need_dw, SD_ACT_NONE, Tensor());
     return out;
   }
   void release_variables() override {
@@ -504,9 +506,8 @@ struct MlpBackward : Node {
     at::NoGradGuard no_grad;
     const int n = (int)ws.size();
     variable_list out(1 + n);
-    if (!grads[0].defined()) return out;
     const Tensor x0 = x.matrix();
-    Tensor g = grad_matrix(grads[0], x0);
+    Tensor g = grads[0].defined() ? grad_matrix(grads[0], x0) : at::zeros({x0.size(0), ws.back().sizes[0]}, x0.options());
     for (int i = n - 1; i >= 0; --i) {
       const Tensor w = ws[i].matrix(), h = i ? hidden[i - 1].matrix() : x0;
       const Lists l = lists[i].get();
@@ -747,11 +748,10 @@ struct ConvBackward : Node {
     std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     variable_list out(2);
-    if (!grads[0].defined()) return out;
     const Tensor w = w2.get().contiguous(), image = x.get();
     const Lists lists = saved.get();
     Tensor patches = cols.matrix();
-    const Tensor dy2 = rows_gradient(grads[0], g, w);
+    const Tensor dy2 = grads[0].defined() ? rows_gradient(grads[0], g, w) : at::zeros({g.rows(), g.k}, w.options());
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
     if (task_should_compute_output(0)) {

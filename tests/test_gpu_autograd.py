@@ -256,6 +256,23 @@ def test_masks_may_be_given_for_some_layers_only():
 
 
 @every_function
+def test_a_gradient_that_is_not_there_counts_as_zeros(name):
+    class Blocks(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    call, wrt, _ = FUNCTIONS[name]()
+    Blocks.apply(call()).float().sum().backward()
+    for t in wrt:
+        assert t.grad is not None and not t.grad.any()
+
+
+@every_function
 def test_a_trace_records_the_function(name):
     """The traced program computes on what it is given, gradients included."""
     import flash_dropout.functional as F
