@@ -561,7 +561,8 @@ Tensor mlp(const Tensor& input, const std::vector<Tensor>& weights, int64_t bs, 
   inputs.insert(inputs.end(), ws.begin(), ws.end());
   refuse_forward_mode(inputs);
   const bool rec = records(inputs);
-  const bool x_grad = rec && x.requires_grad();
+  // (whether it is recorded or not: which of the generator's draws a layer takes does not depend on the gradient mode)
+  const bool x_grad = x.requires_grad();
   std::vector<Lists> lists(n);
   std::vector<Tensor> hidden, pres;
   Tensor h = x;

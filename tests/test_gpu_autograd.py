@@ -305,3 +305,20 @@ def test_a_trace_under_autocast_keeps_its_casts():
     with torch.autocast("cuda", torch.bfloat16):
         traced, want = torch.jit.trace(f, (x, w), check_trace=False), f(x, w)
     assert torch.equal(traced(x, w), want) and want.dtype == torch.bfloat16
+
+
+def test_draws_do_not_depend_on_the_gradient_mode():
+    """A stack whose first layer keeps everything and whose input asks for a gradient takes the same draws of the
+    generator when nothing is recorded."""
+    import flash_dropout.functional as F
+    from flash_dropout.hip import GEMM
+
+    _, (x, *ws), _ = _mlp()
+    ps = (0.0, P, P)
+    GEMM().manual_seed(11)
+    want = F.hip_blockwise_dropout_mlp(x, ws, BS, ps, "relu")
+    after = GEMM().rng_state().clone()
+    GEMM().manual_seed(11)
+    with torch.no_grad():
+        got = F.hip_blockwise_dropout_mlp(x, ws, BS, ps, "relu")
+    assert torch.equal(GEMM().rng_state(), after) and torch.equal(got, want)
