@@ -47,5 +47,8 @@ def blockwise_dropout_mlp(input: torch.Tensor, weights, block_size, p, activatio
         raise ValueError("p must be one probability in [0, 1), or one per layer")
     if masks is not None and len(masks) != len(weights):
         raise ValueError("one mask per layer is needed")
+    # the generator's state is made (a copy from the host) and reseeded when it is asked for: only where a mask is drawn
+    draws = any(m is None for m in masks) if masks is not None else len(weights) > 1 or ps[0] > 0 or input.requires_grad
     return _loader.bridge().mlp(input, weights, _block_size(block_size), ps, _activation(activation),
-                                None if masks is None else list(masks), *draw_source(input, seed))
+                                None if masks is None else list(masks),
+                                *(draw_source(input, seed) if draws else (None, None)))

@@ -320,3 +320,21 @@ def test_a_traced_call_is_one_operation_on_its_tensors():
     assert all(torch.equal(s, t) for s, t in zip(torch.autograd.grad(got, args[:3], dy), torch.autograd.grad(want, args[:3], dy)))
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(got, args[:3], dy)
+
+
+def test_the_generator_is_asked_only_where_a_mask_is_drawn(monkeypatch):
+    import sys
+
+    import flash_dropout.functional as F
+
+    mod = sys.modules[F.hip_blockwise_dropout_mlp.__module__]
+    calls = []
+    monkeypatch.setattr(mod, "draw_source", lambda like, seed: calls.append(seed) or (None, "state"))
+    monkeypatch.setattr(mod._loader, "bridge", lambda: type("B", (), {"mlp": staticmethod(lambda *a: a)}))
+    x, w, m = torch.zeros(4, 4), [torch.zeros(4, 4)] * 2, torch.zeros(1, 1, dtype=torch.bool)
+    for args, kw, drawn in (((w, 64, 0.5), dict(masks=[m, m]), False), ((w, 64, 0.5), dict(masks=[m, None]), True),
+                            ((w, 64, 0.5), {}, True), ((w[:1], 64, 0.0), {}, False), ((w[:1], 64, 0.1), {}, True)):
+        calls.clear()
+        out = F.hip_blockwise_dropout_mlp(x, *args, **kw)
+        assert bool(calls) == drawn and out[-1] == ("state" if drawn else None)
+    assert F.hip_blockwise_dropout_mlp(x.requires_grad_(), w[:1], 64, 0.0)[-1] == "state"  # draws the (all kept) mask
