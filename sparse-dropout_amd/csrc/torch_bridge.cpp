@@ -833,6 +833,9 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   TORCH_CHECK_VALUE(input.dim() == 4 && kernel_in.dim() == 4, "input must be (N, C, H, W) and kernel (K, C, R, S)");
   TORCH_CHECK_VALUE(input.size(1) == kernel_in.size(1), "channel mismatch: input ", input.size(1), ", kernel ",
                     kernel_in.size(1));
+  for (int i = 0; i < 2; ++i)  // (before anything is divided by them)
+    TORCH_CHECK_VALUE(stride[i] > 0 && dilation[i] > 0 && padding[i] >= 0,
+                      "strides and dilations must be positive, paddings non-negative");
   const Tensor x = autocast(input), kernel = autocast(kernel_in).contiguous();
   refuse_forward_mode(std::array<Tensor, 2>{x, kernel});
   TORCH_CHECK_VALUE(x.is_cuda() && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16),

@@ -338,3 +338,15 @@ def test_the_generator_is_asked_only_where_a_mask_is_drawn(monkeypatch):
         out = F.hip_blockwise_dropout_mlp(x, *args, **kw)
         assert bool(calls) == drawn and out[-1] == ("state" if drawn else None)
     assert F.hip_blockwise_dropout_mlp(x.requires_grad_(), w[:1], 64, 0.0)[-1] == "state"  # draws the (all kept) mask
+
+
+@pytest.mark.parametrize("geometry", [dict(stride=0), dict(stride=(1, -1)), dict(dilation=0), dict(padding=(0, -1))])
+def test_conv_geometry_is_checked_before_it_is_used(geometry):
+    """(also in front of every other check of the operands: a stride of 0 is a division by zero in native code)"""
+    import flash_dropout.functional as F
+
+    x, k = torch.zeros(1, 4, 8, 8, dtype=torch.float16), torch.zeros(4, 4, 3, 3, dtype=torch.float16)
+    for call in (lambda: F.im2col_conv2d(x, k, **geometry),
+                 lambda: F.blockwise_dropout_conv2d_mask(x, torch.zeros(1, 1, dtype=torch.bool), 64, 0.5, k, **geometry)):
+        with pytest.raises(ValueError, match="strides and dilations"):
+            call()
