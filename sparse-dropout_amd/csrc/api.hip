@@ -291,7 +291,7 @@ int64_t sd_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t block
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   int splits = generic_splits(M, N, K, sparse ? block_size : 0, sparse ? kDsd : kDense);
   if (!sparse || block_size == 64) {
-    const int fs = fast_splits(M, N, K);
+    const int fs = fast_splits(M, N, K, sparse != 0);
     if (fs > splits) splits = fs;
   }
   return splits > 1 ? (int64_t)splits * M * N * 4 : 0;

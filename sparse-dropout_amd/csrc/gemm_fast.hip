@@ -1779,64 +1779,102 @@ int splits_for(int64_t tiles, int64_t M, int64_t N, int64_t K) {
   while (want > 1 && want * M * N * 4 > (256LL << 20)) --want;
   return want < 2 ? 1 : (int)want;
 }
-// Microseconds a product is expected to take, from measured times per step (a 64-deep slice of the reduction) of a full
-// round of workgroups: 0.32 / 0.42 for 64 x 64 tiles at one / two per CU, 0.55 for 128 x 128 at one, 1.03 at two, 1.62
-// for 256 x 256 (two thirds more where its edges are ragged: that instance runs the older loop), plus what a round costs
-// outside its loop and, for a split reduction, the pass over the fp32 partials.  The drop rate is not known here; a step
-// of the smaller shapes is skipped more often (every row block of the tile must drop it), for which three quarters
-// of the blocks kept are assumed.
-double product_time(int shape, int64_t M, int64_t N, int64_t kb, int splits, bool ragged) {
-  const int64_t wgs = shape_tiles(shape, M, N) * splits;
-  const double steps = (double)((kb + splits - 1) / splits);
-  double t;
-  if (shape == kShapeOne) {
-    const int64_t rounds = (wgs + 511) / 512, last = wgs - (rounds - 1) * 512;
-    t = 0.75 * steps * (0.42 * (double)(rounds - 1) + (last <= 256 ? 0.32 : 0.42)) + 2.0 * (double)rounds;
-  } else if (shape == kShapeQuad) {
-    t = (double)((wgs + 255) / 256) * (0.94 * 0.55 * steps + 3.0);
-  } else if (shape == kShapeWide) {
-    const int64_t rounds = (wgs + 511) / 512, last = wgs - (rounds - 1) * 512;
-    t = 0.94 * steps * (1.03 * (double)(rounds - 1) + (last <= 256 ? 0.70 : 1.03)) + 4.0 * (double)rounds;
-  } else {
-    t = (double)((wgs + 255) / 256) * ((ragged ? 2.7 : 1.62) * steps + 7.0);
+// ---- what a product is expected to take on each shape -----------------------------------------------------------------
+// Microseconds, fitted to graph-replayed times of 6250 drawn layers (64 to 262144 rows, widths of 16 to 8192, up to 8192^3, every
+// shape and up to four cuts of the reduction each, drop rates of 0 to 0.75, both element types): a start, a step (a
+// 64-deep slice of the reduction) of a workgroup when one, two or three share its CU, what a full round of workgroups and a
+// thousand 64 x 64 blocks of the result cost besides.  The shape with the smallest expected time is over the best one by 1.4 %
+// (forward) and 1.0 % (weight gradient) on average.  The constants before these were fitted to a few sizes near one round of
+// workgroups and gave large outputs to the 64 x 64 shape: 4.9 and 6.0 % on the same layers, on those above 4e10 products 6.1
+// and 17.9 %, one in ten 26 and 95 % or more; 4224 x 4800 -> 2048 took 160 us forward (99 on the big shape), the weight gradient
+// of 13888 x 2840 -> 3472 1124 us (346).
+struct ShapeCost {
+  int resident;               // workgroups to a CU
+  double start, step[3];      // step[n - 1]: with n workgroups on the CU
+  double kept;                // share of a step's cost that follows the kept blocks; the rest is paid once any is kept
+  double round;               // per round that fills the chip
+  double store, relu, gelu;   // per thousand blocks
+  double ragged;              // of a step's cost on top
+  double act(int a) const { return a == SD_ACT_GELU ? gelu : (a == SD_ACT_RELU ? relu : 0.0); }
+};
+//                                       resident start  step                kept  round store relu  gelu  ragged
+constexpr ShapeCost kForwardOneFew =    {2,       5.77,  {0.23, 0.43, 0.},   0.,   0.,   5.64, 0.39, 1.85, 0.};
+constexpr ShapeCost kForwardCost[4] = { {3,       5.77,  {0.23, 0.43, 0.70}, 0.,   0.,   5.64, 0.39, 1.85, 0.},
+                                        {1,       7.22,  {0.51, 0., 0.},     0.42, 4.29, 0.98, 0.32, 2.99, 0.},
+                                        {2,       6.34,  {0.62, 0.93, 0.},   0.37, 2.07, 1.73, 0.14, 2.25, 0.},
+                                        {1,       10.61, {1.14, 0., 0.},     0.56, 6.00, 1.23, 0.53, 3.69, 0.48}};
+constexpr ShapeCost kGradientCost[4] = {{2,       4.79,  {0.26, 0.45, 0.},   0.,   0.92, 4.31, 0.,   0.,   0.},
+                                        {1,       6.44,  {0.45, 0., 0.},     0.22, 1.53, 4.69, 0.,   0.,   0.},
+                                        {2,       4.63,  {0.61, 0.81, 0.},   0.18, 0.,   3.41, 0.,   0.,   0.},
+                                        {1,       5.95,  {1.20, 0., 0.},     0.55, 0.,   2.89, 0.,   0.,   0.41}};
+
+// A product on a shape: workgroups, steps of one of them, and what it costs beside them.
+struct ShapeWork {
+  const ShapeCost& cost;
+  double wgs, steps, rest;
+  double time() const {  // in rounds over the 256 CUs
+    const int64_t n = (int64_t)(wgs + 0.999), per_cu = (n + 255) / 256, full = n > 0 ? (per_cu - 1) / cost.resident : 0;
+    const int64_t last = per_cu - full * cost.resident;  // workgroups a CU has in the last round
+    return cost.start + (double)full * (steps * cost.step[cost.resident - 1] + cost.round) + rest +
+           steps * cost.step[last < 1 ? 0 : last - 1];
   }
-  if (splits > 1) t += 4.0 + (double)splits * (double)M * (double)N * 8.0 / 4.0e6;
-  return t;
+};
+
+// kept: fraction of kept blocks a plan counts with
+ShapeWork dsd_work(bool kc, int shape, int64_t M, int64_t N, int64_t K, int splits, double kept, int act) {
+  const int64_t wgs = shape_tiles(shape, M, N) * splits;
+  ShapeWork w{!kc ? kGradientCost[shape] : (shape == kShapeOne && wgs <= 512 ? kForwardOneFew : kForwardCost[shape]), 0., 0., 0.};
+  const int rows = shape == kShapeOne ? 1 : (shape == kShapeBig ? 4 : 2);
+  double none = 1.0;  // chance that no row block of the tile keeps a step
+  for (int r = 0; r < rows; ++r) none *= 1.0 - kept;
+  const bool ragged = M % BS || N % BS || K % BS;
+  w.wgs = (double)wgs;
+  w.steps = (double)((blocks_of(K) + splits - 1) / splits) * ((1.0 - w.cost.kept) * (1.0 - none) + w.cost.kept * kept) *
+            (ragged ? 1.0 + w.cost.ragged : 1.0);
+  w.rest = (w.cost.store + w.cost.act(act)) * (double)(blocks_of(M) * blocks_of(N)) * 1e-3;
+  if (splits > 1) w.rest += 3.5 + (double)splits * (0.02 + 2.2e-6 * (double)M * (double)N);  // the pass over the fp32 partials
+  return w;
 }
+
+// What a plan counts as kept; it is not told the drop rate, which matters little (told it, plans for rates of 0 to 0.75 would be
+// 0.1 to 0.2 % nearer to the best): three quarters of the blocks, nearly all 64-blocks of a mask of 32-blocks, all of a
+// dense product.
+double planned_kept(const GemmArgs& g) { return !g.row_ptr ? 1.0 : (g.quads ? 0.95 : 0.75); }
+
 // kc: reduction-contiguous operands.  Those (the forward) are split by a rule on the extents alone, whatever the shape:
 // where a sum is cut decides its last bit, and a ReLU behind it must see the same signs on every shape.
-DsdPlan plan_dsd(int64_t M, int64_t N, int64_t K, bool kc) {
+DsdPlan plan_dsd(int64_t M, int64_t N, int64_t K, bool kc, double kept, int act) {
   if (M <= 0 || N <= 0 || K <= 0) return {kShapeBig, 1};
   const int policy = tile_policy.load(std::memory_order_relaxed);
   const int64_t kb = blocks_of(K), big = shape_tiles(kShapeBig, M, N);
   if (policy == kTileBig) return {kShapeBig, splits_for(big, M, N, K)};
   const int64_t fixed = !kc ? 0 : splits_for(policy == kTileMid || big <= 128 ? shape_tiles(kShapeQuad, M, N) : big, M, N, K);
-  const bool ragged = M % BS || N % BS || K % BS;
   DsdPlan best{kShapeWide, 1};
   double t_best = 1e30;
   for (int shape = kShapeOne; shape <= kShapeBig; ++shape) {
     if (policy == kTileMid && shape != kShapeQuad && shape != kShapeWide) continue;
-    const int64_t tiles = shape_tiles(shape, M, N);
-    if (shape == kShapeQuad && tiles > 256) continue;
-    // no split, a full round of workgroups, or half of one
-    const int64_t round = shape == kShapeOne ? 512 : 256;
-    for (int64_t want = kc ? fixed : 1;;) {
-      const int64_t most = shape == kShapeBig ? 1024 : kTileMaxSteps;
+    if (shape == kShapeBig && !kc && (M % 8 || N % 8)) continue;  // (DsdForm::big_ok)
+    // results of one column block: even with the 64 x 64 shape in the forward (within 7 % either way on 16384 rows and more),
+    // which loads nothing beside them
+    if (shape == kShapeWide && kc && blocks_of(N) == 1 && policy == kTileAuto) continue;
+    // no split, or half a round, one round or two rounds of workgroups
+    const int64_t tiles = shape_tiles(shape, M, N), round = shape == kShapeOne || shape == kShapeWide ? 512 : 256;
+    const int64_t most = shape == kShapeBig ? 1024 : kTileMaxSteps;
+    int64_t s_before = 0;
+    for (const int64_t want : {kc ? fixed : (int64_t)1, round / 2 / tiles, round / tiles, 2 * round / tiles}) {
       int64_t s = want;
       if (!kc && s > kb / 4) s = kb / 4;
       while (s > 1 && s * M * N * 4 > (256LL << 20)) --s;
       if (s < 1) s = 1;
-      if ((kb + s - 1) / s <= most) {
-        const double t = product_time(shape, M, N, kb, (int)s, ragged);
+      if (s > s_before && (kb + s - 1) / s <= most) {
+        s_before = s;
+        const double t = dsd_work(kc, shape, M, N, K, (int)s, kept, act).time();
         if (t < t_best) {
           t_best = t;
           best = {shape, (int)s};
         }
       }
-      if (kc || shape == kShapeWide || shape == kShapeBig || 2 * tiles > round) break;
-      if (want == 1) want = (round / 2) / tiles > 1 ? (round / 2) / tiles : round / tiles;
-      else if (want == round / tiles) break;
-      else want = round / tiles;
+      if (kc) break;
     }
   }
   return best;
@@ -2072,7 +2110,7 @@ DsdForm dsd_form(const GemmArgs& g) {
 // The plan for this product and these operands, its splits cut down to what the caller's scratch holds; splits == 0: a
 // workgroup could not walk its share of the reduction.
 DsdPlan plan_for(const GemmArgs& g, const DsdForm& f) {
-  DsdPlan plan = plan_dsd(g.M, g.N, g.K, f.kc);
+  DsdPlan plan = plan_dsd(g.M, g.N, g.K, f.kc, planned_kept(g), g.act);
   if (plan.shape == kShapeBig && !f.big_ok) plan.shape = kShapeWide;
   const int64_t part_bytes = g.M * g.N * 4;
   if (plan.splits > 1 && (g.ws == nullptr || g.ws_bytes < part_bytes * plan.splits))
@@ -2237,9 +2275,9 @@ int set_tile_policy(int policy) {
   return tile_policy.exchange(policy, std::memory_order_relaxed);
 }
 
-int fast_splits(int64_t M, int64_t N, int64_t K) {  // for either operand form
-  const int a = plan_dsd(M, N, K, true).splits, b = plan_dsd(M, N, K, false).splits;
-  return a > b ? a : b;
+int fast_splits(int64_t M, int64_t N, int64_t K, bool sparse) {  // for either operand form; a plan takes what scratch there is
+  const double kept = sparse ? 0.75 : 1.0;
+  return std::max(plan_dsd(M, N, K, true, kept, SD_ACT_NONE).splits, plan_dsd(M, N, K, false, kept, SD_ACT_NONE).splits);
 }
 
 }  // namespace sd
