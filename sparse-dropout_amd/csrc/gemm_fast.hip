@@ -1784,10 +1784,10 @@ int splits_for(int64_t tiles, int64_t M, int64_t N, int64_t K) {
 // shape and up to four cuts of the reduction each, drop rates of 0 to 0.75, both element types): a start, a step (a
 // 64-deep slice of the reduction) of a workgroup when one, two or three share its CU, what a full round of workgroups and a
 // thousand 64 x 64 blocks of the result cost besides.  The shape with the smallest expected time is over the best one by 1.4 %
-// (forward) and 1.0 % (weight gradient) on average.  The constants before these were fitted to a few sizes near one round of
-// workgroups and gave large outputs to the 64 x 64 shape: 4.9 and 6.0 % on the same layers, on those above 4e10 products 6.1
-// and 17.9 %, one in ten 26 and 95 % or more; 4224 x 4800 -> 2048 took 160 us forward (99 on the big shape), the weight gradient
-// of 13888 x 2840 -> 3472 1124 us (346).
+// (forward) and 1.0 % (weight gradient) on average, on 900 layers drawn afterwards by 2.3 and 1.2 %.  The constants before
+// these were fitted to a few sizes near one round of workgroups and gave large outputs to the 64 x 64 shape: 4.9 and 6.0 % on
+// the same 6250, on those above 4e10 products 6.1 and 17.9 %, one in ten 26 and 95 % or more; 4224 x 4800 -> 2048 took 160 us
+// forward (99 on the big shape), the weight gradient of 13888 x 2840 -> 3472 1124 us (346).
 struct ShapeCost {
   int resident;               // workgroups to a CU
   double start, step[3];      // step[n - 1]: with n workgroups on the CU
@@ -1807,16 +1807,21 @@ constexpr ShapeCost kGradientCost[4] = {{2,       4.79,  {0.26, 0.45, 0.},   0.,
                                         {1,       6.44,  {0.45, 0., 0.},     0.22, 1.53, 4.69, 0.,   0.,   0.},
                                         {2,       4.63,  {0.61, 0.81, 0.},   0.18, 0.,   3.41, 0.,   0.,   0.},
                                         {1,       5.95,  {1.20, 0., 0.},     0.55, 0.,   2.89, 0.,   0.,   0.41}};
+// SDD: a step is one of the whole reduction's, for a workgroup's kept tiles
+constexpr ShapeCost kSddCost[4] = {     {2,       4.22,  {0.24, 0.40, 0.},   0.,   0.,   4.07, 1.69, 2.82, 0.29},
+                                        {1,       5.47,  {0.46, 0., 0.},     0.,   0.,   4.51, 2.28, 4.83, 0.19},
+                                        {3,       4.73,  {0.52, 0.61, 0.85}, 0.,   0.,   2.03, 1.44, 3.09, 0.24},
+                                        {1,       14.19, {1.20, 0., 0.},     0.,   0.,   2.52, 3.26, 5.49, 0.24}};
 
 // A product on a shape: workgroups, steps of one of them, and what it costs beside them.
 struct ShapeWork {
   const ShapeCost& cost;
   double wgs, steps, rest;
+  double full_step() const { return steps * cost.step[cost.resident - 1]; }  // a workgroup's steps on a full CU
   double time() const {  // in rounds over the 256 CUs
     const int64_t n = (int64_t)(wgs + 0.999), per_cu = (n + 255) / 256, full = n > 0 ? (per_cu - 1) / cost.resident : 0;
     const int64_t last = per_cu - full * cost.resident;  // workgroups a CU has in the last round
-    return cost.start + (double)full * (steps * cost.step[cost.resident - 1] + cost.round) + rest +
-           steps * cost.step[last < 1 ? 0 : last - 1];
+    return cost.start + (double)full * (full_step() + cost.round) + rest + steps * cost.step[last < 1 ? 0 : last - 1];
   }
 };
 
@@ -1915,40 +1920,59 @@ bool sdd_big_ok(const GemmArgs& g) {
          blocks_of(g.N) <= G_MAX_CB;
 }
 
-// Whether the strips of two beat the big shape: on short reductions, where what counts is how the grid fills its rounds and
-// whose store runs under other products, and on few kept tiles.  Fitted (us) to sizes of 4096 to 16384 rows and 1024 to
-// 8192 columns over reductions of 256 to 4096 at p = 0.1, 0.3, 0.5, 0.75, without and with GELU's derivative: the big shape
-// takes whole rounds of 256 groups whatever is kept, the strips (three to a CU) as many rounds as there are kept tiles.
-// With the derivative, at p = 0.1 / 0.5, big against strips: 16384 x 1536 from 384 (a round and a half) 72 / 65 us, 53 / 37;
-// 16384 x 1024 from 256 (one round) 34 / 33, 33 / 24; 4096 x 4096 from 1024 58 / 52, 58 / 39; from 2048 76 / 74, 89 / 60; from
-// 4096 118 / 112, 156 / 107, and at p = 0.75 104 against 62.  Not on outputs wider than twice their height, where a
-// strip's share of W is not in the L2 any more (2048 x 8192 from 2048 at p = 0.5: 61 against 83), nor on masks of
-// 32-blocks or reductions outside that range, which were not measured.
-bool strips_beat_big(const GemmArgs& g) {
-  const double kb = (double)blocks_of(g.K), kept = (double)(blocks_of(g.M) * blocks_of(g.N)) * kept_fraction(g);
-  if (kb < 4 || kb > 64 || g.quads || !g.row_ptr || blocks_of(g.N) > 2 * blocks_of(g.M)) return false;
-  const bool gelu = g.act == SD_ACT_GELU;
-  const double rounds = (double)((sdd_big_groups(g) + 255) / 256), strip_rounds = kept / 1536.0;
-  const double big = rounds * (17.0 + 1.4 * kb) * (rounds >= 4 ? 0.9 : 1.0) + (gelu ? 11.0 * rounds : 0.0);
-  const double strips = 9.0 + (strip_rounds + 0.5) * (2.0 + 0.75 * kb) * (strip_rounds > 4.0 ? 1.2 : 1.0) + (gelu ? 0.0026 * kept : 0.0);
-  return strips < 0.92 * big;
+// Workgroups of an SDD strip shape that have kept tiles, eight times as many as the XCD with the most of them gets.  The grid
+// holds every strip a row could fill, those of one row next to each other, kept ones first; an XCD takes a contiguous eighth
+// of an order that walks eight rows at a time, so that its part can be all kept strips (1371 x 2304 from 7104 at p = 0.5, 64 x 64
+// tiles: 792 workgroups, 396 of them kept, take the time of 792).
+double busy_strips(const GemmArgs& g, int cols, double keep) {
+  const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), per_row = (double)((blocks_of(g.N) + cols - 1) / cols);
+  const double grid = Mb * per_row;
+  if (keep > 0.999) return grid;
+  double kept = Cb * keep / cols + (cols - 1) / (2.0 * cols);  // a row's kept tiles end inside its last strip
+  kept = std::min(std::max(kept, std::min(1.0, Cb * keep)), per_row);
+  const double walk = 8.0 * per_row, run = grid / 8.0, whole = (double)(int64_t)(run / walk);
+  return std::max(1.0, std::min(grid, 8.0 * (whole * 8.0 * kept + std::min(run - whole * walk, 8.0 * kept))));
 }
 
-// The big shape when its grid gives more than half of the CUs a workgroup (on aligned operands: its edge instance runs
-// the older loop), unless strips of two are faster and nothing wants the big shape (`with_big`: a weight gradient on it
-// shares the launch); else by the number of kept tiles: up to about one 64 x 64 tile per CU one to a workgroup, else
-// strips of four while their grid is at most two rounds, else strips of two, three workgroups to a CU.
-int plan_sdd(const GemmArgs& g, bool with_big = false) {
-  const int policy = tile_policy.load(std::memory_order_relaxed);
-  const int64_t Mb = blocks_of(g.M), Cb = blocks_of(g.N);
-  const bool ragged = g.N % BS || g.K % BS;
-  if (sdd_big_ok(g)) {
-    if (policy == kTileBig) return kShapeBig;
-    if (policy == kTileAuto && !ragged && sdd_big_groups(g) > 128) return !with_big && strips_beat_big(g) ? kShapeWide : kShapeBig;
+// The SDD product on a shape: its kept tiles in strips of one, four or two, or groups of the big shape.
+ShapeWork sdd_work(int shape, const GemmArgs& g) {
+  const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), hint = kept_fraction(g);
+  const double keep = g.quads ? 1.0 - (1.0 - hint) * (1.0 - hint) * (1.0 - hint) * (1.0 - hint) : hint;  // of the 64-blocks
+  ShapeWork w{kSddCost[shape], 0., 0., 0.};
+  w.wgs = shape == kShapeBig ? (double)sdd_big_groups(g) : busy_strips(g, shape == kShapeOne ? 1 : (shape == kShapeQuad ? 4 : 2), keep);
+  double extra = g.N % BS || g.K % BS ? w.cost.ragged : 0.0;
+  if (shape == kShapeBig) {
+    w.steps = (double)blocks_of(g.K) * (0.8 + 0.28 * keep);  // groups of more column blocks, fewer of their tiles kept
+  } else {
+    // Rows that end anywhere cost the strips more the more W there is (log2 of its megabytes), tile rows lying across 128-byte
+    // lines; and past 24 MB of W every row's strips fetch their own columns from outside the caches, which strips of two
+    // do twice as often for a row of dY as strips of four (6656 x 6736 from 7008, ragged, p = 0.1: 1474 us; 635 on the big shape).
+    const double mb = std::log2((double)g.N * (double)g.K * 2e-6), cold = std::max(0.0, mb - 4.5);
+    const double each = shape == kShapeWide ? 0.22 - 0.12 * keep + (extra > 0.0 ? 0.16 : 0.0) : (shape == kShapeQuad ? 0.1 : 0.2);
+    extra = extra * (0.6 + 0.25 * std::min(std::max(mb, 0.0), 4.0)) + cold * each;
+    w.steps = (double)blocks_of(g.K);
   }
+  w.steps *= 1.0 + extra;
+  w.rest = (w.cost.store * Mb * Cb + w.cost.act(g.act) * Mb * Cb * keep) * 1e-3;
+  return w;
+}
+
+// The shape with the smallest expected time: 1.5 % over the best one on average on reductions of four blocks and more (1.6 % on
+// 900 layers drawn afterwards).  The rules before (limits on the number of groups, of kept tiles and of strips, and a formula
+// for strips of two on reductions of 256 to 4096) were 8.5 % over it, one in ten 30 % or more, most of them ragged (33 % on
+// average above 4e10 products): dX of 11904 x 6344 from 6112 at p = 0.2 with GELU 2173 us on strips, 920 on the big shape.
+// Shorter reductions stay where they were, on the big shape, when its grid gives more than half of the CUs a workgroup;
+// strips of two are faster there too (11415 x 2560 from 128 with GELU: 62 against 27 us), which is left as it is.
+int plan_sdd(const GemmArgs& g) {
+  const int policy = tile_policy.load(std::memory_order_relaxed);
+  const bool ragged = g.N % BS || g.K % BS, brief = blocks_of(g.K) < 4;
+  const bool big = sdd_big_ok(g);
   if (policy == kTileMid) return kShapeWide;
-  if ((double)(Mb * Cb) * kept_fraction(g) <= 320.0) return kShapeOne;
-  return Mb * ((Cb + 3) / 4) <= 512 ? kShapeQuad : kShapeWide;
+  if (big && (policy == kTileBig || (brief && !ragged && sdd_big_groups(g) > 128))) return kShapeBig;
+  int best = kShapeOne;
+  for (int shape = kShapeQuad; shape <= (big && !brief ? kShapeBig : kShapeWide); ++shape)
+    if (sdd_work(shape, g).time() < sdd_work(best, g).time()) best = shape;
+  return best;
 }
 
 int try_sdd(const GemmArgs& g, int dtype, hipStream_t stream) {
@@ -2241,12 +2265,32 @@ int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipS
   if (!gw.row_ptr || gw.bs != BS || gw.act || !form.ok || form.kc || !form.cm || gw.c_sr != 1) return SD_ERR_UNSUPPORTED;
   const DsdPlan plan = plan_for(gw, form);
   if (plan.splits < 1) return SD_ERR_UNSUPPORTED;
-  const int x_shape = plan_sdd(gx, plan.shape == kShapeBig);
-  // Worth it only while neither product fills the chip by itself: side by side, two large products get in each
-  // other's way in the L2 (8192^3 at p = 0.5: 1.33 ms in one launch against 1.28 in two; 1024^3: 27 us against 46).
-  if (x_shape == kShapeBig || plan.shape == kShapeBig) {
-    if (x_shape != plan.shape || sdd_big_groups(gx) > pair_limit() ||
-        shape_tiles(kShapeBig, gw.M, gw.N) * plan.splits > pair_limit())
+  // Side by side the products fill each other's last rounds and save a launch: measured on 2800 layers with each product on
+  // every shape, one launch against two takes 4 us less on 64 x 64 tiles, 7 on strips of four beside 128 x 128 tiles and 12 on
+  // the big shapes, and more where neither fills its last round: then what counts is the steps of all workgroups laid over
+  // the chip (dX and dW of 3328 x 5632 -> 2240 at p = 0.3 on the big shapes: 113 + 72 us, 139 together).  dX gives up its own
+  // shape where one launch on the weight gradient's is expected to be faster; the weight gradient keeps its cuts and, between
+  // the 64 x 64 and 128 x 128 shapes, its bits.  On those layers the choice is 3.8 % over the best of all ways on average
+  // (5.2 % on 900 drawn afterwards, reductions of less than four blocks included); the rule before, one launch wherever the
+  // shapes allowed it, 9.9 %.  Two large products get in each other's way in the L2 (8192^3 at p = 0.5: 1.33 ms in one launch
+  // against 1.28 in two), hence the limits.
+  const bool big = plan.shape == kShapeBig;
+  const int x_alone = plan_sdd(gx);
+  const int64_t limit = pair_limit();
+  const double kept = planned_kept(gw);
+  auto w_work = [&](int shape) { return dsd_work(false, shape, gw.M, gw.N, gw.K, plan.splits, kept, SD_ACT_NONE); };
+  auto pair_time = [&](int shape) {
+    const ShapeWork w = w_work(shape), x = sdd_work(shape, gx);
+    constexpr double gain[4] = {4.0, 7.0, 0.0, 12.0}, start[4] = {2.6, 5.4, 0.0, 12.1}, spread[4] = {1.07, 1.19, 0.0, 1.16};
+    const double slots = shape == kShapeOne ? 512.0 : 256.0;
+    const double laid = spread[shape] * (w.wgs * w.full_step() + x.wgs * x.full_step()) / slots;
+    return std::min(w.time() + x.time() - gain[shape],
+                    start[shape] + std::max(laid, std::max(w.full_step(), x.full_step())) + w.rest + x.rest);
+  };
+  const double apart = w_work(plan.shape).time() + sdd_work(x_alone, gx).time();
+  if (big) {
+    if (!sdd_big_ok(gx) || (x_alone != kShapeBig && (blocks_of(gx.K) < 4 || pair_time(kShapeBig) > apart)) ||
+        sdd_big_groups(gx) > limit || shape_tiles(kShapeBig, gw.M, gw.N) * plan.splits > limit)
       return SD_ERR_UNSUPPORTED;
     const bool edge = gx.N % BS != 0 || gx.K % BS != 0 || form.ragged;
     int rc;
@@ -2258,15 +2302,24 @@ int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipS
     note_kernel("pair:sdd+dsd:big%s splits=%d", edge ? ":ragged" : "", plan.splits);
     return plan.splits > 1 ? launch_splitk_reduce(gw, plan.splits, true, dtype, stream) : SD_OK;
   }
-  // The loading-wave shapes go together: dX takes the weight gradient's workgroup size (its results are the same bits on
-  // either, and a launch saved is more than the shapes differ by).
-  if (x_shape == kShapeWide || plan.shape == kShapeWide) return SD_ERR_UNSUPPORTED;
-  const int64_t x_wgs = blocks_of(gx.M) * (plan.shape == kShapeOne ? blocks_of(gx.N) : (blocks_of(gx.N) + 3) / 4);
-  if (x_wgs > 2 * pair_limit() || shape_tiles(plan.shape, gw.M, gw.N) * plan.splits > pair_limit()) return SD_ERR_UNSUPPORTED;
-  const int rc = is_bf16(dtype) ? tile_pair<BF16>(gx, gw, plan.shape, plan.splits, stream)
-                                : tile_pair<F16>(gx, gw, plan.shape, plan.splits, stream);
+  if (x_alone == kShapeBig && blocks_of(gx.K) < 4) return SD_ERR_UNSUPPORTED;
+  if (tile_policy.load(std::memory_order_relaxed) != kTileAuto) return SD_ERR_UNSUPPORTED;
+  int shape = -1;
+  double t_best = apart;
+  for (const int s : {(int)kShapeOne, (int)kShapeQuad}) {
+    const int64_t x_wgs = blocks_of(gx.M) * (s == kShapeOne ? blocks_of(gx.N) : (blocks_of(gx.N) + 3) / 4);
+    if (x_wgs > 4 * limit || shape_tiles(s, gw.M, gw.N) * plan.splits > 4 * limit) continue;
+    const double t = pair_time(s);
+    if (t < t_best) {
+      t_best = t;
+      shape = s;
+    }
+  }
+  if (shape < 0) return SD_ERR_UNSUPPORTED;
+  const int rc = is_bf16(dtype) ? tile_pair<BF16>(gx, gw, shape, plan.splits, stream)
+                                : tile_pair<F16>(gx, gw, shape, plan.splits, stream);
   if (rc) return rc;
-  note_kernel("pair:sdd+dsd:%s splits=%d", dsd_name(plan.shape), plan.splits);
+  note_kernel("pair:sdd+dsd:%s splits=%d", dsd_name(shape), plan.splits);
   return plan.splits > 1 ? launch_splitk_reduce(gw, plan.splits, true, dtype, stream) : SD_OK;
 }
 

@@ -48,3 +48,22 @@ def test_large_weight_gradients_leave_the_smallest_shape(M, K, N, bs, p, dtype, 
     assert ext.last_kernel() == "specialised" and not detail.startswith("dsd:one"), detail
     assert detail.endswith("splits=1") != cut, detail
     assert max_tile_rel_fro(dw, O.dsd_dw(to_np(dy)[:, :N], to_np(x), mk, bs, p, np.float32)) <= REL_FRO_TOL
+
+
+@pytest.mark.parametrize("M,K,N,p,act", [
+    (6574, 4808, 5704, 0.5, None),    # 592 us on strips of two, 338 on the big shape's edge instance
+    (6656, 6736, 7008, 0.1, "gelu"),  # 1474 and 635
+])
+def test_large_ragged_input_gradients_stay_on_the_big_shape(M, K, N, p, act):
+    ext, x, w, dy, mk, lists, kbs = _layer(M, K, N, 64, p, torch.float16)
+    s = 1 / (1 - p)
+    if act:
+        dx = ext.gemm_sdd_lists_actgrad(dy, w.t(), lists, kbs, s, act, x, keep_hint=1 - p)
+    else:
+        dx = ext.gemm_sdd_lists(dy, w.t(), lists, kbs, s, keep_hint=1 - p)
+    assert ext.last_kernel_detail() == "sdd:big:ragged", ext.last_kernel_detail()
+    ref = O.sdd_dx(to_np(dy), to_np(w), mk, 64, p, np.float32)
+    if act:
+        t = x.double().cpu()
+        ref = ref * (0.5 * (1 + torch.erf(t * 0.5 ** 0.5)) + t * torch.exp(-0.5 * t * t) * 0.3989422804014327).numpy()
+    assert max_tile_rel_fro(dx, ref) <= REL_FRO_TOL
