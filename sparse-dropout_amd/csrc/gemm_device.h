@@ -66,7 +66,8 @@ __device__ inline void buffer16_to_lds(u32x4 buffer, uint32_t lane_off, uint32_t
 }
 
 // Waits until at most n of the wave's loads are outstanding (they return in order: everything issued before the last
-// n has landed).  n is wave-uniform and only known at run time, the instruction takes an immediate.
+// n has landed).  n is wave-uniform and only known at run time, the instruction takes an immediate; above 16 it waits for
+// the older ones down to 16, which is more than asked.
 __device__ inline void wait_loads_all_but(int n) {
   if (n >= 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
   else if (n == 15) asm volatile("s_waitcnt vmcnt(15)" ::: "memory");

@@ -16,7 +16,10 @@
 //    ragged edges cost one OR per load of the last reduction block and need no instance of their own.
 //  * Accumulators are stored from registers: an exchange of 16-lane rows (v_permlane16_swap) gives every lane 8
 //    consecutive elements of C's contiguous index, which is one 16-byte store; no pass through LDS.
-// NST - 1 steps are on their way while one computes; one barrier per step publishes it and frees the stage before.
+// One barrier per step publishes it and frees the stage before.  NST - 1 steps are put on their way while one computes.  How
+// many stay there depends on a loading wave's loads per step, since its wait counts to 16 (wait_loads_all_but): 8 on the
+// 64 x 64 shapes; 16 on the 128 x 128 ones with loading waves, whose barrier so waits for the step after as well and which
+// have two steps in flight, not three; 20 on the strips of four, where it waits for 4 loads of the step after.
 #pragma once
 #include <type_traits>
 

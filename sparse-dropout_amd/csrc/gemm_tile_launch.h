@@ -20,9 +20,9 @@ namespace {
 //         the other's products (16384 x 384 -> 1536 with a GELU in the store: 65 -> 45 us against the 256 x 256 shape)
 // reduction-contiguous operands (forward, dense): one running sum per element
 using FwdOne = TileShape<1, 1, 4, 2, false, 2, 2>;
-// the same with three stages, three workgroups to a CU: more than the 512 that are resident with four (a result up to 64
-// columns wide), where a workgroup's way to its first tile counts:
-// 200704 x 288 -> 64 at p = 0.25 35 -> 30 us, 219520 x 576 -> 64 at p = 0.5 38 -> 33
+// the same with three stages, three workgroups to a CU: more than the 512 that are resident with four, where a workgroup's way
+// to its first tile counts: 200704 x 288 -> 64 at p = 0.25 35 -> 30 us, 219520 x 576 -> 64 at p = 0.5 38 -> 33 (outputs of one
+// column block are what this shape is taken for at such sizes; wider ones go to the larger shapes)
 using FwdOneMany = TileShape<1, 1, 3, 2, false, 2, 2>;
 using FwdQuad = TileShape<2, 2, 4, 2, false, 4, 2>;
 using FwdWide = TileShape<2, 2, 2, 0, false, 2, 4>;
