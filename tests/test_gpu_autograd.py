@@ -322,3 +322,11 @@ def test_draws_do_not_depend_on_the_gradient_mode():
     with torch.no_grad():
         got = F.hip_blockwise_dropout_mlp(x, ws, BS, ps, "relu")
     assert torch.equal(GEMM().rng_state(), after) and torch.equal(got, want)
+
+
+@every_function
+def test_an_output_changed_in_place_counts_in_the_gradients(name):
+    """No backward reads the result, so it may be overwritten; what the change does to the gradient is not lost."""
+    call, wrt, _ = FUNCTIONS[name]()
+    want = _grads(call().relu(), wrt)
+    assert _same(_grads(call().relu_(), wrt), want)
