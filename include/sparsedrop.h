@@ -501,6 +501,55 @@ int sd_conv2d_dw_lists(const void* x, int64_t x_stride_n, int64_t x_stride_c, in
                        const int32_t* col_ptr, const int32_t* row_idx, int64_t block_size, float scale,
                        int dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ---------------------------------------------------------------------------------------------
+ * Stride-1 convolutions tap by tap: the three products of the (block-dropout) convolution on images and gradients laid out as
+ * rows of channels, [positions, channels], without a patch matrix, kept-block lists or a fold (csrc/conv_taps.hip).
+ * The mask is the one over the patch matrix [N*P*Q, C*R*S], one byte per block_size x block_size block (a multiple of 64),
+ * non-zero = dropped, strides in bytes; NULL = everything kept.  No counterpart in the reference.
+ *
+ * sd_conv2d_taps_fits: whether the kernels take the geometry (1) or not (0): strides 1, 2 <= R*S <= 32, channels and outputs
+ * multiples of 8, and the rows that 256 consecutive positions touch within a CU's LDS.  The calls below return
+ * SD_ERR_UNSUPPORTED, with nothing launched, for every other.  sd_conv2d_taps_taken: whether they are also expected to be faster than
+ * the other routes at drop rate p.
+ *
+ * sd_conv2d_taps_prepare: what a direction needs beforehand, each part left out when its pointer is NULL, in one launch:
+ * up to two sets of planes [n][channels][pixels] (strides sn, sc, unit along the pixels) as rows [n * pixels, channels]; the weights
+ * [k_out, c*r*s] packed into sd_conv2d_taps_packed_bytes bytes (16-byte aligned) for the forward or, with `backward`, for the
+ * input gradient; a mask of mask_mb x mask_kb bytes drawn as sd_random_lists draws it (state NULL: from seed and offset).
+ * ------------------------------------------------------------------------------------------- */
+int sd_conv2d_taps_fits(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h,
+                        int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w);
+int sd_conv2d_taps_taken(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h,
+                         int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, double p);
+int64_t sd_conv2d_taps_packed_bytes(int64_t c, int64_t k_out, int64_t r, int64_t s, int backward);
+int sd_conv2d_taps_prepare(int count, const void* const* planes, const int64_t* sn, const int64_t* sc, void* const* rows,
+                           const int64_t* n, const int64_t* channels, const int64_t* pixels, const void* weight, int64_t weight_ld, int64_t c, int64_t k_out, int64_t r, int64_t s, int backward,
+                           void* packed, uint8_t* mask_out, int64_t mask_mb, int64_t mask_kb, uint64_t* state, uint64_t seed,
+                           uint64_t offset, float p, int dtype, void* stream);
+/* Whether sd_conv2d_dsd_lists takes this call (its arguments without lists and scale): 1 or 0, nothing launched. */
+int sd_conv2d_implicit_taken(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_stride_h, int64_t x_stride_w,
+                             const void* weight, int64_t weight_ld, int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out,
+                             int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
+                             int64_t dil_h, int64_t dil_w);
+/* y[N*P*Q, k_out] from x as rows [N*H*W, c] */
+int sd_conv2d_taps_forward(const void* x_rows, int64_t x_ld, const void* packed, void* y, int64_t y_ld, const uint8_t* mask,
+                           int64_t mask_stride_r, int64_t mask_stride_c, int64_t block_size, int64_t n, int64_t c, int64_t h,
+                           int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h,
+                           int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype, void* stream);
+/* dx [N, C, H, W], contiguous planes or pixels by its strides, from dy as rows [N*P*Q, k_out]; packed with backward = 1 */
+int sd_conv2d_taps_dx(const void* dy_rows, int64_t dy_ld, const void* packed, void* dx, int64_t dx_stride_n, int64_t dx_stride_c,
+                      int64_t dx_stride_h, int64_t dx_stride_w, const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c,
+                      int64_t block_size, int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                      int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale,
+                      int dtype, void* stream);
+/* dw[k_out, c*r*s] from both; workspace: sd_conv2d_taps_dw_workspace_bytes(.., rows = N*P*Q) bytes, 16-byte aligned */
+int64_t sd_conv2d_taps_dw_workspace_bytes(int64_t c, int64_t k_out, int64_t r, int64_t s, int64_t rows);
+int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* dy_rows, int64_t dy_ld, void* dw, int64_t dw_ld,
+                      const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c, int64_t block_size, int64_t n, int64_t c,
+                      int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h,
+                      int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -654,11 +654,14 @@ int sd_col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, in
                 dil_w, mask, msr, msc, bs, dtype, (hipStream_t)stream);
 }
 
-int sd_conv2d_dsd_lists(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, const void* weight,
-                        int64_t wld, void* y, int64_t yld, int64_t n, int64_t c, int64_t h, int64_t w,
-                        int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h,
-                        int64_t stride_w, int64_t dil_h, int64_t dil_w, const int32_t* row_ptr,
-                        const int32_t* col_idx, int64_t bs, float scale, int dtype, void* stream) {
+}  // extern "C"
+
+// The implicit-GEMM forward, or (plan_only) whether it would be launched.
+static int conv_forward(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, const void* weight, int64_t wld, void* y,
+                        int64_t yld, int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                        int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
+                        const int32_t* row_ptr, const int32_t* col_idx, int64_t bs, float scale, int dtype, bool plan_only,
+                        void* stream) {
   SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "dtype must be SD_F16 or SD_BF16 (got %d)", dtype);
   SD_REQUIRE(x && weight && y, "null pointer argument");
   SD_REQUIRE((row_ptr == nullptr) == (col_idx == nullptr), "row_ptr and col_idx must both be given or both be null");
@@ -686,9 +689,27 @@ int sd_conv2d_dsd_lists(const void* x, int64_t sn, int64_t sc, int64_t sh, int64
   cg.units = one_run ? 1 : 4;
   GemmArgs g = make_args(nullptr, 0, 0, weight, wld, 1, y, yld, 1, n * P * Q, k_out, c * r * s, bs, scale, row_ptr,
                          col_idx);
-  const int rc = launch_conv_implicit(g, cg, P, stride_h, stride_w, dil_h, dil_w, r, sw, dtype, (hipStream_t)stream);
-  if (rc == SD_OK) last_kernel = "specialised";
+  const int rc = launch_conv_implicit(g, cg, P, stride_h, stride_w, dil_h, dil_w, r, sw, dtype, plan_only, (hipStream_t)stream);
+  if (rc == SD_OK && !plan_only) last_kernel = "specialised";
   return rc;
+}
+
+extern "C" {
+
+int sd_conv2d_dsd_lists(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, const void* weight,
+                        int64_t wld, void* y, int64_t yld, int64_t n, int64_t c, int64_t h, int64_t w,
+                        int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h,
+                        int64_t stride_w, int64_t dil_h, int64_t dil_w, const int32_t* row_ptr,
+                        const int32_t* col_idx, int64_t bs, float scale, int dtype, void* stream) {
+  return conv_forward(x, sn, sc, sh, sw, weight, wld, y, yld, n, c, h, w, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h,
+                      dil_w, row_ptr, col_idx, bs, scale, dtype, false, stream);
+}
+
+int sd_conv2d_implicit_taken(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, const void* weight, int64_t wld,
+                             int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h,
+                             int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w) {
+  return conv_forward(x, sn, sc, sh, sw, weight, wld, const_cast<void*>(x), k_out, n, c, h, w, k_out, r, s, pad_h, pad_w, stride_h,
+                      stride_w, dil_h, dil_w, nullptr, nullptr, 0, 1.f, SD_F16, true, nullptr) == SD_OK;
 }
 
 int sd_conv2d_dx(const void* dy, int64_t dy_ld, const void* weight, int64_t weight_ld, void* dx, int64_t sn,

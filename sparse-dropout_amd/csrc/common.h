@@ -353,7 +353,7 @@ int launch_forward_with_lists(const GemmArgs& g, const MaskSrc& src, int64_t mb,
 // weight matrix, g.c the [N*P*Q, K_out] output, the lists over the patch matrix's block grid.  Returns
 // SD_ERR_UNSUPPORTED (without an error message) for geometries it does not take.
 int launch_conv_implicit(const GemmArgs& g, const ImplicitConv& cg, int64_t P, int64_t stride_h, int64_t stride_w,
-                         int64_t dil_h, int64_t dil_w, int64_t R, int64_t x_sw, int dtype, hipStream_t stream);
+                         int64_t dil_h, int64_t dil_w, int64_t R, int64_t x_sw, int dtype, bool plan_only, hipStream_t stream);
 // weight gradient of the same convolution without the patch matrix: g.M = C*R*S, g.N = K_out, g.K = N*P*Q, g.b =
 // dY^T, g.c column-major, the lists those of the transposed mask; cg.PR = rows one 64-position block touches.
 int launch_conv_implicit_dw(const GemmArgs& g, ImplicitConv cg, int64_t P, int64_t stride_h, int64_t stride_w,

@@ -2062,7 +2062,7 @@ int conv_dw_splits(int64_t M, int64_t N, int64_t K) {
 }
 
 int launch_conv_implicit(const GemmArgs& g, const ImplicitConv& cg, int64_t P, int64_t stride_h, int64_t stride_w,
-                         int64_t dil_h, int64_t dil_w, int64_t R, int64_t x_sw, int dtype, hipStream_t stream) {
+                         int64_t dil_h, int64_t dil_w, int64_t R, int64_t x_sw, int dtype, bool plan_only, hipStream_t stream) {
   if (g.row_ptr != nullptr && g.bs != BS) return SD_ERR_UNSUPPORTED;
   // the four row blocks of a workgroup: consecutive output rows of one image sharing their input rows (units == 1,
   // P * Q a multiple of 256), or each with its own input rows (units == 4, P * Q a multiple of 64)
@@ -2093,6 +2093,7 @@ int launch_conv_implicit(const GemmArgs& g, const ImplicitConv& cg, int64_t P, i
   const int64_t whole = patch_elems * 2 + Kb * BS * 2;
   const bool whole_ok = whole <= CONV_PATCH_MAX && cg.units == 1;
   if (!step_ok && !whole_ok) return SD_ERR_UNSUPPORTED;
+  if (plan_only) return SD_OK;
   const bool use_steps = step_ok && !(whole_ok && tile_policy.load(std::memory_order_relaxed) == kTileBig);
   const bool ragged = g.N % BS != 0 || g.K % BS != 0;
   if (use_steps) {

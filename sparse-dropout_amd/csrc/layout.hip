@@ -1,6 +1,9 @@
 // Operands brought into the layout the GEMM kernels load: rows that start on 16-byte boundaries and end in zeros, and
 // the rows [N*P*Q, K] of an image tensor stored plane by plane.
 #include "common.h"
+#include "conv_taps.h"
+#include "mask_source.h"
+#include "sparsedrop.h"
 
 namespace sd {
 namespace {
@@ -54,12 +57,18 @@ constexpr int kTurnLd = kTurn + 2;      // halfs per LDS row: 33 words, so that 
 // dst[(n * P + i) * C + c] = src[n * sn + c * sc + i], i < P.  Bound by its reads and writes (a 64 MB copy at 128 images
 // of 128 x 32 x 32): both sides move in 128-byte pieces, 16 bytes per lane, and the tile is turned in LDS.  The
 // elementwise copy it replaces reads 2 bytes per lane, a plane apart.
-__global__ __launch_bounds__(256) void rows_from_planes_kernel(const uint16_t* __restrict__ src, int64_t sn, int64_t sc,
-                                                               uint16_t* __restrict__ dst, int C, int P, int tiles_c,
-                                                               int tiles_p) {
-  __shared__ __attribute__((aligned(4))) uint16_t tile[kTurn * kTurnLd];  // [c][i]
+struct TurnJob {
+  const uint16_t* src;
+  int64_t sn, sc;
+  uint16_t* dst;
+  int C, P, tiles_c, tiles_p;
+};
+__device__ inline void turn_tile(const TurnJob& job, uint32_t b, uint16_t* tile) {  // tile: kTurn * kTurnLd halfs, [c][i]
+  const uint16_t* __restrict__ src = job.src;
+  uint16_t* __restrict__ dst = job.dst;
+  const int64_t sn = job.sn, sc = job.sc;
+  const int C = job.C, P = job.P, tiles_c = job.tiles_c, tiles_p = job.tiles_p;
   const int t = threadIdx.x;
-  const uint32_t b = blockIdx.x;
   const int tc = (int)(b % (uint32_t)tiles_c);
   const uint32_t rest = b / (uint32_t)tiles_c;
   const int tp = (int)(rest % (uint32_t)tiles_p);
@@ -111,6 +120,87 @@ __global__ __launch_bounds__(256) void rows_from_planes_kernel(const uint16_t* _
   }
 }
 
+__global__ __launch_bounds__(256) void rows_from_planes_kernel(TurnJob job) {
+  __shared__ __attribute__((aligned(4))) uint16_t tile[kTurn * kTurnLd];
+  turn_tile(job, blockIdx.x, tile);
+}
+
+// What one direction of a tap-wise convolution (conv_taps.hip) needs beforehand, in one launch: the weights tap by tap, the
+// mask, and image or gradient planes as rows, by `packs`, `draws` and `turns` workgroups.
+// The packed weights' order is TapPacking's (conv_taps.h); behind them lies a word per unit: whether one of its weights is an Inf
+// or NaN.  A workgroup packs a unit.
+struct PackJob {
+  const uint16_t* w;  // [K, C * RS]
+  int64_t ld;
+  uint16_t* dst;
+  TapPacking order;
+  int C, K, backward;
+  uint32_t exponent;  // bits of the element type that are all set in an Inf or NaN
+};
+struct PrepareJobs {
+  TurnJob turn[2];
+  int turns[2];
+  PackJob pack;
+  MaskSrc draw;
+  uint8_t* mask_out;
+  int64_t mask_rows;
+  int packs, draws;
+};
+
+__global__ __launch_bounds__(256) void conv_prepare_kernel(PrepareJobs j) {
+  __shared__ __attribute__((aligned(4))) uint16_t tile[kTurn * kTurnLd];
+  int b = (int)blockIdx.x;
+  // (the few workgroups that pack and draw come first: they finish under the turning ones)
+  if (b < j.packs) {
+    const PackJob& p = j.pack;
+    const int64_t unit = b;
+    const uint32_t piece = threadIdx.x;
+    int n, r0, t;
+    p.order.unit(unit, &n, &r0, &t);
+    n += (int)(piece / 32 * 8 + piece % 8);
+    r0 += (int)(piece / 8 % 4) * 8;
+    const int RS = p.order.RS;
+    uint32_t h[8];
+    int bad = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = r0 + i;
+      h[i] = 0u;
+      // forward: outputs are the K rows, the reduction runs over channels; backward: the other way round, taps in reverse
+      if (p.backward) { if (n < p.C && r < p.K) h[i] = p.w[(int64_t)r * p.ld + (int64_t)n * RS + (RS - 1 - t)]; }
+      else if (n < p.K && r < p.C) h[i] = p.w[(int64_t)n * p.ld + (int64_t)r * RS + t];
+      bad |= (h[i] & p.exponent) == p.exponent;
+    }
+    bad = __syncthreads_or(bad);
+    if (piece == 0) reinterpret_cast<uint32_t*>(p.dst + (int64_t)j.packs * 2048)[unit] = bad ? 1u : 0u;
+    reinterpret_cast<u32x4*>(p.dst)[unit * 256 + piece] =
+        u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+    return;
+  }
+  b -= j.packs;
+  if (b < j.draws) {
+    MaskSrc src = j.draw;
+    src.resolve();
+    write_mask(src, j.mask_rows, j.mask_out, (int64_t)b * 256 + threadIdx.x, (int64_t)j.draws * 256);
+    report_in(const_cast<uint64_t*>(j.draw.state), (unsigned)j.draws);
+    return;
+  }
+  b -= j.draws;
+  const bool second = b >= j.turns[0];
+  turn_tile(j.turn[second], (uint32_t)(second ? b - j.turns[0] : b), tile);
+}
+
+// SD_OK and *blocks workgroups for the planes, or an error
+int turn_job(const void* src, int64_t sn, int64_t sc, void* dst, int64_t n, int64_t c, int64_t p, TurnJob* job, int64_t* blocks) {
+  SD_REQUIRE(src && dst, "rows_from_planes: null pointer");
+  SD_REQUIRE(c < (1LL << 31) && p < (1LL << 31) - kTurn && n < (1LL << 31), "rows_from_planes: too large");
+  const int64_t tiles_c = ceil_div(c, kTurn), tiles_p = ceil_div(p, kTurn);
+  SD_REQUIRE(tiles_c * tiles_p < (1LL << 31) && tiles_c * tiles_p * n < (1LL << 31), "rows_from_planes: too large");
+  *job = TurnJob{static_cast<const uint16_t*>(src), sn, sc, static_cast<uint16_t*>(dst), (int)c, (int)p, (int)tiles_c, (int)tiles_p};
+  *blocks = tiles_c * tiles_p * n;
+  return SD_OK;
+}
+
 }  // namespace
 }  // namespace sd
 
@@ -146,12 +236,58 @@ extern "C" int sd_rows_from_planes(const void* src, int64_t sn, int64_t sc, void
                                    void* stream) {
   SD_REQUIRE(n >= 0 && c >= 0 && p >= 0, "rows_from_planes: negative size");
   if (n == 0 || c == 0 || p == 0) return SD_OK;
-  SD_REQUIRE(src && dst, "rows_from_planes: null pointer");
-  SD_REQUIRE(c < (1LL << 31) && p < (1LL << 31) - kTurn && n < (1LL << 31), "rows_from_planes: too large");
-  const int64_t tiles_c = ceil_div(c, kTurn), tiles_p = ceil_div(p, kTurn);
-  SD_REQUIRE(tiles_c * tiles_p < (1LL << 31) && tiles_c * tiles_p * n < (1LL << 31), "rows_from_planes: too large");
-  hipLaunchKernelGGL(rows_from_planes_kernel, dim3((unsigned)(tiles_c * tiles_p * n)), dim3(256), 0, (hipStream_t)stream,
-                     static_cast<const uint16_t*>(src), sn, sc, static_cast<uint16_t*>(dst), (int)c, (int)p, (int)tiles_c,
-                     (int)tiles_p);
+  TurnJob job;
+  int64_t blocks;
+  if (int rc = turn_job(src, sn, sc, dst, n, c, p, &job, &blocks)) return rc;
+  hipLaunchKernelGGL(rows_from_planes_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, job);
   return check_launch("rows_from_planes_kernel");
+}
+
+extern "C" int64_t sd_conv2d_taps_packed_bytes(int64_t c, int64_t k_out, int64_t r, int64_t s, int backward) {
+  if (c < 1 || k_out < 1 || r < 1 || s < 1) return 0;
+  if (c >= (1 << 20) || k_out >= (1 << 20) || r * s >= (1 << 10)) return 0;
+  const TapPacking order((int)(backward ? k_out : c), (int)(backward ? c : k_out), (int)(r * s), backward != 0);
+  return order.weight_bytes() + (order.units() * 4 + 15) / 16 * 16;
+}
+
+extern "C" int sd_conv2d_taps_prepare(int count, const void* const* planes, const int64_t* sn, const int64_t* sc, void* const* rows,
+                                      const int64_t* n, const int64_t* channels, const int64_t* pixels, const void* weight,
+                                      int64_t weight_ld, int64_t c, int64_t k_out, int64_t r, int64_t s, int backward,
+                                      void* packed, uint8_t* mask_out, int64_t mask_mb, int64_t mask_kb, uint64_t* state,
+                                      uint64_t seed, uint64_t offset, float p, int dtype, void* stream) {
+  SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "conv2d_taps_prepare: dtype");
+  SD_REQUIRE(count >= 0 && count <= 2 && (count == 0 || (planes && sn && sc && rows && n && channels && pixels)) && c >= 0 &&
+                 k_out >= 0 && mask_mb >= 0 && mask_kb >= 0, "conv2d_taps_prepare: argument");
+  PrepareJobs j{};
+  int64_t turns = 0;
+  for (int i = 0; i < count; ++i) {
+    SD_REQUIRE(n[i] >= 0 && channels[i] >= 0 && pixels[i] >= 0, "conv2d_taps_prepare: negative size");
+    int64_t blocks = 0;
+    if (n[i] > 0 && channels[i] > 0 && pixels[i] > 0)
+      if (int rc = turn_job(planes[i], sn[i], sc[i], rows[i], n[i], channels[i], pixels[i], &j.turn[i], &blocks)) return rc;
+    j.turns[i] = (int)blocks;
+    turns += blocks;
+  }
+  if (packed) {
+    const int64_t bytes = sd_conv2d_taps_packed_bytes(c, k_out, r, s, backward);
+    SD_REQUIRE(bytes > 0 && weight && weight_ld >= c * r * s && reinterpret_cast<uintptr_t>(packed) % 16 == 0 && bytes / 16 < (1LL << 31),
+               "conv2d_taps_prepare: weights");
+    const TapPacking order((int)(backward ? k_out : c), (int)(backward ? c : k_out), (int)(r * s), backward != 0);
+    j.pack = PackJob{static_cast<const uint16_t*>(weight), weight_ld, static_cast<uint16_t*>(packed), order, (int)c, (int)k_out,
+                     backward ? 1 : 0, dtype == SD_F16 ? 0x7c00u : 0x7f80u};
+    j.packs = (int)order.units();
+  }
+  if (mask_out && mask_mb * mask_kb > 0) {
+    SD_REQUIRE(p >= 0.f && p < 1.f && mask_mb < (1LL << 31) && mask_kb < (1LL << 31), "conv2d_taps_prepare: mask");
+    j.draw = MaskSrc{nullptr, 0, 0, 1, 1, (int32_t)mask_mb, (int32_t)mask_kb, (uint32_t)seed, (uint32_t)(seed >> 32),
+                     (uint32_t)offset, (uint32_t)(offset >> 32), p, state};
+    j.mask_out = mask_out;
+    j.mask_rows = mask_mb;
+    const int64_t blocks = ceil_div(ceil_div(mask_mb * mask_kb, 4), 256);
+    j.draws = (int)(blocks < 4096 ? blocks : 4096);
+  }
+  SD_REQUIRE(turns + j.packs + j.draws < (1LL << 31), "conv2d_taps_prepare: too large");
+  if (turns + j.packs + j.draws == 0) return SD_OK;
+  hipLaunchKernelGGL(conv_prepare_kernel, dim3((unsigned)(turns + j.packs + j.draws)), dim3(256), 0, (hipStream_t)stream, j);
+  return check_launch("conv_prepare_kernel");
 }

@@ -204,6 +204,7 @@ struct Lists {
   int64_t kernel_bs = 0;  // what the list-taking calls are told: 64, or 32 when the lists carry quadrant bits
   int64_t mb = 0, kb = 0;          // mask grid
   int64_t out_mb = 0, out_kb = 0;  // listed grid
+  bool mask_only = false;          // no lists: the buffer holds a drawn mask or nothing
 
   void shape(int64_t rows, int64_t cols, int64_t bs_) {
     bs = bs_;
@@ -217,14 +218,16 @@ struct Lists {
   }
   void allocate(const Tensor& like, const OptTensor& mask) {
     if (mask) given = check_mask(*mask, mb, kb, like);
-    const int64_t ints = out_mb + out_kb + 2 + 2 * out_mb * out_kb + (mask ? 0 : (mb * kb + 3) / 4);
+    const int64_t ints = (mask_only ? 0 : out_mb + out_kb + 2 + 2 * out_mb * out_kb) + (mask ? 0 : (mb * kb + 3) / 4);
     buf = at::empty({ints}, like.options().dtype(at::kInt));
   }
   int32_t* row_ptr() const { return static_cast<int32_t*>(buf.data_ptr()); }
   int32_t* col_ptr() const { return row_ptr() + out_mb + 1; }
   int32_t* col_idx() const { return col_ptr() + out_kb + 1; }
   int32_t* row_idx() const { return col_idx() + out_mb * out_kb; }
-  uint8_t* drawn() const { return given.defined() ? nullptr : reinterpret_cast<uint8_t*>(row_idx() + out_mb * out_kb); }
+  uint8_t* drawn() const {
+    return given.defined() ? nullptr : reinterpret_cast<uint8_t*>(mask_only ? row_ptr() : row_idx() + out_mb * out_kb);
+  }
   MaskArg mask() const {
     if (given.defined()) return MaskArg(given);
     MaskArg m;
@@ -625,7 +628,7 @@ struct ConvGeom {
 #define GEOM_W(g) (g).pad[0], (g).pad[1], (g).stride[0], (g).stride[1], (g).dil[0], (g).dil[1]
 #define STRIDES4(t) (t).stride(0), (t).stride(1), (t).stride(2), (t).stride(3)
 
-void conv_lists(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
+void conv_mask(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
   check_p(p);
   l.shape(g.rows(), g.cols(), bs);
   if (draw.mask)
@@ -633,6 +636,10 @@ void conv_lists(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const 
                       draw.mask->sizes(), " != [", l.mb, ", ", l.kb, "] for a [", g.rows(), ", ", g.cols(),
                       "] matrix in blocks of ", bs);
   l.allocate(x, draw.mask);
+}
+
+void conv_lists(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
+  conv_mask(x, g, bs, p, draw, l);
   const int64_t split = bs / 64;
   c10::DeviceGuard guard(x.device());
   if (draw.mask) {
@@ -737,14 +744,109 @@ Tensor rows_gradient(const Tensor& grad, const ConvGeom& g, const Tensor& like) 
   return d;
 }
 
+// ---- the convolution tap by tap: images and gradients as rows of channels --------------------------------------------------
+bool on_16_bytes(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// What one direction of it needs, in one launch: planes as rows, the packed weights, the mask.
+struct TapsPrepare {
+  int n = 0;
+  const void* planes[2];
+  void* rows[2];
+  int64_t sn[2], sc[2], images[2], channels[2], pixels[2];
+  std::vector<Tensor> keep;
+  // t [N, C, H, W] as rows [N*H*W, C]: its own memory where its pixels lie one behind the other, else a copy
+  Tensor add(const Tensor& t_) {
+    const Tensor own = on_16_bytes(t_) ? pixel_rows(t_) : Tensor();
+    if (own.defined()) return own;
+    Tensor t = t_;
+    const int64_t h = t.size(2), w = t.size(3);
+    const bool planar = (w == 1 || t.stride(3) == 1) && (h == 1 || t.stride(2) == w) && t.stride(1) >= h * w && t.stride(0) >= 1;
+    if (!planar) t = t.contiguous();
+    keep.push_back(t);
+    Tensor out = new_matrix(t, t.size(0) * h * w, t.size(1));
+    planes[n] = t.data_ptr();
+    rows[n] = out.data_ptr();
+    sn[n] = t.stride(0);
+    sc[n] = t.stride(1);
+    images[n] = t.size(0);
+    channels[n] = t.size(1);
+    pixels[n] = h * w;
+    ++n;
+    return out;
+  }
+  // w: the kernel as [K, C*R*S], undefined for none; draw: a mask for `lists`, or none
+  Tensor launch(const Tensor& like, const Tensor& w, const ConvGeom& g, bool backward, double p, const Draw* draw, const Lists* lists) {
+    Tensor packed;
+    if (w.defined())
+      packed = at::empty({sd_conv2d_taps_packed_bytes(g.c, g.k, g.r, g.s, backward) / 2}, like.options());
+    const bool drawn = draw && !draw->mask;
+    c10::DeviceGuard guard(like.device());
+    check(sd_conv2d_taps_prepare(n, planes, sn, sc, rows, images, channels, pixels, w.defined() ? w.data_ptr() : nullptr, g.cols(),
+                                 g.c, g.k, g.r, g.s, backward, packed.defined() ? packed.data_ptr() : nullptr,
+                                 drawn ? lists->drawn() : nullptr, drawn ? lists->mb : 0, drawn ? lists->kb : 0,
+                                 drawn ? draw->state_ptr() : nullptr, drawn ? draw->seed.value_or(0) : 0, 0, (float)p,
+                                 dtype_of(like), stream_of(like)),
+          "sd_conv2d_taps_prepare");
+    return packed;
+  }
+};
+#define MASK_OF(m, l) (m).ptr, (m).sr, (m).sc, (l) ? (l)->bs : 0
+
+Tensor taps_forward(const Tensor& rows, const Tensor& packed, const ConvGeom& g, const Lists* l, float scale) {
+  Tensor y2 = new_matrix(rows, g.rows(), g.k);
+  const MaskArg m = l ? l->mask() : MaskArg();
+  c10::DeviceGuard guard(rows.device());
+  check(sd_conv2d_taps_forward(rows.data_ptr(), rows.stride(0), packed.data_ptr(), y2.data_ptr(), g.k, MASK_OF(m, l), GEOM_X(g), g.k,
+                               g.r, g.s, GEOM_W(g), scale, dtype_of(rows), stream_of(rows)),
+        "sd_conv2d_taps_forward");
+  return y2;
+}
+
 struct ConvBackward : Node {
   // the kernel as [K, C*R*S], and what the kernel's gradient reads: the patch matrix when the forward made one in memory, else
   // the image (an implicit forward, or a pointwise kernel whose patch matrix is the image's own pixels)
+  // (tap by tap: the image's rows when the forward made a copy of them that nothing else refers to, else the image)
   Saved w2, x, cols;
   SavedLists saved;  // nothing kept: no dropout
   ConvGeom g{};
   double p = 0;
-  bool fused_dx = true, channels_last = false, pixels = false;
+  bool fused_dx = true, channels_last = false, pixels = false, taps = false;
+  // tap by tap: `w` the kernel as a matrix, `image` or `kept_rows` whichever was kept
+  variable_list apply_taps(const Tensor& grad, const Tensor& w, const Tensor& image, Tensor rows, const Lists* l) {
+    variable_list out(2);
+    const bool need_dx = task_should_compute_output(0), need_dw = task_should_compute_output(1);
+    const float scale = (float)(1.0 / (1.0 - p));
+    TapsPrepare prepare;
+    Tensor d = grad.defined() ? grad : at::zeros({g.n, g.k, g.po, g.qo}, w.options());
+    if (d.scalar_type() != w.scalar_type()) d = d.to(w.scalar_type());
+    const Tensor dy2 = prepare.add(d);
+    if (rows.defined()) {
+      if (rows.stride(1) != 1 || rows.stride(0) != g.c || !on_16_bytes(rows)) rows = rows.clone(at::MemoryFormat::Contiguous);
+    } else if (need_dw) {
+      rows = prepare.add(image);
+    }
+    const Tensor packed = prepare.launch(d, need_dx ? w : Tensor(), g, true, 0.0, nullptr, nullptr);
+    const MaskArg m = l ? l->mask() : MaskArg();
+    c10::DeviceGuard guard(d.device());
+    if (need_dx) {
+      Tensor dx = new_image(dy2, g, channels_last);
+      check(sd_conv2d_taps_dx(dy2.data_ptr(), dy2.stride(0), packed.data_ptr(), dx.data_ptr(), STRIDES4(dx), MASK_OF(m, l), GEOM_X(g),
+                              g.k, g.r, g.s, GEOM_W(g), scale, dtype_of(d), stream_of(d)),
+            "sd_conv2d_taps_dx");
+      last_routes[1] = kFused;
+      out[0] = dx;
+    }
+    if (need_dw) {
+      Tensor dw = new_matrix(dy2, g.k, g.cols());
+      Scratch ws(d, sd_conv2d_taps_dw_workspace_bytes(g.c, g.k, g.r, g.s, g.rows()));
+      check(sd_conv2d_taps_dw(rows.data_ptr(), rows.stride(0), dy2.data_ptr(), dy2.stride(0), dw.data_ptr(), dw.stride(0),
+                              MASK_OF(m, l), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), scale, dtype_of(d), ws.ptr, ws.bytes, stream_of(d)),
+            "sd_conv2d_taps_dw");
+      last_routes[2] = kImplicit;
+      out[1] = dw.view({g.k, g.c, g.r, g.s});
+    }
+    return out;
+  }
   variable_list apply(variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
@@ -752,6 +854,7 @@ struct ConvBackward : Node {
     const Tensor w = w2.get().contiguous(), image = x.get();
     const Lists lists = saved.get();
     Tensor patches = cols.matrix();
+    if (taps) return apply_taps(grads[0], w, image, patches, lists.buf.defined() ? &lists : nullptr);
     const Tensor dy2 = grads[0].defined() ? rows_gradient(grads[0], g, w) : at::zeros({g.rows(), g.k}, w.options());
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
@@ -858,7 +961,26 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   Lists lists;
   Tensor y, y2, cols;
   const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;
-  {
+  const bool taps = implicit_forward && fused_dx && sd_conv2d_taps_taken(GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), bs ? p : 0.0);
+  const bool record = records(std::array<Tensor, 2>{x, kernel});
+  if (taps) {
+    NoRecord guard;
+    lists.mask_only = true;
+    const Draw draw{mask, seed, state};
+    if (bs) conv_mask(x, g, bs, p, draw, lists);
+    const Lists* l = bs ? &lists : nullptr;
+    TapsPrepare prepare;
+    Tensor rows = prepare.add(x);
+    const Tensor packed = prepare.launch(x, kernel, g, false, p, l ? &draw : nullptr, l);
+    y2 = taps_forward(rows, packed, g, l, scale);
+    last_routes[0] = kImplicit;
+    last_routes[1] = last_routes[2] = kNone;
+    // What is kept for the kernel's gradient, the image or its rows, follows what the other routes keep, the image or its
+    // patch matrix: a write to the image before the backward is refused or allowed in the same geometries.
+    const bool keeps_image = sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
+    if (record && !keeps_image) cols = rows.is_alias_of(x) ? rows.clone() : rows;
+    y = y2.view({g.n, g.po, g.qo, g.k}).permute({0, 3, 1, 2});
+  } else {
     NoRecord guard;
     if (bs) conv_lists(x, g, bs, p, Draw{mask, seed, state}, lists);
     const Lists* l = bs ? &lists : nullptr;
@@ -893,8 +1015,9 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     // the result is an (N, K, P, Q) view of an (N, P*Q, K) buffer, as the reference's is (im2col_conv2d.py:26-27)
     y = y2.view({g.n, g.po, g.qo, g.k}).permute({0, 3, 1, 2});
   }
-  if (records(std::array<Tensor, 2>{x, kernel})) {
+  if (record) {
     auto node = make_node<ConvBackward>({x, kernel});
+    node->taps = taps;
     node->pixels = cols.defined() && cols.is_alias_of(x);
     if (cols.defined() && !node->pixels) node->cols.keep(cols);
     else node->x.keep(x);

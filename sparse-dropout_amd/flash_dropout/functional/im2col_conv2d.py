@@ -23,10 +23,11 @@ from .blockwise_dropout_matmul_hip import draw_source
 from .tracing import traceable
 
 
-# Use the implicit-GEMM forward (sd_conv2d_dsd_lists) where the library takes the geometry.  Module-level
+# Use the implicit forward (sd_conv2d_taps_forward or sd_conv2d_dsd_lists) where the library takes the geometry.  Module-level
 # switch so that tests and benchmarks can compare both routes.
 IMPLICIT_FORWARD = True
-# Use the one-launch input gradient (sd_conv2d_dx) where the library takes the geometry.
+# Use the one-launch input gradient (sd_conv2d_taps_dx or sd_conv2d_dx) where the library takes the geometry.  (Products run tap
+# by tap when both switches are on.)
 FUSED_INPUT_GRADIENT = True
 
 _ROUTES = (None, "implicit", "fused", "explicit")
@@ -34,7 +35,7 @@ _ROUTES = (None, "implicit", "fused", "explicit")
 
 def conv_last_routes() -> dict:
     """{"forward": ..., "dx": ..., "dw": ...} of the process's last convolution run through this module: "implicit" /
-    "fused" (no patch matrix in memory: sd_conv2d_dsd_lists, sd_conv2d_dw_lists, sd_conv2d_dx) or "explicit" (im2col /
+    "fused" (no patch matrix in memory: sd_conv2d_taps_*, or sd_conv2d_dsd_lists, sd_conv2d_dw_lists, sd_conv2d_dx) or "explicit" (im2col /
     col2im around the GEMMs, taken when the library does not take the geometry or a switch above is off); None for a
     product that was not computed.  Nothing falls back to the patch matrix unseen."""
     return {k: _ROUTES[v] for k, v in zip(("forward", "dx", "dw"), _loader.bridge().conv_routes())}

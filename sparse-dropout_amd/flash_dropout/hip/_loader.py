@@ -88,6 +88,20 @@ SIGNATURES = {
                                    c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
                                    c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
                                    c_void_p, c_void_p, c_int64, c_float, c_int, c_void_p, c_int64, c_void_p]),
+    "sd_conv2d_taps_fits": (c_int, [c_int64] * 13),
+    "sd_conv2d_taps_taken": (c_int, [*([c_int64] * 13), c_double]),
+    "sd_conv2d_taps_packed_bytes": (c_int64, [*([c_int64] * 4), c_int]),
+    "sd_conv2d_implicit_taken": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, *([c_int64] * 14)]),
+    "sd_conv2d_taps_prepare": (c_int, [c_int, *([c_void_p] * 7), c_void_p, *([c_int64] * 5),
+                                       c_int, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_uint64, c_uint64, c_float,
+                                       c_int, c_void_p]),
+    "sd_conv2d_taps_forward": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64,
+                                       *([c_int64] * 13), c_float, c_int, c_void_p]),
+    "sd_conv2d_taps_dx": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, *([c_int64] * 4), c_void_p, c_int64, c_int64, c_int64,
+                                  *([c_int64] * 13), c_float, c_int, c_void_p]),
+    "sd_conv2d_taps_dw_workspace_bytes": (c_int64, [c_int64] * 5),
+    "sd_conv2d_taps_dw": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64,
+                                  *([c_int64] * 13), c_float, c_int, c_void_p, c_int64, c_void_p]),
     "sd_im2col": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64,
                           *([c_int64] * 12), c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "sd_col2im": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,

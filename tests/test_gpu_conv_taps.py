@@ -1,0 +1,166 @@
+"""The tap-wise convolution (csrc/conv_taps.hip): all three products against the oracle at the sizes where its windows, tiles
+and masks end."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from _util import REL_FRO_TOL, cpu_mask, max_tile_rel_fro, to_np
+from oracle import sparsedrop_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# n, c, h, w, k, r, s, padding, dilation: images that end inside a 16-position tile, windows over several images and over the
+# first and last row, a channel tile more or less than a step, tap groups of nine with a rest, results larger and
+# smaller than the image
+GEOMS = [
+    (5, 32, 7, 7, 40, 3, 3, (1, 1), (1, 1)),
+    (3, 40, 14, 14, 136, 3, 3, (1, 1), (1, 1)),
+    (2, 72, 28, 28, 32, 3, 3, (1, 1), (1, 1)),
+    (2, 136, 16, 16, 200, 3, 3, (1, 1), (1, 1)),
+    (2, 64, 30, 30, 64, 5, 5, (2, 2), (1, 1)),
+    (3, 8, 9, 64, 72, 3, 3, (1, 1), (1, 1)),
+    (4, 48, 12, 10, 8, 3, 2, (0, 1), (1, 2)),
+    (4, 32, 6, 9, 64, 3, 3, (3, 4), (1, 1)),
+    (2, 24, 20, 18, 96, 3, 3, (2, 2), (2, 2)),
+    (9, 64, 3, 3, 64, 3, 3, (1, 1), (1, 1)),
+    (2, 32, 1, 40, 64, 1, 7, (0, 3), (1, 1)),
+    (1, 16, 3, 3, 16, 2, 2, (0, 0), (1, 1)),  # four output positions
+]
+
+
+def _tensors(geom, dtype, seed=0):
+    n, c, h, w, k, r, s, pad, dil = geom
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.randn(n, c, h, w, generator=gen).to(dtype)
+    wt = (torch.randn(k, c, r, s, generator=gen) * (c * r * s) ** -0.5).to(dtype)
+    po, qo = O.conv_out_hw(h, w, r, s, padding=pad, stride=(1, 1), dilation=dil)
+    return x, wt, torch.randn(n, k, po, qo, generator=gen).to(dtype), n * po * qo, gen
+
+
+def _products(geom, x, wt, dy, mask, bs, scale, channels_last=False):
+    """y, dx, dw through the library's entry points, whatever route a layer of this size would take."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    lib, call = ext.lib, ext._call
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy = x.cuda(), wt.cuda(), dy.cuda()
+    dt = 1 if x.dtype == torch.bfloat16 else 0
+    geo = (n, c, h, w, k, r, s, *pad, 1, 1, *dil)
+    assert lib.sd_conv2d_taps_fits(*geo) == 1
+    pixels = dy.shape[2] * dy.shape[3]
+    rows = n * pixels
+    new = lambda *shape: torch.empty(*shape, dtype=x.dtype, device="cuda")
+    array = lambda t, *v: (t * len(v))(*v)
+    xr, dyr, y, dw = new(n * h * w, c), new(rows, k), new(rows, k), new(k, c * r * s)
+    packed = [new(lib.sd_conv2d_taps_packed_bytes(c, k, r, s, b) // 2) for b in (0, 1)]
+    st = ext._stream(x)
+    for b, (src, dst, ch, px) in enumerate(((x, xr, c, h * w), (dy, dyr, k, pixels))):
+        call(lib.sd_conv2d_taps_prepare, 1, array(C.c_void_p, src.data_ptr()), array(C.c_int64, src.stride(0)), array(C.c_int64, src.stride(1)),
+             array(C.c_void_p, dst.data_ptr()), array(C.c_int64, n), array(C.c_int64, ch), array(C.c_int64, px), wt.data_ptr(), c * r * s,
+             c, k, r, s, b, packed[b].data_ptr(), None, 0, 0, None, 0, 0, 0.0, dt, st)
+    m = mask.cuda() if mask is not None else None
+    ms = (m.data_ptr(), m.stride(0), m.stride(1), bs) if mask is not None else (None, 0, 0, 0)
+    call(lib.sd_conv2d_taps_forward, xr.data_ptr(), c, packed[0].data_ptr(), y.data_ptr(), k, *ms, *geo, scale, dt, st)
+    dx = torch.full((n, c, h, w), 77.0, dtype=x.dtype, device="cuda")
+    if channels_last:
+        dx = dx.contiguous(memory_format=torch.channels_last)
+    call(lib.sd_conv2d_taps_dx, dyr.data_ptr(), k, packed[1].data_ptr(), dx.data_ptr(), *dx.stride(), *ms, *geo, scale, dt, st)
+    ws = torch.empty(lib.sd_conv2d_taps_dw_workspace_bytes(c, k, r, s, rows), dtype=torch.uint8, device="cuda")
+    call(lib.sd_conv2d_taps_dw, xr.data_ptr(), c, dyr.data_ptr(), k, dw.data_ptr(), c * r * s, *ms, *geo, scale, dt, ws.data_ptr(),
+         ws.numel(), st)
+    return y.view(n, dy.shape[2], dy.shape[3], k).permute(0, 3, 1, 2), dx, dw.view(k, c, r, s)
+
+
+@pytest.mark.parametrize("geom", GEOMS)
+@pytest.mark.parametrize("bs,p", [(64, 0.5), (128, 0.3), (0, 0.0)])
+@pytest.mark.parametrize("channels_last", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_products_tap_by_tap(geom, bs, p, channels_last, dtype):
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, dtype)
+    mask = cpu_mask(O.mask_shape(rows, c * r * s, bs or 64), p, gen)
+    args = (geom, x, wt, dy, mask if bs else None, bs, 1 / (1 - p), channels_last)
+    got = _products(*args)
+    geo = dict(padding=pad, stride=(1, 1), dilation=dil)
+    want = O.conv2d_blockdrop(to_np(x), to_np(wt), mask.numpy(), bs or 64, p, dy=to_np(dy), dtype=np.float64, **geo)
+    for g, ref in zip(got, want):
+        assert max_tile_rel_fro(g, ref) <= REL_FRO_TOL
+    # the same bits once more: every sum has one owner and one order
+    assert all(torch.equal(a, b) for a, b in zip(got, _products(*args)))
+
+
+# (geometry, channels-last image, whether the image is what is kept): rows that fill blocks of 64 and rows that do not
+LAYERS = [((20, 24, 16, 16, 40, 3, 3, (1, 1), (1, 1)), False, True), ((20, 32, 16, 16, 40, 3, 3, (1, 1), (1, 1)), True, False),
+          ((7, 16, 28, 28, 40, 3, 3, (1, 1), (1, 1)), False, False), ((7, 16, 28, 28, 40, 5, 5, (2, 2), (1, 1)), True, False)]
+
+
+@pytest.mark.parametrize("geom,channels_last,keeps_image", LAYERS)
+@pytest.mark.parametrize("drawn", [False, True])
+def test_layers_tap_by_tap(geom, channels_last, keeps_image, drawn):
+    """The autograd function on this route: results, what is kept, and which changes before the backward are refused."""
+    import flash_dropout.functional as F
+    from flash_dropout.hip import GEMM
+
+    n, c, h, w, k, r, s, pad, dil = geom
+    assert GEMM().lib.sd_conv2d_taps_taken(n, c, h, w, k, r, s, *pad, 1, 1, *dil, 0.4) == 1
+    x, wt, dy, rows, gen = _tensors(geom, torch.float16)
+    shape = O.mask_shape(rows, c * r * s, 64)
+    mask = torch.from_numpy(O.random_mask(shape, 0.4, 5)) if drawn else cpu_mask(shape, 0.4, gen)
+    xg = x.cuda()
+    if channels_last:
+        xg = xg.contiguous(memory_format=torch.channels_last)
+    xg.requires_grad_()
+    wg = wt.cuda().requires_grad_()
+    call = lambda: (F.blockwise_dropout_conv2d(xg, wg, 64, 0.4, pad, seed=5) if drawn else
+                    F.blockwise_dropout_conv2d_mask(xg, mask.cuda(), 64, 0.4, wg, pad))
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+        call()
+    big = [q for q in kept if len(q) == 4 or q[0] >= 4096]
+    assert big == [tuple(x.shape) if keeps_image else (n * h * w, c)]
+    y = call()
+    grads = torch.autograd.grad(y, (xg, wg), dy.cuda(), retain_graph=True)
+    assert F.conv_last_routes() == {"forward": "implicit", "dx": "fused", "dw": "implicit"}
+    assert grads[0].stride() == xg.stride()
+    want = O.conv2d_blockdrop(to_np(x), to_np(wt), mask.numpy(), 64, 0.4, dy=to_np(dy), dtype=np.float64, padding=pad, stride=(1, 1),
+                              dilation=dil)
+    for g, ref in zip((y.detach(), *grads), want):
+        assert max_tile_rel_fro(g, ref) <= REL_FRO_TOL
+    with torch.no_grad():
+        xg.mul_(2)
+    if keeps_image:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(y, (xg, wg), dy.cuda())
+    else:
+        again = torch.autograd.grad(y, (xg, wg), dy.cuda())
+        assert all(torch.equal(a, b) for a, b in zip(again, grads))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_what_a_mask_drops_reaches_nothing_tap_by_tap(bad):
+    """An Inf or NaN in an operand reaches the results whose kept blocks read it, and no other."""
+    geom = (3, 32, 14, 14, 64, 3, 3, (1, 1), (1, 1))
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, torch.float16)
+    mask = cpu_mask(O.mask_shape(rows, c * r * s, 64), 0.5, gen)
+    keep = ~mask.repeat_interleave(64, 0).repeat_interleave(64, 1)[:rows, : c * r * s]
+    for which in range(3):
+        ops = [t.clone() for t in (x, wt, dy)]
+        ops[which].view(-1)[ops[which].numel() // 3] = bad
+        y, dx, dw = _products(geom, *ops, mask, 64, 2.0)
+        # counted over kept elements only: where a bad value is not among a sum's terms, the sum is finite
+        cols = torch.nn.functional.unfold(ops[0].double(), (r, s), padding=pad).permute(0, 2, 1).reshape(rows, -1)
+        wm, dm = ops[1].double().reshape(k, -1), ops[2].double().permute(0, 2, 3, 1).reshape(rows, k)
+        b_cols, b_w, b_dy = (~torch.isfinite(t) for t in (cols, wm, dm))
+        kf = keep.double()
+        bad_y = ((b_cols & keep).double() @ torch.ones(c * r * s, k, dtype=torch.double) + kf @ b_w.double().T) > 0
+        bad_cols = keep & ((b_dy.double() @ torch.ones(k, c * r * s, dtype=torch.double) +
+                            torch.ones(rows, k, dtype=torch.double) @ b_w.double()) > 0)
+        bad_dx = torch.nn.functional.fold(bad_cols.double().reshape(n, h * w, -1).permute(0, 2, 1), (h, w), (r, s), padding=pad) > 0
+        bad_dw = (b_dy.double().T @ kf + torch.ones(k, rows, dtype=torch.double) @ (b_cols & keep).double()) > 0
+        assert torch.equal(~torch.isfinite(y.permute(0, 2, 3, 1).reshape(rows, k).cpu()), bad_y), which
+        assert torch.equal(~torch.isfinite(dx.cpu()), bad_dx), which
+        assert torch.equal(~torch.isfinite(dw.cpu().reshape(k, -1)), bad_dw), which
