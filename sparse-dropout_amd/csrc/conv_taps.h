@@ -11,16 +11,21 @@
 
 namespace sd {
 
+SD_BOTH int clamp_int(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+
 // Result position (img, oh, ow) reads source pixel (img, oh - pad_h + r * dl_h, ow - pad_w + s * dl_w) at tap
 // t = r * S + s.  Positions and pixels are counted through all images; in these counts a tap is a constant shift.
 struct TapGeom {
   int IH, IW, OH, OW;  // source and result image
   int R, S, pad_h, pad_w, dl_h, dl_w;
   uint32_t m_image, m_row;  // 2^32 / (OH * OW) and 2^32 / OW, rounded up: prepare() sets them
+  uint32_t row_starts;       // bits r * S: prepare() sets them
   SD_BOTH void prepare() {
     const uint64_t image = (uint64_t)OH * (uint64_t)OW, row = (uint64_t)OW;
     m_image = image > 1 ? (uint32_t)(((1ull << 32) + image - 1) / image) : 0xffffffffu;
     m_row = row > 1 ? (uint32_t)(((1ull << 32) + row - 1) / row) : 0xffffffffu;
+    row_starts = 0;
+    for (int r = 0; r < R && r * S < 32; ++r) row_starts |= 1u << (r * S);
   }
   SD_BOTH int taps() const { return R * S; }
   SD_BOTH int shift(int t) const { return (t / S) * dl_h * IW + (t % S) * dl_w; }
@@ -46,16 +51,30 @@ struct TapPosition {
   }
   // the pixel of tap 0, inside the image or not
   SD_BOTH int pixel(const TapGeom& g) const { return (img * g.IH + oh - g.pad_h) * g.IW + ow - g.pad_w; }
+  // the position `step` positions on (0 < step, at most a row: no division)
+  SD_BOTH void advance(const TapGeom& g, int step) {
+    ow += step;
+    if (ow < g.OW) return;
+    ow -= g.OW;
+    if (++oh < g.OH) return;
+    oh = 0;
+    ++img;
+  }
   // bit t: tap t lies inside the image (R * S <= 32)
   SD_BOTH uint32_t inside(const TapGeom& g) const {
+    if (g.dl_h == 1 && g.dl_w == 1) {  // ranges of rows and columns: a third of the instructions of the loops below
+      const int r0 = clamp_int(g.pad_h - oh, 0, g.R), r1 = clamp_int(g.IH + g.pad_h - oh, 0, g.R);
+      const int s0 = clamp_int(g.pad_w - ow, 0, g.S), s1 = clamp_int(g.IW + g.pad_w - ow, 0, g.S);
+      if (r1 <= r0 || s1 <= s0) return 0u;
+      const uint32_t cols = (~0u >> (32 - (s1 - s0))) << s0;
+      return (g.row_starts & ((~0u >> (32 - (r1 - r0) * g.S)) << (r0 * g.S))) * cols;
+    }
     uint32_t cols = 0, bits = 0;
     for (int s = 0, w = ow - g.pad_w; s < g.S; ++s, w += g.dl_w) cols |= ((unsigned)w < (unsigned)g.IW ? 1u : 0u) << s;
     for (int r = 0, h = oh - g.pad_h, t = 0; r < g.R; ++r, h += g.dl_h, t += g.S) bits |= ((unsigned)h < (unsigned)g.IH ? cols : 0u) << t;
     return bits;
   }
 };
-
-SD_BOTH int clamp_int(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
 // Source pixels [lo, hi) hold everything inside the images that positions first .. last read.
 struct TapWindow {

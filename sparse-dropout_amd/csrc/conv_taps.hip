@@ -14,10 +14,10 @@
 //    block is kept (sums stay in fp32; the two-kernel route rounds every tap's term to the element type).
 // The products cost the dense number of operations and little else: the rows are read once, there is no matrix R*S times
 // the image to write and read back, and no per-element fold.  A step (forward and gradients, kernel times in us):
-//   128 x 64 x 32 x 32 -> 128, 3 x 3, fp16, p = 0.5: rows, weights and mask 25, y 29, dx 37, dw 43 + 5; before: lists 13, y 43
-//   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7.  192 -> 129 a pass.
-//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 28, 29 + 7; before: lists 13, patch matrix 45, y 30, rows of dy 13,
-//   patch gradient 40, fold 52, dw 28 + 6.  227 -> 105.
+//   128 x 64 x 32 x 32 -> 128, 3 x 3, fp16, p = 0.5: rows, weights and mask 25, y 28, dx 37, dw 41 + 5; before: lists 13, y 43
+//   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7.  192 -> 128 a pass.
+//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 28 + 7; before: lists 13, patch matrix 45, y 30, rows of dy 13,
+//   patch gradient 40, fold 52, dw 28 + 6.  227 -> 103.
 #include <atomic>
 
 #include "common.h"
@@ -59,8 +59,14 @@ struct TapArgs {
   float scale;
 };
 
-__device__ inline bool block_kept(const TapArgs& g, int rb, int cb) {
-  return g.mask == nullptr || g.mask[(int64_t)(rb / g.split) * g.msr + (int64_t)(cb / g.split) * g.msc] == 0;
+template <typename A>
+__device__ inline bool block_kept(const A& g, int rb, int cb) {
+  if (g.mask == nullptr) return true;
+  if (g.split != 1) {
+    rb /= g.split;
+    cb /= g.split;
+  }
+  return g.mask[(int64_t)rb * g.msr + (int64_t)cb * g.msc] == 0;
 }
 
 // All ones where bit `at` of `bits` is set, else zero.  (The empty statement keeps the compiler from turning what is done
@@ -83,7 +89,7 @@ __device__ inline float pick(int m, float b, float a) {
 // weights are on their way two steps ahead, and what a wave issues besides (a tap's addresses once per tap, weights in the order
 // of the steps) is kept few: a wave issues an instruction every four or five clocks at best, and the input gradient's picks alone
 // are 128 of the 250 of a step of 32 products.  One workgroup alone, 128 x 64 channels, 18 steps: 17 us (y), 22 (dx); 512 of them,
-// two to a CU: 29 and 37, where the matrix cores are busy a third of the time.
+// two to a CU: 28 and 37, where the matrix cores are busy a third of the time.
 template <typename T, bool DX, int NT, int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_taps_kernel(TapArgs g) {
   constexpr bool WIDE = NT == 8;
@@ -113,19 +119,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     w_dst += (uint32_t)kWeightStage;
     if (w_dst >= w_end) w_dst -= (uint32_t)(kStages * kWeightStage);
   };
-  auto load_rows = [&](int chunk) {
-    const int c = chunk * 64 + lane / 8 * 8;
-    const u32x4 src = buffer_of(reinterpret_cast<const char*>(g.in + (int64_t)lo * g.in_ld + chunk * 64));
-    const uint32_t lane_off = (uint32_t)(((int64_t)(lane % 8) * g.in_ld + lane / 8 * 8) * 2);
-    for (int r = wave * 8; r < nrows; r += 32)
-      buffer16_to_lds(src, c < g.red && r + lane % 8 < nrows ? lane_off + (uint32_t)((int64_t)r * g.in_ld * 2) : kNoData,
-                      smem_a + (uint32_t)(kStages * kWeightStage + r * kRowBytes));
+  auto load_rows = [&](int chunk) {  // what lies past the last row or channel arrives as zeros
+    const int left = g.red - chunk * 64 < 64 ? g.red - chunk * 64 : 64;
+    u32x4 src = buffer_of(reinterpret_cast<const char*>(g.in + (int64_t)lo * g.in_ld + chunk * 64));
+    src.z = nrows > 0 ? uniform((uint32_t)(((nrows - 1) * (int)g.in_ld + left) * 2)) : 0u;
+    uint32_t from = lane / 8 * 8 < left ? (uint32_t)((lane % 8 * (int)g.in_ld + lane / 8 * 8) * 2) : kNoData;
+    const uint32_t row = (uint32_t)g.in_ld * 2u;
+    from += (uint32_t)(wave * 8) * row;
+    uint32_t dst = smem_a + (uint32_t)(kStages * kWeightStage + wave * 8 * kRowBytes);
+    for (int r = wave * 8; r < nrows; r += 32, from += 32u * row, dst += 32 * kRowBytes) buffer16_to_lds(src, from, dst);
   };
   // what the masks of a chunk need, in flight together with its rows (forward)
   auto chunk_kept = [&](int chunk) {
     const int rb = m0 / 64 + wave, cb = chunk * RS + lane;
     return lane < RS && rb * 64 < g.rows && cb < (g.red * RS + 63) / 64 && block_kept(g, rb, cb);
   };
+  // The two workgroups of a CU would stand at their reads, and then at the matrix cores, together: one goes first.  (In one
+  // round, workgroups 256 apart share a CU.  Input gradients of 256 x 32 x 28 x 28 from 64: 25.7 -> 24.2 us, of 128 x 128 x
+  // 28 x 28 from 128: 56 -> 53.)
+  if (DX && ((blockIdx.x >> 8) & 1)) __builtin_amdgcn_s_setprio(2);
   load_rows(0);
   load_next();
   load_next();
@@ -136,15 +148,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   int pix[4];      // DX: the position read at tap 0, counted from the first block of 64 the window touches
   uint32_t in[4];  // taps inside the image
   const int rb0 = lo / 64;
+  {
+    TapPosition p(g.geo, (uint32_t)(m0 + wave * 64 + l16));
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int pos = m0 + wave * 64 + mt * 16 + l16;
-    in[mt] = 0;
-    at[mt] = pix[mt] = 0;
-    if (pos < g.rows) {
-      const TapPosition p(g.geo, (uint32_t)pos);
-      in[mt] = p.inside(g.geo);
+    for (int mt = 0; mt < 4; ++mt) {
+      const int pos = m0 + wave * 64 + mt * 16 + l16;
+      if (mt) {
+        if (g.geo.OW >= 16) p.advance(g.geo, 16);
+        else p = TapPosition(g.geo, (uint32_t)pos);
+      }
       const int px = p.pixel(g.geo);
+      in[mt] = pos < g.rows ? p.inside(g.geo) : 0u;
       at[mt] = (px - lo) * 16;
       pix[mt] = px - rb0 * 64;
     }
@@ -385,9 +399,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   if (!DX || !g.planes) {
     if (NT == 1) return;
     const int c_at = (grp % 2) * 16 + (grp / 2) * 8;  // of a pair of tiles: 8 consecutive channels after the exchange
+    uint16_t* o = g.out + (int64_t)pos0 * g.out_ld + n0 + (l16 * (int)g.out_ld + c_at);
+    const bool whole = pos0 + 64 <= g.rows && n0 + 16 * NT <= g.n_out;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      const int pos = pos0 + mt * 16 + l16;
 #pragma unroll
       for (int nt = 0; nt < NT; nt += 2) {
         float r[8];
@@ -397,11 +412,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
           r[4 + i] = acc[mt][nt + 1][i] * g.scale;
           swap_rows16(r[i], r[4 + i]);
         }
-        const int n = n0 + nt * 16 + c_at;
-        if (pos < g.rows && n < g.n_out)
-          *reinterpret_cast<u32x4_any*>(g.out + (int64_t)pos * g.out_ld + n) =
+        if (whole || (pos0 + mt * 16 + l16 < g.rows && n0 + nt * 16 + c_at < g.n_out))
+          *reinterpret_cast<u32x4_any*>(o + nt * 16) =
               u32x4{T::pack2(r[0], r[1]), T::pack2(r[2], r[3]), T::pack2(r[4], r[5]), T::pack2(r[6], r[7])};
       }
+      o += 16 * g.out_ld;
     }
     return;
   }
@@ -413,24 +428,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) turn[(nt * 16 + 4 * grp + i) * 72 + mt * 16 + l16] = T::from_float(acc[mt][nt][i] * g.scale);
-  const int per = g.geo.OH * g.geo.OW;
+      for (int i = 0; i < 4; i += 2) {
+        const uint32_t two = T::pack2(acc[mt][nt][i] * g.scale, acc[mt][nt][i + 1] * g.scale);
+        uint16_t* d = turn + (nt * 16 + 4 * grp + i) * 72 + mt * 16 + l16;
+        d[0] = (uint16_t)two;
+        d[72] = (uint16_t)(two >> 16);
+      }
+  const int per = g.geo.OH * g.geo.OW, pos = pos0 + lane % 8 * 8;
+  if (pos >= g.rows) return;
+  uint32_t p;
+  const int img = (int)divide((uint32_t)pos, (uint32_t)per, g.geo.m_image, &p);
+  uint16_t* o = g.out + (int64_t)img * g.out_sn + (int64_t)(n0 + lane / 8) * g.out_sc + p;
+  const uint16_t* from = turn + lane / 8 * 72 + lane % 8 * 8;
+  const bool one_image = (int)p + 8 <= per;
 #pragma unroll
-  for (int k = 0; k < 2 * NT; ++k) {
-    const int c = k * 8 + lane / 8, pos = pos0 + lane % 8 * 8, n = n0 + c;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(turn + c * 72 + lane % 8 * 8);
-    if (n >= g.n_out || pos >= g.rows) continue;
-    uint32_t p;
-    const int img = (int)divide((uint32_t)pos, (uint32_t)per, g.geo.m_image, &p);
-    uint16_t* o = g.out + (int64_t)img * g.out_sn + (int64_t)n * g.out_sc + p;
-    if ((int)p + 8 <= per) {
-      *reinterpret_cast<u32x4_any*>(o) = v;
+  for (int k = 0; k < 2 * NT; ++k, o += 8 * g.out_sc, from += 8 * 72) {
+    const int n = n0 + k * 8 + lane / 8;
+    if (n >= g.n_out) break;
+    if (one_image) {
+      *reinterpret_cast<u32x4_any*>(o) = *reinterpret_cast<const u32x4*>(from);
     } else {  // the eight cross into the next image
 #pragma unroll 1
       for (int i = 0; i < 8 && pos + i < g.rows; ++i) {
         uint32_t at_p;
         const int im = (int)divide((uint32_t)(pos + i), (uint32_t)per, g.geo.m_image, &at_p);
-        g.out[(int64_t)im * g.out_sn + (int64_t)n * g.out_sc + at_p] = turn[c * 72 + lane % 8 * 8 + i];
+        g.out[(int64_t)im * g.out_sn + (int64_t)n * g.out_sc + at_p] = from[i];
       }
     }
   }
@@ -543,8 +565,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
     *reinterpret_cast<u32x4*>(smem + tid / 4 * buffer + g.span * kDwPitch + tid % 4 * 16) = u32x4{0u, 0u, 0u, 0u};
   auto kept_bit = [&](int turn) -> bool {  // lane j: block column cb0 + j of this wave's row block
     const int rb = turn * 4 + pb, cb = cb0 + lane;
-    return lane < 32 && rb * 64 < g.rows && cb < cbs &&
-           (g.mask == nullptr || g.mask[(int64_t)(rb / g.split) * g.msr + (int64_t)(cb / g.split) * g.msc] == 0);
+    return lane < 32 && rb * 64 < g.rows && cb < cbs && block_kept(g, rb, cb);
   };
 
   f32x4 acc[kDwTaps][4];
