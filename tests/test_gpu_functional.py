@@ -637,3 +637,36 @@ def test_odd_multiples_of_32_through_autograd_and_the_fused_mlp(bs):
     assert max_tile_rel_fro(xg.grad, rdx, tile=32) <= REL_FRO_TOL
     for got, ref in zip(wgs, rdws):
         assert max_tile_rel_fro(got.grad, ref, tile=32) <= REL_FRO_TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gelu_and_its_derivative_value_by_value(dtype):
+    """The stores' GELU over its whole range, at an identity product, against erfc in 64 bits.  Bound: half a unit of the element
+    type, and 1e-6 for the fp32 arithmetic (the polynomials are within 4e-7 of x * Phi(x) and of its derivative, and the device's
+    exponential and reciprocal are within a unit of 1.2e-7 of values up to 1); below -4, where x * Phi(x) is small, 1 % of the value."""
+    from scipy.special import erfc
+
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    v = torch.cat([torch.linspace(-9, 9, 128 * 64 - 6), torch.tensor([0.0, -0.0, 60.0, -60.0, 3e4, -3e4])]).to(dtype).reshape(128, 64)
+    half = 2.0 ** (-11 if dtype == torch.float16 else -8)  # 10 and 7 bits behind the leading one
+    x = to_np(v).astype(np.float64)
+    cdf = 0.5 * erfc(-x / np.sqrt(2))
+    y, pre = ext.gemm_act(v.cuda(), torch.eye(64, dtype=dtype).cuda(), "gelu", want_pre=True)
+    assert torch.equal(pre.cpu(), v)
+    err = np.abs(to_np(y).astype(np.float64) - x * cdf)
+    assert (err <= half * np.abs(x * cdf) + np.where(x < -4, 1e-2 * np.abs(x * cdf) + 6e-8, 1e-6)).all()
+    ones = torch.zeros(128, 8, dtype=dtype)
+    ones[:, 0] = 1
+    lists = ext.build_lists(torch.zeros(2, 1, dtype=torch.bool, device="cuda"))
+    d = ext.gemm_sdd_lists_actgrad(ones.cuda(), torch.ones(64, 8, dtype=dtype).cuda(), lists, 64, 1.0, "gelu", v.cuda())
+    want = cdf + x * np.exp(-x * x / 2) / np.sqrt(2 * np.pi)
+    assert (np.abs(to_np(d).astype(np.float64) - want) <= half * np.abs(want) + 1e-6).all()
+    # (x * Phi(x) and its derivative as they stand: 0 * Inf is a NaN)
+    w = torch.zeros(8, 8, dtype=dtype)
+    w[0, 0] = 1
+    special = torch.zeros(3, 8, dtype=dtype)
+    special[:, 0] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    got = ext.gemm_act(special.cuda(), w.cuda(), "gelu")[0][:, 0].cpu()
+    assert got[0] == float("inf") and got[1:].isnan().all()
