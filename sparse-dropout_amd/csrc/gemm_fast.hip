@@ -142,13 +142,9 @@ __device__ __forceinline__ void dsd_body(const GemmArgs& g, int tiles_m, int til
   // ---- union of the kept lists of the 4 row blocks: (K block, 4-bit keep flags) per step -------
   for (int i = tid; i < Kb; i += THREADS) scratch[i] = 0;
   __syncthreads();
-  if (ms) {
-    const int rows = (rb0 + R <= Mb) ? R : Mb - rb0;
-    for (int i = tid; i < rows * Kb; i += THREADS) {
-      const int r = i / Kb, k = i - r * Kb;
-      const uint32_t q = ms->merge == 2 ? ms->kept_quads(rb0 + r, kb_lo + k) : (ms->dropped(rb0 + r, kb_lo + k) ? 0u : 0xfu);
-      if (q) atomicOr(&scratch[k], q << (4 * r));
-    }
+  if (ms) {  // (the table lies in the idle stages)
+    static_assert(union_table_bytes(R, MAX_STEPS) <= S::SMEM_STEPS, "the table must fit in the stages");
+    union_of_mask<THREADS>(*ms, rb0, rb0 + R <= Mb ? R : Mb - rb0, kb_lo, Kb, scratch, reinterpret_cast<uint8_t*>(smem), tid);
   } else if (g.row_ptr) {
     for (int r = 0; r < R; ++r) {
       if (rb0 + r >= Mb) break;
@@ -964,7 +960,8 @@ __global__ __launch_bounds__(S::THREADS) void forward_lists_kernel(GemmArgs g, i
                                             bid / tiles, &ms);
   } else {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    flat_lists_block<S::THREADS>(f, bid - n_gemm, reinterpret_cast<int32_t*>(smem));
+    static_assert(flat_lds(kTableEntriesMost) <= S::SMEM_STEPS, "the table lies where the stages would");
+    flat_lists_block<S::THREADS, true>(f, bid - n_gemm, smem);
   }
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }
@@ -2211,7 +2208,7 @@ int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hip
 int launch_forward_with_lists(const GemmArgs& g, const MaskSrc& src, int64_t mb, int64_t kb, int32_t* row_ptr,
                               int32_t* col_idx, int32_t* col_ptr, int32_t* row_idx, uint8_t* mask_out,
                               int64_t mask_rows, int dtype, hipStream_t stream) {
-  if (g.bs != BS || mb * kb > kFlatMaxEntries) return SD_ERR_UNSUPPORTED;
+  if (g.bs != BS || mb * kb > kFlatMaxEntries || (int64_t)src.mb * src.kb > kTableEntriesMost) return SD_ERR_UNSUPPORTED;
   if (mb != (g.M + BS - 1) / BS || kb != (g.K + BS - 1) / BS) return SD_ERR_UNSUPPORTED;
   const DsdForm form = dsd_form(g);
   if (!form.ok || !form.kc || form.cm) return SD_ERR_UNSUPPORTED;

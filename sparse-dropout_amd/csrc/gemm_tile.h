@@ -51,7 +51,7 @@ struct TileShape {
   // the number of steps and the step table behind the stages, for a reduction of kb blocks
   static constexpr int smem_for(int64_t kb) { return SMEM_STEPS + 16 + 4 * (int)((kb < MAX_STEPS ? kb : MAX_STEPS) + TILE_PAD); }
   static constexpr int SMEM = SMEM_STEPS + 16 + 4 * (MAX_STEPS + TILE_PAD);
-  static_assert(LPW * LOADERS == 8 && 4 * MAX_STEPS <= SMEM_STEPS, "loads divide evenly; the merge scratch lies in the stages");
+  static_assert(LPW * LOADERS == 8 && 4 * MAX_STEPS + union_table_bytes(R, MAX_STEPS) <= SMEM_STEPS, "loads divide evenly; the merge scratch lies in the stages");
   static_assert(!HALVES || (MT == 4 && NW * 2 * NT16 * 1024 <= SMEM_STEPS), "the halves meet in the stages");
 };
 
@@ -168,7 +168,8 @@ __device__ inline void store_piece(const GemmArgs& g, f32x4 (&v)[MT][NT16], int 
 
 // The step table of a workgroup that owns row blocks rb0 .. rb0 + R - 1: the union of their kept lists (from the mask
 // source when the lists do not exist yet, from the lists, or everything for a dense product), one word per step.
-// scratch: a uint32 per reduction block; a barrier must follow before anybody reads the table or reuses the scratch.
+// scratch: a uint32 per reduction block and union_table_bytes behind them; a barrier must follow before anybody reads the
+// table or reuses the scratch.
 template <int R, int THREADS>
 __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0, int Mb, int kb_lo, int Kb, uint32_t* scratch,
                                    uint32_t* step_e, int* nsteps_p, int tid, int wave, int lane) {
@@ -177,11 +178,7 @@ __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0
     for (int i = tid; i < Kb; i += THREADS) scratch[i] = 0;
     __syncthreads();
     if (ms) {
-      for (int i = tid; i < rows * Kb; i += THREADS) {
-        const int r = i / Kb, k = i - r * Kb;
-        const uint32_t q = ms->merge == 2 ? ms->kept_quads(rb0 + r, kb_lo + k) : (ms->dropped(rb0 + r, kb_lo + k) ? 0u : 0xfu);
-        if (q) atomicOr(&scratch[k], q << (4 * r));
-      }
+      union_of_mask<THREADS>(*ms, rb0, rows, kb_lo, Kb, scratch, reinterpret_cast<uint8_t*>(scratch + Kb), tid);
     } else {
       for (int r = 0; r < rows; ++r) {
         const int beg = g.row_ptr[rb0 + r], end = g.row_ptr[rb0 + r + 1];

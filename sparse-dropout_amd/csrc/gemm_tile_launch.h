@@ -56,7 +56,8 @@ __global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, in
     tile_dsd_body<T, true, false, S>(g, tiles_m, tiles_n, Mb, Kb, bid, nsplit, &ms);
   } else {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    flat_lists_block<S::THREADS>(f, bid - n_gemm, reinterpret_cast<int32_t*>(smem));
+    static_assert(flat_lds(kTableEntriesMost) <= S::SMEM_STEPS, "the table lies where the stages would");
+    flat_lists_block<S::THREADS, true>(f, bid - n_gemm, smem);
   }
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }

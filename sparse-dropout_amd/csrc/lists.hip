@@ -64,9 +64,10 @@ __device__ inline void block_scan_inplace(int32_t* ptr, int64_t n, int32_t* lds 
 // The single-launch builder (flat_lists_block) as a launch of its own.
 constexpr int kFlatThreads = 1024;
 
+template <bool TABLED>
 __global__ __launch_bounds__(kFlatThreads) void build_lists_flat(FlatJobs f) {
-  __shared__ int32_t lds[kFlatThreads / kWave];
-  flat_lists_block<kFlatThreads>(f, (int)blockIdx.x, lds);
+  __shared__ __attribute__((aligned(16))) char lds[flat_lds(TABLED ? kTableEntries : 0)];
+  flat_lists_block<kFlatThreads, TABLED>(f, (int)blockIdx.x, lds);
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }
 
@@ -142,7 +143,8 @@ static int launch_lists(const MaskSrc& src, int64_t mb, int64_t kb, int32_t* row
   ListJob csc{src, 1, kb, mb, col_ptr, row_idx};
   if (mb * kb <= kFlatMaxEntries) {
     const FlatJobs f = flat_jobs(src, mb, kb, row_ptr, col_idx, col_ptr, row_idx, mask_out, mask_rows, kFlatThreads);
-    hipLaunchKernelGGL(build_lists_flat, dim3(f.blocks()), dim3(kFlatThreads), 0, stream, f);
+    const bool tabled = (int64_t)src.mb * src.kb <= kTableEntries;
+    hipLaunchKernelGGL(tabled ? &build_lists_flat<true> : &build_lists_flat<false>, dim3(f.blocks()), dim3(kFlatThreads), 0, stream, f);
     if (advanced) *advanced = src.state != nullptr;
     return check_launch("build_lists_flat");
   }

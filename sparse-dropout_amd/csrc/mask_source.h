@@ -61,16 +61,17 @@ struct MaskSrc {
       off_hi = (uint32_t)(off >> 32);
     }
   }
-  __device__ inline bool dropped_entry(int32_t si, int32_t sj) const {
+  __device__ __forceinline__ bool dropped_entry(int32_t si, int32_t sj) const {
     if (mask) return mask[si * st_row + sj * st_col] != 0;
     const uint64_t e = (uint64_t)si * (uint32_t)kb + (uint32_t)sj;
     uint32_t c[4] = {(uint32_t)(e >> 2), (uint32_t)(e >> 34), off_lo, off_hi};
     Philox{seed_lo, seed_hi}(c);
     // 24 random bits -> [0, 1) in steps of 2^-24, exact in fp32; True (dropped) with probability p
-    return (float)(c[e & 3] >> 8) * 0x1p-24f < p;
+    const uint32_t word = e & 2u ? (e & 1u ? c[3] : c[2]) : (e & 1u ? c[1] : c[0]);
+    return (float)(word >> 8) * 0x1p-24f < p;
   }
   // One generator call yields the draws of four consecutive entries: bit v = entry 4 * grp + v is dropped.
-  __device__ inline uint32_t dropped4(uint64_t grp) const {
+  __device__ __forceinline__ uint32_t dropped4(uint64_t grp) const {
     uint32_t c[4] = {(uint32_t)grp, (uint32_t)(grp >> 32), off_lo, off_hi};
     Philox{seed_lo, seed_hi}(c);
     uint32_t bits = 0;
@@ -78,22 +79,44 @@ struct MaskSrc {
     for (int v = 0; v < 4; ++v) bits |= ((float)(c[v] >> 8) * 0x1p-24f < p ? 1u : 0u) << v;
     return bits;
   }
-  // merge == 2: keep bits of the four 32-blocks of listed entry (i, j); bit 2a + b = block (2i + a, 2j + b)
-  __device__ inline uint32_t kept_quads(int32_t i, int32_t j) const {
+  // The same for a stored mask of `total` entries
+  __device__ __forceinline__ uint32_t stored4(int32_t grp, int32_t total) const {
+    int32_t si = grp * 4 / kb, sj = grp * 4 - si * kb;
+    uint32_t bits = 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (grp * 4 + v < total && mask[si * st_row + sj * st_col] != 0) bits |= 1u << v;
+      if (++sj == kb) { sj = 0; ++si; }
+    }
+    return bits;
+  }
+  // merge == 2: keep bits of the four 32-blocks of listed entry (i, j); bit 2a + b = block (2i + a, 2j + b).
+  // at(si, sj): whether a stored or drawn entry is dropped
+  template <typename At>
+  __device__ __forceinline__ uint32_t kept_quads(int32_t i, int32_t j, At at) const {
     uint32_t q = 0;
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         // 32-blocks (2i + a, 2j + b); a stored entry covers split x split of them (block size 32 * split)
-        const int32_t si = (2 * i + a) / split, sj = (2 * j + b) / split;
-        if (si < mb && sj < kb && !dropped_entry(si, sj)) q |= 1u << (2 * a + b);
+        int32_t si = 2 * i + a, sj = 2 * j + b;
+        if (split != 1) {
+          si /= split;
+          sj /= split;
+        }
+        if (si < mb && sj < kb && !at(si, sj)) q |= 1u << (2 * a + b);
       }
     return q;
   }
-  __device__ inline bool dropped(int32_t i, int32_t j) const {
-    if (merge == 2) return kept_quads(i, j) == 0;
-    return split == 1 ? dropped_entry(i, j) : dropped_entry(i / split, j / split);
+  template <typename At>
+  __device__ __forceinline__ bool dropped(int32_t i, int32_t j, At at) const {
+    if (merge == 2) return kept_quads(i, j, at) == 0;
+    return split == 1 ? at(i, j) : at(i / split, j / split);
+  }
+  // each entry evaluated where it is asked for
+  __device__ __forceinline__ auto one_by_one() const {
+    return [this](int32_t si, int32_t sj) { return dropped_entry(si, sj); };
   }
 };
 
@@ -104,22 +127,28 @@ struct ListJob {
   int64_t len;     // entries per line
   int32_t* ptr;    // [nlines + 1]
   int32_t* idx;    // [capacity nlines * len]
-  __device__ inline bool kept(int64_t line, int64_t e) const {
-    return by_col ? !src.dropped((int32_t)e, (int32_t)line) : !src.dropped((int32_t)line, (int32_t)e);
+  // 0 where entry e of `line` is dropped; kept: with merge == 2 the four keep bits of its 32-blocks, else 1
+  template <typename At>
+  __device__ __forceinline__ uint32_t keep(int32_t line, int32_t e, At at) const {
+    const int32_t i = by_col ? e : line, j = by_col ? line : e;
+    return src.merge == 2 ? src.kept_quads(i, j, at) : (src.dropped(i, j, at) ? 0u : 1u);
   }
-  // what goes into idx for kept entry e of `line`: e itself, with merge == 2 the four keep bits of its
+  __device__ inline bool kept(int64_t line, int64_t e) const { return keep((int32_t)line, (int32_t)e, src.one_by_one()) != 0u; }
+  // what goes into idx for kept entry e of `line`, q its keep(): e itself, with merge == 2 the four keep bits of its
   // 32-blocks in bits 28-31 (bit 2a + b: row half a, column half b of the LIST's own orientation, i.e.
   // transposed for a list by columns, which is the row list of the transposed mask)
-  __device__ inline int32_t entry(int64_t line, int64_t e) const {
-    if (src.merge != 2) return (int32_t)e;
-    uint32_t q = by_col ? src.kept_quads((int32_t)e, (int32_t)line) : src.kept_quads((int32_t)line, (int32_t)e);
+  __device__ inline int32_t entry_of(int32_t e, uint32_t q) const {
+    if (src.merge != 2) return e;
     if (by_col) q = (q & 0x9u) | ((q & 0x2u) << 1) | ((q & 0x4u) >> 1);
     return (int32_t)((uint32_t)e | (q << 28));
+  }
+  __device__ inline int32_t entry(int64_t line, int64_t e) const {
+    return src.merge != 2 ? (int32_t)e : entry_of((int32_t)e, keep((int32_t)line, (int32_t)e, src.one_by_one()));
   }
 };
 
 // Stores a drawn mask as row-major bytes (1 = dropped) for the caller to keep.
-__device__ inline void write_mask(const MaskSrc& src, int64_t mb, uint8_t* out, int64_t first,
+__device__ __forceinline__ void write_mask(const MaskSrc& src, int64_t mb, uint8_t* out, int64_t first,
                                   int64_t stride) {
   const int64_t total = mb * src.kb;
   if (src.mask == nullptr) {  // drawn: four entries per generator call
@@ -139,6 +168,13 @@ __device__ inline void write_mask(const MaskSrc& src, int64_t mb, uint8_t* out, 
 // THREADS * kFlatPer consecutive flat entries.  Blocks do not talk to each other: each first counts the kept
 // entries in front of its chunk itself (one sweep over at most 2^18 mask bytes, or draws), which replaces
 // the grid-wide scan and keeps the whole build in one launch with every load independent of the others.
+// A generator call costs a wave 600 clocks and more and yields four entries, so a block evaluates the entries of a mask of up to
+// 2^14 (2^17 in a product's launch) once, into a table of four to a byte in LDS, and counts and lists from there (a stored mask comes into the table
+// in loads that do not wait for each other).  With a call per entry and listing, and one per entry in
+// the product's workgroups (union_of_mask), 4096 x 4096 -> 4096 forward took 105 us with a drawn mask of 32-blocks, so 94;
+// 2048^3 with one of 64-blocks 25.6, so 24.5, 4096 x 1024 -> 1024 16.7 and 15.7.
+constexpr int64_t kTableEntries = 1 << 14, kTableEntriesMost = 1 << 17;  // in a launch of its own, and in a product's LDS
+constexpr int flat_lds(int64_t entries) { return 64 + (int)(entries / 4); }
 constexpr int kFlatPer = 4;  // consecutive entries per thread
 constexpr int64_t kFlatMaxEntries = 1 << 18;
 
@@ -206,10 +242,14 @@ __device__ inline void report_in(uint64_t* advance, unsigned blocks_in_launch) {
   }
 }
 
-// Block b (of f.blocks()) of the build, by a block of THREADS threads; lds: THREADS / 64 ints.
-template <int THREADS>
-__device__ inline void flat_lists_block(const FlatJobs& f, int b, int32_t* lds) {
+// Block b (of f.blocks()) of the build, by a workgroup of THREADS threads; smem: 64 bytes of LDS, with TABLED the table
+// (a quarter of a byte per stored or drawn entry) behind them.
+template <int THREADS, bool TABLED>
+__device__ __forceinline__ void flat_lists_block(const FlatJobs& f, int b, char* smem) {
+  static_assert(THREADS <= 1024, "the scan's sums have 64 bytes");
   constexpr int kFlatChunk = THREADS * kFlatPer;
+  int32_t* lds = reinterpret_cast<int32_t*>(smem);
+  uint8_t* table = reinterpret_cast<uint8_t*>(smem + 64);
   const int tid = threadIdx.x;
   if (b >= f.blocks0 + f.blocks1) {  // store the drawn mask for the caller
     MaskSrc src = f.job0.src;
@@ -219,71 +259,132 @@ __device__ inline void flat_lists_block(const FlatJobs& f, int b, int32_t* lds) 
     return;
   }
   const bool second = b >= f.blocks0;
-  ListJob job = second ? f.job1 : f.job0;
+  // (field by field: a copy of either as a whole goes through scratch memory)
+  ListJob job{f.job0.src, second ? f.job1.by_col : f.job0.by_col, second ? f.job1.nlines : f.job0.nlines,
+              second ? f.job1.len : f.job0.len, second ? f.job1.ptr : f.job0.ptr, second ? f.job1.idx : f.job0.idx};
   job.src.resolve();
   if (second) b -= f.blocks0;
   const int len = (int)job.len;
   const int total_entries = (int)(job.nlines * job.len);
   const int f0 = b * kFlatChunk;
-
-  // kept entries in front of this block's chunk
-  // a mask drawn at the listed granularity: entry index = row-major position, four entries share a generator call
-  const bool drawn4 = job.src.mask == nullptr && job.src.split == 1 && job.src.merge == 1 && job.src.kb == (job.by_col ? (int)job.nlines : len);
-  int cnt = 0;
-  if (drawn4 && !job.by_col) {
-    for (int grp = tid; grp * 4 < f0; grp += THREADS) cnt += __popc(~job.src.dropped4((uint64_t)grp) & 0xFu);
-  } else if (drawn4) {
-    // lines are columns: in front of (col0, row0) lies every entry of an earlier column and the rows above in col0
-    const int kb = job.src.kb;
-    const int col0 = f0 / len, row0 = f0 - col0 * len;
-    for (int grp = tid; grp * 4 < total_entries; grp += THREADS) {
-      uint32_t kept = ~job.src.dropped4((uint64_t)grp) & 0xFu;
-      int row = (grp * 4) / kb, col = grp * 4 - row * kb;
+  const int kb = job.src.kb;
+  // entry index = row-major position
+  const bool plain = job.src.split == 1 && job.src.merge == 1 && kb == (job.by_col ? (int)job.nlines : len);
+  auto build = [&](auto at) __attribute__((always_inline)) {
+    // kept entries in front of this block's chunk
+    int cnt = 0;
+    if (!TABLED && job.src.mask == nullptr && plain && !job.by_col) {
+      for (int grp = tid; grp * 4 < f0; grp += THREADS) cnt += __popc(~job.src.dropped4((uint64_t)grp) & 0xFu);
+    } else if (!TABLED && job.src.mask == nullptr && plain) {
+      // lines are columns: in front of (col0, row0) lies every entry of an earlier column and the rows above in col0
+      const int col0 = f0 / len, row0 = f0 - col0 * len;
+      for (int grp = tid; grp * 4 < total_entries; grp += THREADS) {
+        uint32_t kept = ~job.src.dropped4((uint64_t)grp) & 0xFu;
+        int row = (grp * 4) / kb, col = grp * 4 - row * kb;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const bool front = grp * 4 + v < total_entries && (col < col0 || (col == col0 && row < row0));
-        if (!front) kept &= ~(1u << v);
-        if (++col == kb) { col = 0; ++row; }
+        for (int v = 0; v < 4; ++v) {
+          const bool front = grp * 4 + v < total_entries && (col < col0 || (col == col0 && row < row0));
+          if (!front) kept &= ~(1u << v);
+          if (++col == kb) { col = 0; ++row; }
+        }
+        cnt += __popc(kept);
       }
-      cnt += __popc(kept);
+    } else {
+      const int lines_on = THREADS / len, on = THREADS - lines_on * len;
+      int line = tid / len, e = tid - line * len;
+#pragma unroll 1
+      for (int i = tid; i < f0; i += THREADS) {
+        cnt += job.keep(line, e, at) ? 1 : 0;
+        line += lines_on;
+        e += on;
+        if (e >= len) { e -= len; ++line; }
+      }
     }
-  } else {
-    for (int f = tid; f < f0; f += THREADS) {
-      const int line = f / len;
-      cnt += job.kept(line, f - line * len) ? 1 : 0;
-    }
-  }
-  int base;
-  block_exclusive_scan<THREADS>(cnt, lds, base);
+    int base;
+    block_exclusive_scan<THREADS>(cnt, lds, base);
 
-  // this thread's entries
-  const int mine = f0 + tid * kFlatPer;
-  int line = mine / len, e = mine - line * len;
-  uint32_t bits = 0;
-  if (drawn4 && !job.by_col) {  // mine is a multiple of four: one generator call
-    if (mine < total_entries) {
-      bits = ~job.src.dropped4((uint64_t)(mine / 4)) & 0xFu;
-      if (mine + 4 > total_entries) bits &= (1u << (total_entries - mine)) - 1u;
+    // this thread's entries: eight bits of a word each
+    const int mine = f0 + tid * kFlatPer;
+    int line = mine / len, e = mine - line * len;
+    uint32_t keeps = 0;
+    int n = 0;
+    if (!TABLED && job.src.mask == nullptr && plain && !job.by_col) {  // mine is a multiple of four: one generator call
+      const uint32_t bits = mine < total_entries ? ~job.src.dropped4((uint64_t)(mine / 4)) & 0xFu : 0u;
+#pragma unroll
+      for (int v = 0; v < kFlatPer; ++v)
+        if (mine + v < total_entries && ((bits >> v) & 1u)) { keeps |= 1u << (8 * v); ++n; }
+    } else {
+      int l = line, x = e;
+#pragma unroll 1
+      for (int v = 0; v < kFlatPer; ++v) {
+        const uint32_t q = mine + v < total_entries ? job.keep(l, x, at) : 0u;
+        keeps |= q << (8 * v);
+        n += q ? 1 : 0;
+        if (++x == len) { x = 0; ++l; }
+      }
     }
-  } else {
-    int l = line, x = e;
+    int chunk_total;
+    int pos = base + block_exclusive_scan<THREADS>(n, lds, chunk_total);
 #pragma unroll
     for (int v = 0; v < kFlatPer; ++v) {
-      if (mine + v < total_entries && job.kept(l, x)) bits |= 1u << v;
-      if (++x == len) { x = 0; ++l; }
+      if (mine + v < total_entries) {
+        if (e == 0) job.ptr[line] = pos;
+        const uint32_t q = (keeps >> (8 * v)) & 0xffu;
+        if (q) job.idx[pos++] = job.entry_of(e, q);
+      }
+      if (++e == len) { e = 0; ++line; }
     }
+    if (tid == 0 && f0 + kFlatChunk >= total_entries) job.ptr[job.nlines] = base + chunk_total;
+  };
+  if constexpr (TABLED) {
+    int stored = job.src.mb * kb;
+    if (plain && !job.by_col && f0 + kFlatChunk < stored) stored = f0 + kFlatChunk;
+#pragma unroll 1
+    for (int grp = tid; grp * 4 < stored; grp += THREADS)
+      table[grp] = (uint8_t)(job.src.mask ? job.src.stored4(grp, stored) : job.src.dropped4((uint64_t)grp));
+    __syncthreads();
+    build([&](int32_t si, int32_t sj) {
+      const uint32_t e = (uint32_t)(si * kb + sj);
+      return ((table[e >> 2] >> (e & 3u)) & 1u) != 0u;
+    });
+  } else {
+    build(job.src.one_by_one());
   }
-  int chunk_total;
-  int pos = base + block_exclusive_scan<THREADS>(__popc(bits), lds, chunk_total);
-#pragma unroll
-  for (int v = 0; v < kFlatPer; ++v) {
-    if (mine + v < total_entries) {
-      if (e == 0) job.ptr[line] = pos;
-      if (bits & (1u << v)) job.idx[pos++] = job.entry(line, e);
+}
+
+// ---- keep bits of a product's own rows -----------------------------------------------------------------------------------
+// scratch[k] |= the keep bits (four per row block) of row blocks rb0 .. rb0 + rows - 1 at reduction blocks kb_lo .. + Kb - 1.
+// Where a thread would make more than one generator call (the entries of a mask of 32-blocks take four each), the drawn entries
+// are evaluated four to a call into `table` first (LDS: union_table_bytes, apart from the scratch).
+// Fewer are as fast each by itself, without the barrier (1024 x 1024 -> 1024: 7.8 us, through the table 8.4).
+constexpr int union_table_bytes(int rows, int steps) { return (2 * rows + 1) * (steps / 2 + 2); }
+template <int THREADS>
+__device__ __forceinline__ void union_of_mask(const MaskSrc& ms, int rb0, int rows, int kb_lo, int Kb, uint32_t* scratch, uint8_t* table, int tid) {
+  auto gather = [&](auto at) __attribute__((always_inline)) {
+    for (int i = tid; i < rows * Kb; i += THREADS) {
+      const int r = i / Kb, k = i - r * Kb;
+      const uint32_t q = ms.merge == 2 ? ms.kept_quads(rb0 + r, kb_lo + k, at) : (ms.dropped(rb0 + r, kb_lo + k, at) ? 0u : 0xfu);
+      if (q) atomicOr(&scratch[k], q << (4 * r));
     }
-    if (++e == len) { e = 0; ++line; }
+  };
+  if (ms.mask || (ms.merge == 1 && rows * Kb <= THREADS)) {
+    gather(ms.one_by_one());
+    return;
   }
-  if (tid == 0 && f0 + kFlatChunk >= total_entries) job.ptr[job.nlines] = base + chunk_total;
+  const int s0 = rb0 * ms.merge / ms.split, c0 = kb_lo * ms.merge / ms.split;
+  int s1 = ((rb0 + rows) * ms.merge - 1) / ms.split, c1 = ((kb_lo + Kb) * ms.merge - 1) / ms.split;
+  s1 = s1 < ms.mb ? s1 : ms.mb - 1;
+  c1 = c1 < ms.kb ? c1 : ms.kb - 1;
+  const int per_row = (c1 - c0) / 4 + 2;
+  for (int i = tid; i < (s1 - s0 + 1) * per_row; i += THREADS) {
+    const int r = i / per_row;
+    table[i] = (uint8_t)ms.dropped4((((uint64_t)(s0 + r) * (uint32_t)ms.kb + (uint32_t)c0) >> 2) + (uint32_t)(i - r * per_row));
+  }
+  __syncthreads();
+  gather([&](int32_t si, int32_t sj) {
+    const uint32_t e0 = (uint32_t)si * (uint32_t)ms.kb + (uint32_t)c0, e = (e0 & 3u) + (uint32_t)(sj - c0);
+    return ((table[(si - s0) * per_row + (int)(e >> 2)] >> (e & 3u)) & 1u) != 0u;
+  });
 }
 
 }  // namespace sd

@@ -155,3 +155,47 @@ def test_merged_lists_of_odd_multiples_of_32_bit_exact(rows, cols, bs, p):
     # the element mask is the one of the block size: what makes the composition the right oracle
     m32 = O.split_mask(mask.numpy(), k, O.mask_shape(rows, cols, 32))
     assert np.array_equal(O.expand_keep(m32, 32, rows, cols), O.expand_keep(mask.numpy(), bs, rows, cols))
+
+
+@pytest.mark.parametrize("M,K,N,bs,merged", [
+    (192, 25600, 200, 64, True),     # more entries of a workgroup's rows than it has threads, a split reduction
+    (3000, 2088, 264, 96, True),     # three 32-blocks to an entry, ragged, rows of the mask that start inside a group of four
+    (1056, 544, 4160, 32, True),     # 33 x 17 entries of 32-blocks
+    (16400, 2048, 128, 32, True),    # 513 x 64 entries: more than the table of a list build of its own, which evaluates one by one
+    (16416, 8224, 72, 32, False),    # 513 x 257 entries: more than a product's launch evaluates
+])
+def test_masks_evaluated_through_a_table(M, K, N, bs, merged):
+    """Drawn and stored masks on both sides of the limits up to which a workgroup evaluates a mask four entries at a time into
+    LDS: the mask is the oracle's, the lists are numpy's of it, and the product is the one over those lists."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    p, seed = 0.6, 91
+    gen = torch.Generator("cuda").manual_seed(3)
+    x = torch.randn(M, K, generator=gen, device="cuda", dtype=torch.half)
+    w = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).half()
+    mask = O.random_mask(O.mask_shape(M, K, bs), p, seed)
+    # keep bits of the 32-blocks of every 64-block: bit 2a + b = row half a, column half b
+    mb, kb = -(-M // 64), -(-K // 64)
+    fine = np.zeros((2 * mb, 2 * kb), dtype=np.int64)
+    keep = np.repeat(np.repeat(~mask, bs // 32, 0), bs // 32, 1)[:2 * mb, :2 * kb]
+    fine[:keep.shape[0], :keep.shape[1]] = keep
+    quads = sum(fine[a::2, b::2] << (2 * a + b) for a in range(2) for b in range(2))
+    rows, cols = np.nonzero(quads)
+    by_col = np.lexsort((rows, cols))
+    q = quads[rows, cols]
+    q_t = (q & 9) | ((q & 2) << 1) | ((q & 4) >> 1)
+    bits = (lambda e, b: (e | (b << 28)).astype(np.uint32).view(np.int32)) if bs % 64 else (lambda e, b: e.astype(np.int32))
+    want = (np.r_[0, np.cumsum(np.bincount(rows, minlength=mb))], bits(cols, q),
+            np.r_[0, np.cumsum(np.bincount(cols, minlength=kb))], bits(rows[by_col], q_t[by_col]))
+    stored = torch.from_numpy(mask).cuda()
+    for given in (stored, stored.t().contiguous().t(), None):
+        y, m, lists, g = ext.dropout_matmul_forward(x, w, bs, p, **({"seed": seed} if given is None else {"mask": given}))
+        assert ext.last_kernel_detail().startswith("dsd+lists:") == merged, ext.last_kernel_detail()
+        assert np.array_equal(m.cpu().numpy(), mask)
+        for a, b in zip((lists.row_ptr, lists.col_idx[:len(rows)], lists.col_ptr, lists.row_idx[:len(rows)]), want):
+            assert np.array_equal(a.cpu().numpy(), b)
+        alone = ext.build_lists(stored, -(bs // 32) if bs % 64 else bs // 64, (mb, kb))
+        assert all(torch.equal(getattr(alone, n)[:len(b)], getattr(lists, n)[:len(b)])
+                   for n, b in zip(("row_ptr", "col_idx", "col_ptr", "row_idx"), want))
+        assert torch.equal(y, ext.gemm_dsd_lists(x, w, lists, g, 1 / (1 - p)))
