@@ -144,4 +144,32 @@ struct TapPacking {
   }
 };
 
+// ---- LDS of the launches ----------------------------------------------------------------------------------------------------
+constexpr int kLdsLimit = 160 * 1024;
+constexpr int kPos = 256;    // result positions of a workgroup: four waves of 64
+constexpr int kStages = 3;   // steps of packed weights: two on their way
+constexpr int kTapRow = 128; // bytes of an LDS row of 64 channels
+constexpr int kTurnRow = 72; // halfs of a channel's 64 positions where an input gradient is turned into planes
+
+SD_BOTH int64_t span_of(const TapGeom& geo) { return (window_bound(geo, kPos) + 15) / 16 * 16; }
+// Four waves of 16 * nt channels, over everything else when the last product is done.
+SD_BOTH constexpr int taps_turn_bytes(int nt) { return 4 * 16 * nt * kTurnRow * 2; }
+// Forward or input gradient: weights, the window's rows and eight of zeros, tables; the turned result of the latter needs more where
+// the gradient it reads is narrower than the image (1 x 9 on 11 columns without padding: 36 464 bytes, turned in 36 864).
+SD_BOTH int64_t taps_lds(const TapGeom& geo, bool dx, int64_t span) {
+  const int64_t rs = geo.taps(), nrb = (span + 63) / 64 + 2;
+  const int64_t table = dx ? rs * nrb * 16 + ((rs * nrb + 15) & ~15LL) : 4 * rs * 128;
+  const int64_t products = kStages * kTapStep + (span + 8) * kTapRow + table;
+  return dx && products < taps_turn_bytes(4) ? taps_turn_bytes(4) : products;
+}
+
+constexpr int kDwTaps = 9;    // of a workgroup
+constexpr int kDwPitch = 64;  // bytes of an LDS row of 32 channels: the four rows of a transposing read in different banks
+// Weight gradient.  A buffer: rows of the window and one of zeros, 256 rows of dY, a record per position.  In the end two of the
+// four blocks' sums meet there: 2 x 2 waves x 64 lanes x 9 x 16 floats.
+SD_BOTH int64_t dw_lds(int64_t span, int buffers) {
+  const int64_t merge = 2 * 2 * 64 * kDwTaps * 16 * 4, turns = buffers * ((span + 16) * kDwPitch + 256 * 128 + 256 * 8);
+  return turns < merge ? merge : turns;
+}
+
 }  // namespace sd

@@ -28,16 +28,14 @@
 namespace sd {
 namespace {
 
-constexpr int kPos = 256;           // result positions of a workgroup: four waves of 64
 // LDS rows of 64 channels lie eight to a KB, [chunk of 8 channels][row % 8][16 bytes], and packed weights alike
 // ([output / 8][chunk][output % 8]): a fragment read takes its 16 bytes of rows a .. a + 3 and a + 12 .. a + 15 of one chunk and of
 // rows a + 4 .. a + 11 of the next in one go, wherever a lies, and those are then 64 different banks (rows 144 bytes apart, or the
 // GEMM kernels' XOR at an odd a: a third to a half of the LDS cycles conflicts).  The KB is also what a direct load of 8 whole
 // 128-byte lines leaves there, so rows need no registers on their way.
-constexpr int kRowBytes = 128;
+constexpr int kRowBytes = kTapRow;
 constexpr int kWeightStage = kTapStep;  // packed weights of a step
 constexpr int kUnit = kTapUnit;
-constexpr int kStages = 3;              // two steps of weights on their way
 
 struct TapArgs {
   TapGeom geo;  // result positions -> source pixels
@@ -397,7 +395,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   // ---- results: a lane holds channels 4 * grp .. + 3 of a 16-channel tile at position l16
   const int pos0 = m0 + wave * 64;
   if (!DX || !g.planes) {
-    if (NT == 1) return;
+    static_assert(NT % 2 == 0, "stored in pairs of tiles");
     const int c_at = (grp % 2) * 16 + (grp / 2) * 8;  // of a pair of tiles: 8 consecutive channels after the exchange
     uint16_t* o = g.out + (int64_t)pos0 * g.out_ld + n0 + (l16 * (int)g.out_ld + c_at);
     const bool whole = pos0 + 64 <= g.rows && n0 + 16 * NT <= g.n_out;
@@ -422,7 +420,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
   }
   // planes: turned in LDS, 8 consecutive positions of a channel per lane
   __syncthreads();
-  uint16_t* turn = reinterpret_cast<uint16_t*>(smem) + wave * (16 * NT * 72);
+  uint16_t* turn = reinterpret_cast<uint16_t*>(smem + wave * (taps_turn_bytes(NT) / 4));
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -430,19 +428,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
       for (int i = 0; i < 4; i += 2) {
         const uint32_t two = T::pack2(acc[mt][nt][i] * g.scale, acc[mt][nt][i + 1] * g.scale);
-        uint16_t* d = turn + (nt * 16 + 4 * grp + i) * 72 + mt * 16 + l16;
+        uint16_t* d = turn + (nt * 16 + 4 * grp + i) * kTurnRow + mt * 16 + l16;
         d[0] = (uint16_t)two;
-        d[72] = (uint16_t)(two >> 16);
+        d[kTurnRow] = (uint16_t)(two >> 16);
       }
   const int per = g.geo.OH * g.geo.OW, pos = pos0 + lane % 8 * 8;
   if (pos >= g.rows) return;
   uint32_t p;
   const int img = (int)divide((uint32_t)pos, (uint32_t)per, g.geo.m_image, &p);
   uint16_t* o = g.out + (int64_t)img * g.out_sn + (int64_t)(n0 + lane / 8) * g.out_sc + p;
-  const uint16_t* from = turn + lane / 8 * 72 + lane % 8 * 8;
+  const uint16_t* from = turn + lane / 8 * kTurnRow + lane % 8 * 8;
   const bool one_image = (int)p + 8 <= per;
 #pragma unroll
-  for (int k = 0; k < 2 * NT; ++k, o += 8 * g.out_sc, from += 8 * 72) {
+  for (int k = 0; k < 2 * NT; ++k, o += 8 * g.out_sc, from += 8 * kTurnRow) {
     const int n = n0 + k * 8 + lane / 8;
     if (n >= g.n_out) break;
     if (one_image) {
@@ -464,8 +462,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 // serve all its taps, its image fragments are transposing reads of rows shifted by the tap.  The four blocks' sums meet
 // in LDS at the end, so a CU leaves one partial result (a round of 256 of them: 19 MB at any size), which
 // taps_dw_reduce adds up.  Bound by what the waves issue: per tap 17 instructions of picks and some 20 of addresses beside 8 products.
-constexpr int kDwTaps = 9;
-constexpr int kDwPitch = 64;  // bytes of an LDS row of 32 channels: the four rows of a transposing read in different banks
 constexpr int kDwThreads = 512;
 
 struct TapDwArgs {
@@ -482,10 +478,6 @@ struct TapDwArgs {
   int buffers;         // 2: the next turn arrives under this one's products
   int per_split, one_more, k_blocks;
 };
-
-// LDS of a buffer: rows of the window and one of zeros, 256 rows of dY, a record per position
-inline int dw_buffer_bytes(int span) { return (span + 16) * kDwPitch + 256 * 128 + 256 * 8; }
-constexpr int kDwMerge = 2 * 2 * 64 * kDwTaps * 16 * 4;  // two of the four blocks' sums: 2 x 2 waves x 64 lanes x 9 x 16 floats
 
 template <typename T>
 __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_taps_dw_kernel(TapDwArgs g) {
@@ -722,16 +714,6 @@ __global__ __launch_bounds__(256) void taps_dw_reduce(const float* part, uint16_
 }
 
 // ---- host ---------------------------------------------------------------------------------------------------------------
-constexpr int kLdsLimit = 160 * 1024;
-
-int64_t taps_lds(const TapGeom& geo, bool dx, int64_t span) {
-  const int64_t rs = geo.taps(), nrb = (span + 63) / 64 + 2;
-  const int64_t table = dx ? rs * nrb * 16 + ((rs * nrb + 15) & ~15LL) : 4 * rs * 128;
-  return kStages * kWeightStage + (span + 8) * kRowBytes + table;
-}
-
-int64_t span_of(const TapGeom& geo) { return (window_bound(geo, kPos) + 15) / 16 * 16; }
-
 // Lets a kernel have more than 64 KB of LDS, once per device.
 int configure(const void* kernel, std::atomic<bool>* done) {
   int dev = 0;
@@ -792,7 +774,7 @@ bool fits(const ConvShape& v) {
   const TapGeom f = v.forward(), b = v.gradient();
   const int64_t sf = span_of(f), sb = span_of(b);
   if (sf > 1000 || sb > 1000) return false;
-  return taps_lds(f, false, sf) <= kLdsLimit && taps_lds(b, true, sb) <= kLdsLimit && dw_buffer_bytes((int)sf) <= kLdsLimit;
+  return taps_lds(f, false, sf) <= kLdsLimit && taps_lds(b, true, sb) <= kLdsLimit && dw_lds(sf, 1) <= kLdsLimit;
 }
 
 ConvShape shape_of(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
@@ -957,9 +939,8 @@ extern "C" int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* d
   g.per_split = (int)(turns / splits);
   g.one_more = (int)(turns % splits);
   g.k_blocks = (int)ceil_div(k_out, 64);
-  g.buffers = 2 * dw_buffer_bytes(g.span) <= kLdsLimit ? 2 : 1;
-  int smem = g.buffers * dw_buffer_bytes(g.span);
-  if (smem < kDwMerge) smem = kDwMerge;
+  g.buffers = dw_lds(g.span, 2) <= kLdsLimit ? 2 : 1;
+  const int smem = (int)dw_lds(g.span, g.buffers);
   const dim3 grid((unsigned)splits, (unsigned)ceil_div(r * s, kDwTaps), (unsigned)(ceil_div(c, 32) * g.k_blocks));
   const hipStream_t st = (hipStream_t)stream;
   static std::atomic<bool> done[2][16] = {};

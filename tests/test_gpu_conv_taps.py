@@ -27,6 +27,10 @@ GEOMS = [
     (9, 64, 3, 3, 64, 3, 3, (1, 1), (1, 1)),
     (2, 32, 1, 40, 64, 1, 7, (0, 3), (1, 1)),
     (1, 16, 3, 3, 16, 2, 2, (0, 0), (1, 1)),  # four output positions
+    # gradients narrower than the image: the planes of dX are turned in more LDS than its products use
+    (40, 64, 8, 11, 64, 1, 9, (0, 0), (1, 1)),
+    (30, 72, 5, 11, 40, 1, 3, (0, 0), (1, 4)),
+    (20, 40, 6, 15, 72, 1, 12, (0, 0), (1, 1)),
 ]
 
 

@@ -224,6 +224,94 @@ def test_tile_map_keeps_an_xcd_on_a_compact_patch():
         assert len(rows) <= 8 and len(cols) <= 5, (x, sorted(rows), sorted(cols))
 
 
+_TAP_SWEEP = r"""
+#include <stdio.h>
+#include <algorithm>
+#include "conv_taps.h"
+using namespace sd;
+
+static long n_geometries = 0, n_small = 0;
+
+// what a launch asks for holds everything its workgroups put there
+static bool lds_holds(const TapGeom& g, bool dx) {
+  const int64_t span = span_of(g);
+  const int64_t products = kStages * kTapStep + (span + 8) * kTapRow + (dx ? g.taps() * ((span + 63) / 64 + 2) * 17 : 4 * g.taps() * 128);
+  n_small += dx && products < taps_turn_bytes(4);
+  if (taps_lds(g, dx, span) < products || (dx && taps_lds(g, dx, span) < taps_turn_bytes(4))) return false;
+  for (int buffers = 1; buffers <= 2; ++buffers)
+    if (dw_lds(span, buffers) < buffers * ((span + 1) * kDwPitch + kPos * 128 + kPos * 8) || dw_lds(span, buffers) < 147456) return false;
+  return true;
+}
+
+// in-image bits and windows against a loop over everything
+static bool windows_hold(TapGeom g, int images) {
+  g.prepare();
+  const int rows = images * g.OH * g.OW, per = g.IH * g.IW;
+  for (int m0 = 0; m0 < rows; m0 += kPos) {
+    const int last = std::min(m0 + kPos, rows) - 1;
+    const TapWindow w(g, m0, last);
+    if (w.hi - w.lo > window_bound(g, kPos)) return false;
+    for (int pos = m0; pos <= last; ++pos) {
+      const TapPosition p(g, pos);
+      if (p.img != pos / (g.OH * g.OW) || p.oh != pos % (g.OH * g.OW) / g.OW || p.ow != pos % g.OW) return false;
+      uint32_t bits = 0;
+      for (int t = 0; t < g.taps(); ++t) {
+        const int h = p.oh - g.pad_h + t / g.S * g.dl_h, c = p.ow - g.pad_w + t % g.S * g.dl_w;
+        if (h < 0 || h >= g.IH || c < 0 || c >= g.IW) continue;
+        bits |= 1u << t;
+        const int px = p.img * per + h * g.IW + c;
+        if (px != p.pixel(g) + g.shift(t) || px < w.lo || px >= w.hi) return false;
+      }
+      if (bits != p.inside(g)) return false;
+    }
+  }
+  return true;
+}
+
+static int check(int h, int w, int r, int s, int ph, int pw, int dh, int dw, bool windows) {
+  const int po = h + 2 * ph - dh * (r - 1), qo = w + 2 * pw - dw * (s - 1);
+  if (po < 1 || qo < 1 || r * s < 2 || r * s > 32) return 0;
+  const TapGeom f{h, w, po, qo, r, s, ph, pw, dh, dw}, b{po, qo, h, w, r, s, (r - 1) * dh - ph, (s - 1) * dw - pw, dh, dw};
+  if (span_of(f) > 1000 || span_of(b) > 1000) return 0;
+  ++n_geometries;
+  const int images = 1 + 700 / std::max(h * w, po * qo);
+  if (lds_holds(f, false) && lds_holds(b, true) && (!windows || (windows_hold(f, images) && windows_hold(b, images)))) return 0;
+  printf("%d x %d, kernel %d x %d, padding %d %d, dilation %d %d\n", h, w, r, s, ph, pw, dh, dw);
+  return 1;
+}
+
+int main() {
+  // unpadded kernels nearly as wide as the image: the gradient they read is narrow
+  for (int h = 1; h <= 24; ++h)
+    for (int w = 1; w <= 24; ++w)
+      for (int r = 1; r <= 8; ++r)
+        for (int s = 1; s <= 32; ++s)
+          for (int d = 0; d < 9; ++d)
+            if (check(h, w, r, s, 0, 0, 1 + d / 3, 1 + d % 3, false)) return 1;
+  uint32_t x = 12345;
+  auto next = [&](int lo, int hi) { x = x * 1664525u + 1013904223u; return lo + (int)((x >> 8) % (uint32_t)(hi - lo + 1)); };
+  for (int i = 0; i < 6000; ++i) {
+    const int r = next(1, 6), s = next(1, 6);
+    if (check(next(1, 40), next(1, i % 8 ? 40 : 300), r, s, next(0, 5), next(0, 5), next(1, 3), next(1, 3), true)) return 1;
+  }
+  printf("%ld geometries, %ld turned in more than the products use\n", n_geometries, n_small);
+  return n_geometries < 10000 || n_small < 100;
+}
+"""
+
+
+def test_tap_windows_and_lds_hold_what_the_kernels_put_there(tmp_path):
+    """The tap-wise convolution's geometry (csrc/conv_taps.h is plain integer code, the same on host and device): which taps lie
+    inside the image, the window of source rows, its bound, and the LDS of the launches, over geometries of all kinds."""
+    import subprocess
+
+    (tmp_path / "sweep.cpp").write_text(_TAP_SWEEP)
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{ROOT / 'sparse-dropout_amd' / 'csrc'}", str(tmp_path / "sweep.cpp"), "-o",
+                    str(tmp_path / "sweep")], check=True)
+    proc = subprocess.run([str(tmp_path / "sweep")], capture_output=True, text=True, timeout=100)
+    assert proc.returncode == 0, proc.stdout
+
+
 def test_loader_refuses_a_library_built_from_other_sources(monkeypatch):
     from flash_dropout.hip import _loader
 
