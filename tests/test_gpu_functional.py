@@ -670,3 +670,17 @@ def test_gelu_and_its_derivative_value_by_value(dtype):
     special[:, 0] = torch.tensor([float("inf"), float("-inf"), float("nan")])
     got = ext.gemm_act(special.cuda(), w.cuda(), "gelu")[0][:, 0].cpu()
     assert got[0] == float("inf") and got[1:].isnan().all()
+
+
+def test_gelu_far_below_zero():
+    """x * Phi(x) down to where a bf16 holds no more of it, at an identity product, against erfc in 64 bits.  Bound: half a unit of the
+    element type, and the 2.5 % that the store's Phi may be off (2.2 % at -13; its error is relative there)."""
+    from scipy.special import erfc
+
+    from flash_dropout.hip import GEMM
+
+    v = torch.linspace(-13, -4, 128 * 64).to(torch.bfloat16).reshape(128, 64)
+    y, _ = GEMM().gemm_act(v.cuda(), torch.eye(64, dtype=torch.bfloat16).cuda(), "gelu", want_pre=True)
+    x = to_np(v).astype(np.float64)
+    want = x * 0.5 * erfc(-x / np.sqrt(2))
+    assert (np.abs(y.double().cpu().numpy() - want) <= (2.0 ** -8 + 0.025) * np.abs(want)).all()
