@@ -955,7 +955,7 @@ __global__ __launch_bounds__(S::THREADS) void dsd_kernel(GemmArgs g, int tiles_m
 // The forward product and the kept lists of its mask in ONE launch: workgroups [0, n_gemm) are the product's and take
 // their keep bits from the mask source itself (a handful of generator calls or mask bytes per workgroup), the others
 // build the lists the backward will read, and store a drawn mask.  Nothing in the launch waits for anything else.
-template <typename T, bool RAGGED, typename S>
+template <typename T, bool RAGGED, typename S, bool TABLED>
 __global__ __launch_bounds__(S::THREADS) void forward_lists_kernel(GemmArgs g, int tiles_m, int tiles_n, int Mb,
                                                                    int Kb_all, int nsplit, int n_gemm, FlatJobs f) {
   const int bid = (int)blockIdx.x;
@@ -968,7 +968,7 @@ __global__ __launch_bounds__(S::THREADS) void forward_lists_kernel(GemmArgs g, i
   } else {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     static_assert(flat_lds(kTableEntriesMost) <= S::SMEM_STEPS, "the table lies where the stages would");
-    flat_lists_block<S::THREADS, true>(f, bid - n_gemm, smem);
+    flat_lists_block<S::THREADS, TABLED>(f, bid - n_gemm, smem);
   }
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }
@@ -2184,6 +2184,17 @@ int launch_fast(const GemmArgs& g, int mode, int dtype, hipStream_t stream) {
 }
 
 // ---- the forward product and the kept lists of its mask in one launch -------------------------------------------
+// Whether the launch's workgroups evaluate a drawn mask through a table in LDS.  It pays where the list blocks come behind a full round
+// of the product's workgroups and are waited for (us without -> with: 4096 x 784 -> 1024 14.7 -> 14.0, 4096 x 4096 -> 1024 in
+// blocks of 128 37.6 -> 35.6, 8192 x 4096 -> 512 in 32-blocks 61.8 -> 49.9), and for the masks of 32-blocks, whose listed entries take four
+// draws each (16384 x 8192 -> 128, beside which half of the CUs have nothing to do: 164 -> 124).  Elsewhere it is a barrier and
+// more code in front of the first product: 512 x 1024 -> 1024 8.51 -> 8.72, 1024^3 7.40 -> 7.59.  A stored mask is a load an entry, which
+// costs less than the table: 4096^3 70.5 -> 74.7, 2048^3 23.3 -> 23.6, with 32-blocks 82.7 -> 86.4 and 28.1 -> 28.4.
+bool mask_table_pays(const MaskSrc& src, int shape, int64_t workgroups) {
+  if (src.mask != nullptr || (int64_t)src.mb * src.kb > kTableEntriesMost) return false;
+  return src.merge == 2 || workgroups >= (shape == kShapeOne || shape == kShapeWide ? 512 : 256);
+}
+
 // most workgroups the product may have for its lists to ride along (SPARSEDROP_FORWARD_LISTS_LIMIT overrides, for
 // measuring; 0 switches the single launch off)
 int64_t forward_lists_limit() {
@@ -2194,11 +2205,11 @@ int64_t forward_lists_limit() {
   return limit;
 }
 
-template <typename T, bool RAGGED>
+template <typename T, bool RAGGED, bool TABLED>
 int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
   using S = DsdBig;
   static std::atomic<bool> configured[kMaxDevices] = {};
-  auto* kernel = &forward_lists_kernel<T, RAGGED, S>;
+  auto* kernel = &forward_lists_kernel<T, RAGGED, S, TABLED>;
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(kernel), S::SMEM_BYTES, configured)) return rc;
   const int Mb = (int)((g.M + BS - 1) / BS), Kb = (int)((g.K + BS - 1) / BS);
   const int tiles_m = (Mb + S::R - 1) / S::R, tiles_n = (int)((g.N + S::BN - 1) / S::BN);
@@ -2206,6 +2217,11 @@ int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hip
   hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::SMEM_BYTES, stream, g, tiles_m,
                      tiles_n, Mb, Kb, splits, n_gemm, f);
   return check_launch("forward_lists_kernel");
+}
+template <typename T>
+int launch_forward_lists(const GemmArgs& g, bool ragged, int splits, const FlatJobs& f, hipStream_t stream) {
+  if (f.tabled) return ragged ? launch_forward_lists_t<T, true, true>(g, splits, f, stream) : launch_forward_lists_t<T, false, true>(g, splits, f, stream);
+  return ragged ? launch_forward_lists_t<T, true, false>(g, splits, f, stream) : launch_forward_lists_t<T, false, false>(g, splits, f, stream);
 }
 
 // g: the forward product (reduction-contiguous operands, row-major C) on the 64 grid; src: its mask, listed on an
@@ -2215,24 +2231,22 @@ int launch_forward_lists_t(const GemmArgs& g, int splits, const FlatJobs& f, hip
 int launch_forward_with_lists(const GemmArgs& g, const MaskSrc& src, int64_t mb, int64_t kb, int32_t* row_ptr,
                               int32_t* col_idx, int32_t* col_ptr, int32_t* row_idx, uint8_t* mask_out,
                               int64_t mask_rows, int dtype, hipStream_t stream) {
-  if (g.bs != BS || mb * kb > kFlatMaxEntries || (int64_t)src.mb * src.kb > kTableEntriesMost) return SD_ERR_UNSUPPORTED;
+  if (g.bs != BS || mb * kb > kFlatMaxEntries) return SD_ERR_UNSUPPORTED;
   if (mb != (g.M + BS - 1) / BS || kb != (g.K + BS - 1) / BS) return SD_ERR_UNSUPPORTED;
   const DsdForm form = dsd_form(g);
   if (!form.ok || !form.kc || form.cm) return SD_ERR_UNSUPPORTED;
   const DsdPlan plan = plan_for(g, form);
   if (plan.splits < 1 || dsd_tiles<DsdBig>(g.M, g.N) > forward_lists_limit()) return SD_ERR_UNSUPPORTED;
-  const FlatJobs f = flat_jobs(src, mb, kb, row_ptr, col_idx, col_ptr, row_idx, mask_out, mask_rows,
-                               plan.shape == kShapeBig ? DsdBig::THREADS : tile_threads(plan.shape));
+  FlatJobs f = flat_jobs(src, mb, kb, row_ptr, col_idx, col_ptr, row_idx, mask_out, mask_rows,
+                         plan.shape == kShapeBig ? DsdBig::THREADS : tile_threads(plan.shape));
+  f.tabled = mask_table_pays(src, plan.shape, shape_tiles(plan.shape, g.M, g.N) * plan.splits);
   int rc;
   if (plan.shape != kShapeBig)
     rc = is_bf16(dtype) ? tile_forward<BF16>(g, plan.shape, plan.splits, f, stream)
                         : tile_forward<F16>(g, plan.shape, plan.splits, f, stream);
-  else if (is_bf16(dtype))
-    rc = form.ragged ? launch_forward_lists_t<BF16, true>(g, plan.splits, f, stream)
-                     : launch_forward_lists_t<BF16, false>(g, plan.splits, f, stream);
   else
-    rc = form.ragged ? launch_forward_lists_t<F16, true>(g, plan.splits, f, stream)
-                     : launch_forward_lists_t<F16, false>(g, plan.splits, f, stream);
+    rc = is_bf16(dtype) ? launch_forward_lists<BF16>(g, form.ragged, plan.splits, f, stream)
+                        : launch_forward_lists<F16>(g, form.ragged, plan.splits, f, stream);
   if (rc) return rc;
   note_kernel("dsd+lists:%s%s splits=%d", dsd_name(plan.shape), form.ragged && plan.shape == kShapeBig ? ":ragged" : "",
               plan.splits);

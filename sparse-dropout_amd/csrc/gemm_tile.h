@@ -170,7 +170,7 @@ __device__ inline void store_piece(const GemmArgs& g, f32x4 (&v)[MT][NT16], int 
 // source when the lists do not exist yet, from the lists, or everything for a dense product), one word per step.
 // scratch: a uint32 per reduction block and union_table_bytes behind them; a barrier must follow before anybody reads the
 // table or reuses the scratch.
-template <int R, int THREADS>
+template <int R, int THREADS, bool TABLED>
 __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0, int Mb, int kb_lo, int Kb, uint32_t* scratch,
                                    uint32_t* step_e, int* nsteps_p, int tid, int wave, int lane) {
   const int rows = rb0 + R <= Mb ? R : Mb - rb0;
@@ -178,7 +178,7 @@ __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0
     for (int i = tid; i < Kb; i += THREADS) scratch[i] = 0;
     __syncthreads();
     if (ms) {
-      union_of_mask<THREADS>(*ms, rb0, rows, kb_lo, Kb, scratch, reinterpret_cast<uint8_t*>(scratch + Kb), tid);
+      union_of_mask<THREADS, TABLED>(*ms, rb0, rows, kb_lo, Kb, scratch, reinterpret_cast<uint8_t*>(scratch + Kb), tid);
     } else {
       for (int r = 0; r < rows; ++r) {
         const int beg = g.row_ptr[rb0 + r], end = g.row_ptr[rb0 + r + 1];
@@ -213,7 +213,7 @@ __device__ inline void union_steps(const GemmArgs& g, const MaskSrc* ms, int rb0
 // ---- DSD and dense: C = s (keep . A) B^T ------------------------------------------------------------------------------
 // KC: both operands reduction-contiguous (forward) or both reduction-strided (weight gradient).  Arguments as for the
 // large shapes' dsd_body.
-template <typename T, bool KC, bool CM, typename S>
+template <typename T, bool KC, bool CM, typename S, bool TABLED = false>
 __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, int tiles_n, int Mb, int Kb_all, int bid,
                                               int nsplit, const MaskSrc* ms = nullptr) {
   constexpr int R = S::R, C = S::C, NST = S::NST, LPW = S::LPW, MT = S::MT, NT16 = S::NT16, KG = S::HALVES ? 2 : 1;
@@ -235,7 +235,7 @@ __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, in
   const int kb_lo = (int)((int64_t)Kb_all * split / nsplit);
   const int Kb = (int)((int64_t)Kb_all * (split + 1) / nsplit) - kb_lo;
 
-  union_steps<R, S::THREADS>(g, ms, rb0, Mb, kb_lo, Kb, scratch, step_e, nsteps_p, tid, wave, lane);
+  union_steps<R, S::THREADS, TABLED>(g, ms, rb0, Mb, kb_lo, Kb, scratch, step_e, nsteps_p, tid, wave, lane);
 
   // ---- loads
   const int k_valid = (int)(g.K % BS);

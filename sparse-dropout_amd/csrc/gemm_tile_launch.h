@@ -46,18 +46,18 @@ __global__ __launch_bounds__(S::THREADS) void tile_sdd_kernel(GemmArgs g, int ti
 }
 
 // The forward product and the kept lists of its mask in one launch (see forward_lists_kernel of the large shapes).
-template <typename T, typename S>
+template <typename T, typename S, bool TABLED>
 __global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, int tiles_m, int tiles_n, int Mb, int Kb,
                                                                   int nsplit, int n_gemm, FlatJobs f) {
   const int bid = (int)blockIdx.x;
   if (bid < n_gemm) {
     MaskSrc ms = f.job0.src;
     ms.resolve();
-    tile_dsd_body<T, true, false, S>(g, tiles_m, tiles_n, Mb, Kb, bid, nsplit, &ms);
+    tile_dsd_body<T, true, false, S, TABLED>(g, tiles_m, tiles_n, Mb, Kb, bid, nsplit, &ms);
   } else {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     static_assert(flat_lds(kTableEntriesMost) <= S::SMEM_STEPS, "the table lies where the stages would");
-    flat_lists_block<S::THREADS, true>(f, bid - n_gemm, smem);
+    flat_lists_block<S::THREADS, TABLED>(f, bid - n_gemm, smem);
   }
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }
@@ -106,16 +106,21 @@ int dsd_launch(const GemmArgs& g, int splits, hipStream_t stream) {
   return check_launch("tile_dsd_kernel");
 }
 
-template <typename T, typename S>
-int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
+template <typename T, typename S, bool TABLED>
+int forward_launch_t(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
   static std::atomic<bool> done[64] = {};
-  auto* kernel = &tile_forward_kernel<T, S>;
+  auto* kernel = &tile_forward_kernel<T, S, TABLED>;
   if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), S::SMEM, done)) return rc;
   const int Mb = blocks_of(g.M), Kb = blocks_of(g.K), tm = (Mb + S::R - 1) / S::R, tn = (blocks_of(g.N) + S::C - 1) / S::C;
   const int n_gemm = tm * tn * splits;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(n_gemm + f.blocks())), dim3(S::THREADS), S::smem_for(Kb), stream, g, tm, tn, Mb, Kb,
                      splits, n_gemm, f);
   return check_launch("tile_forward_kernel");
+}
+
+template <typename T, typename S>
+int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t stream) {
+  return f.tabled ? forward_launch_t<T, S, true>(g, splits, f, stream) : forward_launch_t<T, S, false>(g, splits, f, stream);
 }
 
 template <typename T, typename S>

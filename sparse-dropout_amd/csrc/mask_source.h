@@ -45,7 +45,7 @@ struct MaskSrc {
   int64_t st_row, st_col;
   int32_t split;
   int32_t merge;  // 1, or 2: four stored / drawn entries per listed entry
-  int32_t mb;     // rows of the stored / drawn mask (only read when merge == 2)
+  int32_t mb;     // rows of the stored / drawn mask
   int32_t kb;  // entries per row of the stored / drawn mask
   uint32_t seed_lo, seed_hi, off_lo, off_hi;
   float p;
@@ -168,11 +168,11 @@ __device__ __forceinline__ void write_mask(const MaskSrc& src, int64_t mb, uint8
 // THREADS * kFlatPer consecutive flat entries.  Blocks do not talk to each other: each first counts the kept
 // entries in front of its chunk itself (one sweep over at most 2^18 mask bytes, or draws), which replaces
 // the grid-wide scan and keeps the whole build in one launch with every load independent of the others.
-// A generator call costs a wave 600 clocks and more and yields four entries, so a block evaluates the entries of a mask of up to
-// 2^14 (2^17 in a product's launch) once, into a table of four to a byte in LDS, and counts and lists from there (a stored mask comes into the table
-// in loads that do not wait for each other).  With a call per entry and listing, and one per entry in
-// the product's workgroups (union_of_mask), 4096 x 4096 -> 4096 forward took 105 us with a drawn mask of 32-blocks, so 94;
-// 2048^3 with one of 64-blocks 25.6, so 24.5, 4096 x 1024 -> 1024 16.7 and 15.7.
+// A generator call costs a wave 600 clocks and more and yields four entries, so a block of a launch of its own evaluates the entries of
+// a mask of up to 2^14 once, into a table of four to a byte in LDS, and counts and lists from there (a stored mask comes into the
+// table in loads that do not wait for each other).  Drawn masks of 64 x 16, 128 x 128 and, of 32-blocks, 128 x 128 entries: 5.8 -> 4.7,
+// 12.0 -> 10.3 and 27.1 -> 10.3 us; stored ones 5.8 -> 5.0, 12.4 -> 11.7, 19.0 -> 11.7.  In a product's launch drawn masks of up to 2^17
+// entries are, where that pays (mask_table_pays in gemm_fast.hip).
 constexpr int64_t kTableEntries = 1 << 14, kTableEntriesMost = 1 << 17;  // in a launch of its own, and in a product's LDS
 constexpr int flat_lds(int64_t entries) { return 64 + (int)(entries / 4); }
 constexpr int kFlatPer = 4;  // consecutive entries per thread
@@ -183,6 +183,7 @@ constexpr int64_t kFlatMaxEntries = 1 << 18;
 struct FlatJobs {
   ListJob job0, job1;
   int32_t blocks0, blocks1, blocks_mask;
+  bool tabled;  // in a product's launch: the mask is evaluated through a table in LDS
   uint8_t* mask_out;
   int64_t mask_rows;
   __host__ __device__ inline int blocks() const { return blocks0 + blocks1 + blocks_mask; }
@@ -199,6 +200,7 @@ inline FlatJobs flat_jobs(const MaskSrc& src, int64_t mb, int64_t kb, int32_t* r
   f.blocks0 = row_ptr ? per_list : 0;
   f.blocks1 = col_ptr ? per_list : 0;
   f.blocks_mask = mask_out ? (int)ceil_div(mask_rows * src.kb, chunk) : 0;
+  f.tabled = false;
   f.mask_out = mask_out;
   f.mask_rows = mask_rows;
   return f;
@@ -354,11 +356,12 @@ __device__ __forceinline__ void flat_lists_block(const FlatJobs& f, int b, char*
 
 // ---- keep bits of a product's own rows -----------------------------------------------------------------------------------
 // scratch[k] |= the keep bits (four per row block) of row blocks rb0 .. rb0 + rows - 1 at reduction blocks kb_lo .. + Kb - 1.
-// Where a thread would make more than one generator call (the entries of a mask of 32-blocks take four each), the drawn entries
-// are evaluated four to a call into `table` first (LDS: union_table_bytes, apart from the scratch).
-// Fewer are as fast each by itself, without the barrier (1024 x 1024 -> 1024: 7.8 us, through the table 8.4).
+// TABLED (a drawn mask): where a thread would make more than one generator call (the entries of a mask of 32-blocks take four
+// each), the entries are evaluated four to a call into `table` first (LDS: union_table_bytes, apart from the scratch).
+// Fewer are as fast each by itself, without the barrier (1024 x 1024 -> 1024: 7.8 us, through the table 8.4).  (Stored masks do not
+// come here TABLED; without the question the compiler's code for the drawn ones is slower: 4096 x 1024 -> 1024 14.8 us and 15.2.)
 constexpr int union_table_bytes(int rows, int steps) { return (2 * rows + 1) * (steps / 2 + 2); }
-template <int THREADS>
+template <int THREADS, bool TABLED>
 __device__ __forceinline__ void union_of_mask(const MaskSrc& ms, int rb0, int rows, int kb_lo, int Kb, uint32_t* scratch, uint8_t* table, int tid) {
   auto gather = [&](auto at) __attribute__((always_inline)) {
     for (int i = tid; i < rows * Kb; i += THREADS) {
@@ -367,7 +370,7 @@ __device__ __forceinline__ void union_of_mask(const MaskSrc& ms, int rb0, int ro
       if (q) atomicOr(&scratch[k], q << (4 * r));
     }
   };
-  if (ms.mask || (ms.merge == 1 && rows * Kb <= THREADS)) {
+  if (!TABLED || ms.mask || (ms.merge == 1 && rows * Kb <= THREADS)) {
     gather(ms.one_by_one());
     return;
   }

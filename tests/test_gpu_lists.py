@@ -162,7 +162,9 @@ def test_merged_lists_of_odd_multiples_of_32_bit_exact(rows, cols, bs, p):
     (3000, 2088, 264, 96, True),     # three 32-blocks to an entry, ragged, rows of the mask that start inside a group of four
     (1056, 544, 4160, 32, True),     # 33 x 17 entries of 32-blocks
     (16400, 2048, 128, 32, True),    # 513 x 64 entries: more than the table of a list build of its own, which evaluates one by one
-    (16416, 8224, 72, 32, False),    # 513 x 257 entries: more than a product's launch evaluates
+    (4100, 20600, 1030, 64, True),   # a full round of workgroups: a mask of 64-blocks through the table, rows of more entries than threads
+    (4544, 416, 6344, 128, True),    # the same on the 256 x 256 shape or what takes its place, an entry to four blocks
+    (16416, 8224, 72, 32, True),     # 513 x 257 entries: more than the table in a product's launch
 ])
 def test_masks_evaluated_through_a_table(M, K, N, bs, merged):
     """Drawn and stored masks on both sides of the limits up to which a workgroup evaluates a mask four entries at a time into
