@@ -789,6 +789,48 @@ int64_t dw_splits(int64_t c, int64_t k, int64_t rs, int64_t rows) {
   return want < 1 ? 1 : (want < turns ? want : turns);
 }
 
+// ---- which convolutions: expected times of forward and both gradients, in microseconds -----------------------------------------
+// The tap-wise products do the dense number of operations whatever is dropped, and a small layer's time is the chain of one workgroup's
+// steps; on the other routes dropped blocks save work, and what they do not save is lists, patch matrix and fold.  Fitted to 644 layers
+// (8 to 256 images of 7 x 7 to 64 x 64, 16 to 1024 channels, 3 x 3 and 5 x 5, drop rates of 0 to 0.95, both element types, graph
+// replays), those whose two times lie near each other counting most: 6 % off the tap-wise times, 9 to 13 % off the others'.  By
+// these a layer takes 1.006 of its better route's time on average; 12 of the 644 take more than 1.02 of the route they would have had
+// without the tap-wise products, 1.17 at worst.  With all of them tap by tap it was 75, 64 x 1024 x 14 x 14 -> 1024 at p = 0.75
+// 1.68 of it (1090 against 649 us), 26 x 40 x 14 x 14 -> 184 with 5 x 5 at p = 0.05 1.51 (148 against 98).
+double expected_taps(const ConvShape& v) {
+  const double rows = (double)(v.n * v.po() * v.qo()), pixels = (double)(v.n * v.h * v.w);
+  const int64_t rs = v.r * v.s, turns = ceil_div((int64_t)rows, kPos);
+  const TapPacking pack((int)v.c, (int)v.k, (int)rs, false);
+  const double narrow_k = v.k > 32 ? 1.0 : 0.6, narrow_c = v.c > 32 ? 1.0 : 0.6;  // products of half the width
+  // steps of a workgroup, and rounds of workgroups behind the first on every CU
+  const double y_steps = pack.steps * narrow_k, dx_steps = (double)(rs * ceil_div(v.k, 64)) * narrow_k * narrow_c;
+  auto behind = [](double wgs) { return wgs > 256.0 ? wgs / 256.0 - 1.0 : 0.0; };
+  const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = dw_splits(v.c, v.k, rs, (int64_t)rows);
+  const double dw_turns = (double)(ceil_div(tiles * splits, 256) * ceil_div(turns, splits));
+  return 32.3 + y_steps * (0.73 + 0.314 * behind((double)(turns * pack.groups))) +
+         dx_steps * (0.85 + 0.803 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 3.0 * dw_turns +
+         2.76e-6 * (double)(splits * v.c * v.k * rs) + 0.73e-6 * pixels * (double)v.c + 1.68e-6 * rows * (double)v.k;
+}
+double expected_others(const ConvShape& v, double p) {
+  const double rows = (double)(v.n * v.po() * v.qo()), k = (double)v.k, cols = (double)(v.c * v.r * v.s), keep = 1.0 - p;
+  const double col_blocks = (double)ceil_div(v.c * v.r * v.s, 64), row_blocks = (double)ceil_div((int64_t)rows, 64);
+  const int64_t po = v.po(), qo = v.qo();
+  const bool implicit = 64 % qo == 0 && po * qo % 64 == 0 && v.w % 8 == 0;  // forward and weight gradient without a patch matrix
+  if (implicit && v.k % 64 == 0 && v.k <= 256 && cols <= 4096.0)            // the input gradient in one launch as well
+    return 43.7 + 2.49e-6 * rows * k + 76.3e-6 * cols * k + 3.07 * col_blocks * keep + 4.09e-3 * row_blocks * col_blocks +
+           6.21e-9 * rows * cols * k * keep;
+  // the fold reads its windows of the patch gradient with their halo, lower bands where little of a window fits its LDS
+  const int64_t halo_h = v.dil_h * (v.r - 1), window_w = v.w + v.dil_w * (v.s - 1);
+  int64_t band = 8;
+  while (band > 1 && ((band < v.h ? band : v.h) + halo_h) * window_w * (8 * v.r * v.s + 2) * 2 > 60 * 1024) band /= 2;
+  band = band < v.h ? band : v.h;
+  const double fold = rows * cols * (double)((band + halo_h) * window_w) / (double)(band * v.w);
+  if (implicit)
+    return 52.8 + 5.23e-9 * rows * cols * k * keep + 2.53e-6 * rows * k + 7.89e-6 * rows * (double)v.c + 1.88 * col_blocks * keep +
+           (0.346e-6 + 0.616e-6 * keep) * fold;
+  return 47.8 + (0.595e-6 + 3.89e-6 * keep) * rows * cols + 2.45e-6 * rows * k + 56.0e-6 * cols * k + 0.332e-6 * fold;
+}
+
 void set_packed(TapArgs& g, const void* packed, const TapPacking& pack) {
   g.pack = pack;
   g.packed = static_cast<const char*>(packed);
@@ -820,11 +862,9 @@ extern "C" int sd_conv2d_taps_taken(int64_t n, int64_t c, int64_t h, int64_t w, 
                                     int64_t dil_w, double p) {
   const ConvShape v = SD_CONV_SHAPE;
   if (!fits(v)) return 0;
-  // Below some 50 workgroups the chain of a workgroup's steps is all there is (17 + 22 + 15 us at 128 x 64 channels, 3 x 3, more with
-  // 5 x 5), which the routes that leave dropped blocks out meet or beat at high drop rates and in all cases under 16.  Over 180
-  // drawn layers of 8 to 256 images of 7 x 7 to 64 x 64 the pass takes 0.66 of what it took; with rows from 4096 on 0.4 to 1.15.
+  // (fewer positions, or between these two numbers a higher drop rate: not measured, and the other routes' as before)
   const int64_t rows = n * v.po() * v.qo();
-  return rows >= 12288 || (rows >= 4096 && p <= 0.5) ? 1 : 0;
+  return (rows >= 12288 || (rows >= 4096 && p <= 0.5)) && expected_taps(v) < expected_others(v, p) ? 1 : 0;
 }
 
 extern "C" int sd_conv2d_taps_forward(const void* x_rows, int64_t x_ld, const void* packed, void* y, int64_t y_ld,

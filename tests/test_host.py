@@ -312,6 +312,25 @@ def test_tap_windows_and_lds_hold_what_the_kernels_put_there(tmp_path):
     assert proc.returncode == 0, proc.stdout
 
 
+@pytest.mark.parametrize("layer,p,taken", [
+    ((128, 64, 32, 32, 128, 3), 0.5, True), ((256, 32, 28, 28, 64, 3), 0.25, True), ((64, 1024, 28, 28, 128, 3), 0.75, True),
+    ((64, 1024, 14, 14, 1024, 3), 0.75, False),  # 1090 us tap by tap, 649 with the dropped blocks left out
+    ((8, 256, 64, 64, 256, 3), 0.95, False),     # 204, 162
+    ((26, 40, 14, 14, 184, 5), 0.05, False),     # 20 workgroups, each a chain of 50 steps: 148, 98
+    ((16, 16, 32, 32, 208, 5), 0.75, False),     # 134, 94
+    ((97, 32, 7, 7, 144, 3), 0.25, False),       # 65, 49
+])
+def test_tap_by_tap_only_where_it_is_expected_to_be_faster(layer, p, taken):
+    """The rule that takes a convolution to the tap-wise products knows what they cost beside the routes that skip dropped blocks."""
+    from flash_dropout.hip import GEMM
+
+    n, c, h, w, k, r = layer
+    geo = (n, c, h, w, k, r, r, r // 2, r // 2, 1, 1, 1, 1)
+    lib = GEMM().lib
+    assert lib.sd_conv2d_taps_fits(*geo) == 1
+    assert lib.sd_conv2d_taps_taken(*geo, p) == int(taken)
+
+
 def test_loader_refuses_a_library_built_from_other_sources(monkeypatch):
     from flash_dropout.hip import _loader
 
