@@ -791,12 +791,12 @@ int64_t dw_splits(int64_t c, int64_t k, int64_t rs, int64_t rows) {
 
 // ---- which convolutions: expected times of forward and both gradients, in microseconds -----------------------------------------
 // The tap-wise products do the dense number of operations whatever is dropped, and a small layer's time is the chain of one workgroup's
-// steps; on the other routes dropped blocks save work, and what they do not save is lists, patch matrix and fold.  Fitted to 644 layers
+// steps; on the other routes dropped blocks save work, and what they do not save is lists, patch matrix and fold.  Fitted to 794 layers
 // (8 to 256 images of 7 x 7 to 64 x 64, 16 to 1024 channels, 3 x 3 and 5 x 5, drop rates of 0 to 0.95, both element types, graph
-// replays), those whose two times lie near each other counting most: 6 % off the tap-wise times, 9 to 13 % off the others'.  By
-// these a layer takes 1.006 of its better route's time on average; 12 of the 644 take more than 1.02 of the route they would have had
-// without the tap-wise products, 1.17 at worst.  With all of them tap by tap it was 75, 64 x 1024 x 14 x 14 -> 1024 at p = 0.75
-// 1.68 of it (1090 against 649 us), 26 x 40 x 14 x 14 -> 184 with 5 x 5 at p = 0.05 1.51 (148 against 98).
+// replays), those whose two times lie near each other counting most: 6 % off the tap-wise times, 6 to 10 % off the others'.  By
+// these a layer takes 1.005 of its better route's time on average and 1.20 at worst; 14 of the 794 take more than 1.02 of the route
+// they would have had without the tap-wise products, 1.17 at worst.  With all of them tap by tap it was 94, 64 x 1024 x 14 x 14
+// -> 1024 at p = 0.75 1.68 of it (1090 against 649 us), 26 x 40 x 14 x 14 -> 184 with 5 x 5 at p = 0.05 1.51 (148 against 98).
 double expected_taps(const ConvShape& v) {
   const double rows = (double)(v.n * v.po() * v.qo()), pixels = (double)(v.n * v.h * v.w);
   const int64_t rs = v.r * v.s, turns = ceil_div((int64_t)rows, kPos);
@@ -807,28 +807,36 @@ double expected_taps(const ConvShape& v) {
   auto behind = [](double wgs) { return wgs > 256.0 ? wgs / 256.0 - 1.0 : 0.0; };
   const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = dw_splits(v.c, v.k, rs, (int64_t)rows);
   const double dw_turns = (double)(ceil_div(tiles * splits, 256) * ceil_div(turns, splits));
-  return 32.3 + y_steps * (0.73 + 0.314 * behind((double)(turns * pack.groups))) +
-         dx_steps * (0.85 + 0.803 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 3.0 * dw_turns +
-         2.76e-6 * (double)(splits * v.c * v.k * rs) + 0.73e-6 * pixels * (double)v.c + 1.68e-6 * rows * (double)v.k;
+  return 32.7 + y_steps * (0.746 + 0.269 * behind((double)(turns * pack.groups))) +
+         dx_steps * (0.826 + 0.813 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 2.97 * dw_turns +
+         2.68e-6 * (double)(splits * v.c * v.k * rs) + 0.83e-6 * pixels * (double)v.c + 1.76e-6 * rows * (double)v.k;
 }
+// The other routes: the start; per million elements of the patch matrix, and of its kept blocks; per million of y, of x and of w; per
+// thousand million products of kept elements; per million elements that the fold of the patch gradient reads, and that
+// are kept; a step of a row block's chain over the kept column blocks; per thousand blocks listed.
+struct OtherCost {
+  double start, patch, patch_kept, y, x, w, product, fold, fold_kept, step, listed;
+};
+constexpr OtherCost kOtherCost[] = {{45.1, 0.687, 3.32, 2.63, 0., 44.3, 0., 0.339, 0., 1.13, 0.},   // through the patch matrix
+                                    {52.7, 0., 0., 2.83, 0., 0., 4.80, 0.798, 0.947, 2.04, 0.},     // without it, up to nine taps
+                                    {54.6, 0., 0., 4.80, 26.2, 0., 0., 0.197, 0.696, 1.79, 0.},     // and more
+                                    {44.7, 0., 0., 2.85, 0., 60.2, 6.83, 0., 0., 3.29, 3.74},       // and without a fold, up to nine
+                                    {92.2, 0., 0., 0., 22.9, 163., 0., 0., 0., 6.57, 0.}};          // and more
 double expected_others(const ConvShape& v, double p) {
-  const double rows = (double)(v.n * v.po() * v.qo()), k = (double)v.k, cols = (double)(v.c * v.r * v.s), keep = 1.0 - p;
-  const double col_blocks = (double)ceil_div(v.c * v.r * v.s, 64), row_blocks = (double)ceil_div((int64_t)rows, 64);
-  const int64_t po = v.po(), qo = v.qo();
-  const bool implicit = 64 % qo == 0 && po * qo % 64 == 0 && v.w % 8 == 0;  // forward and weight gradient without a patch matrix
-  if (implicit && v.k % 64 == 0 && v.k <= 256 && cols <= 4096.0)            // the input gradient in one launch as well
-    return 43.7 + 2.49e-6 * rows * k + 76.3e-6 * cols * k + 3.07 * col_blocks * keep + 4.09e-3 * row_blocks * col_blocks +
-           6.21e-9 * rows * cols * k * keep;
-  // the fold reads its windows of the patch gradient with their halo, lower bands where little of a window fits its LDS
+  const int64_t po = v.po(), qo = v.qo(), rs = v.r * v.s;
+  const double m = 1e-6, keep = 1.0 - p, rows = m * (double)(v.n * po * qo), k = (double)v.k, cols = (double)(v.c * rs);
+  const double col_blocks = (double)ceil_div(v.c * rs, 64);
+  const bool implicit = 64 % qo == 0 && po * qo % 64 == 0 && v.w % 8 == 0, fused = implicit && v.k % 64 == 0 && v.k <= 256 && cols <= 4096.0;
+  const OtherCost& o = kOtherCost[!implicit ? 0 : (fused ? 3 : 1) + (rs > 9 ? 1 : 0)];
+  // the fold reads windows with their halo, of lower bands where little of a window fits its LDS
   const int64_t halo_h = v.dil_h * (v.r - 1), window_w = v.w + v.dil_w * (v.s - 1);
   int64_t band = 8;
-  while (band > 1 && ((band < v.h ? band : v.h) + halo_h) * window_w * (8 * v.r * v.s + 2) * 2 > 60 * 1024) band /= 2;
+  while (band > 1 && ((band < v.h ? band : v.h) + halo_h) * window_w * (8 * rs + 2) * 2 > 60 * 1024) band /= 2;
   band = band < v.h ? band : v.h;
   const double fold = rows * cols * (double)((band + halo_h) * window_w) / (double)(band * v.w);
-  if (implicit)
-    return 52.8 + 5.23e-9 * rows * cols * k * keep + 2.53e-6 * rows * k + 7.89e-6 * rows * (double)v.c + 1.88 * col_blocks * keep +
-           (0.346e-6 + 0.616e-6 * keep) * fold;
-  return 47.8 + (0.595e-6 + 3.89e-6 * keep) * rows * cols + 2.45e-6 * rows * k + 56.0e-6 * cols * k + 0.332e-6 * fold;
+  return o.start + (o.patch + o.patch_kept * keep) * rows * cols + o.y * rows * k + o.x * rows * (double)v.c + o.w * m * cols * k +
+         o.product * 1e-3 * rows * cols * k * keep + (o.fold + o.fold_kept * keep) * fold + o.step * col_blocks * keep +
+         o.listed * 1e3 * rows / 64. * col_blocks;
 }
 
 void set_packed(TapArgs& g, const void* packed, const TapPacking& pack) {
