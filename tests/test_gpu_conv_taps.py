@@ -143,6 +143,36 @@ def test_layers_tap_by_tap(geom, channels_last, keeps_image, drawn):
         assert all(torch.equal(a, b) for a, b in zip(again, grads))
 
 
+@pytest.mark.parametrize("sliced", ["channels", "channels off 16 bytes", "channels at an odd distance", "pixels", "planes"])
+def test_slices_tap_by_tap(sliced):
+    """Images and gradients that are slices: their own rows, copied once, or turned, they give the same bits as whole ones."""
+    import flash_dropout.functional as F
+
+    geom = (20, 32, 16, 16, 40, 3, 3, (1, 1), (1, 1))
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, torch.float16)
+
+    def slice_of(t):
+        b, ch, p, q = t.shape
+        cl = dict(memory_format=torch.channels_last)
+        wide, at = {"channels": ((b, 2 * ch, p, q), (0, ch, 0, 0)), "channels off 16 bytes": ((b, 2 * ch, p, q), (0, 4, 0, 0)),
+                    "channels at an odd distance": ((b, ch + 4, p, q), (0, 0, 0, 0)), "pixels": ((b, ch, p + 2, q + 3), (0, 0, 1, 2)),
+                    "planes": ((b, ch, p + 2, q + 3), (0, 0, 1, 2))}[sliced]
+        big = torch.randn(wide, dtype=t.dtype, device="cuda")
+        big = big.contiguous(**({} if sliced == "planes" else cl))
+        view = big[tuple(slice(o, o + e) for o, e in zip(at, t.shape))]
+        return view.copy_(t)
+
+    def products(xg, dyg):
+        xg, wg = xg.detach().requires_grad_(), wt.cuda().requires_grad_()
+        y = F.blockwise_dropout_conv2d(xg, wg, 64, 0.4, pad, seed=5)
+        return (y, *torch.autograd.grad(y, (xg, wg), dyg))
+
+    whole = products(x.cuda(), dy.cuda())
+    for xg, dyg in ((slice_of(x), dy.cuda()), (x.cuda(), slice_of(dy)), (slice_of(x), slice_of(dy))):
+        assert all(torch.equal(a, b) for a, b in zip(products(xg, dyg), whole))
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_what_a_mask_drops_reaches_nothing_tap_by_tap(bad):
     """An Inf or NaN in an operand reaches the results whose kept blocks read it, and no other."""
