@@ -143,6 +143,26 @@ def test_layers_tap_by_tap(geom, channels_last, keeps_image, drawn):
         assert all(torch.equal(a, b) for a, b in zip(again, grads))
 
 
+def test_rows_are_kept_for_the_kernel_gradient_only():
+    """Where the rows and not the image are what the kernel's gradient reads: a frozen kernel keeps neither, the image may change
+    before the backward as it may otherwise, and dX is the same."""
+    import flash_dropout.functional as F
+
+    geom = LAYERS[1][0]
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, torch.float16)
+    xg = x.cuda().contiguous(memory_format=torch.channels_last).requires_grad_()
+    wg = wt.cuda().requires_grad_()
+    both = torch.autograd.grad(F.blockwise_dropout_conv2d(xg, wg, 64, 0.4, pad, seed=5), (xg, wg), dy.cuda())
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+        y = F.blockwise_dropout_conv2d(xg, wg.detach(), 64, 0.4, pad, seed=5)
+    assert [q for q in kept if len(q) == 4 or q[0] >= 4096] == []
+    with torch.no_grad():
+        xg.mul_(2)
+    assert torch.equal(torch.autograd.grad(y, xg, dy.cuda())[0], both[0])
+
+
 @pytest.mark.parametrize("sliced", ["channels", "channels off 16 bytes", "channels at an odd distance", "pixels", "planes"])
 def test_slices_tap_by_tap(sliced):
     """Images and gradients that are slices: their own rows, copied once, or turned, they give the same bits as whole ones."""
