@@ -31,6 +31,10 @@ GEOMS = [
     (40, 64, 8, 11, 64, 1, 9, (0, 0), (1, 1)),
     (30, 72, 5, 11, 40, 1, 3, (0, 0), (1, 4)),
     (20, 40, 6, 15, 72, 1, 12, (0, 0), (1, 1)),
+    # windows of 784, 912 and 992 rows (1000 are the most): the weight gradient has LDS for one buffer of them
+    (1, 32, 9, 256, 40, 3, 3, (1, 1), (1, 1)),
+    (1, 40, 8, 160, 64, 5, 5, (2, 2), (1, 1)),
+    (1, 24, 7, 360, 72, 3, 3, (1, 1), (1, 1)),
 ]
 
 
