@@ -510,7 +510,7 @@ int sd_conv2d_dw_lists(const void* x, int64_t x_stride_n, int64_t x_stride_c, in
  * sd_conv2d_taps_fits: whether the kernels take the geometry (1) or not (0): strides 1, 2 <= R*S <= 32, channels and outputs
  * multiples of 8, and the rows that 256 consecutive positions touch within a CU's LDS.  The calls below return
  * SD_ERR_UNSUPPORTED, with nothing launched, for every other.  sd_conv2d_taps_taken: whether they are also expected to be faster than
- * the other routes at drop rate p.
+ * the other routes at drop rate p, with a mask in blocks of 64 (.._blocks: of block_size; 0: no mask).
  *
  * sd_conv2d_taps_prepare: what a direction needs beforehand, each part left out when its pointer is NULL, in one launch:
  * up to two sets of planes [n][channels][pixels] (strides sn, sc, unit along the pixels) as rows [n * pixels, channels]; the weights
@@ -521,6 +521,9 @@ int sd_conv2d_taps_fits(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_ou
                         int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w);
 int sd_conv2d_taps_taken(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h,
                          int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, double p);
+int sd_conv2d_taps_taken_blocks(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s, int64_t pad_h,
+                                int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, double p,
+                                int64_t block_size);
 int64_t sd_conv2d_taps_packed_bytes(int64_t c, int64_t k_out, int64_t r, int64_t s, int backward);
 int sd_conv2d_taps_prepare(int count, const void* const* planes, const int64_t* sn, const int64_t* sc, void* const* rows,
                            const int64_t* n, const int64_t* channels, const int64_t* pixels, const void* weight, int64_t weight_ld, int64_t c, int64_t k_out, int64_t r, int64_t s, int backward,

@@ -791,12 +791,13 @@ int64_t dw_splits(int64_t c, int64_t k, int64_t rs, int64_t rows) {
 
 // ---- which convolutions: expected times of forward and both gradients, in microseconds -----------------------------------------
 // The tap-wise products do the dense number of operations whatever is dropped, and a small layer's time is the chain of one workgroup's
-// steps; on the other routes dropped blocks save work, and what they do not save is lists, patch matrix and fold.  Fitted to 794 layers
-// (8 to 256 images of 7 x 7 to 64 x 64, 16 to 1024 channels, 3 x 3 and 5 x 5, drop rates of 0 to 0.95, both element types, graph
-// replays), those whose two times lie near each other counting most: 6 % off the tap-wise times, 6 to 10 % off the others'.  By
-// these a layer takes 1.005 of its better route's time on average and 1.20 at worst; 14 of the 794 take more than 1.02 of the route
-// they would have had without the tap-wise products, 1.17 at worst.  With all of them tap by tap it was 94, 64 x 1024 x 14 x 14
-// -> 1024 at p = 0.75 1.68 of it (1090 against 649 us), 26 x 40 x 14 x 14 -> 184 with 5 x 5 at p = 0.05 1.51 (148 against 98).
+// steps; on the other routes dropped blocks save work, and what they do not save is lists, patch matrix and fold.  Fitted to 944 layers
+// (8 to 256 images of 7 x 7 to 64 x 64, 16 to 1024 channels, 3 x 3 and 5 x 5, drop rates of 0 to 0.95, blocks of 64 and 128, both
+// element types, graph replays), those whose two times lie near each other counting most: 6 % off the tap-wise times, 6 to 10 %
+// off the others'.  Layers within 3 % go tap by tap.  So a layer takes 1.004 of its better route's time on average; 21 of the 944 take
+// more than 1.02 of the route they would have had without the tap-wise products, 1.17 at worst, and 17 more than 1.02 of the tap-wise
+// one.  With all of them tap by tap it was 106, 64 x 1024 x 14 x 14 -> 1024 at p = 0.75 1.68 of it (1090 against 649 us),
+// 26 x 40 x 14 x 14 -> 184 with 5 x 5 at p = 0.05 1.51 (148 against 98).
 double expected_taps(const ConvShape& v) {
   const double rows = (double)(v.n * v.po() * v.qo()), pixels = (double)(v.n * v.h * v.w);
   const int64_t rs = v.r * v.s, turns = ceil_div((int64_t)rows, kPos);
@@ -807,22 +808,23 @@ double expected_taps(const ConvShape& v) {
   auto behind = [](double wgs) { return wgs > 256.0 ? wgs / 256.0 - 1.0 : 0.0; };
   const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = dw_splits(v.c, v.k, rs, (int64_t)rows);
   const double dw_turns = (double)(ceil_div(tiles * splits, 256) * ceil_div(turns, splits));
-  return 32.7 + y_steps * (0.746 + 0.269 * behind((double)(turns * pack.groups))) +
-         dx_steps * (0.826 + 0.813 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 2.97 * dw_turns +
-         2.68e-6 * (double)(splits * v.c * v.k * rs) + 0.83e-6 * pixels * (double)v.c + 1.76e-6 * rows * (double)v.k;
+  return 32.7 + y_steps * (0.751 + 0.281 * behind((double)(turns * pack.groups))) +
+         dx_steps * (0.849 + 0.864 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 2.8 * dw_turns +
+         2.62e-6 * (double)(splits * v.c * v.k * rs) + 0.98e-6 * pixels * (double)v.c + 1.71e-6 * rows * (double)v.k;
 }
 // The other routes: the start; per million elements of the patch matrix, and of its kept blocks; per million of y, of x and of w; per
 // thousand million products of kept elements; per million elements that the fold of the patch gradient reads, and that
-// are kept; a step of a row block's chain over the kept column blocks; per thousand blocks listed.
+// are kept; a step of a row block's chain over the kept column blocks.  Masks of larger blocks besides: their spreading over
+// 64-blocks, and per thousand of these.
 struct OtherCost {
-  double start, patch, patch_kept, y, x, w, product, fold, fold_kept, step, listed;
+  double start, patch, patch_kept, y, x, w, product, fold, fold_kept, step, larger, larger_listed;
 };
-constexpr OtherCost kOtherCost[] = {{45.1, 0.687, 3.32, 2.63, 0., 44.3, 0., 0.339, 0., 1.13, 0.},   // through the patch matrix
-                                    {52.7, 0., 0., 2.83, 0., 0., 4.80, 0.798, 0.947, 2.04, 0.},     // without it, up to nine taps
-                                    {54.6, 0., 0., 4.80, 26.2, 0., 0., 0.197, 0.696, 1.79, 0.},     // and more
-                                    {44.7, 0., 0., 2.85, 0., 60.2, 6.83, 0., 0., 3.29, 3.74},       // and without a fold, up to nine
-                                    {92.2, 0., 0., 0., 22.9, 163., 0., 0., 0., 6.57, 0.}};          // and more
-double expected_others(const ConvShape& v, double p) {
+constexpr OtherCost kOtherCost[] = {{43.7, 0.711, 3.09, 2.65, 0., 44.8, 0., 0.340, 0., 1.28, 0., 2.18},      // through the patch matrix
+                                    {50.9, 0., 0., 2.73, 0., 0., 5.27, 0.814, 0.852, 1.98, 11.6, 0.},        // without it, up to nine taps
+                                    {51.9, 0., 0., 4.71, 32.9, 0., 0., 0.171, 0.407, 2.02, 22.1, 0.},        // and more
+                                    {44.4, 0.904, 0., 2.90, 0., 62.2, 6.80, 0., 0., 3.32, 13.7, 0.},         // and without a fold, up to nine
+                                    {90.4, 0.724, 0., 0., 0., 187., 0., 0., 0., 7.07, 0., 0.}};              // and more
+double expected_others(const ConvShape& v, double p, int64_t block_size) {
   const int64_t po = v.po(), qo = v.qo(), rs = v.r * v.s;
   const double m = 1e-6, keep = 1.0 - p, rows = m * (double)(v.n * po * qo), k = (double)v.k, cols = (double)(v.c * rs);
   const double col_blocks = (double)ceil_div(v.c * rs, 64);
@@ -836,7 +838,7 @@ double expected_others(const ConvShape& v, double p) {
   const double fold = rows * cols * (double)((band + halo_h) * window_w) / (double)(band * v.w);
   return o.start + (o.patch + o.patch_kept * keep) * rows * cols + o.y * rows * k + o.x * rows * (double)v.c + o.w * m * cols * k +
          o.product * 1e-3 * rows * cols * k * keep + (o.fold + o.fold_kept * keep) * fold + o.step * col_blocks * keep +
-         o.listed * 1e3 * rows / 64. * col_blocks;
+         (block_size > 64 ? o.larger + o.larger_listed * 1e3 * rows / 64. * col_blocks : 0.);
 }
 
 void set_packed(TapArgs& g, const void* packed, const TapPacking& pack) {
@@ -865,14 +867,20 @@ extern "C" int sd_conv2d_taps_fits(int64_t n, int64_t c, int64_t h, int64_t w, i
   return fits(SD_CONV_SHAPE) ? 1 : 0;
 }
 
-extern "C" int sd_conv2d_taps_taken(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
-                                    int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h,
-                                    int64_t dil_w, double p) {
+extern "C" int sd_conv2d_taps_taken_blocks(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                                           int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h,
+                                           int64_t dil_w, double p, int64_t block_size) {
   const ConvShape v = SD_CONV_SHAPE;
   if (!fits(v)) return 0;
   // (fewer positions, or between these two numbers a higher drop rate: not measured, and the other routes' as before)
   const int64_t rows = n * v.po() * v.qo();
-  return (rows >= 12288 || (rows >= 4096 && p <= 0.5)) && expected_taps(v) < expected_others(v, p) ? 1 : 0;
+  return (rows >= 12288 || (rows >= 4096 && p <= 0.5)) && expected_taps(v) < 1.03 * expected_others(v, p, block_size) ? 1 : 0;
+}
+
+extern "C" int sd_conv2d_taps_taken(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                                    int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h,
+                                    int64_t dil_w, double p) {
+  return sd_conv2d_taps_taken_blocks(n, c, h, w, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, p, 64);
 }
 
 extern "C" int sd_conv2d_taps_forward(const void* x_rows, int64_t x_ld, const void* packed, void* y, int64_t y_ld,

@@ -973,7 +973,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   Lists lists;
   Tensor y, y2, cols;
   const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;
-  const bool taps = implicit_forward && fused_dx && sd_conv2d_taps_taken(GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), bs ? p : 0.0);
+  const bool taps = implicit_forward && fused_dx && sd_conv2d_taps_taken_blocks(GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), bs ? p : 0.0, bs);
   const bool record = records(std::array<Tensor, 2>{x, kernel});
   bool keeps_input = true;
   if (taps) {

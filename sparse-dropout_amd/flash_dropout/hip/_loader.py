@@ -90,6 +90,7 @@ SIGNATURES = {
                                    c_void_p, c_void_p, c_int64, c_float, c_int, c_void_p, c_int64, c_void_p]),
     "sd_conv2d_taps_fits": (c_int, [c_int64] * 13),
     "sd_conv2d_taps_taken": (c_int, [*([c_int64] * 13), c_double]),
+    "sd_conv2d_taps_taken_blocks": (c_int, [*([c_int64] * 13), c_double, c_int64]),
     "sd_conv2d_taps_packed_bytes": (c_int64, [*([c_int64] * 4), c_int]),
     "sd_conv2d_implicit_taken": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, *([c_int64] * 14)]),
     "sd_conv2d_taps_prepare": (c_int, [c_int, *([c_void_p] * 7), c_void_p, *([c_int64] * 5),
