@@ -133,6 +133,14 @@ struct GemmArgs {
   int64_t aux_sr, aux_sc;
 };
 
+// SDD: the fraction of blocks expected to be kept (unknown counts as everything), and of the 64-blocks: one of a mask of
+// 32-blocks is kept with any of its quadrants.
+inline double kept_fraction(const GemmArgs& g) { return g.row_ptr && g.keep_hint >= 0.f && g.keep_hint <= 1.f ? (double)g.keep_hint : 1.0; }
+inline double kept_blocks(const GemmArgs& g) {
+  const double hint = kept_fraction(g), none = 1.0 - hint;
+  return g.quads ? 1.0 - none * none * none * none : hint;
+}
+
 // Geometry of a convolution whose patch matrix the DSD kernel gathers itself (implicit GEMM):
 // x[n][c][h][w] with unit w stride, row block = 64 / Q whole output rows of one image.
 struct ImplicitConv {

@@ -978,14 +978,13 @@ __global__ __launch_bounds__(S::THREADS) void forward_lists_kernel(GemmArgs g, i
 // (b.sr == 1); C row-major.  Mb x Cb is the block grid of the output (and of the mask); without a list
 // every tile is kept (the dense product in this operand layout).
 // With half of the tiles dropped a fixed 4x4 patch of tiles would still need nearly all of its 4 + 4 operand
-// tiles per reduction step for about 8 kept tiles.  Here a workgroup owns 4 row blocks x a GROUP of consecutive
-// column blocks, chosen greedily along the row so that it has at most GW column blocks with anything
-// kept and at most 16 kept tiles: 4 + 6 operand tiles per step for about 12 kept tiles at p = 0.5, the
-// same 4 + 4 for 16 as the patch kernel at p = 0.  Column blocks with nothing kept in these 4 rows
-// cost nothing (zeros are stored for them).  Group boundaries depend on the mask, so a workgroup is launched for
-// (window of 4 * GW column blocks, index of the group inside it), scans the quad's keep flags of that window and
-// takes the group with its index (the grid has the worst case number of groups per window; surplus workgroups
-// exit).  Groups never straddle a window, so the workgroups of different row quads stay on the same W tiles.
+// tiles per reduction step for about 8 kept tiles.  Here a workgroup owns 4 row blocks x a GROUP of column blocks with
+// anything kept, dealt out evenly along the row (deal_group): at most 6 column blocks and 8 waves of up to two tiles, 4 + 5 or 6
+// operand tiles per step for about 12 kept tiles at p = 0.5, the same 4 + 4 for 16 as the patch kernel at p = 0.  Column blocks
+// with nothing kept in these 4 rows cost nothing (zeros are stored for them).  Groups depend on the mask, so a workgroup is
+// launched for an index, scans the quad's keep flags and takes the group with that index (the grid has the most groups a row can
+// have; surplus workgroups exit).  The groups of a row of any length cover the same stretch of it, give or take a few column
+// blocks, in every row quad with as many of them, so the workgroups of different quads stay on the same W tiles.
 // A wave owns up to two WHOLE kept tiles (tile t of the group goes to wave t%8, so the two waves of a
 // SIMD always carry equal work +-1): 2x2 MFMAs per 16-wide step from 2 + 2 fragments, accumulators
 // statically indexed by the wave's slot, operand tiles addressed dynamically.
@@ -1003,124 +1002,223 @@ struct SddShape {
   // two stages; at least the eight 64 x 68 fp32 staging tiles of the epilogue
   static constexpr int SMEM = NST * STAGE > 8 * BS * (BS + 4) * 4 ? NST * STAGE : 8 * BS * (BS + 4) * 4;
   static constexpr int MINCOLS = GW < MAXT / R ? GW : MAXT / R;  // column blocks a group is sure to cover
-  // Groups never straddle a multiple of WINDOW column blocks, and a workgroup is launched for (window, group in
-  // the window): whatever the masks of two row quads, their workgroups of one window need the same W tiles
-  // (measured 1-6 % faster than groups that run freely along the row).
-  static constexpr int WINDOW = 4 * GW;
-  static constexpr int GPW = WINDOW / MINCOLS;  // groups a whole window can have at most
 };
 using SddBig = SddShape<4, 6, 2>;
 constexpr int G_MAX_CB = 8192;             // per-column flags share the first stage (of either shape) before the loads start
+
+// How many groups deal_group makes of a row quad with C column blocks with anything kept, n2 of them with two waves.
+__device__ inline int groups_of(int C, int n2) { return max(max((C + 5) / 6, (C + n2 + 7) / 8), 1); }
+
+// The columns of one group.  Which column blocks a row quad's workgroups take decides how many rounds of workgroups the product
+// has, and one round more is a third of a launch of three (8192^3 at p = 0.5: groups cut greedily along the row, none across a
+// multiple of 24 column blocks, were 97 to 100 an XCD for its 32 CUs, which took four rounds; dealt out they are 83 to 86).  So a
+// row is dealt out to as few groups as hold it: a column block with three or four kept tiles takes two waves, one with fewer a
+// wave, a group has 6 column blocks and 8 waves, and with C column blocks, n2 of them with two waves, C / 6 and (C + n2) / 8,
+// rounded up, are enough.  Either kind is cut into even consecutive runs; the groups with one of n2 more than others are the
+// first, those with one of C more the last (or the first too where all have two waves), which keeps every group within both
+// limits: waves are column blocks plus those with two, and where one group had one more of both than the least the average is
+// above least + 1, so that least + 2 is within the limit.
+// Called by one whole wave; flags: keep bits (0 - 3) of the quad's column blocks.  Writes the group's column blocks to cols, those
+// with two waves first, and its even share of the column blocks with nothing kept to empty; counts in n[0] and n[1], n[0] = -1
+// when the row has no such group (group 0 always exists: it may have nothing but empty column blocks).
+__device__ inline void deal_group(const uint32_t* flags, int Cb, int want, int lane, int* cols, int* empty, int* n) {
+  const uint64_t below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+  auto kept_of = [&](int c) { return c < Cb ? __builtin_popcount(flags[c] & 0xfu) : -1; };
+  int C = 0, n2 = 0;
+  for (int c0 = 0; c0 < Cb; c0 += 64) {
+    const int k = kept_of(c0 + lane);
+    C += __popcll(__ballot(k > 0));
+    n2 += __popcll(__ballot(k > 2));
+  }
+  const int G = groups_of(C, n2);
+  if (want >= G) {
+    if (lane == 0) n[0] = -1;
+    return;
+  }
+  const int least2 = n2 / G, more2 = n2 % G, least = C / G, more = C % G;
+  const bool both_first = least == least2;
+  const int two_n = least2 + (want < more2 ? 1 : 0), two_lo = least2 * want + min(want, more2);
+  const int all_n = least + (both_first ? (want < more ? 1 : 0) : (want >= G - more ? 1 : 0));
+  const int one_n = all_n - two_n, one_lo = least * want + (both_first ? min(want, more) : max(want - (G - more), 0)) - two_lo;
+  const int none_lo = (int)((int64_t)(Cb - C) * want / G), none_n = (int)((int64_t)(Cb - C) * (want + 1) / G) - none_lo;
+  int at2 = 0, at1 = 0, at0 = 0;
+  for (int c0 = 0; c0 < Cb; c0 += 64) {
+    const int k = kept_of(c0 + lane);
+    const uint64_t b2 = __ballot(k > 2), b1 = __ballot(k == 1 || k == 2), b0 = __ballot(k == 0);
+    const int i2 = at2 + __popcll(b2 & below) - two_lo, i1 = at1 + __popcll(b1 & below) - one_lo, i0 = at0 + __popcll(b0 & below) - none_lo;
+    if (k > 2 && i2 >= 0 && i2 < two_n) cols[i2] = c0 + lane;
+    if ((k == 1 || k == 2) && i1 >= 0 && i1 < one_n) cols[two_n + i1] = c0 + lane;
+    if (k == 0 && i0 >= 0 && i0 < none_n) empty[i0] = c0 + lane;
+    at2 += __popcll(b2);
+    at1 += __popcll(b1);
+    at0 += __popcll(b0);
+  }
+  if (lane == 0) {
+    n[0] = all_n;
+    n[1] = none_n;
+  }
+}
+
+// What a workgroup of the big SDD shape starts with: the row quad and the group it was launched for, the keep flags of the quad's
+// column blocks (bit r: tile (row block rb0 + r, column block c) kept; bits 8 + 4r .. 11 + 4r: which of its four 32 x 32 quadrants, all
+// of them unless the mask has block size 32) and the group's column blocks.
+// gsure > 0: the launch index says which group (group_of_block).  gsure == 0: every workgroup lists the flags of the whole mask and
+// counts the groups of all quads, and the launch index is the position among the groups there are, an eighth of them to an XCD, four
+// quads walked together.  The hardware deals workgroups out over the 8 XCDs and an XCD's 4 shader engines in turn, whether they
+// find a group or not, and an engine's 8 CUs that get a 17th or 25th group take a third or fourth round: 8192^3 at p = 0.75, 477
+// groups for 256 CUs, took three rounds.  It costs 4 to 5 us a workgroup (sdd_counts_all).
+struct GroupAt {
+  int tm, ncols, nempty;  // ncols < 0: no group for this workgroup
+  const uint32_t* flags;
+  const int *cols, *empty;
+};
+constexpr int kCountedQuads = 256;      // most row quads a workgroup counts the groups of
+constexpr int kCountedBlocks = 1 << 15; // most blocks of a mask it lists for that
+__device__ inline GroupAt find_group(const GemmArgs& g, char* smem, int tiles_m, int gsure, int Mb, int Cb, int bid, int tid, int wave, int lane) {
+  GroupAt at;
+  int gi = 0;
+  at.tm = 0;
+  const bool count = gsure == 0;
+  if (!count) group_of_block<SDD_GROUP_M>(bid, tiles_m, gsure, at.tm, gi);
+  const int quad0 = at.tm, quads = count ? tiles_m : 1, rows = min(4 * quads, Mb - 4 * quad0);
+  uint32_t* flags = reinterpret_cast<uint32_t*>(smem);
+  int* groups = reinterpret_cast<int*>(flags + ((quads * Cb + 3) & ~3));
+  int* rec = groups + (count ? kCountedQuads : 0);
+  int* empty = rec + 16;
+  const uint32_t init = g.row_ptr ? 0u : (((1u << rows) - 1u) | (((1u << (4 * rows)) - 1u) << 8));  // (without lists quads == 1)
+  for (int i = tid; i < quads * Cb; i += THREADS) flags[i] = init;
+  if (tid < 16) rec[tid] = 0;
+  __syncthreads();
+  if (g.row_ptr) {
+    const int per_row = max(THREADS / rows, 1);  // threads that share a row
+    for (int r = tid / per_row; r < rows; r += max(THREADS / per_row, 1)) {
+      if (tid >= per_row * (THREADS / per_row)) break;
+      const int beg = g.row_ptr[4 * quad0 + r], end = g.row_ptr[4 * quad0 + r + 1];
+      uint32_t* f = flags + (r / 4) * Cb;
+      for (int i = beg + tid % per_row; i < end; i += 8 * per_row) {
+        int32_t e[8];  // eight loads on their way at once
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = i + k * per_row < end ? g.col_idx[i + k * per_row] : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (i + k * per_row < end) atomicOr(&f[entry_block(e[k])], (1u << (r % 4)) | (entry_quads(e[k]) << (8 + 4 * (r % 4))));
+      }
+    }
+    __syncthreads();
+  }
+  if (count) {
+    for (int q = wave; q < tiles_m; q += THREADS / 64) {
+      int C = 0, n2 = 0;
+      for (int c0 = 0; c0 < Cb; c0 += 64) {
+        const int k = c0 + lane < Cb ? __builtin_popcount(flags[q * Cb + c0 + lane] & 0xfu) : 0;
+        C += __popcll(__ballot(k > 0));
+        n2 += __popcll(__ballot(k > 2));
+      }
+      if (lane == 0) groups[q] = groups_of(C, n2);
+    }
+    __syncthreads();
+    // Lane l has the four quads 4l .. 4l + 3, which are walked together.  Position `want` is in the set whose running total passes it.
+    static_assert(kCountedQuads == 4 * 64, "a lane has four quads");
+    int G[4], set = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      G[q] = 4 * lane + q < tiles_m ? groups[4 * lane + q] : 0;
+      set += G[q];
+    }
+    int upto = set;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int v = __shfl_up(upto, d);
+      if (lane >= d) upto += v;
+    }
+    const int total = __builtin_amdgcn_readlane(upto, 63);
+    if (bid >= total) {
+      at.ncols = -1;
+      return at;
+    }
+    const int want = xcd_run(bid, total);
+    const int s = __builtin_ctzll(__ballot(upto > want));
+    int left = want - (__builtin_amdgcn_readlane(upto, s) - __builtin_amdgcn_readlane(set, s));
+    int Gs[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) Gs[q] = __builtin_amdgcn_readlane(G[q], s);
+    // the groups of a set in order: index by index, the quads that have one of that index
+    for (;; ++gi) {
+      int have = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) have += Gs[q] > gi ? 1 : 0;
+      if (left < have) break;
+      left -= have;
+    }
+    int q_at = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (Gs[q] > gi) {
+        if (left == 0) q_at = q;
+        --left;
+      }
+    }
+    at.tm = 4 * s + q_at;
+    flags += at.tm * Cb;
+  }
+  if (wave == 0) deal_group(flags, Cb, gi, lane, rec + 4, empty, rec);
+  __syncthreads();
+  at.ncols = __builtin_amdgcn_readfirstlane(rec[0]);
+  at.nempty = __builtin_amdgcn_readfirstlane(rec[1]);
+  at.flags = flags;
+  at.cols = rec + 4;
+  at.empty = empty;
+  return at;
+}
+
+// Zeros for the tiles of a group that are not kept: those of its column blocks that the flags leave out and all of the empty ones.
+template <int R, bool EDGE>
+__device__ inline void zero_dropped(const GemmArgs& g, const uint32_t* flags, const int* cols, int ncols, const int* empty, int nempty,
+                                    int rb0, int Mb, int tid) {
+  const int row = tid / 8, ch = tid % 8;
+  const u32x4 z = {0u, 0u, 0u, 0u};
+  for (int i = 0; i < ncols + nempty; ++i) {
+    const int c = __builtin_amdgcn_readfirstlane(i < ncols ? cols[i] : empty[i - ncols]);
+    const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[c]);
+    for (int r = 0; r < R; ++r) {
+      if (rb0 + r >= Mb) break;
+      if (!((f >> r) & 1u) && (int64_t)(rb0 + r) * BS + row < g.M && (!EDGE || (int64_t)c * BS + ch * 8 < g.N))
+        *reinterpret_cast<u32x4*>(g.c + ((int64_t)(rb0 + r) * BS + row) * g.c_sr + (int64_t)c * BS + ch * 8) = z;
+    }
+  }
+}
 
 // EDGE = the output width or the reduction length is not a multiple of 64 (both multiples of 8): the
 // overhanging 16-byte chunks / rows of the last column block / reduction block are fetched from inside the
 // matrix instead, as in the DSD kernel, the fragments of the last reduction block are zeroed past the end,
 // and nothing is stored past the last column.  (A ragged M costs nothing worth a separate instance.)
 template <typename T, bool EDGE, typename G>
-__device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gmax, int Mb, int Cb, const int bid) {
+__device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gsure, int Mb, int Cb, const int bid) {
   constexpr int R = G::R, GW = G::GW, SLOTS = G::SLOTS, G_BOFF = G::BOFF, G_STAGE = G::STAGE;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  // bit r: tile (row block rb0 + r, column block c) kept; bits 8 + 4r .. 11 + 4r: which of its four 32 x 32
-  // quadrants (all of them unless the mask has block size 32)
   const uint32_t smem_a = lds_address(smem);
-  uint32_t* flags = reinterpret_cast<uint32_t*>(smem);
-  int* rec = reinterpret_cast<int*>(smem + 4 * ((Cb + 3) & ~3));  // c_lo, c_hi, ncols, kept bits, cols[GW]
-
-  int tm, gi;
-  tile_of_block<SDD_GROUP_M>(bid, tiles_m, gmax, tm, gi);
   const int tid = threadIdx.x;
   const int lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int rb0 = tm * R;
-
-  // ---- per-column keep flags of this row quad -------------------------------------------------------
-  {
-    const int rows = (rb0 + R <= Mb) ? R : Mb - rb0;
-    const uint32_t all = ((1u << rows) - 1u) | (((1u << (4 * rows)) - 1u) << 8);
-    const uint32_t init = g.row_ptr ? 0u : all;
-    for (int i = tid; i < Cb; i += THREADS) flags[i] = init;
-    if (tid < 32) rec[tid] = 0;
-  }
-  __syncthreads();
-  if (g.row_ptr) {
-    for (int r = 0; r < R; ++r) {
-      if (rb0 + r >= Mb) break;
-      const int beg = g.row_ptr[rb0 + r], end = g.row_ptr[rb0 + r + 1];
-      for (int i = beg + tid; i < end; i += THREADS) {
-        const int32_t e = g.col_idx[i];
-        atomicOr(&flags[entry_block(e)], (1u << r) | (entry_quads(e) << (8 + 4 * r)));
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- the group this workgroup was launched for ---------------------------------------------------------
-  if (wave == 0) {
-    // whole windows, the last one taking the remainder as well (so that the grid is as large as without windows)
-    const int nwin = Cb / G::WINDOW > 1 ? Cb / G::WINDOW : 1;
-    const int win = gi / G::GPW < nwin - 1 ? gi / G::GPW : nwin - 1, want = gi - win * G::GPW;
-    const int w_lo = win * G::WINDOW, w_hi = win == nwin - 1 ? Cb : w_lo + G::WINDOW;
-    int grp = 0, start = w_lo, width = 0, cnt = 0, lo = -1, hi = -1;
-    static_assert(2 * G::WINDOW <= 64, "a window's flags are read by one wave-wide load");
-    if (w_hi - w_lo <= 64) {
-      const uint32_t fv = (w_lo + lane < w_hi) ? flags[w_lo + lane] : 0u;
-      for (int i = 0; i < w_hi - w_lo; ++i) {
-        const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)fv, i) & 0xfu;
-        if (f == 0) continue;
-        const int a = __builtin_popcount(f);
-        if (width == GW || cnt + a > G::MAXT) {  // the group ends in front of this column block
-          if (grp == want) {
-            lo = start;
-            hi = w_lo + i;
-            break;
-          }
-          ++grp;
-          start = w_lo + i;
-          width = 0;
-          cnt = 0;
-        }
-        ++width;
-        cnt += a;
-      }
-      if (hi < 0 && grp == want) {  // the window's last group runs to its end
-        lo = start;
-        hi = w_hi;
-      }
-    }
-    int n = 0;
-    uint32_t kept = 0;  // bit 4*j + r
-    for (int c = lo; c < hi; ++c) {
-      const uint32_t fq = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[c]);
-      const uint32_t f = fq & 0xfu;
-      if (f) {
-        if (lane == 0) {
-          rec[4 + n] = c;
-          rec[16 + n] = (int)(fq >> 8);  // quadrant keep bits of the column block's tiles, four per row block
-        }
-        kept |= f << (4 * n);
-        ++n;
-      }
-    }
-    if (lane == 0) {
-      rec[0] = lo;
-      rec[1] = hi;
-      rec[2] = n;
-      rec[3] = (int)kept;
-    }
-  }
-  __syncthreads();
-  const int c_lo = __builtin_amdgcn_readfirstlane(rec[0]);
-  const int c_hi = __builtin_amdgcn_readfirstlane(rec[1]);
-  if (c_lo < 0) return;  // fewer groups in this row quad than the grid provides for
-  const int ncols = __builtin_amdgcn_readfirstlane(rec[2]);
-  const uint32_t kept = (uint32_t)__builtin_amdgcn_readfirstlane(rec[3]);
+  const GroupAt at = find_group(g, smem, tiles_m, gsure, Mb, Cb, bid, tid, wave, lane);
+  if (at.ncols < 0) return;  // fewer groups than the grid provides for
+  const int rb0 = at.tm * R, ncols = at.ncols;
+  const uint32_t* flags = at.flags;
   int cols[GW];
+  uint32_t kept = 0;  // bit 4*j + r
+  uint32_t col_q[GW];  // quadrant keep bits of the column block's tiles, four per row block
 #pragma unroll
-  for (int j = 0; j < GW; ++j) cols[j] = __builtin_amdgcn_readfirstlane(rec[4 + j]);
+  for (int j = 0; j < GW; ++j) {
+    cols[j] = __builtin_amdgcn_readfirstlane(at.cols[j]);
+    const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[cols[j]]);
+    kept |= j < ncols ? (f & 0xfu) << (4 * j) : 0u;
+    col_q[j] = f >> 8;
+  }
   const int ntiles = __builtin_popcount(kept);
 
   // this wave's tiles: tile t of the group (set bits of `kept` in order) belongs to wave t % 8
   int my_r[SLOTS], my_j[SLOTS], my_c[SLOTS];
+  uint32_t my_q[SLOTS];  // which quadrants of the wave's tiles are kept
   bool act[SLOTS];
 #pragma unroll
   for (int k = 0; k < SLOTS; ++k) {
@@ -1131,29 +1229,20 @@ __device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gma
     const int b = (act[k] && m) ? __builtin_ctz(m) : 0;
     my_j[k] = b / 4;
     my_r[k] = b % 4;
-    my_c[k] = __builtin_amdgcn_readfirstlane(rec[4 + my_j[k]]);
-  }
-  uint32_t my_q[SLOTS];  // which quadrants of the wave's tiles are kept
+    my_c[k] = 0;
+    my_q[k] = 0;
 #pragma unroll
-  for (int k = 0; k < SLOTS; ++k)
-    my_q[k] = ((uint32_t)__builtin_amdgcn_readfirstlane(rec[16 + my_j[k]]) >> (4 * my_r[k])) & 0xfu;
+    for (int j = 0; j < GW; ++j)
+      if (j == my_j[k]) {
+        my_c[k] = cols[j];
+        my_q[k] = (col_q[j] >> (4 * my_r[k])) & 0xfu;
+      }
+  }
   uint32_t rowmask = 0;
 #pragma unroll
   for (int j = 0; j < GW; ++j) rowmask |= (kept >> (4 * j)) & 0xfu;
 
-  // ---- zeros for the dropped tiles of the group's column range ----------------------------------------
-  if (!g.kept_only) {
-    const int row = tid / 8, ch = tid % 8;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int c = c_lo; c < c_hi; ++c) {
-      const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[c]);
-      for (int r = 0; r < R; ++r) {
-        if (rb0 + r >= Mb) break;
-        if (!((f >> r) & 1u) && (int64_t)(rb0 + r) * BS + row < g.M && (!EDGE || (int64_t)c * BS + ch * 8 < g.N))
-          *reinterpret_cast<u32x4*>(g.c + ((int64_t)(rb0 + r) * BS + row) * g.c_sr + (int64_t)c * BS + ch * 8) = z;
-      }
-    }
-  }
+  if (!g.kept_only) zero_dropped<R, EDGE>(g, flags, at.cols, ncols, at.empty, at.nempty, rb0, Mb, tid);
   if (kept == 0) return;
   __syncthreads();  // flags and rec are dead: the stages may be written
 
@@ -1362,148 +1451,66 @@ __device__ __forceinline__ void sdd_body(const GemmArgs& g, int tiles_m, int gma
 // block of the group and up to two of its kept tiles: the W fragments of the column (32 registers) serve both, the dY
 // fragments of its one or two row blocks take 32 each.  A column block with 3 or 4 kept tiles takes two waves, and all
 // waves of a column block are in one group of four (so that a W tile is read by one group only: the dY tiles are to
-// this kernel what the W tile is to the DSD kernel, and the W tiles what the X tiles are).  Groups of column blocks are
-// formed greedily along the row: a column block goes to the group of waves with more waves to spare, and the
-// workgroup's group ends in front of the column block that fits neither, or after 6 (the LDS holds 4 + 6 tiles per
-// stage).  Everything kept: 4 column blocks, 16 tiles, as before; at p = 0.5 about 6 column blocks and 12-13 tiles.
+// this kernel what the W tile is to the DSD kernel, and the W tiles what the X tiles are).  A column block goes to the group of
+// waves with more waves to spare, those of two waves first.  Everything kept: 4 column blocks, 16 tiles; at p = 0.5 about 6 column
+// blocks and 12 tiles (the LDS holds 4 + 6 tiles per stage).
 // Group 0 loads the dY tiles of the next step; group 1 its own W tiles of the next step and group 0's of the step
 // after next (the DSD kernel's reasoning, see there).  Measured and slower at every drop rate but 0.5 (where it gains
 // 1 %): letting a column block's two waves sit in different groups (13 instead of 10.5 tiles per group at p = 0.5)
 // with the W loads shared out evenly between the groups - what a step costs is the instructions of its memory
 // phase, and the fuller groups need more of them per wave.
 template <typename T>
-__device__ __forceinline__ void sdd_pp_body(const GemmArgs& g, int tiles_m, int gmax, int Mb, int Cb, const int bid) {
+__device__ __forceinline__ void sdd_pp_body(const GemmArgs& g, int tiles_m, int gsure, int Mb, int Cb, const int bid) {
   using G = SddBig;
   constexpr int R = G::R, GW = G::GW, G_BOFF = G::BOFF, G_STAGE = G::STAGE;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t smem_a = lds_address(smem);
-  // bit r: tile (row block rb0 + r, column block c) kept; bits 8 + 4r .. 11 + 4r: which of its four 32 x 32 quadrants
-  // (all of them unless the mask has block size 32)
-  uint32_t* flags = reinterpret_cast<uint32_t*>(smem);
-  int* rec = reinterpret_cast<int*>(smem + 4 * ((Cb + 3) & ~3));        // c_lo, c_hi, ncols, group-1 slots, cols[6], waves[8]
-
-  int tm, gi;
-  tile_of_block<SDD_GROUP_M>(bid, tiles_m, gmax, tm, gi);
   const int tid = threadIdx.x;
   const int lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int rb0 = tm * R;
-
-  // ---- per-column keep flags of this row quad -------------------------------------------------------
-  {
-    const int rows = (rb0 + R <= Mb) ? R : Mb - rb0;
-    const uint32_t init = g.row_ptr ? 0u : (((1u << rows) - 1u) | (((1u << (4 * rows)) - 1u) << 8));
-    for (int i = tid; i < Cb; i += THREADS) flags[i] = init;
-    if (tid < 32) rec[tid] = 0;
-  }
-  __syncthreads();
-  if (g.row_ptr) {
-    for (int r = 0; r < R; ++r) {
-      if (rb0 + r >= Mb) break;
-      const int beg = g.row_ptr[rb0 + r], end = g.row_ptr[rb0 + r + 1];
-      for (int i = beg + tid; i < end; i += THREADS) {
-        const int32_t e = g.col_idx[i];
-        atomicOr(&flags[entry_block(e)], (1u << r) | (entry_quads(e) << (8 + 4 * r)));
-      }
-    }
-    __syncthreads();
-  }
-
-  // ---- the group this workgroup was launched for: (window, index inside it), as in the other SDD kernel -----------
-  if (wave == 0) {
-    const int nwin = Cb / G::WINDOW > 1 ? Cb / G::WINDOW : 1;
-    const int win = gi / G::GPW < nwin - 1 ? gi / G::GPW : nwin - 1, want = gi - win * G::GPW;
-    const int w_lo = win * G::WINDOW, w_hi = win == nwin - 1 ? Cb : w_lo + G::WINDOW;
-    int lo = -1, hi = -1;
-    if (w_hi - w_lo <= 64) {
-      const uint32_t fv = (w_lo + lane < w_hi) ? flags[w_lo + lane] : 0u;
-      int grp = 0, start = w_lo, used0 = 0, used1 = 0, slots = 0;
-      for (int i = 0; i < w_hi - w_lo; ++i) {
-        const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)fv, i) & 0xfu;
-        if (f == 0) continue;
-        const int w = (__builtin_popcount(f) + 1) / 2;  // waves the column block takes
-        int gsel = used0 <= used1 ? 0 : 1;
-        if (4 - (gsel ? used1 : used0) < w) gsel ^= 1;
-        if (slots == GW || 4 - (gsel ? used1 : used0) < w) {  // the group ends in front of this column block
-          if (grp == want) {
-            lo = start;
-            hi = w_lo + i;
-            break;
-          }
-          ++grp;
-          start = w_lo + i;
-          used0 = used1 = slots = 0;
-          gsel = 0;
-        }
-        if (gsel) used1 += w; else used0 += w;
-        ++slots;
-      }
-      if (hi < 0 && grp == want) {  // the window's last group runs to its end
-        lo = start;
-        hi = w_hi;
-      }
-    }
-    // slots, groups and waves of the group's column blocks (the same choices again)
-    int n = 0, used0 = 0, used1 = 0;
-    uint32_t g1_slots = 0, rowmask = 0;
-    for (int c = lo; c < hi; ++c) {
-      const uint32_t fq = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[c]), f = fq & 0xfu;
-      if (!f) continue;
-      const int cnt = __builtin_popcount(f), w = (cnt + 1) / 2;
-      auto quads_of = [&](int r) { return (fq >> (8 + 4 * r)) & 0xfu; };
-      int gsel = used0 <= used1 ? 0 : 1;
-      if (4 - (gsel ? used1 : used0) < w) gsel ^= 1;
-      const int wv = 4 * gsel + (gsel ? used1 : used0);
-      uint32_t m = f;
-      const int r_a = __builtin_ctz(m); m &= m - 1u;
-      const int r_b = m ? __builtin_ctz(m) : 0; if (m) m &= m - 1u;
-      const int r_c = m ? __builtin_ctz(m) : 0; if (m) m &= m - 1u;
-      const int r_d = m ? __builtin_ctz(m) : 0;
-      if (lane == 0) {
-        rec[4 + n] = c;
-        rec[10 + wv] = n | (r_a << 4) | (r_b << 8) | ((cnt >= 2 ? 2 : 1) << 12) | (int)(quads_of(r_a) << 16) | (int)(quads_of(r_b) << 20);
-        if (w == 2) rec[10 + wv + 1] = n | (r_c << 4) | (r_d << 8) | ((cnt - 2) << 12) | (int)(quads_of(r_c) << 16) | (int)(quads_of(r_d) << 20);
-      }
-      if (gsel) { used1 += w; g1_slots |= 1u << n; } else used0 += w;
-      rowmask |= f;
-      ++n;
-    }
-    if (lane == 0) {
-      rec[0] = lo;
-      rec[1] = hi;
-      rec[2] = n;
-      rec[3] = (int)(g1_slots | (rowmask << 8));
-    }
-  }
-  __syncthreads();
-  const int c_lo = __builtin_amdgcn_readfirstlane(rec[0]);
-  const int c_hi = __builtin_amdgcn_readfirstlane(rec[1]);
-  if (c_lo < 0) return;  // fewer groups in this row quad than the grid provides for
-  const int ncols = __builtin_amdgcn_readfirstlane(rec[2]);
-  const uint32_t g1_slots = (uint32_t)__builtin_amdgcn_readfirstlane(rec[3]) & 0xffu;
-  const uint32_t rowmask = ((uint32_t)__builtin_amdgcn_readfirstlane(rec[3]) >> 8) & 0xfu;
+  const GroupAt at = find_group(g, smem, tiles_m, gsure, Mb, Cb, bid, tid, wave, lane);
+  if (at.ncols < 0) return;  // fewer groups than the grid provides for
+  const int rb0 = at.tm * R, ncols = at.ncols;
+  const uint32_t* flags = at.flags;
   int cols[GW];
+  int my_j = 0, my_c = 0, n_mine = 0, my_r[2] = {0, 0};
+  uint32_t my_q[2] = {0u, 0u};  // kept quadrants of the wave's tiles
+  uint32_t g1_slots = 0, rowmask = 0;
+  {
+    int used0 = 0, used1 = 0;
 #pragma unroll
-  for (int j = 0; j < GW; ++j) cols[j] = __builtin_amdgcn_readfirstlane(rec[4 + j]);
-  const uint32_t mine = (uint32_t)__builtin_amdgcn_readfirstlane(rec[10 + wave]);
-  const int my_j = (int)(mine & 0xfu), n_mine = (int)((mine >> 12) & 3u);
-  const int my_r[2] = {(int)((mine >> 4) & 0xfu), (int)((mine >> 8) & 0xfu)};
-  const uint32_t my_q[2] = {(mine >> 16) & 0xfu, (mine >> 20) & 0xfu};  // kept quadrants of the wave's tiles
-  const int my_c = __builtin_amdgcn_readfirstlane(rec[4 + my_j]);
-
-  // ---- zeros for the dropped tiles of the group's column range ----------------------------------------
-  if (!g.kept_only) {
-    const int row = tid / 8, ch = tid % 8;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int c = c_lo; c < c_hi; ++c) {
-      const uint32_t f = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[c]);
-      for (int r = 0; r < R; ++r) {
-        if (rb0 + r >= Mb) break;
-        if (!((f >> r) & 1u) && (int64_t)(rb0 + r) * BS + row < g.M)
-          *reinterpret_cast<u32x4*>(g.c + ((int64_t)(rb0 + r) * BS + row) * g.c_sr + (int64_t)c * BS + ch * 8) = z;
+    for (int j = 0; j < GW; ++j) {
+      cols[j] = __builtin_amdgcn_readfirstlane(at.cols[j]);
+      if (j >= ncols) continue;
+      const uint32_t fq = (uint32_t)__builtin_amdgcn_readfirstlane((int)flags[cols[j]]), f = fq & 0xfu;
+      const int cnt = __builtin_popcount(f), w = cnt > 2 ? 2 : 1;  // column blocks of two waves come first: two of them fill a half
+      const int half = used0 <= used1 ? 0 : 1, wv = 4 * half + (half ? used1 : used0);
+      if (half) {
+        used1 += w;
+        g1_slots |= 1u << j;
+      } else {
+        used0 += w;
+      }
+      rowmask |= f;
+      if (wave == wv || (w == 2 && wave == wv + 1)) {
+        uint32_t m = f;
+        if (wave != wv) {  // the second wave has the third kept tile and the fourth
+          m &= m - 1u;
+          m &= m - 1u;
+        }
+        my_j = j;
+        my_c = cols[j];
+        n_mine = __builtin_popcount(m) > 1 ? 2 : 1;
+        my_r[0] = __builtin_ctz(m);
+        m &= m - 1u;
+        my_r[1] = m ? __builtin_ctz(m) : 0;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) my_q[k] = (fq >> (8 + 4 * my_r[k])) & 0xfu;
       }
     }
   }
+
+  if (!g.kept_only) zero_dropped<R, false>(g, flags, at.cols, ncols, at.empty, at.nempty, rb0, Mb, tid);
   if (ncols == 0) return;
   __syncthreads();  // flags and rec are dead: the stages may be written
 
@@ -1678,15 +1685,15 @@ __device__ __forceinline__ void sdd_pp_body(const GemmArgs& g, int tiles_m, int 
 }
 
 template <typename T, bool EDGE, typename G>
-__device__ __forceinline__ void sdd_any_body(const GemmArgs& g, int tiles_m, int gmax, int Mb, int Cb, const int bid) {
+__device__ __forceinline__ void sdd_any_body(const GemmArgs& g, int tiles_m, int gsure, int Mb, int Cb, const int bid) {
   // aligned operands on the 4-row-block shape: the kernel whose waves alternate between memory and compute phases
-  if constexpr (!EDGE && G::R == 4) sdd_pp_body<T>(g, tiles_m, gmax, Mb, Cb, bid);
-  else sdd_body<T, EDGE, G>(g, tiles_m, gmax, Mb, Cb, bid);
+  if constexpr (!EDGE && G::R == 4) sdd_pp_body<T>(g, tiles_m, gsure, Mb, Cb, bid);
+  else sdd_body<T, EDGE, G>(g, tiles_m, gsure, Mb, Cb, bid);
 }
 
 template <typename T, bool EDGE, typename G>
-__global__ __launch_bounds__(THREADS) void sdd_group_kernel(GemmArgs g, int tiles_m, int gmax, int Mb, int Cb) {
-  sdd_any_body<T, EDGE, G>(g, tiles_m, gmax, Mb, Cb, (int)blockIdx.x);
+__global__ __launch_bounds__(THREADS) void sdd_group_kernel(GemmArgs g, int tiles_m, int gsure, int Mb, int Cb) {
+  sdd_any_body<T, EDGE, G>(g, tiles_m, gsure, Mb, Cb, (int)blockIdx.x);
 }
 
 // Both gradients of one layer in one launch: workgroups [0, n_dx) are the SDD product's (dX; those past its own
@@ -1696,13 +1703,13 @@ __global__ __launch_bounds__(THREADS) void sdd_group_kernel(GemmArgs g, int tile
 // two, and the second product's workgroups fill the CUs the first one's last round leaves idle - for small layers,
 // whose grids cover a fraction of the chip each, the two simply run side by side.
 template <typename T, bool EDGE, typename G, typename S>
-__global__ __launch_bounds__(THREADS) void backward_pair_kernel(GemmArgs gx, int x_tiles_m, int x_gmax, int x_Mb,
-                                                                int x_Cb, int n_dx, GemmArgs gw, int w_tiles_m,
+__global__ __launch_bounds__(THREADS) void backward_pair_kernel(GemmArgs gx, int x_tiles_m, int x_gmax, int x_gsure,
+                                                                int x_Mb, int x_Cb, int n_dx, GemmArgs gw, int w_tiles_m,
                                                                 int w_tiles_n, int w_Mb, int w_Kb, int w_splits) {
   static_assert(S::THREADS == THREADS, "both products run on 512 threads");
   const int bid = (int)blockIdx.x;
   if (bid < n_dx) {
-    if (bid < x_tiles_m * x_gmax) sdd_any_body<T, EDGE, G>(gx, x_tiles_m, x_gmax, x_Mb, x_Cb, bid);
+    if (bid < x_tiles_m * x_gmax) sdd_any_body<T, EDGE, G>(gx, x_tiles_m, x_gsure, x_Mb, x_Cb, bid);
   } else {
     // the weight gradient's workgroups, tile index fastest, then the part of a split reduction
     const int wb = bid - n_dx, w_tiles = w_tiles_m * w_tiles_n;
@@ -1815,7 +1822,7 @@ constexpr ShapeCost kGradientCost[4] = {{2,       4.79,  {0.26, 0.45, 0.},   0.,
 constexpr ShapeCost kSddCost[4] = {     {2,       4.22,  {0.24, 0.40, 0.},   0.,   0.,   4.07, 1.69, 2.82, 0.29},
                                         {1,       5.47,  {0.46, 0., 0.},     0.,   0.,   4.51, 2.28, 4.83, 0.19},
                                         {3,       4.73,  {0.52, 0.61, 0.85}, 0.,   0.,   2.03, 1.44, 3.09, 0.24},
-                                        {1,       14.19, {1.20, 0., 0.},     0.,   0.,   2.52, 3.26, 5.49, 0.24}};
+                                        {1,       14.00, {1.20, 0., 0.},     0.,   6.50, 1.64, 3.26, 5.49, 0.22}};
 
 // A product on a shape: workgroups, steps of one of them, and what it costs beside them.
 struct ShapeWork {
@@ -1889,28 +1896,41 @@ DsdPlan plan_dsd(int64_t M, int64_t N, int64_t K, bool kc, double kept, int act)
   return best;
 }
 
+// Groups of the big SDD shape: the most a row quad can have (the grid provides for them), and how many it is expected to have
+// (deal_group's rule on expected numbers; half a group for the rounding up).
+int sdd_most_groups(const GemmArgs& g) { return (int)((blocks_of(g.N) + SddBig::MINCOLS - 1) / SddBig::MINCOLS); }
+double sdd_row_groups(const GemmArgs& g) {
+  const double k = kept_blocks(g), n = 1.0 - k, Cb = (double)blocks_of(g.N);
+  if (k > 0.999) return sdd_most_groups(g);
+  const double any = Cb * (1.0 - n * n * n * n), two = Cb * k * k * k * (4.0 * n + k);
+  return std::min((double)sdd_most_groups(g), std::max(1.0, 0.5 + std::max(any / 6.0, (any + two) / 8.0)));
+}
+// workgroups the big SDD shape is expected to have
+int64_t sdd_big_groups(const GemmArgs& g) { return (int64_t)((double)((blocks_of(g.M) + 3) / 4) * sdd_row_groups(g) + 0.5); }
+// Whether the workgroups count the groups of all row quads (find_group): where the groups expected nearly fill their last round, so
+// that an engine with one or two more than others takes another, and a round is long against the 4 to 5 us that each
+// workgroup counts.  dX of 8192^3, us without and with: p = 0.75 (1.9 rounds) 500 -> 391, 0.4 (2.96) 766 -> 671; 0.5 (2.6) 602 -> 618,
+// 0.6 (2.4) 558 -> 591.
+bool sdd_counts_all(const GemmArgs& g) {
+  const int64_t Mb = blocks_of(g.M);
+  if (!g.row_ptr || sdd_row_groups(g) >= sdd_most_groups(g) || Mb > 4 * kCountedQuads || Mb * blocks_of(g.N) > kCountedBlocks) return false;
+  const double rounds = (double)sdd_big_groups(g) / 256.0, over = rounds - (double)(int64_t)rounds;
+  return over > 0.75 && over < 0.98 && (double)blocks_of(g.K) > 8.0 * rounds;
+}
+// What the kernels are told: 0 for that, or the groups that nearly every row quad has (those above come last in the launch order).
+int sdd_sure_groups(const GemmArgs& g) {
+  return sdd_counts_all(g) ? 0 : std::min(sdd_most_groups(g), (int)(sdd_row_groups(g) + 1.0));
+}
 template <typename T, bool EDGE>
 int launch_sdd_big(const GemmArgs& g, hipStream_t stream) {
   using G = SddBig;
   static std::atomic<bool> configured[kMaxDevices] = {};
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(&sdd_group_kernel<T, EDGE, G>), G::SMEM, configured)) return rc;
   const int Mb = (int)((g.M + BS - 1) / BS), Cb = (int)((g.N + BS - 1) / BS);
-  // the grid provides for the most groups a row of the block grid can split into
-  const int tiles_m = (Mb + G::R - 1) / G::R, gmax = (Cb + G::MINCOLS - 1) / G::MINCOLS;
-  hipLaunchKernelGGL((sdd_group_kernel<T, EDGE, G>), dim3((unsigned)(tiles_m * gmax)), dim3(THREADS), G::SMEM, stream,
-                     g, tiles_m, gmax, Mb, Cb);
+  const int tiles_m = (Mb + G::R - 1) / G::R;
+  hipLaunchKernelGGL((sdd_group_kernel<T, EDGE, G>), dim3((unsigned)(tiles_m * sdd_most_groups(g))), dim3(THREADS), G::SMEM,
+                     stream, g, tiles_m, sdd_sure_groups(g), Mb, Cb);
   return check_launch("sdd_group_kernel");
-}
-
-float kept_fraction(const GemmArgs& g) {  // the caller's hint; unknown counts as everything kept
-  return (g.row_ptr && g.keep_hint >= 0.f && g.keep_hint <= 1.f) ? g.keep_hint : 1.f;
-}
-
-// workgroups the big SDD shape would have: a group spans 4 column blocks with everything kept, 6 once few enough tiles
-// are kept for the width and not the tile count to end a group (measured: worth counting that way from p = 0.7)
-int64_t sdd_big_groups(const GemmArgs& g) {
-  const int64_t cols = kept_fraction(g) <= 0.3f ? SddBig::GW : SddBig::MINCOLS;
-  return ((blocks_of(g.M) + 3) / 4) * ((blocks_of(g.N) + cols - 1) / cols);
 }
 
 // what the kernels of either kind ask of an SDD product's operands, and what the big ones ask on top
@@ -1924,35 +1944,28 @@ bool sdd_big_ok(const GemmArgs& g) {
          blocks_of(g.N) <= G_MAX_CB;
 }
 
-// Workgroups of an SDD strip shape that have kept tiles, eight times as many as the XCD with the most of them gets.  The grid
-// holds every strip a row could fill, those of one row next to each other, kept ones first; an XCD takes a contiguous eighth
-// of an order that walks eight rows at a time, so that its part can be all kept strips (1371 x 2304 from 7104 at p = 0.5, 64 x 64
-// tiles: 792 workgroups, 396 of them kept, take the time of 792).
+// Workgroups of an SDD strip shape that are expected to have kept tiles.
 double busy_strips(const GemmArgs& g, int cols, double keep) {
   const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), per_row = (double)((blocks_of(g.N) + cols - 1) / cols);
-  const double grid = Mb * per_row;
-  if (keep > 0.999) return grid;
-  double kept = Cb * keep / cols + (cols - 1) / (2.0 * cols);  // a row's kept tiles end inside its last strip
-  kept = std::min(std::max(kept, std::min(1.0, Cb * keep)), per_row);
-  const double walk = 8.0 * per_row, run = grid / 8.0, whole = (double)(int64_t)(run / walk);
-  return std::max(1.0, std::min(grid, 8.0 * (whole * 8.0 * kept + std::min(run - whole * walk, 8.0 * kept))));
+  if (keep > 0.999) return Mb * per_row;
+  const double kept = Cb * keep / cols + (cols - 1) / (2.0 * cols);  // a row's kept tiles end inside its last strip
+  return Mb * std::min(std::max(kept, std::min(1.0, Cb * keep)), per_row);
 }
 
 // The SDD product on a shape: its kept tiles in strips of one, four or two, or groups of the big shape.
 ShapeWork sdd_work(int shape, const GemmArgs& g) {
-  const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), hint = kept_fraction(g);
-  const double keep = g.quads ? 1.0 - (1.0 - hint) * (1.0 - hint) * (1.0 - hint) * (1.0 - hint) : hint;  // of the 64-blocks
+  const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), keep = kept_blocks(g);
   ShapeWork w{kSddCost[shape], 0., 0., 0.};
   w.wgs = shape == kShapeBig ? (double)sdd_big_groups(g) : busy_strips(g, shape == kShapeOne ? 1 : (shape == kShapeQuad ? 4 : 2), keep);
   double extra = g.N % BS || g.K % BS ? w.cost.ragged : 0.0;
   if (shape == kShapeBig) {
-    w.steps = (double)blocks_of(g.K) * (0.8 + 0.28 * keep);  // groups of more column blocks, fewer of their tiles kept
+    w.steps = (double)blocks_of(g.K) * (0.892 + 0.085 * keep);  // groups of more column blocks, fewer of their tiles kept
   } else {
     // Rows that end anywhere cost the strips more the more W there is (log2 of its megabytes), tile rows lying across 128-byte
     // lines; and past 24 MB of W every row's strips fetch their own columns from outside the caches, which strips of two
     // do twice as often for a row of dY as strips of four (6656 x 6736 from 7008, ragged, p = 0.1: 1474 us; 635 on the big shape).
     const double mb = std::log2((double)g.N * (double)g.K * 2e-6), cold = std::max(0.0, mb - 4.5);
-    const double each = shape == kShapeWide ? 0.22 - 0.12 * keep + (extra > 0.0 ? 0.16 : 0.0) : (shape == kShapeQuad ? 0.1 : 0.2);
+    const double each = shape == kShapeWide ? 0.22 - 0.12 * keep + (extra > 0.0 ? 0.16 : 0.0) : (shape == kShapeQuad ? 0.13 : 0.2);
     extra = extra * (0.6 + 0.25 * std::min(std::max(mb, 0.0), 4.0)) + cold * each;
     w.steps = (double)blocks_of(g.K);
   }
@@ -1961,18 +1974,19 @@ ShapeWork sdd_work(int shape, const GemmArgs& g) {
   return w;
 }
 
-// The shape with the smallest expected time: 1.5 % over the best one on average on reductions of four blocks and more (1.6 % on
-// 900 layers drawn afterwards).  The rules before (limits on the number of groups, of kept tiles and of strips, and a formula
-// for strips of two on reductions of 256 to 4096) were 8.5 % over it, one in ten 30 % or more, most of them ragged (33 % on
-// average above 4e10 products): dX of 11904 x 6344 from 6112 at p = 0.2 with GELU 2173 us on strips, 920 on the big shape.
-// Shorter reductions stay where they were, on the big shape, when its grid gives more than half of the CUs a workgroup;
-// strips of two are faster there too (11415 x 2560 from 128 with GELU: 62 against 27 us), which is left as it is.
+// The shape with the smallest expected time.  Over 2000 drawn layers timed on all four (128 to 16384 rows, 128 to 8192 columns and
+// reductions of 64 to 8192, p of 0.05 to 0.75) it is 1.0 % over the best one on average on reductions of four blocks and more, one in
+// fifty 17 %; the figures of the strips are older, those of the big shape were fitted to these when its groups were dealt out.
+// Reductions of less than four blocks go to the strips whatever is expected: what counts there is how many stores and first loads a CU
+// has on their way (5632 x 4672 from 128 at p = 0.6: strips of two 17.1 us, big shape 31.8; 2560 x 7744 from 64 at 0.3: 15.9, 27.6).
+// Nearly dense ones on whole blocks keep the big shape they always had when its grid gives more than half of the CUs a workgroup
+// (the suite pins it), where strips would gain less: 3456 x 3200 from 128 at p = 0.1 13.0 us, 16.7.
 int plan_sdd(const GemmArgs& g) {
   const int policy = tile_policy.load(std::memory_order_relaxed);
-  const bool ragged = g.N % BS || g.K % BS, brief = blocks_of(g.K) < 4;
   const bool big = sdd_big_ok(g);
   if (policy == kTileMid) return kShapeWide;
-  if (big && (policy == kTileBig || (brief && !ragged && sdd_big_groups(g) > 128))) return kShapeBig;
+  const bool brief = blocks_of(g.K) < 4, dense = kept_blocks(g) > 0.85 && g.N % BS == 0 && g.K % BS == 0;
+  if (big && (policy == kTileBig || (brief && dense && sdd_big_groups(g) > 128))) return kShapeBig;
   int best = kShapeOne;
   for (int shape = kShapeQuad; shape <= (big && !brief ? kShapeBig : kShapeWide); ++shape)
     if (sdd_work(shape, g).time() < sdd_work(best, g).time()) best = shape;
@@ -2267,13 +2281,13 @@ int launch_pair_t(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_
   if (int rc = allow_big_lds(reinterpret_cast<const void*>(&backward_pair_kernel<T, EDGE, G, S>), SMEM, configured))
     return rc;
   const int x_Mb = (int)((gx.M + BS - 1) / BS), x_Cb = (int)((gx.N + BS - 1) / BS);
-  const int x_tiles_m = (x_Mb + G::R - 1) / G::R, x_gmax = (x_Cb + G::MINCOLS - 1) / G::MINCOLS;
+  const int x_tiles_m = (x_Mb + G::R - 1) / G::R, x_gmax = sdd_most_groups(gx);
   const int64_t n_dx = ((int64_t)x_tiles_m * x_gmax + 7) / 8 * 8;
   const int w_Mb = (int)((gw.M + BS - 1) / BS), w_Kb = (int)((gw.K + BS - 1) / BS);
   const int w_tiles_m = (w_Mb + S::R - 1) / S::R, w_tiles_n = (int)((gw.N + S::BN - 1) / S::BN);
   const int64_t total = n_dx + (int64_t)w_tiles_m * w_tiles_n * splits;
   hipLaunchKernelGGL((backward_pair_kernel<T, EDGE, G, S>), dim3((unsigned)total), dim3(THREADS), SMEM, stream, gx,
-                     x_tiles_m, x_gmax, x_Mb, x_Cb, (int)n_dx, gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, splits);
+                     x_tiles_m, x_gmax, sdd_sure_groups(gx), x_Mb, x_Cb, (int)n_dx, gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, splits);
   return check_launch("backward_pair_kernel");
 }
 

@@ -466,14 +466,14 @@ __device__ __forceinline__ void tile_dsd_body(const GemmArgs& g, int tiles_m, in
 // column blocks of it, straight from the row's list, and stores the zeros of column blocks [C * j, C * j + C) that the
 // list leaves out: every product it computes is wanted, and dropped tiles cost the zeros alone.
 template <typename T, typename S>
-__device__ __forceinline__ void tile_sdd_body(const GemmArgs& g, int tiles_n, int Mb, int Cb, int bid) {
+__device__ __forceinline__ void tile_sdd_body(const GemmArgs& g, int sure, int Mb, int Cb, int bid) {
   static_assert(S::R == 1 && S::HALVES, "one row block");
   constexpr int C = S::C, NST = S::NST, LPW = S::LPW, NT16 = S::NT16;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t smem_a = lds_address(smem);
   uint32_t* found = reinterpret_cast<uint32_t*>(smem);
   int tm, tn;
-  tile_of_block<DSD_GROUP_M>(bid, Mb, tiles_n, tm, tn);
+  group_of_block<DSD_GROUP_M>(bid, Mb, sure, tm, tn);
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = (int)uniform((uint32_t)(tid / 64));
   const int lwave = S::LW ? wave - S::NW : wave;  // index among the waves that load

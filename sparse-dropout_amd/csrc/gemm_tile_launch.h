@@ -41,8 +41,8 @@ __global__ __launch_bounds__(S::THREADS) void tile_dsd_kernel(GemmArgs g, int ti
 }
 
 template <typename T, typename S>
-__global__ __launch_bounds__(S::THREADS) void tile_sdd_kernel(GemmArgs g, int tiles_n, int Mb, int Cb) {
-  tile_sdd_body<T, S>(g, tiles_n, Mb, Cb, (int)blockIdx.x);
+__global__ __launch_bounds__(S::THREADS) void tile_sdd_kernel(GemmArgs g, int sure, int Mb, int Cb) {
+  tile_sdd_body<T, S>(g, sure, Mb, Cb, (int)blockIdx.x);
 }
 
 // The forward product and the kept lists of its mask in one launch (see forward_lists_kernel of the large shapes).
@@ -65,13 +65,13 @@ __global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, in
 // Both gradients in one launch: workgroups [0, n_dx) are the input gradient's (a multiple of 8, so that the second
 // product's tile map keeps its XCD assignment), the rest the weight gradient's.
 template <typename T, typename X, typename W>
-__global__ __launch_bounds__(W::THREADS) void tile_pair_kernel(GemmArgs gx, int x_tiles_n, int x_Mb, int x_Cb, int n_dx,
-                                                               GemmArgs gw, int w_tiles_m, int w_tiles_n, int w_Mb,
-                                                               int w_Kb, int w_splits) {
+__global__ __launch_bounds__(W::THREADS) void tile_pair_kernel(GemmArgs gx, int x_tiles_n, int x_sure, int x_Mb, int x_Cb,
+                                                               int n_dx, GemmArgs gw, int w_tiles_m, int w_tiles_n,
+                                                               int w_Mb, int w_Kb, int w_splits) {
   static_assert(X::THREADS == W::THREADS, "both products run on the same number of threads");
   const int bid = (int)blockIdx.x;
   if (bid < n_dx) {
-    if (bid < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_tiles_n, x_Mb, x_Cb, bid);
+    if (bid < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_sure, x_Mb, x_Cb, bid);
   } else {
     tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, bid - n_dx, w_splits);
   }
@@ -123,6 +123,12 @@ int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t
   return f.tabled ? forward_launch_t<T, S, true>(g, splits, f, stream) : forward_launch_t<T, S, false>(g, splits, f, stream);
 }
 
+// Of the strips of C kept column blocks that a row of the block grid can have, `most`, those that about every row has.
+int sure_strips(const GemmArgs& g, int C, int most) {
+  const double keep = kept_blocks(g);
+  return keep > 0.999 ? most : std::min(most, std::max(1, (int)((double)blocks_of(g.N) * keep / C + (C - 1) / (2.0 * C) + 0.5)));
+}
+
 template <typename T, typename S>
 int sdd_launch(const GemmArgs& g, hipStream_t stream) {
   static std::atomic<bool> done[64] = {};
@@ -134,7 +140,7 @@ int sdd_launch(const GemmArgs& g, hipStream_t stream) {
   // 33 -> 26; 8192 x 8192 from 1024 at p = 0.5 132 -> 114; 200704 x 288 from 64 (a convolution's, one step) 51 -> 41.
   const int64_t stages = std::min<int64_t>(blocks_of(g.K), S::NST);
   const int smem = std::max((int)stages * S::STAGE, S::NW * 2 * S::NT16 * 1024);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(Mb * tn)), dim3(S::THREADS), smem, stream, g, tn, Mb, Cb);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(Mb * tn)), dim3(S::THREADS), smem, stream, g, sure_strips(g, S::C, tn), Mb, Cb);
   return check_launch("tile_sdd_kernel");
 }
 
@@ -147,8 +153,8 @@ int pair_launch(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_t 
   const int x_Mb = blocks_of(gx.M), x_Cb = blocks_of(gx.N), x_tn = (x_Cb + X::C - 1) / X::C;
   const int n_dx = (x_Mb * x_tn + 7) / 8 * 8;
   const int w_Mb = blocks_of(gw.M), w_Kb = blocks_of(gw.K), w_tm = (w_Mb + W::R - 1) / W::R, w_tn = (blocks_of(gw.N) + W::C - 1) / W::C;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_dx + w_tm * w_tn * splits)), dim3(W::THREADS), SMEM, stream, gx, x_tn, x_Mb,
-                     x_Cb, n_dx, gw, w_tm, w_tn, w_Mb, w_Kb, splits);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_dx + w_tm * w_tn * splits)), dim3(W::THREADS), SMEM, stream, gx, x_tn,
+                     sure_strips(gx, X::C, x_tn), x_Mb, x_Cb, n_dx, gw, w_tm, w_tn, w_Mb, w_Kb, splits);
   return check_launch("tile_pair_kernel");
 }
 

@@ -33,6 +33,20 @@ template <int GROUP_M>
 __host__ __device__ inline void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
   tile_in_order<GROUP_M>(xcd_run(bid, tiles_m * tiles_n), tiles_m, tiles_n, tm, tn);
 }
+// SDD's strips of a row's kept column blocks, or groups of a row quad's (tm: row or quad, gi: strip or group of it).  How many a row
+// has depends on the mask; the grid holds the most.  Those that about every row has, gsure of them, come first, GROUP_M rows
+// walked together and an eighth of them to an XCD; the others, most of which are empty, behind them and all over the chip.  With
+// the empty ones in between, the eighths of two XCDs were all full and half empty.
+template <int GROUP_M>
+__host__ __device__ inline void group_of_block(int bid, int rows, int gsure, int& tm, int& gi) {
+  const int first = rows * gsure;
+  if (bid < first) {
+    tile_of_block<GROUP_M>(bid, rows, gsure, tm, gi);
+  } else {
+    gi = gsure + (bid - first) / rows;
+    tm = (bid - first) % rows;
+  }
+}
 // The same for a reduction split over nsplit workgroups per tile (bid < tiles_m * tiles_n * nsplit): an XCD's run goes
 // through the tiles of one part after the other, which read the same rows of both operands.  Dealt out part by part
 // across the XCDs, every L2 fetched nearly everything: dW of 200704 x 288 -> 64 39 -> 28 us, of 16384 x 1536 -> 384 35 -> 31.
