@@ -165,10 +165,10 @@ SD_BOTH int64_t taps_lds(const TapGeom& geo, bool dx, int64_t span) {
 
 constexpr int kDwTaps = 9;    // of a workgroup
 constexpr int kDwPitch = 64;  // bytes of an LDS row of 32 channels: the four rows of a transposing read in different banks
-// Weight gradient.  A buffer: rows of the window and one of zeros, 256 rows of dY, a record per position.  In the end two of the
-// four blocks' sums meet there: 2 x 2 waves x 64 lanes x 9 x 16 floats.
+// Weight gradient.  A buffer: rows of the window and one of zeros, 256 rows of dY, a record per position.  In the end three taps' sums
+// of the eight waves meet there: 8 x 64 lanes x 3 x 16 floats.
 SD_BOTH int64_t dw_lds(int64_t span, int buffers) {
-  const int64_t merge = 2 * 2 * 64 * kDwTaps * 16 * 4, turns = buffers * ((span + 16) * kDwPitch + 256 * 128 + 256 * 8);
+  const int64_t merge = 8 * 64 * 3 * 16 * 4, turns = buffers * ((span + 16) * kDwPitch + 256 * 128 + 256 * 8);
   return turns < merge ? merge : turns;
 }
 

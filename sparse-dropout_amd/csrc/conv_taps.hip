@@ -14,10 +14,10 @@
 //    block is kept (sums stay in fp32; the two-kernel route rounds every tap's term to the element type).
 // The products cost the dense number of operations and little else: the rows are read once, there is no matrix R*S times
 // the image to write and read back, and no per-element fold.  A step (forward and gradients, kernel times in us):
-//   128 x 64 x 32 x 32 -> 128, 3 x 3, fp16, p = 0.5: rows, weights and mask 25, y 28, dx 37, dw 41 + 5; before: lists 13, y 43
-//   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7.  192 -> 128 a pass.
-//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 28 + 7; before: lists 13, patch matrix 45, y 30, rows of dy 13,
-//   patch gradient 40, fold 52, dw 28 + 6.  227 -> 103.
+//   128 x 64 x 32 x 32 -> 128, 3 x 3, fp16, p = 0.5: rows, weights and mask 25, y 28, dx 37, dw 31 + 5; through lists: lists 13, y 43
+//   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7, 192 a pass.
+//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 7; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
+//   patch gradient 40, fold 52, dw 28 + 6, 227 a pass.
 #include <atomic>
 
 #include "common.h"
@@ -461,7 +461,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 // 256.  Two waves take 16 channels each, four pairs of them a 64-position block of the turn each; a wave's dY fragments
 // serve all its taps, its image fragments are transposing reads of rows shifted by the tap.  The four blocks' sums meet
 // in LDS at the end, so a CU leaves one partial result (a round of 256 of them: 19 MB at any size), which
-// taps_dw_reduce adds up.  Bound by what the waves issue: per tap 17 instructions of picks and some 20 of addresses beside 8 products.
+// taps_dw_reduce adds up.  With two waves to a SIMD it is bound by latency and by what the waves issue around the products: a turn of
+// 256 positions takes 2.7 us, 1.1 of them products, the first reads of a turn 0.5 or so, in which nobody multiplies.  Two steps
+// made 3.4 of it 2.7: clearing image fragments (8 instructions a tap) instead of picking results (17), and the order of
+// all_turns.  128 x 64 x 32 x 32 -> 128, p = 0.5: 41.2 -> 31.2 us, 256 x 32 x 28 x 28 -> 64, p = 0.25: 27.9 -> 20.5.
 constexpr int kDwThreads = 512;
 
 struct TapDwArgs {
@@ -511,40 +514,37 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
     }
     column[i / 4] |= (uint32_t)((c * RS + t) / 64 - cb0) << (i % 4 * 8);
   }
-  // ---- loads
-  uint32_t dy_off[4];
+  // ---- loads, by the second four waves (all_turns)
+  const int lw = wave - 4;
+  uint32_t dy_off[2];  // the swizzle of a load's eight rows depends on whether its number is odd
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = (wave * 4 + i) * 8 + lane / 8, ch = (lane % 8) ^ swz_x(row);
+  for (int i = 0; i < 2; ++i) {
+    const int row = i * 8 + lane / 8, ch = (lane % 8) ^ swz_x(row);
     dy_off[i] = k0 + ch * 8 < g.K ? (uint32_t)((row * g.dy_ld + k0 + ch * 8) * 2) : kNoData;
   }
   auto window = [&](int turn) {
     const int m0 = turn * kPos;
     return TapWindow(g.geo, (uint32_t)m0, (uint32_t)(m0 + kPos < g.rows ? m0 + kPos - 1 : g.rows - 1));
   };
-  auto load_dy = [&](int turn, int buf) {
-    const u32x4 d = buffer_of(reinterpret_cast<const char*>(g.dy + (int64_t)turn * kPos * g.dy_ld));
-    const uint32_t dst = smem_a + (uint32_t)(buf * buffer + x_bytes + wave * 4096);
+  auto load = [&](int turn, const TapWindow& w, int buf) {
+    if (lw < 0) return;
+    const int row0 = turn * kPos + lw * 64, left = clamp_int(g.rows - row0, 0, 64);  // rows past the last arrive as zeros
+    u32x4 d = buffer_of(reinterpret_cast<const char*>(g.dy + (int64_t)row0 * g.dy_ld));
+    d.z = uniform((uint32_t)(left * (int)g.dy_ld * 2));
+    const uint32_t dst = smem_a + (uint32_t)(buf * buffer + x_bytes + lw * 8192);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = (wave * 4 + i) * 8 + lane / 8;
-      buffer16_to_lds(d, turn * kPos + row < g.rows ? dy_off[i] : kNoData, dst + (uint32_t)(i * 1024));
-    }
-  };
-  auto load_x = [&](int turn, int buf) {
-    const TapWindow w = window(turn);
+    for (int i = 0; i < 8; ++i) buffer16_to_lds(d, dy_off[i % 2] + (uint32_t)(i / 2 * 32 * (int)g.dy_ld), dst + (uint32_t)(i * 1024));
     const int n = w.hi - w.lo < g.span ? w.hi - w.lo : g.span;
-    const u32x4 d = buffer_of(reinterpret_cast<const char*>(g.x + (int64_t)w.lo * g.x_ld + c0));
-    for (int r0 = wave * 16; r0 < n; r0 += 128) {
+    const u32x4 x = buffer_of(reinterpret_cast<const char*>(g.x + (int64_t)w.lo * g.x_ld + c0));
+    for (int r0 = lw * 16; r0 < n; r0 += 64) {
       const int row = r0 + lane / 4, ch = lane % 4;
       const uint32_t off = row < n && c0 + ch * 8 < g.C ? (uint32_t)((row * g.x_ld + ch * 8) * 2) : kNoData;
-      buffer16_to_lds(d, off, smem_a + (uint32_t)(buf * buffer + r0 * kDwPitch));
+      buffer16_to_lds(x, off, smem_a + (uint32_t)(buf * buffer + r0 * kDwPitch));
     }
   };
   // records: where tap 0 of a position lies in the window, and which of the taps are inside the image
-  auto put_records = [&](int turn, int buf) {
+  auto put_records = [&](int turn, const TapWindow& w, int buf) {
     if (tid >= kPos) return;
-    const TapWindow w = window(turn);
     const int pos = turn * kPos + tid;
     u32x2 rec = {0u, 0u};
     if (pos < g.rows) {
@@ -555,138 +555,195 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
   };
   if (tid < 4 * g.buffers)  // a row of zeros behind the window
     *reinterpret_cast<u32x4*>(smem + tid / 4 * buffer + g.span * kDwPitch + tid % 4 * 16) = u32x4{0u, 0u, 0u, 0u};
-  auto kept_bit = [&](int turn) -> bool {  // lane j: block column cb0 + j of this wave's row block
-    const int rb = turn * 4 + pb, cb = cb0 + lane;
-    return lane < 32 && rb * 64 < g.rows && cb < cbs && block_kept(g, rb, cb);
+  // Lane j: what the mask holds for block column cb0 + j of this wave's row block, 1 past its end.  Loaded in front of a turn's direct
+  // loads and looked at behind the products: the compiler waits for everything on its way where the byte is used.
+  const uint8_t* const mask_col = g.mask + (int64_t)(g.split == 1 ? cb0 + lane : (cb0 + lane) / g.split) * g.msc;
+  auto dropped = [&](int turn) -> uint32_t {
+    const int rb = turn * 4 + pb;
+    uint32_t d = 1u;
+    if (lane < 32 && rb * 64 < g.rows && cb0 + lane < cbs) d = g.mask ? mask_col[(int64_t)(g.split == 1 ? rb : rb / g.split) * g.msr] : 0u;
+    return d;
   };
 
   f32x4 acc[kDwTaps][4];
-#pragma unroll
-  for (int i = 0; i < kDwTaps; ++i)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
   FragmentReads<false> fd[2];
   fd[0].init(lane, 0);
   fd[1].init(lane, 1);
   const int b4 = lane / 16, e = (lane % 16) / 4, j = lane % 4;
-  const int in_block = 8 * b4 + e, x_col = cw * 32 + j * 8, zero_at = g.span * kDwPitch + x_col;
+  const int in_block = 8 * b4 + e, x_col = cw * 32 + j * 8;
 
-  uint32_t kept = 0;
-  if (first < last) {
-    load_dy(first, 0);
-    load_x(first, 0);
-    const bool k1 = kept_bit(first);
-    put_records(first, 0);
-    kept = (uint32_t)__ballot(k1);
-  }
-  for (int turn = first; turn < last; ++turn) {
-    const int buf = g.buffers == 2 ? (turn - first) & 1 : 0;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const bool more = turn + 1 < last;
-    bool k1 = false;
-    if (more) {
-      if (g.buffers == 2) {
-        load_dy(turn + 1, buf ^ 1);
-        load_x(turn + 1, buf ^ 1);
-      }
-      k1 = kept_bit(turn + 1);
+  // All turns.  The second four waves, one to each SIMD, bring the next turn's rows and the first four write its records when their
+  // products are done: with all eight at both, every SIMD's two waves stood at the same loads and reads at the same time (33.5 us at
+  // 128 x 64 x 32 x 32 -> 128, so 32.9).  PICKS: a tap's products are added to the sums of the kept blocks only; else the lane's channel is cleared in the image
+  // fragments of dropped blocks, which is half the instructions and sums the same numbers, unless dY holds an Inf or NaN.
+  auto all_turns = [&](auto picks) {
+    constexpr bool PICKS = decltype(picks)::value;
+#pragma unroll
+    for (int i = 0; i < kDwTaps; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint32_t kept = 0;
+    if (first < last) {
+      const uint32_t d1 = dropped(first);
+      const TapWindow w = window(first);
+      load(first, w, 0);
+      put_records(first, w, 0);
+      kept = (uint32_t)__ballot(d1 == 0u);
     }
-    if (kept) {
-      const char* xl = smem + buf * buffer;
-      const char* dl = xl + x_bytes + pb * TILE;
-      const char* rec = xl + x_bytes + 256 * 128 + pb * 512;
-      int at[4];
-      uint32_t in[4];
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {  // positions 32 * (h / 2) + 4 * (h % 2) + in_block of the block
-        const u32x2 r = *reinterpret_cast<const u32x2*>(rec + (32 * (h / 2) + 4 * (h % 2) + in_block) * 8);
-        at[h] = (int)r.x + x_col;
-        in[h] = r.y;
+    for (int turn = first; turn < last; ++turn) {
+      const int buf = g.buffers == 2 ? (turn - first) & 1 : 0;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      const bool more = turn + 1 < last;
+      uint32_t d1 = 1u;
+      const TapWindow next = window(more ? turn + 1 : turn);
+      if (more) {
+        d1 = dropped(turn + 1);
+        if (g.buffers == 2) load(turn + 1, next, buf ^ 1);
       }
-      u32x4 df[4][2];
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) df[k][kk] = fd[kk].read(dl, k);
-      auto read_tap = [&](int i, u32x4 (&xf)[2]) {
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          u32x2 v[2];
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const uint32_t a = (uint32_t)(at[2 * kk + h] + shift[i]);
-            v[h] = lds_read_tr(xl + ((in[2 * kk + h] >> i) & 1u ? a : (uint32_t)zero_at));
-          }
-          xf[kk] = u32x4{v[0].x, v[0].y, v[1].x, v[1].y};
+      if (kept) {
+        const int x_at = (int)smem_a + buf * buffer + x_col, zero_at = x_at + g.span * kDwPitch;
+        const char* xl = smem + buf * buffer;
+        const char* dl = xl + x_bytes + pb * TILE;
+        const char* rec = xl + x_bytes + 256 * 128 + pb * 512;
+        int at[4];  // where in LDS the lane's positions read tap 0
+        uint32_t in[4];
+  #pragma unroll
+        for (int h = 0; h < 4; ++h) {  // positions 32 * (h / 2) + 4 * (h % 2) + in_block of the block
+          const u32x2 r = *reinterpret_cast<const u32x2*>(rec + (32 * (h / 2) + 4 * (h % 2) + in_block) * 8);
+          at[h] = (int)r.x + x_at;
+          in[h] = r.y;
         }
-      };
-      // the fragments of a tap are read under the products of the one before; the scheduler is held to that order, since
-      // with all nine in its hands it computes their products first and runs out of registers for the picks
-      u32x4 xf[2][2];
-      read_tap(0, xf[0]);
+        u32x4 df[4][2];
+  #pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+  #pragma unroll
+          for (int k = 0; k < 4; ++k) df[k][kk] = fd[kk].read(dl, k);
+        auto read_quarter = [&](int i, int h, u32x4 (&xf)[2]) {
+          const int inside = ones_if(in[h], i);
+          int a = at[h] + shift[i];
+          a = (inside & a) | (~inside & zero_at);
+          const u32x2 v = lds_read_tr_at((uint32_t)a);
+          xf[h / 2][h % 2 * 2] = v.x;
+          xf[h / 2][h % 2 * 2 + 1] = v.y;
+        };
+        auto read_tap = [&](int i, u32x4 (&xf)[2]) {
 #pragma unroll
-      for (int i = 0; i < kDwTaps; ++i) {  // (past nt: no tap is inside, zeros are added, nothing of it is stored)
-        if (i + 1 < kDwTaps) read_tap(i + 1, xf[(i + 1) % 2]);
-        const int m = ones_if(kept, (int)(column[i / 4] >> (i % 4 * 8)));
-        f32x4 d[4];
+          for (int h = 0; h < 4; ++h) read_quarter(i, h, xf);
+        };
+        auto kept_of = [&](int i) { return ones_if(kept, (int)(column[i / 4] >> (i % 4 * 8))); };
+        // (past nt: no tap is inside, zeros are added, nothing of it is stored)
+        if constexpr (PICKS) {
+          // the fragments of a tap are read under the products of the one before; the scheduler is held to that order, since with all
+          // nine in its hands it computes their products first and runs out of registers for the picks
+          u32x4 xf[2][2];
+          read_tap(0, xf[0]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][0], xf[i % 2][0], acc[i][k]);
+          for (int i = 0; i < kDwTaps; ++i) {
+            if (i + 1 < kDwTaps) read_tap(i + 1, xf[(i + 1) % 2]);
+            const int m = kept_of(i);
+            f32x4 d[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][1], xf[i % 2][1], d[k]);
+            for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][0], xf[i % 2][0], acc[i][k]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][1], xf[i % 2][1], d[k]);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) acc[i][k][v] = pick(m, d[k][v], acc[i][k][v]);
-        __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) acc[i][k][v] = pick(m, d[k][v], acc[i][k][v]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          // Behind each product three or four other instructions, which is what fits under it: a quarter of the reads of the tap after
+          // next, or a quarter of the next tap's clears.  In blocks of products and blocks of the others the two add up, whichever of
+          // the SIMD's waves they are from (2.9 us a turn; without the products 1.7, the products alone 1.1).
+          u32x4 xf[3][2];
+          auto clear = [&](u32x4 (&x)[2], int q, uint32_t m) {
+            x[q / 2][q % 2 * 2] &= m;
+            x[q / 2][q % 2 * 2 + 1] &= m;
+          };
+          read_tap(0, xf[0]);
+          read_tap(1, xf[1]);
+          uint32_t m = (uint32_t)kept_of(0);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) clear(xf[0], q, m);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < kDwTaps; ++i) {
+            u32x4(&x)[2] = xf[i % 3];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              acc[i][k] = T::mfma16(df[k][0], x[0], acc[i][k]);
+              if (i + 2 < kDwTaps) read_quarter(i + 2, k, xf[(i + 2) % 3]);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              acc[i][k] = T::mfma16(df[k][1], x[1], acc[i][k]);
+              if (i + 1 < kDwTaps) {
+                if (k == 0) m = (uint32_t)kept_of(i + 1);
+                clear(xf[(i + 1) % 3], k, m);
+              }
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+      }
+      if (more) {
+        if (g.buffers != 2) {
+          __syncthreads();  // every wave is done with the only buffer
+          load(turn + 1, next, 0);
+        }
+        put_records(turn + 1, next, g.buffers == 2 ? buf ^ 1 : 0);
+        asm volatile("" : "+v"(d1));
+        kept = (uint32_t)__ballot(d1 == 0u);
       }
     }
-    if (more) {
-      if (g.buffers != 2) {
-        __syncthreads();  // every wave is done with the only buffer
-        load_dy(turn + 1, 0);
-        load_x(turn + 1, 0);
-      }
-      put_records(turn + 1, g.buffers == 2 ? buf ^ 1 : 0);
-      kept = (uint32_t)__ballot(k1);
-    }
+  };
+  all_turns(std::integral_constant<bool, false>{});
+  if (g.mask) {  // a sum that is not finite: once more, so that what a block drops does not reach it
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < kDwTaps; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bad = __builtin_fmaf(acc[i][k][v], 0.f, bad);
+    uint32_t* again = reinterpret_cast<uint32_t*>(smem + x_bytes);  // (dY's place; the row of zeros stays)
+    __syncthreads();
+    if (tid == 0) *again = 0u;
+    __syncthreads();
+    if (bad != 0.f) *again = 1u;
+    __syncthreads();
+    const uint32_t any = uniform(*again);
+    __syncthreads();
+    if (any) all_turns(std::integral_constant<bool, true>{});
   }
 
-  // ---- the four blocks' sums: 3 into 2 and 1 into 0, then 2 into 0
-  float* meet = reinterpret_cast<float*>(smem);
-  constexpr int WAVE_SUMS = 64 * kDwTaps * 16;
-  auto give = [&](int slot) {
-    float* d = meet + (slot * 2 + cw) * WAVE_SUMS + lane * 4;
-#pragma unroll
-    for (int i = 0; i < kDwTaps; ++i)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4*>(d + (i * 4 + k) * 256) = acc[i][k];
-  };
-  auto take = [&](int slot) {
-    const float* s = meet + (slot * 2 + cw) * WAVE_SUMS + lane * 4;
-#pragma unroll
-    for (int i = 0; i < kDwTaps; ++i)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) acc[i][k] += *reinterpret_cast<const f32x4*>(s + (i * 4 + k) * 256);
-  };
-  __syncthreads();
-  if (pb & 1) give(pb / 2);
-  __syncthreads();
-  if (!(pb & 1)) take(pb / 2);
-  __syncthreads();
-  if (pb == 2) give(0);
-  __syncthreads();
-  if (pb != 0) return;
-  take(0);
-  if (c >= g.C) return;
+  // ---- the four blocks' sums, three taps at a time: of a tap's four tiles every block's wave adds up and stores the one of its number.
+  // (One block after the other into the first, whose two waves then stored everything, took 8 of the 38 us of a workgroup of eight
+  // turns; this takes 3.6, most of it the stores.)
+  constexpr int TAPS = 3, TILES = 4 * TAPS;
+  static_assert(kDwTaps % TAPS == 0, "whole rounds");
+  char* meet = smem + cw * (4 * TILES * 1024) + lane * 16;
   float* part = g.part + (int64_t)sp * RS * g.C * g.K;
+  const int kk = k0 + pb * 16 + 4 * (lane / 16);
 #pragma unroll
-  for (int i = 0; i < kDwTaps; ++i)
+  for (int i0 = 0; i0 < kDwTaps; i0 += TAPS) {
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int kk = k0 + k * 16 + 4 * (lane / 16);
-      if (i < nt && kk < g.K) *reinterpret_cast<f32x4*>(part + ((int64_t)(t0 + i) * g.C + c) * g.K + kk) = acc[i][k];
+    for (int i = 0; i < TAPS; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4*>(meet + (pb * TILES + i * 4 + k) * 1024) = acc[i0 + i][k];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) {
+      const char* m = meet + (i * 4 + pb) * 1024;
+      const f32x4 s01 = *reinterpret_cast<const f32x4*>(m) + *reinterpret_cast<const f32x4*>(m + TILES * 1024);
+      const f32x4 s23 = *reinterpret_cast<const f32x4*>(m + 2 * TILES * 1024) + *reinterpret_cast<const f32x4*>(m + 3 * TILES * 1024);
+      if (i0 + i < nt && c < g.C && kk < g.K) *reinterpret_cast<f32x4*>(part + ((int64_t)(t0 + i0 + i) * g.C + c) * g.K + kk) = s01 + s23;
     }
+  }
 }
 
 // dw[k, c * R * S + t] = scale * sum over the splits of part[split][t][c][k]: four outputs per thread, the splits shared out

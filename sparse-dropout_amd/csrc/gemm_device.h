@@ -97,6 +97,12 @@ __device__ inline u32x2 lds_read_tr(const char* p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// the same at an LDS byte address (lds_address): an address picked out of two stays one instruction
+__device__ inline u32x2 lds_read_tr_at(uint32_t a) {
+  s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)a);
+  return __builtin_bit_cast(u32x2, v);
+}
+
 // Chunk swizzles of tiles kept in memory order [reduction row][columns] (read with ds_read_b64_tr_b16).  One
 // transposing read takes, per 16-lane group, 4 consecutive reduction rows x 32 bytes, and the groups of a wave
 // are 8 reduction rows apart.  A 64-column tile has rows of 128 B: rows r and r+2 would share banks, so bit 2 of

@@ -222,3 +222,25 @@ def test_what_a_mask_drops_reaches_nothing_tap_by_tap(bad):
         assert torch.equal(~torch.isfinite(y.permute(0, 2, 3, 1).reshape(rows, k).cpu()), bad_y), which
         assert torch.equal(~torch.isfinite(dx.cpu()), bad_dx), which
         assert torch.equal(~torch.isfinite(dw.cpu().reshape(k, -1)), bad_dw), which
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("geom", [(16, 128, 32, 32, 128, 3, 3, (1, 1), (1, 1)),   # two turns of 256 positions to a workgroup
+                                  (2, 512, 24, 40, 200, 3, 3, (1, 1), (1, 1)),    # seven, the last one not whole
+                                  (1, 32, 9, 256, 40, 3, 3, (1, 1), (1, 1))])     # one buffer of rows
+def test_gradients_that_are_not_finite_reach_kept_blocks_only(geom, bad):
+    """A weight gradient clears what a block drops in the image, and does without where a sum is not finite: one bad element of dY
+    reaches its output's kept blocks, and everything else is bit for bit what it is with a zero there."""
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, torch.float16)
+    mask = cpu_mask(O.mask_shape(rows, c * r * s, 64), 0.5, gen)
+    at = rows // 2 + 7, k // 3
+    img, pos = divmod(at[0], rows // n)
+    got = []
+    for v in (0.0, bad):
+        dy.view(n, k, -1)[img, at[1], pos] = v
+        got.append(_products(geom, x, wt, dy, mask, 64, 2.0)[2].cpu().reshape(k, -1))
+    reached = torch.zeros(k, c * r * s, dtype=torch.bool)
+    reached[at[1]] = ~mask[at[0] // 64].repeat_interleave(64)[: c * r * s]
+    assert torch.equal(~torch.isfinite(got[1]), reached)
+    assert torch.equal(got[1][~reached], got[0][~reached])
