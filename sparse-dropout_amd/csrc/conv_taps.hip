@@ -16,7 +16,7 @@
 // the image to write and read back, and no per-element fold.  A step (forward and gradients, kernel times in us):
 //   128 x 64 x 32 x 32 -> 128, 3 x 3, fp16, p = 0.5: rows, weights and mask 25, y 28, dx 37, dw 31 + 5; through lists: lists 13, y 43
 //   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7, 192 a pass.
-//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 7; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
+//   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 5; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
 //   patch gradient 40, fold 52, dw 28 + 6, 227 a pass.
 #include <atomic>
 
@@ -747,19 +747,30 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 }
 
 // dw[k, c * R * S + t] = scale * sum over the splits of part[split][t][c][k]: four outputs per thread, the splits shared out
-// over 16 threads.
-template <typename T>
-__global__ __launch_bounds__(256) void taps_dw_reduce(const float* part, uint16_t* dw, int64_t dw_ld, int C, int K, int RS,
-                                                      int splits, float scale) {
-  __shared__ f32x4 lds[16][16];
+// over SHARE threads.  Bound by the latency of the loads where the result is small: 256 parts of 288 x 64 over 16 threads 7.6 us, 196
+// over 64 5.3.
+template <typename T, int SHARE>
+__global__ __launch_bounds__(16 * SHARE) void taps_dw_reduce(const float* part, uint16_t* dw, int64_t dw_ld, int C, int K, int RS,
+                                                             int splits, float scale) {
+  __shared__ f32x4 lds[SHARE][16];
   const int64_t n4 = (int64_t)RS * C * K / 4;
   const int own = threadIdx.x % 16, q = threadIdx.x / 16;
   const int64_t o = (int64_t)blockIdx.x * 16 + own;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  if (o < n4)
-    for (int i = q; i < splits; i += 16) s += *reinterpret_cast<const f32x4*>(part + ((int64_t)i * n4 + o) * 4);
+  if (o < n4) {
+#pragma unroll 4
+    for (int i = q; i < splits; i += SHARE) s += *reinterpret_cast<const f32x4*>(part + ((int64_t)i * n4 + o) * 4);
+  }
   lds[q][own] = s;
   __syncthreads();
+  if (SHARE > 16) {
+    if (q < 16) {
+#pragma unroll
+      for (int i = 16; i < SHARE; i += 16) s += lds[i + q][own];
+      lds[q][own] = s;
+    }
+    __syncthreads();
+  }
   if (q != 0 || o >= n4) return;
 #pragma unroll
   for (int i = 1; i < 16; ++i) s += lds[i][own];
@@ -840,10 +851,11 @@ ConvShape shape_of(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k, int64_
 }
 
 int64_t dw_tiles(int64_t c, int64_t k, int64_t rs) { return ceil_div(c, 32) * ceil_div(k, 64) * ceil_div(rs, kDwTaps); }
-// one workgroup to a CU: as many parts of the positions as fill the chip once
+// one workgroup to a CU: as many parts of the positions as fill the chip once, and no more than that many turns each need
+// (784 turns are four to a part with 196 parts as with 256: a quarter of the partial sums less)
 int64_t dw_splits(int64_t c, int64_t k, int64_t rs, int64_t rows) {
   const int64_t turns = ceil_div(rows, kPos), want = 256 / dw_tiles(c, k, rs);
-  return want < 1 ? 1 : (want < turns ? want : turns);
+  return want < 1 ? 1 : ceil_div(turns, ceil_div(turns, want));
 }
 
 // ---- which convolutions: expected times of forward and both gradients, in microseconds -----------------------------------------
@@ -1065,7 +1077,10 @@ extern "C" int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* d
   if (int rc = check_launch("conv_taps_dw_kernel")) return rc;
   note_kernel("conv_dw:taps splits=%d", (int)splits);
   const unsigned blocks = (unsigned)ceil_div(r * s * c * k_out / 4, 16);
-  if (bf) hipLaunchKernelGGL((taps_dw_reduce<BF16>), dim3(blocks), dim3(256), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
-  else hipLaunchKernelGGL((taps_dw_reduce<F16>), dim3(blocks), dim3(256), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
+  auto reduce = [&](auto* kernel, unsigned share) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(16 * share), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
+  };
+  if (splits >= 128) bf ? reduce(&taps_dw_reduce<BF16, 64>, 64) : reduce(&taps_dw_reduce<F16, 64>, 64);
+  else bf ? reduce(&taps_dw_reduce<BF16, 16>, 16) : reduce(&taps_dw_reduce<F16, 16>, 16);
   return check_launch("taps_dw_reduce");
 }

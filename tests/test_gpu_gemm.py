@@ -690,3 +690,30 @@ def test_odd_multiples_of_32_on_ragged_and_model_shapes(M, N, K, bs):
     s = 1 / (1 - p)
     assert torch.equal(ext.gemm_dsd_lists(A, B, lists, 32, s), C)
     assert torch.equal(ext.gemm_sdd_lists(dC, B.T, lists, 32, s), dA)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (64, 64, 8192),       # few elements, many parts: sixteen threads to an element's parts
+    (256, 320, 4104),     # four
+    (384, 1536, 16384),   # one thread sums all parts
+    (77, 136, 6400),      # rows that end inside a thread's four elements' neighbourhood, an odd extent
+    (61, 23, 8192),       # a result whose size is no multiple of four
+])
+@pytest.mark.parametrize("trans_out", [False, True])
+def test_sums_of_a_split_reduction(M, N, K, trans_out):
+    """C = A^T B over a long reduction with scratch for its parts, into either majorness: fp32 sums rounded once, within one
+    rounding to fp16 (2^-11) of a double product plus the sums' own error (K * 2^-24 at most)."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    pad = lambda n: -(-n // 8) * 8
+    a = torch.randn(K, pad(M), generator=gen, device="cuda").half()[:, :M]
+    b = (torch.randn(K, pad(N), generator=gen, device="cuda") * K ** -0.5).half()[:, :N]
+    mask = torch.rand(K // 64 + (K % 64 > 0), -(-M // 64), generator=gen, device="cuda") < 0.3
+    lists = ext.build_lists(mask).transposed()
+    got = ext.gemm_dsd_lists(a.t(), b.t(), lists, 64, 2.0, transposed_out=trans_out)
+    assert int(ext.last_kernel_detail().rsplit("=", 1)[1]) > 1, ext.last_kernel_detail()
+    keep = (~mask).repeat_interleave(64, 0)[:K].repeat_interleave(64, 1)[:, :M]
+    want = 2.0 * ((a.double() * keep).t() @ b.double())
+    assert (got.double() - want).norm() <= (2.0 ** -11 + K * 2.0 ** -24) * want.norm()
