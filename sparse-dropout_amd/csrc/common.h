@@ -249,12 +249,21 @@ struct StoreLayout {
   }
 };
 
+// The pre-activations that store_eight<SDD> of the same position multiplies by, loaded ahead of it: the compiler may not
+// move a load above the store of the eight in front, so a lane that loads them in store_eight waits out a load for every
+// 16 bytes it stores.  Nothing is read (zeros) where store_eight does not take all eight at once.
+__device__ inline u32x4 aux_eight(const GemmArgs& g, const StoreLayout& s, int64_t si, int64_t ci) {
+  if (!(s.has_aux && s.aux_unit && s.unit && si < s.s_ext && ci + 8 <= s.c_ext)) return u32x4{0u, 0u, 0u, 0u};
+  return *reinterpret_cast<const u32x4_any*>(g.aux + si * s.ald + ci);
+}
+
 // Eight consecutive elements of C's contiguous index, unscaled fp32 accumulators: scaled, put through the fused
 // epilogue, rounded once and stored in one 16-byte piece (element by element at the matrix's edge).  si / ci: position
 // along C's strided / contiguous index (ci a multiple of 8).  part: fp32 partial sums of a split reduction go to `part`
-// (C's element order, unscaled) instead.
+// (C's element order, unscaled) instead.  pre: aux_eight of the position (SDD with an activation only).
 template <typename T, bool SDD>
-__device__ inline void store_eight(const GemmArgs& g, const StoreLayout& s, int64_t si, int64_t ci, float (&r)[8], float* part) {
+__device__ inline void store_eight(const GemmArgs& g, const StoreLayout& s, int64_t si, int64_t ci, float (&r)[8], float* part,
+                                   u32x4 pre) {
   if (si >= s.s_ext || ci >= s.c_ext) return;
   const int valid = s.c_ext - ci < 8 ? (int)(s.c_ext - ci) : 8;
   if (part) {
@@ -285,8 +294,7 @@ __device__ inline void store_eight(const GemmArgs& g, const StoreLayout& s, int6
   // without an activation) against a chain per element under its own execution mask, of 16384 x 1024 from 256 40 -> 33.
   if (g.act != SD_ACT_NONE) {
     if (SDD) {
-      const u32x4 a = *reinterpret_cast<const u32x4_any*>(g.aux + si * s.ald + ci);
-      const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+      const uint32_t w[4] = {pre.x, pre.y, pre.z, pre.w};
       float at[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) at[i] = T::to_float((uint16_t)(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu));
@@ -319,14 +327,21 @@ template <typename T, bool SDD, int ROWS, int COLS>
 __device__ inline void store_staged_tile(const GemmArgs& g, const float* stg, int lane, bool along_n, int64_t s0,
                                          int64_t c0, float* part) {
   constexpr int PITCH = COLS + 4, LPR = COLS / 8, RPP = 64 / LPR;  // lanes per row, rows per pass
+  constexpr int PASSES = ROWS / RPP, AHEAD = PASSES < 4 ? PASSES : 4;
   const StoreLayout s(g, along_n);
+  u32x4 pre[AHEAD] = {};
 #pragma unroll
-  for (int pass = 0; pass < ROWS / RPP; ++pass) {
+  for (int pass = 0; pass < PASSES; ++pass) {
     const int row = pass * RPP + lane / LPR, ch = lane % LPR;
+    if (SDD && s.has_aux && pass % AHEAD == 0) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i)
+        if (pass + i < PASSES) pre[i] = aux_eight(g, s, s0 + row + i * RPP, c0 + ch * 8);
+    }
     const f32x4 lo = *reinterpret_cast<const f32x4*>(stg + row * PITCH + ch * 8);
     const f32x4 hi = *reinterpret_cast<const f32x4*>(stg + row * PITCH + ch * 8 + 4);
     float r[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    store_eight<T, SDD>(g, s, s0 + row, c0 + ch * 8, r, part);
+    store_eight<T, SDD>(g, s, s0 + row, c0 + ch * 8, r, part, pre[pass % AHEAD]);
   }
 }
 
