@@ -141,6 +141,19 @@ inline double kept_blocks(const GemmArgs& g) {
   return g.quads ? 1.0 - none * none * none * none : hint;
 }
 
+// Whether, of both gradients in one launch, the weight gradient's workgroups (rows row blocks each, a reduction of w_kb blocks
+// in `splits` parts, w_wgs of them) come before the input gradient's (gx, x_wgs of them with anything kept).  Workgroups
+// start in their order, so the product with the longer chains of steps has to come first: otherwise those begin when the
+// others are done and run on with half of the chip empty.  64 x 64 tiles, dX and dW of 4096 x 1024 -> 1024 at p = 0.5 (16 steps
+// in 512 workgroups, 32 in 256) 30.3 -> 26.0 us, of 3136 x 1408 -> 256 at p = 0.4 23.8 -> 15.9; 128 x 128 ones, 2568 x 1472 -> 1136
+// at p = 0.25 40.7 -> 32.6.  With chains about as long, or where everything starts at once, the order is worth
+// nothing, or up to 9 % the other way (2024 x 1400 -> 1744 at p = 0.75).
+inline bool dw_before_dx(const GemmArgs& gx, double x_wgs, double w_kb, int rows, int splits, double w_wgs, double resident) {
+  double none = 1.0;  // of a reduction block in all of the rows
+  for (int r = 0; r < rows; ++r) none *= 1.0 - kept_blocks(gx);
+  return (1.0 - none) * w_kb / splits > 1.25 * ((gx.K + 63) / 64) && x_wgs + w_wgs > 0.5 * resident;
+}
+
 // Geometry of a convolution whose patch matrix the DSD kernel gathers itself (implicit GEMM):
 // x[n][c][h][w] with unit w stride, row block = 64 / Q whole output rows of one image.
 struct ImplicitConv {

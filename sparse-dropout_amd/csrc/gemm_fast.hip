@@ -1696,25 +1696,29 @@ __global__ __launch_bounds__(THREADS) void sdd_group_kernel(GemmArgs g, int tile
   sdd_any_body<T, EDGE, G>(g, tiles_m, gsure, Mb, Cb, (int)blockIdx.x);
 }
 
-// Both gradients of one layer in one launch: workgroups [0, n_dx) are the SDD product's (dX; those past its own
-// grid exit: n_dx is rounded up to the 8 XCDs so that the second product's tile map keeps its XCD assignment), the
-// rest the weight gradient's (DSD on reduction-strided operands, column-major C; a split reduction leaves fp32
-// partials for the reduce pass as in the kernel of its own).  One launch instead of
+// Both gradients of one layer in one launch: workgroups [0, n_first) are one product's (those past its own grid exit:
+// n_first is a multiple of 8, so that the second product's tile map keeps its XCD assignment), the rest the other's.  The
+// weight gradient (DSD on reduction-strided operands, column-major C; a split reduction leaves fp32 partials for the
+// reduce pass as in the kernel of its own) comes first where its chains are the longer ones (dw_before_dx).  One launch instead of
 // two, and the second product's workgroups fill the CUs the first one's last round leaves idle - for small layers,
 // whose grids cover a fraction of the chip each, the two simply run side by side.
 template <typename T, bool EDGE, typename G, typename S>
 __global__ __launch_bounds__(THREADS) void backward_pair_kernel(GemmArgs gx, int x_tiles_m, int x_gmax, int x_gsure,
-                                                                int x_Mb, int x_Cb, int n_dx, GemmArgs gw, int w_tiles_m,
-                                                                int w_tiles_n, int w_Mb, int w_Kb, int w_splits) {
+                                                                int x_Mb, int x_Cb, int n_first, bool dw_first,
+                                                                GemmArgs gw, int w_tiles_m, int w_tiles_n, int w_Mb,
+                                                                int w_Kb, int w_splits) {
   static_assert(S::THREADS == THREADS, "both products run on 512 threads");
   const int bid = (int)blockIdx.x;
-  if (bid < n_dx) {
-    if (bid < x_tiles_m * x_gmax) sdd_any_body<T, EDGE, G>(gx, x_tiles_m, x_gsure, x_Mb, x_Cb, bid);
+  const bool second = bid >= n_first;
+  const int i = second ? bid - n_first : bid;
+  if (second == dw_first) {
+    if (i < x_tiles_m * x_gmax) sdd_any_body<T, EDGE, G>(gx, x_tiles_m, x_gsure, x_Mb, x_Cb, i);
   } else {
     // the weight gradient's workgroups, tile index fastest, then the part of a split reduction
-    const int wb = bid - n_dx, w_tiles = w_tiles_m * w_tiles_n;
-    dsd_body<T, true, true, EDGE, S, 0>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, ImplicitConv{}, wb % w_tiles, w_splits,
-                                        wb / w_tiles);
+    const int w_tiles = w_tiles_m * w_tiles_n;
+    if (i < w_tiles * w_splits)
+      dsd_body<T, true, true, EDGE, S, 0>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, ImplicitConv{}, i % w_tiles, w_splits,
+                                          i / w_tiles);
   }
 }
 
@@ -2282,12 +2286,15 @@ int launch_pair_t(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_
     return rc;
   const int x_Mb = (int)((gx.M + BS - 1) / BS), x_Cb = (int)((gx.N + BS - 1) / BS);
   const int x_tiles_m = (x_Mb + G::R - 1) / G::R, x_gmax = sdd_most_groups(gx);
-  const int64_t n_dx = ((int64_t)x_tiles_m * x_gmax + 7) / 8 * 8;
+  const int64_t n_dx = (int64_t)x_tiles_m * x_gmax;
   const int w_Mb = (int)((gw.M + BS - 1) / BS), w_Kb = (int)((gw.K + BS - 1) / BS);
   const int w_tiles_m = (w_Mb + S::R - 1) / S::R, w_tiles_n = (int)((gw.N + S::BN - 1) / S::BN);
-  const int64_t total = n_dx + (int64_t)w_tiles_m * w_tiles_n * splits;
+  const int64_t n_dw = (int64_t)w_tiles_m * w_tiles_n * splits;
+  const bool dw_first = dw_before_dx(gx, (double)sdd_big_groups(gx), w_Kb, S::R, splits, (double)n_dw, 256);
+  const int64_t n_first = ((dw_first ? n_dw : n_dx) + 7) / 8 * 8, total = n_first + (dw_first ? n_dx : n_dw);
   hipLaunchKernelGGL((backward_pair_kernel<T, EDGE, G, S>), dim3((unsigned)total), dim3(THREADS), SMEM, stream, gx,
-                     x_tiles_m, x_gmax, sdd_sure_groups(gx), x_Mb, x_Cb, (int)n_dx, gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, splits);
+                     x_tiles_m, x_gmax, sdd_sure_groups(gx), x_Mb, x_Cb, (int)n_first, dw_first, gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb,
+                     splits);
   return check_launch("backward_pair_kernel");
 }
 

@@ -64,18 +64,20 @@ __global__ __launch_bounds__(S::THREADS) void tile_forward_kernel(GemmArgs g, in
   report_in(const_cast<uint64_t*>(f.job0.src.state), gridDim.x);
 }
 
-// Both gradients in one launch: workgroups [0, n_dx) are the input gradient's (a multiple of 8, so that the second
-// product's tile map keeps its XCD assignment), the rest the weight gradient's.
+// Both gradients in one launch: workgroups [0, n_first) are one product's, the rest the other's.  n_first is a multiple of 8, so
+// that the second product's tile map keeps its XCD assignment.  Which comes first: dw_before_dx.
 template <typename T, typename X, typename W>
 __global__ __launch_bounds__(W::THREADS) void tile_pair_kernel(GemmArgs gx, int x_tiles_n, int x_sure, int x_Mb, int x_Cb,
-                                                               int n_dx, GemmArgs gw, int w_tiles_m, int w_tiles_n,
-                                                               int w_Mb, int w_Kb, int w_splits) {
+                                                               int n_first, bool dw_first, GemmArgs gw, int w_tiles_m,
+                                                               int w_tiles_n, int w_Mb, int w_Kb, int w_splits) {
   static_assert(X::THREADS == W::THREADS, "both products run on the same number of threads");
   const int bid = (int)blockIdx.x;
-  if (bid < n_dx) {
-    if (bid < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_sure, x_Mb, x_Cb, bid);
+  const bool second = bid >= n_first;
+  const int i = second ? bid - n_first : bid;
+  if (second == dw_first) {
+    if (i < x_tiles_n * x_Mb) tile_sdd_body<T, X>(gx, x_sure, x_Mb, x_Cb, i);
   } else {
-    tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, bid - n_dx, w_splits);
+    if (i < w_tiles_m * w_tiles_n * w_splits) tile_dsd_body<T, false, true, W>(gw, w_tiles_m, w_tiles_n, w_Mb, w_Kb, i, w_splits);
   }
 }
 
@@ -153,10 +155,12 @@ int pair_launch(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_t 
   auto* kernel = &tile_pair_kernel<T, X, W>;
   if (int rc = allow_lds(reinterpret_cast<const void*>(kernel), SMEM, done)) return rc;
   const int x_Mb = blocks_of(gx.M), x_Cb = blocks_of(gx.N), x_tn = (x_Cb + X::C - 1) / X::C;
-  const int n_dx = (x_Mb * x_tn + 7) / 8 * 8;
   const int w_Mb = blocks_of(gw.M), w_Kb = blocks_of(gw.K), w_tm = (w_Mb + W::R - 1) / W::R, w_tn = (blocks_of(gw.N) + W::C - 1) / W::C;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_dx + w_tm * w_tn * splits)), dim3(W::THREADS), SMEM, stream, gx, x_tn,
-                     sure_strips(gx, X::C, x_tn), x_Mb, x_Cb, n_dx, gw, w_tm, w_tn, w_Mb, w_Kb, splits);
+  const int n_dx = x_Mb * x_tn, n_dw = w_tm * w_tn * splits;
+  const bool dw_first = dw_before_dx(gx, n_dx * kept_blocks(gx), blocks_of(gw.K), W::R, splits, n_dw, W::R == 1 ? 512 : 256);
+  const int n_first = ((dw_first ? n_dw : n_dx) + 7) / 8 * 8;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n_first + (dw_first ? n_dx : n_dw))), dim3(W::THREADS), SMEM, stream, gx, x_tn,
+                     sure_strips(gx, X::C, x_tn), x_Mb, x_Cb, n_first, dw_first, gw, w_tm, w_tn, w_Mb, w_Kb, splits);
   return check_launch("tile_pair_kernel");
 }
 

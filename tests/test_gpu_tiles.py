@@ -127,3 +127,63 @@ def test_more_small_tiles_than_are_resident(M, N, K, bs, dtype):
     ref = O.dsd_forward(to_np(x), to_np(w), mask.numpy(), bs, 0.4, np.float32)
     assert max_tile_rel_fro(y, ref) <= REL_FRO_TOL and torch.equal(y, again)
     assert max_tile_rel_fro(ext.gemm(x, w), to_np(x) @ to_np(w).T) <= REL_FRO_TOL
+
+
+@pytest.mark.parametrize("M,C,N,bs,shape", [
+    (65, 72, 64, 64, "auto"),       # strips of one: one past a tile, one step
+    (200, 61, 264, 32, "auto"),     # an odd width, whose last eight are stored one by one; quadrant bits
+    (4096, 6144, 256, 64, "auto"),  # strips of two
+    (530, 1029, 136, 64, "big"),    # groups of the large shape, ragged everywhere
+])
+@pytest.mark.parametrize("act", ["relu", "gelu"])
+def test_pre_activations_of_any_rows(M, C, N, bs, shape, act):
+    """The derivative at pre-activations that lie in rows of their own pitch and start, off every boundary: the bits of the
+    same ones in aligned rows, which are held to fp32 (one rounding to bf16, at most 2^-8 relative)."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator(device="cuda").manual_seed(M + C)
+    pad = -C % 8
+    dy = torch.randn(M, N, generator=gen, device="cuda").bfloat16()
+    w = torch.randn(N, C + pad, generator=gen, device="cuda").bfloat16()[:, :C]
+    at = torch.randn(M, C, generator=gen, device="cuda").bfloat16()
+    apart = torch.full((M, C + 3), float("nan"), dtype=torch.bfloat16, device="cuda")
+    apart[:, 1:1 + C] = at
+    mask = torch.rand(-(-M // bs), -(-C // bs), generator=gen, device="cuda") < 0.4
+    lists, kbs = (ext.build_lists(mask, 0 if bs == 32 else 1), bs)
+    before = ext.set_tile_policy(shape)
+    try:
+        got, other = (ext.gemm_sdd_lists_actgrad(dy, w.t(), lists, kbs, 1.5, act, a, keep_hint=0.6)
+                      for a in (at, apart[:, 1:1 + C]))
+    finally:
+        ext.set_tile_policy(before)
+    assert torch.equal(got, other)
+    t = at.float()
+    d = (t > 0).float() if act == "relu" else 0.5 * (1 + torch.erf(t * 0.5 ** 0.5)) + t * torch.exp(-0.5 * t * t) * 0.3989422804014327
+    keep = (~mask).repeat_interleave(bs, 0)[:M].repeat_interleave(bs, 1)[:, :C]
+    ref = 1.5 * (dy.float() @ w.float()) * d * keep
+    assert (got[~keep] == 0).all() and (got.float() - ref).norm() <= 2.0 ** -8 * ref.norm()
+
+
+@pytest.mark.parametrize("M,K,N,bs,p,shape", [
+    (2048, 200, 136, 64, 0.5, "one"),    # the weight gradient's chains are longer, its 12 workgroups no multiple of 8
+    (136, 200, 2056, 64, 0.5, "one"),    # the input gradient's
+    (1032, 1024, 784, 32, 0.6, "one"),   # about as long
+    (4040, 2048, 1000, 64, 0.1, "mid"),
+    (2048, 1096, 3064, 64, 0.25, "mid"),
+])
+def test_both_gradients_in_one_launch_in_either_order(M, K, N, bs, p, shape):
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(M + N + K)
+    x = make_operand(M, K, torch.float16, "cuda", gen=gen)
+    w = make_operand(N, K, torch.float16, "cuda", scale=K ** -0.5, gen=gen)
+    dy = make_operand(M, N, torch.float16, "cuda", gen=gen)
+    mask = cpu_mask(O.mask_shape(M, K, bs), p, gen)
+    _, _, lists, kbs = ext.dropout_matmul_forward(x, w, bs, p, mask=mask.cuda())
+    dx, dw = ext.dropout_matmul_backward(dy, w, x, lists, kbs, p)
+    assert ext.last_kernel_detail().startswith("pair:sdd+dsd:" + shape), ext.last_kernel_detail()
+    mk = mask.numpy()
+    assert max_tile_rel_fro(dx, O.sdd_dx(to_np(dy), to_np(w), mk, bs, p, np.float32)) <= REL_FRO_TOL
+    assert max_tile_rel_fro(dw, O.dsd_dw(to_np(dy), to_np(x), mk, bs, p, np.float32)) <= REL_FRO_TOL
