@@ -145,7 +145,7 @@ inline double kept_blocks(const GemmArgs& g) {
 // in `splits` parts, w_wgs of them) come before the input gradient's (gx, x_wgs of them with anything kept).  Workgroups
 // start in their order, so the product with the longer chains of steps has to come first: otherwise those begin when the
 // others are done and run on with half of the chip empty.  64 x 64 tiles, dX and dW of 4096 x 1024 -> 1024 at p = 0.5 (16 steps
-// in 512 workgroups, 32 in 256) 30.3 -> 26.0 us, of 3136 x 1408 -> 256 at p = 0.4 23.8 -> 15.9; 128 x 128 ones, 2568 x 1472 -> 1136
+// in 512 workgroups, 32 in 256) 30.3 -> 24.8 us, of 3136 x 1408 -> 256 at p = 0.4 23.8 -> 15.9; 128 x 128 ones, 2568 x 1472 -> 1136
 // at p = 0.25 40.7 -> 32.6.  With chains about as long, or where everything starts at once, the order is worth
 // nothing, or up to 9 % the other way (2024 x 1400 -> 1744 at p = 0.75).
 inline bool dw_before_dx(const GemmArgs& gx, double x_wgs, double w_kb, int rows, int splits, double w_wgs, double resident) {
