@@ -18,6 +18,7 @@
 //   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7, 192 a pass.
 //   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 5; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
 //   patch gradient 40, fold 52, dw 28 + 6, 227 a pass.
+#include <algorithm>
 #include <atomic>
 
 #include "common.h"
@@ -875,7 +876,10 @@ double expected_taps(const ConvShape& v) {
   // steps of a workgroup, and rounds of workgroups behind the first on every CU
   const double y_steps = pack.steps * narrow_k, dx_steps = (double)(rs * ceil_div(v.k, 64)) * narrow_k * narrow_c;
   auto behind = [](double wgs) { return wgs > 256.0 ? wgs / 256.0 - 1.0 : 0.0; };
-  const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = dw_splits(v.c, v.k, rs, (int64_t)rows);
+  // The parts that the fit counted: as many as fill the chip once.  dw_splits has since left out those that save no turn; counted here,
+  // they moved one convolution in 400 of those above to the tap-wise side, up to 13 % slower there (149 x 80 x 7 x 7 -> 192
+  // at p = 0.1: 88 us without, 100 tap by tap), and with it to other roundings of the input gradient.
+  const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = std::max<int64_t>(1, std::min(256 / tiles, turns));
   const double dw_turns = (double)(ceil_div(tiles * splits, 256) * ceil_div(turns, splits));
   return 32.7 + y_steps * (0.751 + 0.281 * behind((double)(turns * pack.groups))) +
          dx_steps * (0.849 + 0.864 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 2.8 * dw_turns +

@@ -339,6 +339,28 @@ def test_tap_by_tap_only_where_it_is_expected_to_be_faster(layer, p, taken):
     assert lib.sd_conv2d_taps_taken_blocks(*geo, p, 64) == int(taken)
 
 
+@pytest.mark.parametrize("layer,p,bs", [
+    ((149, 80, 7, 7, 192, 3), 0.1, 64),    # 88 us without, 100 tap by tap
+    ((50, 16, 30, 30, 216, 5), 0.75, 128),  # 156, 170
+    ((221, 56, 7, 7, 152, 3), 0.1, 64),     # 80, 89
+    ((92, 64, 14, 14, 72, 3), 0.75, 64),    # 71, 77
+    ((25, 32, 30, 30, 152, 3), 0.75, 128),  # 85, 70: on the other side of the rule's error
+    ((22, 40, 30, 30, 128, 3), 0.5, 64),
+])
+def test_how_a_weight_gradient_is_cut_moves_no_convolution_to_another_route(layer, p, bs):
+    """Which route a layer takes decides how its input gradient is rounded: the rule counts the parts that it was fitted with, not
+    those that the weight gradient's launch leaves out because they save no turn."""
+    from flash_dropout.hip import GEMM
+
+    n, c, h, w, k, r = layer
+    geo = (n, c, h, w, k, r, r, r // 2, r // 2, 1, 1, 1, 1)
+    lib, rows = GEMM().lib, n * h * w
+    want = max(1, 256 // (-(-c // 32) * -(-k // 64) * -(-r * r // 9)))
+    parts = lib.sd_conv2d_taps_dw_workspace_bytes(c, k, r, r, rows) // (4 * r * r * c * k)
+    assert parts < min(want, -(-rows // 256))  # a layer of which parts are left out
+    assert lib.sd_conv2d_taps_fits(*geo) == 1 and lib.sd_conv2d_taps_taken_blocks(*geo, p, bs) == 0
+
+
 def test_larger_blocks_cost_the_other_routes_more():
     """They spread such a mask over 64-blocks first: 10 x 40 x 32 x 32 -> 168 at p = 0.05 takes 94 us there in blocks of 128, 79
     tap by tap."""
