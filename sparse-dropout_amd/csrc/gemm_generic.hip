@@ -266,36 +266,59 @@ __global__ __launch_bounds__(THREADS) void gemm_generic_kernel(GemmArgs g, int t
 }
 
 // C = scale * sum over splits of the fp32 partial tiles.  A thread takes four elements of C's contiguous order (the workspace is
-// laid out the same way) as one 16-byte load per split and stores them as one 8-byte piece; SHARE threads share out the
-// splits of the same four, and their sums meet in LDS.  Bound by the loads and their latency.  With four threads to the splits
-// everywhere, 64-bit divisions and a 2-byte store per element the parts of 384 x 1536 over 16384 rows took 6.8 us, now 5.2; of
-// 64 x 384 over 10944 4.3, now 3.5.
+// laid out the same way) as one 16-byte load per split and stores them as one 8-byte piece.  Four chains add an element's splits
+// up, chain w the splits w, w + 4, ... in order, then the chains are added in order: all four in one thread (SHARE = 1) or in four
+// threads whose sums meet in LDS (SHARE = 4), with the same bits.  No chain is longer than a quarter of the splits.
+// Bound by the loads and their latency.  With four threads to the splits everywhere, 64-bit divisions and a 2-byte store per element
+// the sum of 7 parts of 384 x 1536 took 4.8 us, now 3.3; of 13 of 64 x 384 3.3, now 2.6; of 8 of 1024 x 4096 22.5, now 21.7.
 template <typename T, int SHARE>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs g, int splits, bool trans) {
   constexpr int OWN = 256 / SHARE;  // threads with elements of their own
-  __shared__ f32x4 part[SHARE > 1 ? SHARE - 1 : 1][OWN];
+  constexpr int CHAINS = 4;
+  static_assert(SHARE == 1 || SHARE == CHAINS, "all chains or one");
+  __shared__ f32x4 part[SHARE > 1 ? CHAINS - 1 : 1][OWN];
   const uint32_t total = (uint32_t)(g.M * g.N), c_ext = (uint32_t)(trans ? g.M : g.N);
-  const uint32_t own = threadIdx.x % OWN, share = threadIdx.x / OWN;
+  const uint32_t own = threadIdx.x % OWN;
+  const int share = SHARE == 1 ? 0 : (int)(threadIdx.x / OWN);
   const uint32_t e0 = (blockIdx.x * OWN + own) * 4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (total % 4 == 0) {
-    if (e0 < total) {
-      const float* src = g.ws + e0;
-#pragma unroll 8
-      for (int s = (int)share; s < splits; s += SHARE) acc += *reinterpret_cast<const f32x4*>(src + (int64_t)s * total);
-    }
-  } else {
-    for (int s = (int)share; s < splits; s += SHARE)
+  f32x4 chain[CHAINS / SHARE] = {};
+  auto add_up = [&](auto load) {
+    int s = share;
+    if constexpr (SHARE == 1) {
+#pragma unroll 2
+      for (; s + CHAINS <= splits; s += CHAINS) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (e0 + v < total) acc[v] += g.ws[(int64_t)s * total + e0 + v];
+        for (int w = 0; w < CHAINS; ++w) chain[w] += load(s + w);
+      }
+#pragma unroll
+      for (int w = 0; w < CHAINS - 1; ++w)
+        if (s + w < splits) chain[w] += load(s + w);
+    } else {
+#pragma unroll 8
+      for (; s < splits; s += CHAINS) chain[0] += load(s);
+    }
+  };
+  typedef f32x4 __attribute__((aligned(4))) f32x4_any;  // where M * N is no multiple of four, parts start anywhere
+  const float* src = g.ws + e0;
+  if (e0 + 4 <= total) {
+    add_up([&](int s) -> f32x4 { return *reinterpret_cast<const f32x4_any*>(src + (int64_t)s * total); });
+  } else {
+    add_up([&](int s) {
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 4 && e0 + i < total; ++i) v[i] = src[(int64_t)s * total + i];
+      return v;
+    });
   }
-  if (SHARE > 1) {
+  f32x4 acc = chain[0];
+  if constexpr (SHARE > 1) {
     if (share > 0) part[share - 1][own] = acc;
     __syncthreads();
     if (share > 0) return;
 #pragma unroll
-    for (int i = 0; i < SHARE - 1; ++i) acc += part[i][own];
+    for (int w = 1; w < CHAINS; ++w) acc += part[w - 1][own];
+  } else {
+#pragma unroll
+    for (int w = 1; w < CHAINS; ++w) acc += chain[w];
   }
   if (e0 >= total) return;
   uint32_t si = e0 / c_ext, ci = e0 - si * c_ext;
@@ -376,14 +399,14 @@ void reduce_shared(const GemmArgs& g, int splits, bool trans_out, int dtype, hip
 }
 }  // namespace
 
-// (Partial sums take at most 256 MiB: element numbers are 32-bit.)  As few threads to an element's splits as still give every CU a
-// workgroup, and at least two splits to each.
+// (Partial sums take at most 256 MiB: element numbers are 32-bit.)  A thread for all of an element's splits where that gives every CU
+// a workgroup; fewer elements are better off with four (7 parts of 64 x 64: 2.6 and 2.4 us; 7 of 77 x 131 4.8 and 3.2), and so are many
+// splits of large results, whose parts come from outside the caches (8 of 1024 x 4096: 25.5 and 21.7; 4 of 2048 x 1024 5.2 and 6.5).
 int launch_splitk_reduce(const GemmArgs& g, int splits, bool trans_out, int dtype, hipStream_t stream) {
   if (g.M * g.N >= (int64_t)1 << 31) return fail(SD_ERR_INVALID, "splitk_reduce: result too large");
   const int64_t quads = ceil_div(g.M * g.N, 4);
-  if (quads >= 256 * 256 || splits < 8) reduce_shared<1>(g, splits, trans_out, dtype, stream);
-  else if (quads >= 256 * 64 || splits < 32) reduce_shared<4>(g, splits, trans_out, dtype, stream);
-  else reduce_shared<16>(g, splits, trans_out, dtype, stream);
+  if (quads >= 256 * 256 && (quads < 1 << 19 || quads * splits < 1 << 22)) reduce_shared<1>(g, splits, trans_out, dtype, stream);
+  else reduce_shared<4>(g, splits, trans_out, dtype, stream);
   return check_launch("splitk_reduce");
 }
 

@@ -693,8 +693,8 @@ def test_odd_multiples_of_32_on_ragged_and_model_shapes(M, N, K, bs):
 
 
 @pytest.mark.parametrize("M,N,K", [
-    (64, 64, 8192),       # few elements, many parts: sixteen threads to an element's parts
-    (256, 320, 4104),     # four
+    (64, 64, 8192),       # few elements, many parts: four threads to an element's parts
+    (256, 320, 4104),
     (384, 1536, 16384),   # one thread sums all parts
     (77, 136, 6400),      # rows that end inside a thread's four elements' neighbourhood, an odd extent
     (61, 23, 8192),       # a result whose size is no multiple of four
@@ -717,3 +717,41 @@ def test_sums_of_a_split_reduction(M, N, K, trans_out):
     keep = (~mask).repeat_interleave(64, 0)[:K].repeat_interleave(64, 1)[:, :M]
     want = 2.0 * ((a.double() * keep).t() @ b.double())
     assert (got.double() - want).norm() <= (2.0 ** -11 + K * 2.0 ** -24) * want.norm()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (64, 64, 8192),       # four threads to an element's parts
+    (384, 1536, 16384),   # one thread
+    (61, 23, 8192),       # parts that start off 16-byte boundaries
+])
+def test_order_in_which_parts_are_added_up(M, N, K):
+    """Bit for bit four chains, chain w the parts w, w + 4, ... in order, then the chains in order, however many threads share them:
+    every part holds one exact product, 2^25, its negative or a small integer, whose fp32 sums depend on the order."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(M + N)
+    pad, blocks = lambda n: -(-n // 8) * 8, K // 64
+    a, b = torch.zeros(K, pad(M)).half(), torch.zeros(K, pad(N)).half()
+    lists = ext.build_lists(torch.zeros(blocks, -(-M // 64), dtype=torch.bool, device="cuda")).transposed()
+    product = lambda: ext.gemm_dsd_lists(a.cuda()[:, :M].t(), b.cuda()[:, :N].t(), lists, 64, 1.0, transposed_out=True)
+    product()
+    parts = int(ext.last_kernel_detail().rsplit("=", 1)[1])
+    assert parts > 4, ext.last_kernel_detail()
+    values = torch.randint(-15, 16, (parts, N), generator=gen).float()
+    for n in range(N):  # a third of the parts or so are large and cancel in pairs
+        at = torch.randperm(parts, generator=gen)[: parts // 3 // 2 * 2 or 2]
+        values[at, n] = 2.0 ** 25 * (1.0 - 2.0 * (torch.arange(len(at)) % 2))
+    for i in range(parts):
+        row = blocks * i // parts * 64 + 5
+        a[row, :M] = 1024.0
+        b[row, :N] = (values[i] / 1024.0).half()
+    chains = [torch.zeros(N) for _ in range(4)]
+    for i in range(parts):
+        chains[i % 4] = chains[i % 4] + values[i]
+    want = ((chains[0] + chains[1]) + chains[2]) + chains[3]
+    serial = torch.zeros(N)
+    for i in range(parts):
+        serial = serial + values[i]
+    assert not torch.equal(want, serial)
+    assert torch.equal(product().cpu().float(), want.expand(M, N))
