@@ -1826,7 +1826,7 @@ constexpr ShapeCost kGradientCost[4] = {{2,       4.79,  {0.26, 0.45, 0.},   0.,
 constexpr ShapeCost kSddCost[4] = {     {2,       4.22,  {0.24, 0.40, 0.},   0.,   0.,   4.07, 1.69, 2.82, 0.29},
                                         {1,       5.47,  {0.46, 0., 0.},     0.,   0.,   4.51, 2.28, 4.83, 0.19},
                                         {3,       4.73,  {0.52, 0.61, 0.85}, 0.,   0.,   2.03, 1.44, 3.09, 0.24},
-                                        {1,       14.00, {1.20, 0., 0.},     0.,   6.50, 1.64, 3.26, 5.49, 0.22}};
+                                        {1,       14.19, {1.20, 0., 0.},     0.,   0.,   2.52, 3.26, 5.49, 0.24}};
 
 // A product on a shape: workgroups, steps of one of them, and what it costs beside them.
 struct ShapeWork {
@@ -1909,7 +1909,7 @@ double sdd_row_groups(const GemmArgs& g) {
   const double any = Cb * (1.0 - n * n * n * n), two = Cb * k * k * k * (4.0 * n + k);
   return std::min((double)sdd_most_groups(g), std::max(1.0, 0.5 + std::max(any / 6.0, (any + two) / 8.0)));
 }
-// workgroups the big SDD shape is expected to have
+// workgroups the big SDD shape is expected to have (plan_sdd counts with sdd_plan_groups)
 int64_t sdd_big_groups(const GemmArgs& g) { return (int64_t)((double)((blocks_of(g.M) + 3) / 4) * sdd_row_groups(g) + 0.5); }
 // Whether the workgroups count the groups of all row quads (find_group): where the groups expected nearly fill their last round, so
 // that an engine with one or two more than others takes another, and a round is long against the 4 to 5 us that each
@@ -1948,28 +1948,44 @@ bool sdd_big_ok(const GemmArgs& g) {
          blocks_of(g.N) <= G_MAX_CB;
 }
 
-// Workgroups of an SDD strip shape that are expected to have kept tiles.
+// Which shape an input gradient runs on decides its last bits: the strips add the two halves of each 64-deep step up by themselves and
+// their sums once, the big shape has one running sum, and in a stack a hidden layer's last bits grow to 2e-4 of the next gradients.
+// So the shapes are chosen by the figures of the fit below, in which strips of one row lay next to each other, kept ones first, and
+// groups were cut greedily along a row, though both are dealt out evenly by now (group_of_block, deal_group).  Counted as they are
+// now, with the fit made again, 14 of 900 drawn layers and stacks changed their bits and took 0.6 to 1.0 of the time.
+
+// Workgroups of the big SDD shape that the fit counted: a group spans 4 column blocks with everything kept, 6 once few enough
+// tiles are kept for the width and not the tile count to end a group.
+int64_t sdd_plan_groups(const GemmArgs& g) {
+  const int64_t cols = kept_fraction(g) <= 0.3f ? SddBig::GW : SddBig::MINCOLS;
+  return ((blocks_of(g.M) + 3) / 4) * ((blocks_of(g.N) + cols - 1) / cols);
+}
+// Workgroups of an SDD strip shape that the fit counted: eight times as many with kept tiles as the XCD with the most of them got, an
+// XCD taking a contiguous eighth of an order that walked eight rows at a time.
 double busy_strips(const GemmArgs& g, int cols, double keep) {
   const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), per_row = (double)((blocks_of(g.N) + cols - 1) / cols);
-  if (keep > 0.999) return Mb * per_row;
-  const double kept = Cb * keep / cols + (cols - 1) / (2.0 * cols);  // a row's kept tiles end inside its last strip
-  return Mb * std::min(std::max(kept, std::min(1.0, Cb * keep)), per_row);
+  const double grid = Mb * per_row;
+  if (keep > 0.999) return grid;
+  double kept = Cb * keep / cols + (cols - 1) / (2.0 * cols);  // a row's kept tiles end inside its last strip
+  kept = std::min(std::max(kept, std::min(1.0, Cb * keep)), per_row);
+  const double walk = 8.0 * per_row, run = grid / 8.0, whole = (double)(int64_t)(run / walk);
+  return std::max(1.0, std::min(grid, 8.0 * (whole * 8.0 * kept + std::min(run - whole * walk, 8.0 * kept))));
 }
 
 // The SDD product on a shape: its kept tiles in strips of one, four or two, or groups of the big shape.
 ShapeWork sdd_work(int shape, const GemmArgs& g) {
   const double Mb = (double)blocks_of(g.M), Cb = (double)blocks_of(g.N), keep = kept_blocks(g);
   ShapeWork w{kSddCost[shape], 0., 0., 0.};
-  w.wgs = shape == kShapeBig ? (double)sdd_big_groups(g) : busy_strips(g, shape == kShapeOne ? 1 : (shape == kShapeQuad ? 4 : 2), keep);
+  w.wgs = shape == kShapeBig ? (double)sdd_plan_groups(g) : busy_strips(g, shape == kShapeOne ? 1 : (shape == kShapeQuad ? 4 : 2), keep);
   double extra = g.N % BS || g.K % BS ? w.cost.ragged : 0.0;
   if (shape == kShapeBig) {
-    w.steps = (double)blocks_of(g.K) * (0.892 + 0.085 * keep);  // groups of more column blocks, fewer of their tiles kept
+    w.steps = (double)blocks_of(g.K) * (0.8 + 0.28 * keep);  // groups of more column blocks, fewer of their tiles kept
   } else {
     // Rows that end anywhere cost the strips more the more W there is (log2 of its megabytes), tile rows lying across 128-byte
     // lines; and past 24 MB of W every row's strips fetch their own columns from outside the caches, which strips of two
     // do twice as often for a row of dY as strips of four (6656 x 6736 from 7008, ragged, p = 0.1: 1474 us; 635 on the big shape).
     const double mb = std::log2((double)g.N * (double)g.K * 2e-6), cold = std::max(0.0, mb - 4.5);
-    const double each = shape == kShapeWide ? 0.22 - 0.12 * keep + (extra > 0.0 ? 0.16 : 0.0) : (shape == kShapeQuad ? 0.13 : 0.2);
+    const double each = shape == kShapeWide ? 0.22 - 0.12 * keep + (extra > 0.0 ? 0.16 : 0.0) : (shape == kShapeQuad ? 0.1 : 0.2);
     extra = extra * (0.6 + 0.25 * std::min(std::max(mb, 0.0), 4.0)) + cold * each;
     w.steps = (double)blocks_of(g.K);
   }
@@ -1978,19 +1994,18 @@ ShapeWork sdd_work(int shape, const GemmArgs& g) {
   return w;
 }
 
-// The shape with the smallest expected time.  Over 2000 drawn layers timed on all four (128 to 16384 rows, 128 to 8192 columns and
-// reductions of 64 to 8192, p of 0.05 to 0.75) it is 1.0 % over the best one on average on reductions of four blocks and more, one in
-// fifty 17 %; the figures of the strips are older, those of the big shape were fitted to these when its groups were dealt out.
-// Reductions of less than four blocks go to the strips whatever is expected: what counts there is how many stores and first loads a CU
-// has on their way (5632 x 4672 from 128 at p = 0.6: strips of two 17.1 us, big shape 31.8; 2560 x 7744 from 64 at 0.3: 15.9, 27.6).
-// Nearly dense ones on whole blocks keep the big shape they always had when its grid gives more than half of the CUs a workgroup
-// (the suite pins it), where strips would gain less: 3456 x 3200 from 128 at p = 0.1 13.0 us, 16.7.
+// The shape with the smallest expected time: when it was fitted 1.5 % over the best one on average on reductions of four blocks and
+// more (1.6 % on 900 layers drawn afterwards).  The rules before (limits on the number of groups, of kept tiles and of strips, and a
+// formula for strips of two on reductions of 256 to 4096) were 8.5 % over it, one in ten 30 % or more, most of them ragged (33 %
+// on average above 4e10 products): dX of 11904 x 6344 from 6112 at p = 0.2 with GELU 2173 us on strips, 920 on the big shape.
+// Shorter reductions keep their bits on the big shape when its grid gives more than half of the CUs a workgroup; strips are
+// faster there (5632 x 4672 from 128 at p = 0.6: strips of two 17.1 us, big shape 31.8).
 int plan_sdd(const GemmArgs& g) {
   const int policy = tile_policy.load(std::memory_order_relaxed);
+  const bool ragged = g.N % BS || g.K % BS, brief = blocks_of(g.K) < 4;
   const bool big = sdd_big_ok(g);
   if (policy == kTileMid) return kShapeWide;
-  const bool brief = blocks_of(g.K) < 4, dense = kept_blocks(g) > 0.85 && g.N % BS == 0 && g.K % BS == 0;
-  if (big && (policy == kTileBig || (brief && dense && sdd_big_groups(g) > 128))) return kShapeBig;
+  if (big && (policy == kTileBig || (brief && !ragged && sdd_plan_groups(g) > 128))) return kShapeBig;
   int best = kShapeOne;
   for (int shape = kShapeQuad; shape <= (big && !brief ? kShapeBig : kShapeWide); ++shape)
     if (sdd_work(shape, g).time() < sdd_work(best, g).time()) best = shape;
@@ -2330,7 +2345,7 @@ int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipS
   const double apart = w_work(plan.shape).time() + sdd_work(x_alone, gx).time();
   if (big) {
     if (!sdd_big_ok(gx) || (x_alone != kShapeBig && (blocks_of(gx.K) < 4 || pair_time(kShapeBig) > apart)) ||
-        sdd_big_groups(gx) > limit || shape_tiles(kShapeBig, gw.M, gw.N) * plan.splits > limit)
+        sdd_plan_groups(gx) > limit || shape_tiles(kShapeBig, gw.M, gw.N) * plan.splits > limit)
       return SD_ERR_UNSUPPORTED;
     const bool edge = gx.N % BS != 0 || gx.K % BS != 0 || form.ragged;
     int rc;

@@ -565,6 +565,39 @@ def test_sdd_shape_choice_follows_the_keep_hint_not_the_scale(tile_policy):
         ext.gemm_sdd_lists(dC, B, lists, 64, 1.0, keep_hint=1.5)
 
 
+@pytest.mark.parametrize("M,N,K,p,shape", [
+    (15424, 5184, 128, 0.6, "big"),       # short reductions on whole blocks
+    (2752, 7232, 192, 0.3, "big"),
+    (14851, 1472, 128, 0.5, "big"),
+    (560, 7936, 1984, 0.3, "mid"),
+    (14592, 6912, 1728, 0.5, "mid"),
+    (6208, 7424, 1856, 0.6, "mid"),
+    (14976, 3072, 768, 0.5, "mid"),
+    (2702, 3328, 4864, 0.75, "small"),
+])
+def test_input_gradients_keep_the_shape_that_their_bits_come_from(M, N, K, p, shape, tile_policy):
+    """How groups and strips are dealt out moves no input gradient between the big shape, one running sum per element, and the
+    strips, two sums over the depth: layers whose choice is near, and the two shapes' last bits do differ."""
+    if tile_policy != "auto":
+        pytest.skip("the choice under test is the automatic one")
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    dy = torch.randn(M, K, generator=gen, device="cuda").half()
+    w = torch.randn(K, N, generator=gen, device="cuda").half()
+    lists = ext.build_lists(torch.rand(-(-M // 64), -(-N // 64), generator=gen, device="cuda") < p)
+    got = ext.gemm_sdd_lists(dy, w.t(), lists, 64, 1.0, keep_hint=1 - p)
+    assert ext.last_kernel_detail() == "sdd:" + shape
+    before = ext.set_tile_policy("mid" if shape == "big" else "big")
+    try:
+        other = ext.gemm_sdd_lists(dy, w.t(), lists, 64, 1.0)
+    finally:
+        ext.set_tile_policy(before)
+    assert not torch.equal(got, other)
+    assert (got.float() - other.float()).norm() <= 2.0 ** -11 * got.float().norm()
+
+
 @pytest.mark.parametrize("M,N,K", [(512, 256, 576), (1000, 128, 200), (4096, 64, 4104)])
 def test_sdd_kept_only_leaves_dropped_tiles_untouched(M, N, K):
     """sd_gemm_sdd_lists_kept: kept tiles equal the ordinary call's, dropped tiles keep what the buffer held."""
