@@ -18,7 +18,6 @@
 //   (implicit), rows of dy 11, dx 73 (products and fold), dw 49 + 7, 192 a pass.
 //   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 5; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
 //   patch gradient 40, fold 52, dw 28 + 6, 227 a pass.
-#include <algorithm>
 #include <atomic>
 
 #include "common.h"
@@ -748,30 +747,33 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 }
 
 // dw[k, c * R * S + t] = scale * sum over the splits of part[split][t][c][k]: four outputs per thread, the splits shared out
-// over SHARE threads.  Bound by the latency of the loads where the result is small: 256 parts of 288 x 64 over 16 threads 7.6 us, 196
-// over 64 5.3.
-template <typename T, int SHARE>
-__global__ __launch_bounds__(16 * SHARE) void taps_dw_reduce(const float* part, uint16_t* dw, int64_t dw_ld, int C, int K, int RS,
-                                                             int splits, float scale) {
-  __shared__ f32x4 lds[SHARE][16];
+// over 16 threads, each of which adds every sixteenth in order; then the sixteen are added in order.  Bound by the loads and their
+// latency, so a thread has AHEAD on their way at once (what is past the last split adds zeros): 256 parts of 288 x 64 with eight 5.1 us,
+// with one 7.5; 14 parts of 2200 x 112, at most one to a thread, 5.7 and 4.8.  More threads would make other, shorter chains and
+// with them other last bits.
+template <typename T, int AHEAD>
+__global__ __launch_bounds__(256) void taps_dw_reduce(const float* part, uint16_t* dw, int64_t dw_ld, int C, int K, int RS, int splits,
+                                                      float scale) {
+  __shared__ f32x4 lds[16][16];
   const int64_t n4 = (int64_t)RS * C * K / 4;
   const int own = threadIdx.x % 16, q = threadIdx.x / 16;
   const int64_t o = (int64_t)blockIdx.x * 16 + own;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   if (o < n4) {
-#pragma unroll 4
-    for (int i = q; i < splits; i += SHARE) s += *reinterpret_cast<const f32x4*>(part + ((int64_t)i * n4 + o) * 4);
+    for (int i0 = q; i0 < splits; i0 += 16 * AHEAD) {
+      f32x4 v[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        const int i = i0 + 16 * j;
+        v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (i < splits) v[j] = *reinterpret_cast<const f32x4*>(part + ((int64_t)i * n4 + o) * 4);
+      }
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) s += v[j];
+    }
   }
   lds[q][own] = s;
   __syncthreads();
-  if (SHARE > 16) {
-    if (q < 16) {
-#pragma unroll
-      for (int i = 16; i < SHARE; i += 16) s += lds[i + q][own];
-      lds[q][own] = s;
-    }
-    __syncthreads();
-  }
   if (q != 0 || o >= n4) return;
 #pragma unroll
   for (int i = 1; i < 16; ++i) s += lds[i][own];
@@ -852,11 +854,12 @@ ConvShape shape_of(int64_t n, int64_t c, int64_t h, int64_t w, int64_t k, int64_
 }
 
 int64_t dw_tiles(int64_t c, int64_t k, int64_t rs) { return ceil_div(c, 32) * ceil_div(k, 64) * ceil_div(rs, kDwTaps); }
-// one workgroup to a CU: as many parts of the positions as fill the chip once, and no more than that many turns each need
-// (784 turns are four to a part with 196 parts as with 256: a quarter of the partial sums less)
+// One workgroup to a CU: as many parts of the positions as fill the chip once.  Where a sum is cut decides its last bits, and the rule
+// below was fitted to these parts: fewer, where they take no more turns each (784 turns are four to a part with 196 parts as
+// with 256), would change both.
 int64_t dw_splits(int64_t c, int64_t k, int64_t rs, int64_t rows) {
   const int64_t turns = ceil_div(rows, kPos), want = 256 / dw_tiles(c, k, rs);
-  return want < 1 ? 1 : ceil_div(turns, ceil_div(turns, want));
+  return want < 1 ? 1 : (want < turns ? want : turns);
 }
 
 // ---- which convolutions: expected times of forward and both gradients, in microseconds -----------------------------------------
@@ -876,10 +879,7 @@ double expected_taps(const ConvShape& v) {
   // steps of a workgroup, and rounds of workgroups behind the first on every CU
   const double y_steps = pack.steps * narrow_k, dx_steps = (double)(rs * ceil_div(v.k, 64)) * narrow_k * narrow_c;
   auto behind = [](double wgs) { return wgs > 256.0 ? wgs / 256.0 - 1.0 : 0.0; };
-  // The parts that the fit counted: as many as fill the chip once.  dw_splits has since left out those that save no turn; counted here,
-  // they moved one convolution in 400 of those above to the tap-wise side, up to 13 % slower there (149 x 80 x 7 x 7 -> 192
-  // at p = 0.1: 88 us without, 100 tap by tap), and with it to other roundings of the input gradient.
-  const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = std::max<int64_t>(1, std::min(256 / tiles, turns));
+  const int64_t tiles = dw_tiles(v.c, v.k, rs), splits = dw_splits(v.c, v.k, rs, (int64_t)rows);
   const double dw_turns = (double)(ceil_div(tiles * splits, 256) * ceil_div(turns, splits));
   return 32.7 + y_steps * (0.751 + 0.281 * behind((double)(turns * pack.groups))) +
          dx_steps * (0.849 + 0.864 * behind((double)(ceil_div((int64_t)pixels, kPos) * ceil_div(v.c, 64)))) + 2.8 * dw_turns +
@@ -1081,10 +1081,10 @@ extern "C" int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* d
   if (int rc = check_launch("conv_taps_dw_kernel")) return rc;
   note_kernel("conv_dw:taps splits=%d", (int)splits);
   const unsigned blocks = (unsigned)ceil_div(r * s * c * k_out / 4, 16);
-  auto reduce = [&](auto* kernel, unsigned share) {
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(16 * share), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
+  auto reduce = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
   };
-  if (splits >= 128) bf ? reduce(&taps_dw_reduce<BF16, 64>, 64) : reduce(&taps_dw_reduce<F16, 64>, 64);
-  else bf ? reduce(&taps_dw_reduce<BF16, 16>, 16) : reduce(&taps_dw_reduce<F16, 16>, 16);
+  if (splits > 32) bf ? reduce(&taps_dw_reduce<BF16, 8>) : reduce(&taps_dw_reduce<F16, 8>);
+  else bf ? reduce(&taps_dw_reduce<BF16, 1>) : reduce(&taps_dw_reduce<F16, 1>);
   return check_launch("taps_dw_reduce");
 }

@@ -244,3 +244,40 @@ def test_gradients_that_are_not_finite_reach_kept_blocks_only(geom, bad):
     reached[at[1]] = ~mask[at[0] // 64].repeat_interleave(64)[: c * r * s]
     assert torch.equal(~torch.isfinite(got[1]), reached)
     assert torch.equal(got[1][~reached], got[0][~reached])
+
+
+@pytest.mark.parametrize("geom", [
+    (256, 32, 28, 28, 64, 3, 3, (1, 1), (1, 1)),  # 784 turns in 256 parts, three or four each
+    (24, 64, 32, 32, 64, 3, 3, (1, 1), (1, 1)),   # 96 in 96 of at most 128
+    (35, 72, 16, 20, 200, 3, 3, (1, 1), (1, 1)),  # 44 in 21
+])
+def test_order_in_which_a_weight_gradients_parts_are_added_up(geom):
+    """Bit for bit: as many parts as fill the chip once, sixteen chains, chain j the parts j, j + 16, ... in order, then the chains in
+    order.  Every part holds one exact product at the middle tap, 2^25, its negative or a small integer, whose fp32 sums
+    depend on the order."""
+    n, c, h, w, k, r, s, pad, dil = geom
+    rows, gen = n * h * w, torch.Generator().manual_seed(k)
+    turns, tiles = -(-rows // 256), -(-c // 32) * -(-k // 64)
+    parts = min(256 // tiles, turns)
+    first = [i * (turns // parts) + min(i, turns % parts) for i in range(parts)]
+    values = torch.randint(-15, 16, (parts, k), generator=gen).float()
+    for j in range(k):
+        at = torch.randperm(parts, generator=gen)[: parts // 4 * 2]
+        values[at, j] = 2.0 ** 25 * (1.0 - 2.0 * (torch.arange(len(at)) % 2))
+    x, dy = torch.zeros(n, c, h * w).half(), torch.zeros(n, k, h * w).half()
+    for i, turn in enumerate(first):
+        img, at = divmod(turn * 256 + 100, h * w)
+        x[img, :, at] = 1024.0
+        dy[img, :, at] = (values[i] / 1024.0).half()
+    wt = torch.zeros(k, c, r, s).half()
+    mask = torch.zeros(O.mask_shape(rows, c * r * s, 64), dtype=torch.bool)
+    dw = _products(geom, x.view(n, c, h, w), wt, dy.view(n, k, h, w), mask, 64, 1.0)[2].cpu().reshape(k, c, r * s)
+    def in_order(terms):
+        total = torch.zeros(k)
+        for t in terms:
+            total = total + t
+        return total
+    want = in_order([in_order(values[j::16]) for j in range(16)])
+    for other in (in_order(values), in_order([in_order(values[j::64]) for j in range(64)])):
+        assert not torch.equal(want, other)
+    assert torch.equal(dw[:, :, 4].float(), want[:, None].expand(k, c))

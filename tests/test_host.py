@@ -348,8 +348,8 @@ def test_tap_by_tap_only_where_it_is_expected_to_be_faster(layer, p, taken):
     ((22, 40, 30, 30, 128, 3), 0.5, 64),
 ])
 def test_how_a_weight_gradient_is_cut_moves_no_convolution_to_another_route(layer, p, bs):
-    """Which route a layer takes decides how its input gradient is rounded: the rule counts the parts that it was fitted with, not
-    those that the weight gradient's launch leaves out because they save no turn."""
+    """Which route a layer takes decides how its input gradient is rounded, and the rule counts the weight gradient's parts: as many as
+    fill the chip once, also in layers where fewer would take as many turns each."""
     from flash_dropout.hip import GEMM
 
     n, c, h, w, k, r = layer
@@ -357,7 +357,8 @@ def test_how_a_weight_gradient_is_cut_moves_no_convolution_to_another_route(laye
     lib, rows = GEMM().lib, n * h * w
     want = max(1, 256 // (-(-c // 32) * -(-k // 64) * -(-r * r // 9)))
     parts = lib.sd_conv2d_taps_dw_workspace_bytes(c, k, r, r, rows) // (4 * r * r * c * k)
-    assert parts < min(want, -(-rows // 256))  # a layer of which parts are left out
+    turns = -(-rows // 256)
+    assert parts == min(want, turns) and -(-turns // -(-turns // parts)) < parts
     assert lib.sd_conv2d_taps_fits(*geo) == 1 and lib.sd_conv2d_taps_taken_blocks(*geo, p, bs) == 0
 
 
