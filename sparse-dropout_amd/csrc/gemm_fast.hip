@@ -1911,20 +1911,21 @@ double sdd_row_groups(const GemmArgs& g) {
 }
 // workgroups the big SDD shape is expected to have (plan_sdd counts with sdd_plan_groups)
 int64_t sdd_big_groups(const GemmArgs& g) { return (int64_t)((double)((blocks_of(g.M) + 3) / 4) * sdd_row_groups(g) + 0.5); }
-// Whether the workgroups count the groups of all row quads (find_group): where the groups expected nearly fill their last round, so
-// that an engine with one or two more than others takes another, and a round is long against the 4 to 5 us that each
-// workgroup counts.  dX of 8192^3, us without and with: p = 0.75 (1.9 rounds) 500 -> 391, 0.4 (2.96) 766 -> 671; 0.5 (2.6) 602 -> 618,
-// 0.6 (2.4) 558 -> 591.
+// Whether the workgroups of a launch of the input gradient alone count the groups of all row quads (find_group).  It saves a round
+// where the groups expected nearly fill their last one, of two to four, and an engine with one or two more than others would take another;
+// it costs 4 to 5 us a round.  How far engines differ goes with how much of a row is dropped: where up to 0.65 of the blocks
+// are kept, 18 of 19 drawn layers gain (0.80 of the time on average, 1.05 at worst); where more are kept 45 of 63 lose, up to 7 %, and with
+// fewer than 48 steps or less of the last round filled 15 of 23, up to 11 %.  dX of 8192^3, us without and with: p = 0.75 (1.9
+// rounds) 500 -> 391, 0.4 (2.96) 766 -> 671; 0.5 (2.6) 602 -> 618, 0.6 (2.4) 558 -> 591.  Beside the weight gradient, whose workgroups
+// fill that round, nothing is gained: all of 16 layers lost, 0.6 to 5 %.
 bool sdd_counts_all(const GemmArgs& g) {
   const int64_t Mb = blocks_of(g.M);
-  if (!g.row_ptr || sdd_row_groups(g) >= sdd_most_groups(g) || Mb > 4 * kCountedQuads || Mb * blocks_of(g.N) > kCountedBlocks) return false;
+  if (!g.row_ptr || kept_blocks(g) > 0.65 || blocks_of(g.K) < 48 || Mb > 4 * kCountedQuads || Mb * blocks_of(g.N) > kCountedBlocks) return false;
   const double rounds = (double)sdd_big_groups(g) / 256.0, over = rounds - (double)(int64_t)rounds;
-  return over > 0.75 && over < 0.98 && (double)blocks_of(g.K) > 8.0 * rounds;
+  return rounds > 1.0 && rounds < 4.0 && over > 0.85 && over < 0.98;
 }
-// What the kernels are told: 0 for that, or the groups that nearly every row quad has (those above come last in the launch order).
-int sdd_sure_groups(const GemmArgs& g) {
-  return sdd_counts_all(g) ? 0 : std::min(sdd_most_groups(g), (int)(sdd_row_groups(g) + 1.0));
-}
+// The groups that nearly every row quad has (those above come last in the launch order).
+int sdd_sure_groups(const GemmArgs& g) { return std::min(sdd_most_groups(g), (int)(sdd_row_groups(g) + 1.0)); }
 template <typename T, bool EDGE>
 int launch_sdd_big(const GemmArgs& g, hipStream_t stream) {
   using G = SddBig;
@@ -1933,7 +1934,7 @@ int launch_sdd_big(const GemmArgs& g, hipStream_t stream) {
   const int Mb = (int)((g.M + BS - 1) / BS), Cb = (int)((g.N + BS - 1) / BS);
   const int tiles_m = (Mb + G::R - 1) / G::R;
   hipLaunchKernelGGL((sdd_group_kernel<T, EDGE, G>), dim3((unsigned)(tiles_m * sdd_most_groups(g))), dim3(THREADS), G::SMEM,
-                     stream, g, tiles_m, sdd_sure_groups(g), Mb, Cb);
+                     stream, g, tiles_m, sdd_counts_all(g) ? 0 : sdd_sure_groups(g), Mb, Cb);
   return check_launch("sdd_group_kernel");
 }
 
@@ -2018,7 +2019,7 @@ int try_sdd(const GemmArgs& g, int dtype, hipStream_t stream) {
   const int shape = plan_sdd(g);
   const bool ragged = g.N % BS != 0 || g.K % BS != 0;
   if (shape == kShapeBig) {
-    note_kernel("sdd:big%s", ragged ? ":ragged" : "");
+    note_kernel("sdd:big%s%s", ragged ? ":ragged" : "", sdd_counts_all(g) ? ":counted" : "");
     if (is_bf16(dtype)) return ragged ? launch_sdd_big<BF16, true>(g, stream) : launch_sdd_big<BF16, false>(g, stream);
     return ragged ? launch_sdd_big<F16, true>(g, stream) : launch_sdd_big<F16, false>(g, stream);
   }

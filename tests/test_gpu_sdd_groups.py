@@ -21,19 +21,19 @@ def quad_rows(n1, n2, Cb, gen):
     return keep
 
 
-def check(ext, dy, w, mask, p, hint, policy):
+def check(ext, dy, w, mask, p, hint, policy, bs=64):
     """dX against fp32 on the same rounded operands: one rounding to fp16 is 2^-11 of an element at most, and a sum of K products
     in fp32 adds K * 2^-24 of the terms' size, so 2^-10 of a tile's norm holds both."""
-    lists = ext.build_lists(mask)
+    lists = ext.build_lists(mask, 0 if bs == 32 else 1)
     M, N = dy.shape[0], w.shape[1]
     out = torch.full((M, N), 7.0, dtype=dy.dtype, device="cuda")
     before = ext.set_tile_policy(policy)
     try:
-        ext.gemm_sdd_lists(dy, w.t(), lists, 64, 1.0 / (1.0 - p), out=out, keep_hint=hint)
+        ext.gemm_sdd_lists(dy, w.t(), lists, bs, 1.0 / (1.0 - p), out=out, keep_hint=hint)
         detail = ext.last_kernel_detail()
     finally:
         ext.set_tile_policy(before)
-    keep = (~mask).repeat_interleave(64, 0)[:M].repeat_interleave(64, 1)[:, :N]
+    keep = (~mask).repeat_interleave(bs, 0)[:M].repeat_interleave(bs, 1)[:, :N]
     ref = (dy.float() @ w.float()) / (1.0 - p) * keep
     assert max_tile_rel_fro(out, ref) <= 2.0 ** -10
     return detail
@@ -53,21 +53,50 @@ def test_rows_dealt_out_to_groups(N, hint, policy):
     assert detail.startswith("sdd:" + policy)
 
 
-@pytest.mark.parametrize("M,N,K,p", [
-    (2048, 8192, 512, 0.25),    # 8 row quads, most of their groups in one round that they nearly fill: counted
-    (2304, 7368, 640, 0.25),    # the same on ragged column blocks, 9 row quads
-    (12288, 1088, 512, 0.3),    # 48 row quads, 17 column blocks
-    (4096, 4096, 256, 0.5),     # not counted
+@pytest.mark.parametrize("M,N,K,p,bs,counted", [
+    (2048, 24320, 3072, 0.5, 64, True),    # 8 row quads
+    (2304, 22056, 3080, 0.5, 64, True),    # 9, ragged column blocks and steps
+    (12288, 3584, 3072, 0.8, 32, True),    # 48, masks of 32-blocks
+    (33280, 1344, 3072, 0.5, 64, True),    # 130: a thread to a row of blocks, two turns of them
+    (65530, 576, 3072, 0.5, 64, True),     # 256, the most that are counted, the last row block not whole
+    (65600, 576, 3072, 0.5, 64, False),    # 257
+    (2048, 24320, 3008, 0.5, 64, False),   # 47 steps
+    (12288, 1088, 512, 0.3, 64, False),    # three quarters of a round
+    (4096, 4096, 256, 0.5, 64, False),
 ])
-def test_positions_counted_over_all_row_quads(M, N, K, p):
+def test_positions_counted_over_all_row_quads(M, N, K, p, bs, counted):
     from flash_dropout.hip import GEMM
 
     gen = torch.Generator(device="cuda").manual_seed(M + N)
     dy = torch.randn(M, K, generator=gen, device="cuda").half()
     w = torch.randn(K, N, generator=gen, device="cuda").half()
-    mask = torch.rand(-(-M // 64), -(-N // 64), generator=gen, device="cuda") < p
-    mask[: 8, ::2] = True  # quads with fewer groups than the others
-    check(GEMM(), dy, w, mask, p, 1.0 - p, "big")
+    mask = torch.rand(-(-M // bs), -(-N // bs), generator=gen, device="cuda") < p
+    mask[: 512 // bs, ::2] = True  # quads with fewer groups than the others
+    detail = check(GEMM(), dy, w, mask, p, 1.0 - p, "big", bs)
+    assert detail.startswith("sdd:big") and detail.endswith(":counted") == counted, detail
+
+
+def test_positions_are_not_counted_beside_the_weight_gradient():
+    """The weight gradient's workgroups fill the last round there: the pair's dX has the bits of the launch alone, whichever way
+    its positions are found."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    M, N, K, p, bs = 65280, 768, 3072, 0.75, 64  # 255 row quads
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    x, w, dy = (torch.randn(*s, generator=gen, device="cuda").half() for s in ((M, N), (K, N), (M, K)))
+    mask = torch.rand(M // bs, N // bs, generator=gen, device="cuda") < p
+    before = ext.set_tile_policy("big")
+    try:
+        _, _, lists, kbs = ext.dropout_matmul_forward(x, w, bs, p, mask=mask)
+        dx, _ = ext.dropout_matmul_backward(dy, w, x, lists, kbs, p)
+        pair = ext.last_kernel_detail()
+        alone, _ = ext.dropout_matmul_backward(dy, w, x, lists, kbs, p, need_dw=False)
+        assert ext.last_kernel_detail() == "sdd:big:counted"
+    finally:
+        ext.set_tile_policy(before)
+    assert pair.startswith("pair:sdd+dsd:big") and "counted" not in pair, pair
+    assert torch.equal(dx, alone)
 
 
 @pytest.mark.parametrize("bs", [32, 64])
