@@ -3,6 +3,7 @@
 #pragma once
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "gemm_tile.h"
 #include "gemm_tile_api.h"
@@ -127,10 +128,13 @@ int forward_launch(const GemmArgs& g, int splits, const FlatJobs& f, hipStream_t
   return f.tabled ? forward_launch_t<T, S, true>(g, splits, f, stream) : forward_launch_t<T, S, false>(g, splits, f, stream);
 }
 
-// Of the strips of C kept column blocks that a row of the block grid can have, `most`, those that about every row has.
+// Of the strips of C kept column blocks that a row of the block grid can have, `most`, those that all but one row in six have: the
+// average and a standard deviation.  A strip past them starts last and reads its row of dY far from the others that do.
+// On 600 drawn layers, against all strips in the walk: 0.985 of the time on average, 1.09 at worst; with the average 0.984 and
+// 1.50 (dX of 4304 x 1008 from 5784 at p = 0.25: 60.0 us, 60.3 and 89.8), with two deviations 0.987 and 1.07.
 int sure_strips(const GemmArgs& g, int C, int most) {
-  const double keep = kept_blocks(g);
-  return keep > 0.999 ? most : std::min(most, std::max(1, (int)((double)blocks_of(g.N) * keep / C + (C - 1) / (2.0 * C) + 0.5)));
+  const double keep = kept_blocks(g), Cb = (double)blocks_of(g.N), spread = std::sqrt(Cb * keep * (1.0 - keep));
+  return keep > 0.999 ? most : std::min(most, std::max(1, (int)((Cb * keep + spread) / C + (C - 1) / (2.0 * C) + 0.5)));
 }
 
 template <typename T, typename S>
