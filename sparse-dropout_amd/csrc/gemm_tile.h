@@ -181,7 +181,7 @@ __device__ inline void load_aux(const GemmArgs& g, int lane, int64_t m0, int64_t
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NT16; nt += 2)
-      pre[mt * (NT16 / 2) + nt / 2] = s.has_aux ? aux_eight(g, s, m0 + mt * 16 + lane % 16, n0 + nt * 16 + piece_at(lane)) : u32x4{0u, 0u, 0u, 0u};
+      pre[mt * (NT16 / 2) + nt / 2] = aux_eight(g, s, m0 + mt * 16 + lane % 16, n0 + nt * 16 + piece_at(lane));
 }
 
 // The step table of a workgroup that owns row blocks rb0 .. rb0 + R - 1: the union of their kept lists (from the mask
@@ -667,7 +667,7 @@ __device__ __forceinline__ void tile_sdd_body(const GemmArgs& g, int sure, int M
   // at p = 0.3 58.2 -> 54.4 us, 16384 x 1536 from 384 at p = 0.1 53.1 -> 51.1
   const int64_t m_out = m0 + 32 * kk, n_out = (int64_t)my_col * BS + b_t0 * 16;
   u32x4 pre[NT16] = {};
-  if (active) load_aux<2, NT16>(g, lane, m_out, n_out, pre);
+  if (active && g.act != SD_ACT_NONE) load_aux<2, NT16>(g, lane, m_out, n_out, pre);
   f32x4 half[2][NT16];
   meet_halves<NT16>(acc, half, smem, wave, kk, lane);
   if (!active) return;
