@@ -85,11 +85,17 @@ const char* sd_last_kernel_detail(void);
 const char* sd_source_hash(void);
 
 /* The workgroup-to-tile map of the specialised kernels, evaluated on the host: launch index `block` of a
- * tiles_m x tiles_n grid -> (tile_m, tile_n); kind 0 = DSD / dense order, 1 = SDD order.  The hardware deals
+ * tiles_m x tiles_n grid -> (tile_m, tile_n); kind 0 = DSD / dense order, 1 = the order of SDD groups where every row quad
+ * has all of them (sd_group_of_block has the others).  The hardware deals
  * consecutive workgroup ids round-robin to the 8 XCDs; the map gives each XCD a compact patch of the grid.  It
  * must be a bijection onto the grid, which tests check through this entry point; the reference's counterpart is
  * threadblock_swizzle (flash_dropout/cuda/src/gemm.cuh:84-97). */
 int sd_tile_of_block(int kind, int64_t block, int64_t tiles_m, int64_t tiles_n, int32_t* tile_m, int32_t* tile_n);
+
+/* The same for SDD, whose rows have as many groups as their masks leave: launch index `block` of a grid of `groups` groups, the most
+ * a row can have, for each of `rows` rows -> (row, group).  The first `sure` groups of all rows come first.  kind 0: strips of
+ * a row block's kept tiles, 1: groups of a row quad's column blocks.  It must be a bijection for every `sure`. */
+int sd_group_of_block(int kind, int64_t block, int64_t rows, int64_t groups, int64_t sure, int32_t* row, int32_t* group);
 
 /* Workgroup shape of the specialised DSD / dense kernels: SD_TILE_AUTO picks from the shape (256 x 256
  * output tiles when there are more than 128 of them, 128 x 128 otherwise; the SDD kernel's group shape follows the

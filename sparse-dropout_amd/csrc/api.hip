@@ -207,6 +207,22 @@ int sd_tile_of_block(int kind, int64_t block, int64_t tiles_m, int64_t tiles_n, 
   return SD_OK;
 }
 
+int sd_group_of_block(int kind, int64_t block, int64_t rows, int64_t groups, int64_t sure, int32_t* row, int32_t* group) {
+  SD_REQUIRE(kind == 0 || kind == 1, "group_of_block: kind must be 0 (strips) or 1 (groups of the large shape)");
+  SD_REQUIRE(row && group, "group_of_block: null output");
+  SD_REQUIRE(rows > 0 && groups > 0 && rows < kMaxDim && groups < kMaxDim && rows * groups < kMaxDim, "group_of_block: bad grid");
+  SD_REQUIRE(sure > 0 && sure <= groups, "group_of_block: sure groups outside 1 .. groups");
+  SD_REQUIRE(block >= 0 && block < rows * groups, "group_of_block: block outside the grid");
+  int tm = 0, gi = 0;
+  if (kind == 0)
+    group_of_block<DSD_GROUP_M>((int)block, (int)rows, (int)sure, tm, gi);
+  else
+    group_of_block<SDD_GROUP_M>((int)block, (int)rows, (int)sure, tm, gi);
+  *row = tm;
+  *group = gi;
+  return SD_OK;
+}
+
 int sd_set_tile_policy(int policy) { return sd::set_tile_policy(policy); }
 
 int64_t sd_workspace_bytes(int64_t mb, int64_t kb) {

@@ -207,6 +207,31 @@ def test_tile_map_is_a_bijection_onto_the_tile_grid(kind):
     assert lib.sd_tile_of_block(2, 0, 3, 4, ctypes.byref(tm), ctypes.byref(tn)) == 1
 
 
+@pytest.mark.parametrize("kind", [0, 1])
+def test_group_map_is_a_bijection_for_every_number_of_sure_groups(kind):
+    """What the input gradient's kernels launch by: every group that a row can have exactly once, those that are sure to exist in
+    front, and with all of them sure the plain tile order."""
+    from flash_dropout.hip import _loader
+
+    lib = _loader.load()
+    tm, gi, tm2, tn2 = (ctypes.c_int32() for _ in range(4))
+    for rows in (1, 2, 3, 4, 5, 7, 8, 9, 17, 40):
+        for groups in (1, 2, 3, 6, 7, 13):
+            for sure in range(1, groups + 1):
+                seen = set()
+                for b in range(rows * groups):
+                    assert lib.sd_group_of_block(kind, b, rows, groups, sure, ctypes.byref(tm), ctypes.byref(gi)) == 0
+                    assert 0 <= tm.value < rows and 0 <= gi.value < groups
+                    assert (gi.value < sure) == (b < rows * sure), (rows, groups, sure, b)
+                    seen.add((tm.value, gi.value))
+                    if sure == groups and kind == 1:
+                        assert lib.sd_tile_of_block(1, b, rows, groups, ctypes.byref(tm2), ctypes.byref(tn2)) == 0
+                        assert (tm.value, gi.value) == (tm2.value, tn2.value)
+                assert len(seen) == rows * groups, (rows, groups, sure)
+    for bad in ((kind, 12, 3, 4, 2), (kind, -1, 3, 4, 2), (kind, 0, 3, 4, 0), (kind, 0, 3, 4, 5), (2, 0, 3, 4, 2)):
+        assert lib.sd_group_of_block(*bad, ctypes.byref(tm), ctypes.byref(gi)) == 1
+
+
 def test_tile_map_keeps_an_xcd_on_a_compact_patch():
     """What the map is for: the 32 workgroups an XCD holds at a time (launch indices x, x+8, x+16, ...) cover
     at most 8 tile rows x 4+1 tile columns of a large grid, not a scattered set."""
