@@ -224,13 +224,46 @@ def test_what_a_mask_drops_reaches_nothing_tap_by_tap(bad):
         assert torch.equal(~torch.isfinite(dw.cpu().reshape(k, -1)), bad_dw), which
 
 
+def _dw_turns(geom):
+    """Least and most turns of 256 positions that a workgroup of the weight gradient has."""
+    from flash_dropout.hip import GEMM
+
+    n, c, h, w, k, r, s, pad, dil = geom
+    rows = n * h * w  # (as many positions as pixels)
+    turns, parts = -(-rows // 256), GEMM().lib.sd_conv2d_taps_dw_workspace_bytes(c, k, r, s, rows) // (4 * c * k * r * s)
+    return turns // parts, -(-turns // parts)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("geom,turns", [
+    ((1, 512, 12, 256, 256, 3, 3, (1, 1), (1, 1)), (3, 3)),  # a window of 784 rows: the only buffer is filled again
+    ((2, 264, 11, 256, 232, 3, 3, (1, 1), (1, 1)), (3, 4)),  # parts of uneven length, channels and outputs that end inside a tile
+    ((3, 512, 24, 40, 200, 3, 3, (1, 1), (1, 1)), (3, 3)),    # two, the first of them used twice, the last turn not whole
+])
+def test_weight_gradient_over_several_turns(geom, turns, dtype):
+    assert _dw_turns(geom) == turns
+    n, c, h, w, k, r, s, pad, dil = geom
+    x, wt, dy, rows, gen = _tensors(geom, dtype)
+    mask = cpu_mask(O.mask_shape(rows, c * r * s, 64), 0.5, gen)
+    dw = _products(geom, x, wt, dy, mask, 64, 2.0)[2]
+    want = O.conv2d_blockdrop(to_np(x), to_np(wt), mask.numpy(), 64, 0.5, dy=to_np(dy), dtype=np.float32, padding=pad, stride=(1, 1),
+                              dilation=dil)[2]
+    assert max_tile_rel_fro(dw, want) <= REL_FRO_TOL
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
-@pytest.mark.parametrize("geom", [(16, 128, 32, 32, 128, 3, 3, (1, 1), (1, 1)),   # two turns of 256 positions to a workgroup
-                                  (2, 512, 24, 40, 200, 3, 3, (1, 1), (1, 1)),    # seven, the last one not whole
-                                  (1, 32, 9, 256, 40, 3, 3, (1, 1), (1, 1))])     # one buffer of rows
-def test_gradients_that_are_not_finite_reach_kept_blocks_only(geom, bad):
+@pytest.mark.parametrize("geom,turns", [
+    ((16, 128, 32, 32, 128, 3, 3, (1, 1), (1, 1)), (2, 2)),
+    ((2, 512, 24, 40, 200, 3, 3, (1, 1), (1, 1)), (2, 2)),    # the last turn not whole
+    ((3, 512, 24, 40, 200, 3, 3, (1, 1), (1, 1)), (3, 3)),
+    ((1, 32, 9, 256, 40, 3, 3, (1, 1), (1, 1)), (1, 1)),    # one buffer
+    ((1, 512, 12, 256, 256, 3, 3, (1, 1), (1, 1)), (3, 3)),
+])
+def test_gradients_that_are_not_finite_reach_kept_blocks_only(geom, turns, bad):
     """A weight gradient clears what a block drops in the image, and does without where a sum is not finite: one bad element of dY
-    reaches its output's kept blocks, and everything else is bit for bit what it is with a zero there."""
+    reaches its output's kept blocks, and everything else is bit for bit what it is with a zero there.  The turns are gone through
+    a second time for that, with one and with two buffers for their rows."""
+    assert _dw_turns(geom) == turns
     n, c, h, w, k, r, s, pad, dil = geom
     x, wt, dy, rows, gen = _tensors(geom, torch.float16)
     mask = cpu_mask(O.mask_shape(rows, c * r * s, 64), 0.5, gen)
