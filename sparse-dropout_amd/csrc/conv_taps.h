@@ -166,8 +166,9 @@ SD_BOTH int64_t taps_lds(const TapGeom& geo, bool dx, int64_t span) {
 constexpr int kDwTaps = 9;    // of a workgroup
 constexpr int kDwPitch = 64;  // bytes of an LDS row of 32 channels: the four rows of a transposing read in different banks
 // Weight gradient.  A buffer: rows of the window and one of zeros, 256 rows of dY, a record per position.  In the end three taps' sums
-// of the eight waves meet there: 8 x 64 lanes x 3 x 16 floats, 96 KB.  No launch asks for less than 144 KB: its registers give a
-// workgroup the CU to itself, and what it asks for says so.
+// of the eight waves meet there: 8 x 64 lanes x 3 x 16 floats, 96 KB.  No launch asks for less than the 144 KB that they took when
+// all nine taps met at once: the host test holds launches to it, and it costs nothing, since by its registers a workgroup has the
+// CU to itself.
 constexpr int kDwLeast = 144 * 1024;
 SD_BOTH int64_t dw_lds(int64_t span, int buffers) {
   constexpr int64_t merge = 8 * 64 * 3 * 16 * 4;

@@ -533,7 +533,9 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
     d.z = uniform((uint32_t)(left * (int)g.dy_ld * 2));
     const uint32_t dst = smem_a + (uint32_t)(buf * buffer + x_bytes + lw * 8192);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) buffer16_to_lds(d, dy_off[i % 2] + (uint32_t)(i / 2 * 32 * (int)g.dy_ld), dst + (uint32_t)(i * 1024));
+    for (int i = 0; i < 8; ++i) {
+      buffer16_to_lds(d, dy_off[i % 2] + (uint32_t)(i / 2 * 32 * (int)g.dy_ld), dst + (uint32_t)(i * 1024));
+    }
     const int n = w.hi - w.lo < g.span ? w.hi - w.lo : g.span;
     const u32x4 x = buffer_of(reinterpret_cast<const char*>(g.x + (int64_t)w.lo * g.x_ld + c0));
     for (int r0 = lw * 16; r0 < n; r0 += 64) {
@@ -561,7 +563,8 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
   auto dropped = [&](int turn) -> uint32_t {
     const int rb = turn * 4 + pb;
     uint32_t d = 1u;
-    if (lane < 32 && rb * 64 < g.rows && cb0 + lane < cbs) d = g.mask ? mask_col[(int64_t)(g.split == 1 ? rb : rb / g.split) * g.msr] : 0u;
+    if (lane < 32 && rb * 64 < g.rows && cb0 + lane < cbs)
+      d = g.mask ? mask_col[(int64_t)(g.split == 1 ? rb : rb / g.split) * g.msr] : 0u;
     return d;
   };
 
@@ -608,16 +611,16 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
         const char* rec = xl + x_bytes + 256 * 128 + pb * 512;
         int at[4];  // where in LDS the lane's positions read tap 0
         uint32_t in[4];
-  #pragma unroll
+#pragma unroll
         for (int h = 0; h < 4; ++h) {  // positions 32 * (h / 2) + 4 * (h % 2) + in_block of the block
           const u32x2 r = *reinterpret_cast<const u32x2*>(rec + (32 * (h / 2) + 4 * (h % 2) + in_block) * 8);
           at[h] = (int)r.x + x_at;
           in[h] = r.y;
         }
         u32x4 df[4][2];
-  #pragma unroll
+#pragma unroll
         for (int kk = 0; kk < 2; ++kk)
-  #pragma unroll
+#pragma unroll
           for (int k = 0; k < 4; ++k) df[k][kk] = fd[kk].read(dl, k);
         auto read_quarter = [&](int i, int h, u32x4 (&xf)[2]) {
           const int inside = ones_if(in[h], i);
@@ -1082,7 +1085,8 @@ extern "C" int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* d
   note_kernel("conv_dw:taps splits=%d", (int)splits);
   const unsigned blocks = (unsigned)ceil_div(r * s * c * k_out / 4, 16);
   auto reduce = [&](auto* kernel) {
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s), (int)splits, scale);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, st, g.part, static_cast<uint16_t*>(dw), dw_ld, g.C, g.K, (int)(r * s),
+                       (int)splits, scale);
   };
   if (splits > 32) bf ? reduce(&taps_dw_reduce<BF16, 8>) : reduce(&taps_dw_reduce<F16, 8>);
   else bf ? reduce(&taps_dw_reduce<BF16, 1>) : reduce(&taps_dw_reduce<F16, 1>);

@@ -1074,7 +1074,8 @@ struct GroupAt {
 };
 constexpr int kCountedQuads = 256;      // most row quads a workgroup counts the groups of
 constexpr int kCountedBlocks = 1 << 15; // most blocks of a mask it lists for that
-__device__ inline GroupAt find_group(const GemmArgs& g, char* smem, int tiles_m, int gsure, int Mb, int Cb, int bid, int tid, int wave, int lane) {
+__device__ inline GroupAt find_group(const GemmArgs& g, char* smem, int tiles_m, int gsure, int Mb, int Cb, int bid, int tid, int wave,
+                                     int lane) {
   GroupAt at;
   int gi = 0;
   at.tm = 0;
@@ -1702,6 +1703,10 @@ __global__ __launch_bounds__(THREADS) void sdd_group_kernel(GemmArgs g, int tile
 // reduce pass as in the kernel of its own) comes first where its chains are the longer ones (dw_before_dx).  One launch instead of
 // two, and the second product's workgroups fill the CUs the first one's last round leaves idle - for small layers,
 // whose grids cover a fraction of the chip each, the two simply run side by side.
+// The input gradient's body stays the first branch, which is laid out in front: the weight gradient's spills a few registers over
+// its loop and reads them back behind it, and with that in front of the other the compiler waited for the reloads where it next
+// touched those registers, in the input gradient's step loop, and with them for the wave's direct loads (three waits in a
+// step; 4096^3 in blocks of 32 300 -> 271 us without).
 template <typename T, bool EDGE, typename G, typename S>
 __global__ __launch_bounds__(THREADS) void backward_pair_kernel(GemmArgs gx, int x_tiles_m, int x_gmax, int x_gsure,
                                                                 int x_Mb, int x_Cb, int n_first, bool dw_first,
@@ -1852,7 +1857,9 @@ ShapeWork dsd_work(bool kc, int shape, int64_t M, int64_t N, int64_t K, int spli
   w.steps = (double)((blocks_of(K) + splits - 1) / splits) * ((1.0 - w.cost.kept) * (1.0 - none) + w.cost.kept * kept) *
             (ragged ? 1.0 + w.cost.ragged : 1.0);
   w.rest = (w.cost.store + w.cost.act(act)) * (double)(blocks_of(M) * blocks_of(N)) * 1e-3;
-  if (splits > 1) w.rest += 3.5 + (double)splits * (0.02 + 2.2e-6 * (double)M * (double)N);  // the pass over the fp32 partials
+  // The pass over the fp32 partials as it was when the rest was fitted (7 parts of 384 x 1536 count 12.7 us; they take 3.3 by now, and 5.2
+  // with what the product's stores of them cost).  How a reduction is cut decides last bits, so the cuts stay those of the fit.
+  if (splits > 1) w.rest += 3.5 + (double)splits * (0.02 + 2.2e-6 * (double)M * (double)N);
   return w;
 }
 
@@ -1920,7 +1927,8 @@ int64_t sdd_big_groups(const GemmArgs& g) { return (int64_t)((double)((blocks_of
 // fill that round, nothing is gained: all of 16 layers lost, 0.6 to 5 %.
 bool sdd_counts_all(const GemmArgs& g) {
   const int64_t Mb = blocks_of(g.M);
-  if (!g.row_ptr || kept_blocks(g) > 0.65 || blocks_of(g.K) < 48 || Mb > 4 * kCountedQuads || Mb * blocks_of(g.N) > kCountedBlocks) return false;
+  if (!g.row_ptr || kept_blocks(g) > 0.65 || blocks_of(g.K) < 48) return false;
+  if (Mb > 4 * kCountedQuads || Mb * blocks_of(g.N) > kCountedBlocks) return false;
   const double rounds = (double)sdd_big_groups(g) / 256.0, over = rounds - (double)(int64_t)rounds;
   return rounds > 1.0 && rounds < 4.0 && over > 0.85 && over < 0.98;
 }

@@ -325,7 +325,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs g, int spli
   acc *= g.scale;
   if (ci + 4 <= c_ext && g.act == SD_ACT_NONE && (trans ? g.c_sr : g.c_sc) == 1) {
     typedef u32x2 __attribute__((aligned(2))) u32x2_any;
-    *reinterpret_cast<u32x2_any*>(g.c + (int64_t)si * (trans ? g.c_sc : g.c_sr) + ci) = u32x2{T::pack2(acc[0], acc[1]), T::pack2(acc[2], acc[3])};
+    uint16_t* const dst = g.c + (int64_t)si * (trans ? g.c_sc : g.c_sr) + ci;
+    *reinterpret_cast<u32x2_any*>(dst) = u32x2{T::pack2(acc[0], acc[1]), T::pack2(acc[2], acc[3])};
     return;
   }
 #pragma unroll
