@@ -8,6 +8,7 @@
 // q while reading (consecutive pixels of an image row), the 64x64 tile is turned in LDS, and lanes run
 // along the column index while writing, so both sides are coalesced.  With a kept-block list only
 // kept blocks are produced: dropped blocks are never read by the DSD kernels, so they are not written.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -125,16 +126,21 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict_
 //    one behind the other, listed in `src_row` once per workgroup.  Nothing ties the image size to the group.
 //  * Column space: `tpg` column tiles' channels are staged at a time (all of them where they fit), with one barrier pair
 //    per group of tiles; the tiles themselves follow without barriers.
+//  * Few rows: the groups of column tiles are dealt out over blockIdx.y, `gpw` to a workgroup, until there are four workgroups to
+//    a CU.  With one to 64 rows, whatever the number of columns, a layer of little more than 64 rows took the time of one
+//    workgroup's chain: 45 x 208 x 8 x 8, 5 x 5 by two, p = 0.6 (12 row groups of 82 tiles) 175 us,
+//    25 on 984 workgroups.
 // 256 x 32 x 28 x 28, 3 x 3, p = 0.25: 126 us on im2col_kernel, 46 here; 70 x 64 x 56 x 56, p = 0.5: 102 with the image's
 // channels staged tile by tile, 90.
 constexpr int PATCH_MAX_BYTES = 48 * 1024;
 constexpr int PATCH_ROWS_MAX = 256;
+constexpr int64_t PATCH_WORKGROUPS = 1024;
 
 __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __restrict__ x,
                                                            uint16_t* __restrict__ cols, int64_t ld,
                                                            ConvGeom g, const int32_t* row_ptr,
                                                            const int32_t* col_idx, int bs, int wp,
-                                                           int tpg) {
+                                                           int tpg, int gpw) {
   extern __shared__ __attribute__((aligned(16))) char patch_mem[];
   int* col_off = reinterpret_cast<int*>(patch_mem);                     // [tpg * 64]: offset of a column in the copy
   uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp]
@@ -182,21 +188,38 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
   const int sub_per_block = bs / TILE;
   const int ntiles = (ncols + TILE - 1) / TILE;
   const int per_ch = hp * wp;
+  // column tiles [t_lo, t_hi) are this workgroup's
+  const int t_lo = (int)blockIdx.y * gpw * tpg, t_hi = t_lo + gpw * tpg < ntiles ? t_lo + gpw * tpg : ntiles;
   int32_t pos = 0, end = 0;
   if (row_ptr) {
     const int64_t rb = r0 / bs;
     pos = row_ptr[rb];
     end = row_ptr[rb + 1];
+    if (t_lo > 0) {  // past the entries of the workgroups before, 64 at a time
+      for (int32_t from = pos; from < end; from += 64) {
+        const int32_t i = from + t % 64;
+        const bool before = i < end && (int64_t)(col_idx[i] + 1) * sub_per_block <= t_lo;
+        const int n = __popcll(__ballot(before));
+        pos = from + n;
+        if (n < 64) break;
+      }
+    }
   }
-  int sub = 0, ct = -1, group = -1;
+  int sub = 0, ct = t_lo - 1, group = -1;
+  int32_t entry = pos < end ? col_idx[pos] : 0;
   for (;;) {
     if (row_ptr) {
       if (pos >= end) break;
-      ct = col_idx[pos] * sub_per_block + sub;
-      if (++sub == sub_per_block) { sub = 0; ++pos; }
-      if (ct >= ntiles) continue;
+      ct = entry * sub_per_block + sub;
+      if (++sub == sub_per_block) {
+        sub = 0;
+        ++pos;
+        entry = pos < end ? col_idx[pos] : 0;  // (on its way under this tile)
+      }
+      if (ct < t_lo) continue;
+      if (ct >= t_hi) break;
     } else {
-      if (++ct >= ntiles) break;
+      if (++ct >= t_hi) break;
     }
     if (ct / tpg != group) {  // the same for every thread
       group = ct / tpg;
@@ -606,12 +629,15 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
   };
   if (ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 && hp <= PATCH_ROWS_MAX &&
       group_bytes(1) <= PATCH_MAX_BYTES) {
-    // as many tiles to a group as fit a quarter of the LDS a workgroup may ask for: several workgroups share a CU
+    // as many tiles to a group as fit a quarter of the LDS a workgroup may ask for: several workgroups share a CU.  Fewer
+    // where there are few rows, so that the column groups make PATCH_WORKGROUPS workgroups with them.
+    const int64_t split = std::min(ntiles, ceil_div(PATCH_WORKGROUPS, blocks)), most = ceil_div(ntiles, split);
     int64_t tpg = 1;
-    while (tpg < ntiles && group_bytes(tpg + 1) <= PATCH_MAX_BYTES / 2) ++tpg;
-    hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks), dim3(256), (size_t)group_bytes(tpg), stream,
-                       (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
-                       row_ptr ? (int)bs : TILE, (int)wp, (int)tpg);
+    while (tpg < most && group_bytes(tpg + 1) <= PATCH_MAX_BYTES / 2) ++tpg;
+    const int64_t groups = ceil_div(ntiles, tpg), gpw = ceil_div(groups, split);
+    hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks, (unsigned)ceil_div(groups, gpw)), dim3(256),
+                       (size_t)group_bytes(tpg), stream, (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
+                       row_ptr ? (int)bs : TILE, (int)wp, (int)tpg, (int)gpw);
     return check_launch("im2col_patch");
   }
   hipLaunchKernelGGL(im2col_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,

@@ -69,6 +69,38 @@ def test_im2col_writes_only_kept_blocks(cfg, bs):
     assert bool((part[~keep] == 7.0).all())  # dropped blocks are not touched
 
 
+@pytest.mark.parametrize("cfg", [
+    dict(n=1, c=40, h=8, w=8, r=5, s=5, padding=(2, 2), stride=(1, 1), dilation=(1, 1)),     # 1 row group, 16 column tiles: one to a workgroup
+    dict(n=3, c=208, h=8, w=8, r=5, s=5, padding=(2, 2), stride=(2, 2), dilation=(1, 1)),    # 82 tiles, the last ragged
+    dict(n=7, c=232, h=7, w=7, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),    # 6 row groups, 33 tiles
+    dict(n=20, c=96, h=24, w=24, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),  # 180 row groups: some tiles to a workgroup
+])
+@pytest.mark.parametrize("channels_last", [False, True])
+@pytest.mark.parametrize("p,bs", [(None, 64), (0.5, 64), (0.9, 64), (0.5, 128), (0.5, 192)])
+def test_im2col_of_few_rows_deals_out_its_columns(cfg, channels_last, p, bs):
+    """Few row groups: the column tiles, or the kept ones of them, are dealt out over workgroups.  A gather, so bit exact, with
+    every kept block written and no other."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(cfg["c"])
+    x = torch.randn(cfg["n"], cfg["c"], cfg["h"], cfg["w"], generator=gen).half()
+    ks = (cfg["r"], cfg["s"])
+    ref = torch.from_numpy(O.im2col(x.float().numpy(), *ks, **_geo(cfg))).half()
+    xg = x.cuda()
+    if channels_last:
+        xg = xg.contiguous(memory_format=torch.channels_last)
+    if p is None:
+        assert torch.equal(ext.im2col(xg, ks, **_geo(cfg)).cpu(), ref)
+        return
+    mask = cpu_mask(O.mask_shape(*ref.shape, bs), p, gen)
+    lists = ext.build_lists(mask.cuda())
+    part = torch.full(ref.shape, 7.0, dtype=torch.float16, device="cuda")
+    ext.im2col(xg, ks, lists=lists, block_size=bs, out=part, **_geo(cfg))
+    keep = torch.from_numpy(O.expand_keep(mask.numpy(), bs, *ref.shape))
+    assert torch.equal(part.cpu(), torch.where(keep, ref, torch.tensor(7.0, dtype=torch.float16)))
+
+
 @pytest.mark.parametrize("cfg", GEOMS)
 @pytest.mark.parametrize("channels_last", [False, True])
 def test_col2im_vs_oracle(cfg, channels_last):
