@@ -441,19 +441,24 @@ __global__ __launch_bounds__(256) void col2im_tile_kernel(const uint16_t* __rest
   }
 }
 
-// The same for unit stride and dilation (the usual 3x3 / 5x5 layer), where output (h, w) takes tap
-// (r, s) from patch row (h + pad_h - r, w + pad_w - s): the staged window gets a zero halo, rows and
-// columns outside the patch matrix included, so the tap loop has no bounds checks and walks LDS with
-// constant strides.  A thread owns one (channel, w) column of the band and runs down its rows.
+// The same for unit dilation and strides of ST both ways (1: the usual 3x3 / 5x5 layer, 2: a layer that halves the image), where
+// output (h, w) takes tap (r, s) from patch row ((h + pad_h - r) / ST, (w + pad_w - s) / ST) if both are whole: the staged
+// window gets a zero halo, rows and columns outside the patch matrix included, so the tap loop has no bounds checks
+// and walks LDS with constant strides.  A thread owns one (channel, w) column of the band and runs down its rows.
 // RT: the kernel size where it is known (RT x RT).  The taps of an output are then unrolled: with loop counters the sum is
 // one LDS latency per tap.  m_qe: ceil(2^32 / window columns), exact while position * columns < 2^32.
 // 256 x 32 x 28 x 28, 3 x 3, p = 0.25: 73 -> 53 us; 167 x 88 x 16 x 16, 5 x 5, p = 0.4: 197 -> 146; 123 x 48 x 7 x 7, 5 x 5: 18 -> 10.
-template <typename T, int RT>
+// By two (from col2im_tile_kernel): 199 x 32 x 48 x 48, 3 x 3, p = 0.25: 127 us there, 45 here.
+template <int ST>
+__device__ __host__ inline int floor_div(int v) {  // |v| < 2^30
+  return ST == 1 ? v : (v + ST * (1 << 28)) / ST - (1 << 28);
+}
+template <typename T, int RT, int ST>
 __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __restrict__ cols, int64_t ld,
                                                           uint16_t* __restrict__ dx, ConvGeom g,
                                                           const uint8_t* mask, int64_t msr, int64_t msc,
-                                                          int bs, int hb, int bands, uint32_t m_qe) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t seg[];  // [hb + R - 1][W + S - 1][8*R*S + 2]
+                                                          int bs, int bands, int hb, int qe, uint32_t m_qe) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t seg[];  // [rows of the window][qe][8*R*S + 2]
   const int t = threadIdx.x;
   const int gr = RT ? RT : g.r, gs = RT ? RT : g.s;
   const int rs_n = gr * gs;
@@ -467,8 +472,8 @@ __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __rest
   const int n_i = b / cgs;
   const int h0 = band * hb;
   const int h1 = (h0 + hb < g.h ? h0 + hb : g.h);
-  const int pe = (h1 - h0) + gr - 1, qe = g.w + gs - 1;     // staged window
-  const int p_first = h0 + g.pad_h - (gr - 1), q_first = g.pad_w - (gs - 1);  // its top-left (p, q)
+  const int p_first = floor_div<ST>(h0 + g.pad_h - (gr - 1)), q_first = floor_div<ST>(g.pad_w - (gs - 1));  // staged window: its top-left (p, q)
+  const int pe = floor_div<ST>(h1 - 1 + g.pad_h) - p_first + 1;                                           // and rows
 
   // ---- stage: R*S 16-byte chunks per window position, zeros outside the matrix and for dropped blocks
   const int chunks = pe * qe * rs_n;
@@ -542,7 +547,8 @@ __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __rest
   }
   __syncthreads();
 
-  // ---- sum the taps: window position of tap (r, s) of output (h, w) is (h - h0 + R-1-r, w + S-1-s) ---
+  // ---- sum the taps: those of output (h, w) are r = (h + pad_h) % ST + i * ST, at window row (h + pad_h) / ST - p_first - i, and
+  //      s likewise
   const bool c_fast = g.xs_c == 1;
   const int pairs = C2I_CG * g.w;
   const int row_h = qe * seg_h;  // halfs per window row
@@ -550,25 +556,34 @@ __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __rest
   for (int pr = t; pr < pairs; pr += 256) {
     const int c_l = c_fast ? pr % C2I_CG : pr / g.w;
     const int wi = c_fast ? pr / C2I_CG : pr % g.w;
-    // tap (0, 0) of the band's first row
-    const uint16_t* base = seg + (gr - 1) * row_h + (wi + gs - 1) * seg_h + c_l * rs_n;
+    const int s0 = (wi + g.pad_w) % ST;
+    // the first tap's column in the window's first row
+    const uint16_t* base = seg + ((wi + g.pad_w) / ST - q_first) * seg_h + c_l * rs_n + s0;
     uint16_t* out = dxn + (int64_t)(c0 + c_l) * g.xs_c + (int64_t)h0 * g.xs_h + (int64_t)wi * g.xs_w;
     for (int hl = 0; hl < h1 - h0; ++hl) {
       float acc = 0.f;
-      const uint16_t* tap_r = base + hl * row_h;
+      const int hp = h0 + hl + g.pad_h, r0 = hp % ST;
+      const uint16_t* tap_r = base + (hp / ST - p_first) * row_h + r0 * gs;
       if constexpr (RT > 0) {
+        constexpr int N = (RT + ST - 1) / ST;
 #pragma unroll
-        for (int rr = 0; rr < RT; ++rr)
+        for (int i = 0; i < N; ++i) {
+          if (i * ST + ST > RT && r0 + i * ST >= RT) break;  // the same for every thread
 #pragma unroll
-          for (int ss = 0; ss < RT; ++ss) acc += T::to_float(tap_r[rr * (RT - row_h) - ss * (seg_h - 1)]);
-      } else {
-        for (int rr = 0; rr < gr; ++rr) {
-          const uint16_t* tap = tap_r;
-          for (int ss = 0; ss < gs; ++ss) {
-            acc += T::to_float(*tap);
-            tap -= seg_h - 1;  // one window column to the left, next s
+          for (int k = 0; k < N; ++k) {
+            const bool there = k * ST + ST <= RT || s0 + k * ST < RT;
+            const float v = T::to_float(tap_r[i * (ST * RT - row_h) + (there ? k * (ST - seg_h) : -s0)]);
+            acc += there ? v : 0.f;
           }
-          tap_r -= row_h - gs;  // one window row up, next r
+        }
+      } else {
+        for (int rr = r0; rr < gr; rr += ST) {
+          const uint16_t* tap = tap_r;
+          for (int ss = s0; ss < gs; ss += ST) {
+            acc += T::to_float(*tap);
+            tap -= seg_h - ST;  // one window column to the left, ST taps on
+          }
+          tap_r -= row_h - ST * gs;  // one window row up
         }
       }
       out[(int64_t)hl * g.xs_h] = T::from_float(acc);
@@ -661,27 +676,33 @@ int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64
   if (c % C2I_CG == 0 && ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 &&
       (!mask || bs % 8 == 0)) {
     const int seg_bytes = (C2I_CG * g.r * g.s + 2) * 2;
-    const bool unit = g.str_h == 1 && g.str_w == 1 && g.dil_h == 1 && g.dil_w == 1;
+    const int st = g.str_h == g.str_w && g.dil_h == 1 && g.dil_w == 1 && g.str_h <= 2 && g.h < (1 << 28) && g.w < (1 << 28) &&
+                           g.pad_h < (1 << 28) && g.pad_w < (1 << 28) && g.r < (1 << 28) && g.s < (1 << 28) ? g.str_h : 0;
     for (int band_rows = 8; band_rows >= 1; band_rows /= 2) {  // the tallest band whose staging fits
       const int hb = band_rows < g.h ? band_rows : g.h;
-      if (unit) {
-        const int64_t lds = (int64_t)(hb + g.r - 1) * (g.w + g.s - 1) * seg_bytes;
+      if (st) {
+        const int64_t pe = st == 1 ? hb + g.r - 1 : (hb + g.r - 2) / 2 + 2;  // at most
+        const int64_t qe = st == 1 ? g.w + g.s - 1 : floor_div<2>(g.w - 1 + g.pad_w) - floor_div<2>(g.pad_w - (g.s - 1)) + 1;
+        const int64_t lds = pe * qe * seg_bytes;
         const int64_t bands = ceil_div(g.h, hb);
         const int64_t wgs = n * (c / C2I_CG) * bands;
         if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL) continue;
-        const int64_t qe = g.w + g.s - 1;
         const uint32_t m_qe = qe <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)qe - 1) / (uint64_t)qe);
         auto launch = [&](auto* kernel) {
           hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), (size_t)lds, stream, (const uint16_t*)cols, ld,
-                             (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, hb, (int)bands, m_qe);
+                             (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, (int)bands, hb, (int)qe, m_qe);
         };
         const int rt = g.r == g.s && (g.r == 1 || g.r == 3 || g.r == 5) ? g.r : 0;
-        if (dtype == SD_BF16)
-          rt == 1 ? launch(&col2im_unit_kernel<BF16, 1>) : rt == 3 ? launch(&col2im_unit_kernel<BF16, 3>)
-          : rt == 5 ? launch(&col2im_unit_kernel<BF16, 5>) : launch(&col2im_unit_kernel<BF16, 0>);
-        else
-          rt == 1 ? launch(&col2im_unit_kernel<F16, 1>) : rt == 3 ? launch(&col2im_unit_kernel<F16, 3>)
-          : rt == 5 ? launch(&col2im_unit_kernel<F16, 5>) : launch(&col2im_unit_kernel<F16, 0>);
+        auto pick = [&](auto type, auto step) {
+          using T = decltype(type);
+          constexpr int ST = decltype(step)::value;
+          rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST>) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST>)
+          : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST>) : launch(&col2im_unit_kernel<T, 0, ST>);
+        };
+        const std::integral_constant<int, 1> one;
+        const std::integral_constant<int, 2> two;
+        if (dtype == SD_BF16) st == 1 ? pick(BF16{}, one) : pick(BF16{}, two);
+        else st == 1 ? pick(F16{}, one) : pick(F16{}, two);
         return check_launch("col2im_unit");
       }
       const int np_max = (hb - 1 + (g.r - 1) * g.dil_h) / g.str_h + 1;

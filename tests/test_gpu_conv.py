@@ -124,6 +124,44 @@ def test_col2im_vs_oracle(cfg, channels_last):
 
 
 @pytest.mark.parametrize("cfg", [
+    dict(n=2, c=16, h=48, w=48, r=3, s=3, padding=(1, 1)),   # 24 x 24 outputs: the last row and column of the image meet one tap
+    dict(n=2, c=8, h=7, w=9, r=3, s=3, padding=(1, 1)),      # odd sizes
+    dict(n=2, c=24, h=14, w=14, r=1, s=1, padding=(0, 0)),   # three pixels in four meet no tap: zeros
+    dict(n=2, c=8, h=14, w=13, r=1, s=1, padding=(1, 1)),
+    dict(n=2, c=16, h=33, w=20, r=5, s=5, padding=(2, 2)),
+    dict(n=1, c=8, h=17, w=11, r=5, s=5, padding=(0, 3)),    # no padding down: the first and the last rows meet fewer taps
+    dict(n=2, c=8, h=12, w=16, r=2, s=2, padding=(0, 0)),    # taps by loop counters
+    dict(n=1, c=8, h=13, w=10, r=4, s=3, padding=(3, 1)),
+    dict(n=1, c=8, h=9, w=200, r=7, s=3, padding=(3, 1)),    # rows so long that the band shrinks
+    dict(n=3, c=8, h=10, w=10, r=3, s=3, padding=(2, 2)),    # more padding than the kernel reaches over
+])
+@pytest.mark.parametrize("channels_last", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [None, 64, 128])
+def test_col2im_with_stride_two(cfg, channels_last, dtype, bs):
+    from flash_dropout.hip import GEMM
+
+    geo = dict(padding=cfg["padding"], stride=(2, 2), dilation=(1, 1))
+    gen = torch.Generator().manual_seed(cfg["h"])
+    shape, ks = (cfg["n"], cfg["c"], cfg["h"], cfg["w"]), (cfg["r"], cfg["s"])
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], *ks, **geo)
+    rows, ncols = cfg["n"] * p_ * q_, cfg["c"] * cfg["r"] * cfg["s"]
+    g = torch.randn(rows, ncols, generator=gen).to(dtype)
+    given, mask = g.clone(), None
+    if bs:
+        mask = cpu_mask(O.mask_shape(rows, ncols, bs), 0.4, gen)
+        keep = torch.from_numpy(O.expand_keep(mask.numpy(), bs, rows, ncols))
+        given[~keep] = float("nan")  # dropped blocks are not read
+        g = torch.where(keep, g, torch.zeros_like(g))
+        mask = mask.cuda()
+    dx = GEMM().col2im(given.cuda(), shape, ks, mask=mask, block_size=bs, channels_last=channels_last, **geo)
+    ref = torch.from_numpy(O.col2im(g.double().numpy(), shape, *ks, **geo))
+    # one rounding to the element type of a sum of fewer than 32 terms in fp32
+    eps = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert bool(((dx.cpu().double() - ref).abs() <= eps * ref.abs() + 2.0 ** -18).all())
+
+
+@pytest.mark.parametrize("cfg", [
     dict(n=8, c=64, h=32, w=32, k=128, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),
     dict(n=4, c=24, h=17, w=15, k=40, r=3, s=3, padding=(1, 0), stride=(2, 1), dilation=(1, 1)),
 ])
