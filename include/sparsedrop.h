@@ -497,6 +497,13 @@ int sd_conv2d_dx(const void* dy, int64_t dy_ld, const void* weight, int64_t weig
                  int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
                  int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
                  int64_t block_size, float scale, int dtype, void* stream);
+/* The same for masks of any multiple of 64: an entry stands for its block_size / 64 blocks in each direction. */
+int sd_conv2d_dx_blocks(const void* dy, int64_t dy_ld, const void* weight, int64_t weight_ld,
+                        void* dx, int64_t dx_stride_n, int64_t dx_stride_c, int64_t dx_stride_h, int64_t dx_stride_w,
+                        const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c,
+                        int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                        int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
+                        int64_t block_size, float scale, int dtype, void* stream);
 
 int64_t sd_conv2d_dw_workspace_bytes(int64_t n, int64_t c, int64_t k_out, int64_t r, int64_t s, int64_t p, int64_t q);
 int sd_conv2d_dw_lists(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_stride_h,

@@ -413,7 +413,7 @@ int conv_dw_splits(int64_t M, int64_t N, int64_t K);
 // input gradient of the stride-1 convolution straight from dY and the weights (kept 64 x 64 tiles of the patch
 // matrix's gradient are formed and folded in LDS); SD_ERR_UNSUPPORTED without a message for what it does not take
 int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, void* dx, int64_t sn, int64_t sc,
-                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t n, int64_t c,
+                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t split, int64_t n, int64_t c,
                    int64_t h, int64_t wd, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
                    int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype,
                    hipStream_t stream);

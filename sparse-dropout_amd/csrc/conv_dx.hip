@@ -67,7 +67,8 @@ struct DxArgs {
   int64_t w_ld;
   uint16_t* dx;        // [N, C, H, W] by element strides
   int64_t sn, sc, sh, sw;
-  const uint8_t* mask;  // [N*P*Q/64, ceil(C*R*S/64)] bytes, non-zero = dropped; null = keep everything
+  const uint8_t* mask;  // a byte per `split` x `split` blocks of 64, non-zero = dropped; null = keep everything
+  int split;
   int64_t msr, msc;
   int C, H, W, P, Q, R, S, pad_h, pad_w;
   int sth, stw, dlh, dlw;  // strides and dilations
@@ -109,7 +110,14 @@ __global__ __launch_bounds__(THREADS) void conv_dx_kernel(DxArgs g) {
     const int pb = pb0 + b;
     const bool valid = pb >= 0 && pb < pbn;
     bool k = valid && lane < g.Kb;
-    if (k && g.mask) k = g.mask[((int64_t)img * g.blocks_per_img + pb) * g.msr + lane * g.msc] == 0;
+    if (k && g.mask) {
+      int rb = img * g.blocks_per_img + pb, cb = lane;
+      if (g.split != 1) {
+        rb /= g.split;
+        cb /= g.split;
+      }
+      k = g.mask[(int64_t)rb * g.msr + (int64_t)cb * g.msc] == 0;
+    }
     const uint64_t bits = __ballot(k);
     if (tid == 0) keep[b] = bits;
   }
@@ -302,7 +310,7 @@ int launch_t(const DxArgs& g, int64_t wgs, hipStream_t stream) {
 
 // Returns SD_ERR_UNSUPPORTED (no message, nothing launched) for geometries the kernel does not take.
 int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, void* dx, int64_t sn, int64_t sc,
-                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t n, int64_t c,
+                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t split, int64_t n, int64_t c,
                    int64_t h, int64_t wd, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
                    int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype,
                    hipStream_t stream) {
@@ -333,7 +341,7 @@ int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, v
   if (!align_ok) return SD_ERR_UNSUPPORTED;
   const int64_t bands = (h + HB - 1) / HB;
   const int64_t wgs = n * bands;
-  if (wgs > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
+  if (wgs > 0x7fffffffLL || n * (P * Q / BS) > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
   DxArgs g;
   g.dy = static_cast<const uint16_t*>(dy);
   g.dy_ld = dy_ld;
@@ -345,6 +353,7 @@ int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, v
   g.sh = sh;
   g.sw = sw;
   g.mask = mask;
+  g.split = (int)split;
   g.msr = msr;
   g.msc = msc;
   g.C = (int)c;

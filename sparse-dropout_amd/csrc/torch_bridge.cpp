@@ -701,30 +701,15 @@ Tensor new_image(const Tensor& like, const ConvGeom& g, bool channels_last) {
                                                                                      : at::MemoryFormat::Contiguous));
 }
 
-// The mask on the 64 grid the fused input gradient works on: every entry of a larger block size repeated.
-Tensor mask_on_64_grid(const Tensor& like, const Lists& l) {
-  Tensor m = l.given.defined() ? l.given
-                               : at::from_blob(l.drawn(), {l.mb, l.kb}, like.options().dtype(at::kBool));
-  const int64_t f = l.bs / 64;
-  if (f == 1) return m;
-  m = m.repeat_interleave(f, 0).repeat_interleave(f, 1);
-  return m.narrow(0, 0, l.out_mb).narrow(1, 0, l.out_kb).contiguous();
-}
-
 Tensor conv_dx(const Tensor& dy2, const Tensor& w2, const ConvGeom& g, const Lists* l, float scale, bool channels_last) {
-  Tensor m64;
-  MaskArg m;
-  if (l) {
-    m64 = mask_on_64_grid(dy2, *l);
-    m = MaskArg(m64);
-  }
+  const MaskArg m = l ? l->mask() : MaskArg();
   Tensor dx = new_image(dy2, g, channels_last);
   c10::DeviceGuard guard(dy2.device());
-  const int rc = sd_conv2d_dx(dy2.data_ptr(), dy2.stride(0), w2.data_ptr(), w2.stride(0), dx.data_ptr(), STRIDES4(dx),
-                              m.ptr, m.sr, m.sc, GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), 64, scale, dtype_of(dy2),
-                              stream_of(dy2));
+  const int rc = sd_conv2d_dx_blocks(dy2.data_ptr(), dy2.stride(0), w2.data_ptr(), w2.stride(0), dx.data_ptr(), STRIDES4(dx),
+                                     m.ptr, m.sr, m.sc, GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), l ? l->bs : 64, scale, dtype_of(dy2),
+                                     stream_of(dy2));
   if (rc == SD_ERR_UNSUPPORTED) return Tensor();
-  check(rc, "sd_conv2d_dx");
+  check(rc, "sd_conv2d_dx_blocks");
   return dx;
 }
 
