@@ -136,14 +136,32 @@ constexpr int PATCH_MAX_BYTES = 48 * 1024;
 constexpr int PATCH_ROWS_MAX = 256;
 constexpr int64_t PATCH_WORKGROUPS = 1024;
 
+// V elements, moved at once where they are more than one
+template <int V>
+struct Piece {
+  typedef uint16_t Vec __attribute__((ext_vector_type(V)));
+  Vec v;
+  __device__ inline Piece() : v(0) {}
+  __device__ inline void load(const uint16_t* p) { v = *reinterpret_cast<const Vec*>(p); }
+  __device__ inline void store(uint16_t* p) const { *reinterpret_cast<Vec*>(p) = v; }
+  __device__ inline uint16_t at(int i) const { return v[i]; }
+};
+template <>
+struct Piece<1> {
+  uint16_t v = 0;
+  __device__ inline void load(const uint16_t* p) { v = *p; }
+  __device__ inline void store(uint16_t* p) const { *p = v; }
+  __device__ inline uint16_t at(int) const { return v; }
+};
+
 __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __restrict__ x,
                                                            uint16_t* __restrict__ cols, int64_t ld,
                                                            ConvGeom g, const int32_t* row_ptr,
-                                                           const int32_t* col_idx, int bs, int wp,
-                                                           int tpg, int gpw) {
+                                                           const int32_t* col_idx, int bs, int wp, int padl,
+                                                           int vec, int tpg, int gpw) {
   extern __shared__ __attribute__((aligned(16))) char patch_mem[];
   int* col_off = reinterpret_cast<int*>(patch_mem);                     // [tpg * 64]: offset of a column in the copy
-  uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp]
+  uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp], pixel 0 of a row at column padl
   __shared__ int64_t src_row[PATCH_ROWS_MAX];  // element offset of an input row in x (channel 0), -1: zeros
   const int t = threadIdx.x;
   const int ncols = g.c * g.r * g.s;
@@ -181,13 +199,13 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
     row_off[i] = 0;
     if (row < rows) {
       const int n = (int)(row / pq), at = (int)(row - (int64_t)n * pq), pp = at / g.q;
-      row_off[i] = (base_of(n) + (pp - (n == n_lo ? p_first : 0)) * g.str_h) * wp + (at - pp * g.q) * g.str_w;
+      row_off[i] = (base_of(n) + (pp - (n == n_lo ? p_first : 0)) * g.str_h) * wp + (at - pp * g.q) * g.str_w + padl - g.pad_w;
     }
   }
 
   const int sub_per_block = bs / TILE;
   const int ntiles = (ncols + TILE - 1) / TILE;
-  const int per_ch = hp * wp;
+  const int per_ch = hp * wp, ch_unit = g.xs_c == 1 && g.xs_w != 1 ? vec : 1;
   // column tiles [t_lo, t_hi) are this workgroup's
   const int t_lo = (int)blockIdx.y * gpw * tpg, t_hi = t_lo + gpw * tpg < ntiles ? t_lo + gpw * tpg : ntiles;
   int32_t pos = 0, end = 0;
@@ -224,56 +242,76 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
     if (ct / tpg != group) {  // the same for every thread
       group = ct / tpg;
       const int g0 = group * tpg * TILE, g_end = g0 + tpg * TILE < ncols ? g0 + tpg * TILE : ncols;
-      const int ch_lo = g0 / rs_n, nch = (g_end - 1) / rs_n - ch_lo + 1;
+      const int ch_hi = (g_end - 1) / rs_n + 1, ch_lo = g0 / rs_n / ch_unit * ch_unit;  // whole pieces of a channels-last pixel
+      const int nch = (ch_hi - ch_lo + ch_unit - 1) / ch_unit * ch_unit;
       __syncthreads();  // src_row is written; nobody reads the previous group's copy any more
-      // A channels-last image is read along the channels, any other along its rows, LW lanes to a line and four lines'
-      // loads ahead of their stores.  Copying costs instructions, not bytes: no division per line along the rows.
+      // Copying costs instructions, not bytes, so up to 16 bytes move at a time: V channels of a pixel of a channels-last image (V = 8
+      // or 1), V pixels of a row of any other (8, 4, 2 or 1, whatever row length and alignment allow), four rows' loads
+      // ahead of their stores, no division anywhere.  199 x 32 x 48 x 48 channels last, 3 x 3 by two, p = 0.25: 91 us with
+      // 2 bytes and a division each, 52 so; 16 x 96 x 48 x 48 channels last, pointwise by two, p = 0.6: 36 and 10.
       if (g.xs_c == 1 && g.xs_w != 1) {
-        for (int ci = t % 32; ci < nch; ci += 32)
-          for (int line0 = t / 32; line0 < per_ch; line0 += 32) {
-            uint16_t v[4];
+        auto along_channels = [&](auto width) {
+          constexpr int V = decltype(width)::value, LC = V == 8 ? 4 : 32;  // lanes along the channels
+          for (int ci = t % LC * V; ci < nch; ci += LC * V)
+            for (int w0 = t / LC % (64 / LC); w0 < wp; w0 += 64 / LC) {
+              const int ww = w0 - padl;
+              const bool w_ok = ww >= 0 && ww < g.w;
+              const uint16_t* xc = x + (int64_t)ww * g.xs_w + ch_lo + ci;
+              uint16_t* to = patch + ci * per_ch + w0;
+              for (int h0 = t / 64; h0 < hp; h0 += 16) {
+                Piece<V> v[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const int line = line0 + 8 * k;
-              v[k] = 0;
-              if (line < per_ch) {
-                const int hr = line / wp, ww = line - hr * wp - g.pad_w;
-                const int64_t so = src_row[hr];
-                if (so >= 0 && ww >= 0 && ww < g.w) v[k] = x[so + (int64_t)ww * g.xs_w + ch_lo + ci];
+                for (int k = 0; k < 4; ++k) {
+                  v[k] = Piece<V>();
+                  const int64_t so = w_ok && h0 + 4 * k < hp ? src_row[h0 + 4 * k] : -1;
+                  if (so >= 0) v[k].load(xc + so);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                  if (h0 + 4 * k < hp) {
+#pragma unroll
+                    for (int j = 0; j < V; ++j) to[j * per_ch + (h0 + 4 * k) * wp] = v[k].at(j);
+                  }
               }
             }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-              if (line0 + 8 * k < per_ch) patch[ci * per_ch + line0 + 8 * k] = v[k];
-          }
+        };
+        if (vec == 8) along_channels(std::integral_constant<int, 8>{});
+        else along_channels(std::integral_constant<int, 1>{});
       } else {
-        auto along_rows = [&](auto lanes) {
-          constexpr int LW = decltype(lanes)::value;
-          for (int w0 = t % LW; w0 < wp; w0 += LW) {
-            const int ww = w0 - g.pad_w;
+        auto along_rows = [&](auto width, auto lanes) {
+          constexpr int V = decltype(width)::value, LW = decltype(lanes)::value;
+          for (int w0 = t % LW * V; w0 < wp; w0 += LW * V) {
+            const int ww = w0 - padl;
             const bool w_ok = ww >= 0 && ww < g.w;
             for (int ci = t / LW; ci < nch; ci += 256 / LW) {
               const uint16_t* xc = x + (int64_t)(ch_lo + ci) * g.xs_c + (int64_t)ww * g.xs_w;
               uint16_t* to = patch + ci * per_ch + w0;
               for (int h0 = 0; h0 < hp; h0 += 4) {
-                uint16_t v[4];
+                Piece<V> v[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                  v[k] = 0;
-                  if (w_ok && h0 + k < hp) {
-                    const int64_t so = src_row[h0 + k];
-                    if (so >= 0) v[k] = xc[so];
-                  }
+                  v[k] = Piece<V>();
+                  const int64_t so = w_ok && h0 + k < hp ? src_row[h0 + k] : -1;
+                  if (so >= 0) v[k].load(xc + so);
                 }
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                  if (h0 + k < hp) to[(h0 + k) * wp] = v[k];
+                  if (h0 + k < hp) v[k].store(to + (h0 + k) * wp);
               }
             }
           }
         };
-        if (wp <= 16) along_rows(std::integral_constant<int, 16>{});
-        else along_rows(std::integral_constant<int, 32>{});
+        auto lanes_for = [&](auto width) {
+          constexpr int V = decltype(width)::value;
+          if (wp <= 4 * V) along_rows(width, std::integral_constant<int, 4>{});
+          else if (wp <= 8 * V) along_rows(width, std::integral_constant<int, 8>{});
+          else if (wp <= 16 * V) along_rows(width, std::integral_constant<int, 16>{});
+          else along_rows(width, std::integral_constant<int, 32>{});
+        };
+        if (vec == 8) lanes_for(std::integral_constant<int, 8>{});
+        else if (vec == 4) lanes_for(std::integral_constant<int, 4>{});
+        else if (vec == 2) lanes_for(std::integral_constant<int, 2>{});
+        else lanes_for(std::integral_constant<int, 1>{});
       }
       for (int i = t; i < tpg * TILE; i += 256) {
         const int col = g0 + i;
@@ -635,13 +673,29 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
   const int64_t spread = out_rows < images ? out_rows : images;
   const int64_t one = (out_rows - 1) * g.str_h + reach, many = (out_rows - spread) * g.str_h + spread * reach;
   const int64_t hp = one > many ? one : many;
-  const int64_t wp = (int64_t)(g.q - 1) * g.str_w + (int64_t)(g.s - 1) * g.dil_w + 1;
+  // what is copied at a time: channels of a pixel, or pixels of a row, whose copy then starts and ends on whole pieces
+  const bool pixelwise = g.xs_c == 1 && g.xs_w != 1;
+  auto pieces_of = [&](int64_t v) {
+    const int64_t inner = pixelwise ? g.c : g.w, near = pixelwise ? g.xs_w : g.xs_c;
+    return (pixelwise ? g.xs_c : g.xs_w) == 1 && inner % v == 0 && near % v == 0 && g.xs_h % v == 0 && g.xs_n % v == 0 &&
+           reinterpret_cast<uintptr_t>(x) % (2 * v) == 0;
+  };
+  int64_t vec = pieces_of(8) ? 8 : (pixelwise ? 1 : (pieces_of(4) ? 4 : (pieces_of(2) ? 2 : 1))), padl, wp;
+  auto copied_in = [&](int64_t v) {
+    const int64_t unit = pixelwise ? 1 : v;
+    vec = v;
+    padl = ceil_div(g.pad_w, unit) * unit;
+    wp = ceil_div(padl - g.pad_w + (int64_t)(g.q - 1) * g.str_w + (int64_t)(g.s - 1) * g.dil_w + 1, unit) * unit;
+  };
+  copied_in(vec);
   const int64_t ntiles = ceil_div(c * r * s, TILE);
   auto group_bytes = [&](int64_t tiles) {
     int64_t ch = (tiles * TILE + r * s - 2) / (r * s) + 1;
+    if (pixelwise && vec > 1) ch = (ceil_div(ch, vec) + 1) * vec;  // (the first of them need not start a piece)
     if (ch > c) ch = c;
     return tiles * TILE * 4 + (ch * hp * wp * 2 + 15) / 16 * 16;
   };
+  if (group_bytes(1) > PATCH_MAX_BYTES) copied_in(1);  // the smallest copy
   if (ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 && hp <= PATCH_ROWS_MAX &&
       group_bytes(1) <= PATCH_MAX_BYTES) {
     // as many tiles to a group as fit a quarter of the LDS a workgroup may ask for: several workgroups share a CU.  Fewer
@@ -652,7 +706,7 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
     const int64_t groups = ceil_div(ntiles, tpg), gpw = ceil_div(groups, split);
     hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks, (unsigned)ceil_div(groups, gpw)), dim3(256),
                        (size_t)group_bytes(tpg), stream, (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
-                       row_ptr ? (int)bs : TILE, (int)wp, (int)tpg, (int)gpw);
+                       row_ptr ? (int)bs : TILE, (int)wp, (int)padl, (int)vec, (int)tpg, (int)gpw);
     return check_launch("im2col_patch");
   }
   hipLaunchKernelGGL(im2col_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,

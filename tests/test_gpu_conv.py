@@ -101,6 +101,39 @@ def test_im2col_of_few_rows_deals_out_its_columns(cfg, channels_last, p, bs):
     assert torch.equal(part.cpu(), torch.where(keep, ref, torch.tensor(7.0, dtype=torch.float16)))
 
 
+@pytest.mark.parametrize("c,h,w,padding,r,s", [
+    (16, 12, 24, (1, 1), 3, 3),    # rows in pieces of 8 pixels
+    (16, 6, 28, (2, 2), 5, 5),     # of 4
+    (24, 7, 14, (0, 3), 2, 7),     # of 2, more padding than a piece
+    (8, 9, 15, (1, 1), 3, 3),      # one by one
+    (40, 8, 8, (9, 9), 3, 3),      # padding past a row's length
+    (72, 10, 10, (0, 0), 1, 1),    # channels last: pieces of 8 channels, tiles that start inside one
+    (8, 20, 48, (1, 1), 5, 5),     # 2.56 channels to a tile
+    (12, 11, 13, (1, 1), 3, 3),    # channels one by one
+])
+@pytest.mark.parametrize("stride", [(1, 1), (2, 2), (2, 1)])
+@pytest.mark.parametrize("layout", ["planes", "channels_last", "cropped", "channels", "offset"])
+def test_im2col_copies_in_pieces(c, h, w, padding, r, s, stride, layout):
+    """Images whose rows or pixels can be copied several elements at a time, and slices of larger ones that cannot."""
+    from flash_dropout.hip import GEMM
+
+    gen = torch.Generator().manual_seed(w)
+    n, geo = 3, dict(padding=padding, stride=stride, dilation=(1, 1))
+    if layout == "cropped":      # rows four pixels longer than the image's
+        x = torch.randn(n, c, h, w + 4, generator=gen).half().cuda()[..., 2:2 + w]
+    elif layout == "channels":   # some of a channels-last image's channels
+        x = torch.randn(n, c + 5, h, w, generator=gen).half().cuda().contiguous(memory_format=torch.channels_last)[:, 3:3 + c]
+    elif layout == "offset":     # a tensor that starts 2 bytes behind a boundary
+        x = torch.randn(n * c * h * w + 1, generator=gen).half().cuda()[1:].view(n, c, h, w)
+    else:
+        x = torch.randn(n, c, h, w, generator=gen).half().cuda()
+        if layout == "channels_last":
+            x = x.contiguous(memory_format=torch.channels_last)
+    cols = GEMM().im2col(x, (r, s), **geo)
+    ref = O.im2col(x.float().cpu().numpy(), r, s, **geo)
+    assert np.array_equal(cols.float().cpu().numpy(), ref)
+
+
 @pytest.mark.parametrize("cfg", GEOMS)
 @pytest.mark.parametrize("channels_last", [False, True])
 def test_col2im_vs_oracle(cfg, channels_last):
