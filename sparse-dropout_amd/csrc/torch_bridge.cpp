@@ -669,6 +669,18 @@ Tensor pixel_rows(const Tensor& x) {
   return pixels ? x.as_strided({x.size(0) * h * w, c}, {c, 1}) : Tensor();
 }
 
+// Which products of a masked convolution that the library takes without a patch matrix go through one all the same (the image is
+// what is kept then too, and gathered once more for the kernel's gradient).  Measured on 298 drawn layers of 24 to 950 thousand
+// rows, 32 fused input gradients among them; times through the matrix against those without, geometric means:
+//  * forward: a workgroup takes 256 rows x 128 outputs and builds its tiles step by step; fewer than 64 of them 0.67 (9 x 96 x 8 x 8 ->
+//    192, 5 x 5, p = 0.5, six of them: 45 us a pass for 306), 64 to 128 1.02, more 1.3; pointwise kernels, a step each, 1.04 to 1.3
+//  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16
+//  * input gradient, SDD and col2im against the fused kernel: 0.35, 1.03 at most, 0.6 to 0.85 on 42 to 130 MB (187 x 48 x 32 x 32 -> 64
+//    by two 102 -> 85 us a pass); 1.03 to 1.09 where the matrix is one block wide.  Past 256 MB it stays out of memory.
+bool forward_by_patches(const ConvGeom& g) { return g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64; }
+bool dw_by_patches(const ConvGeom& g) { return g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
+bool dx_by_patches(const ConvGeom& g) { return g.cols() > 64 && g.rows() * g.cols() * 2 <= 256LL << 20; }
+
 Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
   if (pointwise(g) && g.c % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0) {
     const Tensor rows = pixel_rows(x);
@@ -857,7 +869,7 @@ struct ConvBackward : Node {
     const float scale = (float)(1.0 / (1.0 - p));
     if (task_should_compute_output(0)) {
       Tensor dx;
-      if (fused_dx) dx = conv_dx(dy2, w, g, l, scale, channels_last);
+      if (fused_dx && !(l && dx_by_patches(g))) dx = conv_dx(dy2, w, g, l, scale, channels_last);
       last_routes[1] = dx.defined() ? kFused : kExplicit;
       if (!dx.defined()) {
         dx = new_image(dy2, g, channels_last);
@@ -891,8 +903,8 @@ struct ConvBackward : Node {
     if (task_should_compute_output(1)) {
       Tensor dk;
       if (pixels) patches = im2col(image, g, l);
-      if (!patches.defined()) {  // the forward was implicit
-        dk = conv_dw(image, dy2, g, l, scale);
+      if (!patches.defined()) {  // the image was kept
+        if (!(l && dw_by_patches(g))) dk = conv_dw(image, dy2, g, l, scale);
         if (!dk.defined()) patches = im2col(image, g, l);
       }
       last_routes[2] = dk.defined() ? kImplicit : kExplicit;
@@ -987,7 +999,9 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     y2 = new_matrix(x, g.rows(), g.k);
     bool done = false;
     c10::DeviceGuard device(x.device());
-    if (implicit_forward) {  // no patch matrix in memory where the library takes the geometry
+    const bool takes_implicit = implicit_forward && sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(),
+                                                                              GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
+    if (takes_implicit && !(bs && forward_by_patches(g))) {  // no patch matrix in memory
       const int rc = sd_conv2d_dsd_lists(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(), y2.data_ptr(),
                                          y2.stride(0), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), l ? l->row_ptr() : nullptr,
                                          l ? l->col_idx() : nullptr, l ? l->kernel_bs : 0, scale, dtype_of(x),
@@ -1012,6 +1026,8 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
         check(sd_gemm(MAT(am), MAT(bm), MAT(cm), g.rows(), g.k, g.cols(), dtype_of(x), ws.ptr, ws.bytes, stream_of(x)),
               "sd_gemm");
     }
+    // (in the geometries that the implicit products take the image is kept, and gathered once more for the kernel's gradient)
+    if (takes_implicit) cols = Tensor();
     // the result is an (N, K, P, Q) view of an (N, P*Q, K) buffer, as the reference's is (im2col_conv2d.py:26-27)
     y = y2.view({g.n, g.po, g.qo, g.k}).permute({0, 3, 1, 2});
   }

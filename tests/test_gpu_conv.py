@@ -571,3 +571,53 @@ def test_conv_routes_are_reported_and_block_sizes_above_64_stay_fused(bs, dx_rou
             assert max_tile_rel_fro(xg.grad, rdx) <= REL_FRO_TOL
         finally:
             mod.IMPLICIT_FORWARD, mod.FUSED_INPUT_GRADIENT = old
+
+
+@pytest.mark.parametrize("cfg,p,routes", [
+    # few rows: gather and small tiles
+    (dict(n=9, c=24, h=8, w=8, k=64, r=3, s=3, stride=(1, 1), padding=(1, 1)), 0.5, ("explicit", "explicit", "explicit")),
+    (dict(n=6, c=16, h=16, w=16, k=64, r=5, s=5, stride=(2, 2), padding=(2, 2)), 0.3, ("explicit", "explicit", "explicit")),
+    (dict(n=4, c=16, h=32, w=32, k=64, r=2, s=2, stride=(2, 2), padding=(0, 0)), 0.0, ("explicit", "fused", "explicit")),  # one block wide
+    # 63 and 64 workgroups of the implicit forward, below 8192 rows and not
+    (dict(n=31, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("explicit", "explicit", "explicit")),
+    (dict(n=63, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("explicit", "explicit", "implicit")),
+    (dict(n=64, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("implicit", "explicit", "implicit")),
+    # pointwise kernels: the forward stays implicit, the kernel's gradient from 16384 rows on
+    (dict(n=15, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("implicit", "fused", "explicit")),
+    (dict(n=16, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("implicit", "fused", "implicit")),
+    # 300 MB of patch gradient stay out of memory
+    (dict(n=192, c=32, h=64, w=64, k=64, r=5, s=5, stride=(2, 2), padding=(2, 2)), 0.9, ("implicit", "fused", "implicit")),
+])
+def test_masked_convolutions_go_through_a_patch_matrix_where_that_is_faster(cfg, p, routes):
+    import flash_dropout.functional as F
+
+    gen = torch.Generator().manual_seed(cfg["n"])
+    geo = dict(padding=cfg["padding"], stride=cfg["stride"], dilation=(1, 1))
+    fan_in = cfg["c"] * cfg["r"] * cfg["s"]
+    x = torch.randn(cfg["n"], cfg["c"], cfg["h"], cfg["w"], generator=gen).half()
+    k = (torch.randn(cfg["k"], cfg["c"], cfg["r"], cfg["s"], generator=gen) * fan_in ** -0.5).half()
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], cfg["r"], cfg["s"], **geo)
+    rows = cfg["n"] * p_ * q_
+    mask = cpu_mask(O.mask_shape(rows, fan_in, 64), p, gen)
+    dy = torch.randn(cfg["n"], cfg["k"], p_, q_, generator=gen).half()
+    xg, kg = x.cuda().requires_grad_(), k.cuda().requires_grad_()
+    call = lambda: F.blockwise_dropout_conv2d_mask(xg, mask.cuda(), 64, p, kg, **geo)
+    y = call()
+    y.backward(dy.cuda())
+    assert tuple(F.conv_last_routes()[n] for n in ("forward", "dx", "dw")) == routes
+    if cfg["n"] < 100:
+        ry, rdx, rdk = O.conv2d_blockdrop(to_np(x), to_np(k), mask.numpy(), 64, p, dy=to_np(dy), dtype=np.float32, **geo)
+        assert max_tile_rel_fro(y, ry) <= REL_FRO_TOL
+        assert max_tile_rel_fro(xg.grad, rdx) <= REL_FRO_TOL
+        assert max_tile_rel_fro(kg.grad, rdk) <= REL_FRO_TOL
+    # the image is kept, whichever way the products went: a write to it before the backward is refused
+    y = call()
+    with torch.no_grad():
+        xg.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward(dy.cuda())
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+        y = call()
+    assert tuple(x.shape) in kept and (rows, fan_in) not in kept
+    y.backward(dy.cuda())
