@@ -377,6 +377,17 @@ int sd_dropout_matmul_backward(const void* dY, int64_t dy_stride_r, int64_t dy_s
                                int64_t M, int64_t N, int64_t K, int64_t block_size, double p, int dtype,
                                void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same with dropped blocks of dX left as they are, for callers that do not read them (sd_col2im with the mask). */
+int sd_dropout_matmul_backward_kept(const void* dY, int64_t dy_stride_r, int64_t dy_stride_c,
+                                    const void* W, int64_t w_stride_r, int64_t w_stride_c,
+                                    const void* X, int64_t x_stride_r, int64_t x_stride_c,
+                                    void* dX, int64_t dx_stride_r, int64_t dx_stride_c,
+                                    void* dW, int64_t dw_stride_r, int64_t dw_stride_c,
+                                    const int32_t* row_ptr, const int32_t* col_idx,
+                                    const int32_t* col_ptr, const int32_t* row_idx,
+                                    int64_t M, int64_t N, int64_t K, int64_t block_size, double p, int dtype,
+                                    void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The same with the derivative of an activation multiplied into dX (sd_gemm_sdd_lists_actgrad's epilogue):
  * dX = (dY . W) . keep / (1 - p) * act'(act_at[m, k]), for a layer whose input is act(previous layer's output);
  * act = SD_ACT_NONE is the plain call.  No counterpart in the reference, whose layers run the activation gradient as a
@@ -435,6 +446,18 @@ int sd_im2col(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_s
               int64_t dil_h, int64_t dil_w,
               const int32_t* row_ptr, const int32_t* col_idx, int64_t block_size,
               int dtype, void* stream);
+
+/* The same for the blocks that a mask keeps, before there are lists of it: a stored mask (one byte per block, strides in
+ * bytes), or with mask NULL the draw that sd_random_lists (seed, offset) or sd_random_lists_state (state, which is read
+ * and not moved on) makes.  block_size: a multiple of 64. */
+int sd_im2col_masked(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_stride_h,
+                     int64_t x_stride_w, void* cols, int64_t cols_ld,
+                     int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
+                     int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
+                     int64_t dil_h, int64_t dil_w,
+                     const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c,
+                     const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t block_size,
+                     int dtype, void* stream);
 
 int sd_col2im(const void* cols, int64_t cols_ld, void* dx, int64_t dx_stride_n,
               int64_t dx_stride_c, int64_t dx_stride_h, int64_t dx_stride_w,

@@ -29,6 +29,11 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
            int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
            int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
            const int32_t* row_ptr, const int32_t* col_idx, int64_t bs, hipStream_t stream);
+int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
+                  int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
+                  int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
+                  int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t mb,
+                  int64_t kb, int64_t bs, hipStream_t stream);
 int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
            int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
            int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
@@ -592,6 +597,62 @@ int sd_dropout_matmul_forward_act(const void* X, int64_t xsr, int64_t xsc, const
                                stream);
 }
 
+// kept_only: dropped blocks of dX are left as they are instead of being zeroed
+static int dropout_matmul_backward(const void* dY, int64_t gsr, int64_t gsc, const void* W, int64_t wsr, int64_t wsc,
+                                   const void* X, int64_t xsr, int64_t xsc, void* dX, int64_t dxsr, int64_t dxsc,
+                                   void* dW, int64_t dwsr, int64_t dwsc, const int32_t* row_ptr,
+                                   const int32_t* col_idx, const int32_t* col_ptr, const int32_t* row_idx, int64_t M,
+                                   int64_t N, int64_t K, int64_t bs, double p, int dtype, int act, const void* act_at,
+                                   int64_t at_stride_r, int64_t at_stride_c, void* workspace, int64_t workspace_bytes,
+                                   int kept_only, void* stream) {
+  SD_REQUIRE(p >= 0.f && p < 1.f, "dropout_matmul_backward: p must be in [0, 1) (got %g)", (double)p);
+  if (dX) {
+    if (int rc = check_act(act, act_at, at_stride_r, at_stride_c, M, K, true)) return rc;
+  }
+  if (int rc = check_sparse(bs, 1.f)) return rc;
+  SD_REQUIRE(dX || dW, "dropout_matmul_backward: nothing to compute");
+  const int64_t g = lists_block_size(bs);  // 32: lists on the 64 grid with quadrant bits
+  const float scale = (float)(1.0 / (1.0 - p));  // in double, as the reference's Python evaluates it
+  if (dX && dW && row_ptr && col_idx && col_ptr && row_idx && !generic_forced() && !separate_backward_forced()) {
+    // both gradients in one launch where the pair qualifies (same operands and checks as the two calls below)
+    if (int rc = check_common(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, M, K, N, dtype)) return rc;
+    if (int rc = check_common(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, K, N, M, dtype)) return rc;
+    GemmArgs gx = make_args(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, M, K, N, g, scale, row_ptr, col_idx);
+    gx.keep_hint = (float)(1.0 - p);
+    gx.kept_only = kept_only != 0;
+    gx.act = act;
+    gx.aux = act != SD_ACT_NONE ? const_cast<uint16_t*>(static_cast<const uint16_t*>(act_at)) : nullptr;
+    gx.aux_sr = at_stride_r;
+    gx.aux_sc = at_stride_c;
+    GemmArgs gw = make_args(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, K, N, M, g, scale, col_ptr, row_idx, workspace,
+                            workspace_bytes);
+    const int rc = launch_backward_pair(gx, gw, dtype, (hipStream_t)stream);
+    if (rc != SD_ERR_UNSUPPORTED) {
+      last_kernel = "specialised";
+      return rc;
+    }
+  }
+  if (dX) {
+    // dX[M,K] = scale * (dY[M,N] . W[N,K]) where kept: A = dY, B = W^T as the [K, N] view of W
+    SD_REQUIRE(row_ptr && col_idx, "dropout_matmul_backward: dX needs the CSR lists");
+    if (kept_only) {
+      if (int rc = sd_gemm_sdd_lists_ex(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, row_ptr, col_idx, M, K, N, g, scale, dtype, 1,
+                                        (float)(1.0 - p), stream))
+        return rc;
+    } else if (int rc = sd_gemm_sdd_lists_actgrad(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, row_ptr, col_idx, M, K, N, g,
+                                           scale, dtype, act, act_at, at_stride_r, at_stride_c, (float)(1.0 - p), stream))
+      return rc;
+  }
+  if (dW) {
+    // dW^T[K,N] = scale * X^T[K,M] (kept blocks) . dY[M,N]: A = X^T, B = dY^T, C = dW^T, lists of the transposed mask
+    SD_REQUIRE(col_ptr && row_idx, "dropout_matmul_backward: dW needs the CSC lists");
+    if (int rc = sd_gemm_dsd_lists(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, col_ptr, row_idx, K, N, M, g, scale, dtype,
+                                   workspace, workspace_bytes, stream))
+      return rc;
+  }
+  return SD_OK;
+}
+
 int sd_dropout_matmul_backward(const void* dY, int64_t gsr, int64_t gsc, const void* W, int64_t wsr, int64_t wsc,
                                const void* X, int64_t xsr, int64_t xsc, void* dX, int64_t dxsr, int64_t dxsc,
                                void* dW, int64_t dwsr, int64_t dwsc, const int32_t* row_ptr, const int32_t* col_idx,
@@ -609,47 +670,18 @@ int sd_dropout_matmul_backward_act(const void* dY, int64_t gsr, int64_t gsc, con
                                    int64_t N, int64_t K, int64_t bs, double p, int dtype, int act, const void* act_at,
                                    int64_t at_stride_r, int64_t at_stride_c, void* workspace, int64_t workspace_bytes,
                                    void* stream) {
-  SD_REQUIRE(p >= 0.f && p < 1.f, "dropout_matmul_backward: p must be in [0, 1) (got %g)", (double)p);
-  if (dX) {
-    if (int rc = check_act(act, act_at, at_stride_r, at_stride_c, M, K, true)) return rc;
-  }
-  if (int rc = check_sparse(bs, 1.f)) return rc;
-  SD_REQUIRE(dX || dW, "dropout_matmul_backward: nothing to compute");
-  const int64_t g = lists_block_size(bs);  // 32: lists on the 64 grid with quadrant bits
-  const float scale = (float)(1.0 / (1.0 - p));  // in double, as the reference's Python evaluates it
-  if (dX && dW && row_ptr && col_idx && col_ptr && row_idx && !generic_forced() && !separate_backward_forced()) {
-    // both gradients in one launch where the pair qualifies (same operands and checks as the two calls below)
-    if (int rc = check_common(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, M, K, N, dtype)) return rc;
-    if (int rc = check_common(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, K, N, M, dtype)) return rc;
-    GemmArgs gx = make_args(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, M, K, N, g, scale, row_ptr, col_idx);
-    gx.keep_hint = (float)(1.0 - p);
-    gx.act = act;
-    gx.aux = act != SD_ACT_NONE ? const_cast<uint16_t*>(static_cast<const uint16_t*>(act_at)) : nullptr;
-    gx.aux_sr = at_stride_r;
-    gx.aux_sc = at_stride_c;
-    GemmArgs gw = make_args(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, K, N, M, g, scale, col_ptr, row_idx, workspace,
-                            workspace_bytes);
-    const int rc = launch_backward_pair(gx, gw, dtype, (hipStream_t)stream);
-    if (rc != SD_ERR_UNSUPPORTED) {
-      last_kernel = "specialised";
-      return rc;
-    }
-  }
-  if (dX) {
-    // dX[M,K] = scale * (dY[M,N] . W[N,K]) where kept: A = dY, B = W^T as the [K, N] view of W
-    SD_REQUIRE(row_ptr && col_idx, "dropout_matmul_backward: dX needs the CSR lists");
-    if (int rc = sd_gemm_sdd_lists_actgrad(dY, gsr, gsc, W, wsc, wsr, dX, dxsr, dxsc, row_ptr, col_idx, M, K, N, g,
-                                           scale, dtype, act, act_at, at_stride_r, at_stride_c, (float)(1.0 - p), stream))
-      return rc;
-  }
-  if (dW) {
-    // dW^T[K,N] = scale * X^T[K,M] (kept blocks) . dY[M,N]: A = X^T, B = dY^T, C = dW^T, lists of the transposed mask
-    SD_REQUIRE(col_ptr && row_idx, "dropout_matmul_backward: dW needs the CSC lists");
-    if (int rc = sd_gemm_dsd_lists(X, xsc, xsr, dY, gsc, gsr, dW, dwsc, dwsr, col_ptr, row_idx, K, N, M, g, scale, dtype,
-                                   workspace, workspace_bytes, stream))
-      return rc;
-  }
-  return SD_OK;
+  return dropout_matmul_backward(dY, gsr, gsc, W, wsr, wsc, X, xsr, xsc, dX, dxsr, dxsc, dW, dwsr, dwsc, row_ptr, col_idx, col_ptr,
+                                 row_idx, M, N, K, bs, p, dtype, act, act_at, at_stride_r, at_stride_c, workspace,
+                                 workspace_bytes, 0, stream);
+}
+
+int sd_dropout_matmul_backward_kept(const void* dY, int64_t gsr, int64_t gsc, const void* W, int64_t wsr, int64_t wsc,
+                                    const void* X, int64_t xsr, int64_t xsc, void* dX, int64_t dxsr, int64_t dxsc,
+                                    void* dW, int64_t dwsr, int64_t dwsc, const int32_t* row_ptr, const int32_t* col_idx,
+                                    const int32_t* col_ptr, const int32_t* row_idx, int64_t M, int64_t N, int64_t K,
+                                    int64_t bs, double p, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return dropout_matmul_backward(dY, gsr, gsc, W, wsr, wsc, X, xsr, xsc, dX, dxsr, dxsc, dW, dwsr, dwsc, row_ptr, col_idx, col_ptr,
+                                 row_idx, M, N, K, bs, p, dtype, SD_ACT_NONE, nullptr, 0, 0, workspace, workspace_bytes, 1, stream);
 }
 
 int sd_im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
@@ -659,6 +691,24 @@ int sd_im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, voi
   SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "dtype must be SD_F16 or SD_BF16 (got %d)", dtype);
   return im2col(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h,
                 dil_w, row_ptr, col_idx, bs, (hipStream_t)stream);
+}
+
+int sd_im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
+                     int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
+                     int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
+                     int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t bs,
+                     int dtype, void* stream) {
+  SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "dtype must be SD_F16 or SD_BF16 (got %d)", dtype);
+  SD_REQUIRE(bs > 0 && bs % 64 == 0 && bs < kMaxDim, "im2col_masked: block_size must be a multiple of 64");
+  SD_REQUIRE(mask == nullptr || (msr >= 1 && msc >= 1), "im2col_masked: mask strides");
+  SD_REQUIRE(mask != nullptr || (p >= 0.f && p < 1.f), "im2col_masked: p must be in [0, 1) (got %g)", (double)p);
+  SD_REQUIRE(state == nullptr || reinterpret_cast<uintptr_t>(state) % 8 == 0, "im2col_masked: state must be an aligned device pointer");
+  SD_REQUIRE(n > 0 && c > 0 && r > 0 && s > 0 && stride_h > 0 && stride_w > 0, "im2col_masked: sizes and strides must be positive");
+  const int64_t p_out = (h + 2 * pad_h - dil_h * (r - 1) - 1) / stride_h + 1, q_out = (w + 2 * pad_w - dil_w * (s - 1) - 1) / stride_w + 1;
+  const int64_t mb = ceil_div(n * p_out * q_out, bs), kb = ceil_div(c * r * s, bs);
+  SD_REQUIRE(mb < kMaxDim && kb < kMaxDim, "im2col_masked: mask too large");
+  return im2col_masked(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, mask, msr, msc,
+                       state, seed, offset, p, mb, kb, bs, (hipStream_t)stream);
 }
 
 int sd_col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,

@@ -2323,7 +2323,7 @@ int launch_pair_t(const GemmArgs& gx, const GemmArgs& gw, int splits, hipStream_
 }
 
 int launch_backward_pair(const GemmArgs& gx, const GemmArgs& gw, int dtype, hipStream_t stream) {
-  if (!gx.row_ptr || gx.bs != BS || gx.kept_only || !sdd_operands_ok(gx)) return SD_ERR_UNSUPPORTED;
+  if (!gx.row_ptr || gx.bs != BS || !sdd_operands_ok(gx)) return SD_ERR_UNSUPPORTED;
   // the weight gradient in the one form the autograd step produces
   const DsdForm form = dsd_form(gw);
   if (!gw.row_ptr || gw.bs != BS || gw.act || !form.ok || form.kc || !form.cm || gw.c_sr != 1) return SD_ERR_UNSUPPORTED;

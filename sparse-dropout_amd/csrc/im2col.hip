@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "mask_source.h"
 
 namespace sd {
 namespace {
@@ -22,13 +23,31 @@ struct ConvGeom {
   int64_t xs_n, xs_c, xs_h, xs_w;  // element strides of the image tensor
 };
 
+// Which blocks of the patch matrix are wanted: those of a list by rows, those that a mask source keeps, or all of them.  A mask
+// source is what there is before any list: the gather needs no launch in front of it, and the product behind it makes the lists.
+struct Wanted {
+  const int32_t* row_ptr;
+  const int32_t* col_idx;
+  int bs;        // of the lists
+  bool masked;
+  MaskSrc src;   // on the 64 grid
+};
+// Bit j: column tile `first` + j of row block rb is kept.  All lanes of a wave ask together.
+__device__ inline uint64_t kept_tiles(const MaskSrc& src, int rb, int first, int ntiles) {
+  const int j = first + (int)(threadIdx.x % 64);
+  return __ballot(j < ntiles && !src.dropped(rb, j, src.one_by_one()));
+}
+
 constexpr int TILE = 64;
 constexpr int TLD = TILE + 2;  // 33 words per LDS row: both the 2-byte column writes and the 4-byte row reads are conflict-free
 
 __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict__ x,
                                                      uint16_t* __restrict__ cols, int64_t ld,
-                                                     ConvGeom g, const int32_t* row_ptr,
-                                                     const int32_t* col_idx, int bs) {
+                                                     ConvGeom g, Wanted want) {
+  const int32_t* row_ptr = want.row_ptr;
+  const int32_t* col_idx = want.col_idx;
+  const int bs = want.bs;
+  if (want.masked) want.src.resolve();
   __shared__ __attribute__((aligned(4))) uint16_t tile[TILE * TLD];  // [row][col]
   const int t = threadIdx.x;
   const int lane = t % 64;
@@ -62,6 +81,7 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict_
     end = row_ptr[rb + 1];
   }
   int sub = 0, ct = -1;
+  uint64_t kept = 0;  // of 64 tiles
   for (;;) {
     // next column tile: all of them, or the tiles of the kept blocks of this row block
     if (row_ptr) {
@@ -71,6 +91,10 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict_
       if (ct >= ntiles) continue;
     } else {
       if (++ct >= ntiles) break;
+      if (want.masked) {
+        if (ct % 64 == 0) kept = kept_tiles(want.src, (int)blockIdx.x, ct, ntiles);
+        if (!((kept >> (ct % 64)) & 1u)) continue;
+      }
     }
     const int c0 = ct * TILE;
     // gather: wave w takes columns w, w+4, ...; the column's (c, r, s) is wave-uniform
@@ -154,11 +178,17 @@ struct Piece<1> {
   __device__ inline uint16_t at(int) const { return v; }
 };
 
+// V, PIXELS: how much is copied at a time (see below).  MASKED: the wanted blocks are those of a mask source.  Each is an instance of its own
+// since with all in one the kernel took 170 registers, two or three workgroups to a CU.
+template <int V, bool PIXELS, bool MASKED>
 __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __restrict__ x,
                                                            uint16_t* __restrict__ cols, int64_t ld,
-                                                           ConvGeom g, const int32_t* row_ptr,
-                                                           const int32_t* col_idx, int bs, int wp, int padl,
-                                                           int vec, int tpg, int gpw) {
+                                                           ConvGeom g, Wanted want, int wp, int padl, int tpg,
+                                                           int gpw) {
+  const int32_t* row_ptr = want.row_ptr;
+  const int32_t* col_idx = want.col_idx;
+  const int bs = want.bs;
+  if (MASKED) want.src.resolve();
   extern __shared__ __attribute__((aligned(16))) char patch_mem[];
   int* col_off = reinterpret_cast<int*>(patch_mem);                     // [tpg * 64]: offset of a column in the copy
   uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp], pixel 0 of a row at column padl
@@ -205,11 +235,11 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
 
   const int sub_per_block = bs / TILE;
   const int ntiles = (ncols + TILE - 1) / TILE;
-  const int per_ch = hp * wp, ch_unit = g.xs_c == 1 && g.xs_w != 1 ? vec : 1;
+  const int per_ch = hp * wp, ch_unit = PIXELS ? V : 1;
   // column tiles [t_lo, t_hi) are this workgroup's
   const int t_lo = (int)blockIdx.y * gpw * tpg, t_hi = t_lo + gpw * tpg < ntiles ? t_lo + gpw * tpg : ntiles;
   int32_t pos = 0, end = 0;
-  if (row_ptr) {
+  if (!MASKED && row_ptr) {
     const int64_t rb = r0 / bs;
     pos = row_ptr[rb];
     end = row_ptr[rb + 1];
@@ -225,8 +255,9 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
   }
   int sub = 0, ct = t_lo - 1, group = -1;
   int32_t entry = pos < end ? col_idx[pos] : 0;
+  uint64_t kept = 0;  // of 64 tiles from t_lo, t_lo + 64, ... on
   for (;;) {
-    if (row_ptr) {
+    if (!MASKED && row_ptr) {
       if (pos >= end) break;
       ct = entry * sub_per_block + sub;
       if (++sub == sub_per_block) {
@@ -238,6 +269,10 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
       if (ct >= t_hi) break;
     } else {
       if (++ct >= t_hi) break;
+      if (MASKED) {
+        if ((ct - t_lo) % 64 == 0) kept = kept_tiles(want.src, (int)blockIdx.x, ct, ntiles);
+        if (!((kept >> ((ct - t_lo) % 64)) & 1u)) continue;
+      }
     }
     if (ct / tpg != group) {  // the same for every thread
       group = ct / tpg;
@@ -249,37 +284,33 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
       // or 1), V pixels of a row of any other (8, 4, 2 or 1, whatever row length and alignment allow), four rows' loads
       // ahead of their stores, no division anywhere.  199 x 32 x 48 x 48 channels last, 3 x 3 by two, p = 0.25: 91 us with
       // 2 bytes and a division each, 52 so; 16 x 96 x 48 x 48 channels last, pointwise by two, p = 0.6: 36 and 10.
-      if (g.xs_c == 1 && g.xs_w != 1) {
-        auto along_channels = [&](auto width) {
-          constexpr int V = decltype(width)::value, LC = V == 8 ? 4 : 32;  // lanes along the channels
-          for (int ci = t % LC * V; ci < nch; ci += LC * V)
-            for (int w0 = t / LC % (64 / LC); w0 < wp; w0 += 64 / LC) {
-              const int ww = w0 - padl;
-              const bool w_ok = ww >= 0 && ww < g.w;
-              const uint16_t* xc = x + (int64_t)ww * g.xs_w + ch_lo + ci;
-              uint16_t* to = patch + ci * per_ch + w0;
-              for (int h0 = t / 64; h0 < hp; h0 += 16) {
-                Piece<V> v[4];
+      if constexpr (PIXELS) {
+        constexpr int LC = V == 8 ? 4 : 32;  // lanes along the channels
+        for (int ci = t % LC * V; ci < nch; ci += LC * V)
+          for (int w0 = t / LC % (64 / LC); w0 < wp; w0 += 64 / LC) {
+            const int ww = w0 - padl;
+            const bool w_ok = ww >= 0 && ww < g.w;
+            const uint16_t* xc = x + (int64_t)ww * g.xs_w + ch_lo + ci;
+            uint16_t* to = patch + ci * per_ch + w0;
+            for (int h0 = t / 64; h0 < hp; h0 += 16) {
+              Piece<V> v[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                  v[k] = Piece<V>();
-                  const int64_t so = w_ok && h0 + 4 * k < hp ? src_row[h0 + 4 * k] : -1;
-                  if (so >= 0) v[k].load(xc + so);
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                  if (h0 + 4 * k < hp) {
-#pragma unroll
-                    for (int j = 0; j < V; ++j) to[j * per_ch + (h0 + 4 * k) * wp] = v[k].at(j);
-                  }
+              for (int k = 0; k < 4; ++k) {
+                v[k] = Piece<V>();
+                const int64_t so = w_ok && h0 + 4 * k < hp ? src_row[h0 + 4 * k] : -1;
+                if (so >= 0) v[k].load(xc + so);
               }
+#pragma unroll
+              for (int k = 0; k < 4; ++k)
+                if (h0 + 4 * k < hp) {
+#pragma unroll
+                  for (int j = 0; j < V; ++j) to[j * per_ch + (h0 + 4 * k) * wp] = v[k].at(j);
+                }
             }
-        };
-        if (vec == 8) along_channels(std::integral_constant<int, 8>{});
-        else along_channels(std::integral_constant<int, 1>{});
+          }
       } else {
-        auto along_rows = [&](auto width, auto lanes) {
-          constexpr int V = decltype(width)::value, LW = decltype(lanes)::value;
+        auto along_rows = [&](auto lanes) {
+          constexpr int LW = decltype(lanes)::value;
           for (int w0 = t % LW * V; w0 < wp; w0 += LW * V) {
             const int ww = w0 - padl;
             const bool w_ok = ww >= 0 && ww < g.w;
@@ -301,17 +332,10 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
             }
           }
         };
-        auto lanes_for = [&](auto width) {
-          constexpr int V = decltype(width)::value;
-          if (wp <= 4 * V) along_rows(width, std::integral_constant<int, 4>{});
-          else if (wp <= 8 * V) along_rows(width, std::integral_constant<int, 8>{});
-          else if (wp <= 16 * V) along_rows(width, std::integral_constant<int, 16>{});
-          else along_rows(width, std::integral_constant<int, 32>{});
-        };
-        if (vec == 8) lanes_for(std::integral_constant<int, 8>{});
-        else if (vec == 4) lanes_for(std::integral_constant<int, 4>{});
-        else if (vec == 2) lanes_for(std::integral_constant<int, 2>{});
-        else lanes_for(std::integral_constant<int, 1>{});
+        if (wp <= 4 * V) along_rows(std::integral_constant<int, 4>{});
+        else if (wp <= 8 * V) along_rows(std::integral_constant<int, 8>{});
+        else if (wp <= 16 * V) along_rows(std::integral_constant<int, 16>{});
+        else along_rows(std::integral_constant<int, 32>{});
       }
       for (int i = t; i < tpg * TILE; i += 256) {
         const int col = g0 + i;
@@ -650,18 +674,17 @@ static int make_geom(ConvGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, in
   return SD_OK;
 }
 
-int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
-           int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
-           int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
-           const int32_t* row_ptr, const int32_t* col_idx, int64_t bs, hipStream_t stream) {
+static int gather(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld, int64_t n, int64_t c,
+                  int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
+                  int64_t dil_h, int64_t dil_w, const Wanted& want, hipStream_t stream) {
   ConvGeom g;
   if (int rc = make_geom(g, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, sn, sc,
                          sh, sw))
     return rc;
   SD_REQUIRE(x && cols, "im2col: null pointer");
   SD_REQUIRE(ld >= c * r * s, "im2col: cols_ld %lld < C*R*S %lld", (long long)ld, (long long)(c * r * s));
-  SD_REQUIRE((row_ptr == nullptr) == (col_idx == nullptr), "im2col: pass both list arrays or neither");
-  if (row_ptr) SD_REQUIRE(bs > 0 && bs % TILE == 0, "im2col: block_size must be a multiple of 64");
+  SD_REQUIRE((want.row_ptr == nullptr) == (want.col_idx == nullptr), "im2col: pass both list arrays or neither");
+  if (want.row_ptr) SD_REQUIRE(want.bs > 0 && want.bs % TILE == 0, "im2col: block_size must be a multiple of 64");
   const int64_t rows = n * g.p * g.q;
   const int64_t blocks = ceil_div(rows, TILE);
   SD_REQUIRE(blocks <= 0x7fffffffLL, "im2col: too many rows");
@@ -704,15 +727,47 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
     int64_t tpg = 1;
     while (tpg < most && group_bytes(tpg + 1) <= PATCH_MAX_BYTES / 2) ++tpg;
     const int64_t groups = ceil_div(ntiles, tpg), gpw = ceil_div(groups, split);
-    hipLaunchKernelGGL(im2col_patch_kernel, dim3((unsigned)blocks, (unsigned)ceil_div(groups, gpw)), dim3(256),
-                       (size_t)group_bytes(tpg), stream, (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
-                       row_ptr ? (int)bs : TILE, (int)wp, (int)padl, (int)vec, (int)tpg, (int)gpw);
+    auto launch = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (unsigned)ceil_div(groups, gpw)), dim3(256), (size_t)group_bytes(tpg), stream,
+                         (const uint16_t*)x, (uint16_t*)cols, ld, g, want, (int)wp, (int)padl, (int)tpg, (int)gpw);
+    };
+    auto pick = [&](auto masked) {
+      constexpr bool M = decltype(masked)::value;
+      if (pixelwise) vec == 8 ? launch(&im2col_patch_kernel<8, true, M>) : launch(&im2col_patch_kernel<1, true, M>);
+      else vec == 8 ? launch(&im2col_patch_kernel<8, false, M>) : vec == 4 ? launch(&im2col_patch_kernel<4, false, M>)
+           : vec == 2 ? launch(&im2col_patch_kernel<2, false, M>) : launch(&im2col_patch_kernel<1, false, M>);
+    };
+    if (want.masked) pick(std::true_type{});
+    else pick(std::false_type{});
     return check_launch("im2col_patch");
   }
   hipLaunchKernelGGL(im2col_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
-                     (const uint16_t*)x, (uint16_t*)cols, ld, g, row_ptr, col_idx,
-                     row_ptr ? (int)bs : TILE);
+                     (const uint16_t*)x, (uint16_t*)cols, ld, g, want);
   return check_launch("im2col");
+}
+
+int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
+           int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
+           int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
+           const int32_t* row_ptr, const int32_t* col_idx, int64_t bs, hipStream_t stream) {
+  Wanted want{};
+  want.row_ptr = row_ptr;
+  want.col_idx = col_idx;
+  want.bs = row_ptr ? (int)bs : TILE;
+  return gather(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, want, stream);
+}
+
+int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
+                  int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
+                  int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
+                  int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t mb,
+                  int64_t kb, int64_t bs, hipStream_t stream) {
+  Wanted want{};
+  want.bs = TILE;
+  want.masked = true;
+  want.src = MaskSrc{mask, msr, msc, (int32_t)(bs / TILE), 1, (int32_t)mb, (int32_t)kb, (uint32_t)seed, (uint32_t)(seed >> 32),
+                     (uint32_t)offset, (uint32_t)(offset >> 32), p, state};
+  return gather(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, want, stream);
 }
 
 int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,

@@ -333,8 +333,9 @@ Tensor layer_forward(Tensor x, Tensor w, int64_t bs, double p, const Draw& draw,
 }
 
 // dX and / or dW of one layer in one library call; act_at: what dX's fused activation derivative is evaluated at.
+// kept_only (without an activation): dropped blocks of dX are left as they are.
 std::pair<Tensor, Tensor> layer_products(const Tensor& dy, const Tensor& w, const Tensor& x, const Lists& lists, double p,
-                                         bool need_dx, bool need_dw, int act, const Tensor& act_at) {
+                                         bool need_dx, bool need_dw, int act, const Tensor& act_at, bool kept_only = false) {
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   Tensor dx = need_dx ? new_matrix(x, M, K) : Tensor(), dw = need_dw ? new_matrix(x, N, K) : Tensor();
   if (!(need_dx || need_dw) || M == 0 || K == 0) return {dx, dw};
@@ -348,6 +349,13 @@ std::pair<Tensor, Tensor> layer_products(const Tensor& dy, const Tensor& w, cons
   if (need_dw) dwm = Mat(dw);
   const Mat gm(dy), wm(w), xm(x);
   c10::DeviceGuard guard(x.device());
+  if (kept_only) {
+    check(sd_dropout_matmul_backward_kept(MAT(gm), MAT(wm), MAT(xm), MAT(dxm), MAT(dwm), lists.row_ptr(), lists.col_idx(),
+                                          lists.col_ptr(), lists.row_idx(), M, N, K, lists.kernel_bs, p, dtype_of(x), ws.ptr,
+                                          ws.bytes, stream_of(x)),
+          "sd_dropout_matmul_backward_kept");
+    return {dx, dw};
+  }
   check(sd_dropout_matmul_backward_act(MAT(gm), MAT(wm), MAT(xm), MAT(dxm), MAT(dwm), lists.row_ptr(), lists.col_idx(),
                                        lists.col_ptr(), lists.row_idx(), M, N, K, lists.kernel_bs, p, dtype_of(x), act,
                                        MAT(am), ws.ptr, ws.bytes, stream_of(x)),
@@ -628,13 +636,16 @@ struct ConvGeom {
 #define GEOM_W(g) (g).pad[0], (g).pad[1], (g).stride[0], (g).stride[1], (g).dil[0], (g).dil[1]
 #define STRIDES4(t) (t).stride(0), (t).stride(1), (t).stride(2), (t).stride(3)
 
-void conv_mask(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
+void check_conv_mask(const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
   check_p(p);
   l.shape(g.rows(), g.cols(), bs);
   if (draw.mask)
     TORCH_CHECK_VALUE(draw.mask->dim() == 2 && draw.mask->size(0) == l.mb && draw.mask->size(1) == l.kb, "mask shape ",
                       draw.mask->sizes(), " != [", l.mb, ", ", l.kb, "] for a [", g.rows(), ", ", g.cols(),
                       "] matrix in blocks of ", bs);
+}
+void conv_mask(const Tensor& x, const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
+  check_conv_mask(g, bs, p, draw, l);
   l.allocate(x, draw.mask);
 }
 
@@ -679,13 +690,16 @@ Tensor pixel_rows(const Tensor& x) {
 //    by two 102 -> 85 us a pass); 1.03 to 1.09 where the matrix is one block wide.  Past 256 MB it stays out of memory.
 bool forward_by_patches(const ConvGeom& g) { return g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64; }
 bool dw_by_patches(const ConvGeom& g) { return g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
+bool dx_may_fuse(const ConvGeom& g) { return g.k % 64 == 0 && g.k <= 256 && g.qo <= 64 && 64 % g.qo == 0 && g.po * g.qo % 64 == 0; }
 bool dx_by_patches(const ConvGeom& g) { return g.cols() > 64 && g.rows() * g.cols() * 2 <= 256LL << 20; }
 
+// The image itself where it is its own patch matrix, else undefined
+Tensor own_patches(const Tensor& x, const ConvGeom& g) {
+  return pointwise(g) && g.c % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 ? pixel_rows(x) : Tensor();
+}
 Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
-  if (pointwise(g) && g.c % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0) {
-    const Tensor rows = pixel_rows(x);
-    if (rows.defined()) return rows;
-  }
+  const Tensor rows = own_patches(x, g);
+  if (rows.defined()) return rows;
   Tensor cols = new_matrix(x, g.rows(), g.cols());
   c10::DeviceGuard guard(x.device());
   check(sd_im2col(x.data_ptr(), STRIDES4(x), cols.data_ptr(), cols.stride(0), GEOM_X(g), g.r, g.s, GEOM_W(g),
@@ -694,6 +708,25 @@ Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
         "sd_im2col");
   return cols;
 }
+
+// Forward of a masked convolution through its patch matrix in two launches where there were three: the gather asks the mask's source,
+// the product makes the lists.  cols: the patch matrix.
+Tensor patches_forward(const Tensor& x, const Tensor& w2, const ConvGeom& g, int64_t bs, double p, Draw draw, Lists& l, Tensor* cols) {
+  check_conv_mask(g, bs, p, draw, l);
+  if (draw.mask) draw.mask = check_mask(*draw.mask, l.mb, l.kb, x);
+  *cols = own_patches(x, g);
+  if (!cols->defined()) {
+    *cols = new_matrix(x, g.rows(), g.cols());
+    const MaskArg m = draw.mask ? MaskArg(*draw.mask) : MaskArg();
+    c10::DeviceGuard guard(x.device());
+    check(sd_im2col_masked(x.data_ptr(), STRIDES4(x), cols->data_ptr(), cols->stride(0), GEOM_X(g), g.r, g.s, GEOM_W(g), m.ptr, m.sr,
+                           m.sc, draw.state_ptr(), draw.seed.value_or(0), 0, (float)p, bs, dtype_of(x), stream_of(x)),
+          "sd_im2col_masked");
+  }
+  return layer_forward(*cols, w2, bs, p, draw, SD_ACT_NONE, false, l, nullptr);
+}
+// Whether a layer's products take its operands as they are (else the calls one by one, which take any)
+bool layer_takes(const ConvGeom& g, const Tensor& w2) { return g.cols() % 8 == 0 && g.k % 8 == 0 && rows_on_16_bytes(w2); }
 
 Tensor conv_dw(const Tensor& x, const Tensor& dy2, const ConvGeom& g, const Lists* l, float scale) {
   Tensor dw = new_matrix(x, g.k, g.cols());
@@ -867,6 +900,30 @@ struct ConvBackward : Node {
     const Tensor dy2 = grads[0].defined() ? rows_gradient(grads[0], g, w) : at::zeros({g.rows(), g.k}, w.options());
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
+    // both gradients through the patch matrix: one launch where the pair qualifies, and the fold
+    const bool dw_through = pixels || patches.defined() || dw_by_patches(g), dx_through = !fused_dx || dx_by_patches(g) || !dx_may_fuse(g);
+    if (l && task_should_compute_output(0) && task_should_compute_output(1) && dw_through && dx_through && layer_takes(g, w) && rows_on_16_bytes(dy2)) {
+      if (!patches.defined()) patches = im2col(image, g, l);
+      if (rows_on_16_bytes(patches)) {
+        // a pointwise kernel's patch gradient is that of a channels-last image: the product writes it in place, zeros included
+        const bool in_place = pointwise(g) && channels_last;
+        auto [dcols, dk] = layer_products(dy2, w, patches, *l, p, true, true, SD_ACT_NONE, Tensor(), !in_place);
+        last_routes[1] = last_routes[2] = kExplicit;
+        if (in_place) {
+          out[0] = dcols.view({g.n, g.h, g.w, g.c}).permute({0, 3, 1, 2});
+        } else {
+          Tensor dx = new_image(dy2, g, channels_last);
+          const MaskArg m = l->mask();
+          c10::DeviceGuard guard(dy2.device());
+          check(sd_col2im(dcols.data_ptr(), dcols.stride(0), dx.data_ptr(), STRIDES4(dx), GEOM_X(g), g.r, g.s, GEOM_W(g), m.ptr,
+                          m.sr, m.sc, l->bs, dtype_of(dy2), stream_of(dy2)),
+                "sd_col2im");
+          out[0] = dx;
+        }
+        out[1] = dk.view({g.k, g.c, g.r, g.s});
+        return out;
+      }
+    }
     if (task_should_compute_output(0)) {
       Tensor dx;
       if (fused_dx && !(l && dx_by_patches(g))) dx = conv_dx(dy2, w, g, l, scale, channels_last);
@@ -994,14 +1051,18 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     y = y2.view({g.n, g.po, g.qo, g.k}).permute({0, 3, 1, 2});
   } else {
     NoRecord guard;
-    if (bs) conv_lists(x, g, bs, p, Draw{mask, seed, state}, lists);
     const Lists* l = bs ? &lists : nullptr;
-    y2 = new_matrix(x, g.rows(), g.k);
     bool done = false;
     c10::DeviceGuard device(x.device());
+    const Tensor w2 = kernel.detach().view({g.k, g.cols()});
     const bool takes_implicit = implicit_forward && sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(),
                                                                               GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
-    if (takes_implicit && !(bs && forward_by_patches(g))) {  // no patch matrix in memory
+    const bool implicit = takes_implicit && !(bs && forward_by_patches(g)), layer = bs && layer_takes(g, w2);
+    if (implicit || !layer) {
+      if (bs) conv_lists(x, g, bs, p, Draw{mask, seed, state}, lists);
+      y2 = new_matrix(x, g.rows(), g.k);
+    }
+    if (implicit) {  // no patch matrix in memory
       const int rc = sd_conv2d_dsd_lists(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(), y2.data_ptr(),
                                          y2.stride(0), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), l ? l->row_ptr() : nullptr,
                                          l ? l->col_idx() : nullptr, l ? l->kernel_bs : 0, scale, dtype_of(x),
@@ -1011,7 +1072,9 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     }
     last_routes[0] = done ? kImplicit : kExplicit;
     last_routes[1] = last_routes[2] = kNone;
-    if (!done) {
+    if (!done && layer && !implicit) {
+      y2 = patches_forward(x, w2, g, bs, p, Draw{mask, seed, state}, lists, &cols);
+    } else if (!done) {
       cols = im2col(x, g, l);
       Mat am(cols), bm, cm(y2);
       bm.ptr = kernel.data_ptr();

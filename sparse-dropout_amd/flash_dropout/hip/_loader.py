@@ -72,6 +72,9 @@ SIGNATURES = {
     "sd_dropout_matmul_backward": (c_int, [*_mat, *_mat, *_mat, *_mat, *_mat, c_void_p, c_void_p, c_void_p, c_void_p,
                                            c_int64, c_int64, c_int64, c_int64, c_double, c_int, c_void_p, c_int64,
                                            c_void_p]),
+    "sd_dropout_matmul_backward_kept": (c_int, [*_mat, *_mat, *_mat, *_mat, *_mat, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                c_int64, c_int64, c_int64, c_int64, c_double, c_int, c_void_p, c_int64,
+                                                c_void_p]),
     "sd_dropout_matmul_backward_act": (c_int, [*_mat, *_mat, *_mat, *_mat, *_mat, c_void_p, c_void_p, c_void_p,
                                                c_void_p, c_int64, c_int64, c_int64, c_int64, c_double, c_int,
                                                c_int, *_mat, c_void_p, c_int64, c_void_p]),
@@ -111,6 +114,8 @@ SIGNATURES = {
                                   *([c_int64] * 13), c_float, c_int, c_void_p, c_int64, c_void_p]),
     "sd_im2col": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64,
                           *([c_int64] * 12), c_void_p, c_void_p, c_int64, c_int, c_void_p]),
+    "sd_im2col_masked": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, *([c_int64] * 12),
+                                 c_void_p, c_int64, c_int64, c_void_p, c_uint64, c_uint64, c_float, c_int64, c_int, c_void_p]),
     "sd_col2im": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                           *([c_int64] * 12), c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
 }

@@ -621,3 +621,68 @@ def test_masked_convolutions_go_through_a_patch_matrix_where_that_is_faster(cfg,
         y = call()
     assert tuple(x.shape) in kept and (rows, fan_in) not in kept
     y.backward(dy.cuda())
+
+
+@pytest.mark.parametrize("cfg", [
+    dict(n=3, c=208, h=8, w=8, r=5, s=5, padding=(2, 2), stride=(2, 2), dilation=(1, 1)),    # 82 tiles over workgroups, the last ragged
+    dict(n=20, c=24, h=14, w=14, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),  # ragged rows
+    dict(n=1, c=5, h=9, w=260, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),    # rows off 16-byte boundaries: the turning kernel
+])
+@pytest.mark.parametrize("bs", [64, 128, 192])
+@pytest.mark.parametrize("source", ["given", "given by columns", "seed", "state"])
+def test_im2col_of_a_mask_source_writes_the_blocks_of_its_lists(cfg, bs, source):
+    """The gather that asks the mask itself against the bytes that the list builder stores of the same draw; it does not move
+    the generator on."""
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(bs)
+    x = torch.randn(cfg["n"], cfg["c"], cfg["h"], cfg["w"], generator=gen).half().cuda()
+    ks = (cfg["r"], cfg["s"])
+    ref = torch.from_numpy(O.im2col(x.float().cpu().numpy(), *ks, **_geo(cfg))).half()
+    shape = O.mask_shape(*ref.shape, bs)
+    mask, state, seed = None, None, 0
+    if source.startswith("given"):
+        mask = cpu_mask(shape, 0.4, gen).cuda()
+        if "columns" in source:
+            mask = mask.t().contiguous().t()
+    elif source == "state":
+        state = ext.rng_state(x.device)
+    else:
+        seed = 91
+    part = torch.full(ref.shape, 7.0, dtype=torch.float16, device="cuda")
+    before = None if state is None else state.clone()
+    rc = ext.lib.sd_im2col_masked(x.data_ptr(), *x.stride(), part.data_ptr(), part.stride(0), *x.shape, *ks, *cfg["padding"],
+                                  *cfg["stride"], *cfg["dilation"], None if mask is None else mask.data_ptr(),
+                                  *((0, 0) if mask is None else mask.stride()), None if state is None else state.data_ptr(), seed, 0,
+                                  0.4, bs, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    if state is not None:
+        assert torch.equal(before, state)
+    if mask is None:
+        mask = ext.random_lists(shape, 0.4, seed=None if state is not None else seed, device=x.device)[0]
+    keep = torch.from_numpy(O.expand_keep(mask.cpu().numpy(), bs, *ref.shape))
+    assert torch.equal(part.cpu(), torch.where(keep, ref, torch.tensor(7.0, dtype=torch.float16)))
+
+
+@pytest.mark.parametrize("bs", [64, 128])
+@pytest.mark.parametrize("c,k,r,stride", [(16, 40, 3, 1), (24, 72, 5, 2), (72, 64, 1, 2)])
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_both_gradients_through_the_patch_matrix_match_one_at_a_time(bs, c, k, r, stride, channels_last):
+    """One launch for both products, dropped blocks of the patch gradient left as they are, against one product at a time."""
+    import flash_dropout.functional as F
+
+    gen = torch.Generator().manual_seed(c)
+    x = torch.randn(7, c, 14, 14, generator=gen).half().cuda()
+    if channels_last:
+        x = x.contiguous(memory_format=torch.channels_last)
+    w = (torch.randn(k, c, r, r, generator=gen) * (c * r * r) ** -0.5).half().cuda().requires_grad_()
+    x.requires_grad_()
+    y = F.blockwise_dropout_conv2d(x, w, bs, 0.4, r // 2, stride, seed=3)
+    dy = torch.randn(y.shape, generator=gen).half().cuda()
+    both = torch.autograd.grad(y, (x, w), dy, retain_graph=True)
+    assert F.conv_last_routes()["dx"] == "explicit" and both[0].stride() == x.stride()
+    for one, wrt in zip(both, (x, w)):
+        alone, = torch.autograd.grad(y, wrt, dy, retain_graph=True)
+        # sums in fp32 in another order, one rounding to fp16 of a product and, for dx, one of the fold
+        assert rel_fro(one, to_np(alone)) <= 1e-3
