@@ -448,16 +448,14 @@ int sd_im2col(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_s
               int dtype, void* stream);
 
 /* The same for the blocks that a mask keeps, before there are lists of it: a stored mask (one byte per block, strides in
- * bytes), or with mask NULL the draw that sd_random_lists (seed, offset) or sd_random_lists_state (state, which is read
- * and not moved on) makes.  block_size: a multiple of 64. */
+ * bytes), or with mask NULL the draw that sd_random_lists makes of (seed, offset).  block_size: a multiple of 64. */
 int sd_im2col_masked(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_stride_h,
                      int64_t x_stride_w, void* cols, int64_t cols_ld,
                      int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
                      int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
                      int64_t dil_h, int64_t dil_w,
                      const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c,
-                     const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t block_size,
-                     int dtype, void* stream);
+                     uint64_t seed, uint64_t offset, float p, int64_t block_size, int dtype, void* stream);
 
 int sd_col2im(const void* cols, int64_t cols_ld, void* dx, int64_t dx_stride_n,
               int64_t dx_stride_c, int64_t dx_stride_h, int64_t dx_stride_w,

@@ -32,7 +32,7 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
 int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
                   int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
                   int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
-                  int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t mb,
+                  int64_t msr, int64_t msc, uint64_t seed, uint64_t offset, float p, int64_t mb,
                   int64_t kb, int64_t bs, hipStream_t stream);
 int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
            int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
@@ -696,19 +696,18 @@ int sd_im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, voi
 int sd_im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
                      int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
                      int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
-                     int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t bs,
+                     int64_t msr, int64_t msc, uint64_t seed, uint64_t offset, float p, int64_t bs,
                      int dtype, void* stream) {
   SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "dtype must be SD_F16 or SD_BF16 (got %d)", dtype);
   SD_REQUIRE(bs > 0 && bs % 64 == 0 && bs < kMaxDim, "im2col_masked: block_size must be a multiple of 64");
   SD_REQUIRE(mask == nullptr || (msr >= 1 && msc >= 1), "im2col_masked: mask strides");
   SD_REQUIRE(mask != nullptr || (p >= 0.f && p < 1.f), "im2col_masked: p must be in [0, 1) (got %g)", (double)p);
-  SD_REQUIRE(state == nullptr || reinterpret_cast<uintptr_t>(state) % 8 == 0, "im2col_masked: state must be an aligned device pointer");
   SD_REQUIRE(n > 0 && c > 0 && r > 0 && s > 0 && stride_h > 0 && stride_w > 0, "im2col_masked: sizes and strides must be positive");
   const int64_t p_out = (h + 2 * pad_h - dil_h * (r - 1) - 1) / stride_h + 1, q_out = (w + 2 * pad_w - dil_w * (s - 1) - 1) / stride_w + 1;
   const int64_t mb = ceil_div(n * p_out * q_out, bs), kb = ceil_div(c * r * s, bs);
   SD_REQUIRE(mb < kMaxDim && kb < kMaxDim, "im2col_masked: mask too large");
   return im2col_masked(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, mask, msr, msc,
-                       state, seed, offset, p, mb, kb, bs, (hipStream_t)stream);
+                       seed, offset, p, mb, kb, bs, (hipStream_t)stream);
 }
 
 int sd_col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,

@@ -23,8 +23,9 @@ struct ConvGeom {
   int64_t xs_n, xs_c, xs_h, xs_w;  // element strides of the image tensor
 };
 
-// Which blocks of the patch matrix are wanted: those of a list by rows, those that a mask source keeps, or all of them.  A mask
-// source is what there is before any list: the gather needs no launch in front of it, and the product behind it makes the lists.
+// Which blocks of the patch matrix are wanted: those of a list by rows, those that a mask source (a stored mask or a seed's draw)
+// keeps, or all of them.  A mask source is what there is before any list: the gather needs no launch in front of it, and the product
+// behind it makes the lists.
 struct Wanted {
   const int32_t* row_ptr;
   const int32_t* col_idx;
@@ -47,7 +48,6 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* __restrict_
   const int32_t* row_ptr = want.row_ptr;
   const int32_t* col_idx = want.col_idx;
   const int bs = want.bs;
-  if (want.masked) want.src.resolve();
   __shared__ __attribute__((aligned(4))) uint16_t tile[TILE * TLD];  // [row][col]
   const int t = threadIdx.x;
   const int lane = t % 64;
@@ -188,7 +188,6 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
   const int32_t* row_ptr = want.row_ptr;
   const int32_t* col_idx = want.col_idx;
   const int bs = want.bs;
-  if (MASKED) want.src.resolve();
   extern __shared__ __attribute__((aligned(16))) char patch_mem[];
   int* col_off = reinterpret_cast<int*>(patch_mem);                     // [tpg * 64]: offset of a column in the copy
   uint16_t* patch = reinterpret_cast<uint16_t*>(col_off + tpg * TILE);  // [channels][hp][wp], pixel 0 of a row at column padl
@@ -760,13 +759,13 @@ int im2col(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* 
 int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw, void* cols, int64_t ld,
                   int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
                   int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
-                  int64_t msr, int64_t msc, const uint64_t* state, uint64_t seed, uint64_t offset, float p, int64_t mb,
+                  int64_t msr, int64_t msc, uint64_t seed, uint64_t offset, float p, int64_t mb,
                   int64_t kb, int64_t bs, hipStream_t stream) {
   Wanted want{};
   want.bs = TILE;
   want.masked = true;
   want.src = MaskSrc{mask, msr, msc, (int32_t)(bs / TILE), 1, (int32_t)mb, (int32_t)kb, (uint32_t)seed, (uint32_t)(seed >> 32),
-                     (uint32_t)offset, (uint32_t)(offset >> 32), p, state};
+                     (uint32_t)offset, (uint32_t)(offset >> 32), p, nullptr};
   return gather(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, want, stream);
 }
 

@@ -709,8 +709,8 @@ Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
   return cols;
 }
 
-// Forward of a masked convolution through its patch matrix in two launches where there were three: the gather asks the mask's source,
-// the product makes the lists.  cols: the patch matrix.
+// Forward of a masked convolution through its patch matrix in two launches where there were three: the gather asks the mask's source
+// (a stored mask or a seed), the product makes the lists.  cols: the patch matrix.
 Tensor patches_forward(const Tensor& x, const Tensor& w2, const ConvGeom& g, int64_t bs, double p, Draw draw, Lists& l, Tensor* cols) {
   check_conv_mask(g, bs, p, draw, l);
   if (draw.mask) draw.mask = check_mask(*draw.mask, l.mb, l.kb, x);
@@ -720,7 +720,7 @@ Tensor patches_forward(const Tensor& x, const Tensor& w2, const ConvGeom& g, int
     const MaskArg m = draw.mask ? MaskArg(*draw.mask) : MaskArg();
     c10::DeviceGuard guard(x.device());
     check(sd_im2col_masked(x.data_ptr(), STRIDES4(x), cols->data_ptr(), cols->stride(0), GEOM_X(g), g.r, g.s, GEOM_W(g), m.ptr, m.sr,
-                           m.sc, draw.state_ptr(), draw.seed.value_or(0), 0, (float)p, bs, dtype_of(x), stream_of(x)),
+                           m.sc, draw.seed.value_or(0), 0, (float)p, bs, dtype_of(x), stream_of(x)),
           "sd_im2col_masked");
   }
   return layer_forward(*cols, w2, bs, p, draw, SD_ACT_NONE, false, l, nullptr);
@@ -1057,9 +1057,12 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     const Tensor w2 = kernel.detach().view({g.k, g.cols()});
     const bool takes_implicit = implicit_forward && sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(),
                                                                               GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
-    const bool implicit = takes_implicit && !(bs && forward_by_patches(g)), layer = bs && layer_takes(g, w2);
+    const Draw draw{mask, seed, state};
+    // A draw from the generator's state is made by one launch and read from what that stored: between two launches that each
+    // make it another stream may move the state on, and the product would read blocks that were not gathered.
+    const bool implicit = takes_implicit && !(bs && forward_by_patches(g)), layer = bs && layer_takes(g, w2) && !draw.state_ptr();
     if (implicit || !layer) {
-      if (bs) conv_lists(x, g, bs, p, Draw{mask, seed, state}, lists);
+      if (bs) conv_lists(x, g, bs, p, draw, lists);
       y2 = new_matrix(x, g.rows(), g.k);
     }
     if (implicit) {  // no patch matrix in memory
@@ -1073,7 +1076,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     last_routes[0] = done ? kImplicit : kExplicit;
     last_routes[1] = last_routes[2] = kNone;
     if (!done && layer && !implicit) {
-      y2 = patches_forward(x, w2, g, bs, p, Draw{mask, seed, state}, lists, &cols);
+      y2 = patches_forward(x, w2, g, bs, p, draw, lists, &cols);
     } else if (!done) {
       cols = im2col(x, g, l);
       Mat am(cols), bm, cm(y2);

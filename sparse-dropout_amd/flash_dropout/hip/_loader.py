@@ -115,7 +115,7 @@ SIGNATURES = {
     "sd_im2col": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64,
                           *([c_int64] * 12), c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "sd_im2col_masked": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, *([c_int64] * 12),
-                                 c_void_p, c_int64, c_int64, c_void_p, c_uint64, c_uint64, c_float, c_int64, c_int, c_void_p]),
+                                 c_void_p, c_int64, c_int64, c_uint64, c_uint64, c_float, c_int64, c_int, c_void_p]),
     "sd_col2im": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                           *([c_int64] * 12), c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
 }

@@ -629,10 +629,9 @@ def test_masked_convolutions_go_through_a_patch_matrix_where_that_is_faster(cfg,
     dict(n=1, c=5, h=9, w=260, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),    # rows off 16-byte boundaries: the turning kernel
 ])
 @pytest.mark.parametrize("bs", [64, 128, 192])
-@pytest.mark.parametrize("source", ["given", "given by columns", "seed", "state"])
+@pytest.mark.parametrize("source", ["given", "given by columns", "seed"])
 def test_im2col_of_a_mask_source_writes_the_blocks_of_its_lists(cfg, bs, source):
-    """The gather that asks the mask itself against the bytes that the list builder stores of the same draw; it does not move
-    the generator on."""
+    """The gather that asks the mask itself against the bytes that the list builder stores of the same draw."""
     from flash_dropout.hip import GEMM
 
     ext = GEMM()
@@ -641,26 +640,20 @@ def test_im2col_of_a_mask_source_writes_the_blocks_of_its_lists(cfg, bs, source)
     ks = (cfg["r"], cfg["s"])
     ref = torch.from_numpy(O.im2col(x.float().cpu().numpy(), *ks, **_geo(cfg))).half()
     shape = O.mask_shape(*ref.shape, bs)
-    mask, state, seed = None, None, 0
+    mask, seed = None, 0
     if source.startswith("given"):
         mask = cpu_mask(shape, 0.4, gen).cuda()
         if "columns" in source:
             mask = mask.t().contiguous().t()
-    elif source == "state":
-        state = ext.rng_state(x.device)
     else:
         seed = 91
     part = torch.full(ref.shape, 7.0, dtype=torch.float16, device="cuda")
-    before = None if state is None else state.clone()
     rc = ext.lib.sd_im2col_masked(x.data_ptr(), *x.stride(), part.data_ptr(), part.stride(0), *x.shape, *ks, *cfg["padding"],
                                   *cfg["stride"], *cfg["dilation"], None if mask is None else mask.data_ptr(),
-                                  *((0, 0) if mask is None else mask.stride()), None if state is None else state.data_ptr(), seed, 0,
-                                  0.4, bs, 0, torch.cuda.current_stream().cuda_stream)
+                                  *((0, 0) if mask is None else mask.stride()), seed, 0, 0.4, bs, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
-    if state is not None:
-        assert torch.equal(before, state)
     if mask is None:
-        mask = ext.random_lists(shape, 0.4, seed=None if state is not None else seed, device=x.device)[0]
+        mask = ext.random_lists(shape, 0.4, seed=seed, device=x.device)[0]
     keep = torch.from_numpy(O.expand_keep(mask.cpu().numpy(), bs, *ref.shape))
     assert torch.equal(part.cpu(), torch.where(keep, ref, torch.tensor(7.0, dtype=torch.float16)))
 
@@ -686,3 +679,29 @@ def test_both_gradients_through_the_patch_matrix_match_one_at_a_time(bs, c, k, r
         alone, = torch.autograd.grad(y, wrt, dy, retain_graph=True)
         # sums in fp32 in another order, one rounding to fp16 of a product and, for dx, one of the fold
         assert rel_fro(one, to_np(alone)) <= 1e-3
+
+
+@pytest.mark.parametrize("bs", [64, 128])
+@pytest.mark.parametrize("c,k,r,stride", [(16, 40, 3, 1), (72, 64, 1, 2), (24, 64, 5, 2)])
+def test_conv_draws_of_the_generator_state_are_those_of_its_seed(bs, c, k, r, stride):
+    """A draw of the state is made by one launch and read from what it stored, one of a seed by gather and product each: the same
+    mask, results equal to rounding, and the state moves on by one draw a call."""
+    import flash_dropout.functional as F
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(c)
+    x = torch.randn(7, c, 14, 14, generator=gen).half().cuda().requires_grad_()
+    w = (torch.randn(k, c, r, r, generator=gen) * (c * r * r) ** -0.5).half().cuda().requires_grad_()
+    ext.manual_seed(77)
+    try:
+        y = F.blockwise_dropout_conv2d(x, w, bs, 0.4, r // 2, stride)
+        assert ext.rng_state(x.device).tolist() == [77, 1, 0, 0]
+        pinned = F.blockwise_dropout_conv2d(x, w, bs, 0.4, r // 2, stride, seed=77)
+        dy = torch.randn(y.shape, generator=gen).half().cuda()
+        grads, pinned_grads = (torch.autograd.grad(v, (x, w), dy) for v in (y, pinned))
+        # sums in fp32 in another order at most, one rounding to fp16 of a product and, for dx, one of the fold
+        for one, other in zip((y, *grads), (pinned, *pinned_grads)):
+            assert rel_fro(one, to_np(other)) <= 1e-3
+    finally:
+        ext.manual_seed(torch.initial_seed())
