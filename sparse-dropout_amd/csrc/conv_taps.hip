@@ -19,6 +19,7 @@
 //   256 x 32 x 28 x 28 -> 64, 3 x 3, bf16, p = 0.25: 20, 24, 26, 21 + 5; through lists: lists 13, patch matrix 45, y 30, rows of dy 13,
 //   patch gradient 40, fold 52, dw 28 + 6, 227 a pass.
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
 #include "conv_taps.h"
@@ -88,9 +89,15 @@ __device__ inline float pick(int m, float b, float a) {
 // of the steps) is kept few: a wave issues an instruction every four or five clocks at best, and the input gradient's picks alone
 // are 128 of the 250 of a step of 32 products.  One workgroup alone, 128 x 64 channels, 18 steps: 17 us (y), 22 (dx); 512 of them,
 // two to a CU: 28 and 37, where the matrix cores are busy a third of the time.
-template <typename T, bool DX, int NT, int KS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_taps_kernel(TapArgs g) {
-  constexpr bool WIDE = NT == 8;
+//
+// WIDE: the packed weights' steps are 128 outputs of one slab.  Tiles of 16 outputs that lie past the last are left out two at a time, and
+// with HALF_CHUNK (input gradient) the second slab of the last chunk, which holds nothing but zeros, so that 88 channels cost 96 and not
+// 128 on either side.  The loops of a whole and of a half chunk stand one behind the other: chosen between per chunk, the sums were
+// copied and spilled (69 registers, passes 1.2 of what they were).  A pass, every sum as before: 94 x 88 x 32 x 32 -> 88, 5 x 5, p = 0.4 310 ->
+// 286 us, 50 x 144 x 30 x 30 -> 160, 3 x 3, p = 0.1 170 -> 152, 64 x 72 x 32 x 32 -> 72, 3 x 3, p = 0.2 100 -> 94.
+template <typename T, bool DX, bool WIDE, int NT, int KS, bool HALF_CHUNK>
+__device__ __forceinline__ void conv_taps_body(const TapArgs& g) {
+  static_assert(!DX || !WIDE, "an input gradient's steps are taps");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* rows_l = smem + kStages * kWeightStage;
   char* table = rows_l + (g.span + 8) * kRowBytes;
@@ -236,30 +243,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     return ((r16 & 0x70u) | (uint32_t)(grp * 128)) | ((r16 >> 7) << 10);
   };
 
-  for (int chunk = 0; chunk < nchunk; ++chunk) {
+  auto enter_chunk = [&](int chunk) {
     if (chunk) {
       __syncthreads();  // every wave is done with the rows of the chunk before
       load_rows(chunk);
       if (!DX && g.mask) k1 = chunk_kept(chunk);
     }
     first_tap();
-    if constexpr (DX) {
-      u32x4 w[KS][NT], a0[KS], a1[KS];
+  };
+  if constexpr (DX) {
+    auto all_taps = [&](auto slabs) __attribute__((always_inline)) {
+      constexpr int KC = decltype(slabs)::value;
+      u32x4 w[KC][NT], a0[KC], a1[KC];
       uint32_t b0 = 0, b1 = 0;
       auto read_w = [&](int kk) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) w[kk][nt] = *reinterpret_cast<const u32x4*>(wst + kk * kUnit + nt * 1024);
       };
-      auto read_a = [&](int mt, u32x4 (&a)[KS], uint32_t& bits) {
+      auto read_a = [&](int mt, u32x4 (&a)[KC], uint32_t& bits) {
         const uint32_t r = row_at(mt);
 #pragma unroll
-        for (int kk = 0; kk < KS; ++kk) a[kk] = *reinterpret_cast<const u32x4*>(rows_l + r + kk * 512);
+        for (int kk = 0; kk < KC; ++kk) a[kk] = *reinterpret_cast<const u32x4*>(rows_l + r + kk * 512);
         const uint32_t b16 = if_inside(mt, (pix[mt] + shift) >> 2, (nrb - 1) * 16) & ~15u;  // 16 * the row block
         bits = *reinterpret_cast<const uint32_t*>(table + (uint32_t)(tap * nrb * 16 + grp * 4) + b16);
       };
       enter(true);
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) read_w(kk);
+      for (int kk = 0; kk < KC; ++kk) read_w(kk);
       read_a(0, a0, b0);
       for (int t = 0; t < RS; ++t) {
         const bool more = t + 1 < RS;
@@ -273,8 +283,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         };
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-          u32x4(&ac)[KS] = mt % 2 ? a1 : a0;
-          u32x4(&an)[KS] = mt % 2 ? a0 : a1;
+          u32x4(&ac)[KC] = mt % 2 ? a1 : a0;
+          u32x4(&an)[KC] = mt % 2 ? a0 : a1;
           uint32_t& bn = mt % 2 ? b0 : b1;
           bits[mt] = mt % 2 ? b1 : b0;
           if (mt < 3) {
@@ -286,7 +296,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int kk = 0; kk < KS; ++kk) {
+          for (int kk = 0; kk < KC; ++kk) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) d[mt % 2][nt] = T::mfma16(w[kk][nt], ac[kk], kk ? d[mt % 2][nt] : acc[mt][nt]);
             if (mt == 3) {  // the next tap's weights, as soon as this one's have been used for the last time
@@ -301,7 +311,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         picks(3);
         __builtin_amdgcn_sched_barrier(0);
       }
-    } else {
+    };
+    const int whole = HALF_CHUNK ? nchunk - 1 : nchunk;
+    for (int chunk = 0; chunk < whole; ++chunk) {
+      enter_chunk(chunk);
+      all_taps(std::integral_constant<int, KS>{});
+    }
+    if constexpr (HALF_CHUNK) {
+      enter_chunk(nchunk - 1);
+      all_taps(std::integral_constant<int, 1>{});
+    }
+  } else {
+    for (int chunk = 0; chunk < nchunk; ++chunk) {
+      enter_chunk(chunk);
       uint64_t kept = ~0ull;
       if (g.mask) {
         kept = __ballot(k1);
@@ -313,8 +335,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
       }
       const bool mixed = kept != ~0ull;
       const int two = chunk * 64 + 32 < g.red ? 2 : 1, npairs = RS * two;  // (tap, slab) pairs
-      constexpr int NW = NT < 4 ? NT : 4;
-      u32x4 a0[4], a1[4], w0[NW], w1[NW], c0 = {}, c1 = {};
+      constexpr int NW = NT < 4 ? NT : 4, NW1 = WIDE && NT > 4 ? NT - 4 : NW;  // tiles of a step's first and second unit
+      u32x4 a0[4], a1[4], w0[NW], w1[NW1], c0 = {}, c1 = {};
       uint32_t row[4];  // where the rows of a tap lie
       auto read_a = [&](int j, u32x4 (&a)[4], u32x4& m) {  // j = 0, 1, 2, ... one after the other
         const int slab = two == 2 ? j & 1 : 0;
@@ -327,9 +349,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         for (int mt = 0; mt < 4; ++mt) a[mt] = *reinterpret_cast<const u32x4*>(rows_l + row[mt] + slab * 512);
         m = *reinterpret_cast<const u32x4*>(pat + tap * 128 + slab * 64 + grp * 16);  // (only used when mixed)
       };
-      auto read_w = [&](u32x4 (&w)[NW], int unit) {
+      auto read_w = [&](auto& w, int unit) {
 #pragma unroll
-        for (int nt = 0; nt < NW; ++nt) w[nt] = *reinterpret_cast<const u32x4*>(wst + unit * kUnit + nt * 1024);
+        for (int nt = 0; nt < (int)(sizeof(w) / sizeof(w[0])); ++nt) w[nt] = *reinterpret_cast<const u32x4*>(wst + unit * kUnit + nt * 1024);
       };
       auto clear = [&](u32x4 (&a)[4], const u32x4& m) {
         if (mixed) {
@@ -337,20 +359,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
           for (int mt = 0; mt < 4; ++mt) a[mt] &= m;
         }
       };
-      auto multiply = [&](const u32x4 (&a)[4], u32x4 (&w)[NW], const u32x4& m, int n_at) {
+      auto multiply = [&](const u32x4 (&a)[4], auto& w, const u32x4& m, int n_at) {
+        constexpr int N = (int)(sizeof(w) / sizeof(w[0]));
         if (mixed && clear_weights) {
 #pragma unroll
-          for (int nt = 0; nt < NW; ++nt) w[nt] &= m;
+          for (int nt = 0; nt < N; ++nt) w[nt] &= m;
         }
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-          for (int nt = 0; nt < NW; ++nt) acc[mt][n_at + nt] = T::mfma16(w[nt], a[mt], acc[mt][n_at + nt]);
+          for (int nt = 0; nt < N; ++nt) acc[mt][n_at + nt] = T::mfma16(w[nt], a[mt], acc[mt][n_at + nt]);
       };
       enter(true);
       read_a(0, a0, c0);
       read_w(w0, 0);
-      if constexpr (WIDE) {
+      if constexpr (WIDE && NT > 4) {
         auto pair = [&](int j, u32x4 (&ac)[4], u32x4& cc, u32x4 (&an)[4], u32x4& cn) {
           read_w(w1, 1);
           __builtin_amdgcn_sched_barrier(0);
@@ -363,7 +386,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
             read_w(w0, 0);
           }
           __builtin_amdgcn_sched_barrier(0);
-          if (kept) multiply(ac, w1, cc, NT - 4);
+          if (kept) multiply(ac, w1, cc, 4);
           __builtin_amdgcn_sched_barrier(0);
         };
         for (int j = 0; j < npairs; j += 2) {
@@ -383,7 +406,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
           __builtin_amdgcn_sched_barrier(0);
         };
         for (int j = 0; j < npairs; j += 2) {
-          pair(j, 1, a0, w0, c0, a1, w1, c1);
+          pair(j, WIDE ? 0 : 1, a0, w0, c0, a1, w1, c1);
           if (j + 1 < npairs) pair(j + 1, 0, a1, w1, c1, a0, w0, c0);
         }
       }
@@ -454,6 +477,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
       }
     }
   }
+}
+
+// LAST: the last group has tiles to leave out.  Layers without take the instances without: four bodies in one kernel spill scalar
+// registers (117, ahead of the loops).
+template <typename T, bool DX, int NT, int KS, bool LAST, bool HALF_CHUNK>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void conv_taps_kernel(TapArgs g) {
+  constexpr bool WIDE = NT == 8;
+  if constexpr (LAST) {
+    const int left = g.n_out - (int)blockIdx.y * (WIDE ? 128 : 64);
+    if constexpr (WIDE) {
+      if (left <= 32) return conv_taps_body<T, DX, true, 2, KS, HALF_CHUNK>(g);
+      if (left <= 64) return conv_taps_body<T, DX, true, 4, KS, HALF_CHUNK>(g);
+      if (left <= 96) return conv_taps_body<T, DX, true, 6, KS, HALF_CHUNK>(g);
+    } else {
+      if (left <= 32) return conv_taps_body<T, DX, false, 2, KS, HALF_CHUNK>(g);
+    }
+  }
+  conv_taps_body<T, DX, WIDE, NT, KS, HALF_CHUNK>(g);
 }
 
 // ---- weight gradient --------------------------------------------------------------------------------------------------
@@ -800,24 +841,31 @@ int configure(const void* kernel, std::atomic<bool>* done) {
   return SD_OK;
 }
 
-template <typename T, bool DX, int NT, int KS>
+template <typename T, bool DX, int NT, int KS, bool LAST = false, bool HALF_CHUNK = false>
 int launch_taps_t(const TapArgs& g, int smem, hipStream_t stream) {
   static std::atomic<bool> done[16] = {};
-  if (int rc = configure(reinterpret_cast<const void*>(&conv_taps_kernel<T, DX, NT, KS>), done)) return rc;
+  auto* kernel = &conv_taps_kernel<T, DX, NT, KS, LAST, HALF_CHUNK>;
+  if (int rc = configure(reinterpret_cast<const void*>(kernel), done)) return rc;
   const dim3 grid((unsigned)((g.rows + kPos - 1) / kPos), (unsigned)g.pack.groups);
-  hipLaunchKernelGGL((conv_taps_kernel<T, DX, NT, KS>), grid, dim3(256), smem, stream, g);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), smem, stream, g);
   return check_launch("conv_taps_kernel");
 }
 
 template <typename T>
 int launch_taps(const TapArgs& g, bool dx, int smem, hipStream_t stream) {
   if (dx) {
-    if (g.n_out <= 32) return g.red <= 32 ? launch_taps_t<T, true, 2, 1>(g, smem, stream) : launch_taps_t<T, true, 2, 2>(g, smem, stream);
-    return g.red <= 32 ? launch_taps_t<T, true, 4, 1>(g, smem, stream) : launch_taps_t<T, true, 4, 2>(g, smem, stream);
+    const bool half = g.red > 32 && (g.red - 1) % 64 < 32, last = (g.n_out - 1) % 64 < 32;
+    if (g.n_out <= 32) {
+      if (g.red <= 32) return launch_taps_t<T, true, 2, 1>(g, smem, stream);
+      return half ? launch_taps_t<T, true, 2, 2, false, true>(g, smem, stream) : launch_taps_t<T, true, 2, 2>(g, smem, stream);
+    }
+    if (g.red <= 32) return last ? launch_taps_t<T, true, 4, 1, true>(g, smem, stream) : launch_taps_t<T, true, 4, 1>(g, smem, stream);
+    if (half) return last ? launch_taps_t<T, true, 4, 2, true, true>(g, smem, stream) : launch_taps_t<T, true, 4, 2, false, true>(g, smem, stream);
+    return last ? launch_taps_t<T, true, 4, 2, true>(g, smem, stream) : launch_taps_t<T, true, 4, 2>(g, smem, stream);
   }
   if (g.n_out <= 32) return launch_taps_t<T, false, 2, 2>(g, smem, stream);
   if (g.n_out <= 64) return launch_taps_t<T, false, 4, 2>(g, smem, stream);
-  return launch_taps_t<T, false, 8, 1>(g, smem, stream);
+  return (g.n_out - 1) % 128 < 96 ? launch_taps_t<T, false, 8, 1, true>(g, smem, stream) : launch_taps_t<T, false, 8, 1>(g, smem, stream);
 }
 
 struct ConvShape {

@@ -100,6 +100,23 @@ def test_products_tap_by_tap(geom, bs, p, channels_last, dtype):
     assert all(torch.equal(a, b) for a, b in zip(got, _products(*args)))
 
 
+# channels, outputs: last groups of 8 to 128 outputs (of 64 channels in the input gradient) and last chunks of one slab and of two,
+# first groups and chunks in front of them and not
+@pytest.mark.parametrize("c,k", [(72, 72), (96, 88), (104, 96), (40, 104), (64, 136), (160, 160), (168, 184), (224, 232), (128, 256),
+                                 (88, 32), (24, 80), (136, 24)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs,p,channels_last", [(64, 0.4, False), (0, 0.0, True)])
+def test_channels_that_end_inside_a_tile_group(c, k, dtype, bs, p, channels_last):
+    geom = (3, c, 10, 13, k, 3, 3, (1, 1), (1, 1))
+    x, wt, dy, rows, gen = _tensors(geom, dtype, seed=c + k)
+    mask = cpu_mask(O.mask_shape(rows, c * 9, bs or 64), p, gen)
+    got = _products(geom, x, wt, dy, mask if bs else None, bs, 1 / (1 - p), channels_last)
+    want = O.conv2d_blockdrop(to_np(x), to_np(wt), mask.numpy(), bs or 64, p, dy=to_np(dy), dtype=np.float64, padding=(1, 1),
+                              stride=(1, 1), dilation=(1, 1))
+    for g, ref in zip(got, want):
+        assert max_tile_rel_fro(g, ref) <= REL_FRO_TOL
+
+
 # (geometry, channels-last image, whether the image is what is kept): rows that fill blocks of 64 and rows that do not
 LAYERS = [((20, 24, 16, 16, 40, 3, 3, (1, 1), (1, 1)), False, True), ((20, 32, 16, 16, 40, 3, 3, (1, 1), (1, 1)), True, False),
           ((7, 16, 28, 28, 40, 3, 3, (1, 1), (1, 1)), False, False), ((7, 16, 28, 28, 40, 5, 5, (2, 2), (1, 1)), True, False)]
