@@ -523,7 +523,10 @@ struct TapDwArgs {
   int per_split, one_more, k_blocks;
 };
 
-template <typename T>
+// KT: tiles of 16 outputs of a workgroup.  As many workgroups as blocks of 64 outputs share them evenly: 88 outputs are two times three
+// tiles, not four and two, since the launch waits for the slowest workgroup.  The same sums in the same order; 200 x 16 x 48 x 48 -> 72,
+// 3 x 3: 46 -> 41 us, 94 x 88 x 32 x 32 -> 88, 5 x 5: 71 -> 66.
+template <typename T, int KT>
 __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2))) void conv_taps_dw_kernel(TapDwArgs g) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t smem_a = lds_address(smem);
@@ -532,7 +535,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
   const int cw = wave % 2, pb = wave / 2;
   const int sp = (int)blockIdx.x, tg = (int)blockIdx.y;
   const int cb = (int)blockIdx.z / g.k_blocks;
-  const int k0 = ((int)blockIdx.z - cb * g.k_blocks) * 64, c0 = cb * 32;
+  const int k0 = ((int)blockIdx.z - cb * g.k_blocks) * (16 * KT), c0 = cb * 32;
   const int RS = g.geo.taps(), t0 = tg * kDwTaps, nt = RS - t0 < kDwTaps ? RS - t0 : kDwTaps;
   // turns of this part: the first `turns % splits` parts have one more
   const int first = sp * g.per_split + (sp < g.one_more ? sp : g.one_more), last = first + g.per_split + (sp < g.one_more ? 1 : 0);
@@ -561,7 +564,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = i * 8 + lane / 8, ch = (lane % 8) ^ swz_x(row);
-    dy_off[i] = k0 + ch * 8 < g.K ? (uint32_t)((row * g.dy_ld + k0 + ch * 8) * 2) : kNoData;
+    dy_off[i] = ch < 2 * KT && k0 + ch * 8 < g.K ? (uint32_t)((row * g.dy_ld + k0 + ch * 8) * 2) : kNoData;
   }
   auto window = [&](int turn) {
     const int m0 = turn * kPos;
@@ -609,7 +612,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
     return d;
   };
 
-  f32x4 acc[kDwTaps][4];
+  f32x4 acc[kDwTaps][KT];
   FragmentReads<false> fd[2];
   fd[0].init(lane, 0);
   fd[1].init(lane, 1);
@@ -625,7 +628,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
     for (int i = 0; i < kDwTaps; ++i)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int k = 0; k < KT; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint32_t kept = 0;
     if (first < last) {
       const uint32_t d1 = dropped(first);
@@ -658,11 +661,11 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
           at[h] = (int)r.x + x_at;
           in[h] = r.y;
         }
-        u32x4 df[4][2];
+        u32x4 df[KT][2];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-          for (int k = 0; k < 4; ++k) df[k][kk] = fd[kk].read(dl, k);
+          for (int k = 0; k < KT; ++k) df[k][kk] = fd[kk].read(dl, k);
         auto read_quarter = [&](int i, int h, u32x4 (&xf)[2]) {
           const int inside = ones_if(in[h], i);
           int a = at[h] + shift[i];
@@ -686,13 +689,13 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
           for (int i = 0; i < kDwTaps; ++i) {
             if (i + 1 < kDwTaps) read_tap(i + 1, xf[(i + 1) % 2]);
             const int m = kept_of(i);
-            f32x4 d[4];
+            f32x4 d[KT];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][0], xf[i % 2][0], acc[i][k]);
+            for (int k = 0; k < KT; ++k) d[k] = T::mfma16(df[k][0], xf[i % 2][0], acc[i][k]);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) d[k] = T::mfma16(df[k][1], xf[i % 2][1], d[k]);
+            for (int k = 0; k < KT; ++k) d[k] = T::mfma16(df[k][1], xf[i % 2][1], d[k]);
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
+            for (int k = 0; k < KT; ++k)
 #pragma unroll
               for (int v = 0; v < 4; ++v) acc[i][k][v] = pick(m, d[k][v], acc[i][k][v]);
             __builtin_amdgcn_sched_barrier(0);
@@ -717,13 +720,13 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
             u32x4(&x)[2] = xf[i % 3];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-              acc[i][k] = T::mfma16(df[k][0], x[0], acc[i][k]);
+              if (k < KT) acc[i][k] = T::mfma16(df[k][0], x[0], acc[i][k]);
               if (i + 2 < kDwTaps) read_quarter(i + 2, k, xf[(i + 2) % 3]);
               __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-              acc[i][k] = T::mfma16(df[k][1], x[1], acc[i][k]);
+              if (k < KT) acc[i][k] = T::mfma16(df[k][1], x[1], acc[i][k]);
               if (i + 1 < kDwTaps) {
                 if (k == 0) m = (uint32_t)kept_of(i + 1);
                 clear(xf[(i + 1) % 3], k, m);
@@ -750,7 +753,7 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
     for (int i = 0; i < kDwTaps; ++i)
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < KT; ++k)
 #pragma unroll
         for (int v = 0; v < 4; ++v) bad = __builtin_fmaf(acc[i][k][v], 0.f, bad);
     uint32_t* again = reinterpret_cast<uint32_t*>(smem + x_bytes);  // (dY's place; the row of zeros stays)
@@ -778,10 +781,11 @@ __global__ __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
     for (int i = 0; i < TAPS; ++i)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4*>(meet + (pb * TILES + i * 4 + k) * 1024) = acc[i0 + i][k];
+      for (int k = 0; k < KT; ++k) *reinterpret_cast<f32x4*>(meet + (pb * TILES + i * 4 + k) * 1024) = acc[i0 + i][k];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TAPS; ++i) {
+      if (KT < 4 && pb >= KT) break;  // the same for the whole wave
       const char* m = meet + (i * 4 + pb) * 1024;
       const f32x4 s01 = *reinterpret_cast<const f32x4*>(m) + *reinterpret_cast<const f32x4*>(m + TILES * 1024);
       const f32x4 s23 = *reinterpret_cast<const f32x4*>(m + 2 * TILES * 1024) + *reinterpret_cast<const f32x4*>(m + 3 * TILES * 1024);
@@ -1123,12 +1127,20 @@ extern "C" int sd_conv2d_taps_dw(const void* x_rows, int64_t x_ld, const void* d
   const int smem = (int)dw_lds(g.span, g.buffers);
   const dim3 grid((unsigned)splits, (unsigned)ceil_div(r * s, kDwTaps), (unsigned)(ceil_div(c, 32) * g.k_blocks));
   const hipStream_t st = (hipStream_t)stream;
-  static std::atomic<bool> done[2][16] = {};
   const bool bf = dtype == SD_BF16;
-  const void* kernel = bf ? reinterpret_cast<const void*>(&conv_taps_dw_kernel<BF16>) : reinterpret_cast<const void*>(&conv_taps_dw_kernel<F16>);
-  if (int rc = configure(kernel, done[bf])) return rc;
-  if (bf) hipLaunchKernelGGL((conv_taps_dw_kernel<BF16>), grid, dim3(kDwThreads), smem, st, g);
-  else hipLaunchKernelGGL((conv_taps_dw_kernel<F16>), grid, dim3(kDwThreads), smem, st, g);
+  const int tiles = (int)ceil_div(ceil_div(k_out, 16), g.k_blocks);  // of a workgroup
+  auto launch = [&](auto type, auto kt) -> int {
+    static std::atomic<bool> done[16] = {};
+    auto* kernel = &conv_taps_dw_kernel<decltype(type), decltype(kt)::value>;
+    if (int rc = configure(reinterpret_cast<const void*>(kernel), done)) return rc;
+    hipLaunchKernelGGL(kernel, grid, dim3(kDwThreads), smem, st, g);
+    return SD_OK;
+  };
+  auto pick = [&](auto type) {
+    if (tiles <= 2) return launch(type, std::integral_constant<int, 2>{});
+    return tiles == 3 ? launch(type, std::integral_constant<int, 3>{}) : launch(type, std::integral_constant<int, 4>{});
+  };
+  if (int rc = bf ? pick(BF16{}) : pick(F16{})) return rc;
   if (int rc = check_launch("conv_taps_dw_kernel")) return rc;
   note_kernel("conv_dw:taps splits=%d", (int)splits);
   const unsigned blocks = (unsigned)ceil_div(r * s * c * k_out / 4, 16);
