@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "mask_source.h"
+#include "tile_map.h"
 
 namespace sd {
 namespace {
@@ -415,6 +416,7 @@ __global__ __launch_bounds__(256) void col2im_kernel(const uint16_t* __restrict_
 // with zeros instead of being read), then each thread sums the taps of its outputs out of LDS.  Global
 // reads are whole segments instead of one 2-byte element per lane and cache line.
 constexpr int C2I_CG = 8;
+constexpr int64_t C2I_WORKGROUPS = 2048;
 constexpr int C2I_MAX_LDS = 60 * 1024;  // below the 64 KB a kernel gets without asking
 
 template <typename T>
@@ -509,145 +511,158 @@ __global__ __launch_bounds__(256) void col2im_tile_kernel(const uint16_t* __rest
 // RT: the kernel size where it is known (RT x RT).  The taps of an output are then unrolled: with loop counters the sum is
 // one LDS latency per tap.  m_qe: ceil(2^32 / window columns), exact while position * columns < 2^32.
 // 256 x 32 x 28 x 28, 3 x 3, p = 0.25: 73 -> 53 us; 167 x 88 x 16 x 16, 5 x 5, p = 0.4: 197 -> 146; 123 x 48 x 7 x 7, 5 x 5: 18 -> 10.
-// By two (from col2im_tile_kernel): 199 x 32 x 48 x 48, 3 x 3, p = 0.25: 127 us there, 45 here.
+// What a wave issues around its loads, sums and stores is what bounds it, not the bytes: without the loads or without the stores
+// 190 x 136 x 30 x 30, 3 x 3 by two, took the same 53 us, without the sums 35.  So with many workgroups one takes up to four groups of channels (RUNS), and
+// what it works out in front of them once: 53 -> 43 us, 51 x 152 x 48 x 48 41 -> 36 (with fewer than 4096, pointwise kernels and
+// channels-last images the loop costs more than it saves: 53 x 144 x 64 x 64 pointwise 33.4 -> 36).  Channels-last images are written in
+// pieces of 16 bytes of a line that eight workgroups share, so those run on one XCD: 199 x 32 x 48 x 48, 3 x 3 by two, 43 -> 30.
+// m_bs: ceil(2^32 / bs), exact for what is divided by it (less than 2^16).
 template <int ST>
 __device__ __host__ inline int floor_div(int v) {  // |v| < 2^30
   return ST == 1 ? v : (v + ST * (1 << 28)) / ST - (1 << 28);
 }
-template <typename T, int RT, int ST>
+template <typename T, int RT, int ST, bool RUNS>
 __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __restrict__ cols, int64_t ld,
                                                           uint16_t* __restrict__ dx, ConvGeom g,
                                                           const uint8_t* mask, int64_t msr, int64_t msc,
-                                                          int bs, int bands, int hb, int qe, uint32_t m_qe) {
+                                                          int bs, uint32_t m_bs, int bands, int hb, int qe, uint32_t m_qe, int per) {
   extern __shared__ __attribute__((aligned(16))) uint16_t seg[];  // [rows of the window][qe][8*R*S + 2]
   const int t = threadIdx.x;
   const int gr = RT ? RT : g.r, gs = RT ? RT : g.s;
   const int rs_n = gr * gs;
   const int seg_h = C2I_CG * rs_n + 2;
-  const int bs_shift = (bs & (bs - 1)) == 0 ? 31 - __builtin_clz((unsigned)bs) : -1;
-  int b = blockIdx.x;
+  int b = g.xs_c == 1 ? xcd_run((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   const int band = b % bands;
   b /= bands;
-  const int cgs = g.c / C2I_CG;
-  const int c0 = (b % cgs) * C2I_CG;
-  const int n_i = b / cgs;
+  if (!RUNS) per = 1;
+  const int cgs = g.c / C2I_CG, runs = RUNS ? (cgs + per - 1) / per : cgs;
+  const int cg0 = b % runs * per, cg_n = RUNS && cg0 + per > cgs ? cgs - cg0 : per;  // groups of channels, one after the other
+  const int c0 = cg0 * C2I_CG, n_i = b / runs;
   const int h0 = band * hb;
   const int h1 = (h0 + hb < g.h ? h0 + hb : g.h);
   const int p_first = floor_div<ST>(h0 + g.pad_h - (gr - 1)), q_first = floor_div<ST>(g.pad_w - (gs - 1));  // staged window: its top-left (p, q)
   const int pe = floor_div<ST>(h1 - 1 + g.pad_h) - p_first + 1;                                           // and rows
 
-  // ---- stage: R*S 16-byte chunks per window position, zeros outside the matrix and for dropped blocks
-  const int chunks = pe * qe * rs_n;
+  // ---- stage: R*S 16-byte chunks per window position, zeros outside the matrix and for dropped blocks.  A thread keeps its chunk
+  //      and goes from position to position, and the mask entries that the window can touch (few: blocks of 64 and more) are copied
+  //      to LDS first, so that nothing is divided and nothing branches per 16 bytes.
   const int col0 = c0 * rs_n;
-  // the few mask entries the window can touch are copied to LDS first, so that the staging loop does not
-  // chain a global mask read in front of every data load
   __shared__ uint8_t mtab[256];
+  int cb_lo = 0, cb_n = 0, at0 = 0;  // without a mask every chunk looks at entry 0
   int64_t rb_lo = 0;
-  int cb_lo = 0, cb_n = 1;
-  bool mask_in_lds = false;
+  bool in_table = true;
+  auto block_of = [&](int v) { return (int)__umulhi((uint32_t)v, m_bs); };  // of a row or column counted from the first of a block
   if (mask) {
-    const int pp_lo = p_first > 0 ? p_first : 0;
-    const int pp_hi = p_first + pe - 1 < g.p - 1 ? p_first + pe - 1 : g.p - 1;
-    rb_lo = (((int64_t)n_i * g.p + pp_lo) * g.q) / bs;
-    const int64_t rb_hi = (((int64_t)n_i * g.p + pp_hi) * g.q + g.q - 1) / bs;
+    const int64_t image_row = (int64_t)n_i * g.p * g.q;
+    const int pp_lo = p_first > 0 ? p_first : 0, pp_hi = p_first + pe - 1 < g.p - 1 ? p_first + pe - 1 : g.p - 1;
+    const int64_t row_lo = image_row + (int64_t)pp_lo * g.q;
+    rb_lo = row_lo / bs;
+    at0 = (int)(image_row - rb_lo * bs);
+    const int64_t rb_n = pp_hi >= pp_lo ? (row_lo - rb_lo * bs + (int64_t)(pp_hi - pp_lo + 1) * g.q - 1) / bs + 1 : 0;
     cb_lo = col0 / bs;
-    cb_n = (col0 + C2I_CG * rs_n - 1) / bs - cb_lo + 1;
-    const int64_t rb_n = pp_hi >= pp_lo ? rb_hi - rb_lo + 1 : 0;
-    mask_in_lds = rb_n * cb_n <= 256;
-    if (mask_in_lds) {
-      if (t < rb_n * cb_n) mtab[t] = mask[(rb_lo + t / cb_n) * msr + (cb_lo + t % cb_n) * msc];
-      __syncthreads();
+    cb_n = (col0 + cg_n * C2I_CG * rs_n - 1) / bs - cb_lo + 1;
+    in_table = rb_n * cb_n <= 256;
+    if (in_table && t < rb_n * cb_n) {
+      const int rb = t / cb_n;
+      mtab[t] = mask[(rb_lo + rb) * msr + (cb_lo + t - rb * cb_n) * msc];
     }
-  }
-  const uint16_t* image = cols + (int64_t)n_i * g.p * g.q * ld;
-  const int at0 = (int)((int64_t)n_i * g.p * g.q - rb_lo * bs);
-  for (int ch0 = t; ch0 < chunks; ch0 += 4 * 256) {
-    u32x4 v[4];
-    const uint16_t* src[4];  // null: zeros
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {  // four independent mask reads, then four independent loads, per lane
-      const int ch = ch0 + i * 256;
-      src[i] = nullptr;
-      uint8_t dropped = 0;
-      if (ch < chunks) {
-        const int pos = ch / rs_n, k = ch - pos * rs_n;
-        const int pl = qe == 1 ? pos : (int)__umulhi((uint32_t)pos, m_qe);
-        const int pp = p_first + pl, qq = q_first + pos - pl * qe;
-        if (pp >= 0 && pp < g.p && qq >= 0 && qq < g.q) {
-          const int row = pp * g.q + qq;  // inside the image
-          const int col = col0 + k * 8;
-          src[i] = image + (int64_t)row * ld + col;
-          if (mask) {
-            // block sizes are powers of two in practice: a shift instead of a division per chunk
-            const int at = row + at0;  // behind the first position of row block rb_lo
-            const int rb = bs_shift >= 0 ? at >> bs_shift : at / bs;
-            const int cb = bs_shift >= 0 ? col >> bs_shift : col / bs;
-            dropped = mask_in_lds ? mtab[rb * cb_n + (cb - cb_lo)] : mask[(rb_lo + rb) * msr + cb * msc];
-          }
-        }
-      }
-      if (dropped) src[i] = nullptr;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = u32x4{0u, 0u, 0u, 0u};
-      if (src[i]) v[i] = *reinterpret_cast<const u32x4*>(src[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = ch0 + i * 256;
-      if (ch < chunks) {
-        const int pos = ch / rs_n, k = ch - pos * rs_n;
-        uint32_t* dst = reinterpret_cast<uint32_t*>(seg + pos * seg_h + k * 8);
-        dst[0] = v[i].x;
-        dst[1] = v[i].y;
-        dst[2] = v[i].z;
-        dst[3] = v[i].w;
-      }
-    }
+  } else if (t == 0) {
+    mtab[0] = 0;
   }
   __syncthreads();
-
-  // ---- sum the taps: those of output (h, w) are r = (h + pad_h) % ST + i * ST, at window row (h + pad_h) / ST - p_first - i, and
-  //      s likewise
+  const uint16_t* image = cols + (int64_t)n_i * g.p * g.q * ld + col0;
+  const int kw = rs_n < 256 ? rs_n : 256, step = 256 / kw, npos = pe * qe;  // threads to a position, positions at a time
+  const int down = step / qe, right = step - down * qe, first = t / kw;
+  const int row_on = down * g.q + right, wrap = g.q - qe;  // rows of the matrix on with a step, and more at the end of a window row
+  const int col_in = mask ? col0 - cb_lo * bs : 0;  // of its block
   const bool c_fast = g.xs_c == 1;
   const int pairs = C2I_CG * g.w;
   const int row_h = qe * seg_h;  // halfs per window row
-  uint16_t* dxn = dx + (int64_t)n_i * g.xs_n;
-  for (int pr = t; pr < pairs; pr += 256) {
-    const int c_l = c_fast ? pr % C2I_CG : pr / g.w;
-    const int wi = c_fast ? pr / C2I_CG : pr % g.w;
-    const int s0 = (wi + g.pad_w) % ST;
-    // the first tap's column in the window's first row
-    const uint16_t* base = seg + ((wi + g.pad_w) / ST - q_first) * seg_h + c_l * rs_n + s0;
-    uint16_t* out = dxn + (int64_t)(c0 + c_l) * g.xs_c + (int64_t)h0 * g.xs_h + (int64_t)wi * g.xs_w;
-    for (int hl = 0; hl < h1 - h0; ++hl) {
-      float acc = 0.f;
-      const int hp = h0 + hl + g.pad_h, r0 = hp % ST;
-      const uint16_t* tap_r = base + (hp / ST - p_first) * row_h + r0 * gs;
-      if constexpr (RT > 0) {
-        constexpr int N = (RT + ST - 1) / ST;
+  uint16_t* dxn = dx + (int64_t)n_i * g.xs_n + (int64_t)c0 * g.xs_c + (int64_t)h0 * g.xs_h;
+  for (int cg = 0; cg < cg_n; ++cg, image += C2I_CG * rs_n, dxn += C2I_CG * g.xs_c) {
+    if (cg) __syncthreads();  // nobody reads the group before any more
+    if (first < step) {
+      for (int k = t - first * kw; k < rs_n; k += kw) {
+        const int cb = mask ? block_of(col_in + (cg * rs_n + k) * C2I_CG) : 0;
+        const uint16_t* from = image + k * 8;
+        const int pl = qe == 1 ? first : (int)__umulhi((uint32_t)first, m_qe);
+        int qq = first - pl * qe, row = (p_first + pl) * g.q + q_first + qq, pp = p_first + pl;
+        uint16_t* to = seg + first * seg_h + k * 8;
+        for (int pos = first; pos < npos; pos += 4 * step) {
+          u32x4 v[4];
+          const uint16_t* src[4];
+          bool there[4];
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-          if (i * ST + ST > RT && r0 + i * ST >= RT) break;  // the same for every thread
+          for (int i = 0; i < 4; ++i) {  // four independent mask reads, then four independent loads, per lane
+            const bool inside = (pos + i * step < npos) & ((unsigned)pp < (unsigned)g.p) & ((unsigned)(q_first + qq) < (unsigned)g.q);
+            const int rb = block_of(inside ? row + at0 : 0);
+            const uint8_t dropped = in_table ? mtab[rb * cb_n + cb] : (inside ? mask[(rb_lo + rb) * msr + (cb_lo + cb) * msc] : 0);
+            there[i] = inside & (dropped == 0);
+            src[i] = from + (int64_t)row * ld;
+            qq += right;
+            const int over = qq >= qe ? 1 : 0;
+            qq -= over ? qe : 0;
+            pp += down + over;
+            row += row_on + (over ? wrap : 0);
+          }
 #pragma unroll
-          for (int k = 0; k < N; ++k) {
-            const bool there = k * ST + ST <= RT || s0 + k * ST < RT;
-            const float v = T::to_float(tap_r[i * (ST * RT - row_h) + (there ? k * (ST - seg_h) : -s0)]);
-            acc += there ? v : 0.f;
+          for (int i = 0; i < 4; ++i) {
+            v[i] = u32x4{0u, 0u, 0u, 0u};
+            if (there[i]) v[i] = *reinterpret_cast<const u32x4*>(src[i]);
           }
-        }
-      } else {
-        for (int rr = r0; rr < gr; rr += ST) {
-          const uint16_t* tap = tap_r;
-          for (int ss = s0; ss < gs; ss += ST) {
-            acc += T::to_float(*tap);
-            tap -= seg_h - ST;  // one window column to the left, ST taps on
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (pos + i * step < npos) {
+              uint32_t* dst = reinterpret_cast<uint32_t*>(to);
+              dst[0] = v[i].x;
+              dst[1] = v[i].y;
+              dst[2] = v[i].z;
+              dst[3] = v[i].w;
+            }
+            to += step * seg_h;
           }
-          tap_r -= row_h - ST * gs;  // one window row up
         }
       }
-      out[(int64_t)hl * g.xs_h] = T::from_float(acc);
+    }
+    __syncthreads();
+
+    // ---- sum the taps: those of output (h, w) are r = (h + pad_h) % ST + i * ST, at window row (h + pad_h) / ST - p_first - i, and
+    //      s likewise
+    for (int pr = t; pr < pairs; pr += 256) {
+      const int c_l = c_fast ? pr % C2I_CG : pr / g.w;
+      const int wi = c_fast ? pr / C2I_CG : pr % g.w;
+      const int s0 = (wi + g.pad_w) % ST;
+      // the first tap's column in the window's first row
+      const uint16_t* base = seg + ((wi + g.pad_w) / ST - q_first) * seg_h + c_l * rs_n + s0;
+      uint16_t* out = dxn + (int64_t)c_l * g.xs_c + (int64_t)wi * g.xs_w;
+      for (int hl = 0; hl < h1 - h0; ++hl) {
+        float acc = 0.f;
+        const int hp = h0 + hl + g.pad_h, r0 = hp % ST;
+        const uint16_t* tap_r = base + (hp / ST - p_first) * row_h + r0 * gs;
+        if constexpr (RT > 0) {
+          constexpr int N = (RT + ST - 1) / ST;
+#pragma unroll
+          for (int i = 0; i < N; ++i) {
+            if (i * ST + ST > RT && r0 + i * ST >= RT) break;  // the same for every thread
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+              const bool there = k * ST + ST <= RT || s0 + k * ST < RT;
+              const float v = T::to_float(tap_r[i * (ST * RT - row_h) + (there ? k * (ST - seg_h) : -s0)]);
+              acc += there ? v : 0.f;
+            }
+          }
+        } else {
+          for (int rr = r0; rr < gr; rr += ST) {
+            const uint16_t* tap = tap_r;
+            for (int ss = s0; ss < gs; ss += ST) {
+              acc += T::to_float(*tap);
+              tap -= seg_h - ST;  // one window column to the left, ST taps on
+            }
+            tap_r -= row_h - ST * gs;  // one window row up
+          }
+        }
+        out[(int64_t)hl * g.xs_h] = T::from_float(acc);
+      }
     }
   }
 }
@@ -793,19 +808,24 @@ int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64
         const int64_t qe = st == 1 ? g.w + g.s - 1 : floor_div<2>(g.w - 1 + g.pad_w) - floor_div<2>(g.pad_w - (g.s - 1)) + 1;
         const int64_t lds = pe * qe * seg_bytes;
         const int64_t bands = ceil_div(g.h, hb);
-        const int64_t wgs = n * (c / C2I_CG) * bands;
-        if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL) continue;
+        const int64_t groups = n * (c / C2I_CG) * bands;
+        const int rt = g.r == g.s && (g.r == 1 || g.r == 3 || g.r == 5) ? g.r : 0;
+        const bool in_runs = rt > 1 && sc != 1 && groups >= 2 * C2I_WORKGROUPS;
+        const int64_t per = in_runs ? std::min<int64_t>(4, groups / C2I_WORKGROUPS) : 1;
+        const int64_t wgs = n * ceil_div(c / C2I_CG, per) * bands;
+        if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL || (mask && (bs > 32768 || pe * g.q > 32768))) continue;
         const uint32_t m_qe = qe <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)qe - 1) / (uint64_t)qe);
+        const uint32_t m_bs = !mask || bs <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)bs - 1) / (uint64_t)bs);
         auto launch = [&](auto* kernel) {
           hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), (size_t)lds, stream, (const uint16_t*)cols, ld,
-                             (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, (int)bands, hb, (int)qe, m_qe);
+                             (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs, (int)bands, hb, (int)qe, m_qe, (int)per);
         };
-        const int rt = g.r == g.s && (g.r == 1 || g.r == 3 || g.r == 5) ? g.r : 0;
         auto pick = [&](auto type, auto step) {
           using T = decltype(type);
           constexpr int ST = decltype(step)::value;
-          rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST>) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST>)
-          : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST>) : launch(&col2im_unit_kernel<T, 0, ST>);
+          if (in_runs) rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, true>) : launch(&col2im_unit_kernel<T, 5, ST, true>);
+          else rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST, false>) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, false>)
+               : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST, false>) : launch(&col2im_unit_kernel<T, 0, ST, false>);
         };
         const std::integral_constant<int, 1> one;
         const std::integral_constant<int, 2> two;

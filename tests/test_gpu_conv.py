@@ -194,6 +194,38 @@ def test_col2im_with_stride_two(cfg, channels_last, dtype, bs):
     assert bool(((dx.cpu().double() - ref).abs() <= eps * ref.abs() + 2.0 ** -18).all())
 
 
+# two, three and four groups of channels to a workgroup, the last with fewer, in one band and in two of unequal height
+@pytest.mark.parametrize("cfg", [
+    dict(n=600, c=56, h=6, w=5, r=3, padding=(1, 1), stride=(2, 2)),
+    dict(n=850, c=64, h=4, w=7, r=3, padding=(1, 1), stride=(1, 1)),
+    dict(n=700, c=48, h=11, w=6, r=3, padding=(0, 2), stride=(2, 2)),
+    dict(n=300, c=120, h=9, w=4, r=5, padding=(2, 2), stride=(2, 2)),
+])
+@pytest.mark.parametrize("bs,p", [(None, 0.0), (64, 0.5), (192, 0.3)])
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_col2im_of_many_workgroups(cfg, bs, p, channels_last):
+    from flash_dropout.hip import GEMM
+
+    geo = dict(padding=cfg["padding"], stride=cfg["stride"], dilation=(1, 1))
+    shape, ks = (cfg["n"], cfg["c"], cfg["h"], cfg["w"]), (cfg["r"], cfg["r"])
+    assert cfg["n"] * (cfg["c"] // 8) * -(-cfg["h"] // 8) >= 4096
+    gen = torch.Generator().manual_seed(cfg["n"])
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], *ks, **geo)
+    rows, ncols = cfg["n"] * p_ * q_, cfg["c"] * cfg["r"] ** 2
+    g = torch.randn(rows, ncols, generator=gen).half()
+    given, mask = g.clone(), None
+    if bs:
+        mask = cpu_mask(O.mask_shape(rows, ncols, bs), p, gen)
+        keep = torch.from_numpy(O.expand_keep(mask.numpy(), bs, rows, ncols))
+        given[~keep] = float("nan")  # dropped blocks are not read
+        g = torch.where(keep, g, torch.zeros_like(g))
+        mask = mask.cuda()
+    dx = GEMM().col2im(given.cuda(), shape, ks, mask=mask, block_size=bs, channels_last=channels_last, **geo)
+    ref = torch.nn.functional.fold(g.double().reshape(cfg["n"], p_ * q_, ncols).permute(0, 2, 1), shape[2:], ks, padding=cfg["padding"],
+                                   stride=cfg["stride"])
+    assert bool(((dx.cpu().double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 2.0 ** -18).all())  # as above
+
+
 @pytest.mark.parametrize("cfg", [
     dict(n=8, c=64, h=32, w=32, k=128, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),
     dict(n=4, c=24, h=17, w=15, k=40, r=3, s=3, padding=(1, 0), stride=(2, 1), dilation=(1, 1)),
