@@ -194,6 +194,48 @@ def test_col2im_with_stride_two(cfg, channels_last, dtype, bs):
     assert bool(((dx.cpu().double() - ref).abs() <= eps * ref.abs() + 2.0 ** -18).all())
 
 
+# pixels and channels that fill a tile of 64 and that do not, images that start and end inside a block of rows
+@pytest.mark.parametrize("n,c,h,w", [(3, 64, 8, 8), (2, 8, 7, 7), (5, 72, 9, 15), (1, 130, 3, 70), (4, 65, 1, 5), (3, 1, 16, 12), (2, 200, 20, 13)])
+@pytest.mark.parametrize("bs", [None, 64, 128, 192])
+@pytest.mark.parametrize("sliced", [False, True])
+def test_col2im_of_pointwise_kernels(n, c, h, w, bs, sliced):
+    from flash_dropout.hip import GEMM
+
+    gen = torch.Generator().manual_seed(n * c + h)
+    rows = n * h * w
+    g = torch.randn(rows, c, generator=gen).half()
+    given, mask = g.clone(), None
+    if bs:
+        mask = cpu_mask(O.mask_shape(rows, c, bs), 0.4, gen)
+        keep = torch.from_numpy(O.expand_keep(mask.numpy(), bs, rows, c))
+        given[~keep] = float("nan")  # dropped blocks are not read
+        g = torch.where(keep, g, torch.zeros_like(g))
+        mask = mask.cuda()
+    given = given.cuda()
+    if sliced:  # rows that start on any boundary
+        given = torch.cat([given.new_zeros(rows, 3), given], 1)[:, 3:]
+    dx = GEMM().col2im(given, (n, c, h, w), (1, 1), mask=mask, block_size=bs)
+    assert torch.equal(dx.cpu(), g.reshape(n, h * w, c).permute(0, 2, 1).reshape(n, c, h, w))
+
+
+@pytest.mark.parametrize("n,c,h,w,k", [(9, 72, 15, 13, 40), (3, 24, 56, 56, 72), (20, 104, 7, 7, 100), (2, 200, 30, 30, 64)])
+@pytest.mark.parametrize("bs", [64, 128])
+@pytest.mark.parametrize("sliced", [False, True])
+def test_pointwise_convolutions_of_planes_and_of_pixels_agree(n, c, h, w, k, bs, sliced):
+    import flash_dropout.functional as F
+
+    gen = torch.Generator().manual_seed(c)
+    x = torch.randn(n, c + 8 * sliced, h, w, generator=gen).half().cuda()[:, 4 * sliced:][:, :c]
+    wt = (torch.randn(k, c, 1, 1, generator=gen) * c ** -0.5).half().cuda().requires_grad_()
+    dy = torch.randn(n, k, h, w, generator=gen).half().cuda()
+    got = []
+    for image in (x, x.contiguous(memory_format=torch.channels_last)):
+        image = image.detach().requires_grad_()
+        y = F.blockwise_dropout_conv2d(image, wt, bs, 0.4, 0, 1, seed=11)
+        got.append((y, *torch.autograd.grad(y, (image, wt), dy)))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 # two, three and four groups of channels to a workgroup, the last with fewer, in one band and in two of unequal height
 @pytest.mark.parametrize("cfg", [
     dict(n=600, c=56, h=6, w=5, r=3, padding=(1, 1), stride=(2, 2)),
