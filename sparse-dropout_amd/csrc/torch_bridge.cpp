@@ -680,19 +680,6 @@ Tensor pixel_rows(const Tensor& x) {
   return pixels ? x.as_strided({x.size(0) * h * w, c}, {c, 1}) : Tensor();
 }
 
-// Which products of a masked convolution that the library takes without a patch matrix go through one all the same (the image is
-// what is kept then too, and gathered once more for the kernel's gradient).  Measured on 298 drawn layers of 24 to 950 thousand
-// rows, 32 fused input gradients among them; times through the matrix against those without, geometric means:
-//  * forward: a workgroup takes 256 rows x 128 outputs and builds its tiles step by step; fewer than 64 of them 0.67 (9 x 96 x 8 x 8 ->
-//    192, 5 x 5, p = 0.5, six of them: 45 us a pass for 306), 64 to 128 1.02, more 1.3; pointwise kernels, a step each, 1.04 to 1.3
-//  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16
-//  * input gradient, SDD and col2im against the fused kernel: 0.35, 1.03 at most, 0.6 to 0.85 on 42 to 130 MB (187 x 48 x 32 x 32 -> 64
-//    by two 102 -> 85 us a pass); 1.03 to 1.09 where the matrix is one block wide.  Past 256 MB it stays out of memory.
-bool forward_by_patches(const ConvGeom& g) { return g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64; }
-bool dw_by_patches(const ConvGeom& g) { return g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
-bool dx_may_fuse(const ConvGeom& g) { return g.k % 64 == 0 && g.k <= 256 && g.qo <= 64 && 64 % g.qo == 0 && g.po * g.qo % 64 == 0; }
-bool dx_by_patches(const ConvGeom& g) { return g.cols() > 64 && g.rows() * g.cols() * 2 <= 256LL << 20; }
-
 // [N*H*W, C] rows of a tensor stored plane by plane, in memory of their own
 bool whole_planes(const Tensor& t) {
   return t.stride(3) == 1 && (t.size(2) == 1 || t.stride(2) == t.size(3)) && t.stride(1) >= t.size(2) * t.size(3) && t.size(1) > 1 &&
@@ -706,6 +693,28 @@ Tensor rows_of_planes(const Tensor& t) {
         "sd_rows_from_planes");
   return rows;
 }
+// Whether that is the cheapest patch matrix of a pointwise kernel (own_patches)
+bool turned(const Tensor& x, const ConvGeom& g) {
+  return pointwise(g) && g.n > 0 && whole_planes(x) && g.rows() * g.c * 2 <= 64LL << 20;
+}
+
+// Which products of a masked convolution that the library takes without a patch matrix go through one all the same (the image is
+// what is kept then too, and gathered once more for the kernel's gradient).  Measured on 298 drawn layers of 24 to 950 thousand
+// rows, 32 fused input gradients among them; times through the matrix against those without, geometric means:
+//  * forward: a workgroup takes 256 rows x 128 outputs and builds its tiles step by step; fewer than 64 of them 0.67 (9 x 96 x 8 x 8 ->
+//    192, 5 x 5, p = 0.5, six of them: 45 us a pass for 306), 64 to 128 1.02, more 1.3; pointwise kernels, a step each, 1.04 to 1.3
+//    gathered
+//  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16 gathered
+//  * both of pointwise kernels whose image's planes are turned: passes of 14 layers that the GPU bounds 0.92 of those without, 1.00 at
+//    worst (32 x 40 x 64 x 64 -> 176, p = 0.5 105 -> 85 us, 215 x 32 x 64 x 64 -> 56, p = 0.6 264 -> 222)
+//  * input gradient, SDD and col2im against the fused kernel: 0.35, 1.03 at most, 0.6 to 0.85 on 42 to 130 MB (187 x 48 x 32 x 32 -> 64
+//    by two 102 -> 85 us a pass); 1.03 to 1.09 where the matrix is one block wide.  Past 256 MB it stays out of memory.
+bool forward_by_patches(const Tensor& x, const ConvGeom& g) {
+  return turned(x, g) || (g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64);
+}
+bool dw_by_patches(const Tensor& x, const ConvGeom& g) { return turned(x, g) || g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
+bool dx_may_fuse(const ConvGeom& g) { return g.k % 64 == 0 && g.k <= 256 && g.qo <= 64 && 64 % g.qo == 0 && g.po * g.qo % 64 == 0; }
+bool dx_by_patches(const ConvGeom& g) { return g.cols() > 64 && g.rows() * g.cols() * 2 <= 256LL << 20; }
 
 // The patch matrix of a pointwise kernel: the image itself where it is its own, up to 64 MB the rows of its planes, else undefined.  Turning
 // whole planes costs less than gathering the kept blocks of them, where blocks, rows and columns are looked up, as long as the caches hold
@@ -714,7 +723,7 @@ Tensor rows_of_planes(const Tensor& t) {
 Tensor own_patches(const Tensor& x, const ConvGeom& g) {
   if (!pointwise(g) || g.n == 0) return Tensor();
   const Tensor own = g.c % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 ? pixel_rows(x) : Tensor();
-  return own.defined() || !whole_planes(x) || g.rows() * g.c * 2 > 64LL << 20 ? own : rows_of_planes(x);
+  return own.defined() || !turned(x, g) ? own : rows_of_planes(x);
 }
 Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
   const Tensor rows = own_patches(x, g);
@@ -913,7 +922,7 @@ struct ConvBackward : Node {
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
     // both gradients through the patch matrix: one launch where the pair qualifies, and the fold
-    const bool dw_through = pixels || patches.defined() || dw_by_patches(g), dx_through = !fused_dx || dx_by_patches(g) || !dx_may_fuse(g);
+    const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g), dx_through = !fused_dx || dx_by_patches(g) || !dx_may_fuse(g);
     if (l && task_should_compute_output(0) && task_should_compute_output(1) && dw_through && dx_through && layer_takes(g, w) && rows_on_16_bytes(dy2)) {
       if (!patches.defined()) patches = im2col(image, g, l);
       if (rows_on_16_bytes(patches)) {
@@ -973,7 +982,7 @@ struct ConvBackward : Node {
       Tensor dk;
       if (pixels) patches = im2col(image, g, l);
       if (!patches.defined()) {  // the image was kept
-        if (!(l && dw_by_patches(g))) dk = conv_dw(image, dy2, g, l, scale);
+        if (!(l && dw_by_patches(image, g))) dk = conv_dw(image, dy2, g, l, scale);
         if (!dk.defined()) patches = im2col(image, g, l);
       }
       last_routes[2] = dk.defined() ? kImplicit : kExplicit;
@@ -1072,7 +1081,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     const Draw draw{mask, seed, state};
     // A draw from the generator's state is made by one launch and read from what that stored: between two launches that each
     // make it another stream may move the state on, and the product would read blocks that were not gathered.
-    const bool implicit = takes_implicit && !(bs && forward_by_patches(g)), layer = bs && layer_takes(g, w2) && !draw.state_ptr();
+    const bool implicit = takes_implicit && !(bs && forward_by_patches(x, g)), layer = bs && layer_takes(g, w2) && !draw.state_ptr();
     if (implicit || !layer) {
       if (bs) conv_lists(x, g, bs, p, draw, lists);
       y2 = new_matrix(x, g.rows(), g.k);

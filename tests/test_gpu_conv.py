@@ -656,9 +656,13 @@ def test_conv_routes_are_reported_and_block_sizes_above_64_stay_fused(bs, dx_rou
     (dict(n=31, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("explicit", "explicit", "explicit")),
     (dict(n=63, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("explicit", "explicit", "implicit")),
     (dict(n=64, c=8, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1)), 0.3, ("implicit", "explicit", "implicit")),
-    # pointwise kernels: the forward stays implicit, the kernel's gradient from 16384 rows on
-    (dict(n=15, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("implicit", "fused", "explicit")),
-    (dict(n=16, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("implicit", "fused", "implicit")),
+    # pointwise kernels: planes of up to 64 MB are turned, by two the forward stays implicit, the kernel's gradient from 16384 rows on
+    (dict(n=15, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("explicit", "fused", "explicit")),
+    (dict(n=16, c=16, h=32, w=32, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("explicit", "fused", "explicit")),
+    (dict(n=15, c=16, h=64, w=64, k=64, r=1, s=1, stride=(2, 2), padding=(0, 0)), 0.3, ("implicit", "explicit", "explicit")),
+    (dict(n=16, c=16, h=64, w=64, k=64, r=1, s=1, stride=(2, 2), padding=(0, 0)), 0.3, ("implicit", "explicit", "implicit")),
+    (dict(n=128, c=64, h=64, w=64, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("explicit", "explicit", "explicit")),  # 64 MB
+    (dict(n=129, c=64, h=64, w=64, k=64, r=1, s=1, stride=(1, 1), padding=(0, 0)), 0.3, ("implicit", "explicit", "implicit")),
     # 300 MB of patch gradient stay out of memory
     (dict(n=192, c=32, h=64, w=64, k=64, r=5, s=5, stride=(2, 2), padding=(2, 2)), 0.9, ("implicit", "fused", "implicit")),
 ])
