@@ -416,6 +416,7 @@ __global__ __launch_bounds__(256) void col2im_kernel(const uint16_t* __restrict_
 // with zeros instead of being read), then each thread sums the taps of its outputs out of LDS.  Global
 // reads are whole segments instead of one 2-byte element per lane and cache line.
 constexpr int C2I_CG = 8;
+constexpr int C2I_FEW_LDS = 30 * 1024;
 constexpr int64_t C2I_WORKGROUPS = 2048;
 constexpr int C2I_MAX_LDS = 60 * 1024;  // below the 64 KB a kernel gets without asking
 
@@ -516,13 +517,15 @@ __global__ __launch_bounds__(256) void col2im_tile_kernel(const uint16_t* __rest
 // what it works out in front of them once: 53 -> 43 us, 51 x 152 x 48 x 48 41 -> 36 (with fewer than 4096, pointwise kernels and
 // channels-last images the loop costs more than it saves: 53 x 144 x 64 x 64 pointwise 33.4 -> 36).  Channels-last images are written in
 // pieces of 16 bytes of a line that eight workgroups share, so those run on one XCD: 199 x 32 x 48 x 48, 3 x 3 by two, 43 -> 30.
+// THREADS: 512 where at most five workgroups' windows of a 5 x 5 kernel fit a CU, two threads to a column of a band: 179 x 112 x 32 x 32 by two
+// 121 -> 103 us, 36 x 152 x 8 x 8 18 -> 13.  (With windows of 20 to 30 KB, 3 x 3 kernels, 30 -> 40 on 199 x 32 x 48 x 48.)
 // m_bs: ceil(2^32 / bs), exact for what is divided by it (less than 2^16).
 template <int ST>
 __device__ __host__ inline int floor_div(int v) {  // |v| < 2^30
   return ST == 1 ? v : (v + ST * (1 << 28)) / ST - (1 << 28);
 }
-template <typename T, int RT, int ST, bool RUNS>
-__global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __restrict__ cols, int64_t ld,
+template <typename T, int RT, int ST, bool RUNS, int THREADS>
+__global__ __launch_bounds__(THREADS) void col2im_unit_kernel(const uint16_t* __restrict__ cols, int64_t ld,
                                                           uint16_t* __restrict__ dx, ConvGeom g,
                                                           const uint8_t* mask, int64_t msr, int64_t msc,
                                                           int bs, uint32_t m_bs, int bands, int hb, int qe, uint32_t m_qe, int per) {
@@ -571,7 +574,7 @@ __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __rest
   }
   __syncthreads();
   const uint16_t* image = cols + (int64_t)n_i * g.p * g.q * ld + col0;
-  const int kw = rs_n < 256 ? rs_n : 256, step = 256 / kw, npos = pe * qe;  // threads to a position, positions at a time
+  const int kw = rs_n < THREADS ? rs_n : THREADS, step = THREADS / kw, npos = pe * qe;  // threads to a position, positions at a time
   const int down = step / qe, right = step - down * qe, first = t / kw;
   const int row_on = down * g.q + right, wrap = g.q - qe;  // rows of the matrix on with a step, and more at the end of a window row
   const int col_in = mask ? col0 - cb_lo * bs : 0;  // of its block
@@ -628,14 +631,14 @@ __global__ __launch_bounds__(256) void col2im_unit_kernel(const uint16_t* __rest
 
     // ---- sum the taps: those of output (h, w) are r = (h + pad_h) % ST + i * ST, at window row (h + pad_h) / ST - p_first - i, and
     //      s likewise
-    for (int pr = t; pr < pairs; pr += 256) {
+    for (int pr = THREADS == 256 ? t : t % 256; pr < pairs; pr += 256) {
       const int c_l = c_fast ? pr % C2I_CG : pr / g.w;
       const int wi = c_fast ? pr / C2I_CG : pr % g.w;
       const int s0 = (wi + g.pad_w) % ST;
       // the first tap's column in the window's first row
       const uint16_t* base = seg + ((wi + g.pad_w) / ST - q_first) * seg_h + c_l * rs_n + s0;
       uint16_t* out = dxn + (int64_t)c_l * g.xs_c + (int64_t)wi * g.xs_w;
-      for (int hl = 0; hl < h1 - h0; ++hl) {
+      for (int hl = THREADS == 256 ? 0 : t / 256; hl < h1 - h0; hl += THREADS / 256) {
         float acc = 0.f;
         const int hp = h0 + hl + g.pad_h, r0 = hp % ST;
         const uint16_t* tap_r = base + (hp / ST - p_first) * row_h + r0 * gs;
@@ -894,16 +897,18 @@ int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64
         if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL || (mask && (bs > 32768 || pe * g.q > 32768))) continue;
         const uint32_t m_qe = qe <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)qe - 1) / (uint64_t)qe);
         const uint32_t m_bs = !mask || bs <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)bs - 1) / (uint64_t)bs);
-        auto launch = [&](auto* kernel) {
-          hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), (size_t)lds, stream, (const uint16_t*)cols, ld,
+        auto launch = [&](auto* kernel, int threads) {
+          hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), (size_t)lds, stream, (const uint16_t*)cols, ld,
                              (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs, (int)bands, hb, (int)qe, m_qe, (int)per);
         };
+        const bool wide = rt == 5 && lds > C2I_FEW_LDS;
         auto pick = [&](auto type, auto step) {
           using T = decltype(type);
           constexpr int ST = decltype(step)::value;
-          if (in_runs) rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, true>) : launch(&col2im_unit_kernel<T, 5, ST, true>);
-          else rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST, false>) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, false>)
-               : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST, false>) : launch(&col2im_unit_kernel<T, 0, ST, false>);
+          if (wide) in_runs ? launch(&col2im_unit_kernel<T, 5, ST, true, 512>, 512) : launch(&col2im_unit_kernel<T, 5, ST, false, 512>, 512);
+          else if (in_runs) rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, true, 256>, 256) : launch(&col2im_unit_kernel<T, 5, ST, true, 256>, 256);
+          else rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST, false, 256>, 256) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, false, 256>, 256)
+               : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST, false, 256>, 256) : launch(&col2im_unit_kernel<T, 0, ST, false, 256>, 256);
         };
         const std::integral_constant<int, 1> one;
         const std::integral_constant<int, 2> two;

@@ -242,6 +242,8 @@ def test_pointwise_convolutions_of_planes_and_of_pixels_agree(n, c, h, w, k, bs,
     dict(n=850, c=64, h=4, w=7, r=3, padding=(1, 1), stride=(1, 1)),
     dict(n=700, c=48, h=11, w=6, r=3, padding=(0, 2), stride=(2, 2)),
     dict(n=300, c=120, h=9, w=4, r=5, padding=(2, 2), stride=(2, 2)),
+    dict(n=280, c=64, h=9, w=19, r=5, padding=(2, 2), stride=(2, 2)),  # windows of more than 30 KB: 512 threads
+    dict(n=520, c=64, h=6, w=7, r=5, padding=(2, 1), stride=(1, 1)),
 ])
 @pytest.mark.parametrize("bs,p", [(None, 0.0), (64, 0.5), (192, 0.3)])
 @pytest.mark.parametrize("channels_last", [False, True])
