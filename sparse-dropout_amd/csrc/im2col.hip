@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "mask_source.h"
+#include "reciprocal.h"
 #include "tile_map.h"
 
 namespace sd {
@@ -376,11 +377,15 @@ __global__ __launch_bounds__(256) void im2col_patch_kernel(const uint16_t* __res
 
 // Adjoint: one thread per image element sums the (at most R*S) patch-matrix entries that were
 // gathered from it; fp32 accumulation, one rounding.  Lanes run along w.
+// The instructions of a tap bound it, and the mask's share of them is two divisions by the block size.  m_bs: ceil(2^32 / bs) where
+// multiplying by it is exact for every row counted from the first block of an image and every column (exact_reciprocal), else 0 and
+// they are divided.  With 64-bit divisions a masked fold took 1.7 of one without: 5 x 5 by two, 12 x 64 x 80 x 80, p = 0.5 235 us,
+// 6 x 6 by two, 17 x 64 x 60 x 60 287; so 152 and 183, without a mask 134 and 156 (col2im_tile_kernel: 209 and 223).
 template <typename T>
 __global__ __launch_bounds__(256) void col2im_kernel(const uint16_t* __restrict__ cols, int64_t ld,
                                                      uint16_t* __restrict__ dx, ConvGeom g,
                                                      const uint8_t* mask, int64_t msr, int64_t msc,
-                                                     int bs) {
+                                                     int bs, uint32_t m_bs) {
   const int64_t total = (int64_t)g.n * g.c * g.h * g.w;
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= total) return;
@@ -388,6 +393,14 @@ __global__ __launch_bounds__(256) void col2im_kernel(const uint16_t* __restrict_
   const int hi = (int)((e / g.w) % g.h);
   const int ci = (int)((e / ((int64_t)g.w * g.h)) % g.c);
   const int ni = (int)(e / ((int64_t)g.w * g.h * g.c));
+  const int64_t row0 = (int64_t)ni * g.p * g.q;
+  uint32_t at0 = 0;  // where the image's first row lies in its block
+  if (mask) {
+    const int64_t rb0 = row0 / bs;
+    at0 = (uint32_t)(row0 - rb0 * bs);
+    mask += rb0 * msr;
+  }
+  auto block_of = [&](uint32_t v) { return m_bs ? __umulhi(v, m_bs) : v / (uint32_t)bs; };
   float acc = 0.f;
   for (int rr = 0; rr < g.r; ++rr) {
     const int pu = hi + g.pad_h - rr * g.dil_h;
@@ -399,16 +412,15 @@ __global__ __launch_bounds__(256) void col2im_kernel(const uint16_t* __restrict_
       if (qu < 0 || qu % g.str_w) continue;
       const int qq = qu / g.str_w;
       if (qq >= g.q) continue;
-      const int64_t row = ((int64_t)ni * g.p + pp) * g.q + qq;
+      const int row = pp * g.q + qq;  // of the image
       const int col = (ci * g.r + rr) * g.s + ss;
-      if (mask && mask[(row / bs) * msr + (col / bs) * msc]) continue;
-      acc += T::to_float(cols[row * ld + col]);
+      if (mask && mask[(int64_t)block_of(at0 + (uint32_t)row) * msr + (int64_t)block_of((uint32_t)col) * msc]) continue;
+      acc += T::to_float(cols[(row0 + row) * ld + col]);
     }
   }
   dx[(int64_t)ni * g.xs_n + (int64_t)ci * g.xs_c + (int64_t)hi * g.xs_h + (int64_t)wi * g.xs_w] =
       T::from_float(acc);
 }
-
 // Tiled adjoint for aligned patch matrices.  A workgroup owns one image, a band of `hb` input rows and a
 // group of 8 channels.  Everything of the patch matrix that feeds those outputs — the 8*R*S columns of
 // the channel group, for every output row p that touches the band and every q — is copied to LDS first
@@ -935,12 +947,14 @@ int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64
   const int64_t total = n * c * h * w;
   const int64_t blocks = ceil_div(total, 256);
   SD_REQUIRE(blocks <= 0x7fffffffLL, "col2im: image too large");
+  const int64_t pq = (int64_t)g.p * g.q;
+  const uint32_t m_bs = mask ? exact_reciprocal(bs, std::max(pq + bs, c * r * s)) : 0;
   if (dtype == SD_BF16)
     hipLaunchKernelGGL(col2im_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1);
+                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs);
   else
     hipLaunchKernelGGL(col2im_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1);
+                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs);
   return check_launch("col2im");
 }
 

@@ -785,3 +785,35 @@ def test_conv_draws_of_the_generator_state_are_those_of_its_seed(bs, c, k, r, st
             assert rel_fro(one, to_np(other)) <= 1e-3
     finally:
         ext.manual_seed(torch.initial_seed())
+
+
+# folds that run one thread to an element: channels that do not fill groups of eight, windows by two that do not fit the LDS
+@pytest.mark.parametrize("cfg", [
+    dict(n=3, c=12, h=13, w=9, r=3, s=3, padding=(1, 1), stride=(1, 1), dilation=(1, 1)),
+    dict(n=5, c=5, h=10, w=11, r=4, s=2, padding=(2, 0), stride=(2, 3), dilation=(1, 2)),
+    dict(n=2, c=8, h=7, w=300, r=3, s=3, padding=(1, 1), stride=(2, 2), dilation=(1, 1)),
+    dict(n=2, c=8, h=33, w=32, r=7, s=7, padding=(3, 3), stride=(2, 2), dilation=(1, 1)),
+    dict(n=1, c=16, h=100, w=96, r=5, s=5, padding=(2, 2), stride=(2, 2), dilation=(1, 1)),
+])
+# 65535: a block size whose reciprocal is exact for no image at all
+@pytest.mark.parametrize("bs", [1, 30, 64, 72, 96, 192, 65535])
+@pytest.mark.parametrize("by_columns", [False, True])
+def test_masked_folds_of_single_elements(cfg, bs, by_columns):
+    from flash_dropout.hip import GEMM
+
+    gen = torch.Generator().manual_seed(cfg["w"] + bs)
+    shape, ks = (cfg["n"], cfg["c"], cfg["h"], cfg["w"]), (cfg["r"], cfg["s"])
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], *ks, **_geo(cfg))
+    rows, ncols = cfg["n"] * p_ * q_, cfg["c"] * cfg["r"] * cfg["s"]
+    g = torch.randn(rows, ncols, generator=gen).half()
+    mask = torch.rand(O.mask_shape(rows, ncols, bs), generator=gen) < 0.4
+    keep = torch.from_numpy(O.expand_keep(mask.numpy(), bs, rows, ncols))
+    given = torch.where(keep, g, torch.tensor(float("nan"), dtype=g.dtype))  # dropped blocks are not read
+    mask = mask.cuda()
+    if by_columns:
+        mask = mask.t().contiguous().t()
+    dx = GEMM().col2im(given.cuda(), shape, ks, mask=mask, block_size=bs, **_geo(cfg))
+    kept = torch.where(keep, g, torch.zeros_like(g)).double()
+    ref, size = (torch.from_numpy(O.col2im(t.numpy(), shape, *ks, **_geo(cfg))) for t in (kept, kept.abs()))
+    # one rounding to fp16 of a sum of fewer than 64 terms in fp32
+    assert bool(((dx.cpu().double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 2.0 ** -18 * size + 2.0 ** -25).all())

@@ -344,6 +344,50 @@ def test_tap_windows_and_lds_hold_what_the_kernels_put_there(tmp_path):
     assert proc.returncode == 0, proc.stdout
 
 
+_RECIPROCALS = r"""
+#include <stdio.h>
+#include <initializer_list>
+#include "reciprocal.h"
+
+static long n_exact = 0, n_none = 0;
+static bool holds(int64_t d, int64_t below) {
+  const uint64_t m = sd::exact_reciprocal(d, below);
+  ++(m ? n_exact : n_none);
+  if (m == 0) return true;
+  auto same = [&](int64_t v) { return v < 0 || v >= below || (int64_t)((uint64_t)v * m >> 32) == v / d; };
+  // quotients can only be wrong next to multiples of d, and first at the largest
+  for (int64_t k = 0; k <= 2000; ++k)
+    if (!same(k * d - 1) || !same(k * d) || !same(((below - 1) / d - k) * d - 1) || !same((below - 1) / d * d - k * d)) return false;
+  return same(below - 1);
+}
+int main() {
+  uint64_t x = 12345;
+  auto next = [&](int64_t hi) { x = x * 6364136223846793005ull + 1442695040888963407ull; return 1 + (int64_t)((x >> 20) % (uint64_t)hi); };
+  for (int64_t d = 1; d <= 4096; ++d)
+    for (int64_t below : {(int64_t)1, d + 100000, (int64_t)1 << 24, ((int64_t)1 << 31) + d, (int64_t)1 << 32})
+      if (!holds(d, below)) return printf("%ld below %ld\n", (long)d, (long)below), 1;
+  for (int i = 0; i < 20000; ++i) {
+    const int64_t d = next(1LL << (1 + i % 32)), below = next(1LL << (1 + i % 33));
+    if (!holds(d, below)) return printf("%ld below %ld\n", (long)d, (long)below), 1;
+  }
+  for (int64_t d : {(int64_t)64, (int64_t)128, (int64_t)32768, (int64_t)1 << 30})  // powers of two: for anything
+    if (sd::exact_reciprocal(d, (int64_t)1 << 32) == 0) return 1;
+  if (sd::exact_reciprocal(192, 20 << 20) == 0 || sd::exact_reciprocal(65535, 65540) != 0) return 1;
+  return n_exact < 10000 || n_none < 1000;
+}
+"""
+
+
+def test_reciprocals_divide_exactly_in_the_range_that_they_state(tmp_path):
+    import subprocess
+
+    (tmp_path / "sweep.cpp").write_text(_RECIPROCALS)
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{ROOT / 'sparse-dropout_amd' / 'csrc'}", str(tmp_path / "sweep.cpp"), "-o",
+                    str(tmp_path / "sweep")], check=True)
+    proc = subprocess.run([str(tmp_path / "sweep")], capture_output=True, text=True, timeout=100)
+    assert proc.returncode == 0, proc.stdout
+
+
 @pytest.mark.parametrize("layer,p,taken", [
     ((128, 64, 32, 32, 128, 3), 0.5, True), ((256, 32, 28, 28, 64, 3), 0.25, True), ((64, 1024, 28, 28, 128, 3), 0.75, True),
     ((64, 1024, 14, 14, 1024, 3), 0.75, False),  # 1090 us tap by tap, 649 with the dropped blocks left out
