@@ -465,6 +465,18 @@ int sd_col2im(const void* cols, int64_t cols_ld, void* dx, int64_t dx_stride_n,
               const uint8_t* mask, int64_t mask_stride_r, int64_t mask_stride_c, int64_t block_size,
               int dtype, void* stream);
 
+/* Which kernel sd_col2im folds with, for a patch gradient that starts on a 16-byte boundary and an image of these strides;
+ * block_size: of the mask, 0 without one.  SD_FOLD_NONE: refused geometry.  Nothing is launched. */
+#define SD_FOLD_NONE 0
+#define SD_FOLD_ELEMENTS 1 /* a thread to an element of the image */
+#define SD_FOLD_TILE 2     /* bands of rows staged in LDS, for any strides and dilations */
+#define SD_FOLD_WINDOW 3   /* bands staged with their halo, for strides of 1 or 2 and no dilation */
+#define SD_FOLD_TURN 4     /* pointwise kernels: rows turned to planes */
+int sd_col2im_kernel(int64_t cols_ld, int64_t dx_stride_c, int64_t dx_stride_h, int64_t dx_stride_w,
+                     int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
+                     int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
+                     int64_t dil_h, int64_t dil_w, int64_t block_size);
+
 /* ---------------------------------------------------------------------------------------------
  * Implicit-GEMM forward of the block-dropout convolution: the product sd_im2col + sd_gemm_dsd_lists
  * compute, y[(n*P+p)*Q+q, k] = scale * sum over the kept blocks (row_ptr/col_idx, block_size 64, over the

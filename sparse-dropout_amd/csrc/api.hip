@@ -34,6 +34,8 @@ int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
                   int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, const uint8_t* mask,
                   int64_t msr, int64_t msc, uint64_t seed, uint64_t offset, float p, int64_t mb,
                   int64_t kb, int64_t bs, hipStream_t stream);
+int col2im_kernel_of(int64_t ld, int64_t sc, int64_t sh, int64_t sw, int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
+                     int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, int64_t bs);
 int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
            int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
            int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
@@ -717,6 +719,11 @@ int sd_col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, in
   SD_REQUIRE(dtype == SD_F16 || dtype == SD_BF16, "dtype must be SD_F16 or SD_BF16 (got %d)", dtype);
   return col2im(cols, ld, dx, sn, sc, sh, sw, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h,
                 dil_w, mask, msr, msc, bs, dtype, (hipStream_t)stream);
+}
+
+int sd_col2im_kernel(int64_t ld, int64_t sc, int64_t sh, int64_t sw, int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
+                     int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, int64_t bs) {
+  return col2im_kernel_of(ld, sc, sh, sw, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, bs);
 }
 
 }  // extern "C"

@@ -868,6 +868,112 @@ int im2col_masked(const void* x, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
   return gather(x, sn, sc, sh, sw, cols, ld, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, want, stream);
 }
 
+// ---- which kernel folds, and with what window
+struct FoldPlan {
+  int kernel;  // SD_FOLD_*
+  int64_t wgs;
+  int64_t tiles_c, tiles_p;  // SD_FOLD_TURN
+  int hb;                    // the others but SD_FOLD_ELEMENTS: image rows of a band
+  int64_t bands, lds;
+  int np_max;                // SD_FOLD_TILE
+  int st, rt;                // SD_FOLD_WINDOW: the stride, the kernel size where it is unrolled
+  bool in_runs;
+  int64_t qe, per;
+};
+// aligned: the patch gradient and its rows start on 16-byte boundaries; sc, sh, sw: strides of the image; bs: of the mask, 0 without
+static FoldPlan plan_fold(const ConvGeom& g, bool aligned, int64_t sc, int64_t sh, int64_t sw, int64_t bs) {
+  FoldPlan f{};
+  const int64_t n = g.n, c = g.c, h = g.h, w = g.w;
+  if (g.r == 1 && g.s == 1 && g.str_h == 1 && g.str_w == 1 && g.pad_h == 0 && g.pad_w == 0 && sw == 1 && sh == w && sc >= h * w &&
+      (bs == 0 || (bs % TILE == 0 && bs < (1 << 30)))) {
+    const int64_t pixels = h * w;
+    f.tiles_c = ceil_div(c, TILE);
+    f.tiles_p = ceil_div(pixels, TILE);
+    f.wgs = n * f.tiles_c * f.tiles_p;
+    f.kernel = SD_FOLD_TURN;
+    if (f.wgs <= 0x7fffffffLL) return f;
+  }
+  // 16-byte loads of 8-channel column groups need aligned rows and whole groups
+  if (c % C2I_CG == 0 && aligned && bs % 8 == 0) {
+    const int64_t seg_bytes = (C2I_CG * (int64_t)g.r * g.s + 2) * 2;
+    f.st = g.str_h == g.str_w && g.dil_h == 1 && g.dil_w == 1 && g.str_h <= 2 && g.h < (1 << 28) && g.w < (1 << 28) &&
+                   g.pad_h < (1 << 28) && g.pad_w < (1 << 28) && g.r < (1 << 28) && g.s < (1 << 28) ? g.str_h : 0;
+    f.rt = g.r == g.s && (g.r == 1 || g.r == 3 || g.r == 5) ? g.r : 0;
+    for (int band_rows = 8; band_rows >= 1; band_rows /= 2) {  // the tallest band whose staging fits
+      f.hb = band_rows < g.h ? band_rows : g.h;
+      f.bands = ceil_div(g.h, f.hb);
+      const int64_t groups = n * (c / C2I_CG) * f.bands;
+      if (f.st) {
+        const int64_t pe = f.st == 1 ? f.hb + g.r - 1 : (f.hb + g.r - 2) / 2 + 2;  // at most
+        f.qe = f.st == 1 ? w + g.s - 1 : floor_div<2>(g.w - 1 + g.pad_w) - floor_div<2>(g.pad_w - (g.s - 1)) + 1;
+        f.lds = pe * f.qe * seg_bytes;
+        f.in_runs = f.rt > 1 && sc != 1 && groups >= 2 * C2I_WORKGROUPS;
+        f.per = f.in_runs ? std::min<int64_t>(4, groups / C2I_WORKGROUPS) : 1;
+        f.wgs = n * ceil_div(c / C2I_CG, f.per) * f.bands;
+        f.kernel = SD_FOLD_WINDOW;
+        if (f.lds <= C2I_MAX_LDS && f.wgs <= 0x7fffffffLL && (bs == 0 || (bs <= 32768 && pe * g.q <= 32768))) return f;
+        // (A window by two that fits at no height is left to single elements: col2im_tile_kernel, whose staging still fits some of
+        // these images, takes 1.7 of their time.  3 x 3, 3 x 64 x 288 x 288, p = 0.5 229 us against 184; 5 x 5, 12 x 64 x 80 x 80 209, 152.)
+      } else {
+        f.np_max = (f.hb - 1 + (g.r - 1) * g.dil_h) / g.str_h + 1;
+        f.lds = (int64_t)f.np_max * g.q * seg_bytes;
+        f.wgs = groups;
+        f.kernel = SD_FOLD_TILE;
+        if (f.lds <= C2I_MAX_LDS && f.wgs <= 0x7fffffffLL) return f;
+      }
+    }
+  }
+  f.wgs = ceil_div(n * c * h * w, 256);
+  f.kernel = SD_FOLD_ELEMENTS;
+  return f;
+}
+
+int col2im_kernel_of(int64_t ld, int64_t sc, int64_t sh, int64_t sw, int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s,
+                     int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, int64_t bs) {
+  ConvGeom g;
+  if (make_geom(g, n, c, h, w, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, 0, sc, sh, sw) != SD_OK || bs < 0) return SD_FOLD_NONE;
+  return plan_fold(g, ld % 8 == 0, sc, sh, sw, bs).kernel;
+}
+
+template <typename T>
+static int fold(const FoldPlan& f, const ConvGeom& g, const uint16_t* cols, int64_t ld, uint16_t* dx, const uint8_t* mask, int64_t msr,
+                int64_t msc, int bs, hipStream_t stream) {
+  const dim3 grid((unsigned)f.wgs);
+  if (f.kernel == SD_FOLD_TURN) {
+    hipLaunchKernelGGL(planes_from_rows_kernel, grid, dim3(256), 0, stream, cols, ld, dx, g.xs_n, g.xs_c, g.c, (int)((int64_t)g.h * g.w),
+                       (int)f.tiles_c, (int)f.tiles_p, mask, msr, msc, mask ? bs : TILE);
+    return check_launch("planes_from_rows");
+  }
+  if (f.kernel == SD_FOLD_WINDOW) {
+    const uint32_t m_qe = f.qe <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)f.qe - 1) / (uint64_t)f.qe);
+    const uint32_t m_bs = bs <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)bs - 1) / (uint64_t)bs);
+    auto launch = [&](auto* kernel, int threads) {
+      hipLaunchKernelGGL(kernel, grid, dim3(threads), (size_t)f.lds, stream, cols, ld, dx, g, mask, msr, msc, bs, m_bs, (int)f.bands, f.hb,
+                         (int)f.qe, m_qe, (int)f.per);
+    };
+    const bool wide = f.rt == 5 && f.lds > C2I_FEW_LDS;
+    auto pick = [&](auto step) {
+      constexpr int ST = decltype(step)::value;
+      if (wide) f.in_runs ? launch(&col2im_unit_kernel<T, 5, ST, true, 512>, 512) : launch(&col2im_unit_kernel<T, 5, ST, false, 512>, 512);
+      else if (f.in_runs) f.rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, true, 256>, 256) : launch(&col2im_unit_kernel<T, 5, ST, true, 256>, 256);
+      else f.rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST, false, 256>, 256) : f.rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, false, 256>, 256)
+           : f.rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST, false, 256>, 256) : launch(&col2im_unit_kernel<T, 0, ST, false, 256>, 256);
+    };
+    if (f.st == 1) pick(std::integral_constant<int, 1>{});
+    else pick(std::integral_constant<int, 2>{});
+    return check_launch("col2im_unit");
+  }
+  if (f.kernel == SD_FOLD_TILE) {
+    hipLaunchKernelGGL(col2im_tile_kernel<T>, grid, dim3(256), (size_t)f.lds, stream, cols, ld, dx, g, mask, msr, msc, bs, f.hb, f.np_max,
+                       (int)f.bands);
+    return check_launch("col2im_tile");
+  }
+  SD_REQUIRE(f.wgs <= 0x7fffffffLL, "col2im: image too large");
+  const uint32_t m_bs = mask ? exact_reciprocal(bs, std::max<int64_t>((int64_t)g.p * g.q + bs, (int64_t)g.c * g.r * g.s)) : 0;
+  hipLaunchKernelGGL(col2im_kernel<T>, grid, dim3(256), 0, stream, cols, ld, dx, g, mask, msr, msc, bs, m_bs);
+  return check_launch("col2im");
+}
+
 int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64_t sh, int64_t sw,
            int64_t n, int64_t c, int64_t h, int64_t w, int64_t r, int64_t s, int64_t pad_h,
            int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
@@ -879,83 +985,10 @@ int col2im(const void* cols, int64_t ld, void* dx, int64_t sn, int64_t sc, int64
   SD_REQUIRE(dx && cols, "col2im: null pointer");
   SD_REQUIRE(ld >= c * r * s, "col2im: cols_ld %lld < C*R*S %lld", (long long)ld, (long long)(c * r * s));
   if (mask) SD_REQUIRE(bs > 0, "col2im: block_size must be positive with a mask");
-  if (r == 1 && s == 1 && g.str_h == 1 && g.str_w == 1 && pad_h == 0 && pad_w == 0 && sw == 1 && sh == w && sc >= h * w &&
-      (!mask || (bs % TILE == 0 && bs < (1 << 30)))) {
-    const int64_t pixels = h * w, tiles_c = ceil_div(c, TILE), tiles_p = ceil_div(pixels, TILE), wgs = n * tiles_c * tiles_p;
-    if (wgs <= 0x7fffffffLL) {
-      hipLaunchKernelGGL(planes_from_rows_kernel, dim3((unsigned)wgs), dim3(256), 0, stream, (const uint16_t*)cols, ld, (uint16_t*)dx, sn, sc,
-                         (int)c, (int)pixels, (int)tiles_c, (int)tiles_p, mask, msr, msc, mask ? (int)bs : TILE);
-      return check_launch("planes_from_rows");
-    }
-  }
-  // tiled kernel: 16-byte loads of 8-channel column groups need aligned rows and whole groups
-  if (c % C2I_CG == 0 && ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0 &&
-      (!mask || bs % 8 == 0)) {
-    const int seg_bytes = (C2I_CG * g.r * g.s + 2) * 2;
-    const int st = g.str_h == g.str_w && g.dil_h == 1 && g.dil_w == 1 && g.str_h <= 2 && g.h < (1 << 28) && g.w < (1 << 28) &&
-                           g.pad_h < (1 << 28) && g.pad_w < (1 << 28) && g.r < (1 << 28) && g.s < (1 << 28) ? g.str_h : 0;
-    for (int band_rows = 8; band_rows >= 1; band_rows /= 2) {  // the tallest band whose staging fits
-      const int hb = band_rows < g.h ? band_rows : g.h;
-      if (st) {
-        const int64_t pe = st == 1 ? hb + g.r - 1 : (hb + g.r - 2) / 2 + 2;  // at most
-        const int64_t qe = st == 1 ? g.w + g.s - 1 : floor_div<2>(g.w - 1 + g.pad_w) - floor_div<2>(g.pad_w - (g.s - 1)) + 1;
-        const int64_t lds = pe * qe * seg_bytes;
-        const int64_t bands = ceil_div(g.h, hb);
-        const int64_t groups = n * (c / C2I_CG) * bands;
-        const int rt = g.r == g.s && (g.r == 1 || g.r == 3 || g.r == 5) ? g.r : 0;
-        const bool in_runs = rt > 1 && sc != 1 && groups >= 2 * C2I_WORKGROUPS;
-        const int64_t per = in_runs ? std::min<int64_t>(4, groups / C2I_WORKGROUPS) : 1;
-        const int64_t wgs = n * ceil_div(c / C2I_CG, per) * bands;
-        if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL || (mask && (bs > 32768 || pe * g.q > 32768))) continue;
-        const uint32_t m_qe = qe <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)qe - 1) / (uint64_t)qe);
-        const uint32_t m_bs = !mask || bs <= 1 ? 0u : (uint32_t)(((1ull << 32) + (uint64_t)bs - 1) / (uint64_t)bs);
-        auto launch = [&](auto* kernel, int threads) {
-          hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(threads), (size_t)lds, stream, (const uint16_t*)cols, ld,
-                             (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs, (int)bands, hb, (int)qe, m_qe, (int)per);
-        };
-        const bool wide = rt == 5 && lds > C2I_FEW_LDS;
-        auto pick = [&](auto type, auto step) {
-          using T = decltype(type);
-          constexpr int ST = decltype(step)::value;
-          if (wide) in_runs ? launch(&col2im_unit_kernel<T, 5, ST, true, 512>, 512) : launch(&col2im_unit_kernel<T, 5, ST, false, 512>, 512);
-          else if (in_runs) rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, true, 256>, 256) : launch(&col2im_unit_kernel<T, 5, ST, true, 256>, 256);
-          else rt == 1 ? launch(&col2im_unit_kernel<T, 1, ST, false, 256>, 256) : rt == 3 ? launch(&col2im_unit_kernel<T, 3, ST, false, 256>, 256)
-               : rt == 5 ? launch(&col2im_unit_kernel<T, 5, ST, false, 256>, 256) : launch(&col2im_unit_kernel<T, 0, ST, false, 256>, 256);
-        };
-        const std::integral_constant<int, 1> one;
-        const std::integral_constant<int, 2> two;
-        if (dtype == SD_BF16) st == 1 ? pick(BF16{}, one) : pick(BF16{}, two);
-        else st == 1 ? pick(F16{}, one) : pick(F16{}, two);
-        return check_launch("col2im_unit");
-      }
-      const int np_max = (hb - 1 + (g.r - 1) * g.dil_h) / g.str_h + 1;
-      const int64_t lds = (int64_t)np_max * g.q * seg_bytes;
-      const int64_t bands = ceil_div(g.h, hb);
-      const int64_t wgs = n * (c / C2I_CG) * bands;
-      if (lds > C2I_MAX_LDS || wgs > 0x7fffffffLL) continue;
-      if (dtype == SD_BF16)
-        hipLaunchKernelGGL(col2im_tile_kernel<BF16>, dim3((unsigned)wgs), dim3(256), (size_t)lds, stream,
-                           (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, hb,
-                           np_max, (int)bands);
-      else
-        hipLaunchKernelGGL(col2im_tile_kernel<F16>, dim3((unsigned)wgs), dim3(256), (size_t)lds, stream,
-                           (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, hb,
-                           np_max, (int)bands);
-      return check_launch("col2im_tile");
-    }
-  }
-  const int64_t total = n * c * h * w;
-  const int64_t blocks = ceil_div(total, 256);
-  SD_REQUIRE(blocks <= 0x7fffffffLL, "col2im: image too large");
-  const int64_t pq = (int64_t)g.p * g.q;
-  const uint32_t m_bs = mask ? exact_reciprocal(bs, std::max(pq + bs, c * r * s)) : 0;
-  if (dtype == SD_BF16)
-    hipLaunchKernelGGL(col2im_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs);
-  else
-    hipLaunchKernelGGL(col2im_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       (const uint16_t*)cols, ld, (uint16_t*)dx, g, mask, msr, msc, mask ? (int)bs : 1, m_bs);
-  return check_launch("col2im");
+  const FoldPlan f = plan_fold(g, ld % 8 == 0 && reinterpret_cast<uintptr_t>(cols) % 16 == 0, sc, sh, sw, mask ? bs : 0);
+  const int mask_bs = mask ? (int)bs : 1;
+  return dtype == SD_BF16 ? fold<BF16>(f, g, (const uint16_t*)cols, ld, (uint16_t*)dx, mask, msr, msc, mask_bs, stream)
+                          : fold<F16>(f, g, (const uint16_t*)cols, ld, (uint16_t*)dx, mask, msr, msc, mask_bs, stream);
 }
 
 }  // namespace sd

@@ -707,14 +707,22 @@ bool turned(const Tensor& x, const ConvGeom& g) {
 //  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16 gathered
 //  * both of pointwise kernels whose image's planes are turned: passes of 14 layers that the GPU bounds 0.92 of those without, 1.00 at
 //    worst (32 x 40 x 64 x 64 -> 176, p = 0.5 105 -> 85 us, 215 x 32 x 64 x 64 -> 56, p = 0.6 264 -> 222)
-//  * input gradient, SDD and col2im against the fused kernel: 0.35, 1.03 at most, 0.6 to 0.85 on 42 to 130 MB (187 x 48 x 32 x 32 -> 64
-//    by two 102 -> 85 us a pass); 1.03 to 1.09 where the matrix is one block wide.  Past 256 MB it stays out of memory.
+//  * input gradient, SDD and col2im against the fused kernel, both alone, 800 drawn geometries with kernels of 1 to 7 x 7, dilations and
+//    strides of 1 to 4: 0.25 where the fold stages windows (344, nine of them above 1.05, 3 x 3 but for one, 1.46 at worst), 0.34 where
+//    it goes element by element (311, four, and 1.7), but 0.59 with the tile kernel (144, 33 above 1.1, 5.3 at worst: 128 x 32 x 32 x 32
+//    -> 64, 3 x 3 by two down and one across, 83 -> 127 us a pass), so the fused kernel keeps those.  1.03 to 1.09 where the matrix is one
+//    block wide.  Past 256 MB it stays out of memory.
 bool forward_by_patches(const Tensor& x, const ConvGeom& g) {
   return turned(x, g) || (g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64);
 }
 bool dw_by_patches(const Tensor& x, const ConvGeom& g) { return turned(x, g) || g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
 bool dx_may_fuse(const ConvGeom& g) { return g.k % 64 == 0 && g.k <= 256 && g.qo <= 64 && 64 % g.qo == 0 && g.po * g.qo % 64 == 0; }
-bool dx_by_patches(const ConvGeom& g) { return g.cols() > 64 && g.rows() * g.cols() * 2 <= 256LL << 20; }
+bool dx_by_patches(const ConvGeom& g, bool channels_last, int64_t bs) {
+  if (g.cols() <= 64 || g.rows() * g.cols() * 2 > 256LL << 20) return false;
+  if (pointwise(g) && channels_last) return true;  // written in place
+  const int64_t sc = channels_last ? 1 : g.h * g.w, sw = channels_last ? g.c : 1;
+  return sd_col2im_kernel(g.cols(), sc, g.w * sw, sw, GEOM_X(g), g.r, g.s, GEOM_W(g), bs) != SD_FOLD_TILE;
+}
 
 // The patch matrix of a pointwise kernel: the image itself where it is its own, up to 64 MB the rows of its planes, else undefined.  Turning
 // whole planes costs less than gathering the kept blocks of them, where blocks, rows and columns are looked up, as long as the caches hold
@@ -922,7 +930,7 @@ struct ConvBackward : Node {
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
     // both gradients through the patch matrix: one launch where the pair qualifies, and the fold
-    const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g), dx_through = !fused_dx || dx_by_patches(g) || !dx_may_fuse(g);
+    const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g), dx_through = !fused_dx || (l && dx_by_patches(g, channels_last, l->bs)) || !dx_may_fuse(g);
     if (l && task_should_compute_output(0) && task_should_compute_output(1) && dw_through && dx_through && layer_takes(g, w) && rows_on_16_bytes(dy2)) {
       if (!patches.defined()) patches = im2col(image, g, l);
       if (rows_on_16_bytes(patches)) {
@@ -947,7 +955,7 @@ struct ConvBackward : Node {
     }
     if (task_should_compute_output(0)) {
       Tensor dx;
-      if (fused_dx && !(l && dx_by_patches(g))) dx = conv_dx(dy2, w, g, l, scale, channels_last);
+      if (fused_dx && !(l && dx_by_patches(g, channels_last, l->bs))) dx = conv_dx(dy2, w, g, l, scale, channels_last);
       last_routes[1] = dx.defined() ? kFused : kExplicit;
       if (!dx.defined()) {
         dx = new_image(dy2, g, channels_last);

@@ -118,6 +118,7 @@ SIGNATURES = {
                                  c_void_p, c_int64, c_int64, c_uint64, c_uint64, c_float, c_int64, c_int, c_void_p]),
     "sd_col2im": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64,
                           *([c_int64] * 12), c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
+    "sd_col2im_kernel": (c_int, [c_int64] * 17),
 }
 
 

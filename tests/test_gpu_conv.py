@@ -817,3 +817,39 @@ def test_masked_folds_of_single_elements(cfg, bs, by_columns):
     ref, size = (torch.from_numpy(O.col2im(t.numpy(), shape, *ks, **_geo(cfg))) for t in (kept, kept.abs()))
     # one rounding to fp16 of a sum of fewer than 64 terms in fp32
     assert bool(((dx.cpu().double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 2.0 ** -18 * size + 2.0 ** -25).all())
+
+
+@pytest.mark.parametrize("cfg,dx", [
+    # folds that the tile kernel would do stay with the fused input gradient
+    (dict(n=6, c=32, h=32, w=32, k=64, r=3, s=3, stride=(2, 1), padding=(1, 1), dilation=(1, 1)), "fused"),
+    (dict(n=6, c=32, h=32, w=32, k=64, r=3, s=3, stride=(1, 2), padding=(1, 1), dilation=(1, 1)), "fused"),
+    (dict(n=5, c=32, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(2, 2), dilation=(2, 2)), "fused"),
+    (dict(n=4, c=8, h=32, w=64, k=128, r=4, s=4, stride=(4, 4), padding=(0, 0), dilation=(1, 1)), "fused"),
+    # by windows, element by element
+    (dict(n=6, c=32, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1), dilation=(1, 1)), "explicit"),
+    (dict(n=6, c=12, h=32, w=32, k=64, r=4, s=4, stride=(2, 2), padding=(1, 1), dilation=(1, 1)), "explicit"),
+    (dict(n=3, c=16, h=32, w=32, k=64, r=7, s=7, stride=(2, 2), padding=(3, 3), dilation=(1, 1)), "explicit"),
+])
+@pytest.mark.parametrize("bs", [64, 128])
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_the_fused_input_gradient_is_replaced_where_the_fold_is_fast(cfg, dx, bs, channels_last):
+    import flash_dropout.functional as F
+
+    gen = torch.Generator().manual_seed(cfg["r"])
+    fan_in = cfg["c"] * cfg["r"] * cfg["s"]
+    x = torch.randn(cfg["n"], cfg["c"], cfg["h"], cfg["w"], generator=gen).half()
+    k = (torch.randn(cfg["k"], cfg["c"], cfg["r"], cfg["s"], generator=gen) * fan_in ** -0.5).half()
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], cfg["r"], cfg["s"], **_geo(cfg))
+    mask = cpu_mask(O.mask_shape(cfg["n"] * p_ * q_, fan_in, bs), 0.4, gen)
+    dy = torch.randn(cfg["n"], cfg["k"], p_, q_, generator=gen).half()
+    xg, kg = x.cuda(), k.cuda().requires_grad_()
+    if channels_last:
+        xg = xg.contiguous(memory_format=torch.channels_last)
+    xg.requires_grad_()
+    y = F.blockwise_dropout_conv2d_mask(xg, mask.cuda(), bs, 0.4, kg, **_geo(cfg))
+    y.backward(dy.cuda())
+    assert F.conv_last_routes()["dx"] == dx
+    ry, rdx, rdk = O.conv2d_blockdrop(to_np(x), to_np(k), mask.numpy(), bs, 0.4, dy=to_np(dy), dtype=np.float32, **_geo(cfg))
+    assert max_tile_rel_fro(y, ry) <= REL_FRO_TOL
+    assert max_tile_rel_fro(xg.grad, rdx) <= REL_FRO_TOL
+    assert max_tile_rel_fro(kg.grad, rdk) <= REL_FRO_TOL

@@ -344,6 +344,30 @@ def test_tap_windows_and_lds_hold_what_the_kernels_put_there(tmp_path):
     assert proc.returncode == 0, proc.stdout
 
 
+@pytest.mark.parametrize("c,hw,r,stride,dil,layout,ld_off,bs,kernel", [
+    (64, 32, 3, (1, 1), 1, "planes", 0, 64, "window"), (64, 32, 3, (2, 2), 1, "planes", 0, 0, "window"),
+    (64, 32, 4, (2, 2), 1, "channels last", 0, 64, "window"), (64, 32, 3, (2, 2), 1, "planes", 4, 64, "elements"),
+    (12, 32, 4, (2, 2), 1, "planes", 0, 64, "elements"), (64, 32, 3, (2, 2), 1, "planes", 0, 30, "elements"),
+    # windows by two that fit at no height, and the widest that do
+    (16, 272, 3, (2, 2), 1, "planes", 0, 64, "window"), (16, 320, 3, (2, 2), 1, "planes", 0, 64, "elements"),
+    (16, 72, 5, (2, 2), 1, "planes", 0, 64, "window"), (16, 96, 5, (2, 2), 1, "planes", 0, 64, "elements"),
+    (16, 32, 7, (2, 2), 1, "planes", 0, 64, "elements"), (16, 23, 7, (2, 2), 1, "planes", 0, 64, "window"),
+    # other strides, dilations
+    (32, 32, 3, (2, 1), 1, "planes", 0, 64, "tile"), (32, 32, 3, (1, 2), 1, "channels last", 0, 64, "tile"),
+    (32, 32, 3, (2, 2), 2, "planes", 0, 64, "tile"), (32, 32, 3, (4, 4), 1, "planes", 0, 0, "tile"),
+    (32, 32, 1, (1, 1), 1, "planes", 0, 64, "turn"), (12, 32, 1, (1, 1), 1, "planes", 0, 0, "turn"),
+    (32, 32, 1, (1, 1), 1, "channels last", 0, 64, "window"), (32, 32, 1, (2, 2), 1, "planes", 0, 64, "window"),
+    (32, 2, 5, (1, 1), 2, "planes", 0, 64, None),  # a kernel that does not fit the image
+])
+def test_which_kernel_folds_a_patch_gradient(c, hw, r, stride, dil, layout, ld_off, bs, kernel):
+    from flash_dropout.hip import GEMM
+
+    pad = 0 if kernel is None else dil * (r - 1) // 2 if r % 2 else 0
+    strides = (hw * hw, hw, 1) if layout == "planes" else (1, hw * c, c)
+    got = GEMM().lib.sd_col2im_kernel(c * r * r + ld_off, *strides, 4, c, hw, hw, r, r, pad, pad, *stride, dil, dil, bs)
+    assert (None, "elements", "tile", "window", "turn")[got] == kernel
+
+
 _RECIPROCALS = r"""
 #include <stdio.h>
 #include <initializer_list>
