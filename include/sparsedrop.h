@@ -538,6 +538,11 @@ int sd_conv2d_dx_blocks(const void* dy, int64_t dy_ld, const void* weight, int64
                         int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w,
                         int64_t block_size, float scale, int dtype, void* stream);
 
+/* Whether sd_conv2d_dx_blocks takes this call (without a mask, or with one of blocks of a multiple of 64): 1 or 0, nothing launched. */
+int sd_conv2d_dx_taken(const void* dy, int64_t dy_ld, const void* weight, int64_t weight_ld,
+                       int64_t n, int64_t c, int64_t h, int64_t w, int64_t k_out, int64_t r, int64_t s,
+                       int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w);
+
 int64_t sd_conv2d_dw_workspace_bytes(int64_t n, int64_t c, int64_t k_out, int64_t r, int64_t s, int64_t p, int64_t q);
 int sd_conv2d_dw_lists(const void* x, int64_t x_stride_n, int64_t x_stride_c, int64_t x_stride_h,
                        int64_t x_stride_w, const void* dy, int64_t dy_ld, void* dw, int64_t dw_ld,

@@ -779,7 +779,6 @@ static int conv_input_gradient(const void* dy, int64_t dy_ld, const void* weight
              "strides and dilations must be positive, paddings non-negative");
   SD_REQUIRE(scale == scale, "scale is NaN");
   if (mask != nullptr && (larger ? bs < 64 || bs % 64 != 0 : bs != 64)) return SD_ERR_UNSUPPORTED;
-  if (h > (1 << 20) || w > (1 << 12) || c * r * s > (1 << 16)) return SD_ERR_UNSUPPORTED;
   const int rc = launch_conv_dx(dy, dy_ld, weight, weight_ld, dx, sn, sc, sh, sw, mask, msr, msc, mask ? bs / 64 : 1,
                                 n, c, h, w, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w, scale, dtype, (hipStream_t)stream);
   if (rc == SD_OK) last_kernel = "specialised";
@@ -820,6 +819,13 @@ int sd_conv2d_dx_blocks(const void* dy, int64_t dy_ld, const void* weight, int64
                         void* stream) {
   return conv_input_gradient(dy, dy_ld, weight, weight_ld, dx, sn, sc, sh, sw, mask, msr, msc, n, c, h, w, k_out, r, s, pad_h, pad_w,
                              stride_h, stride_w, dil_h, dil_w, bs, scale, dtype, true, stream);
+}
+
+int sd_conv2d_dx_taken(const void* dy, int64_t dy_ld, const void* weight, int64_t weight_ld, int64_t n, int64_t c, int64_t h, int64_t w,
+                       int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w,
+                       int64_t dil_h, int64_t dil_w) {
+  if (!(n > 0 && c > 0 && h > 0 && w > 0 && k_out > 0 && r > 0 && s > 0 && pad_h >= 0 && pad_w >= 0)) return 0;
+  return conv_dx_taken(dy, dy_ld, weight, weight_ld, n, c, h, w, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w) ? 1 : 0;
 }
 
 int64_t sd_conv2d_dw_workspace_bytes(int64_t n, int64_t c, int64_t k_out, int64_t r, int64_t s, int64_t p, int64_t q) {

@@ -417,6 +417,9 @@ int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, v
                    int64_t h, int64_t wd, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
                    int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype,
                    hipStream_t stream);
+// whether it does: a question to the host alone
+bool conv_dx_taken(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, int64_t n, int64_t c, int64_t h, int64_t wd, int64_t k_out,
+                   int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w);
 // which workgroup shape the DSD kernel runs in: chosen from the shape, or forced (tuning and tests);
 // returns the previous policy, -1 for an unknown one
 enum { kTileAuto = 0, kTileBig = 1, kTileMid = 2 };

@@ -290,7 +290,6 @@ __global__ __launch_bounds__(THREADS) void conv_dx_kernel(DxArgs g) {
 template <typename T, int RT, int ST, int KS_MAX>
 int launch_t(const DxArgs& g, int64_t wgs, hipStream_t stream) {
   const int smem = DxLds<KS_MAX>::OFF_ACC + g.ring_n * g.HB * g.W * 4;
-  if (smem > DxLds<KS_MAX>::DYN_LDS_MAX) return SD_ERR_UNSUPPORTED;  // the ring of open channel sums does not fit
   static std::atomic<bool> configured[16] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16)
@@ -306,22 +305,19 @@ int launch_t(const DxArgs& g, int64_t wgs, hipStream_t stream) {
   return check_launch("conv_dx_kernel");
 }
 
-}  // namespace
-
-// Returns SD_ERR_UNSUPPORTED (no message, nothing launched) for geometries the kernel does not take.
-int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, void* dx, int64_t sn, int64_t sc,
-                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t split, int64_t n, int64_t c,
-                   int64_t h, int64_t wd, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
-                   int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype,
-                   hipStream_t stream) {
-  if (stride_h < 1 || stride_w < 1 || dil_h < 1 || dil_w < 1 || stride_h > 8 || stride_w > 8 || dil_h > 8 || dil_w > 8)
-    return SD_ERR_UNSUPPORTED;
+// Whether the kernel takes these arguments, and what follows from the sizes: everything of g but the pointers, the image's strides, the mask
+// and the scale.
+bool plan_conv_dx(DxArgs& g, const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, int64_t n, int64_t c, int64_t h, int64_t wd,
+                  int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h,
+                  int64_t dil_w) {
+  if (h > (1 << 20) || wd > (1 << 12) || c * r * s > (1 << 16)) return false;
+  if (stride_h < 1 || stride_w < 1 || dil_h < 1 || dil_w < 1 || stride_h > 8 || stride_w > 8 || dil_h > 8 || dil_w > 8) return false;
   const int64_t P = (h + 2 * pad_h - dil_h * (r - 1) - 1) / stride_h + 1;
   const int64_t Q = (wd + 2 * pad_w - dil_w * (s - 1) - 1) / stride_w + 1;
-  if (P <= 0 || Q <= 0 || Q > BS || BS % Q != 0 || (P * Q) % BS != 0) return SD_ERR_UNSUPPORTED;
-  if (k_out % BS != 0 || k_out > BS * KS_LIMIT) return SD_ERR_UNSUPPORTED;
+  if (P <= 0 || Q <= 0 || Q > BS || BS % Q != 0 || (P * Q) % BS != 0) return false;
+  if (k_out % BS != 0 || k_out > BS * KS_LIMIT) return false;
   const int64_t K = c * r * s, Kb = (K + BS - 1) / BS;
-  if (Kb > 64 || K % 8 != 0 || r * s > BS) return SD_ERR_UNSUPPORTED;  // keep flags are one 64-bit word per row block
+  if (Kb > 64 || K % 8 != 0 || r * s > BS) return false;  // keep flags are one 64-bit word per row block
   const int64_t rpb = BS / Q;
   // a channel's columns span at most two blocks; the ring holds every channel a block column can touch
   const int64_t ring_n = (BS + r * s - 1) / (r * s) + 2;
@@ -333,29 +329,14 @@ int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, v
   auto rows_fit = [&](int64_t hb) { return (rpb - 1) + (hb - 1 + (r - 1) * dil_h) / stride_h + 1 <= NB * rpb; };
   int64_t HB = 2 * rpb * stride_h;
   while (HB > 1 && (HB * wd > THREADS || ring_n * HB * wd * 4 > ring_max || !rows_fit(HB))) HB /= 2;
-  if (!rows_fit(HB)) return SD_ERR_UNSUPPORTED;
+  if (!rows_fit(HB)) return false;
   const int64_t hw_n = HB * wd;
-  if (hw_n > THREADS) return SD_ERR_UNSUPPORTED;
+  if (hw_n > THREADS || ring_n * hw_n * 4 > ring_max) return false;
   const bool align_ok = reinterpret_cast<uintptr_t>(dy) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
                         dy_ld % 8 == 0 && w_ld % 8 == 0 && dy_ld >= k_out && w_ld >= K;
-  if (!align_ok) return SD_ERR_UNSUPPORTED;
+  if (!align_ok) return false;
   const int64_t bands = (h + HB - 1) / HB;
-  const int64_t wgs = n * bands;
-  if (wgs > 0x7fffffffLL || n * (P * Q / BS) > 0x7fffffffLL) return SD_ERR_UNSUPPORTED;
-  DxArgs g;
-  g.dy = static_cast<const uint16_t*>(dy);
-  g.dy_ld = dy_ld;
-  g.w = static_cast<const uint16_t*>(w);
-  g.w_ld = w_ld;
-  g.dx = static_cast<uint16_t*>(dx);
-  g.sn = sn;
-  g.sc = sc;
-  g.sh = sh;
-  g.sw = sw;
-  g.mask = mask;
-  g.split = (int)split;
-  g.msr = msr;
-  g.msc = msc;
+  if (n * bands > 0x7fffffffLL || n * (P * Q / BS) > 0x7fffffffLL) return false;
   g.C = (int)c;
   g.H = (int)h;
   g.W = (int)wd;
@@ -377,8 +358,42 @@ int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, v
   g.K = (int)K;
   g.Kb = (int)Kb;
   g.KS = (int)(k_out / BS);
-  g.scale = scale;
   g.ring_n = (int)ring_n;
+  return true;
+}
+
+}  // namespace
+
+bool conv_dx_taken(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, int64_t n, int64_t c, int64_t h, int64_t wd, int64_t k_out,
+                   int64_t r, int64_t s, int64_t pad_h, int64_t pad_w, int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w) {
+  DxArgs g;
+  return plan_conv_dx(g, dy, dy_ld, w, w_ld, n, c, h, wd, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w);
+}
+
+// Returns SD_ERR_UNSUPPORTED (no message, nothing launched) for geometries the kernel does not take.
+int launch_conv_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, void* dx, int64_t sn, int64_t sc,
+                   int64_t sh, int64_t sw, const uint8_t* mask, int64_t msr, int64_t msc, int64_t split, int64_t n, int64_t c,
+                   int64_t h, int64_t wd, int64_t k_out, int64_t r, int64_t s, int64_t pad_h, int64_t pad_w,
+                   int64_t stride_h, int64_t stride_w, int64_t dil_h, int64_t dil_w, float scale, int dtype,
+                   hipStream_t stream) {
+  DxArgs g;
+  if (!plan_conv_dx(g, dy, dy_ld, w, w_ld, n, c, h, wd, k_out, r, s, pad_h, pad_w, stride_h, stride_w, dil_h, dil_w))
+    return SD_ERR_UNSUPPORTED;
+  const int64_t wgs = n * g.bands;
+  g.dy = static_cast<const uint16_t*>(dy);
+  g.dy_ld = dy_ld;
+  g.w = static_cast<const uint16_t*>(w);
+  g.w_ld = w_ld;
+  g.dx = static_cast<uint16_t*>(dx);
+  g.sn = sn;
+  g.sc = sc;
+  g.sh = sh;
+  g.sw = sw;
+  g.mask = mask;
+  g.split = (int)split;
+  g.msr = msr;
+  g.msc = msc;
+  g.scale = scale;
   const bool bf = dtype == SD_BF16, wide = k_out > 2 * BS;
   if (r == 3 && s == 3) {
     if (wide) return bf ? launch_t<BF16, 3, 3, 4>(g, wgs, stream) : launch_t<F16, 3, 3, 4>(g, wgs, stream);

@@ -716,7 +716,9 @@ bool forward_by_patches(const Tensor& x, const ConvGeom& g) {
   return turned(x, g) || (g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64);
 }
 bool dw_by_patches(const Tensor& x, const ConvGeom& g) { return turned(x, g) || g.rows() < (g.r * g.s > 1 ? 8192 : 16384); }
-bool dx_may_fuse(const ConvGeom& g) { return g.k % 64 == 0 && g.k <= 256 && g.qo <= 64 && 64 % g.qo == 0 && g.po * g.qo % 64 == 0; }
+bool dx_fuses(const Tensor& dy2, const Tensor& w2, const ConvGeom& g) {
+  return sd_conv2d_dx_taken(dy2.data_ptr(), dy2.stride(0), w2.data_ptr(), w2.stride(0), GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
+}
 bool dx_by_patches(const ConvGeom& g, bool channels_last, int64_t bs) {
   if (g.cols() <= 64 || g.rows() * g.cols() * 2 > 256LL << 20) return false;
   if (pointwise(g) && channels_last) return true;  // written in place
@@ -930,8 +932,9 @@ struct ConvBackward : Node {
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
     // both gradients through the patch matrix: one launch where the pair qualifies, and the fold
-    const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g), dx_through = !fused_dx || (l && dx_by_patches(g, channels_last, l->bs)) || !dx_may_fuse(g);
-    if (l && task_should_compute_output(0) && task_should_compute_output(1) && dw_through && dx_through && layer_takes(g, w) && rows_on_16_bytes(dy2)) {
+    const bool fused = fused_dx && !(l && dx_by_patches(g, channels_last, l->bs)) && dx_fuses(dy2, w, g);
+    const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g);
+    if (l && task_should_compute_output(0) && task_should_compute_output(1) && dw_through && !fused && layer_takes(g, w) && rows_on_16_bytes(dy2)) {
       if (!patches.defined()) patches = im2col(image, g, l);
       if (rows_on_16_bytes(patches)) {
         // a pointwise kernel's patch gradient is that of a channels-last image: the product writes it in place, zeros included
@@ -955,7 +958,7 @@ struct ConvBackward : Node {
     }
     if (task_should_compute_output(0)) {
       Tensor dx;
-      if (fused_dx && !(l && dx_by_patches(g, channels_last, l->bs))) dx = conv_dx(dy2, w, g, l, scale, channels_last);
+      if (fused) dx = conv_dx(dy2, w, g, l, scale, channels_last);
       last_routes[1] = dx.defined() ? kFused : kExplicit;
       if (!dx.defined()) {
         dx = new_image(dy2, g, channels_last);

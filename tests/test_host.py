@@ -368,6 +368,25 @@ def test_which_kernel_folds_a_patch_gradient(c, hw, r, stride, dil, layout, ld_o
     assert (None, "elements", "tile", "window", "turn")[got] == kernel
 
 
+@pytest.mark.parametrize("n,c,hw,k,r,stride,dil,taken", [
+    (4, 64, 32, 128, 3, 1, 1, 1), (3, 8, 32, 64, 5, 1, 1, 1), (2, 8, 32, 64, 3, 2, 1, 1), (2, 24, 32, 64, 3, 1, 2, 1),
+    (2, 16, 32, 256, 1, 1, 1, 1), (2, 16, 64, 256, 1, 2, 1, 1),
+    (2, 16, 64, 64, 1, 2, 1, 0),    # the open sums of 66 channels over 64-wide rows, beside half a CU's LDS
+    (2, 16, 32, 64, 8, 2, 1, 1), (2, 16, 32, 64, 9, 2, 1, 0),   # 81 taps
+    (2, 512, 32, 64, 3, 1, 1, 0),   # 72 block columns
+    (2, 12, 32, 64, 3, 1, 1, 0),    # 108 columns
+    (2, 16, 64, 64, 3, 1, 8, 0),    # taps of more output rows than the waves hold
+    (2, 16, 32, 96, 3, 1, 1, 0), (2, 16, 30, 64, 3, 1, 1, 0), (2, 16, 32, 64, 3, 9, 1, 0), (0, 16, 32, 64, 3, 1, 1, 0),
+])
+def test_which_convolutions_have_their_input_gradient_fused(n, c, hw, k, r, stride, dil, taken):
+    from flash_dropout.hip import GEMM
+
+    lib, cols, pad = GEMM().lib, c * r * r, dil * (r - 1) // 2
+    ask = lambda dy, dy_ld, w, w_ld: lib.sd_conv2d_dx_taken(dy, dy_ld, w, w_ld, n, c, hw, hw, k, r, r, pad, pad, stride, stride, dil, dil)
+    assert ask(256, k, 512, cols) == taken
+    assert ask(264, k, 512, cols) == ask(256, k, 520, cols) == ask(256, k + 4, 512, cols) == ask(256, k, 512, cols + 4) == 0
+
+
 _RECIPROCALS = r"""
 #include <stdio.h>
 #include <initializer_list>
