@@ -22,6 +22,7 @@
 #include <atomic>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "sparsedrop.h"
@@ -307,27 +308,28 @@ void check_p(double p) { TORCH_CHECK_VALUE(p >= 0.0 && p < 1.0, "p must be in [0
 
 // ---- the products of one layer ----------------------------------------------------------------------------------------
 // Y = act(s (keep . X) W^T) with mask and lists, one library call; pre: receives the pre-activation when wanted.
+// drawn: the lists are allocated and hold a drawn mask, and `draw` isn't asked.
 Tensor layer_forward(Tensor x, Tensor w, int64_t bs, double p, const Draw& draw, int act, bool want_pre, Lists& lists,
-                     Tensor* pre) {
+                     Tensor* pre, bool drawn = false) {
   check_pair(x, w);
   check_p(p);
   lists.shape(x.size(0), x.size(1), bs);
   if (bs % 32 == 0) pad_reduction(x, w);  // (a width rounded up to 8 has the same block grid)
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  lists.allocate(x, draw.mask);
+  if (!drawn) lists.allocate(x, draw.mask);
   Tensor y = new_matrix(x, M, N);
   if (want_pre && act != SD_ACT_NONE) *pre = new_matrix(x, M, N);
   const int64_t g = bs % 32 == 0 ? 64 : bs;
   Scratch ws(x, sd_splitk_workspace_bytes(M, N, K, g, 1));
-  const MaskArg given = draw.mask ? lists.mask() : MaskArg();
+  const MaskArg given = draw.mask || drawn ? lists.mask() : MaskArg();
   Mat pm;
   if (pre && pre->defined()) pm = Mat(*pre);
   const Mat xm(x), wm(w), ym(y);
   c10::DeviceGuard guard(x.device());
-  check(sd_dropout_matmul_forward_act(MAT(xm), MAT(wm), MAT(ym), given.ptr, given.sr, given.sc, draw.state_ptr(),
-                                      draw.seed.value_or(0), 0, p, lists.drawn(), lists.row_ptr(), lists.col_idx(),
-                                      lists.col_ptr(), lists.row_idx(), M, N, K, bs, dtype_of(x), act, MAT(pm), ws.ptr,
-                                      ws.bytes, stream_of(x)),
+  check(sd_dropout_matmul_forward_act(MAT(xm), MAT(wm), MAT(ym), given.ptr, given.sr, given.sc,
+                                      drawn ? nullptr : draw.state_ptr(), draw.seed.value_or(0), 0, p,
+                                      drawn ? nullptr : lists.drawn(), lists.row_ptr(), lists.col_idx(), lists.col_ptr(),
+                                      lists.row_idx(), M, N, K, bs, dtype_of(x), act, MAT(pm), ws.ptr, ws.bytes, stream_of(x)),
         "sd_dropout_matmul_forward_act");
   return y;
 }
@@ -693,6 +695,29 @@ Tensor rows_of_planes(const Tensor& t) {
         "sd_rows_from_planes");
   return rows;
 }
+// The same of two tensors in one launch
+std::pair<Tensor, Tensor> rows_of_planes(const Tensor& a, const Tensor& b) {
+  Tensor out[2];
+  const void* planes[2];
+  void* rows[2];
+  int64_t sn[2], sc[2], n[2], c[2], pixels[2];
+  for (int i = 0; i < 2; ++i) {
+    const Tensor& t = i ? b : a;
+    n[i] = t.size(0);
+    c[i] = t.size(1);
+    pixels[i] = t.size(2) * t.size(3);
+    out[i] = new_matrix(t, n[i] * pixels[i], c[i]);
+    planes[i] = t.data_ptr();
+    rows[i] = out[i].data_ptr();
+    sn[i] = t.stride(0);
+    sc[i] = t.stride(1);
+  }
+  c10::DeviceGuard guard(a.device());
+  check(sd_conv2d_taps_prepare(2, planes, sn, sc, rows, n, c, pixels, nullptr, 0, 0, 0, 1, 1, 0, nullptr, nullptr, 0, 0, nullptr, 0, 0, 0.f,
+                               dtype_of(a), stream_of(a)),
+        "sd_conv2d_taps_prepare");
+  return {out[0], out[1]};
+}
 // Whether that is the cheapest patch matrix of a pointwise kernel (own_patches)
 bool turned(const Tensor& x, const ConvGeom& g) {
   return pointwise(g) && g.n > 0 && whole_planes(x) && g.rows() * g.c * 2 <= 64LL << 20;
@@ -749,14 +774,28 @@ Tensor im2col(const Tensor& x, const ConvGeom& g, const Lists* l) {
 
 // Forward of a masked convolution through its patch matrix in two launches where there were three: the gather asks the mask's source
 // (a stored mask or a seed), the product makes the lists.  cols: the patch matrix.
+// A draw from the generator's state is made by one launch and read from what that stored: between two launches that each make it another
+// stream may move the state on, and the product would read blocks that were not gathered.  Turning planes asks for no mask, so
+// the launch that turns them makes the draw (31 x 16 x 16 x 16 -> 80, p = 0.75: the kernels of a pass 33 us with a launch of its own, 31 so).
 Tensor patches_forward(const Tensor& x, const Tensor& w2, const ConvGeom& g, int64_t bs, double p, Draw draw, Lists& l, Tensor* cols) {
   check_conv_mask(g, bs, p, draw, l);
   if (draw.mask) draw.mask = check_mask(*draw.mask, l.mb, l.kb, x);
+  c10::DeviceGuard guard(x.device());
+  if (uint64_t* st = draw.state_ptr()) {  // (turned(x, g): the caller's business)
+    l.allocate(x, OptTensor());
+    *cols = new_matrix(x, g.rows(), g.c);
+    const void* planes = x.data_ptr();
+    void* rows = cols->data_ptr();
+    const int64_t sn = x.stride(0), sc = x.stride(1), pixels = g.h * g.w;
+    check(sd_conv2d_taps_prepare(1, &planes, &sn, &sc, &rows, &g.n, &g.c, &pixels, nullptr, 0, g.c, g.k, 1, 1, 0, nullptr,
+                                 l.drawn(), l.mb, l.kb, st, 0, 0, (float)p, dtype_of(x), stream_of(x)),
+          "sd_conv2d_taps_prepare");
+    return layer_forward(*cols, w2, bs, p, draw, SD_ACT_NONE, false, l, nullptr, true);
+  }
   *cols = own_patches(x, g);
   if (!cols->defined()) {
     *cols = new_matrix(x, g.rows(), g.cols());
     const MaskArg m = draw.mask ? MaskArg(*draw.mask) : MaskArg();
-    c10::DeviceGuard guard(x.device());
     check(sd_im2col_masked(x.data_ptr(), STRIDES4(x), cols->data_ptr(), cols->stride(0), GEOM_X(g), g.r, g.s, GEOM_W(g), m.ptr, m.sr,
                            m.sc, draw.seed.value_or(0), 0, (float)p, bs, dtype_of(x), stream_of(x)),
           "sd_im2col_masked");
@@ -928,9 +967,16 @@ struct ConvBackward : Node {
     const Lists lists = saved.get();
     Tensor patches = cols.matrix();
     if (taps) return apply_taps(grads[0], w, image, patches, lists.buf.defined() ? &lists : nullptr);
-    const Tensor dy2 = grads[0].defined() ? rows_gradient(grads[0], g, w) : at::zeros({g.rows(), g.k}, w.options());
     const Lists* l = lists.buf.defined() ? &lists : nullptr;
     const float scale = (float)(1.0 / (1.0 - p));
+    Tensor dy2;
+    // the image of a pointwise kernel is turned with the output gradient (31 x 16 x 16 x 16 -> 80, p = 0.75: the kernels of a pass 31 us
+    // with a launch for either, 29 so; 60 x 64 x 64 x 64 -> 64, p = 0.1 148 and 143)
+    if (l && task_should_compute_output(1) && !patches.defined() && grads[0].defined() && grads[0].scalar_type() == w.scalar_type() &&
+        whole_planes(grads[0]) && turned(image, g))
+      std::tie(dy2, patches) = rows_of_planes(grads[0], image);
+    else
+      dy2 = grads[0].defined() ? rows_gradient(grads[0], g, w) : at::zeros({g.rows(), g.k}, w.options());
     // both gradients through the patch matrix: one launch where the pair qualifies, and the fold
     const bool fused = fused_dx && !(l && dx_by_patches(g, channels_last, l->bs)) && dx_fuses(dy2, w, g);
     const bool dw_through = pixels || patches.defined() || dw_by_patches(image, g);
@@ -1057,7 +1103,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   g.qo = out_size(g.w, g.pad[1], g.dil[1], g.s, g.stride[1]);
   TORCH_CHECK_VALUE(g.po > 0 && g.qo > 0, "kernel does not fit the padded image");
   Lists lists;
-  Tensor y, y2, cols;
+  Tensor y, y2, cols, w2;
   const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;
   const bool taps = implicit_forward && fused_dx && sd_conv2d_taps_taken_blocks(GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), bs ? p : 0.0, bs);
   const bool record = records(std::array<Tensor, 2>{x, kernel});
@@ -1086,13 +1132,12 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     const Lists* l = bs ? &lists : nullptr;
     bool done = false;
     c10::DeviceGuard device(x.device());
-    const Tensor w2 = kernel.detach().view({g.k, g.cols()});
+    w2 = kernel.detach().view({g.k, g.cols()});
     const bool takes_implicit = implicit_forward && sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(),
                                                                               GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
     const Draw draw{mask, seed, state};
-    // A draw from the generator's state is made by one launch and read from what that stored: between two launches that each
-    // make it another stream may move the state on, and the product would read blocks that were not gathered.
-    const bool implicit = takes_implicit && !(bs && forward_by_patches(x, g)), layer = bs && layer_takes(g, w2) && !draw.state_ptr();
+    const bool implicit = takes_implicit && !(bs && forward_by_patches(x, g));
+    const bool layer = bs && layer_takes(g, w2) && (!draw.state_ptr() || turned(x, g));  // (see patches_forward)
     if (implicit || !layer) {
       if (bs) conv_lists(x, g, bs, p, draw, lists);
       y2 = new_matrix(x, g.rows(), g.k);
@@ -1135,7 +1180,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     node->pixels = cols.defined() && cols.is_alias_of(x);
     if (cols.defined() && !node->pixels) node->cols.keep(cols);
     else if (keeps_input) node->x.keep(x);
-    node->w2.keep(kernel.detach().view({g.k, g.cols()}));
+    node->w2.keep(w2.defined() ? w2 : kernel.detach().view({g.k, g.cols()}));
     if (bs) node->saved.keep(std::move(lists), mask.value_or(Tensor()));
     node->g = g;
     node->p = bs ? p : 0.0;

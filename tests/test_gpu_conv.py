@@ -853,3 +853,48 @@ def test_the_fused_input_gradient_is_replaced_where_the_fold_is_fast(cfg, dx, bs
     assert max_tile_rel_fro(y, ry) <= REL_FRO_TOL
     assert max_tile_rel_fro(xg.grad, rdx) <= REL_FRO_TOL
     assert max_tile_rel_fro(kg.grad, rdk) <= REL_FRO_TOL
+
+
+@pytest.mark.parametrize("bs", [64, 128, 192])
+@pytest.mark.parametrize("n,c,h,w,k", [(7, 72, 14, 14, 64), (1, 8, 3, 2, 8), (9, 200, 15, 13, 40), (20, 20, 16, 16, 24)])
+def test_pointwise_draws_of_the_generator_state_are_those_of_its_seed(bs, n, c, h, w, k):
+    """The launch that turns the planes draws the mask (for widths that are no multiple of 8 the lists' launch does): the same lists,
+    so the same bits, and the state moves on by one draw a call, captured ones too."""
+    import flash_dropout.functional as F
+    from flash_dropout.hip import GEMM
+
+    ext = GEMM()
+    gen = torch.Generator().manual_seed(c)
+    x = torch.randn(n, c, h, w, generator=gen).half().cuda().requires_grad_()
+    wt = (torch.randn(k, c, 1, 1, generator=gen) * c ** -0.5).half().cuda().requires_grad_()
+    dy = torch.randn(n, k, h, w, generator=gen).half().cuda()
+    passed = lambda y: (y, *torch.autograd.grad(y, (x, wt), dy))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    try:
+        with torch.cuda.stream(stream):
+            ext.manual_seed(77)
+            drawn = passed(F.blockwise_dropout_conv2d(x, wt, bs, 0.4))
+            assert F.conv_last_routes()["forward"] == "explicit"
+            assert ext.rng_state(x.device).tolist() == [77, 1, 0, 0]
+            pinned = passed(F.blockwise_dropout_conv2d(x, wt, bs, 0.4, seed=77))
+            if c % 8 == 0:
+                assert all(torch.equal(a, b) for a, b in zip(drawn, pinned))
+            else:  # sums in fp32 in another order, one rounding to fp16 of a product and, for dx, one of the fold
+                assert all(rel_fro(a, to_np(b)) <= 1e-3 for a, b in zip(drawn, pinned))
+            y = F.blockwise_dropout_conv2d(x.detach(), wt, bs, 0.4, seed=77)
+            assert rel_fro(torch.autograd.grad(y, wt, dy)[0], to_np(pinned[2])) <= 1e-3  # on its own, as above
+            with torch.no_grad():
+                want = [F.blockwise_dropout_conv2d(x, wt, bs, 0.4) for _ in range(3)]
+                ext.manual_seed(77)
+                F.blockwise_dropout_conv2d(x, wt, bs, 0.4)
+                stream.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=stream):
+                    y = F.blockwise_dropout_conv2d(x, wt, bs, 0.4)
+                for draw in want:
+                    graph.replay()
+                    assert torch.equal(y, draw)
+    finally:
+        torch.cuda.synchronize()
+        ext.manual_seed(torch.initial_seed())
