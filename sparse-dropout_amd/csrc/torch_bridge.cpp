@@ -725,18 +725,23 @@ bool turned(const Tensor& x, const ConvGeom& g) {
 
 // Which products of a masked convolution that the library takes without a patch matrix go through one all the same (the image is
 // what is kept then too, and gathered once more for the kernel's gradient).  Measured on 298 drawn layers of 24 to 950 thousand
-// rows, 32 fused input gradients among them; times through the matrix against those without, geometric means:
+// rows; times through the matrix against those without, geometric means:
 //  * forward: a workgroup takes 256 rows x 128 outputs and builds its tiles step by step; fewer than 64 of them 0.67 (9 x 96 x 8 x 8 ->
 //    192, 5 x 5, p = 0.5, six of them: 45 us a pass for 306), 64 to 128 1.02, more 1.3; pointwise kernels, a step each, 1.04 to 1.3
 //    gathered
 //  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16 gathered
 //  * both of pointwise kernels whose image's planes are turned: passes of 14 layers that the GPU bounds 0.92 of those without, 1.00 at
 //    worst (32 x 40 x 64 x 64 -> 176, p = 0.5 105 -> 85 us, 215 x 32 x 64 x 64 -> 56, p = 0.6 264 -> 222)
+// Drawn from the generator's state the gather waits for a launch that draws (but for planes that are turned): passes of 180 layers of 4 to
+// 256 images, kernels of 1 to 5 x 5, 0.61 of those without where the same seeds take 0.57, 1.001 at worst.  The matrices of rows this few
+// come to 0.8 GB at most (63 x 512 x 16 x 16 -> 64, 7 x 7, p = 0.5 1590 us a pass for 1910).
 //  * input gradient, SDD and col2im against the fused kernel, both alone, 800 drawn geometries with kernels of 1 to 7 x 7, dilations and
-//    strides of 1 to 4: 0.25 where the fold stages windows (344, nine of them above 1.05, 3 x 3 but for one, 1.46 at worst), 0.34 where
-//    it goes element by element (311, four, and 1.7), but 0.59 with the tile kernel (144, 33 above 1.1, 5.3 at worst: 128 x 32 x 32 x 32
-//    -> 64, 3 x 3 by two down and one across, 83 -> 127 us a pass), so the fused kernel keeps those.  1.03 to 1.09 where the matrix is one
-//    block wide.  Past 256 MB it stays out of memory.
+//    strides of 1 to 4: 0.25 where the fold stages windows (344, nine of them above 1.05, 3 x 3 but for one, 1.46 at worst), but 0.59 with
+//    the tile kernel (144, 33 above 1.1, 5.3 at worst: 128 x 32 x 32 x 32 -> 64, 3 x 3 by two down and one across, 83 -> 127 us a pass),
+//    so the fused kernel keeps those.  Element by element 0.34 (311), 1.06 at worst but for unit strides with 64 outputs, where the fused
+//    kernel's reduction is short and the fold's sums are not: of more than 8 million terms three in seven took longer, 1.7 at worst
+//    (145 x 10 x 17 x 33 -> 64, 4 x 4, p = 0.25 112 -> 156 us a pass), of fewer 0.73 at worst.  1.03 to 1.09 where the matrix is one block
+//    wide.  Past 256 MB it stays out of memory.
 bool forward_by_patches(const Tensor& x, const ConvGeom& g) {
   return turned(x, g) || (g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64);
 }
@@ -748,7 +753,9 @@ bool dx_by_patches(const ConvGeom& g, bool channels_last, int64_t bs) {
   if (g.cols() <= 64 || g.rows() * g.cols() * 2 > 256LL << 20) return false;
   if (pointwise(g) && channels_last) return true;  // written in place
   const int64_t sc = channels_last ? 1 : g.h * g.w, sw = channels_last ? g.c : 1;
-  return sd_col2im_kernel(g.cols(), sc, g.w * sw, sw, GEOM_X(g), g.r, g.s, GEOM_W(g), bs) != SD_FOLD_TILE;
+  const int fold = sd_col2im_kernel(g.cols(), sc, g.w * sw, sw, GEOM_X(g), g.r, g.s, GEOM_W(g), bs);
+  if (fold == SD_FOLD_ELEMENTS && g.stride[0] == 1 && g.stride[1] == 1 && g.k <= 64) return g.n * g.h * g.w * g.cols() <= 8 << 20;
+  return fold != SD_FOLD_TILE;
 }
 
 // The patch matrix of a pointwise kernel: the image itself where it is its own, up to 64 MB the rows of its planes, else undefined.  Turning

@@ -825,6 +825,10 @@ def test_masked_folds_of_single_elements(cfg, bs, by_columns):
     (dict(n=6, c=32, h=32, w=32, k=64, r=3, s=3, stride=(1, 2), padding=(1, 1), dilation=(1, 1)), "fused"),
     (dict(n=5, c=32, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(2, 2), dilation=(2, 2)), "fused"),
     (dict(n=4, c=8, h=32, w=64, k=128, r=4, s=4, stride=(4, 4), padding=(0, 0), dilation=(1, 1)), "fused"),
+    # and long folds of single elements at unit strides, where there are few outputs
+    (dict(n=100, c=10, h=17, w=33, k=64, r=4, s=4, stride=(1, 1), padding=(1, 1), dilation=(1, 1)), "fused"),
+    (dict(n=60, c=10, h=17, w=33, k=64, r=4, s=4, stride=(1, 1), padding=(1, 1), dilation=(1, 1)), "explicit"),
+    (dict(n=100, c=10, h=17, w=33, k=128, r=4, s=4, stride=(1, 1), padding=(1, 1), dilation=(1, 1)), "explicit"),
     # by windows, element by element
     (dict(n=6, c=32, h=32, w=32, k=64, r=3, s=3, stride=(2, 2), padding=(1, 1), dilation=(1, 1)), "explicit"),
     (dict(n=6, c=12, h=32, w=32, k=64, r=4, s=4, stride=(2, 2), padding=(1, 1), dilation=(1, 1)), "explicit"),
