@@ -902,3 +902,39 @@ def test_pointwise_draws_of_the_generator_state_are_those_of_its_seed(bs, n, c, 
     finally:
         torch.cuda.synchronize()
         ext.manual_seed(torch.initial_seed())
+
+
+@pytest.mark.parametrize("cfg", [
+    dict(n=32, c=24, h=32, w=32, k=128, r=3, s=3, stride=(2, 1), padding=(1, 1), dilation=(1, 1)),
+    dict(n=64, c=24, h=32, w=32, k=128, r=3, s=3, stride=(2, 2), padding=(2, 2), dilation=(2, 2)),
+    dict(n=64, c=16, h=32, w=32, k=128, r=2, s=2, stride=(2, 2), padding=(0, 0), dilation=(1, 1)),  # one block column
+])
+def test_strided_convolutions_without_and_with_a_patch_matrix_agree(cfg):
+    """Layers whose three products need no patch matrix, off the tap-wise route, against the same with the switches off."""
+    import sys
+
+    import flash_dropout.functional as F
+
+    mod = sys.modules["flash_dropout.functional.im2col_conv2d"]  # the package re-exports a function of that name
+    gen = torch.Generator().manual_seed(cfg["n"])
+    fan_in = cfg["c"] * cfg["r"] * cfg["s"]
+    x = torch.randn(cfg["n"], cfg["c"], cfg["h"], cfg["w"], generator=gen).half().cuda()
+    k = (torch.randn(cfg["k"], cfg["c"], cfg["r"], cfg["s"], generator=gen) * fan_in ** -0.5).half().cuda()
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], cfg["r"], cfg["s"], **_geo(cfg))
+    dy = torch.randn(cfg["n"], cfg["k"], p_, q_, generator=gen).half().cuda()
+    mask = cpu_mask(O.mask_shape(cfg["n"] * p_ * q_, fan_in, 64), 0.5, gen).cuda()
+    out = []
+    for routes in (("implicit", "fused", "implicit"), ("explicit", "explicit", "explicit")):
+        old = mod.IMPLICIT_FORWARD, mod.FUSED_INPUT_GRADIENT
+        mod.IMPLICIT_FORWARD = mod.FUSED_INPUT_GRADIENT = routes[0] == "implicit"
+        try:
+            xg, kg = x.clone().requires_grad_(), k.clone().requires_grad_()
+            y = F.blockwise_dropout_conv2d_mask(xg, mask, 64, 0.5, kg, **_geo(cfg))
+            y.backward(dy)
+            assert tuple(F.conv_last_routes()[name] for name in ("forward", "dx", "dw")) == routes
+            out.append((y.detach(), xg.grad, kg.grad))
+        finally:
+            mod.IMPLICIT_FORWARD, mod.FUSED_INPUT_GRADIENT = old
+    for a, b, what in zip(*out, ("y", "dx", "dk")):
+        # sums in fp32 in another order, one rounding to fp16 of a product and, for dx, one of the fold
+        assert rel_fro(a, to_np(b)) <= 1e-3, what
