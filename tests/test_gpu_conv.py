@@ -938,3 +938,38 @@ def test_strided_convolutions_without_and_with_a_patch_matrix_agree(cfg):
     for a, b, what in zip(*out, ("y", "dx", "dk")):
         # sums in fp32 in another order, one rounding to fp16 of a product and, for dx, one of the fold
         assert rel_fro(a, to_np(b)) <= 1e-3, what
+
+
+# masks of blocks larger than the kernel's 64: rows and columns that end inside a block of the mask
+@pytest.mark.parametrize("cfg", [
+    dict(n=3, c=24, h=8, w=8, k=64, r=3, s=3, stride=(1, 1), padding=(1, 1), dilation=(1, 1)),      # 192 rows, 216 columns
+    dict(n=5, c=40, h=32, w=32, k=128, r=3, s=3, stride=(2, 2), padding=(1, 1), dilation=(1, 1)),   # 1280 rows, 360 columns
+    dict(n=1, c=16, h=16, w=16, k=192, r=5, s=3, stride=(2, 1), padding=(2, 1), dilation=(1, 1)),   # one image, 128 rows
+])
+@pytest.mark.parametrize("bs", [64, 128, 192, 1024])
+@pytest.mark.parametrize("by_columns", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fused_input_gradient_reads_masks_of_larger_blocks(cfg, bs, by_columns, dtype):
+    from flash_dropout.hip import GEMM
+
+    gen = torch.Generator().manual_seed(cfg["c"] + bs)
+    shape, ks = (cfg["n"], cfg["c"], cfg["h"], cfg["w"]), (cfg["r"], cfg["s"])
+    cols = cfg["c"] * cfg["r"] * cfg["s"]
+    p_, q_ = O.conv_out_hw(cfg["h"], cfg["w"], *ks, **_geo(cfg))
+    rows = cfg["n"] * p_ * q_
+    dy2 = torch.randn(rows, cfg["k"], generator=gen).to(dtype).cuda()
+    w2 = (torch.randn(cfg["k"], cols, generator=gen) * cfg["k"] ** -0.5).to(dtype).cuda()
+    mask = cpu_mask(O.mask_shape(rows, cols, bs), 0.4, gen)
+    given = mask.t().contiguous().t().cuda() if by_columns else mask.cuda()
+    strides = (1, max(given.shape[0], 1)) if by_columns else (given.shape[1], 1)
+    dx = torch.full(shape, float("nan"), dtype=dtype, device="cuda")
+    rc = GEMM().lib.sd_conv2d_dx_blocks(dy2.data_ptr(), dy2.stride(0), w2.data_ptr(), w2.stride(0), dx.data_ptr(), *dx.stride(),
+                                        given.data_ptr(), *strides, *shape, cfg["k"], *ks, *cfg["padding"], *cfg["stride"],
+                                        *cfg["dilation"], bs, 1 / 0.6, int(dtype == torch.bfloat16),
+                                        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    ref = O.col2im(O.sdd_dx(to_np(dy2), to_np(w2), mask.numpy(), bs, 0.4, np.float32), shape, *ks, **_geo(cfg))
+    assert max_tile_rel_fro(dx, ref) <= REL_FRO_TOL
+    # the same mask in blocks of 64: the same bits
+    fine = mask.repeat_interleave(bs // 64, 0).repeat_interleave(bs // 64, 1)[:-(-rows // 64), :-(-cols // 64)].contiguous().cuda()
+    assert torch.equal(dx, GEMM().conv2d_dx(dy2, w2, shape, ks, mask=fine, block_size=64, scale=1 / 0.6, **_geo(cfg)))
