@@ -640,6 +640,7 @@ struct ConvGeom {
 
 void check_conv_mask(const ConvGeom& g, int64_t bs, double p, const Draw& draw, Lists& l) {
   check_p(p);
+  TORCH_CHECK_VALUE(draw.mask || (float)p < 1.f, "p must be in [0, 1) in 32 bits to draw a mask, got ", p);  // whichever launch draws
   l.shape(g.rows(), g.cols(), bs);
   if (draw.mask)
     TORCH_CHECK_VALUE(draw.mask->dim() == 2 && draw.mask->size(0) == l.mb && draw.mask->size(1) == l.kb, "mask shape ",
@@ -1109,6 +1110,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   g.po = out_size(g.h, g.pad[0], g.dil[0], g.r, g.stride[0]);
   g.qo = out_size(g.w, g.pad[1], g.dil[1], g.s, g.stride[1]);
   TORCH_CHECK_VALUE(g.po > 0 && g.qo > 0, "kernel does not fit the padded image");
+  TORCH_CHECK_VALUE(g.k > 0 || !implicit_forward, "the kernel has no outputs");  // (the implicit products' refusal, on every route)
   Lists lists;
   Tensor y, y2, cols, w2;
   const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;

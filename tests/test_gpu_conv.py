@@ -973,3 +973,21 @@ def test_fused_input_gradient_reads_masks_of_larger_blocks(cfg, bs, by_columns, 
     # the same mask in blocks of 64: the same bits
     fine = mask.repeat_interleave(bs // 64, 0).repeat_interleave(bs // 64, 1)[:-(-rows // 64), :-(-cols // 64)].contiguous().cuda()
     assert torch.equal(dx, GEMM().conv2d_dx(dy2, w2, shape, ks, mask=fine, block_size=64, scale=1 / 0.6, **_geo(cfg)))
+
+
+@pytest.mark.parametrize("c,hw,r,stride", [(24, 16, 1, 1), (9, 7, 1, 1), (16, 32, 3, 2), (24, 8, 5, 1), (32, 28, 3, 1)])
+@pytest.mark.parametrize("channels_last", [False, True])
+def test_every_route_refuses_kernels_without_outputs_and_rates_that_round_to_one(c, hw, r, stride, channels_last):
+    import flash_dropout.functional as F
+
+    x = torch.ones(6, c, hw, hw, device="cuda", dtype=torch.float16)
+    if channels_last:
+        x = x.contiguous(memory_format=torch.channels_last)
+    wt = torch.ones(40, c, r, r, device="cuda", dtype=torch.float16)
+    for seed in (3, None):
+        with pytest.raises(ValueError):
+            F.blockwise_dropout_conv2d(x, wt[:0], 64, 0.4, r // 2, stride, seed=seed)
+        with pytest.raises(ValueError):
+            F.blockwise_dropout_conv2d(x, wt, 64, 1 - 1e-9, r // 2, stride, seed=seed)
+    with pytest.raises(ValueError):
+        F.im2col_conv2d(x, wt[:0], r // 2, stride)
