@@ -686,7 +686,7 @@ __global__ __launch_bounds__(THREADS) void col2im_unit_kernel(const uint16_t* __
 // channels at a time through LDS, both sides in pieces of 16 bytes; dropped blocks are not read.  Bound by its reads and writes:
 // 30 x 256 x 14 x 14 8.7 us with the kernel above, 4.5 so; 53 x 144 x 64 x 64 at p = 0.3 34 and 23; 200 x 200 x 56 x 56
 // at p = 0.6 136 and 77.
-constexpr int TURN_LD = TILE + 2;  // halfs per LDS row: 33 words, the reads down a column hit every bank once
+constexpr int TURN_LD = TILE + 2;  // halfs per LDS row: 33 words, so that the reads down a column meet no bank twice (32 words, two lanes to each)
 __global__ __launch_bounds__(256) void planes_from_rows_kernel(const uint16_t* __restrict__ rows, int64_t ld, uint16_t* __restrict__ dx,
                                                                int64_t sn, int64_t sc, int C, int P, int tiles_c, int tiles_p,
                                                                const uint8_t* mask, int64_t msr, int64_t msc, int bs) {

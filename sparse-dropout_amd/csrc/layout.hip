@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kPadThreads) void pad_rows_kernel(PadJobs js) {
 }
 
 constexpr int kTurn = 64;               // a workgroup turns a 64 x 64 tile
-constexpr int kTurnLd = kTurn + 2;      // halfs per LDS row: 33 words, so that the reads down a column hit every bank once
+constexpr int kTurnLd = kTurn + 2;      // halfs per LDS row: 33 words, so that the reads down a column meet no bank twice (32 words, two lanes to each)
 
 // dst[(n * P + i) * C + c] = src[n * sn + c * sc + i], i < P.  Bound by its reads and writes (a 64 MB copy at 128 images
 // of 128 x 32 x 32): both sides move in 128-byte pieces, 16 bytes per lane, and the tile is turned in LDS.  The

@@ -735,7 +735,7 @@ bool turned(const Tensor& x, const ConvGeom& g) {
 //    worst (32 x 40 x 64 x 64 -> 176, p = 0.5 105 -> 85 us, 215 x 32 x 64 x 64 -> 56, p = 0.6 264 -> 222)
 // Drawn from the generator's state the gather waits for a launch that draws (but for planes that are turned): passes of 180 layers of 4 to
 // 256 images, kernels of 1 to 5 x 5, 0.61 of those without where the same seeds take 0.57, 1.001 at worst.  The matrices of rows this few
-// come to 0.8 GB at most (63 x 512 x 16 x 16 -> 64, 7 x 7, p = 0.5 1590 us a pass for 1910).
+// stay under 0.9 GB (63 x 512 x 16 x 16 -> 64, 7 x 7, 809 MB, p = 0.5: 1590 us a pass for 1910).
 //  * input gradient, SDD and col2im against the fused kernel, both alone, 800 drawn geometries with kernels of 1 to 7 x 7, dilations and
 //    strides of 1 to 4: 0.25 where the fold stages windows (344, nine of them above 1.05, 3 x 3 but for one, 1.46 at worst), but 0.59 with
 //    the tile kernel (144, 33 above 1.1, 5.3 at worst: 128 x 32 x 32 x 32 -> 64, 3 x 3 by two down and one across, 83 -> 127 us a pass),
@@ -923,8 +923,9 @@ Tensor taps_forward(const Tensor& rows, const Tensor& packed, const ConvGeom& g,
 }
 
 struct ConvBackward : Node {
-  // the kernel as [K, C*R*S], and what the kernel's gradient reads: the patch matrix when the forward made one in memory, else
-  // the image (an implicit forward, or a pointwise kernel whose patch matrix is the image's own pixels)
+  // the kernel as [K, C*R*S], and what the kernel's gradient reads or is gathered from: the image in the geometries that the
+  // implicit products take, whichever way the forward went, and where a pointwise kernel's patch matrix is the image's own pixels,
+  // else the patch matrix that the forward made
   // (tap by tap: the image's rows when the forward made a copy of them that nothing else refers to, else the image)
   Saved w2, x, cols;
   SavedLists saved;  // nothing kept: no dropout

@@ -23,11 +23,13 @@ from .blockwise_dropout_matmul_hip import draw_source
 from .tracing import traceable
 
 
-# Use the implicit forward (sd_conv2d_taps_forward or sd_conv2d_dsd_lists) where the library takes the geometry.  Module-level
-# switch so that tests and benchmarks can compare both routes.
+# Let the forward run without a patch matrix (sd_conv2d_taps_forward or sd_conv2d_dsd_lists).  Module-level switch so that tests and
+# benchmarks can compare both routes: off, the forward goes through the matrix; on, where the library takes the geometry and,
+# with a mask, where that is expected to be faster (few rows and pointwise kernels of planes go through the matrix all the same).
 IMPLICIT_FORWARD = True
-# Use the one-launch input gradient (sd_conv2d_taps_dx or sd_conv2d_dx) where the library takes the geometry.  (Products run tap
-# by tap when both switches are on.)
+# The same for the input gradient in one launch (sd_conv2d_taps_dx or sd_conv2d_dx_blocks): on, masked layers whose matrix is wider than a
+# block, at most 256 MB and folded fast make the gradient of the patch matrix all the same.  (Products run tap by tap when both
+# switches are on.)
 FUSED_INPUT_GRADIENT = True
 
 _ROUTES = (None, "implicit", "fused", "explicit")
@@ -35,9 +37,10 @@ _ROUTES = (None, "implicit", "fused", "explicit")
 
 def conv_last_routes() -> dict:
     """{"forward": ..., "dx": ..., "dw": ...} of the process's last convolution run through this module: "implicit" /
-    "fused" (no patch matrix in memory: sd_conv2d_taps_*, or sd_conv2d_dsd_lists, sd_conv2d_dw_lists, sd_conv2d_dx) or "explicit" (im2col /
-    col2im around the GEMMs, taken when the library does not take the geometry or a switch above is off); None for a
-    product that was not computed.  Nothing falls back to the patch matrix unseen."""
+    "fused" (no patch matrix in memory: sd_conv2d_taps_*, or sd_conv2d_dsd_lists, sd_conv2d_dw_lists, sd_conv2d_dx_blocks) or "explicit"
+    (the patch matrix or its gradient in memory around the GEMMs: the library does not take the geometry, a switch above
+    is off, or, with a mask, that is expected to be faster); None for a product that was not computed.  Nothing falls back
+    to the patch matrix unseen."""
     return {k: _ROUTES[v] for k, v in zip(("forward", "dx", "dw"), _loader.bridge().conv_routes())}
 
 
@@ -84,8 +87,8 @@ def blockwise_dropout_conv2d_mask(input, mask, block_size, p: float, kernel, pad
 @traceable
 def blockwise_dropout_conv2d(input, kernel, block_size, p: float, padding=(0, 0), stride=(1, 1),
                              dilation=(1, 1), seed: int | None = None) -> torch.Tensor:
-    """Block-dropout convolution with a fresh mask over the patch matrix, drawn on the device inside the
-    list-building launch (``seed`` pins it, as for the matmul)."""
+    """Block-dropout convolution with a fresh mask over the patch matrix, drawn on the device by a launch that
+    the call needs anyway (``seed`` pins it, as for the matmul; gather and product of a pinned draw each evaluate it)."""
     if not 0 <= p < 1:
         raise ValueError("Dropout probability must be in [0, 1)")
     bs = _block_size(block_size)
