@@ -1113,7 +1113,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
   TORCH_CHECK_VALUE(g.po > 0 && g.qo > 0, "kernel does not fit the padded image");
   TORCH_CHECK_VALUE(g.k > 0 || !implicit_forward, "the kernel has no outputs");  // (the implicit products' refusal, on every route)
   Lists lists;
-  Tensor y, y2, cols, w2;
+  Tensor y, y2, cols;
   const float scale = bs ? (float)(1.0 / (1.0 - p)) : 1.f;
   const bool taps = implicit_forward && fused_dx && sd_conv2d_taps_taken_blocks(GEOM_X(g), g.k, g.r, g.s, GEOM_W(g), bs ? p : 0.0, bs);
   const bool record = records(std::array<Tensor, 2>{x, kernel});
@@ -1142,7 +1142,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     const Lists* l = bs ? &lists : nullptr;
     bool done = false;
     c10::DeviceGuard device(x.device());
-    w2 = kernel.detach().view({g.k, g.cols()});
+    const Tensor w2 = kernel.detach().view({g.k, g.cols()});  // (not what is kept: below autograd it has no part in kernel's version)
     const bool takes_implicit = implicit_forward && sd_conv2d_implicit_taken(x.data_ptr(), STRIDES4(x), kernel.data_ptr(), g.cols(),
                                                                               GEOM_X(g), g.k, g.r, g.s, GEOM_W(g));
     const Draw draw{mask, seed, state};
@@ -1190,7 +1190,7 @@ Tensor conv2d(const Tensor& input, const Tensor& kernel_in, const OptTensor& mas
     node->pixels = cols.defined() && cols.is_alias_of(x);
     if (cols.defined() && !node->pixels) node->cols.keep(cols);
     else if (keeps_input) node->x.keep(x);
-    node->w2.keep(w2.defined() ? w2 : kernel.detach().view({g.k, g.cols()}));
+    node->w2.keep(kernel.detach().view({g.k, g.cols()}));
     if (bs) node->saved.keep(std::move(lists), mask.value_or(Tensor()));
     node->g = g;
     node->p = bs ? p : 0.0;
