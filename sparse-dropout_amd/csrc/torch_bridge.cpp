@@ -733,9 +733,6 @@ bool turned(const Tensor& x, const ConvGeom& g) {
 //  * kernel's gradient: below 8192 rows 0.73, up to 16384 1.02, more 1.3; pointwise 0.90 below 16384 rows, above 1.16 gathered
 //  * both of pointwise kernels whose image's planes are turned: passes of 14 layers that the GPU bounds 0.92 of those without, 1.00 at
 //    worst (32 x 40 x 64 x 64 -> 176, p = 0.5 105 -> 85 us, 215 x 32 x 64 x 64 -> 56, p = 0.6 264 -> 222)
-// Drawn from the generator's state the gather waits for a launch that draws (but for planes that are turned): passes of 180 layers of 4 to
-// 256 images, kernels of 1 to 5 x 5, 0.61 of those without where the same seeds take 0.57, 1.001 at worst.  The matrices of rows this few
-// stay under 0.9 GB (63 x 512 x 16 x 16 -> 64, 7 x 7, 809 MB, p = 0.5: 1590 us a pass for 1910).
 //  * input gradient, SDD and col2im against the fused kernel, both alone, 800 drawn geometries with kernels of 1 to 7 x 7, dilations and
 //    strides of 1 to 4: 0.25 where the fold stages windows (344, nine of them above 1.05, 3 x 3 but for one, 1.46 at worst), but 0.59 with
 //    the tile kernel (144, 33 above 1.1, 5.3 at worst: 128 x 32 x 32 x 32 -> 64, 3 x 3 by two down and one across, 83 -> 127 us a pass),
@@ -743,6 +740,9 @@ bool turned(const Tensor& x, const ConvGeom& g) {
 //    kernel's reduction is short and the fold's sums are not: of more than 8 million terms three in seven took longer, 1.7 at worst
 //    (145 x 10 x 17 x 33 -> 64, 4 x 4, p = 0.25 112 -> 156 us a pass), of fewer 0.73 at worst.  1.03 to 1.09 where the matrix is one block
 //    wide.  Past 256 MB it stays out of memory.
+// Drawn from the generator's state the gather waits for a launch that draws (but for planes that are turned): passes of 180 layers of 4 to
+// 256 images, kernels of 1 to 5 x 5, 0.61 of those without where the same seeds take 0.57, 1.001 at worst.  The matrices of rows this few
+// stay under 0.9 GB (63 x 512 x 16 x 16 -> 64, 7 x 7, 809 MB, p = 0.5: 1590 us a pass for 1910).
 bool forward_by_patches(const Tensor& x, const ConvGeom& g) {
   return turned(x, g) || (g.r * g.s > 1 && ceil_div(g.rows(), 256) * ceil_div(g.k, 128) < 64);
 }
